@@ -1,396 +1,511 @@
-// Batched bf16 GEMM of the expert FFN, written for gfx950's matrix cores, and the transpose that
-// brings an operand into k-major form where the direct forms do not apply.
+// Batched bf16 GEMM of the expert FFN, written for gfx950's matrix cores, and the transpose of its operands.
 //
 //   C[e][m][n] = act( bf16( bf16( sum_k A[e][m][k] * B[e][n][k] ) + bias[e][n] ) )
 //
 // A matrix-core operand is eight consecutive k per lane.  An operand stored with k running fastest
 // ("N" for A, "T" for B) gives that as one 16-byte read of LDS; an operand stored the other way round
-// is read through LDS reads that transpose (ds_read_b64_tr_b16), so the direct-to-LDS kernel below
-// takes either operand either way.  The reference's experts (experts/ffn.py:63-82) compute
-// x @ fc1_w -> activation -> @ fc2_w with weights stored [experts, in, out]; the GEMM shapes of its
-// forward and backward pass are
+// is read through LDS reads that transpose (ds_read_b64_tr_b16), so the kernel takes either operand
+// either way.  The reference's experts (experts/ffn.py:63-82) compute x @ fc1_w -> activation -> @ fc2_w
+// with weights stored [experts, in, out]; the GEMM shapes of its forward and backward pass are
 //   forward   y  = x  @ W          A = x  [rows, in],   B = W  [in, out]      planmoe_gemm_nn_bf16
 //   backward  dx = dy @ W^T        A = dy [rows, out],  B = W  [in, out]      planmoe_gemm_nt_bf16
 //             dW = x^T @ dy        A = x  [rows, in],   B = dy [rows, out]    planmoe_gemm_tn_bf16
-// all with the operands as they lie in memory when the reduction length is a multiple of 64; for other
-// lengths planmoe_gemm_nt_bf16 serves on transposed copies (the register-staged kernel, any k % 8 == 0).
-//
-// Tile 256 x 256 x 64 per work-group of four waves; a wave owns 128 x 128 as 4 x 4 tiles of
-// v_mfma_f32_32x32x16_bf16 (256 accumulator registers, so one wave per SIMD: latency is covered by
-// what the wave itself has in flight).  Per k-step of 16 a wave reads 8 fragments of 1 KB from LDS
-// for 16 MFMAs of 32 cycles: LDS carries 64 bytes per clock for the four waves where 128 x 128
-// tiles of 16 x 16 x 32 MFMAs (64 x 64 per wave) need 256.  LDS rows are 144 bytes apart (128 of
-// data + 16): consecutive rows shift by one 16-byte unit, so the 8 / 16 rows that one pass of a
-// fragment read or of a tile write touches fall into different banks whether the LDS serves 32 or
-// 64 banks per clock.  LDS holds two k-tiles of both operands (144 KB); global loads run two
-// k-tiles ahead in two register sets; one LDS-only barrier per k-tile, so the loads in flight
-// stay in flight across it.  Epilogue: every wave passes its 128 x 128 quadrant through its own
-// LDS region and stores whole 16-byte pieces of rows.
+// all with the operands as they lie in memory.
 #include "common.hpp"
 
 namespace pm {
 
 typedef float  f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 gemm_bf16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int GEMM_BM = 256, GEMM_BN = 256, GEMM_BK = 64;
-constexpr int GEMM_PITCH = 144;                             // bytes between LDS rows of a k-tile
-constexpr int GEMM_TILE = 256 * GEMM_PITCH;                 // one operand's k-tile in LDS
-constexpr int GEMM_CPITCH = 272;                            // bytes between rows of a wave's output quadrant in LDS
-constexpr int GEMM_LDS = 4 * GEMM_TILE;                     // A0 B0 A1 B1 (the epilogue's 4 x 128 x 272 fits inside)
-static_assert(4 * 128 * GEMM_CPITCH <= GEMM_LDS, "the output quadrants reuse the operand space");
-
-__device__ __forceinline__ void gemm_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-struct GemmArgs {
-    const uint16_t *A, *B, *bias;
-    uint16_t *C;
-    int M, N, K;                  // rows of A, rows of B, reduction length
-    int lda, ldb, ldc;            // elements between rows
-    int64_t sA, sB, sC, sBias;    // elements between batches
-    int batches;
-};
-
-template <int ACT>
-__global__ __launch_bounds__(256, 1) void gemm_nt_bf16_kernel(const GemmArgs p)
-{
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int e = blockIdx.z, m0 = blockIdx.y * GEMM_BM, n0 = blockIdx.x * GEMM_BN;
-    const uint8_t *A = reinterpret_cast<const uint8_t *>(p.A + (int64_t)e * p.sA);
-    const uint8_t *B = reinterpret_cast<const uint8_t *>(p.B + (int64_t)e * p.sB);
-
-    // what a thread fetches of one k-tile: chunk lc (8 values) of rows lr + 32 i of both operands.
-    // Byte offsets from the batch's base (the host checks that they fit 32 bits); rows past the end
-    // read the last row again (their products land in rows / columns nobody stores).
-    const int lr = tid >> 3, lc = tid & 7;
-    uint32_t ao[8], bo[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        ao[i] = (uint32_t)min(m0 + lr + 32 * i, p.M - 1) * (uint32_t)p.lda * 2u;
-        bo[i] = (uint32_t)min(n0 + lr + 32 * i, p.N - 1) * (uint32_t)p.ldb * 2u;
-    }
-    // Every load is unconditional and straight-line (a chunk past
-    // the end of K reads the row's last chunk instead and is zeroed by `keep` on its way into LDS).
-    struct Fetched { uint4 a0, a1, a2, a3, a4, a5, a6, a7, b0, b1, b2, b3, b4, b5, b6, b7; uint32_t keep; } f0;
-    const int KT = (p.K + GEMM_BK - 1) / GEMM_BK;
-    const uint32_t last_chunk = (uint32_t)(p.K - 8) * 2u;
-    auto load_tile = [&](Fetched &f, int kt) {
-        const uint32_t kb = min((uint32_t)(kt * GEMM_BK + lc * 8) * 2u, last_chunk);
-        f.keep = (kt < KT && kt * GEMM_BK + lc * 8 < p.K) ? 0xffffffffu : 0u;
-#define PM_LD(dst, base, o) f.dst = *reinterpret_cast<const uint4 *>(base + (o + kb))
-        PM_LD(a0, A, ao[0]); PM_LD(a1, A, ao[1]); PM_LD(a2, A, ao[2]); PM_LD(a3, A, ao[3]);
-        PM_LD(a4, A, ao[4]); PM_LD(a5, A, ao[5]); PM_LD(a6, A, ao[6]); PM_LD(a7, A, ao[7]);
-        PM_LD(b0, B, bo[0]); PM_LD(b1, B, bo[1]); PM_LD(b2, B, bo[2]); PM_LD(b3, B, bo[3]);
-        PM_LD(b4, B, bo[4]); PM_LD(b5, B, bo[5]); PM_LD(b6, B, bo[6]); PM_LD(b7, B, bo[7]);
-#undef PM_LD
-    };
-    auto store_tile = [&](const Fetched &f, int buf) {
-        uint8_t *sa = lds + buf * 2 * GEMM_TILE + lr * GEMM_PITCH + lc * 16, *sb = sa + GEMM_TILE;
-        const uint32_t k = f.keep;
-#define PM_ST(base, i, v) *reinterpret_cast<uint4 *>(base + (i) * 32 * GEMM_PITCH) = make_uint4(f.v.x & k, f.v.y & k, f.v.z & k, f.v.w & k)
-        PM_ST(sa, 0, a0); PM_ST(sa, 1, a1); PM_ST(sa, 2, a2); PM_ST(sa, 3, a3);
-        PM_ST(sa, 4, a4); PM_ST(sa, 5, a5); PM_ST(sa, 6, a6); PM_ST(sa, 7, a7);
-        PM_ST(sb, 0, b0); PM_ST(sb, 1, b1); PM_ST(sb, 2, b2); PM_ST(sb, 3, b3);
-        PM_ST(sb, 4, b4); PM_ST(sb, 5, b5); PM_ST(sb, 6, b6); PM_ST(sb, 7, b7);
-#undef PM_ST
-    };
-
-    f32x16 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-
-    // lane l of a fragment: row l % 32, k-chunk l / 32 of the step.  The fragments of step s + 1 are
-    // requested before the MFMAs of step s are issued (two fragment sets, used in turn).
-    const int fr = lane & 31, fc = lane >> 5;
-    struct Frags { gemm_bf16x8 a0, a1, a2, a3, b0, b1, b2, b3; };
-    auto read_frags = [&](Frags &f, const uint8_t *sa, const uint8_t *sb, int ks) {
-        f.a0 = *reinterpret_cast<const gemm_bf16x8 *>(sa + 0 * 32 * GEMM_PITCH + ks * 32);
-        f.a1 = *reinterpret_cast<const gemm_bf16x8 *>(sa + 1 * 32 * GEMM_PITCH + ks * 32);
-        f.a2 = *reinterpret_cast<const gemm_bf16x8 *>(sa + 2 * 32 * GEMM_PITCH + ks * 32);
-        f.a3 = *reinterpret_cast<const gemm_bf16x8 *>(sa + 3 * 32 * GEMM_PITCH + ks * 32);
-        f.b0 = *reinterpret_cast<const gemm_bf16x8 *>(sb + 0 * 32 * GEMM_PITCH + ks * 32);
-        f.b1 = *reinterpret_cast<const gemm_bf16x8 *>(sb + 1 * 32 * GEMM_PITCH + ks * 32);
-        f.b2 = *reinterpret_cast<const gemm_bf16x8 *>(sb + 2 * 32 * GEMM_PITCH + ks * 32);
-        f.b3 = *reinterpret_cast<const gemm_bf16x8 *>(sb + 3 * 32 * GEMM_PITCH + ks * 32);
-    };
-#define PM_MMA(i, j, x, y) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc[i][j], 0, 0, 0)
-    auto mma_step = [&](const Frags &f) {
-        PM_MMA(0, 0, f.a0, f.b0); PM_MMA(0, 1, f.a0, f.b1); PM_MMA(0, 2, f.a0, f.b2); PM_MMA(0, 3, f.a0, f.b3);
-        PM_MMA(1, 0, f.a1, f.b0); PM_MMA(1, 1, f.a1, f.b1); PM_MMA(1, 2, f.a1, f.b2); PM_MMA(1, 3, f.a1, f.b3);
-        PM_MMA(2, 0, f.a2, f.b0); PM_MMA(2, 1, f.a2, f.b1); PM_MMA(2, 2, f.a2, f.b2); PM_MMA(2, 3, f.a2, f.b3);
-        PM_MMA(3, 0, f.a3, f.b0); PM_MMA(3, 1, f.a3, f.b1); PM_MMA(3, 2, f.a3, f.b2); PM_MMA(3, 3, f.a3, f.b3);
-    };
-#undef PM_MMA
-    auto multiply = [&](int buf) {
-        const uint8_t *sa = lds + buf * 2 * GEMM_TILE + (wm * 128 + fr) * GEMM_PITCH + fc * 16;
-        const uint8_t *sb = lds + buf * 2 * GEMM_TILE + GEMM_TILE + (wn * 128 + fr) * GEMM_PITCH + fc * 16;
-        Frags g0, g1;
-        read_frags(g0, sa, sb, 0);
-        read_frags(g1, sa, sb, 1);
-        mma_step(g0);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(g0, sa, sb, 2);
-        mma_step(g1);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(g1, sa, sb, 3);
-        mma_step(g0);
-        __builtin_amdgcn_sched_barrier(0);
-        mma_step(g1);
-    };
-
-    // one k-tile in registers on its way to LDS while the tile before it is multiplied
-    load_tile(f0, 0);
-    store_tile(f0, 0);
-    gemm_lds_barrier();
-    for (int kt = 0; kt < KT; ++kt) {
-        load_tile(f0, kt + 1);                   // (past the end: zeros, never multiplied)
-        multiply(kt & 1);
-        store_tile(f0, (kt + 1) & 1);
-        gemm_lds_barrier();
-    }
-    // every wave is done with the operand tiles before a quadrant overwrites them
-    __syncthreads();
-
-    // epilogue: acc[i][j][q] is row 32 i + 8 (q / 4) + 4 (lane / 32) + q % 4, column 32 j + lane % 32 of the quadrant
-    uint8_t *quad = lds + wave * 128 * GEMM_CPITCH;
-    const uint16_t *bias = p.bias ? p.bias + (int64_t)e * p.sBias + n0 + wn * 128 : nullptr;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = 32 * j + fr;
-        const float fb = bias && n0 + wn * 128 + col < p.N ? bf16_to_f32(bias[col]) : 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int row = 32 * i + 8 * (q >> 2) + 4 * fc + (q & 3);
-                float v = bf16_to_f32(f32_to_bf16(acc[i][j][q]));       // the matmul's own rounding
-                if (bias) v = bf16_to_f32(f32_to_bf16(v + fb));         // torch.add in bf16
-                if (ACT == 1) v = fmaxf(v, 0.f);
-                *reinterpret_cast<uint16_t *>(quad + row * GEMM_CPITCH + col * 2) = (uint16_t)f32_to_bf16(v);
-            }
-    }
-    __builtin_amdgcn_wave_barrier();
-    uint16_t *C = p.C + (int64_t)e * p.sC;
-#pragma unroll 4
-    for (int t = 0; t < 32; ++t) {
-        const int q = lane + 64 * t, row = q >> 4, c = q & 15;
-        const int gr = m0 + wm * 128 + row, gc = n0 + wn * 128 + c * 8;
-        if (gr < p.M && gc < p.N)
-            *reinterpret_cast<uint4 *>(C + (int64_t)gr * p.ldc + gc) = *reinterpret_cast<const uint4 *>(quad + row * GEMM_CPITCH + c * 16);
-    }
-}
-
-// ---- the same product with the operands loaded straight into LDS (global_load_lds_dwordx4: the
-// memory pipeline writes LDS itself, 16 bytes per lane at consecutive addresses, no register and no
-// LDS-store instruction in between).  k-tiles of 64; LDS holds two of them for both operands and
-// the loads of a tile are in flight during the MFMAs of the tile before it.  A load instruction
-// fills 1 KB = 8 rows of 128 bytes; which 16-byte chunk of its row a lane fetches is chosen so
-// that chunk c of row r lies at unit c ^ (r >> 1) & 7 of the row.  The LDS of this GPU serves 64
-// banks (256 bytes) per clock, a 16-byte read 16 lanes at a time: the 16 consecutive rows of such a
-// pass are 8 pairs of rows, the rows of a pair in different halves of the 256 bytes, the pairs at
-// 8 different units.  (Measured with SQ_LDS_BANK_CONFLICT: 1.3 M conflict cycles per launch at
-// 8 x 5120 x 4096 x 4096 against 85 M with c ^ r & 7, which would suit an LDS of 32 banks.)
-// Needs k % 64 == 0.
-constexpr int DMA_BK = 64, DMA_STAGES = 2;
-constexpr int DMA_ROW = DMA_BK * 2;                         // bytes of a row of a k-tile
-constexpr int DMA_OPERAND = 256 * DMA_ROW;                  // bytes of one operand's k-tile
-constexpr int DMA_STAGE = 2 * DMA_OPERAND;
-constexpr int DMA_LOADS = DMA_OPERAND / 1024 / 4;           // load instructions per wave, operand and k-tile
-static_assert(DMA_STAGES * DMA_STAGE <= GEMM_LDS, "the kernels share the launch's LDS size");
-
-__device__ __forceinline__ void gemm_dma16(const void *gbase, uint32_t voff, uint32_t lds_addr)
-{
-    // 16 bytes per lane from gbase + voff to LDS at lds_addr + 16 * lane
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_addr), "v"(voff), "s"(gbase) : "memory", "m0");
-}
-// where chunk c of row r lies in its row of 8 units
-__device__ __forceinline__ int dma_unit(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
-
-// TA / TB = true: the operand is stored the other way round, a[e][k][m] / b[e][k][n] (both: c = a^T b, the
-// weight gradient x^T dy; only b: c = a b with a weight as experts/ffn.py stores it; no transposed copies
-// either way): a k-tile of such an operand is 64 rows of 512 bytes,
-// a load instruction fills two of them, chunk c of row k lies at unit c ^ (k & 3) << 2, and a fragment
-// comes out of LDS through ds_read_b64_tr_b16, which hands lane i of every 16 lanes element i % 4 of
-// the 8 bytes that lanes i / 4, i / 4 + 4, i / 4 + 8, i / 4 + 12 point at: with lane s pointing at row
-// s / 4, columns 4 (s % 4) .. + 3 of a 4 x 16 patch, lane i receives 4 consecutive k of column i --
-// the matrix cores' operand layout.  Two such reads make the 8 k of a step; the 4 rows of a patch lie
-// in different quarters of the 256 bytes the LDS serves per clock.  Needs k % 64 == 0.
 typedef short gemm_s16x4 __attribute__((ext_vector_type(4)));
 typedef short gemm_s16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ gemm_bf16x8 gemm_read_tr(const uint8_t *lo, const uint8_t *hi)
+typedef uint32_t gemm_u32x4 __attribute__((ext_vector_type(4)));
+typedef const uint8_t __attribute__((address_space(3))) *gemm_lds_ptr;
+
+// ds_read_b64_tr_b16 hands lane i of every 16 lanes element i % 4 of the 8 bytes that lanes i / 4, i / 4 + 4, i / 4 + 8,
+// i / 4 + 12 point at: with lane s pointing at row s / 4, columns 4 (s % 4) .. + 3 of a 4 x 16 patch, lane i receives 4
+// consecutive k of column i -- the matrix cores' operand layout.  Two such reads make the 8 k of a step.
+__device__ __forceinline__ gemm_bf16x8 gemm_read_tr(gemm_lds_ptr lo, gemm_lds_ptr hi)
 {
     typedef gemm_s16x4 __attribute__((address_space(3))) *lds_s16x4;
     const gemm_s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)lo);
     const gemm_s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)hi);
-    const gemm_s16x8 v = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(gemm_bf16x8, v);
+    return __builtin_bit_cast(gemm_bf16x8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int ACT, bool TA = false, bool TB = false>
-__global__ __launch_bounds__(256, 1) void gemm_nt_bf16_dma_kernel(const GemmArgs p)
+// ---------------------------------------------------------------- the kernel
+// Tiles of 256 x 256 (or 128 on a side), k-tiles of 64, four waves.  Each side of a tile is two halves;
+// a wave has 32 I rows of either A half and 32 J columns of either B half, so its share of the tile is
+// four quadrants and a k-tile is four phases, one quadrant each: 4 I J v_mfma_f32_32x32x16_bf16.
+// During a phase the wave reads from LDS the one half of an operand that the next phase needs and has
+// not got (the quadrants of successive k-tiles are walked so that this is always one half), and asks
+// for one half of a k-tile two further on, straight into LDS (buffer_load ... lds), into the space
+// that the phase before has finished reading.  So a half is asked for seven phases (about 3500 clocks
+// at 256 x 256) before it is read, LDS holds two k-tiles, and a phase ends in one wait -- by count, for
+// the half the next phase reads -- and one barrier.  The loads and LDS reads are placed between the
+// MFMAs one at a time: a wave issues in order, and a burst of them would leave its matrix core idle.
+//
+// The stream of k-tiles does not stop at the end of an output tile: work-groups stay (one per compute
+// unit) and go from tile to tile, and the loads of the next tile's first k-tiles are in flight while
+// the results of this one are rounded and stored.
+//
+// Out of range is the buffer descriptor's business: rows past the end, reduction rows past the end and
+// everything behind the last tile read as zero, stores past the end are dropped.
+//
+// What bounds it: with operands of zeros 8 x 5120 x 4096 x 4096 takes 740 us (1860 TFLOP/s, 0.74 of the
+// 2.5 PFLOP/s), with N(0, 1) operands 1030 - 1130 us (1220 - 1340): the clock the GPU holds under the
+// matrix cores.  (A kernel with the same tile that waited for a whole k-tile at a time and issued its
+// loads and LDS reads in bursts took 1260 us, 890 us with zeros.)
+constexpr int GEMM_BK = 64;
+constexpr int GEMM_WG = 256;
+constexpr int GEMM_TABLE_BYTES = 2 * 64 * 4;                // tiles before each batch, its rows (with `live`)
+constexpr int GEMM_BIAS_BYTES = 2 * 1024;                   // the tile's slice of the bias, two tiles in turn
+
+struct GemmArgs {
+    const uint16_t *A, *B, *bias;
+    const uint16_t *mask;         // GRAD: c is kept where mask > 0 (c's shape and pitches), else zero
+    uint16_t *C;
+    float *colsum;                // GRAD: [batches][2 tile rows][N] column sums of what was stored, NULL: none
+    const int *live;              // [live_planes][batches]: rows in use per batch (k of a tn product), NULL: all
+    int live_planes, live_round;
+    int M, N, K;
+    int lda, ldb, ldc;            // elements between rows
+    int64_t sA, sB, sC;           // elements between batches
+    int batches, relu;
+    bool bias_by_value;           // the bias is not 16-byte aligned: read where it is used
+};
+
+__device__ __forceinline__ gemm_u32x4 gemm_desc(const void *base, int64_t bytes)
 {
+    const uint64_t a = (uint64_t)base;
+    const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffff ? 0x7fffffffu : (uint32_t)bytes;
+    return gemm_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, n, 0x00020000u};
+}
+constexpr uint32_t GEMM_NOWHERE = 0x80000000u;              // an offset that is out of any descriptor's range
+// 16 bytes per lane from the buffer at voff + soff to LDS at lds_addr + 16 * lane
+__device__ __forceinline__ void gemm_dma16(gemm_u32x4 desc, uint32_t voff, uint32_t soff, uint32_t lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
+}
+template <int N> __device__ __forceinline__ void gemm_phase_wait()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
+// I, J: a tile is 128 I rows by 128 J columns
+template <int I, int J>
+struct GemmShape {
+    static constexpr int BM = 128 * I, BN = 128 * J;
+    // LDS: both stages of A, both stages of B (so that an operand's halves are all within the 64 KB that an
+    // LDS instruction's offset covers), the waves' output pieces (32 rows of 32 J values each), tables
+    static constexpr int half_at(int o, int stage, int h)
+    {
+        return o == 0 ? (2 * stage + h) * 8192 * I : 4 * 8192 * I + (2 * stage + h) * 8192 * J;
+    }
+    static constexpr int OPERANDS = 4 * 8192 * (I + J);
+    static constexpr int PITCH = 64 * J + 16;               // bytes between rows of an output piece
+    static constexpr int TABLE = OPERANDS + 4 * 32 * PITCH, BIAS = TABLE + GEMM_TABLE_BYTES;
+    static constexpr int LDS = BIAS + GEMM_BIAS_BYTES;
+    static constexpr int STORES = 8 * I * J;                // 16-byte stores of a lane per tile
+    // loads a wave issues in phase p, and how many of them may be outstanding at its end: the half that
+    // phase p + 1 reads was asked for six phases before p, what is younger is not needed yet
+    static constexpr int loads(int p) { return (p & 3) < 2 ? 2 * J : 2 * I; }
+    static constexpr int wait(int p)
+    {
+        int s = 0;
+        for (int j = 0; j < 6; ++j) s += loads(p - j + 8);
+        return s;
+    }
+    static_assert(wait(3) + STORES < 64 && wait(1) + STORES < 64, "the counter of outstanding loads and stores has six bits");
+    static constexpr int WAVES_PER_SIMD = LDS * 2 <= 160 * 1024 ? 2 : 1;     // (= work-groups per compute unit)
+};
+
+template <int I, int J, bool TA, bool TB, bool GRAD>
+__global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void gemm_bf16_kernel(const GemmArgs p)
+{
+    using S = GemmShape<I, J>;
     extern __shared__ __align__(16) uint8_t lds[];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    // Work-groups go to the 8 XCDs in turn, each XCD with an L2 of its own: XCD j (work-groups j, j + 8,
-    // ...) takes the j-th eighth of the tiles, in the order batch, panel of 8 tile columns, tile row,
-    // column of the panel, so that the 32 tiles it works on at a time are a 4 x 8 block of one batch
-    // (12 operand tiles for 32 products; measured at 8 x 5120 x 4096 x 4096: L2 hits 69 -> 80 %, HBM reads
-    // 3.3 -> 2.0 GB per launch).  The grid is one-dimensional, a multiple of 8; the surplus returns.
-    const int tiles_m = (p.M + GEMM_BM - 1) / GEMM_BM, tiles_n = (p.N + GEMM_BN - 1) / GEMM_BN;
-    const int64_t tiles = (int64_t)tiles_m * tiles_n * p.batches, per_xcd = (tiles + 7) / 8;
-    const int64_t tile = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (tile >= tiles) return;
-    const int e = (int)(tile / (tiles_m * tiles_n));
-    int in_batch = (int)(tile - (int64_t)e * tiles_m * tiles_n);
-    const int panel = in_batch / (tiles_m * 8);
-    in_batch -= panel * tiles_m * 8;
-    const int panel_width = min(8, tiles_n - panel * 8);
-    const int m0 = (in_batch / panel_width) * GEMM_BM, n0 = (panel * 8 + in_batch % panel_width) * GEMM_BN;
-    const uint8_t *A = reinterpret_cast<const uint8_t *>(p.A + (int64_t)e * p.sA);
-    const uint8_t *B = reinterpret_cast<const uint8_t *>(p.B + (int64_t)e * p.sB);
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);        // (in a scalar register: LDS addresses of the loads are)
 
-    // wave w brings in rows 64 w .. 64 w + 63 of both operands: 8 loads of 8 rows each.  Lane l of a
-    // load fills unit l % 8 of row l / 8 of the block, i.e. fetches the chunk that belongs there.
-    uint32_t ao[DMA_LOADS], bo[DMA_LOADS];
-#pragma unroll
-    for (int i = 0; i < DMA_LOADS; ++i) {
-        // an operand with the reduction index slow: wave w brings in rows (k) 16 w .. 16 w + 15 of its
-        // tile, 8 loads of 2 rows of 512 bytes
-        const int trow = 16 * wave + 2 * i + (lane >> 5), tchunk = (lane & 31) ^ ((trow & 3) << 2);
-        const int row = 64 * wave + 8 * i + (lane >> 3), chunk = dma_unit(row, lane & 7);
-        ao[i] = TA ? (uint32_t)trow * (uint32_t)p.lda * 2u + (uint32_t)min(m0 + tchunk * 8, p.M - 8) * 2u
-                   : (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.lda * 2u + chunk * 16;
-        bo[i] = TB ? (uint32_t)trow * (uint32_t)p.ldb * 2u + (uint32_t)min(n0 + tchunk * 8, p.N - 8) * 2u
-                   : (uint32_t)min(n0 + row, p.N - 1) * (uint32_t)p.ldb * 2u + chunk * 16;
-    }
-    const int KT = p.K / DMA_BK;
-    // a quarter of the loads of tile kt (a tile's loads go out in four parts, one before each k-step
-    // of the tile before: 16 loads in a row hold the wave up at the address unit, and arrive in one burst)
-    auto load_part = [&](int kt, int part) {
-        // past the end: the last tile once more, into a buffer nobody reads again (keeps the number
-        // of loads in flight the same in every round, which the waits below count on)
-        const int k = min(kt, KT - 1);
-        const uint8_t *ga = A + (TA ? (int64_t)k * DMA_BK * p.lda * 2 : (int64_t)k * (DMA_BK * 2));
-        const uint8_t *gb = B + (TB ? (int64_t)k * DMA_BK * p.ldb * 2 : (int64_t)k * (DMA_BK * 2));
-        const uint32_t sa = lds0 + (kt % DMA_STAGES) * DMA_STAGE + wave_u * (64 * DMA_ROW), sb = sa + DMA_OPERAND;   // (a wave's share is 8 KB either way)
-        constexpr int PER = DMA_LOADS / 4;
-#pragma unroll
-        for (int i = PER * part; i < PER * part + PER; ++i) gemm_dma16(ga, ao[i], sa + i * 1024);
-#pragma unroll
-        for (int i = PER * part; i < PER * part + PER; ++i) gemm_dma16(gb, bo[i], sb + i * 1024);
-    };
-    static_assert(DMA_LOADS % 4 == 0, "a tile's loads go out in four parts");
-
-    f32x16 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-
-    // fragment of a step: lane l holds row l % 32, chunk 2 ks + l / 32 of its rows
-    const int fr = lane & 31, fc = lane >> 5;
-    struct Frags { gemm_bf16x8 a0, a1, a2, a3, b0, b1, b2, b3; };
-    // an operand with the reduction index slow: lane = (group g of 16 lanes, s): row 8 (g / 2) + s / 4 of the step's 16, bytes 8 (s % 4) of the
-    // 32 that columns 16 (g % 2) .. + 15 of the fragment take; unit of the row swizzled by s / 4 = row & 3
-    const int tg = lane >> 4, ts = lane & 15;
-    const int t_row = (8 * (tg >> 1) + (ts >> 2)) * 512;
-    int t_col[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t_col[i] = (4 * (i ^ (ts >> 2)) + 2 * (tg & 1) + ((ts & 3) >> 1)) * 16 + 8 * (ts & 1);
-    auto read_frags = [&](Frags &f, const uint8_t *st, int ks) {
-#define PM_FT(base, i) gemm_read_tr(base + t_col[i], base + t_col[i] + 4 * 512)
-#define PM_FR(base, i) *reinterpret_cast<const gemm_bf16x8 *>(base + (i) * 32 * DMA_ROW + dma_unit(32 * (i) + fr, 2 * ks + fc) * 16)
-        if constexpr (TA) {
-            const uint8_t *sa = st + t_row + ks * (16 * 512) + wm * 256;
-            f.a0 = PM_FT(sa, 0); f.a1 = PM_FT(sa, 1); f.a2 = PM_FT(sa, 2); f.a3 = PM_FT(sa, 3);
-        } else {
-            const uint8_t *sa = st + (wm * 128 + fr) * DMA_ROW;
-            f.a0 = PM_FR(sa, 0); f.a1 = PM_FR(sa, 1); f.a2 = PM_FR(sa, 2); f.a3 = PM_FR(sa, 3);
+    // ---- the tiles: work-groups go to the 8 XCDs in turn, each XCD (with an L2 of its own) takes an
+    // eighth of the tiles in a row, in the order batch, panel of 8 tile columns, tile row, column, so
+    // that the tiles it works on at a time share operands (12 operand tiles for 32 products at 256 x 256).
+    // With `live` the tiles of a batch are those of its rows in use: table[e] is the number before batch e.
+    const int tiles_n = (p.N + S::BN - 1) / S::BN;
+    int total;
+    int *table = reinterpret_cast<int *>(lds + S::TABLE);
+    if (p.live) {
+        int n = 0;
+        if (lane < p.batches)
+            for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + lane];
+        const int rows = min(TA ? p.K : p.M, (n + p.live_round - 1) / p.live_round * p.live_round);
+        const int mine = lane < p.batches ? ((TA ? p.M : rows) + S::BM - 1) / S::BM * tiles_n : 0;
+        int inc = mine;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d);
+            if (lane >= d) inc += o;
         }
-        if constexpr (TB) {
-            const uint8_t *sb = st + DMA_OPERAND + t_row + ks * (16 * 512) + wn * 256;
-            f.b0 = PM_FT(sb, 0); f.b1 = PM_FT(sb, 1); f.b2 = PM_FT(sb, 2); f.b3 = PM_FT(sb, 3);
-        } else {
-            const uint8_t *sb = st + DMA_OPERAND + (wn * 128 + fr) * DMA_ROW;
-            f.b0 = PM_FR(sb, 0); f.b1 = PM_FR(sb, 1); f.b2 = PM_FR(sb, 2); f.b3 = PM_FR(sb, 3);
-        }
-#undef PM_FR
-#undef PM_FT
-    };
-#define PM_MMA(i, j, x, y) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc[i][j], 0, 0, 0)
-    auto mma_step = [&](const Frags &f) {
-        PM_MMA(0, 0, f.a0, f.b0); PM_MMA(0, 1, f.a0, f.b1); PM_MMA(0, 2, f.a0, f.b2); PM_MMA(0, 3, f.a0, f.b3);
-        PM_MMA(1, 0, f.a1, f.b0); PM_MMA(1, 1, f.a1, f.b1); PM_MMA(1, 2, f.a1, f.b2); PM_MMA(1, 3, f.a1, f.b3);
-        PM_MMA(2, 0, f.a2, f.b0); PM_MMA(2, 1, f.a2, f.b1); PM_MMA(2, 2, f.a2, f.b2); PM_MMA(2, 3, f.a2, f.b3);
-        PM_MMA(3, 0, f.a3, f.b0); PM_MMA(3, 1, f.a3, f.b1); PM_MMA(3, 2, f.a3, f.b2); PM_MMA(3, 3, f.a3, f.b3);
-    };
-#undef PM_MMA
-
-#pragma unroll
-    for (int part = 0; part < 4; ++part) load_part(0, part);
-    for (int kt = 0; kt < KT; ++kt) {
-        // this wave's loads of tile kt are in; behind the barrier everybody's are, and everybody is
-        // done reading tile kt - 1, whose buffer the loads of tile kt + 1 then fill during this tile's MFMAs
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-        const uint8_t *st = lds + (kt % DMA_STAGES) * DMA_STAGE;
-        Frags g0, g1;
-        read_frags(g0, st, 0);
-        read_frags(g1, st, 1);
-        load_part(kt + 1, 0);
-        mma_step(g0);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(g0, st, 2);
-        load_part(kt + 1, 1);
-        mma_step(g1);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(g1, st, 3);
-        load_part(kt + 1, 2);
-        mma_step(g0);
-        __builtin_amdgcn_sched_barrier(0);
-        load_part(kt + 1, 3);
-        mma_step(g1);
+        // (every wave writes the same values and reads only what it wrote itself)
+        table[lane] = lane < p.batches ? inc - mine : 0x7fffffff;
+        table[64 + lane] = rows;
+        total = __builtin_amdgcn_readlane(inc, 63);
+    } else {
+        total = (p.M + S::BM - 1) / S::BM * tiles_n * p.batches;
     }
-    // nothing may still be on its way into LDS when the quadrants overwrite it
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    const int per_xcd = (total + 7) / 8;
+    const int first_tile = blockIdx.x % 8 * per_xcd, stride = gridDim.x / 8;
+    struct Where { int e, m0, n0, rows; };        // rows: M of the batch (its K for a tn product)
+    auto locate = [&](int j) {                    // j-th tile of this XCD (in range)
+        const int tile = first_tile + j;
+        Where w;
+        int first, tm;
+        if (p.live) {
+            // (batches without tiles share the next one's number: the last of them is the one)
+            const int before = table[lane], rows = table[64 + lane];
+            w.e = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before <= tile)) - 1);
+            first = __builtin_amdgcn_readlane(before, w.e);
+            w.rows = __builtin_amdgcn_readlane(rows, w.e);
+            tm = ((TA ? p.M : w.rows) + S::BM - 1) / S::BM;
+        } else {
+            tm = (p.M + S::BM - 1) / S::BM;
+            w.e = tile / (tm * tiles_n);
+            first = w.e * tm * tiles_n;
+            w.rows = TA ? p.K : p.M;
+        }
+        int in = tile - first;
+        const int panel = in / (tm * 8);
+        in -= panel * tm * 8;
+        const int width = min(8, tiles_n - panel * 8);
+        w.m0 = in / width * S::BM;
+        w.n0 = (panel * 8 + in % width) * S::BN;
+        return w;
+    };
+    auto in_range = [&](int j) { return j < per_xcd && first_tile + j < total; };
 
-    uint8_t *quad = lds + wave * 128 * GEMM_CPITCH;
-    const uint16_t *bias = p.bias ? p.bias + (int64_t)e * p.sBias + n0 + wn * 128 : nullptr;
+    // ---- where the loads are: a cursor over the k-tiles of this work-group's tiles, one after another.
+    // A tile takes an even number of k-tiles (the loop below does two at a time); the odd one past the end reads as zero.
+    struct Cursor { const uint8_t *a, *b; int64_t ra, rb; int left, real, j; };    // left: k-tiles of the tile, real: without the padding
+    const int64_t step_a = TA ? (int64_t)GEMM_BK * p.lda * 2 : GEMM_BK * 2, step_b = TB ? (int64_t)GEMM_BK * p.ldb * 2 : GEMM_BK * 2;
+    auto k_of = [&](const Where &w) { return TA ? w.rows : p.K; };
+    auto pairs = [](int K) { return max(1, (K + 2 * GEMM_BK - 1) / (2 * GEMM_BK)); };
+    auto seek = [&](Cursor &c) {                  // to the first k-tile of tile c.j
+        if (!in_range(c.j)) { c.ra = c.rb = 0; c.left = c.real = 0x7fffffff; return; }
+        const Where w = locate(c.j);
+        const int K = k_of(w), M = TA ? p.M : w.rows;
+        c.a = reinterpret_cast<const uint8_t *>(p.A + w.e * p.sA + (TA ? (int64_t)w.m0 : (int64_t)w.m0 * p.lda));
+        c.b = reinterpret_cast<const uint8_t *>(p.B + w.e * p.sB + (TB ? (int64_t)w.n0 : (int64_t)w.n0 * p.ldb));
+        c.ra = TA ? ((int64_t)(K - 1) * p.lda + (M - w.m0)) * 2 : ((int64_t)(M - w.m0 - 1) * p.lda + K) * 2;
+        c.rb = TB ? ((int64_t)(K - 1) * p.ldb + (p.N - w.n0)) * 2 : ((int64_t)(p.N - w.n0 - 1) * p.ldb + K) * 2;
+        c.real = (K + GEMM_BK - 1) / GEMM_BK;
+        c.left = pairs(K) * 2;
+        if (K <= 0) c.ra = c.rb = 0;
+    };
+    auto advance = [&](Cursor &c) {
+        if (--c.left == 0) { c.j += stride; seek(c); return; }
+        c.a += step_a; c.b += step_b; c.ra -= step_a; c.rb -= step_b;
+        if (--c.real <= 0) c.ra = c.rb = 0;
+    };
+
+    // ---- which 16 bytes of a half a lane fetches.  k fast: 64 X rows of 128 bytes, a load fills eight of
+    // them, chunk c of row r lies at unit c ^ (r >> 1) & 7 (the 16 rows that one pass of a fragment read
+    // touches then lie two by two in the halves of the LDS's 256 bytes, at eight different units).  k slow:
+    // 64 rows of 128 X bytes, chunk c of row k at unit c ^ (k & 3) << 2 (128-byte rows: c ^ (k >> 1 & 1) << 2),
+    // so that the 4 rows of a transposing read's patch lie in different quarters of the 256 bytes.
+    // Load i of a half: k fast, rows 8 i on (the swizzle turns with the parity of i); k slow, rows 8 / X i on.
+    auto fetch = [&](bool T, int X, int i, int ld) -> uint32_t {
+        if (T) {
+            const int kr = 16 * wave + lane / (8 * X), u = lane % (8 * X);
+            return (uint32_t)kr * (uint32_t)ld * 2u + (uint32_t)(X == 2 ? u ^ ((kr & 3) << 2) : u ^ (((kr >> 1) & 1) << 2)) * 16u;
+        }
+        const int row = 16 * X * wave + 8 * i + (lane >> 3);
+        return (uint32_t)row * (uint32_t)ld * 2u + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    };
+    uint32_t va[2], vb[2];
+    va[0] = fetch(TA, I, 0, p.lda); va[1] = TA ? va[0] : fetch(TA, I, 1, p.lda);
+    vb[0] = fetch(TB, J, 0, p.ldb); vb[1] = TB ? vb[0] : fetch(TB, J, 1, p.ldb);
+    // a reduction length that is no multiple of 64: the chunks of a k-fast row past its end are asked for
+    // out of range in a tile's last k-tile.  Chunk of a lane in load i: (lane & 7) ^ (4 i + (lane >> 4) & 7)
+    const int k_tail = TA || p.K % GEMM_BK == 0 ? GEMM_BK : p.K % GEMM_BK;      // (tn: both operands are k-slow)
+    auto past = [&](int i) -> uint32_t {
+        return (int)(((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 8) >= k_tail ? GEMM_NOWHERE : 0u;
+    };
+    const uint32_t past0 = past(0), past1 = past(1);
+    auto load = [&](int stage, int o, int h, int i, const Cursor &c) {
+        const int X = o == 0 ? I : J;
+        const bool T = o == 0 ? TA : TB;
+        const uint32_t dst = lds0 + S::half_at(o, stage, h) + wave * (2048 * X) + i * 1024;
+        const uint32_t ld = (uint32_t)(o == 0 ? p.lda : p.ldb), first = h ? 64u * X : 0u;
+        const uint32_t soff = T ? ld * 2u * (uint32_t)(8 / X * i) + first * 2u : ld * 2u * ((uint32_t)(8 * (i & ~1)) + first);
+        uint32_t v = o == 0 ? va[i & 1] : vb[i & 1];
+        if (!T && k_tail != GEMM_BK) v |= c.real == 1 ? ((i & 1) ? past1 : past0) : 0u;
+        gemm_dma16(o == 0 ? gemm_desc(c.a, c.ra) : gemm_desc(c.b, c.rb), v, soff, dst);
+    };
+
+    // ---- fragments: 32 rows (columns) x 16 k; lane = row l % 32, k-chunk l / 32.  Where a lane's piece of the
+    // first fragment of a half lies: k fast, one place for each of the four steps (the swizzle); k slow, one
+    // for each fragment of the half
+    gemm_bf16x8 fa[2][I][4], fb[2][J][4];
+    const int fr = lane & 31, fc = lane >> 5, tg = lane >> 4, ts = lane & 15;
+    uint32_t ra[4], rb[4];
+    auto place = [&](bool T, int X, int n, int w) -> uint32_t {
+        if (T) {
+            // lane = (group of 16 lanes, s): k row 8 (g / 2) + s / 4 of the step's 16, 8 bytes s % 4 of the 32 that columns
+            // 16 (g % 2) .. + 15 of the fragment take
+            const int row = 8 * (tg >> 1) + (ts >> 2), c = 4 * X * w + 4 * n + 2 * (tg & 1) + ((ts & 3) >> 1);
+            const int u = X == 2 ? c ^ ((ts >> 2) << 2) : c ^ ((ts >> 3) << 2);
+            return row * (128 * X) + u * 16 + 8 * (ts & 1);
+        }
+        return (32 * X * w + fr) * 128 + (((2 * n + fc) ^ ((fr >> 1) & 7)) * 16);
+    };
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = 32 * j + fr;
-        const float fb = bias && n0 + wn * 128 + col < p.N ? bf16_to_f32(bias[col]) : 0.f;
+    for (int n = 0; n < (TA ? I : 4); ++n) ra[n] = lds0 + place(TA, I, n, wm);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int n = 0; n < (TB ? J : 4); ++n) rb[n] = lds0 + S::half_at(1, 0, 0) + place(TB, J, n, wn);
+    auto read = [&](int stage, int o, int h, int r) {
+        const int X = o == 0 ? I : J, ks = r / X, i = r % X;
+        const uint32_t at = (uint32_t)(S::half_at(o, stage, h) - S::half_at(o, 0, 0));
+        gemm_bf16x8 f;
+        if (o == 0 ? TA : TB) {
+            const gemm_lds_ptr q = (gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[i] : rb[i]) + at + ks * (16 * 128 * X);
+            f = gemm_read_tr(q, q + 4 * 128 * X);
+        } else {
+            f = *(const gemm_bf16x8 __attribute__((address_space(3))) *)((gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[ks] : rb[ks]) + at + i * 4096);
+        }
+        if (o == 0) fa[h][i][ks] = f; else fb[h][i][ks] = f;
+    };
+
+    f32x16 acc[2][2][I][J];
+    int fresh = 0;                                // the stores of the tile before have just gone out
+
+    // one phase: quadrant (qa, qb); read half (ro, rh) of stage rs; ask for half (lo, lh) into stage lst
+    // (the second operand first in the MFMA: a lane then holds four consecutive columns of one row)
+#define PM_PHASE(P, qa, qb, rs, ro, rh, lst, lo, lh, cur)                                                            \
+    do {                                                                                                             \
+        constexpr int n_ = 4 * I * J, half_ = n_ / 2, reads_ = 4 * ((ro) == 0 ? I : J), loads_ = S::loads(P);         \
+        constexpr int rper_ = (reads_ + half_ - 1) / half_, lper_ = (loads_ + half_ - 1) / half_;                     \
+        constexpr int lgap_ = half_ / loads_ > 0 ? half_ / loads_ : 1;                                               \
+        _Pragma("unroll") for (int s_ = 0; s_ < n_; ++s_) {                                                          \
+            const int ks_ = s_ / (I * J), i_ = s_ / J % I, j_ = s_ % J;                                              \
+            acc[qa][qb][i_][j_] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[qb][j_][ks_], fa[qa][i_][ks_], acc[qa][qb][i_][j_], 0, 0, 0); \
+            __builtin_amdgcn_sched_barrier(0);                                                                       \
+            if (s_ < half_) {                                                                                        \
+                _Pragma("unroll") for (int x_ = 0; x_ < rper_; ++x_)                                                 \
+                    if (s_ * rper_ + x_ < reads_) read(rs, ro, rh, s_ * rper_ + x_);                                 \
+                __builtin_amdgcn_sched_barrier(0);                                                                   \
+            } else if ((s_ - half_) % lgap_ == 0) {                                                                  \
+                _Pragma("unroll") for (int x_ = 0; x_ < lper_; ++x_) {                                               \
+                    const int l_ = (s_ - half_) / lgap_ * lper_ + x_;                                                \
+                    if (l_ < loads_) load(lst, lo, lh, l_, cur);                                                     \
+                }                                                                                                    \
+                __builtin_amdgcn_sched_barrier(0);                                                                   \
+            }                                                                                                        \
+        }                                                                                                            \
+        /* (until a half that was asked for behind the stores is needed, the stores need not be through) */          \
+        if ((P) < 6 && fresh) gemm_phase_wait<S::wait(P) + S::STORES>();                                             \
+        else gemm_phase_wait<S::wait(P)>();                                                                          \
+        __builtin_amdgcn_sched_barrier(0);                                                                           \
+    } while (0)
+
+    int j = blockIdx.x / 8;
+    if (!in_range(j)) return;
+    Cursor c0, c1, c2, c3;                        // k-tiles 0 .. 3 from here
+    c0.j = j;
+    seek(c0);
+    c1 = c0; advance(c1);
+    c2 = c1; advance(c2);
+    c3 = c2; advance(c3);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int row = 32 * i + 8 * (q >> 2) + 4 * fc + (q & 3);
-                float v = bf16_to_f32(f32_to_bf16(acc[i][j][q]));
-                if (bias) v = bf16_to_f32(f32_to_bf16(v + fb));
-                if (ACT == 1) v = fmaxf(v, 0.f);
-                *reinterpret_cast<uint16_t *>(quad + row * GEMM_CPITCH + col * 2) = (uint16_t)f32_to_bf16(v);
+    for (int i = 0; i < 2 * I; ++i) load(0, 0, 0, i, c0);
+#pragma unroll
+    for (int i = 0; i < 2 * J; ++i) load(0, 1, 0, i, c0);
+#pragma unroll
+    for (int i = 0; i < 2 * J; ++i) load(0, 1, 1, i, c0);
+#pragma unroll
+    for (int i = 0; i < 2 * I; ++i) load(0, 0, 1, i, c0);
+#pragma unroll
+    for (int i = 0; i < 2 * I; ++i) load(1, 0, 0, i, c1);
+#pragma unroll
+    for (int i = 0; i < 2 * J; ++i) load(1, 1, 1, i, c1);
+#pragma unroll
+    for (int i = 0; i < 2 * J; ++i) load(1, 1, 0, i, c1);
+#pragma unroll
+    for (int i = 0; i < 2 * I; ++i) load(1, 0, 1, i, c1);
+    gemm_phase_wait<6 * (I + J)>();
+#pragma unroll
+    for (int r = 0; r < 4 * I; ++r) read(0, 0, 0, r);
+#pragma unroll
+    for (int r = 0; r < 4 * J; ++r) read(0, 1, 0, r);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * I; ++i) load(0, 0, 0, i, c2);
+    gemm_phase_wait<S::wait(7)>();
+    __builtin_amdgcn_sched_barrier(0);
+
+    Where here = locate(j);
+    int left = pairs(k_of(here)), turn = 0;
+    // the tile's slice of the bias goes into LDS ahead of the tile's own loads, so it is there with them
+    auto ask_bias = [&] {
+        if (!GRAD && p.bias && !p.bias_by_value && wave == 0)
+            gemm_dma16(gemm_desc(p.bias + (int64_t)here.e * p.N + here.n0, (int64_t)(p.N - here.n0) * 2), lane * 16, 0u, lds0 + S::BIAS + turn * 1024);
+    };
+    ask_bias();
+
+    // where a lane's 16-byte pieces go, from the tile's corner; the uniform part of a piece's place is the store's scalar offset
+    const int put_col = wn * 32 * J + lane % (4 * J) * 8;
+    const uint32_t put = ((uint32_t)(wm * 32 * I + lane / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
+    auto finish = [&] {                           // the results of the tile to memory
+        uint8_t *piece = lds + S::OPERANDS + wave * (32 * S::PITCH);
+        const uint8_t *get = piece + lane / (4 * J) * S::PITCH + lane % (4 * J) * 16;
+        uint8_t *lay = piece + fr * S::PITCH + fc * 8;
+        const int M = TA ? p.M : here.rows;
+        const int64_t corner = (int64_t)here.e * p.sC + (int64_t)here.m0 * p.ldc + here.n0;
+        const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2);
+        const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t mask = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(GRAD ? p.mask + corner : p.C), 0, GRAD ? bytes : 0, 0x00020000);
+        const uint32_t put0 = here.n0 + put_col < p.N ? put : GEMM_NOWHERE, put1 = here.n0 + 64 * J + put_col < p.N ? put : GEMM_NOWHERE;
+        float add[2][8];                          // bias of the lane's columns (GRAD: their sums)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int x = 0; x < 8; ++x) add[b][x] = 0.f;
+        if (!GRAD && p.bias) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if (p.bias_by_value) {
+                    for (int x = 0; x < 8; ++x) add[b][x] = bf16_to_f32(p.bias[(int64_t)here.e * p.N + min(here.n0 + 64 * J * b + put_col + x, p.N - 1)]);
+                    continue;
+                }
+                Elem<PLANMOE_BF16>::unpack(*reinterpret_cast<const uint4 *>(lds + S::BIAS + turn * 1024 + (64 * J * b + put_col) * 2), add[b]);
             }
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int i = 0; i < I; ++i)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    auto so = [&](int t) { return ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u; };
+                    pm_u32x4 keep[2 * J];
+                    if (GRAD)
+#pragma unroll
+                        for (int t = 0; t < 2 * J; ++t) keep[t] = __builtin_amdgcn_raw_buffer_load_b128(mask, b ? put1 : put0, so(t), 0);
+#pragma unroll
+                    for (int jj = 0; jj < J; ++jj)
+                        asm volatile("" : "+a"(acc[a][b][i][jj]));      // (in the accumulator registers until here: copied all at once they would not fit)
+#pragma unroll
+                    for (int jj = 0; jj < J; ++jj)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const f32x16 &c = acc[a][b][i][jj];
+                            *reinterpret_cast<uint2 *>(lay + (32 * jj + 8 * q) * 2) =
+                                make_uint2(f32x2_to_bf16x2(c[4 * q], c[4 * q + 1]), f32x2_to_bf16x2(c[4 * q + 2], c[4 * q + 3]));
+                        }
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int t = 0; t < 2 * J; ++t) {
+                        pm_u32x4 v = *reinterpret_cast<const pm_u32x4 *>(get + t * (16 / J) * S::PITCH);
+                        if (!GRAD && p.bias) {    // the matmul's rounding is done; torch.add in bf16
+#pragma unroll
+                            for (int x = 0; x < 4; ++x)
+                                v[x] = f32x2_to_bf16x2(__uint_as_float(v[x] << 16) + add[b][2 * x], __uint_as_float(v[x] & 0xffff0000u) + add[b][2 * x + 1]);
+                        }
+                        if (!GRAD && p.relu) {    // (negative bf16 are negative int16; a NaN stays)
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                typedef short s16x2 __attribute__((ext_vector_type(2)));
+                                v[x] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, (uint32_t)v[x]), (s16x2)(short)0));
+                            }
+                        }
+                        if (GRAD) {               // relu's backward: kept where its output was positive
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                const uint32_t k = keep[t][x];
+                                v[x] &= ((int)(k << 16) > 0 ? 0xffffu : 0u) | ((int)k >= 0x10000 ? 0xffff0000u : 0u);
+                                add[b][2 * x] += __uint_as_float(v[x] << 16);
+                                add[b][2 * x + 1] += __uint_as_float(v[x] & 0xffff0000u);
+                            }
+                        }
+                        __builtin_amdgcn_raw_buffer_store_b128(v, out, b ? put1 : put0, so(t), 0);
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        if (GRAD && p.colsum) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int x = 0; x < 8; ++x)
+#pragma unroll
+                    for (int d = 4 * J; d < 64; d <<= 1) add[b][x] += __shfl_xor(add[b][x], d);
+                if (lane < 4 * J && here.n0 + 64 * J * b + put_col < p.N) {
+                    const int slots = (p.M + S::BM - 1) / S::BM * 2;
+                    float *to = p.colsum + ((int64_t)here.e * slots + here.m0 / S::BM * 2 + wm) * p.N + here.n0 + 64 * J * b + put_col;
+#pragma unroll
+                    for (int x = 0; x < 8; x += 4) *reinterpret_cast<float4 *>(to + x) = make_float4(add[b][x], add[b][x + 1], add[b][x + 2], add[b][x + 3]);
+                }
+            }
+        }
+    };
+
+    while (true) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < I; ++i)
+#pragma unroll
+                    for (int jj = 0; jj < J; ++jj)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) acc[a][b][i][jj][q] = 0.f;
+        do {
+            PM_PHASE(0, 0, 0, 0, 1, 1, 0, 1, 0, c2);
+            PM_PHASE(1, 0, 1, 0, 0, 1, 0, 1, 1, c2);
+            PM_PHASE(2, 1, 1, 1, 0, 0, 0, 0, 1, c2);
+            PM_PHASE(3, 1, 0, 1, 1, 1, 1, 0, 0, c3);
+            c2 = c3; advance(c3);
+            PM_PHASE(4, 0, 1, 1, 1, 0, 1, 1, 1, c2);
+            PM_PHASE(5, 0, 0, 1, 0, 1, 1, 1, 0, c2);
+            PM_PHASE(6, 1, 0, 0, 0, 0, 1, 0, 1, c2);
+            PM_PHASE(7, 1, 1, 0, 1, 0, 0, 0, 0, c3);
+            c2 = c3; advance(c3);
+            fresh = 0;
+        } while (--left);
+        finish();
+        fresh = 1;
+        j += stride;
+        if (!in_range(j)) break;
+        here = locate(j);
+        left = pairs(k_of(here));
+        turn ^= 1;
+        ask_bias();
     }
-    __builtin_amdgcn_wave_barrier();
-    uint16_t *C = p.C + (int64_t)e * p.sC;
-#pragma unroll 4
-    for (int t = 0; t < 32; ++t) {
-        const int q = lane + 64 * t, row = q >> 4, c = q & 15;
-        const int gr = m0 + wm * 128 + row, gc = n0 + wn * 128 + c * 8;
-        if (gr < p.M && gc < p.N)
-            *reinterpret_cast<uint4 *>(C + (int64_t)gr * p.ldc + gc) = *reinterpret_cast<const uint4 *>(quad + row * GEMM_CPITCH + c * 16);
+    // nothing may still be on its way into LDS that another work-group gets
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#undef PM_PHASE
+}
+
+// the column sums of the tiles of a batch, in tile order, as the bias gradient
+__global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restrict__ parts, const int *__restrict__ live, int live_planes,
+                                                          int live_round, int batches, int M, int N, int BM, uint16_t *__restrict__ out)
+{
+    const int e = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x, slots = (M + BM - 1) / BM * 2;
+    int rows = M;
+    if (live) {
+        int c = 0;
+        for (int j = 0; j < live_planes; ++j) c += live[j * batches + e];
+        rows = min(M, (c + live_round - 1) / live_round * live_round);
     }
+    if (n >= N) return;
+    const int used = (rows + BM - 1) / BM * 2;
+    const float *from = parts + (int64_t)e * slots * N + n;
+    float s = 0.f;
+    for (int i = 0; i < used; ++i) s += from[(int64_t)i * N];
+    out[(int64_t)e * N + n] = (uint16_t)f32_to_bf16(s);
 }
 
 // out[e][c][r] = in[e][r][c] for r < rows, zero for rows <= r < rows_out (the padding of a k dimension):
@@ -427,6 +542,72 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t *__r
 
 using namespace pm;
 
+namespace {
+
+int compute_units()
+{
+    static int known[64];                        // (written once per device, with the same value by whoever is first)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev < 64 && known[dev]) return known[dev];
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
+    if (dev < 64) known[dev] = n;
+    return n;
+}
+
+template <int I, int J, bool TA, bool TB, bool GRAD>
+int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
+{
+    using S = GemmShape<I, J>;
+    const auto kernel = gemm_bf16_kernel<I, J, TA, TB, GRAD>;
+    static bool ready[64];                       // (per device; setting the attribute twice does no harm)
+    int dev = 0;
+    PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
+    if (dev >= 64 || !ready[dev]) {
+        PM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS) == hipSuccess,
+                   "%s: the kernel needs %d bytes of LDS", who, S::LDS);
+        if (dev < 64) ready[dev] = true;
+    }
+    const int64_t tiles = ((int64_t)p.M + S::BM - 1) / S::BM * (((int64_t)p.N + S::BN - 1) / S::BN) * p.batches;
+    PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
+    const int64_t stay = (int64_t)compute_units() * S::WAVES_PER_SIMD / 8 * 8;
+    kernel<<<dim3((unsigned)(tiles + 7 < stay ? (tiles + 7) / 8 * 8 : stay)), GEMM_WG, S::LDS, stream>>>(p);
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+// Which tile: 256 x 256 moves the fewest operand bytes per product, 128 x 128 (two work-groups per compute
+// unit) leaves fewer compute units idle where there are few tiles and loses less in a last round that is
+// not full.  A launch takes its rounds; a round takes its k-tiles and what a tile costs once (start,
+// results).  Microseconds, fitted to 22 shapes from 8 x 4 x 4096 x 1024 to 8 x 4928 x 4096 x 1024 (within 10 % there):
+// a k-tile of 256 x 256 takes 1.0 us with few compute units at work and 1.3 with all of them (the clock sinks
+// under the matrix cores), one of 128 x 128 takes 0.45 alone on its compute unit and 0.8 for two at a time.
+// Example: 8 x 512 x 2048 x 2048 takes 37 us in the small tiles and 49 in the large, 8 x 1024 x 2048 x 2048 69 and 59.
+bool gemm_wants_small(int batches, int64_t rows, int64_t cols, int64_t k)
+{
+    const int64_t cu = compute_units();
+    const int64_t big = (rows + 255) / 256 * ((cols + 255) / 256) * batches, small = (rows + 127) / 128 * ((cols + 127) / 128) * batches;
+    const double kt = (double)(k + 63) / 64;
+    const int64_t rest_b = big % cu, rest_s = small % (2 * cu);
+    const double t_big = (double)(big / cu) * (1.3 * kt + 10) + (rest_b ? (1.0 + 0.3 * (double)rest_b / (double)cu) * kt + 10 : 0.);
+    const double t_small = (double)(small / (2 * cu)) * (0.8 * kt + 5) + (rest_s == 0 ? 0. : rest_s <= cu ? 0.45 * kt + 5 : 0.8 * kt + 5);
+    return t_small < t_big;
+}
+
+template <bool TA, bool TB, bool GRAD>
+int gemm_run(const GemmArgs &p, int64_t rows_hint, hipStream_t stream, const char *who, int *tile_rows = nullptr)
+{
+    const int64_t side = TA ? p.M : rows_hint;
+    const bool small = gemm_wants_small(p.batches, side, p.N, TA ? rows_hint : p.K);
+    if (tile_rows) *tile_rows = small ? 128 : 256;
+    return small ? gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who) : gemm_launch<2, 2, TA, TB, GRAD>(p, stream, who);
+}
+
+// what the buffer descriptors cover: from a tile's corner, a tile of a k-fast operand and 64 rows of a k-slow one
+bool gemm_pitch_fits(int ld) { return (int64_t)ld * 2 * 256 < ((int64_t)1 << 31); }
+
+}  // namespace
+
 extern "C" int planmoe_gemm_nt_bf16(const void *a, const void *b, const void *bias, int activation, int batches,
                                     int m, int n, int k, int lda, int ldb, int ldc, int64_t batch_stride_a,
                                     int64_t batch_stride_b, int64_t batch_stride_c, void *c, void *stream)
@@ -439,33 +620,10 @@ extern "C" int planmoe_gemm_nt_bf16(const void *a, const void *b, const void *bi
                "planmoe_gemm_nt_bf16: k, n and the row pitches must be multiples of 8 (16-byte pieces); pitches cover their rows");
     PM_REQUIRE(batch_stride_a % 8 == 0 && batch_stride_b % 8 == 0 && batch_stride_c % 8 == 0 && aligned16(a) && aligned16(b) && aligned16(c),
                "planmoe_gemm_nt_bf16: operands must be 16-byte aligned");
-    const int64_t tm = ((int64_t)m + GEMM_BM - 1) / GEMM_BM, tn = ((int64_t)n + GEMM_BN - 1) / GEMM_BN;
-    PM_REQUIRE(tm <= 65535 && batches <= 65535, "planmoe_gemm_nt_bf16: too many row tiles or batches");
-    PM_REQUIRE((int64_t)m * lda * 2 < ((int64_t)1 << 32) && (int64_t)n * ldb * 2 < ((int64_t)1 << 32),
-               "planmoe_gemm_nt_bf16: an operand of one batch must stay under 4 GiB");
-    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, (uint16_t *)c, m, n, k, lda, ldb, ldc,
-               batch_stride_a, batch_stride_b, batch_stride_c, (int64_t)n, batches};
-    const void *fn = activation == 0 ? (const void *)gemm_nt_bf16_kernel<0> : (const void *)gemm_nt_bf16_kernel<1>;
-    PM_REQUIRE(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) == hipSuccess,
-               "planmoe_gemm_nt_bf16: the kernel needs %d bytes of LDS", GEMM_LDS);
-    const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)batches);
-    if (k % DMA_BK == 0) {
-        // operands straight into LDS, loads three k-tiles ahead
-        const void *fd = activation == 0 ? (const void *)gemm_nt_bf16_dma_kernel<0> : (const void *)gemm_nt_bf16_dma_kernel<1>;
-        PM_REQUIRE(hipFuncSetAttribute(fd, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) == hipSuccess,
-                   "planmoe_gemm_nt_bf16: the kernel needs %d bytes of LDS", GEMM_LDS);
-        const int64_t per_xcd = (tm * tn * batches + 7) / 8;
-        PM_REQUIRE(per_xcd * 8 < ((int64_t)1 << 31), "planmoe_gemm_nt_bf16: too many tiles");
-        const dim3 tiles((unsigned)(per_xcd * 8));
-        if (activation == 0) gemm_nt_bf16_dma_kernel<0><<<tiles, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-        else gemm_nt_bf16_dma_kernel<1><<<tiles, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-        PM_LAUNCH_CHECK("planmoe_gemm_nt_bf16");
-        return 0;
-    }
-    if (activation == 0) gemm_nt_bf16_kernel<0><<<grid, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-    else gemm_nt_bf16_kernel<1><<<grid, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-    PM_LAUNCH_CHECK("planmoe_gemm_nt_bf16");
-    return 0;
+    PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_nt_bf16: 256 rows of an operand must stay under 2 GiB");
+    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, !aligned16(bias)};
+    return gemm_run<false, false, false>(p, m, (hipStream_t)stream, "planmoe_gemm_nt_bf16");
 }
 
 extern "C" int planmoe_gemm_nn_bf16(const void *a, const void *b, const void *bias, int activation, int batches,
@@ -476,27 +634,15 @@ extern "C" int planmoe_gemm_nn_bf16(const void *a, const void *b, const void *bi
     if (batches == 0 || m == 0 || n == 0) return 0;
     PM_REQUIRE(a && b && c, "planmoe_gemm_nn_bf16: NULL argument");
     PM_REQUIRE(activation == 0 || activation == 1, "planmoe_gemm_nn_bf16: activation is 0 (none) or 1 (relu)");
-    PM_REQUIRE(k % DMA_BK == 0, "planmoe_gemm_nn_bf16: k must be a multiple of %d", DMA_BK);
+    PM_REQUIRE(k % GEMM_BK == 0, "planmoe_gemm_nn_bf16: k must be a multiple of %d", GEMM_BK);
     PM_REQUIRE(n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 8 == 0 && lda >= k && ldb >= n && ldc >= n,
                "planmoe_gemm_nn_bf16: n and the row pitches must be multiples of 8 (16-byte pieces); pitches cover their rows");
     PM_REQUIRE(batch_stride_a % 8 == 0 && batch_stride_b % 8 == 0 && batch_stride_c % 8 == 0 && aligned16(a) && aligned16(b) && aligned16(c),
                "planmoe_gemm_nn_bf16: operands must be 16-byte aligned");
-    PM_REQUIRE((int64_t)m * lda * 2 < ((int64_t)1 << 32) && (int64_t)DMA_BK * ldb * 2 < ((int64_t)1 << 31),
-               "planmoe_gemm_nn_bf16: the first operand of one batch must stay under 4 GiB, 64 rows of the second under 2 GiB");
-    const int64_t tm = ((int64_t)m + GEMM_BM - 1) / GEMM_BM, tn = ((int64_t)n + GEMM_BN - 1) / GEMM_BN;
-    const int64_t per_xcd = (tm * tn * batches + 7) / 8;
-    PM_REQUIRE(per_xcd * 8 < ((int64_t)1 << 31), "planmoe_gemm_nn_bf16: too many tiles");
-    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, (uint16_t *)c, m, n, k, lda, ldb, ldc,
-               batch_stride_a, batch_stride_b, batch_stride_c, (int64_t)n, batches};
-    const void *fd = activation == 0 ? (const void *)gemm_nt_bf16_dma_kernel<0, false, true>
-                                     : (const void *)gemm_nt_bf16_dma_kernel<1, false, true>;
-    PM_REQUIRE(hipFuncSetAttribute(fd, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) == hipSuccess,
-               "planmoe_gemm_nn_bf16: the kernel needs %d bytes of LDS", GEMM_LDS);
-    const dim3 tiles((unsigned)(per_xcd * 8));
-    if (activation == 0) gemm_nt_bf16_dma_kernel<0, false, true><<<tiles, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-    else gemm_nt_bf16_dma_kernel<1, false, true><<<tiles, 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-    PM_LAUNCH_CHECK("planmoe_gemm_nn_bf16");
-    return 0;
+    PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_nn_bf16: 256 rows of an operand must stay under 2 GiB");
+    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, !aligned16(bias)};
+    return gemm_run<false, true, false>(p, m, (hipStream_t)stream, "planmoe_gemm_nn_bf16");
 }
 
 extern "C" int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, int m, int n, int k, int lda, int ldb,
@@ -506,24 +652,15 @@ extern "C" int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, i
     PM_REQUIRE(batches >= 0 && m >= 0 && n >= 0 && k >= 64, "planmoe_gemm_tn_bf16: bad shape");
     if (batches == 0 || m == 0 || n == 0) return 0;
     PM_REQUIRE(a && b && c, "planmoe_gemm_tn_bf16: NULL argument");
-    PM_REQUIRE(k % DMA_BK == 0, "planmoe_gemm_tn_bf16: k must be a multiple of %d", DMA_BK);
+    PM_REQUIRE(k % GEMM_BK == 0, "planmoe_gemm_tn_bf16: k must be a multiple of %d", GEMM_BK);
     PM_REQUIRE(m % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 8 == 0 && lda >= m && ldb >= n && ldc >= n,
                "planmoe_gemm_tn_bf16: m, n and the row pitches must be multiples of 8 (16-byte pieces); pitches cover their rows");
     PM_REQUIRE(batch_stride_a % 8 == 0 && batch_stride_b % 8 == 0 && batch_stride_c % 8 == 0 && aligned16(a) && aligned16(b) && aligned16(c),
                "planmoe_gemm_tn_bf16: operands must be 16-byte aligned");
-    PM_REQUIRE((int64_t)DMA_BK * lda * 2 < ((int64_t)1 << 31) && (int64_t)DMA_BK * ldb * 2 < ((int64_t)1 << 31),
-               "planmoe_gemm_tn_bf16: 64 rows of an operand must stay under 2 GiB");
-    const int64_t tm = ((int64_t)m + GEMM_BM - 1) / GEMM_BM, tn = ((int64_t)n + GEMM_BN - 1) / GEMM_BN;
-    const int64_t per_xcd = (tm * tn * batches + 7) / 8;
-    PM_REQUIRE(per_xcd * 8 < ((int64_t)1 << 31), "planmoe_gemm_tn_bf16: too many tiles");
-    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (uint16_t *)c, m, n, k, lda, ldb, ldc,
-               batch_stride_a, batch_stride_b, batch_stride_c, 0, batches};
-    const void *fd = (const void *)gemm_nt_bf16_dma_kernel<0, true, true>;
-    PM_REQUIRE(hipFuncSetAttribute(fd, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) == hipSuccess,
-               "planmoe_gemm_tn_bf16: the kernel needs %d bytes of LDS", GEMM_LDS);
-    gemm_nt_bf16_dma_kernel<0, true, true><<<dim3((unsigned)(per_xcd * 8)), 256, GEMM_LDS, (hipStream_t)stream>>>(p);
-    PM_LAUNCH_CHECK("planmoe_gemm_tn_bf16");
-    return 0;
+    PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_tn_bf16: 256 rows of an operand must stay under 2 GiB");
+    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, 0, false};
+    return gemm_run<true, true, false>(p, k, (hipStream_t)stream, "planmoe_gemm_tn_bf16");
 }
 
 extern "C" int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int rows_out, void *out, void *stream)
