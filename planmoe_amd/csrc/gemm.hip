@@ -11,7 +11,7 @@
 //   backward  dx = dy @ W^T        A = dy [rows, out],  B = W  [in, out]      planmoe_gemm_nt_bf16
 //             dW = x^T @ dy        A = x  [rows, in],   B = dy [rows, out]    planmoe_gemm_tn_bf16
 // all with the operands as they lie in memory.
-#include "common.hpp"
+#include "gemm_f32.hpp"
 
 namespace pm {
 
@@ -490,8 +490,9 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 }
 
 // the column sums of the tiles of a batch, in tile order, as the bias gradient
+template <int DT>
 __global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restrict__ parts, const int *__restrict__ live, int live_planes,
-                                                          int live_round, int batches, int M, int N, int BM, uint16_t *__restrict__ out)
+                                                          int live_round, int batches, int M, int N, int BM, void *__restrict__ out)
 {
     const int e = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x, slots = (M + BM - 1) / BM * 2;
     int rows = M;
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restric
     const float *from = parts + (int64_t)e * slots * N + n;
     float s = 0.f;
     for (int i = 0; i < used; ++i) s += from[(int64_t)i * N];
-    out[(int64_t)e * N + n] = (uint16_t)f32_to_bf16(s);
+    Elem<DT>::store(out, (int64_t)e * N + n, s);
 }
 
 // out[e][c][r] = in[e][r][c] for r < rows, zero for rows <= r < rows_out (the padding of a k dimension):
@@ -661,6 +662,81 @@ extern "C" int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, i
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
                lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, 0, false};
     return gemm_run<true, true, false>(p, k, (hipStream_t)stream, "planmoe_gemm_tn_bf16");
+}
+
+// ---------------------------------------------------------------- the experts' products on contiguous buffers
+static int expert_gemm_check(const char *who, int form, int dtype, const void *a, const void *b, int batches, int m, int n, int k,
+                             const int32_t *live, int live_planes, int live_round, const void *c)
+{
+    PM_REQUIRE(form >= 0 && form <= 2, "%s: form is 0 (a b), 1 (a b^T) or 2 (a^T b)", who);
+    PM_REQUIRE(dtype == PLANMOE_BF16 || dtype == PLANMOE_F32, "%s: bf16 or fp32", who);
+    PM_REQUIRE(batches >= 1 && m >= 1 && n >= 1 && k >= 1, "%s: bad shape", who);
+    PM_REQUIRE(a && b && c && aligned16(a) && aligned16(b) && aligned16(c), "%s: NULL or unaligned operand", who);
+    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
+    // (what is read and stored in 16-byte pieces: the fast index of every operand and of the result)
+    PM_REQUIRE(n % vec == 0 && (form == 2 ? m : k) % vec == 0, "%s: the fast index of every operand must be a multiple of %d", who, vec);
+    PM_REQUIRE(!live || (batches <= 64 && live_planes >= 1 && live_round >= 1), "%s: row counts for up to 64 batches", who);
+    const int widest = n > k ? (n > m ? n : m) : (k > m ? k : m);
+    PM_REQUIRE((int64_t)widest * 2 * 256 * (dtype == PLANMOE_F32 ? 2 : 1) < ((int64_t)1 << 31), "%s: 256 rows of an operand must stay under 2 GiB", who);
+    return 0;
+}
+
+extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const void *b, const void *bias, int activation,
+                                   int batches, int m, int n, int k, const int32_t *live, int live_planes, int live_round,
+                                   int rows_hint, void *c, void *stream)
+{
+    const char *who = "planmoe_expert_gemm";
+    if (expert_gemm_check(who, form, dtype, a, b, batches, m, n, k, live, live_planes, live_round, c)) return 1;
+    PM_REQUIRE(activation == 0 || activation == 1, "%s: activation is 0 (none) or 1 (relu)", who);
+    PM_REQUIRE(!bias || form != 2, "%s: a weight gradient has no bias", who);
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == PLANMOE_F32) {
+        Gemm32Args p{(const float *)a, (const float *)b, (const float *)bias, nullptr, (float *)c, nullptr, live, live_planes, live_round,
+                     m, n, k, batches, activation};
+        return gemm_f32_run(form, p, st, who);
+    }
+    const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n, most = form == 2 ? k : m;
+    GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, live, live_planes,
+               live_round, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, activation, !aligned16(bias)};
+    const int64_t hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
+    if (form == 0) return gemm_run<false, true, false>(p, hint, st, who);
+    if (form == 1) return gemm_run<false, false, false>(p, hint, st, who);
+    return gemm_run<true, true, false>(p, hint, st, who);
+}
+
+extern "C" size_t planmoe_expert_gemm_relu_bwd_workspace_bytes(int batches, int m, int n)
+{
+    if (batches < 1 || m < 1 || n < 1) return 16;
+    return (size_t)batches * 2 * ((m + 127) / 128) * n * 4;
+}
+
+extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void *b, const void *h, int batches, int m, int n,
+                                            int k, const int32_t *live, int live_planes, int live_round, int rows_hint, void *c,
+                                            void *dbias, void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_expert_gemm_relu_bwd";
+    if (expert_gemm_check(who, 1, dtype, a, b, batches, m, n, k, live, live_planes, live_round, c)) return 1;
+    PM_REQUIRE(h && aligned16(h), "%s: NULL or unaligned activations", who);
+    PM_REQUIRE(!dbias || (workspace && aligned16(workspace) && workspace_bytes >= planmoe_expert_gemm_relu_bwd_workspace_bytes(batches, m, n)), "%s: workspace too small", who);
+    PM_REQUIRE(batches <= 65535, "%s: too many batches", who);
+    hipStream_t st = (hipStream_t)stream;
+    float *parts = dbias ? (float *)workspace : nullptr;
+    int tile_rows = G32_B;
+    if (dtype == PLANMOE_F32) {
+        Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
+        if (gemm_f32_run(1, p, st, who)) return 1;
+    } else {
+        GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
+                   m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, false};
+        if (gemm_run<false, false, true>(p, rows_hint >= 1 && rows_hint < m ? rows_hint : m, st, who, &tile_rows)) return 1;
+    }
+    if (dbias) {
+        const dim3 grid((unsigned)((n + 255) / 256), (unsigned)batches);
+        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, dbias);
+        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, dbias);
+        PM_LAUNCH_CHECK(who);
+    }
+    return 0;
 }
 
 extern "C" int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int rows_out, void *out, void *stream)

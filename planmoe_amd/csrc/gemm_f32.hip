@@ -1,0 +1,223 @@
+// Batched fp32 GEMM of the expert FFN (experts/ffn.py:63-82 and its backward pass) on gfx950's fp32 matrix
+// cores (v_mfma_f32_32x32x2_f32: fp32 products and sums, 157 TFLOP/s):
+//   C[e][m][n] = act( sum_k A[e][m][k] * B[e][n][k] + bias[e][n] )
+// with either operand stored k fast or k slow, as planmoe_gemm_*_bf16.
+//
+// A 32 x 32 x 2 MFMA takes 64 clocks, so unlike bf16 nothing here is bound by operand traffic: a 128 x 128
+// tile reads 32 KB per k-tile of 32 for 4096 clocks of matrix core.  Four waves of 64 x 64, operands straight
+// into LDS (buffer_load ... lds), the next k-tile in flight during the MFMAs of this one, two work-groups
+// per compute unit so that one's barrier and epilogue fall under the other's MFMAs.  A k-fast operand is
+// read four k at a time (16 bytes per lane); which k a lane holds does not matter to the sum as long as
+// both operands agree, so step q of eight k takes k = q from lanes 0 .. 31 and k = 4 + q from lanes 32 .. 63.
+#include "gemm_f32.hpp"
+
+namespace pm {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t g32_u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int G32_BK = 32;
+constexpr int G32_OPERAND = G32_B * G32_BK * 4;             // one operand's k-tile in LDS
+constexpr int G32_LDS = 4 * G32_OPERAND;                    // A0 A1 B0 B1
+
+__device__ __forceinline__ g32_u32x4 g32_desc(const void *base, int64_t bytes)
+{
+    const uint64_t a = (uint64_t)base;
+    const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffff ? 0x7fffffffu : (uint32_t)bytes;
+    return g32_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, n, 0x00020000u};
+}
+__device__ __forceinline__ void g32_dma16(g32_u32x4 desc, uint32_t voff, uint32_t soff, uint32_t lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
+{
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+
+    // XCD j (work-groups j, j + 8, ...) takes the j-th eighth of the tiles: batch, panel of 8 columns, row, column
+    const int tiles_m = (p.M + G32_B - 1) / G32_B, tiles_n = (p.N + G32_B - 1) / G32_B;
+    const int total = tiles_m * tiles_n * p.batches, per_xcd = (total + 7) / 8;
+    const int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per_xcd || tile >= total) return;
+    const int e = tile / (tiles_m * tiles_n);
+    int in = tile - e * tiles_m * tiles_n;
+    const int panel = in / (tiles_m * 8);
+    in -= panel * tiles_m * 8;
+    const int width = min(8, tiles_n - panel * 8);
+    const int m0 = in / width * G32_B, n0 = (panel * 8 + in % width) * G32_B;
+    int M = p.M, K = p.K;
+    if (p.live) {
+        int n = 0;
+        for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
+        n = (n + p.live_round - 1) / p.live_round * p.live_round;
+        if (TA) K = min(K, n); else M = min(M, n);
+    }
+    if (m0 >= M) return;
+
+    const int lda = TA ? p.M : p.K, ldb = TB ? p.N : p.K;
+    const uint8_t *A = reinterpret_cast<const uint8_t *>(p.A + (int64_t)e * p.M * p.K + (TA ? (int64_t)m0 : (int64_t)m0 * lda));
+    const uint8_t *B = reinterpret_cast<const uint8_t *>(p.B + (int64_t)e * p.N * p.K + (TB ? (int64_t)n0 : (int64_t)n0 * ldb));
+    const int64_t ra = TA ? ((int64_t)(K - 1) * lda + (p.M - m0)) * 4 : ((int64_t)(M - m0 - 1) * lda + p.K) * 4;
+    const int64_t rb = TB ? ((int64_t)(K - 1) * ldb + (p.N - n0)) * 4 : ((int64_t)(p.N - n0 - 1) * ldb + p.K) * 4;
+    const int64_t step_a = TA ? (int64_t)G32_BK * lda * 4 : G32_BK * 4, step_b = TB ? (int64_t)G32_BK * ldb * 4 : G32_BK * 4;
+    const int KT = (K + G32_BK - 1) / G32_BK, k_tail = K % G32_BK ? K % G32_BK : G32_BK;
+
+    // k fast: 128 rows of 128 bytes, a load fills eight, chunk c of row r at unit c ^ (r >> 1) & 7.
+    // k slow: 32 rows of 512 bytes, a load fills two.
+    auto fetch = [&](bool T, int i, int ld) -> uint32_t {
+        if (T) return (uint32_t)(8 * wave + (lane >> 5)) * (uint32_t)ld * 4u + (uint32_t)(lane & 31) * 16u;
+        const int row = 32 * wave + 8 * i + (lane >> 3);
+        return (uint32_t)row * (uint32_t)ld * 4u + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    };
+    const uint32_t va[2] = {fetch(TA, 0, lda), fetch(TA, TA ? 0 : 1, lda)}, vb[2] = {fetch(TB, 0, ldb), fetch(TB, TB ? 0 : 1, ldb)};
+    // (chunks of a k-fast row past the end of K are asked for out of range)
+    auto past = [&](int i) -> uint32_t { return (int)(((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 4) >= k_tail ? 0x80000000u : 0u; };
+    const uint32_t past0 = past(0), past1 = past(1);
+    auto load_tile = [&](int kt) {
+        if (kt >= KT) return;
+        const g32_u32x4 da = g32_desc(A + kt * step_a, ra - kt * step_a), db = g32_desc(B + kt * step_b, rb - kt * step_b);
+        const uint32_t sa = lds0 + (kt & 1) * G32_OPERAND + wave * 4096, sb = sa + 2 * G32_OPERAND;
+        const bool last = kt == KT - 1 && k_tail != G32_BK;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            g32_dma16(da, va[i & 1] | (!TA && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)lda * 4u * (TA ? 2 * i : 8 * (i & ~1)), sa + i * 1024);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            g32_dma16(db, vb[i & 1] | (!TB && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)ldb * 4u * (TB ? 2 * i : 8 * (i & ~1)), sb + i * 1024);
+    };
+
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+    const int fr = lane & 31, fc = lane >> 5;
+    // eight k of a side's two 32-row fragments: element q of fragment i
+    auto read8 = [&](bool T, const uint8_t *base, int w, int s, f32x4 (&f)[2]) {
+        if (T) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    f[i][q] = *reinterpret_cast<const float *>(base + (8 * s + 4 * fc + q) * 512 + (64 * w + 32 * i + fr) * 4);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                f[i] = *reinterpret_cast<const f32x4 *>(base + (64 * w + 32 * i + fr) * 128 + (((2 * s + fc) ^ ((fr >> 1) & 7)) * 16));
+        }
+    };
+
+    load_tile(0);
+    for (int kt = 0; kt < KT; ++kt) {
+        // this wave's share of k-tile kt is in; behind the barrier everybody's is, and everybody is done with kt - 1
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        load_tile(kt + 1);
+        const uint8_t *a = lds + (kt & 1) * G32_OPERAND, *b = a + 2 * G32_OPERAND;
+        f32x4 fa[2][2], fb[2][2];
+        read8(TA, a, wm, 0, fa[0]);
+        read8(TB, b, wn, 0, fb[0]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (s < 3) { read8(TA, a, wm, s + 1, fa[(s + 1) & 1]); read8(TB, b, wn, s + 1, fb[(s + 1) & 1]); }
+            // (the second operand first: a lane then holds four consecutive columns of one row)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[s & 1][j][q], fa[s & 1][i][q], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    const int64_t corner = (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0;
+    const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - m0 - 1) * p.N + (p.N - n0)) * 4);
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
+    float sums[2][4][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int col = wn * 64 + 32 * j + 8 * q + 4 * fc;
+            const bool in_n = n0 + col < p.N;
+            f32x4 add = {0.f, 0.f, 0.f, 0.f};
+            if (p.bias && in_n) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) add[x] = p.bias[(int64_t)e * p.N + n0 + col + x];
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x) sums[j][q][x] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = wm * 64 + 32 * i + fr;
+                f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                if (p.bias) v += add;
+                if (p.relu) {
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = v[x] < 0.f ? 0.f : v[x];
+                }
+                const bool inside = in_n && m0 + row < M;
+                if (p.mask) {
+                    f32x4 k = {0.f, 0.f, 0.f, 0.f};
+                    if (inside) k = *reinterpret_cast<const f32x4 *>(p.mask + corner + (int64_t)row * p.N + col);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) { v[x] = k[x] > 0.f ? v[x] : 0.f; sums[j][q][x] += inside ? v[x] : 0.f; }
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(pm_u32x4, v), out, in_n ? ((uint32_t)row * (uint32_t)p.N + (uint32_t)col) * 4u : 0x80000000u, 0, 0);
+            }
+        }
+    if (p.colsum) {
+        const int slots = tiles_m * 2;
+        float *to = p.colsum + ((int64_t)e * slots + m0 / G32_B * 2 + wm) * p.N + n0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+#pragma unroll
+                    for (int d = 1; d < 32; d <<= 1) sums[j][q][x] += __shfl_xor(sums[j][q][x], d);
+                const int col = wn * 64 + 32 * j + 8 * q + 4 * fc;
+                if (fr == 0 && n0 + col < p.N) *reinterpret_cast<float4 *>(to + col) = make_float4(sums[j][q][0], sums[j][q][1], sums[j][q][2], sums[j][q][3]);
+            }
+    }
+}
+
+template <bool TA, bool TB>
+static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
+{
+    const auto kernel = gemm_f32_kernel<TA, TB>;
+    static bool ready[64];                       // (per device; setting the attribute twice does no harm)
+    int dev = 0;
+    PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
+    if (dev >= 64 || !ready[dev]) {
+        PM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G32_LDS) == hipSuccess,
+                   "%s: the kernel needs %d bytes of LDS", who, G32_LDS);
+        if (dev < 64) ready[dev] = true;
+    }
+    const int64_t tiles = ((int64_t)p.M + G32_B - 1) / G32_B * (((int64_t)p.N + G32_B - 1) / G32_B) * p.batches;
+    PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
+    kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, G32_LDS, stream>>>(p);
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+int gemm_f32_run(int form, const Gemm32Args &p, hipStream_t stream, const char *who)
+{
+    PM_REQUIRE((int64_t)p.K * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.M * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.N * 4 * 128 < ((int64_t)1 << 31),
+               "%s: 128 rows of an operand must stay under 2 GiB", who);
+    if (form == 0) return gemm_f32_launch<false, true>(p, stream, who);
+    if (form == 1) return gemm_f32_launch<false, false>(p, stream, who);
+    return gemm_f32_launch<true, true>(p, stream, who);
+}
+
+} // namespace pm

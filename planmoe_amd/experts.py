@@ -1,52 +1,30 @@
 """Fused expert FFN -- mirror of the reference's experts/ffn.py (two batched GEMMs with bias and
-activation between dispatch and combine).  On the GPU in bf16 both GEMMs, and the four of their
-backward pass, are planmoe_gemm_nt_bf16 / _nn_ / _tn_ (one hand-written kernel for the matrix cores
-that reads either operand either way round; no library GEMM is called at the layer's sizes); forward_from_codes() takes the int8 codes of the receive buffer
-straight into the first GEMM."""
+activation between dispatch and combine).  On the GPU in bf16 and fp32 both GEMMs, and the four of their
+backward pass, are planmoe_expert_gemm (hand-written kernels for the matrix cores that read either operand
+either way round; no library GEMM is called); forward_from_codes() takes the int8 codes of the receive
+buffer straight into the first GEMM."""
 import torch
 
 
 def _kernel_serves(x, w):
-    """planmoe_gemm_nt_bf16 takes bf16 operands on the GPU whose row lengths are multiples of 8."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 3 and
-            w.shape[1] % 8 == 0 and w.shape[2] % 8 == 0 and x.shape[0] == w.shape[0] and x.shape[2] == w.shape[1])
-
-
-class _WeightForms:
-    """The [E, out, in] copy of a weight stored [E, in, out] (what the forward GEMM wants as its second
-    operand), made again only when the weight has changed (in-place updates bump ._version, a .data
-    swap changes the pointer)."""
-
-    def __init__(self):
-        self.key, self.value = None, None
-
-    def k_major(self, w):
-        from . import ops
-        key = (w._version, w.data_ptr(), w.device, w.dtype, tuple(w.shape))
-        if self.key != key:
-            self.value = ops.transpose_bf16(w.detach())
-            self.key = key
-        return self.value
+    """planmoe_expert_gemm takes bf16 / fp32 operands on the GPU whose row lengths are whole 16-byte pieces."""
+    vec = 8 if x.dtype == torch.bfloat16 else 4
+    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and x.dim() == 3 and x.numel() > 0 and
+            w.shape[1] % vec == 0 and w.shape[2] % vec == 0 and x.shape[0] == w.shape[0] and x.shape[2] == w.shape[1] and
+            not torch.is_autocast_enabled(x.device.type))
 
 
 class _BatchedLinear(torch.autograd.Function):
     """y = act(x @ w + bias) over experts: x [E, R, in], w [E, in, out] (as the reference stores it),
     bias [E, out], act = relu or nothing; torch.add(torch.matmul(x, w), bias.unsqueeze(1)) of
-    experts/ffn.py:77-79 with its two bf16 roundings.  All three products read their operands as they
-    lie in memory when the reduction length is a multiple of 64 (planmoe_gemm_nn_bf16 for y,
-    planmoe_gemm_nt_bf16 for dx = dy @ w^T, planmoe_gemm_tn_bf16 for dw = x^T @ dy); otherwise y takes a
-    transposed copy of w (kept per weight version) and dw transposed copies of x and dy whose row index
-    (the reduction) is padded with zeros to the kernel's k-tile.  dbias sums in fp32."""
+    experts/ffn.py:77-79 with its roundings.  All three products read their operands as they lie in
+    memory.  dbias sums in fp32."""
 
     @staticmethod
-    def forward(ctx, x, w, bias, relu, forms):
+    def forward(ctx, x, w, bias, relu):
         from . import ops
-        x = x.contiguous()
-        b = bias.detach() if bias is not None else None
-        if x.shape[2] % 64 == 0:
-            y = ops.gemm_nn_bf16(x, w.detach().contiguous(), b, relu=relu)          # the weight as it is stored
-        else:
-            y = ops.gemm_nt_bf16(x, forms.k_major(w), b, relu=relu)
+        x, w = x.contiguous(), w.contiguous()
+        y = ops.expert_gemm('nn', x, w, bias, relu=relu)
         ctx.save_for_backward(x, w, y if relu else None)
         ctx.relu, ctx.has_bias = relu, bias is not None
         return y
@@ -60,15 +38,12 @@ class _BatchedLinear(torch.autograd.Function):
             gy = torch.ops.aten.threshold_backward(gy, y, 0.0)      # relu's own backward: one pass over dy and y
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = ops.gemm_nt_bf16(gy, w.detach().contiguous())                    # [E, R, out] x [E, in, out]^T
+            dx = ops.expert_gemm('nt', gy, w)                       # [E, R, out] x [E, in, out]^T
         if ctx.needs_input_grad[1]:
-            if x.shape[1] % 64 == 0:
-                dw = ops.gemm_tn_bf16(x, gy)                                          # x^T dy, both as they lie
-            else:
-                dw = ops.gemm_nt_bf16(ops.transpose_bf16(x, 64), ops.transpose_bf16(gy, 64))      # [E, in, R'] x [E, out, R']^T
+            dw = ops.expert_gemm('tn', x, gy)                       # x^T dy
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = gy.sum(dim=1, dtype=torch.float32).to(gy.dtype)
-        return dx, dw, db, None, None
+        return dx, dw, db, None
 
 
 class FusedExpertsNetwork(torch.nn.Module):
@@ -107,17 +82,15 @@ class FusedExpertsNetwork(torch.nn.Module):
         self.batched_fc1_bias = torch.nn.Parameter(fc1_b)
         self.batched_fc2_bias = torch.nn.Parameter(fc2_b)
         self._fc1_k_major = None
-        self._fc1_forms, self._fc2_forms = _WeightForms(), _WeightForms()
 
-    # a batched library GEMM is not issued above this many multiply-adds: at the layer's real sizes
-    # ([8, 5120, 4096] x [8, 4096, 4096]) torch.matmul's batched bf16 kernel once ended a GPU run with
-    # an illegal-address error whose cause could not be established, so the layer stays off that call
+    # a batched library GEMM (the dtypes and sizes the kernels do not serve) is not issued above this many
+    # multiply-adds: torch's batched kernels with a transposed view as the right operand (what the backward
+    # pass of a batched product makes) have faulted the GPU; large products go one expert at a time
     LIBRARY_BATCHED_LIMIT = 1 << 32
 
-    def _linear(self, x, w, bias, relu, forms):
+    def _linear(self, x, w, bias, relu):
         if _kernel_serves(x, w):
-            return _BatchedLinear.apply(x, w, bias, relu, forms)
-        # other dtypes / odd sizes: the reference's composite; large products one expert at a time
+            return _BatchedLinear.apply(x, w, bias, relu)
         if x.is_cuda and x.shape[0] > 1 and x.shape[0] * x.shape[1] * w.shape[1] * w.shape[2] > self.LIBRARY_BATCHED_LIMIT:
             y = torch.stack([torch.addmm(bias[e], x[e], w[e]) for e in range(x.shape[0])])
         else:
@@ -126,10 +99,10 @@ class FusedExpertsNetwork(torch.nn.Module):
 
     def forward(self, x, ctx):
         # experts/ffn.py:63-82
-        y = self._linear(x, self.batched_fc1_w, self.batched_fc1_bias, self._relu, self._fc1_forms)
+        y = self._linear(x, self.batched_fc1_w, self.batched_fc1_bias, self._relu)
         if not self._relu:
             y = self.activation_fn(y)
-        return self._linear(y, self.batched_fc2_w, self.batched_fc2_bias, False, self._fc2_forms)
+        return self._linear(y, self.batched_fc2_w, self.batched_fc2_bias, False)
 
     def forward_from_codes(self, codes, bias, scale, exact=True):
         """The same forward with the int8 codes of the receive buffer as input (inference: no autograd
@@ -158,7 +131,7 @@ class FusedExpertsNetwork(torch.nn.Module):
         else:
             y = ops.ffn_fc1_int8_affine(codes, bias, scale, cached[1], cached[2], self.batched_fc1_bias.detach())
         y = self.activation_fn(y)
-        return self._linear(y, self.batched_fc2_w, self.batched_fc2_bias, False, self._fc2_forms)
+        return self._linear(y, self.batched_fc2_w, self.batched_fc2_bias, False)
 
 
 ExpertModule = FusedExpertsNetwork

@@ -1,0 +1,122 @@
+"""planmoe_expert_gemm / planmoe_expert_gemm_relu_bwd (the experts' products, bf16 and fp32, with row counts)
+and the two column reductions of the layer's backward pass, against fp64 on the host.
+
+Tolerances: fp32 sums of n terms are within (n + 2) 2^-24 of the sum of their magnitudes, whatever their
+order; a bf16 result adds 2^-8 of itself (half an ulp is 2^-9)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _bound(ref, mag, terms, dtype):
+    return (terms + 2) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0) + 1e-30
+
+
+# tiles are 256 x 256 or 128 x 128, k-tiles 64 (bf16) or 32 (fp32) and taken in pairs: sizes one piece either side of
+# those, one k-tile, an odd number of them, more than eight tile columns, one row
+SHAPES = [(1, 1, 8, 8), (2, 127, 136, 64), (3, 129, 264, 72), (2, 255, 520, 136), (2, 257, 128, 200), (1, 300, 2312, 64), (5, 40, 256, 320)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("B,m,n,k", SHAPES)
+def test_expert_gemm_against_fp64(B, m, n, k, form, dtype):
+    from planmoe_amd import ops
+    if form == "tn":
+        m = (m + 7) // 8 * 8                     # the fast index of a
+    print("case", form, dtype, B, m, n, k, flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(*((B, k, m) if form == "tn" else (B, m, k)), generator=g).to(dtype)
+    b = torch.randn(*((B, n, k) if form == "nt" else (B, k, n)), generator=g).to(dtype)
+    with_bias = form == "nn"
+    bias = torch.randn(B, n, generator=g).to(dtype) if with_bias else None
+    got = ops.expert_gemm(form, a.to(DEV), b.to(DEV), bias.to(DEV) if with_bias else None, relu=with_bias)
+    torch.cuda.synchronize()
+    ad, bd = a.double(), b.double()
+    ad, bd = (ad.transpose(1, 2) if form == "tn" else ad), (bd.transpose(1, 2) if form == "nt" else bd)
+    ref, mag = ad @ bd, ad.abs() @ bd.abs()
+    tol = _bound(ref, mag, k, dtype)
+    if with_bias:
+        ref, tol = ref + bias.double()[:, None, :], tol + _bound(ref + bias.double()[:, None, :], bias.double().abs()[:, None, :], 1, dtype)
+        ref = ref.clamp(min=0)                   # (clamping both sides of a comparison cannot move them apart)
+    assert bool(((got.double().cpu() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,cap,n,k,hint", [(4, 200, 264, 136, 0), (6, 520, 520, 64, 100), (64, 20, 72, 72, 5)])
+def test_expert_gemm_takes_the_rows_in_use_only(B, cap, n, k, hint, dtype):
+    """Row counts from two planes, rounded up to 1 and 4: none, few, more than the capacity; rows of the operands beyond
+    them hold NaN, rows of the result beyond them keep what was there; a tn product sums over the rows in use."""
+    from planmoe_amd import ops
+    g = torch.Generator().manual_seed(B + cap)
+    live = torch.randint(0, cap, (2, B), generator=g, dtype=torch.int32) // 2
+    live[:, 0] = 0
+    live[:, 1] = cap
+    live[0, 2], live[1, 2] = 1, 0
+    for rnd in (1, 4):
+        rows = [min(cap, (int(c) + rnd - 1) // rnd * rnd) for c in live.sum(0)]
+        a = torch.randn(B, cap, k, generator=g).to(dtype)
+        w = torch.randn(B, k, n, generator=g).to(dtype)
+        dy = torch.randn(B, cap, n, generator=g).to(dtype)
+        for e, r in enumerate(rows):
+            a[e, r:] = float("nan")
+            dy[e, r:] = float("nan")
+        out = torch.full((B, cap, n), 7.0, dtype=dtype, device=DEV)
+        ops.expert_gemm("nn", a.to(DEV), w.to(DEV), None, live=live.to(DEV), live_round=rnd, rows_hint=hint, out=out)
+        dw = ops.expert_gemm("tn", a.to(DEV), dy.to(DEV), live=live.to(DEV), live_round=rnd, rows_hint=hint)
+        torch.cuda.synchronize()
+        out, dw = out.cpu(), dw.cpu()
+        for e, r in enumerate(rows):
+            x, d = a[e, :r].double(), dy[e, :r].double()
+            ref, mag = x @ w[e].double(), x.abs() @ w[e].double().abs()
+            assert bool(((out[e, :r].double() - ref).abs() <= _bound(ref, mag, k, dtype)).all()), (e, r)
+            assert bool((out[e, r:] == 7.0).all()), (e, r)
+            ref, mag = x.t() @ d, x.abs().t() @ d.abs()
+            assert bool(((dw[e].double() - ref).abs() <= _bound(ref, mag, cap, dtype)).all()), (e, r)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,m,n,k,counted", [(2, 130, 136, 72, False), (3, 300, 520, 128, True), (1, 8, 8, 8, False)])
+def test_expert_gemm_relu_backward_and_its_bias_gradient(B, m, n, k, counted, dtype):
+    from planmoe_amd import ops
+    g = torch.Generator().manual_seed(m + n)
+    dy, w = torch.randn(B, m, k, generator=g).to(dtype), torch.randn(B, n, k, generator=g).to(dtype)
+    h = torch.randn(B, m, n, generator=g).clamp(min=0).to(dtype)
+    live = torch.tensor([[m // 2 + 3 * e for e in range(B)]], dtype=torch.int32) if counted else None
+    got, db = ops.expert_gemm_relu_bwd(dy.to(DEV), w.to(DEV), h.to(DEV), live=live.to(DEV) if counted else None)
+    torch.cuda.synchronize()
+    got, db = got.cpu(), db.cpu()
+    for e in range(B):
+        r = min(m, int(live[0, e])) if counted else m
+        ref, mag = dy[e, :r].double() @ w[e].double().t(), dy[e, :r].double().abs() @ w[e].double().abs().t()
+        keep = h[e, :r] > 0
+        assert bool(((got[e, :r].double() - ref * keep).abs() <= _bound(ref, mag, k, dtype)).all())
+        stored = got[e, :r].double()             # the sums are of what was stored
+        tol = _bound(stored.sum(0), stored.abs().sum(0), r, dtype)
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,M,E", [(1, 8, 1), (33, 520, 3), (1000, 264, 9), (517, 2056, 16)])
+def test_gate_weight_gradient_and_row_sums(T, M, E, dtype):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    g = torch.Generator().manual_seed(T + M)
+    x, gl = torch.randn(T, M, generator=g).to(dtype), torch.randn(T, E, generator=g)
+    xd, gd = x.to(DEV), gl.to(DEV)
+    dw = torch.empty(E, M, dtype=dtype, device=DEV)
+    ws = torch.empty(lib.planmoe_gate_dw_workspace_bytes(T, M, E), dtype=torch.uint8, device=DEV)
+    check(lib.planmoe_gate_dw(ops._ptr(xd), ops._dt(xd, "t"), ops._ptr(gd), T, M, E, ops._ptr(dw), ops._ptr(ws), ws.numel(), ops._stream(xd)))
+    live = torch.tensor([[T // 2], [T - T // 2 - T // 3]], dtype=torch.int32, device=DEV)
+    out = torch.empty(1, M, dtype=dtype, device=DEV)
+    ws2 = torch.empty(lib.planmoe_rows_colsum_workspace_bytes(1, T, M), dtype=torch.uint8, device=DEV)
+    check(lib.planmoe_rows_colsum(ops._ptr(xd), ops._dt(xd, "t"), 1, T, M, ops._ptr(live), 2, 4, ops._ptr(out), ops._ptr(ws2), ws2.numel(), ops._stream(xd)))
+    torch.cuda.synchronize()
+    gr = gl.to(dtype).double()
+    ref, mag = gr.t() @ x.double(), gr.abs().t() @ x.double().abs()
+    half = 2.0 ** -8 if dtype != torch.float32 else 0.0
+    assert bool(((dw.double().cpu() - ref).abs() <= (T + 2) * 2.0 ** -24 * mag + half * ref.abs() + 1e-30).all())
+    rows = x[:min(T, (T - T // 3 + 3) // 4 * 4)].double()
+    assert bool(((out[0].double().cpu() - rows.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * rows.abs().sum(0) + half * rows.sum(0).abs() + 1e-30).all())
