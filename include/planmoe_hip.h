@@ -427,6 +427,67 @@ int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, int m, int n
 int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int rows_out, void *out,
                            void *stream);
 
+/* The experts' products on their contiguous buffers, bf16 or fp32 (fp32: fp32 matrix cores), as the layer
+ * with the built-in experts issues them (experts/ffn.py:63-82 and its autograd).  form 0: c = act(a b + bias),
+ * a [batches, m, k], b [batches, k, n]; form 1: c = a b^T, b [batches, n, k]; form 2: c = a^T b, a [batches,
+ * k, m], b [batches, k, n].  Roundings as planmoe_gemm_*_bf16 (fp32: none but the fp32 sums' own).
+ * live, if not NULL: int32 [live_planes][batches], e.g. the expert_counts of the routing.  Batch e then has
+ * min(sum of its entries rounded up to live_round, m) rows (form 2: that many k) in use; rows of c beyond
+ * them are not written, rows of a and b beyond them are not read (up to 64 batches).  rows_hint: the number
+ * of rows in use to expect (what the tile is picked by; 0: all).  n, and k (form 2: m), multiples of 8
+ * (fp32: 4). */
+int planmoe_expert_gemm(int form, int dtype, const void *a, const void *b, const void *bias, int activation,
+                        int batches, int m, int n, int k, const int32_t *live, int live_planes,
+                        int live_round, int rows_hint, void *c, void *stream);
+
+/* The gradient through the first product's relu: c = a b^T where h > 0, else 0 (a [batches, m, k] the
+ * gradient of the second product's result, b [batches, n, k] its weight, h [batches, m, n] the activations),
+ * and the first bias's gradient dbias [batches, n] = column sums of c over the rows in use (NULL: not
+ * wanted; workspace: planmoe_expert_gemm_relu_bwd_workspace_bytes).  The rest as planmoe_expert_gemm. */
+size_t planmoe_expert_gemm_relu_bwd_workspace_bytes(int batches, int m, int n);
+int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void *b, const void *h, int batches, int m,
+                                 int n, int k, const int32_t *live, int live_planes, int live_round,
+                                 int rows_hint, void *c, void *dbias, void *workspace,
+                                 size_t workspace_bytes, void *stream);
+
+/* ---------------------------------------------------------------- the layer on one rank
+ * planmoe_forward_plain for a buffer that stays on this GPU: rows of empty capacity slots are not written,
+ * and with codec = 1 a row arrives as Int8Compressor::decompress(compress(row)) would leave it
+ * (int8.cpp:10-24, 46-60; what overlap.py:12-34 does around a one-rank exchange), same bits, without the
+ * codes.  codec = 0: the row itself. */
+int planmoe_layer_dispatch(const void *x, const void *wg, int dtype, int fp32_gate, const float *logit_bias,
+                           int samples, int model_dim, int experts, int top_k, int normalize_gate,
+                           int capacity, int codec, int32_t *indices, int32_t *locations, void *gates,
+                           int64_t plane_stride, void *scores_out, float *l_aux, int32_t *expert_counts,
+                           void *rows, void *workspace, size_t workspace_bytes, void *stream);
+
+/* fast_decode (fast_dispatch.py:203-207) of the experts' rows, each taken through the int8 codec first when
+ * codec = 1 (as the receive side's Compress / Decompress pair would, overlap.py:66-74).  Reads only rows that hold a
+ * token.  gates NULL: all ones.  model_dim a multiple of 8 (fp32: 4), at most 8192 (fp32: 4096). */
+int planmoe_layer_combine(const void *rows, int dtype, int codec, const float *gates, const int32_t *indices,
+                          const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                          int model_dim, int experts, int capacity, void *out, void *stream);
+
+/* Its backward pass (GatingDecoder.backward, fast_dispatch.py:62-79): grad_gates[j][t] = <grad[t],
+ * codec(rows[slot])> and grad_rows[slot] = codec(gate * grad[t]); rows of empty slots are not written. */
+int planmoe_layer_combine_bwd(const void *grad, const void *rows, int dtype, int codec, const float *gates,
+                              const int32_t *indices, const int32_t *locations, int64_t plane_stride,
+                              int top_k, int samples, int model_dim, int experts, int capacity,
+                              void *grad_rows, float *grad_gates, void *stream);
+
+/* out[e][c] = sum over the rows in use of a[e] (live as planmoe_expert_gemm): a bias gradient of
+ * experts/ffn.py:77-79.  fp32 sums, one rounding. */
+size_t planmoe_rows_colsum_workspace_bytes(int batches, int rows, int cols);
+int planmoe_rows_colsum(const void *a, int dtype, int batches, int rows, int cols, const int32_t *live,
+                        int live_planes, int live_round, void *out, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
+/* The gate weight's gradient (the autograd of gates/top.py:21-26): out[e][m] = sum over the tokens of
+ * grad_logits[t][e] * x[t][m], grad_logits rounded to x's dtype, fp32 sums, one rounding. */
+size_t planmoe_gate_dw_workspace_bytes(int samples, int model_dim, int experts);
+int planmoe_gate_dw(const void *x, int dtype, const float *grad_logits, int samples, int model_dim,
+                    int experts, void *out, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------- zfp fixed-rate codec
  * Replaces ZfpCompressor::compress / ::decompress (custom/compressor/zfpc.cpp:23-86), i.e.
  * zfp_compress / zfp_decompress of the third-party zfp library in fixed-rate mode on fp32.

@@ -80,6 +80,23 @@ SIGNATURES = {
                                      c_int64, c_int64, c_int64, c_void_p, c_void_p]),
     "planmoe_gemm_tn_bf16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64,
                                      c_int64, c_int64, c_void_p, c_void_p]),
+    "planmoe_expert_gemm": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
+                                    c_int, c_int, c_void_p, c_void_p]),
+    "planmoe_expert_gemm_relu_bwd_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "planmoe_expert_gemm_relu_bwd": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
+                                             c_int, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "planmoe_layer_dispatch": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                       c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                       c_size_t, c_void_p]),
+    "planmoe_layer_combine": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                      c_void_p, c_void_p]),
+    "planmoe_layer_combine_bwd": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
+                                          c_int, c_int, c_void_p, c_void_p, c_void_p]),
+    "planmoe_rows_colsum_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "planmoe_rows_colsum": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_size_t,
+                                    c_void_p]),
+    "planmoe_gate_dw_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "planmoe_gate_dw": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
     "planmoe_transpose_bf16": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "planmoe_forward_int8_static": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int,
                                             c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,

@@ -1,5 +1,6 @@
-"""Builds schemoe_custom_kernel*.so (the reference's pybind module name) in planmoe_amd/csrc/ext with
-g++ against torch's headers and libplanmoe_hip.so.  Run by __graft_entry__.build()."""
+"""Builds schemoe_custom_kernel*.so (the reference's pybind module name) and _planmoe_layer*.so (the layer's
+host side) in planmoe_amd/csrc/ext with g++ against torch's headers and libplanmoe_hip.so.  Run by
+__graft_entry__.build()."""
 import os
 import subprocess
 import sys
@@ -11,28 +12,30 @@ from torch.utils import cpp_extension as ce
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.abspath(os.path.join(HERE, "..", "..", ".."))
 NAME = "schemoe_custom_kernel"
+LAYER = "_planmoe_layer"
 
 
-def target():
-    return os.path.join(HERE, NAME + sysconfig.get_config_var("EXT_SUFFIX"))
+def target(name=NAME):
+    return os.path.join(HERE, name + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
-def _flags():
+def _flags(name):
     return ["-O2", "-std=c++17", "-fPIC", "-Wno-deprecated-declarations",
-            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=" + NAME,
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=" + name,
             "-DTORCH_API_INCLUDE_EXTENSION_H", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
             "-I" + os.path.join(ROOT, "include"), "-I/opt/rocm/include", "-I" + sysconfig.get_paths()["include"]] + \
            ["-I" + p for p in ce.include_paths()]
 
 
 def _objects():
-    return [(os.path.join(HERE, NAME + ".cpp"), os.path.join(HERE, NAME + ".o")),
-            (os.path.join(HERE, "example_third_party_compressor.cpp"), os.path.join(HERE, "example_third_party_compressor.o"))]
+    return [(NAME, os.path.join(HERE, NAME + ".cpp"), os.path.join(HERE, NAME + ".o")),
+            (NAME, os.path.join(HERE, "example_third_party_compressor.cpp"), os.path.join(HERE, "example_third_party_compressor.o")),
+            (LAYER, os.path.join(HERE, "layer.cpp"), os.path.join(HERE, LAYER + ".o"))]
 
 
 def compile_objects():
-    """The two sources to objects, side by side (each is a minute of torch headers); needs no libplanmoe_hip.so yet."""
-    procs = [subprocess.Popen(["g++"] + _flags() + ["-c", src, "-o", obj]) for src, obj in _objects()]
+    """The sources to objects, side by side (each is a minute of torch headers); needs no libplanmoe_hip.so yet."""
+    procs = [subprocess.Popen(["g++"] + _flags(name) + ["-c", src, "-o", obj]) for name, src, obj in _objects()]
     codes = [p.wait() for p in procs]
     if any(codes):
         raise subprocess.CalledProcessError(max(codes), "g++ -c (extension objects)")
@@ -40,14 +43,15 @@ def compile_objects():
 
 def link():
     csrc = os.path.join(ROOT, "planmoe_amd", "csrc")
-    (_, module_obj), (_, example_obj) = _objects()
+    (_, _, module_obj), (_, _, example_obj), (_, _, layer_obj) = _objects()
     libs = ["-L" + p for p in ce.library_paths()] + ["-L/opt/rocm/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
             "-ltorch", "-ltorch_python", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"] + ["-Wl,-rpath," + p for p in ce.library_paths()]
     subprocess.check_call(["g++", "-shared", module_obj, "-o", target(), "-L" + csrc, "-lplanmoe_hip", "-Wl,-rpath," + csrc] + libs)
+    subprocess.check_call(["g++", "-shared", layer_obj, "-o", target(LAYER), "-L" + csrc, "-lplanmoe_hip", "-Wl,-rpath," + csrc] + libs)
     # the example plug-in: a compressor compiled against include/planmoe/compressor/abstract.h with the
     # same flags and linked against the module just built
     subprocess.check_call(["g++", "-shared", example_obj, "-o", example_target(), target(), "-Wl,-rpath," + HERE] + libs)
-    for _, obj in _objects():
+    for _, _, obj in _objects():
         os.remove(obj)
     return target()
 

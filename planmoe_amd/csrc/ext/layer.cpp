@@ -1,0 +1,336 @@
+// The layer with its built-in experts as one node: gate, routing, encode, codec, FFN, codec, decode, and
+// the backward pass of all of them, driven from C++.
+//
+// A forward pass is five to nine launches of a few microseconds each at decode sizes; driven step by step
+// from Python (an autograd node, a dozen tensor operations and a ctypes call with two dozen arguments for
+// each) the host took 160 us for 40 us of GPU work.  Here a pass is one call: outputs and workspaces from
+// torch's caching allocator, launches through the C ABI of libplanmoe_hip.
+//
+// With one rank the exchange delivers what was sent, so the "int8" codec is applied to rows in registers
+// (planmoe_layer_dispatch, planmoe_layer_combine, planmoe_layer_combine_bwd) and the rows of empty capacity
+// slots are neither written nor multiplied: the products get the number of rows in use of every expert.
+#include "planmoe_hip.h"
+
+#include <ATen/hip/HIPEvent.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/extension.h>
+
+#include <algorithm>
+
+namespace {
+
+using torch::Tensor;
+
+enum Codec { CODEC_NONE = 0, CODEC_INT8 = 1, CODEC_ZFP = 2, CODEC_LZ = 3 };
+constexpr double ZFP_RATE = 8.0;             // zfpc.h:17
+
+void *current_stream() { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
+#define PM_CALL(expr) TORCH_CHECK((expr) == 0, planmoe_last_error())
+
+int pm_dtype(at::ScalarType t)
+{
+    TORCH_CHECK(t == at::kFloat || t == at::kBFloat16 || t == at::kHalf, "planmoe: unsupported dtype (float32, bfloat16 or float16)");
+    return t == at::kFloat ? PLANMOE_F32 : t == at::kBFloat16 ? PLANMOE_BF16 : PLANMOE_F16;
+}
+const int32_t *ints(const Tensor &t) { return t.data_ptr<int32_t>(); }
+const float *floats(const Tensor &t) { return t.data_ptr<float>(); }
+void *raw(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+struct Shape {
+    int T, M, E, H, k, cap, dt;
+    int64_t rows() const { return (int64_t)E * cap; }
+    // rows an expert is expected to have in use: what the products pick their tiles by
+    int hint() const { return (int)std::min<int64_t>(cap, ((int64_t)T * k + E - 1) / E); }
+};
+
+// which rows of an expert's buffer count: the tokens' own, a zfp block's four rows together, or (lz: the codec
+// runs over the whole buffer) all of them
+struct Live {
+    const int32_t *counts;
+    int planes, round;
+};
+
+struct Pass {
+    Tensor y, l_aux, gates, indices, locations, counts, scores, xe, h, ye, stream;
+};
+
+Tensor bytes(int64_t n, const Tensor &like) { return at::empty({std::max<int64_t>(n, 16)}, like.options().dtype(at::kByte)); }
+
+Tensor lz_round_trip(const Tensor &buf, void *st)
+{
+    const int64_t n = (int64_t)buf.nbytes(), blocks = planmoe_lz_blocks(n);
+    Tensor offsets = at::empty({2, blocks + 1 + (-(blocks + 1) & 3)}, buf.options().dtype(at::kInt));      // (rows 16-byte aligned)
+    Tensor flags = bytes(blocks * 64, buf), data = bytes(blocks * 2048, buf), ws = bytes((int64_t)planmoe_lz_workspace_bytes(n), buf);
+    int32_t *fo = offsets.data_ptr<int32_t>(), *dof = fo + offsets.size(1);
+    Tensor out = at::empty_like(buf);
+    PM_CALL(planmoe_lz_compress(buf.data_ptr(), n, fo, dof, flags.data_ptr<uint8_t>(), data.data_ptr<uint8_t>(), ws.data_ptr(), (size_t)ws.numel(), st));
+    PM_CALL(planmoe_lz_decompress(out.data_ptr(), n, fo, dof, flags.data_ptr<uint8_t>(), data.data_ptr<uint8_t>(), st));
+    return out;
+}
+
+Tensor zfp_stream_of(const Tensor &rows, const Shape &s, void *st)
+{
+    Tensor out = bytes((int64_t)planmoe_zfp_max_bytes(2, s.M, s.rows(), ZFP_RATE), rows);
+    PM_CALL(planmoe_zfp_compress(floats(rows), 2, s.M, s.rows(), ZFP_RATE, out.data_ptr(), (size_t)out.numel(), st));
+    return out;
+}
+
+Tensor zfp_dispatch(const Tensor &x, const float *gates, const Pass &p, const Shape &s, void *st)
+{
+    Tensor coded = bytes((int64_t)planmoe_zfp_max_bytes(2, s.M, s.rows(), ZFP_RATE), x);
+    Tensor ws = bytes((int64_t)planmoe_dispatch_zfp_workspace_bytes(s.E, s.cap), x), out = at::empty({s.rows(), s.M}, x.options());
+    PM_CALL(planmoe_dispatch_zfp(floats(x), gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap, ZFP_RATE,
+                                 coded.data_ptr(), (size_t)coded.numel(), ws.data_ptr(), (size_t)ws.numel(), st));
+    PM_CALL(planmoe_zfp_decompress(coded.data_ptr(), 2, s.M, s.rows(), ZFP_RATE, out.data_ptr<float>(), st));
+    return out;
+}
+
+Tensor zfp_combine(const Tensor &stream, const float *gates, const Pass &p, const Shape &s, void *st)
+{
+    Tensor out = at::empty({s.T, s.M}, stream.options().dtype(at::kFloat)), ws = bytes((int64_t)planmoe_combine_zfp_workspace_bytes(s.E, s.cap), stream);
+    PM_CALL(planmoe_combine_zfp(stream.data_ptr(), ZFP_RATE, gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap,
+                                out.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
+    return out;
+}
+
+// fast_encode's buffer with zeros in the empty slots
+Tensor dispatch_rows(const Tensor &x, const float *gates, const Pass &p, const Shape &s, void *st)
+{
+    Tensor out = at::empty({s.rows(), s.M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(s.E, s.cap), x);
+    PM_CALL(planmoe_dispatch_fwd(x.data_ptr(), s.dt, gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap,
+                                 out.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), st));
+    return out;
+}
+
+Live live_rows(const Pass &p, const Shape &s, int codec)
+{
+    if (codec == CODEC_LZ) return Live{nullptr, 1, 1};
+    return Live{ints(p.counts), s.k, codec == CODEC_ZFP ? 4 : 1};
+}
+
+Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
+
+Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, const Shape &s,
+                  bool fp32_gate, bool normalize, int codec, bool keep)
+{
+    void *st = current_stream();
+    Pass p;
+    const auto score_type = fp32_gate ? at::kFloat : x.scalar_type();
+    const auto i32 = x.options().dtype(at::kInt);
+    // [k, T] of indices and of locations, [k, E] of counts
+    Tensor planes = at::empty({2 * (int64_t)s.k * s.T + (int64_t)s.k * s.E}, i32);
+    p.indices = planes.narrow(0, 0, (int64_t)s.k * s.T);
+    p.locations = planes.narrow(0, (int64_t)s.k * s.T, (int64_t)s.k * s.T);
+    p.counts = planes.narrow(0, 2 * (int64_t)s.k * s.T, (int64_t)s.k * s.E);
+    p.gates = at::empty({s.k, s.T}, x.options().dtype(score_type));
+    p.l_aux = at::empty({}, x.options().dtype(at::kFloat));
+    if (keep) p.scores = at::empty({s.T, s.E}, x.options().dtype(score_type));
+    Tensor ws = bytes((int64_t)planmoe_forward_workspace_bytes(s.T, s.E, s.k), x);
+    int32_t *idx = p.indices.data_ptr<int32_t>(), *loc = p.locations.data_ptr<int32_t>(), *cnt = p.counts.data_ptr<int32_t>();
+    if (codec == CODEC_ZFP) {
+        PM_CALL(planmoe_gate_route(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, idx, loc, raw(p.gates),
+                                   s.T, nullptr, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, ws.data_ptr(), (size_t)ws.numel(), st));
+        p.xe = zfp_dispatch(x, nullptr, p, s, st);
+    } else if (codec == CODEC_LZ) {
+        p.xe = at::empty({s.rows(), s.M}, x.options());
+        PM_CALL(planmoe_forward_plain(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, idx, loc,
+                                      raw(p.gates), s.T, nullptr, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
+                                      (size_t)ws.numel(), st));
+        p.xe = lz_round_trip(p.xe, st);
+    } else {
+        p.xe = at::empty({s.rows(), s.M}, x.options());
+        PM_CALL(planmoe_layer_dispatch(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, codec, idx, loc,
+                                       raw(p.gates), s.T, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
+                                       (size_t)ws.numel(), st));
+    }
+    const Live live = live_rows(p, s, codec);
+    p.h = at::empty({s.rows(), s.H}, x.options());
+    PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
+                                s.hint(), p.h.data_ptr(), st));
+    p.ye = at::empty({s.rows(), s.M}, x.options());
+    PM_CALL(planmoe_expert_gemm(0, s.dt, p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
+                                s.hint(), p.ye.data_ptr(), st));
+    const Tensor gates = float_gates(p.gates);
+    if (codec == CODEC_ZFP) {
+        p.stream = zfp_stream_of(p.ye, s, st);
+        p.ye = Tensor();                     // (the backward pass reads the stream)
+        p.y = zfp_combine(p.stream, floats(gates), p, s, st);
+        return p;
+    }
+    if (codec == CODEC_LZ) p.ye = lz_round_trip(p.ye, st);
+    p.y = at::empty({s.T, s.M}, x.options());
+    PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, codec == CODEC_INT8, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
+    return p;
+}
+
+Shape shape_of(const Tensor &x, const Tensor &wg, const Tensor &w1, int64_t k, int64_t cap)
+{
+    Shape s;
+    s.T = (int)x.size(0);
+    s.M = (int)x.size(1);
+    s.E = (int)wg.size(0);
+    s.H = (int)w1.size(2);
+    s.k = (int)k;
+    s.cap = (int)cap;
+    s.dt = pm_dtype(x.scalar_type());
+    return s;
+}
+
+void check(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, int64_t k, int64_t cap)
+{
+    TORCH_CHECK(x.dim() == 2 && wg.dim() == 2 && w1.dim() == 3 && w2.dim() == 3 && b1.dim() == 2 && b2.dim() == 2, "ffn_layer: wrong ranks");
+    const int64_t M = x.size(1), E = wg.size(0), H = w1.size(2);
+    TORCH_CHECK(wg.size(1) == M && w1.size(0) == E && w1.size(1) == M && w2.size(0) == E && w2.size(1) == H && w2.size(2) == M &&
+                b1.size(0) == E && b1.size(1) == H && b2.size(0) == E && b2.size(1) == M, "ffn_layer: shapes do not fit");
+    TORCH_CHECK(k >= 1 && k <= E && cap >= 1 && x.size(0) >= 1, "ffn_layer: bad routing shape");
+    for (const Tensor *t : {&x, &wg, &w1, &b1, &w2, &b2})
+        TORCH_CHECK(t->is_cuda() && t->is_contiguous() && t->scalar_type() == x.scalar_type() && t->device() == x.device(),
+                    "ffn_layer: contiguous GPU tensors of one dtype on one device");
+}
+
+struct FfnLayer : public torch::autograd::Function<FfnLayer> {
+    static torch::autograd::variable_list forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &wg, const Tensor &w1,
+                                                  const Tensor &b1, const Tensor &w2, const Tensor &b2, int64_t k, int64_t cap, bool fp32_gate,
+                                                  bool normalize, int64_t codec)
+    {
+        const Shape s = shape_of(x, wg, w1, k, cap);
+        Pass p = forward_pass(x, wg, w1, b1, w2, b2, s, fp32_gate, normalize, (int)codec, true);
+        ctx->save_for_backward({x, wg, w1, w2, p.scores, p.gates, p.indices, p.locations, p.counts, p.xe, p.h, codec == CODEC_ZFP ? p.stream : p.ye});
+        ctx->saved_data["k"] = k;
+        ctx->saved_data["cap"] = cap;
+        ctx->saved_data["normalize"] = normalize;
+        ctx->saved_data["codec"] = codec;
+        return {p.y, p.l_aux};
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &wg = saved[1], &w1 = saved[2], &w2 = saved[3], &scores = saved[4];
+        const c10::DeviceGuard guard(x.device());
+        const int codec = (int)ctx->saved_data["codec"].toInt();
+        const bool normalize = ctx->saved_data["normalize"].toBool();
+        const Shape s = shape_of(x, wg, w1, ctx->saved_data["k"].toInt(), ctx->saved_data["cap"].toInt());
+        void *st = current_stream();
+        Pass p;
+        p.gates = saved[5];
+        p.indices = saved[6];
+        p.locations = saved[7];
+        p.counts = saved[8];
+        p.xe = saved[9];
+        p.h = saved[10];
+        const Tensor &ye = saved[11];
+        const int32_t *idx = ints(p.indices), *loc = ints(p.locations);
+        const bool need_x = ctx->needs_input_grad(0), need_gate = ctx->needs_input_grad(1), need_w1 = ctx->needs_input_grad(2),
+                   need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
+        Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates;
+        if (grads[0].defined()) {
+            const Tensor grad = grads[0].contiguous();
+            const Tensor gates = float_gates(p.gates);
+            const Live live = live_rows(p, s, codec);
+            grad_gates = at::empty({s.k, s.T}, x.options().dtype(at::kFloat));
+            Tensor gye;
+            if (codec == CODEC_ZFP) {
+                gye = zfp_dispatch(grad, floats(gates), p, s, st);
+                Tensor ws = bytes((int64_t)planmoe_combine_zfp_workspace_bytes(s.E, s.cap), x);
+                PM_CALL(planmoe_bwd_gate_zfp(ye.data_ptr(), ZFP_RATE, floats(grad), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                                             grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
+            } else if (codec == CODEC_LZ) {
+                gye = lz_round_trip(dispatch_rows(grad, floats(gates), p, s, st), st);
+                PM_CALL(planmoe_bwd_gate(grad.data_ptr(), ye.data_ptr(), s.dt, idx, loc, s.T, s.k, s.T, s.M, s.cap, grad_gates.data_ptr<float>(), st));
+            } else {
+                gye = at::empty({s.rows(), s.M}, x.options());
+                PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, codec == CODEC_INT8, floats(gates), idx, loc, s.T, s.k, s.T, s.M,
+                                                  s.E, s.cap, gye.data_ptr(), grad_gates.data_ptr<float>(), st));
+            }
+            auto colsum = [&](const Tensor &a, int cols) {
+                Tensor out = at::empty({s.E, cols}, x.options()), ws = bytes((int64_t)planmoe_rows_colsum_workspace_bytes(s.E, s.cap, cols), x);
+                PM_CALL(planmoe_rows_colsum(a.data_ptr(), s.dt, s.E, s.cap, cols, live.counts, live.planes, live.round, out.data_ptr(), ws.data_ptr(),
+                                            (size_t)ws.numel(), st));
+                return out;
+            };
+            if (need_w2) {
+                dw2 = at::empty_like(w2);
+                PM_CALL(planmoe_expert_gemm(2, s.dt, p.h.data_ptr(), gye.data_ptr(), nullptr, 0, s.E, s.H, s.M, s.cap, live.counts, live.planes, live.round,
+                                            s.hint(), dw2.data_ptr(), st));
+            }
+            if (need_b2) db2 = colsum(gye, s.M);
+            if (need_x || need_w1 || need_b1) {
+                Tensor gh = at::empty({s.rows(), s.H}, x.options()), ws;
+                if (need_b1) {
+                    db1 = at::empty({s.E, s.H}, x.options());
+                    ws = bytes((int64_t)planmoe_expert_gemm_relu_bwd_workspace_bytes(s.E, s.cap, s.H), x);
+                }
+                PM_CALL(planmoe_expert_gemm_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
+                                                     live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), ws.defined() ? (size_t)ws.numel() : 0, st));
+                if (need_w1) {
+                    dw1 = at::empty_like(w1);
+                    PM_CALL(planmoe_expert_gemm(2, s.dt, p.xe.data_ptr(), gh.data_ptr(), nullptr, 0, s.E, s.M, s.H, s.cap, live.counts, live.planes,
+                                                live.round, s.hint(), dw1.data_ptr(), st));
+                }
+                if (need_x) {
+                    Tensor gxe = at::empty({s.rows(), s.M}, x.options());
+                    PM_CALL(planmoe_expert_gemm(1, s.dt, gh.data_ptr(), w1.data_ptr(), nullptr, 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
+                                                s.hint(), gxe.data_ptr(), st));
+                    if (codec == CODEC_ZFP) {
+                        dx = zfp_combine(zfp_stream_of(gxe, s, st), nullptr, p, s, st);
+                    } else {
+                        if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
+                        dx = at::empty_like(x);
+                        PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                                                      dx.data_ptr(), st));
+                    }
+                }
+            }
+        }
+        // gates and loss back through the routing into the gate's weight and x
+        if ((grad_gates.defined() || grads[1].defined()) && (need_x || need_gate)) {
+            Tensor gg = grad_gates.defined() ? grad_gates.to(scores.scalar_type()) : at::zeros({s.k, s.T}, scores.options());
+            Tensor gl = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
+            Tensor g = at::empty_like(scores);
+            PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), idx, gg.data_ptr(), s.T, s.T, s.E, s.k, normalize,
+                                      gl.defined() ? floats(gl) : nullptr, gl.defined() ? ints(p.counts) : nullptr, 1, g.data_ptr(), st));
+            const Tensor gf = g.scalar_type() == at::kFloat ? g : g.to(at::kFloat);
+            if (need_gate) {
+                dwg = at::empty_like(wg);
+                Tensor ws = bytes((int64_t)planmoe_gate_dw_workspace_bytes(s.T, s.M, s.E), x);
+                PM_CALL(planmoe_gate_dw(x.data_ptr(), s.dt, floats(gf), s.T, s.M, s.E, dwg.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), st));
+            }
+            if (need_x) {
+                if (!dx.defined()) {
+                    dx = at::mm(g.to(x.scalar_type()), wg);
+                } else if (s.E <= 8) {
+                    PM_CALL(planmoe_gate_dx_accumulate(dx.data_ptr(), s.dt, floats(gf), wg.data_ptr(), s.T, s.M, s.E, st));
+                } else {
+                    dx.addmm_(g.to(x.scalar_type()), wg);
+                }
+            }
+        }
+        return {dx, dwg, dw1, db1, dw2, db2, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// (y [T, M], l_aux fp32); codec: 0 none, 1 int8, 2 zfp, 3 lz
+std::tuple<Tensor, Tensor> ffn_layer(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2,
+                                     int64_t k, int64_t cap, bool fp32_gate, bool normalize, int64_t codec)
+{
+    check(x, wg, w1, b1, w2, b2, k, cap);
+    const c10::DeviceGuard guard(x.device());
+    bool grad = false;
+    if (at::GradMode::is_enabled())
+        for (const Tensor *t : {&x, &wg, &w1, &b1, &w2, &b2}) grad |= t->requires_grad();
+    if (!grad) {
+        const at::NoGradGuard no_grad;
+        Pass p = forward_pass(x, wg, w1, b1, w2, b2, shape_of(x, wg, w1, k, cap), fp32_gate, normalize, (int)codec, false);
+        return {p.y, p.l_aux};
+    }
+    auto out = FfnLayer::apply(x, wg, w1, b1, w2, b2, k, cap, fp32_gate, normalize, codec);
+    return {out[0], out[1]};
+}
+
+} // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    m.def("ffn_layer", &ffn_layer, pybind11::call_guard<pybind11::gil_scoped_release>(), "the layer with its built-in experts, forward (and its autograd node)");
+}

@@ -480,9 +480,13 @@ __global__ __launch_bounds__(256) void route_locations_merged_kernel(
 // none of its choices leaves without reading its row.  Pays when many tokens are dropped (a
 // capacity factor of 1 with skewed routing drops half of them); otherwise the row is requested
 // first so that it travels while the slots are being worked out.
-// PLAIN: no codec -- `codes` is the dispatched buffer in x's dtype and a kept row arrives there as
-// 0 + x (what fast_encode's accumulation into zeros leaves: -0 becomes +0), an empty slot as zeros.
-template <int DT, int CACHE, bool MERGED, bool SLOT_FIRST = false, bool PLAIN = false>
+// OUT: what a kept row arrives as.  CODES: codes with bias and scale.  ROWS: no codec -- `codes` is the
+// dispatched buffer in x's dtype and a kept row arrives there as 0 + x (what fast_encode's accumulation
+// into zeros leaves: -0 becomes +0), an empty slot as zeros.  DECODED: the same buffer with what the
+// decompressor makes of the row's codes (the codes stay in registers: one pass where dispatch + int8
+// and the decompressor write and read them).
+enum { OUT_CODES = 0, OUT_ROWS = 1, OUT_DECODED = 2 };
+template <int DT, int CACHE, bool MERGED, bool SLOT_FIRST = false, int OUT = OUT_CODES>
 __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
     const void *__restrict__ x, const int32_t *__restrict__ indices, int32_t *__restrict__ locations,
     int64_t stride, int top_k, int samples, int model_dim, int experts, int capacity,
@@ -537,7 +541,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
             const int e = s / capacity;
             const int filled = MERGED ? s_tot[e] : totals[e];
             if (s - e * capacity < filled) continue;             // slot holds a token
-            if constexpr (PLAIN) {
+            if constexpr (OUT != OUT_CODES) {
                 uint4 *row = reinterpret_cast<uint4 *>(codes + (int64_t)s * units * 16);
                 for (int u = lane; u < units; u += WAVE) stream_store(row + u, make_uint4(0u, 0u, 0u, 0u));
                 continue;
@@ -600,7 +604,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
         if (__ballot(slot >= 0) == 0) return;
     }
 
-    if constexpr (PLAIN) {
+    if constexpr (OUT == OUT_ROWS) {
         auto copy = [&](int u, const uint4 &raw) {
             float f[V];
             E::unpack(raw, f);
@@ -636,13 +640,27 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
         stats.finish(mn, mx);
     }
     const float scale = E::round(mx - mn);
-    if (slot >= 0) { E::store(bias_out, slot, mn); E::store(scale_out, slot, scale); }
+    if constexpr (OUT == OUT_CODES) {
+        if (slot >= 0) { E::store(bias_out, slot, mn); E::store(scale_out, slot, scale); }
+    }
     const RowEncoder<DT> enc(mn, scale);
+    const RowDecoder<DT> dec(mn, scale);
 
     auto body = [&](auto mode) {
         auto emit = [&](int u, const uint4 &raw) {
             uint32_t w[2];
             enc.template encode<decltype(mode)::value>(raw, w);
+            if constexpr (OUT == OUT_DECODED) {
+                float f[V];
+#pragma unroll
+                for (int q = 0; q < V / 4; ++q) dec.word(w[q], f + 4 * q);
+                const uint4 v = E::pack(f);
+                for (int j = 0; j < top_k; ++j) {
+                    const int s = rl_i(slot, j);
+                    if (s >= 0) stream_store(reinterpret_cast<uint4 *>(codes + (int64_t)s * units * 16) + u, v);
+                }
+                return;
+            }
             for (int j = 0; j < top_k; ++j) {
                 const int s = rl_i(slot, j);
                 if (s < 0) continue;
@@ -691,25 +709,26 @@ static void launch_dispatch_routed(int per_lane, unsigned grid, hipStream_t st, 
                                    const float *loss_part, int loss_parts, float *l_aux,
                                    const float *row_min, const float *row_max, bool merged,
                                    const int32_t *hist_t, const float *me_t, int groups, int gstride,
-                                   int fill_blocks, int32_t *counts, int fill_first, bool plain = false)
+                                   int fill_blocks, int32_t *counts, int fill_first, int out)
 {
     // a capacity factor of at most 1: every imbalance of the routing drops tokens
     const bool slot_first = merged && (int64_t)experts * capacity <= (int64_t)top_k * samples;
-#define PM_DR_(CACHE, MERGED, FIRST, PLAIN)                                                          \
-    dispatch_int8_routed_kernel<DT, CACHE, MERGED, FIRST, PLAIN><<<grid, 256, 0, st>>>(x, indices, locations, stride, top_k, \
+#define PM_DR_(CACHE, MERGED, FIRST, OUT)                                                            \
+    dispatch_int8_routed_kernel<DT, CACHE, MERGED, FIRST, OUT><<<grid, 256, 0, st>>>(x, indices, locations, stride, top_k, \
         samples, model_dim, experts, capacity, codes, bias, scale, offs, totals, rank, group_tokens,  \
         token_blocks, loss_part, loss_parts, l_aux, row_min, row_max, hist_t, me_t, groups, gstride,  \
         fill_blocks, counts, fill_first)
-#define PM_DR(CACHE) do { if (plain) { if (slot_first) PM_DR_(CACHE, true, true, true); else if (merged) PM_DR_(CACHE, true, false, true); \
-                                       else PM_DR_(CACHE, false, false, true); }                      \
-                          else if (slot_first) PM_DR_(CACHE, true, true, false); else if (merged) PM_DR_(CACHE, true, false, false); \
-                          else PM_DR_(CACHE, false, false, false); } while (0)
+#define PM_DR__(CACHE, OUT) do { if (slot_first) PM_DR_(CACHE, true, true, OUT); else if (merged) PM_DR_(CACHE, true, false, OUT); \
+                                 else PM_DR_(CACHE, false, false, OUT); } while (0)
+#define PM_DR(CACHE) do { if (out == OUT_ROWS) PM_DR__(CACHE, OUT_ROWS); else if (out == OUT_DECODED) PM_DR__(CACHE, OUT_DECODED); \
+                          else PM_DR__(CACHE, OUT_CODES); } while (0)
     if (per_lane <= 2) PM_DR(2);
     else if (per_lane <= 4) PM_DR(4);
     else if (per_lane <= 8) PM_DR(8);
     else if (per_lane <= 16) PM_DR(16);
     else PM_DR(0);
 #undef PM_DR
+#undef PM_DR__
 #undef PM_DR_
 }
 
@@ -841,11 +860,11 @@ static int run_gate_route(const void *x, const void *wg, int dtype, int fp32_gat
 static int run_dispatch_routed(const void *x, int dtype, int samples, int model_dim, int experts,
                                int capacity, const int32_t *indices, int32_t *locations, int64_t stride,
                                float *l_aux, int32_t *counts, uint8_t *codes, void *bias, void *scale,
-                               const FwdPlan &plan, hipStream_t st, bool plain = false)
+                               const FwdPlan &plan, hipStream_t st, int out = OUT_CODES, bool fill = true)
 {
     const int slots = experts * capacity;
     const int token_blocks = (samples + 3) / 4;
-    int fill_blocks = min((slots + 3) / 4, 2048);
+    int fill_blocks = fill ? min((slots + 3) / 4, 2048) : 0;        // (fill: zero rows for the empty slots)
     if (plan.merged) {
         // every zero-fill block reads the whole transposed histogram once: keep that under ~32 MB
         const int64_t table = (int64_t)plan.k * experts * plan.ws.gstride * 4;
@@ -862,7 +881,7 @@ static int run_dispatch_routed(const void *x, int dtype, int samples, int model_
                                    dtype == PLANMOE_BF16 ? plan.ws.row_min : nullptr,
                                    dtype == PLANMOE_BF16 ? plan.ws.row_max : nullptr, plan.merged,
                                    plan.ws.hist_t, plan.ws.me_t, plan.groups, plan.ws.gstride, fill_blocks, counts,
-                                   plan.merged && plan.k * experts > 32, plain));
+                                   plan.merged && plan.k * experts > 32, out));
     return 0;
 }
 
@@ -1058,8 +1077,37 @@ extern "C" int planmoe_forward_plain(const void *x, const void *wg, int dtype, i
                        l_aux, expert_counts, workspace, st, plan, !plan.merged)) return 1;
     if (run_dispatch_routed(x, dtype, samples, model_dim, experts, capacity, indices, locations,
                             plane_stride, l_aux, expert_counts, (uint8_t *)dispatched, nullptr, nullptr, plan, st,
-                            true)) return 1;
+                            OUT_ROWS)) return 1;
     PM_LAUNCH_CHECK("planmoe_forward_plain");
+    return 0;
+}
+
+extern "C" int planmoe_layer_dispatch(const void *x, const void *wg, int dtype, int fp32_gate,
+                                      const float *logit_bias, int samples, int model_dim, int experts,
+                                      int top_k, int normalize_gate, int capacity, int codec, int32_t *indices,
+                                      int32_t *locations, void *gates, int64_t plane_stride,
+                                      void *scores_out, float *l_aux, int32_t *expert_counts, void *rows,
+                                      void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_layer_dispatch";
+    PM_REQUIRE(codec == 0 || codec == 1, "%s: codec is 0 (none) or 1 (int8)", who);
+    PM_REQUIRE(capacity >= 0 && (int64_t)experts * capacity < (1ll << 31), "%s: bad capacity", who);
+    if (fused_check(who, x, wg, dtype, samples, model_dim, experts, top_k, plane_stride)) return 1;
+    PM_REQUIRE(indices && locations && gates, "%s: NULL routing output", who);
+    PM_REQUIRE(rows || capacity == 0, "%s: NULL output", who);
+    PM_REQUIRE(aligned16(rows), "%s: the dispatched buffer must be 16-byte aligned", who);
+    PM_REQUIRE(workspace && workspace_bytes >= planmoe_forward_workspace_bytes(samples, experts, top_k), "%s: workspace too small", who);
+    workspace = fwd_tables(workspace);
+    hipStream_t st = (hipStream_t)stream;
+    FwdPlan plan;
+    fwd_plan(plan, workspace, samples, experts, top_k);
+    if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k, normalize_gate, indices,
+                       locations, gates, plane_stride, nullptr, scores_out, l_aux, expert_counts, workspace, st, plan,
+                       !plan.merged)) return 1;
+    if (run_dispatch_routed(x, dtype, samples, model_dim, experts, capacity, indices, locations, plane_stride, l_aux,
+                            expert_counts, (uint8_t *)rows, nullptr, nullptr, plan, st, codec ? OUT_DECODED : OUT_ROWS,
+                            false)) return 1;
+    PM_LAUNCH_CHECK(who);
     return 0;
 }
 

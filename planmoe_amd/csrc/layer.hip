@@ -1,0 +1,400 @@
+// The row passes of the layer whose experts' buffers never leave the GPU: combine and its backward
+// pass with the codec of the exchange in between, and the small reductions of the backward pass.
+//
+// On one rank the all-to-all delivers what was sent, so what "int8" does to a row is
+// decompress(compress(row)) (int8.cpp:10-24, 46-60).  The kernels here apply that to a row while it is
+// in registers -- the same roundings, the same values -- instead of writing codes that the next launch
+// decodes: the combine reads the experts' rows once (T k M values) where compress, then combine from the
+// codes, read E C M values, wrote and read their codes.  Only rows that hold a token are touched: empty
+// capacity slots are never written and never read.
+#include "rows.hpp"
+#include <type_traits>
+#include "int8_core.hpp"
+
+namespace pm {
+
+// decompress(compress(row)) of a row held as CACHE vectors per lane (vectors past the end: copies of the last)
+template <int DT, int CACHE, bool CANON>
+__device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
+{
+    using E = Elem<DT>;
+    RowStats<DT, CANON> stats;
+    stats.init();
+#pragma unroll
+    for (int c = 0; c < CACHE; ++c) stats.add(row[c]);
+    float mn, mx;
+    stats.finish(mn, mx);
+    const float scale = E::round(mx - mn);
+    const RowEncoder<DT> enc(mn, scale);
+    const RowDecoder<DT> dec(mn, scale);
+    auto body = [&](auto mode) {
+#pragma unroll
+        for (int c = 0; c < CACHE; ++c) {
+            uint32_t w[2];
+            float f[E::VEC];
+            enc.template encode<decltype(mode)::value>(row[c], w);
+#pragma unroll
+            for (int q = 0; q < E::VEC / 4; ++q) dec.word(w[q], f + 4 * q);
+            row[c] = E::pack(f);
+        }
+    };
+    if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
+}
+
+// out[t] = sum_j gate_j * codec(rows[slot_j]), planes left to right, one rounding at the end.
+// One wave per token; the rows of two choices are requested before either is used.  Bound by HBM: at 16384 x 4096 bf16, top-2,
+// codec int8 it moves 403 MB.
+template <int DT, int CACHE>
+__global__ __launch_bounds__(256) void layer_combine_kernel(
+    const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
+    const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples, int model_dim, int capacity,
+    void *__restrict__ out)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC;
+    const int lane = lane_id(), units = model_dim / V;
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= samples) return;
+    const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
+    auto request = [&](int s, uint4 (&r)[CACHE]) {
+        const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)max(s, 0) * row_bytes);
+#pragma unroll
+        for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
+    };
+    float acc[CACHE][V];
+    auto take = [&](bool first, int s, float g, uint4 (&r)[CACHE]) {
+        if (s >= 0) through_int8<DT, CACHE, false>(r);
+#pragma unroll
+        for (int c = 0; c < CACHE; ++c) {
+            float f[V];
+            E::unpack(r[c], f);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const float v = s >= 0 ? g * f[i] : 0.f;
+                acc[c][i] = first ? v : acc[c][i] + v;
+            }
+        }
+    };
+    for (int j0 = 0; j0 < top_k; j0 += WAVE) {
+        const int np = min(top_k - j0, WAVE);
+        int slot; float gate;
+        fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
+        for (int j = 0; j < np; j += 2) {
+            uint4 r0[CACHE], r1[CACHE];
+            const int s0 = rl_i(slot, j), s1 = j + 1 < np ? rl_i(slot, j + 1) : -1;
+            request(s0, r0);
+            request(s1, r1);
+            take(j0 + j == 0, s0, rl_f(gate, j), r0);
+            if (j + 1 < np) take(false, s1, rl_f(gate, j + 1), r1);
+        }
+    }
+    uint4 *dst = reinterpret_cast<uint4 *>((char *)out + (int64_t)t * row_bytes);
+#pragma unroll
+    for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(acc[c]));
+}
+
+// Backward of the combine: grad_gates_j = <grad[t], codec(rows[slot_j])> and grad_rows[slot_j] =
+// codec(round(gate_j * grad[t])) (GatingDecoder.backward, fast_dispatch.py:62-79, with the two codec
+// passes around it, overlap.py:19-34).
+template <int DT, int CACHE, bool INT8>
+__global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
+    const void *__restrict__ grad, const void *__restrict__ rows, const float *__restrict__ gates,
+    const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples,
+    int model_dim, int capacity, void *__restrict__ grad_rows, float *__restrict__ grad_gates)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC;
+    const int lane = lane_id(), units = model_dim / V;
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= samples) return;
+    const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
+    uint4 g_row[CACHE];
+    {
+        const uint4 *src = reinterpret_cast<const uint4 *>((const char *)grad + (int64_t)t * row_bytes);
+#pragma unroll
+        for (int c = 0; c < CACHE; ++c) g_row[c] = src[min(c * WAVE + lane, units - 1)];
+    }
+    for (int j0 = 0; j0 < top_k; j0 += WAVE) {
+        const int np = min(top_k - j0, WAVE);
+        int slot; float gate;
+        fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
+        if (lane < np && slot < 0) grad_gates[(int64_t)(j0 + lane) * stride + t] = 0.f;
+        for (int j = 0; j < np; ++j) {
+            const int s = rl_i(slot, j);
+            if (s < 0) continue;
+            const float g = rl_f(gate, j);
+            uint4 r[CACHE];
+            const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)s * row_bytes);
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
+            if constexpr (INT8) through_int8<DT, CACHE, false>(r);
+            float acc = 0.f;
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) {
+                float a[V], b[V];
+                E::unpack(g_row[c], a);
+                E::unpack(r[c], b);
+                if (c * WAVE + lane < units) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) acc = fmaf(b[i], a[i], acc);
+                }
+            }
+            acc = wave_sum(acc);
+            if (lane == 0) grad_gates[(int64_t)(j0 + j) * stride + t] = acc;
+            // the gradient row as the dispatcher stores it for this gate: round(0 + g * x)
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) {
+                float a[V];
+                E::unpack(g_row[c], a);
+#pragma unroll
+                for (int i = 0; i < V; ++i) a[i] = E::round(0.f + g * a[i]);
+                r[c] = E::pack(a);
+            }
+            if constexpr (INT8) through_int8<DT, CACHE, false>(r);
+            uint4 *dst = reinterpret_cast<uint4 *>((char *)grad_rows + (int64_t)s * row_bytes);
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, r[c]);
+        }
+    }
+}
+
+// Column sums of the rows in use of every batch: out[e][n] = sum_{r < rows_e} a[e][r][n] (the bias gradient).
+// A work-group takes 64 vectors of columns and a share of the rows, four rows at a time side by side; the
+// shares' sums go to `parts` and the second kernel adds them in order.
+template <int DT>
+__global__ __launch_bounds__(256) void rows_colsum_kernel(const void *__restrict__ a, const int *__restrict__ live, int live_planes,
+                                                          int live_round, int batches, int rows, int cols, int shares, float *__restrict__ parts)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC;
+    __shared__ float s_sum[4][WAVE][V + 1];
+    const int e = blockIdx.z, share = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6;
+    const int units = cols / V, u = blockIdx.x * WAVE + lane, uc = min(u, units - 1);
+    int used = rows;
+    if (live) {
+        int n = 0;
+        for (int j = 0; j < live_planes; ++j) n += live[j * batches + e];
+        used = min(rows, (n + live_round - 1) / live_round * live_round);
+    }
+    const int per = (used + shares - 1) / shares, r0 = share * per, r1 = min(used, r0 + per);
+    const uint4 *src = reinterpret_cast<const uint4 *>((const char *)a + (int64_t)e * rows * cols * (int64_t)sizeof(typename E::store_t));
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    constexpr int R = 4;
+    for (int r = r0 + wave * R; r < r1; r += 4 * R) {
+        uint4 v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = src[(int64_t)min(r + q, r1 - 1) * units + uc];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            float f[V];
+            E::unpack(v[q], f);
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] += r + q < r1 ? f[i] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) s_sum[wave][lane][i] = acc[i];
+    __syncthreads();
+    for (int x = threadIdx.x; x < WAVE * V; x += 256) {
+        const int l = x / V, i = x % V, col = (blockIdx.x * WAVE + l) * V + i;
+        if (col < cols) parts[((int64_t)e * shares + share) * cols + col] = s_sum[0][l][i] + s_sum[1][l][i] + s_sum[2][l][i] + s_sum[3][l][i];
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void parts_sum_kernel(const float *__restrict__ parts, int shares, int cols, void *__restrict__ out)
+{
+    const int e = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= cols) return;
+    float s = 0.f;
+    for (int i = 0; i < shares; ++i) s += parts[((int64_t)e * shares + i) * cols + c];
+    Elem<DT>::store(out, (int64_t)e * cols + c, s);
+}
+
+// Gate weight gradient: parts[share][e][m] = sum_{t in share} g[t][e] * x[t][m]; a work-group takes 64 vectors
+// of columns and a share of the tokens, its waves every fourth token; EP experts per pass.
+template <int DT, int EP>
+__global__ __launch_bounds__(256) void gate_dw_kernel(const void *__restrict__ x, const float *__restrict__ g, int samples, int model_dim,
+                                                      int experts, int e0, int shares, float *__restrict__ parts)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC;
+    __shared__ float s_sum[3][WAVE][EP * V + 1];
+    const int share = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6;
+    const int units = model_dim / V, u = blockIdx.x * WAVE + lane, uc = min(u, units - 1);
+    const int per = (samples + shares - 1) / shares, t0 = share * per, t1 = min(samples, t0 + per);
+    const uint4 *src = reinterpret_cast<const uint4 *>(x);
+    float acc[EP][V];
+#pragma unroll
+    for (int e = 0; e < EP; ++e)
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[e][i] = 0.f;
+    constexpr int R = 4;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    for (int t = t0 + wave_u * R; t < t1; t += 4 * R) {
+        uint4 v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = src[(int64_t)min(t + q, t1 - 1) * units + uc];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            float f[V];
+            E::unpack(v[q], f);
+            const int tq = min(t + q, t1 - 1);
+#pragma unroll
+            for (int e = 0; e < EP; ++e) {
+                // (uniform: scalar loads; g rounded to x's dtype first, as the cast before a library GEMM would)
+                const float ge = e0 + e < experts && t + q < t1 ? E::round(g[(int64_t)tq * experts + e0 + e]) : 0.f;
+#pragma unroll
+                for (int i = 0; i < V; ++i) acc[e][i] = fmaf(ge, f[i], acc[e][i]);
+            }
+        }
+    }
+    if (wave > 0)
+#pragma unroll
+        for (int e = 0; e < EP; ++e)
+#pragma unroll
+            for (int i = 0; i < V; ++i) s_sum[wave - 1][lane][e * V + i] = acc[e][i];
+    __syncthreads();
+    if (wave == 0 && u < units) {
+#pragma unroll
+        for (int e = 0; e < EP; ++e) {
+            if (e0 + e >= experts) break;
+            float *to = parts + ((int64_t)share * experts + e0 + e) * model_dim + (int64_t)u * V;
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                to[i] = acc[e][i] + s_sum[0][lane][e * V + i] + s_sum[1][lane][e * V + i] + s_sum[2][lane][e * V + i];
+        }
+    }
+}
+
+} // namespace pm
+
+using namespace pm;
+
+namespace {
+
+int rows_check(const char *who, int dtype, const void *rows, const int32_t *indices, const int32_t *locations, int64_t stride,
+               int top_k, int samples, int model_dim, int experts, int capacity, int codec)
+{
+    if (check_planes(who, indices, locations, stride, top_k, samples)) return 1;
+    PM_REQUIRE(dtype_ok(dtype), "%s: bad dtype %d", who, dtype);
+    PM_REQUIRE(codec == 0 || codec == 1, "%s: codec is 0 (none) or 1 (int8)", who);
+    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
+    PM_REQUIRE(model_dim >= 1 && model_dim % vec == 0 && model_dim <= 16 * WAVE * vec,
+               "%s: model_dim must be a multiple of %d, at most %d", who, vec, 16 * WAVE * vec);
+    PM_REQUIRE(capacity >= 1 && experts >= 1 && (int64_t)experts * capacity < (1ll << 31), "%s: bad capacity", who);
+    PM_REQUIRE((rows && aligned16(rows)) || samples == 0, "%s: NULL or unaligned rows", who);
+    return 0;
+}
+
+}  // namespace
+
+// the rows a wave keeps in registers: 1, 2, 4, 8 or 16 vectors per lane
+#define PM_ROW_CACHE(CALL)                                    \
+    do {                                                      \
+        if (per_lane <= 1) CALL(1);                           \
+        else if (per_lane <= 2) CALL(2);                      \
+        else if (per_lane <= 4) CALL(4);                      \
+        else if (per_lane <= 8) CALL(8);                      \
+        else CALL(16);                                        \
+    } while (0)
+
+extern "C" int planmoe_layer_combine(const void *rows, int dtype, int codec, const float *gates, const int32_t *indices,
+                                     const int32_t *locations, int64_t plane_stride, int top_k, int samples, int model_dim,
+                                     int experts, int capacity, void *out, void *stream)
+{
+    const char *who = "planmoe_layer_combine";
+    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
+    if (codec == 0) return planmoe_combine_fwd(rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, stream);
+    if (samples == 0) return 0;
+    PM_REQUIRE(out && aligned16(out), "%s: NULL or unaligned output", who);
+    const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
+    hipStream_t st = (hipStream_t)stream;
+#define PM_LC(CACHE) (layer_combine_kernel<DT, CACHE><<<(samples + 3) / 4, 256, 0, st>>>(rows, gates, indices, locations, \
+        plane_stride, top_k, samples, model_dim, capacity, out))
+    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LC));
+#undef PM_LC
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+extern "C" int planmoe_layer_combine_bwd(const void *grad, const void *rows, int dtype, int codec, const float *gates,
+                                         const int32_t *indices, const int32_t *locations, int64_t plane_stride, int top_k,
+                                         int samples, int model_dim, int experts, int capacity, void *grad_rows,
+                                         float *grad_gates, void *stream)
+{
+    const char *who = "planmoe_layer_combine_bwd";
+    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
+    if (samples == 0) return 0;
+    PM_REQUIRE(grad && grad_rows && grad_gates && gates && aligned16(grad) && aligned16(grad_rows), "%s: NULL or unaligned argument", who);
+    const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
+    hipStream_t st = (hipStream_t)stream;
+#define PM_LB_(CACHE, INT8) (layer_combine_bwd_kernel<DT, CACHE, INT8><<<(samples + 3) / 4, 256, 0, st>>>(grad, rows, gates, indices, \
+        locations, plane_stride, top_k, samples, model_dim, capacity, grad_rows, grad_gates))
+#define PM_LB(CACHE) do { if (codec) PM_LB_(CACHE, true); else PM_LB_(CACHE, false); } while (0)
+    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LB));
+#undef PM_LB
+#undef PM_LB_
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+// how many shares a reduction over `rows` is cut into for `blocks` column blocks: enough work-groups for the GPU, at least 32 rows each
+static int reduction_shares(int64_t rows, int64_t blocks)
+{
+    int64_t s = (1024 + blocks - 1) / blocks;
+    if (s > (rows + 31) / 32) s = (rows + 31) / 32;
+    return (int)(s < 1 ? 1 : s > 256 ? 256 : s);
+}
+
+extern "C" size_t planmoe_rows_colsum_workspace_bytes(int batches, int rows, int cols)
+{
+    if (batches < 1 || rows < 1 || cols < 1) return 16;
+    return (size_t)batches * reduction_shares(rows, (int64_t)batches * ((cols + 255) / 256)) * cols * 4;
+}
+
+extern "C" int planmoe_rows_colsum(const void *a, int dtype, int batches, int rows, int cols, const int32_t *live, int live_planes,
+                                   int live_round, void *out, void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_rows_colsum";
+    PM_REQUIRE(dtype_ok(dtype) && batches >= 1 && rows >= 1 && cols >= 1, "%s: bad shape", who);
+    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
+    PM_REQUIRE(cols % vec == 0 && a && out && aligned16(a), "%s: cols must be a multiple of %d, the rows 16-byte aligned", who, vec);
+    PM_REQUIRE(batches < 65536 && (!live || (live_planes >= 1 && live_round >= 1)), "%s: bad live rows", who);
+    PM_REQUIRE(workspace && workspace_bytes >= planmoe_rows_colsum_workspace_bytes(batches, rows, cols), "%s: workspace too small", who);
+    const int shares = reduction_shares(rows, (int64_t)batches * ((cols + 255) / 256));
+    const dim3 grid((unsigned)((cols / vec + WAVE - 1) / WAVE), (unsigned)shares, (unsigned)batches);
+    hipStream_t st = (hipStream_t)stream;
+    PM_DTYPE_SWITCH(dtype, DT,
+        (rows_colsum_kernel<DT><<<grid, 256, 0, st>>>(a, live, live_planes, live_round, batches, rows, cols, shares, (float *)workspace),
+         parts_sum_kernel<DT><<<dim3((unsigned)((cols + 255) / 256), (unsigned)batches), 256, 0, st>>>((const float *)workspace, shares, cols, out)));
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+extern "C" size_t planmoe_gate_dw_workspace_bytes(int samples, int model_dim, int experts)
+{
+    if (samples < 1 || model_dim < 1 || experts < 1) return 16;
+    return (size_t)reduction_shares(samples, (model_dim + 255) / 256) * experts * model_dim * 4;
+}
+
+extern "C" int planmoe_gate_dw(const void *x, int dtype, const float *grad_logits, int samples, int model_dim, int experts, void *out,
+                               void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_gate_dw";
+    PM_REQUIRE(dtype_ok(dtype) && samples >= 1 && model_dim >= 1 && experts >= 1, "%s: bad shape", who);
+    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
+    PM_REQUIRE(model_dim % vec == 0 && x && grad_logits && out && aligned16(x), "%s: model_dim must be a multiple of %d, x 16-byte aligned", who, vec);
+    PM_REQUIRE(workspace && workspace_bytes >= planmoe_gate_dw_workspace_bytes(samples, model_dim, experts), "%s: workspace too small", who);
+    const int shares = reduction_shares(samples, (model_dim + 255) / 256);
+    const dim3 grid((unsigned)((model_dim / vec + WAVE - 1) / WAVE), (unsigned)shares);
+    hipStream_t st = (hipStream_t)stream;
+    for (int e0 = 0; e0 < experts; e0 += 8)
+        PM_DTYPE_SWITCH(dtype, DT, (gate_dw_kernel<DT, 8><<<grid, 256, 0, st>>>(x, grad_logits, samples, model_dim, experts, e0, shares, (float *)workspace)));
+    PM_DTYPE_SWITCH(dtype, DT, (parts_sum_kernel<DT><<<dim3((unsigned)(((int64_t)experts * model_dim + 255) / 256), 1u), 256, 0, st>>>(
+        (const float *)workspace, shares, experts * model_dim, out)));
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}

@@ -1,4 +1,4 @@
-"""Loader of the torch C++ extension that carries the reference's pybind surface
+"""Loaders of the torch C++ extensions: the layer's host side, and the one that carries the reference's pybind surface
 (``schemoe_custom_kernel``: compress_operation / comm_operation / decompress_operation /
 clear_ptr_lst, and ``torch.ops.tutel_ops.cumsum``) on top of libplanmoe_hip.
 
@@ -18,7 +18,24 @@ from . import _lib  # noqa: F401  (loads libplanmoe_hip.so first; raises if it i
 _HERE = os.path.dirname(os.path.abspath(__file__))
 NAME = "schemoe_custom_kernel"
 PATH = os.path.join(_HERE, "csrc", "ext", NAME + sysconfig.get_config_var("EXT_SUFFIX"))
+LAYER_NAME = "_planmoe_layer"
+LAYER_PATH = os.path.join(_HERE, "csrc", "ext", LAYER_NAME + sysconfig.get_config_var("EXT_SUFFIX"))
 _module = None
+_layer = None
+
+
+def layer():
+    """The host side of the layer with its built-in experts (csrc/ext/layer.cpp)."""
+    global _layer
+    if _layer is None:
+        if not os.path.exists(LAYER_PATH):
+            raise ImportError("planmoe_amd: %s is missing; build it with "
+                              "python planmoe_amd/csrc/ext/build.py (or __graft_entry__.build())" % LAYER_PATH)
+        spec = importlib.util.spec_from_file_location(LAYER_NAME, LAYER_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _layer = mod
+    return _layer
 
 
 def load():

@@ -19,6 +19,7 @@ import torch
 
 from . import experts as _experts
 from . import gates as _gates
+from . import ext as _ext
 from . import losses, ops
 from . import overlap as _overlap
 from .fast_dispatch import extract_critical, fast_decode, fast_encode, route
@@ -152,7 +153,10 @@ class MOELayer(torch.nn.Module):
     # ------------------------------------------------------------------ forward
     def _deliver(self, y, l_aux, shape, dtype):
         """Common tail of every path (moe_layer.py:306-311)."""
-        y = y.view(list(shape)).to(dtype)
+        if y.shape != shape:
+            y = y.view(shape)
+        if y.dtype != dtype:
+            y = y.to(dtype)
         self.l_aux = y.l_aux = l_aux
         return self.result_func(y) if self.result_func is not None else y
 
@@ -165,9 +169,9 @@ class MOELayer(torch.nn.Module):
         shape, dtype = input.shape, input.dtype
         assert len(shape) >= 2, "Input data must be at least 2D tensor: (s)amples, .., (m)odel_dim"
         reserve_shape = shape[-reserve_dims:]
-        x = input.reshape(-1, reserve_shape.numel())
-        first = next(iter(self.experts.parameters()), None)
-        if first is not None:
+        x = input if len(shape) == 2 and reserve_dims == 1 else input.reshape(-1, reserve_shape.numel())
+        first = next(self.experts.parameters(), None)
+        if first is not None and x.dtype != first.dtype:
             x = x.to(first.dtype)
 
         gate = self.gates[gate_index]
@@ -197,6 +201,16 @@ class MOELayer(torch.nn.Module):
             kk = min(k, E)
             cap = ops.capacity(x.size(0), E, kk, cf, alignment)
             loss_dtype = torch.float32 if getattr(gate, 'fp32_gate', False) else x.dtype
+            codec = _overlap.native_codec(self, gate, x, degree, reserve_dims, cap)
+            if codec is not None:
+                # built-in gate and experts: the whole pass as one call and one node of the graph
+                count_step()
+                experts = self.experts
+                y, l_aux = _ext.layer().ffn_layer(x.contiguous(), gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias,
+                                                  experts.batched_fc2_w, experts.batched_fc2_bias, kk, cap, bool(gate.fp32_gate),
+                                                  bool(self.normalize_gate), codec)
+                self.protected_shape = torch.Size((E, cap, x.shape[1]))
+                return self._deliver(y, l_aux if l_aux.dtype == loss_dtype else l_aux.to(loss_dtype), shape, dtype)
             if _overlap.FUSE_GATE and _overlap.fused_gate_eligible(x, gate, E, self.compress_name, degree,
                                                                    self.is_postscore):
                 # gate GEMM, routing, encode and compress as one call; decompress + decode in one pass

@@ -731,6 +731,56 @@ def gemm_tn_bf16(a, b, out=None):
     return out
 
 
+_FORMS = {'nn': 0, 'nt': 1, 'tn': 2}
+
+
+def expert_gemm(form, a, b, bias=None, relu=False, live=None, live_round=1, rows_hint=0, out=None):
+    """The experts' batched products, bf16 or fp32 (planmoe_expert_gemm): 'nn' act(a @ b + bias), 'nt' a @ b^T,
+    'tn' a^T @ b; a, b contiguous [batches, ., .].  live: int32 [planes, batches], the rows in use of every
+    batch (rows of the result beyond them are left as they are; 'tn': the rows of a and b to sum over)."""
+    _need_gpu(a, "expert_gemm")
+    a, b = _contig(a, "expert_gemm"), _contig(b, "expert_gemm")
+    if a.dtype != b.dtype or a.dim() != 3 or b.dim() != 3 or a.shape[0] != b.shape[0]:
+        raise PlanMoEError("expert_gemm: two [batches, ., .] operands of one dtype")
+    B = a.shape[0]
+    k, m = (a.shape[1], a.shape[2]) if form == 'tn' else (a.shape[2], a.shape[1])
+    kb, n = (b.shape[2], b.shape[1]) if form == 'nt' else (b.shape[1], b.shape[2])
+    if k != kb:
+        raise PlanMoEError("expert_gemm: operands disagree: a %s, b %s" % (tuple(a.shape), tuple(b.shape)))
+    if bias is not None:
+        bias = _contig(bias.to(a.dtype), "expert_gemm")
+        if tuple(bias.shape) != (B, n):
+            raise PlanMoEError("expert_gemm: bias must be [batches, n]")
+    if live is not None and (live.dtype != torch.int32 or live.dim() != 2 or live.shape[1] != B or not live.is_contiguous()):
+        raise PlanMoEError("expert_gemm: live must be a contiguous int32 [planes, batches] tensor")
+    if out is None:
+        out = torch.empty((B, m, n), dtype=a.dtype, device=a.device)
+    elif tuple(out.shape) != (B, m, n) or out.dtype != a.dtype or not out.is_contiguous():
+        raise PlanMoEError("expert_gemm: out must be a contiguous [batches, m, n] tensor")
+    check(lib.planmoe_expert_gemm(_FORMS[form], _dt(a, "expert_gemm"), _ptr(a), _ptr(b), _ptr(bias), int(bool(relu)), B, m, n, k,
+                                  _ptr(live), 1 if live is None else live.shape[0], int(live_round), int(rows_hint), _ptr(out),
+                                  _stream(a)))
+    return out
+
+
+def expert_gemm_relu_bwd(a, b, h, live=None, live_round=1, rows_hint=0, out=None):
+    """(c, dbias): c = a @ b^T where h > 0, else 0; dbias its column sums (planmoe_expert_gemm_relu_bwd)."""
+    _need_gpu(a, "expert_gemm_relu_bwd")
+    a, b, h = _contig(a, "expert_gemm_relu_bwd"), _contig(b, "expert_gemm_relu_bwd"), _contig(h, "expert_gemm_relu_bwd")
+    B, m, k = a.shape
+    n = b.shape[1]
+    if a.dtype != b.dtype or a.dtype != h.dtype or tuple(b.shape) != (B, n, k) or tuple(h.shape) != (B, m, n):
+        raise PlanMoEError("expert_gemm_relu_bwd: operands disagree")
+    if out is None:
+        out = torch.empty((B, m, n), dtype=a.dtype, device=a.device)
+    dbias = torch.empty((B, n), dtype=a.dtype, device=a.device)
+    ws = _ws(lib.planmoe_expert_gemm_relu_bwd_workspace_bytes(B, m, n), a.device)
+    check(lib.planmoe_expert_gemm_relu_bwd(_dt(a, "expert_gemm_relu_bwd"), _ptr(a), _ptr(b), _ptr(h), B, m, n, k, _ptr(live),
+                                           1 if live is None else live.shape[0], int(live_round), int(rows_hint), _ptr(out),
+                                           _ptr(dbias), _ptr(ws), ws.numel(), _stream(a)))
+    return out, dbias
+
+
 # ------------------------------------------------------------------------------ zfp codec
 def zfp_stream_bytes(dims, nx, ny, rate=8.0):
     return int(lib.planmoe_zfp_stream_bytes(dims, nx, ny, float(rate)))

@@ -144,6 +144,47 @@ def ffn_from_codes_fn(module, x, degree, reserve_dims):
     return module.forward_from_codes
 
 
+# the layer with its built-in experts (relu between the two products) as one node driven from C++
+# (csrc/ext/layer.cpp): the same routing and the same codec values, products over the rows in use only
+NATIVE_LAYER = True
+_NATIVE_CODECS = {'int8': 1, 'zfp': 2, 'lz': 3}
+
+
+def _hooked(module):
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def native_codec(layer, gate, x, degree, reserve_dims, capacity):
+    """The codec number for csrc/ext/layer.cpp when the whole layer is its business, else None.  What is left to
+    the steps below: experts or gates that are not the built-in ones or carry hooks, other dtypes (a gate in
+    fp32 next to 16-bit rows among them), overlap slices, autocast, and every option that asks for the
+    reference's structure."""
+    from .experts import FusedExpertsNetwork
+    from .gates import LinearTopKGate
+    experts = layer.experts
+    if not (NATIVE_LAYER and FUSE_GATE and FUSE_INT8 and FUSE_ZFP and not FFN_FROM_CODES and not _ck.SINGLE_RANK_COMM_COPIES and
+            degree == 1 and reserve_dims == 1 and layer.is_postscore and x.is_cuda and capacity >= 1 and x.shape[0] >= 1 and
+            type(experts) is FusedExpertsNetwork and experts._relu and type(gate) is LinearTopKGate and
+            layer.num_global_experts <= 64):
+        return None
+    dtype, M, H = x.dtype, x.shape[1], experts.hidden_size_per_expert
+    vec = 8 if dtype == torch.bfloat16 else 4
+    if not ((dtype == torch.bfloat16 or dtype == torch.float32) and M % vec == 0 and H % vec == 0 and M <= 1024 * vec and
+            experts.output_dim in (None, M)):
+        return None
+    for p in (gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias):
+        if p.dtype != dtype or not p.is_contiguous():
+            return None
+    if _hooked(experts) or _hooked(gate) or torch.is_autocast_enabled(x.device.type):
+        return None
+    codec = _NATIVE_CODECS.get(layer.compress_name, 0)
+    if codec == 2 and not fused_zfp_eligible(x, 'zfp', degree, True, layer.num_global_experts, capacity):
+        return None
+    if codec == 3 and (dtype != torch.float32 or 'lz' in _ck.registered()):
+        return None
+    return codec
+
+
 class _GaveUp:
     """The give-up flag of a one-launch forward on its way to the host without stalling the stream:
     an asynchronous copy into pinned memory and an event behind it.  Asked at the end of the
