@@ -42,9 +42,11 @@ __device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
 }
 
 // out[t] = sum_j gate_j * codec(rows[slot_j]), planes left to right, one rounding at the end.
-// One wave per token; the rows of two choices are requested before either is used.  Bound by HBM: at 16384 x 4096 bf16, top-2,
-// codec int8 it moves 403 MB.
-template <int DT, int CACHE>
+// One wave per token; the rows of two choices are requested before either is used and stay as they lie in
+// memory until both have been through the codec (two 8 KB rows and their sum in fp32 took 230 registers
+// and left two waves per SIMD: 112 us at 16384 x 4096 bf16, top-2, for 403 MB).  More than two choices
+// keep their sum in fp32.
+template <int DT, int CACHE, bool TWO>
 __global__ __launch_bounds__(256) void layer_combine_kernel(
     const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
     const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples, int model_dim, int capacity,
@@ -56,39 +58,65 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= samples) return;
     const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
+    uint4 *dst = reinterpret_cast<uint4 *>((char *)out + (int64_t)t * row_bytes);
     auto request = [&](int s, uint4 (&r)[CACHE]) {
         const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)max(s, 0) * row_bytes);
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
     };
-    float acc[CACHE][V];
-    auto take = [&](bool first, int s, float g, uint4 (&r)[CACHE]) {
-        if (s >= 0) through_int8<DT, CACHE, false>(r);
+    if constexpr (TWO) {
+        int slot; float gate;
+        fetch_planes(gates, indices, locations, stride, t, 0, top_k, 0x7fffffff, capacity, slot, gate);
+        uint4 r0[CACHE], r1[CACHE];
+        const int s0 = rl_i(slot, 0), s1 = top_k > 1 ? rl_i(slot, 1) : -1;
+        const float g0 = rl_f(gate, 0), g1 = rl_f(gate, 1);
+        request(s0, r0);
+        if (s1 >= 0) request(s1, r1);
+        if (s0 >= 0) through_int8<DT, CACHE, false>(r0);
+        if (s1 >= 0) through_int8<DT, CACHE, false>(r1);
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) {
-            float f[V];
-            E::unpack(r[c], f);
+            float f[V], h[V];
+            E::unpack(r0[c], f);
 #pragma unroll
-            for (int i = 0; i < V; ++i) {
-                const float v = s >= 0 ? g * f[i] : 0.f;
-                acc[c][i] = first ? v : acc[c][i] + v;
+            for (int i = 0; i < V; ++i) f[i] = s0 >= 0 ? g0 * f[i] : 0.f;
+            if (top_k > 1) {
+                if (s1 >= 0) {
+                    E::unpack(r1[c], h);
+#pragma unroll
+                    for (int i = 0; i < V; ++i) f[i] += g1 * h[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) f[i] += 0.f;
+                }
             }
+            if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(f));
         }
-    };
+        return;
+    }
+    float acc[CACHE][V];
     for (int j0 = 0; j0 < top_k; j0 += WAVE) {
         const int np = min(top_k - j0, WAVE);
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
-        for (int j = 0; j < np; j += 2) {
-            uint4 r0[CACHE], r1[CACHE];
-            const int s0 = rl_i(slot, j), s1 = j + 1 < np ? rl_i(slot, j + 1) : -1;
-            request(s0, r0);
-            request(s1, r1);
-            take(j0 + j == 0, s0, rl_f(gate, j), r0);
-            if (j + 1 < np) take(false, s1, rl_f(gate, j + 1), r1);
+        for (int j = 0; j < np; ++j) {
+            uint4 r[CACHE];
+            const int s = rl_i(slot, j);
+            const float g = rl_f(gate, j);
+            request(s, r);
+            if (s >= 0) through_int8<DT, CACHE, false>(r);
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) {
+                float f[V];
+                E::unpack(r[c], f);
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const float v = s >= 0 ? g * f[i] : 0.f;
+                    acc[c][i] = j0 + j == 0 ? v : acc[c][i] + v;
+                }
+            }
         }
     }
-    uint4 *dst = reinterpret_cast<uint4 *>((char *)out + (int64_t)t * row_bytes);
 #pragma unroll
     for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(acc[c]));
 }
@@ -119,14 +147,22 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
         if (lane < np && slot < 0) grad_gates[(int64_t)(j0 + lane) * stride + t] = 0.f;
+        // the next choice's row is on its way while this one's is worked on (a dropped choice reads slot 0, unused)
+        uint4 next[CACHE];
+        auto request = [&](int j) {
+            const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)max(rl_i(slot, j), 0) * row_bytes);
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) next[c] = src[min(c * WAVE + lane, units - 1)];
+        };
+        request(0);
         for (int j = 0; j < np; ++j) {
             const int s = rl_i(slot, j);
-            if (s < 0) continue;
             const float g = rl_f(gate, j);
             uint4 r[CACHE];
-            const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)s * row_bytes);
 #pragma unroll
-            for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
+            for (int c = 0; c < CACHE; ++c) r[c] = next[c];
+            if (j + 1 < np) request(j + 1);
+            if (s < 0) continue;
             if constexpr (INT8) through_int8<DT, CACHE, false>(r);
             float acc = 0.f;
 #pragma unroll
@@ -203,14 +239,26 @@ __global__ __launch_bounds__(256) void rows_colsum_kernel(const void *__restrict
     }
 }
 
+// out[e][c] = sum over the shares, in order within a wave's quarter: 64 columns per work-group, eight loads in flight
+// (a thread per column that walked the shares one by one took 35 us for 256 shares of 8 x 1024)
 template <int DT>
 __global__ __launch_bounds__(256) void parts_sum_kernel(const float *__restrict__ parts, int shares, int cols, void *__restrict__ out)
 {
-    const int e = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= cols) return;
+    __shared__ float s_sum[4][WAVE];
+    const int e = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6, c = blockIdx.x * WAVE + lane;
+    const float *from = parts + (int64_t)e * shares * cols + min(c, cols - 1);
+    const int per = (shares + 3) / 4, i1 = min(shares, (wave + 1) * per);
     float s = 0.f;
-    for (int i = 0; i < shares; ++i) s += parts[((int64_t)e * shares + i) * cols + c];
-    Elem<DT>::store(out, (int64_t)e * cols + c, s);
+    for (int i = wave * per; i < i1; i += 8) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = from[(int64_t)min(i + q, i1 - 1) * cols];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += i + q < i1 ? v[q] : 0.f;
+    }
+    s_sum[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && c < cols) Elem<DT>::store(out, (int64_t)e * cols + c, s_sum[0][lane] + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane]);
 }
 
 // Gate weight gradient: parts[share][e][m] = sum_{t in share} g[t][e] * x[t][m]; a work-group takes 64 vectors
@@ -312,10 +360,12 @@ extern "C" int planmoe_layer_combine(const void *rows, int dtype, int codec, con
     PM_REQUIRE(out && aligned16(out), "%s: NULL or unaligned output", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
     hipStream_t st = (hipStream_t)stream;
-#define PM_LC(CACHE) (layer_combine_kernel<DT, CACHE><<<(samples + 3) / 4, 256, 0, st>>>(rows, gates, indices, locations, \
+#define PM_LC_(CACHE, TWO) (layer_combine_kernel<DT, CACHE, TWO><<<(samples + 3) / 4, 256, 0, st>>>(rows, gates, indices, locations, \
         plane_stride, top_k, samples, model_dim, capacity, out))
+#define PM_LC(CACHE) do { if (top_k <= 2) PM_LC_(CACHE, true); else PM_LC_(CACHE, false); } while (0)
     PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LC));
 #undef PM_LC
+#undef PM_LC_
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -369,7 +419,7 @@ extern "C" int planmoe_rows_colsum(const void *a, int dtype, int batches, int ro
     hipStream_t st = (hipStream_t)stream;
     PM_DTYPE_SWITCH(dtype, DT,
         (rows_colsum_kernel<DT><<<grid, 256, 0, st>>>(a, live, live_planes, live_round, batches, rows, cols, shares, (float *)workspace),
-         parts_sum_kernel<DT><<<dim3((unsigned)((cols + 255) / 256), (unsigned)batches), 256, 0, st>>>((const float *)workspace, shares, cols, out)));
+         parts_sum_kernel<DT><<<dim3((unsigned)((cols + WAVE - 1) / WAVE), (unsigned)batches), 256, 0, st>>>((const float *)workspace, shares, cols, out)));
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -393,7 +443,7 @@ extern "C" int planmoe_gate_dw(const void *x, int dtype, const float *grad_logit
     hipStream_t st = (hipStream_t)stream;
     for (int e0 = 0; e0 < experts; e0 += 8)
         PM_DTYPE_SWITCH(dtype, DT, (gate_dw_kernel<DT, 8><<<grid, 256, 0, st>>>(x, grad_logits, samples, model_dim, experts, e0, shares, (float *)workspace)));
-    PM_DTYPE_SWITCH(dtype, DT, (parts_sum_kernel<DT><<<dim3((unsigned)(((int64_t)experts * model_dim + 255) / 256), 1u), 256, 0, st>>>(
+    PM_DTYPE_SWITCH(dtype, DT, (parts_sum_kernel<DT><<<dim3((unsigned)(((int64_t)experts * model_dim + WAVE - 1) / WAVE), 1u), 256, 0, st>>>(
         (const float *)workspace, shares, experts * model_dim, out)));
     PM_LAUNCH_CHECK(who);
     return 0;

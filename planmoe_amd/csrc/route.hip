@@ -312,13 +312,13 @@ __global__ __launch_bounds__(TILE) void route_finish_kernel(
 //   l_aux = sum_e me[e] ce[e] / T            =>  ds[t][e] += dl * ce[e] / T,  ce[e] = count0[e] * E / T
 //   softmax: dlogit_e = s_e * (ds_e - sum_i ds_i s_i)
 template <int DT>
-__global__ __launch_bounds__(256) void route_bwd_kernel(
+__global__ __launch_bounds__(64) void route_bwd_kernel(
     const void *__restrict__ scores, const int32_t *__restrict__ indices, const void *__restrict__ dgates,
     int64_t stride, int samples, int experts, int k, int normalize_gate, const float *__restrict__ dl_aux,
     const int32_t *__restrict__ count0, int through_softmax, void *__restrict__ dscores)
 {
     using E = Elem<DT>;
-    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int t = blockIdx.x * 64 + threadIdx.x;          // (a wave per work-group: a thread's few hundred dependent loads want many of them)
     if (t >= samples) return;
     const int64_t base = (int64_t)t * experts;
     const float dl = dl_aux ? dl_aux[0] : 0.f;
@@ -459,7 +459,7 @@ extern "C" int planmoe_route_bwd(const void *scores, int dtype, const int32_t *i
     PM_REQUIRE(scores && indices && grad_gates && grad_scores, "planmoe_route_bwd: NULL argument");
     const int k = top_k < experts ? top_k : experts;
     PM_DTYPE_SWITCH(dtype, DT,
-        (route_bwd_kernel<DT><<<(samples + 255) / 256, 256, 0, (hipStream_t)stream>>>(
+        (route_bwd_kernel<DT><<<(samples + 63) / 64, 64, 0, (hipStream_t)stream>>>(
             scores, indices, grad_gates, plane_stride, samples, experts, k, normalize_gate, grad_l_aux,
             grad_l_aux ? first_choice_counts : nullptr, through_softmax, grad_scores)));
     PM_LAUNCH_CHECK("planmoe_route_bwd");
