@@ -12,6 +12,8 @@
 //             dW = x^T @ dy        A = x  [rows, in],   B = dy [rows, out]    planmoe_gemm_tn_bf16
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
+#include "gemm_skinny.hpp"
+#include <cmath>
 
 namespace pm {
 
@@ -65,13 +67,15 @@ struct GemmArgs {
     const uint16_t *A, *B, *bias;
     const uint16_t *mask;         // GRAD: c is kept where mask > 0 (c's shape and pitches), else zero
     uint16_t *C;
-    float *colsum;                // GRAD: [batches][2 tile rows][N] column sums of what was stored, NULL: none
+    float *colsum;                // GRAD: [batches][2 ceil(M / 128)][N] column sums of what was stored, by 128 rows and wave row, NULL: none
     const int *live;              // [live_planes][batches]: rows in use per batch (k of a tn product), NULL: all
     int live_planes, live_round;
     int M, N, K;
     int lda, ldb, ldc;            // elements between rows
     int64_t sA, sB, sC;           // elements between batches
     int batches, relu;
+    int split;                    // 0: all tiles; 1: all but the last round's (gemm_last_round); 2: those, as quarters
+    int stay;                     // work-groups of the 256 x 256 launch
     bool bias_by_value;           // the bias is not 16-byte aligned: read where it is used
 };
 
@@ -80,6 +84,12 @@ __device__ __forceinline__ gemm_u32x4 gemm_desc(const void *base, int64_t bytes)
     const uint64_t a = (uint64_t)base;
     const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffff ? 0x7fffffffu : (uint32_t)bytes;
     return gemm_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, n, 0x00020000u};
+}
+// how many of the 256 x 256 tiles, on work-groups that stay, would be left for a last round that is at most half full
+__host__ __device__ inline int gemm_last_round(int tiles, int stay)
+{
+    const int last = tiles % stay;
+    return 2 * last <= stay ? last : 0;
 }
 constexpr uint32_t GEMM_NOWHERE = 0x80000000u;              // an offset that is out of any descriptor's range
 // 16 bytes per lane from the buffer at voff + soff to LDS at lds_addr + 16 * lane
@@ -134,15 +144,17 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
     // eighth of the tiles in a row, in the order batch, panel of 8 tile columns, tile row, column, so
     // that the tiles it works on at a time share operands (12 operand tiles for 32 products at 256 x 256).
     // With `live` the tiles of a batch are those of its rows in use: table[e] is the number before batch e.
-    const int tiles_n = (p.N + S::BN - 1) / S::BN;
-    int total;
+    static_assert(I == J, "square tiles");
+    const int side = p.split == 2 ? 256 : S::BM;            // (of the tiles that are counted)
+    const int tiles_n = (p.N + side - 1) / side;
+    int total, base = 0;
     int *table = reinterpret_cast<int *>(lds + S::TABLE);
     if (p.live) {
         int n = 0;
         if (lane < p.batches)
             for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + lane];
         const int rows = min(TA ? p.K : p.M, (n + p.live_round - 1) / p.live_round * p.live_round);
-        const int mine = lane < p.batches ? ((TA ? p.M : rows) + S::BM - 1) / S::BM * tiles_n : 0;
+        const int mine = lane < p.batches ? ((TA ? p.M : rows) + side - 1) / side * tiles_n : 0;
         int inc = mine;
         for (int d = 1; d < 64; d <<= 1) {
             const int o = __shfl_up(inc, d);
@@ -153,13 +165,19 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         table[64 + lane] = rows;
         total = __builtin_amdgcn_readlane(inc, 63);
     } else {
-        total = (p.M + S::BM - 1) / S::BM * tiles_n * p.batches;
+        total = (p.M + side - 1) / side * tiles_n * p.batches;
+    }
+    if (p.split == 1) total -= gemm_last_round(total, p.stay);
+    if (p.split == 2) {
+        const int last = gemm_last_round(total, p.stay);
+        base = total - last;
+        total = 4 * last;
     }
     const int per_xcd = (total + 7) / 8;
     const int first_tile = blockIdx.x % 8 * per_xcd, stride = gridDim.x / 8;
     struct Where { int e, m0, n0, rows; };        // rows: M of the batch (its K for a tn product)
     auto locate = [&](int j) {                    // j-th tile of this XCD (in range)
-        const int tile = first_tile + j;
+        const int number = first_tile + j, tile = p.split == 2 ? base + number / 4 : number;
         Where w;
         int first, tm;
         if (p.live) {
@@ -168,9 +186,9 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
             w.e = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before <= tile)) - 1);
             first = __builtin_amdgcn_readlane(before, w.e);
             w.rows = __builtin_amdgcn_readlane(rows, w.e);
-            tm = ((TA ? p.M : w.rows) + S::BM - 1) / S::BM;
+            tm = ((TA ? p.M : w.rows) + side - 1) / side;
         } else {
-            tm = (p.M + S::BM - 1) / S::BM;
+            tm = (p.M + side - 1) / side;
             w.e = tile / (tm * tiles_n);
             first = w.e * tm * tiles_n;
             w.rows = TA ? p.K : p.M;
@@ -179,8 +197,8 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         const int panel = in / (tm * 8);
         in -= panel * tm * 8;
         const int width = min(8, tiles_n - panel * 8);
-        w.m0 = in / width * S::BM;
-        w.n0 = (panel * 8 + in % width) * S::BN;
+        w.m0 = in / width * side + (p.split == 2 ? (number & 2) * 64 : 0);
+        w.n0 = (panel * 8 + in % width) * side + (p.split == 2 ? (number & 1) * 128 : 0);
         return w;
     };
     auto in_range = [&](int j) { return j < per_xcd && first_tile + j < total; };
@@ -354,45 +372,45 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
     };
     ask_bias();
 
-    // where a lane's 16-byte pieces go, from the tile's corner; the uniform part of a piece's place is the store's scalar offset
-    const int put_col = wn * 32 * J + lane % (4 * J) * 8;
-    const uint32_t put = ((uint32_t)(wm * 32 * I + lane / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
     auto finish = [&] {                           // the results of the tile to memory
+        // (the lane number is hidden from the compiler: what follows from it is worked out here once per tile
+        // instead of in registers that the loop over k needs)
+        int l = lane;
+        asm volatile("" : "+v"(l));
         uint8_t *piece = lds + S::OPERANDS + wave * (32 * S::PITCH);
-        const uint8_t *get = piece + lane / (4 * J) * S::PITCH + lane % (4 * J) * 16;
-        uint8_t *lay = piece + fr * S::PITCH + fc * 8;
+        const uint8_t *get = piece + l / (4 * J) * S::PITCH + l % (4 * J) * 16;
+        uint8_t *lay = piece + (l & 31) * S::PITCH + (l >> 5) * 8;
+        // where a lane's 16-byte pieces go, from the tile's corner; the uniform part of a piece's place is the store's scalar offset
+        const int put_col = wn * 32 * J + l % (4 * J) * 8;
+        const uint32_t put = ((uint32_t)(wm * 32 * I + l / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
         const int M = TA ? p.M : here.rows;
         const int64_t corner = (int64_t)here.e * p.sC + (int64_t)here.m0 * p.ldc + here.n0;
         const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2);
         const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t mask = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(GRAD ? p.mask + corner : p.C), 0, GRAD ? bytes : 0, 0x00020000);
-        const uint32_t put0 = here.n0 + put_col < p.N ? put : GEMM_NOWHERE, put1 = here.n0 + 64 * J + put_col < p.N ? put : GEMM_NOWHERE;
-        float add[2][8];                          // bias of the lane's columns (GRAD: their sums)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b) {
+            const uint32_t put_b = here.n0 + 64 * J * b + put_col < p.N ? put : GEMM_NOWHERE;
+            float add[8];                         // bias of the lane's columns (GRAD: their sums)
 #pragma unroll
-            for (int x = 0; x < 8; ++x) add[b][x] = 0.f;
-        if (!GRAD && p.bias) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
+            for (int x = 0; x < 8; ++x) add[x] = 0.f;
+            if (!GRAD && p.bias) {
                 if (p.bias_by_value) {
-                    for (int x = 0; x < 8; ++x) add[b][x] = bf16_to_f32(p.bias[(int64_t)here.e * p.N + min(here.n0 + 64 * J * b + put_col + x, p.N - 1)]);
-                    continue;
+#pragma unroll
+                    for (int x = 0; x < 8; ++x) add[x] = bf16_to_f32(p.bias[(int64_t)here.e * p.N + min(here.n0 + 64 * J * b + put_col + x, p.N - 1)]);
+                } else {
+                    Elem<PLANMOE_BF16>::unpack(*reinterpret_cast<const uint4 *>(lds + S::BIAS + turn * 1024 + (64 * J * b + put_col) * 2), add);
                 }
-                Elem<PLANMOE_BF16>::unpack(*reinterpret_cast<const uint4 *>(lds + S::BIAS + turn * 1024 + (64 * J * b + put_col) * 2), add[b]);
             }
-        }
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+            for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int i = 0; i < I; ++i)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
+                for (int i = 0; i < I; ++i) {
                     auto so = [&](int t) { return ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u; };
                     pm_u32x4 keep[2 * J];
                     if (GRAD)
 #pragma unroll
-                        for (int t = 0; t < 2 * J; ++t) keep[t] = __builtin_amdgcn_raw_buffer_load_b128(mask, b ? put1 : put0, so(t), 0);
+                        for (int t = 0; t < 2 * J; ++t) keep[t] = __builtin_amdgcn_raw_buffer_load_b128(mask, put_b, so(t), 0);
 #pragma unroll
                     for (int jj = 0; jj < J; ++jj)
                         asm volatile("" : "+a"(acc[a][b][i][jj]));      // (in the accumulator registers until here: copied all at once they would not fit)
@@ -411,7 +429,7 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
                         if (!GRAD && p.bias) {    // the matmul's rounding is done; torch.add in bf16
 #pragma unroll
                             for (int x = 0; x < 4; ++x)
-                                v[x] = f32x2_to_bf16x2(__uint_as_float(v[x] << 16) + add[b][2 * x], __uint_as_float(v[x] & 0xffff0000u) + add[b][2 * x + 1]);
+                                v[x] = f32x2_to_bf16x2(__uint_as_float(v[x] << 16) + add[2 * x], __uint_as_float(v[x] & 0xffff0000u) + add[2 * x + 1]);
                         }
                         if (!GRAD && p.relu) {    // (negative bf16 are negative int16; a NaN stays)
 #pragma unroll
@@ -425,28 +443,36 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
                             for (int x = 0; x < 4; ++x) {
                                 const uint32_t k = keep[t][x];
                                 v[x] &= ((int)(k << 16) > 0 ? 0xffffu : 0u) | ((int)k >= 0x10000 ? 0xffff0000u : 0u);
-                                add[b][2 * x] += __uint_as_float(v[x] << 16);
-                                add[b][2 * x + 1] += __uint_as_float(v[x] & 0xffff0000u);
+                                add[2 * x] += __uint_as_float(v[x] << 16);
+                                add[2 * x + 1] += __uint_as_float(v[x] & 0xffff0000u);
+                                // (added here: moved to where the sums are wanted, the additions would keep every value of the tile alive)
+                                asm volatile("" : "+v"(add[2 * x]), "+v"(add[2 * x + 1]));
                             }
                         }
-                        __builtin_amdgcn_raw_buffer_store_b128(v, out, b ? put1 : put0, so(t), 0);
+                        __builtin_amdgcn_raw_buffer_store_b128(v, out, put_b, so(t), 0);
+                        if (GRAD) __builtin_amdgcn_sched_barrier(0);         // (one piece's temporaries at a time: the registers are full)
                     }
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_sched_barrier(0);
                 }
-        if (GRAD && p.colsum) {
+            if (GRAD && p.colsum) {
+                // the 16 / J lanes that hold a column meet in the wave's piece of LDS
+                float *sums = reinterpret_cast<float *>(piece);
+                *reinterpret_cast<float4 *>(sums + l * 8) = make_float4(add[0], add[1], add[2], add[3]);
+                *reinterpret_cast<float4 *>(sums + l * 8 + 4) = make_float4(add[4], add[5], add[6], add[7]);
+                __builtin_amdgcn_wave_barrier();
+                float s = 0.f;
+                const int c = l % (32 * J);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-#pragma unroll
-                for (int x = 0; x < 8; ++x)
-#pragma unroll
-                    for (int d = 4 * J; d < 64; d <<= 1) add[b][x] += __shfl_xor(add[b][x], d);
-                if (lane < 4 * J && here.n0 + 64 * J * b + put_col < p.N) {
-                    const int slots = (p.M + S::BM - 1) / S::BM * 2;
-                    float *to = p.colsum + ((int64_t)here.e * slots + here.m0 / S::BM * 2 + wm) * p.N + here.n0 + 64 * J * b + put_col;
-#pragma unroll
-                    for (int x = 0; x < 8; x += 4) *reinterpret_cast<float4 *>(to + x) = make_float4(add[b][x], add[b][x + 1], add[b][x + 2], add[b][x + 3]);
+                for (int r = 0; r < 16 / J; ++r) s += sums[(c / 8 + 4 * J * r) * 8 + c % 8];
+                const int col = here.n0 + 64 * J * b + wn * 32 * J + c, slots = (p.M + 127) / 128 * 2, slot = here.m0 / 128 * 2 + wm;
+                if (l < 32 * J && col < p.N && slot < slots) {
+                    float *to = p.colsum + ((int64_t)here.e * slots + slot) * p.N + col;
+                    to[0] = s;
+                    if (I == 2 && slot + 2 < slots) to[2 * (int64_t)p.N] = 0.f;        // (a tile of 256 rows: all in the first slot)
                 }
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -489,24 +515,34 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 #undef PM_PHASE
 }
 
-// the column sums of the tiles of a batch, in tile order, as the bias gradient
+// the column sums of the tiles of a batch, in order, as the bias gradient: 64 columns per
+// work-group, its waves every fourth slot, eight loads in flight
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restrict__ parts, const int *__restrict__ live, int live_planes,
-                                                          int live_round, int batches, int M, int N, int BM, void *__restrict__ out)
+                                                          int live_round, int batches, int M, int N, int BM, int slots,
+                                                          void *__restrict__ out)
 {
-    const int e = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x, slots = (M + BM - 1) / BM * 2;
+    __shared__ float s_sum[4][64];
+    const int e = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
     int rows = M;
     if (live) {
         int c = 0;
         for (int j = 0; j < live_planes; ++j) c += live[j * batches + e];
         rows = min(M, (c + live_round - 1) / live_round * live_round);
     }
-    if (n >= N) return;
-    const int used = (rows + BM - 1) / BM * 2;
-    const float *from = parts + (int64_t)e * slots * N + n;
+    const int used = min(slots, (rows + BM - 1) / BM * 2);
+    const float *from = parts + (int64_t)e * slots * N + min(n, N - 1);
     float s = 0.f;
-    for (int i = 0; i < used; ++i) s += from[(int64_t)i * N];
-    Elem<DT>::store(out, (int64_t)e * N + n, s);
+    for (int i0 = wave * 8; i0 < used; i0 += 32) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = from[(int64_t)min(i0 + q, used - 1) * N];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += i0 + q < used ? v[q] : 0.f;
+    }
+    s_sum[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && n < N) Elem<DT>::store(out, (int64_t)e * N + n, s_sum[0][lane] + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane]);
 }
 
 // out[e][c][r] = in[e][r][c] for r < rows, zero for rows <= r < rows_out (the padding of a k dimension):
@@ -569,8 +605,10 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
                    "%s: the kernel needs %d bytes of LDS", who, S::LDS);
         if (dev < 64) ready[dev] = true;
     }
-    const int64_t tiles = ((int64_t)p.M + S::BM - 1) / S::BM * (((int64_t)p.N + S::BN - 1) / S::BN) * p.batches;
+    const int64_t side = p.split == 2 ? 256 : S::BM;
+    int64_t tiles = ((int64_t)p.M + side - 1) / side * (((int64_t)p.N + side - 1) / side) * p.batches;
     PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
+    if (p.split == 2) tiles = 4 * (tiles < p.stay / 2 ? tiles : p.stay / 2);
     const int64_t stay = (int64_t)compute_units() * S::WAVES_PER_SIMD / 8 * 8;
     kernel<<<dim3((unsigned)(tiles + 7 < stay ? (tiles + 7) / 8 * 8 : stay)), GEMM_WG, S::LDS, stream>>>(p);
     PM_LAUNCH_CHECK(who);
@@ -584,24 +622,46 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 // a k-tile of 256 x 256 takes 1.0 us with few compute units at work and 1.3 with all of them (the clock sinks
 // under the matrix cores), one of 128 x 128 takes 0.45 alone on its compute unit and 0.8 for two at a time.
 // Example: 8 x 512 x 2048 x 2048 takes 37 us in the small tiles and 49 in the large, 8 x 1024 x 2048 x 2048 69 and 59.
-bool gemm_wants_small(int batches, int64_t rows, int64_t cols, int64_t k)
+//
+// A last round of large tiles that is at most half full is a launch of its own, in quarters (8 experts of 4096 +- 100
+// rows by 1024 columns: 512 tiles and a few, whose third round would take half as long again as the other two).
+double gemm_cost_small(int64_t tiles, double kt, int64_t cu)
 {
-    const int64_t cu = compute_units();
-    const int64_t big = (rows + 255) / 256 * ((cols + 255) / 256) * batches, small = (rows + 127) / 128 * ((cols + 127) / 128) * batches;
-    const double kt = (double)(k + 63) / 64;
-    const int64_t rest_b = big % cu, rest_s = small % (2 * cu);
-    const double t_big = (double)(big / cu) * (1.3 * kt + 10) + (rest_b ? (1.0 + 0.3 * (double)rest_b / (double)cu) * kt + 10 : 0.);
-    const double t_small = (double)(small / (2 * cu)) * (0.8 * kt + 5) + (rest_s == 0 ? 0. : rest_s <= cu ? 0.45 * kt + 5 : 0.8 * kt + 5);
-    return t_small < t_big;
+    const int64_t rest = tiles % (2 * cu);
+    return (double)(tiles / (2 * cu)) * (0.8 * kt + 5) + (rest == 0 ? 0. : rest <= cu ? 0.45 * kt + 5 : 0.8 * kt + 5);
+}
+
+// few rows per batch against a whole weight
+bool gemm_is_skinny(int64_t m, int64_t n, int64_t k, int64_t batches)
+{
+    return m <= SKINNY_ROWS && batches <= 65535 && n * k * 2 < ((int64_t)1 << 31);
 }
 
 template <bool TA, bool TB, bool GRAD>
-int gemm_run(const GemmArgs &p, int64_t rows_hint, hipStream_t stream, const char *who, int *tile_rows = nullptr)
+int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who)
 {
-    const int64_t side = TA ? p.M : rows_hint;
-    const bool small = gemm_wants_small(p.batches, side, p.N, TA ? rows_hint : p.K);
-    if (tile_rows) *tile_rows = small ? 128 : 256;
-    return small ? gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who) : gemm_launch<2, 2, TA, TB, GRAD>(p, stream, who);
+    const bool contiguous = p.lda == p.K && p.ldb == (TB ? p.N : p.K) && p.ldc == p.N && p.sB == (int64_t)p.N * p.K && p.sA == (int64_t)p.M * p.K &&
+                            p.sC == (int64_t)p.M * p.N;
+    if (!TA && contiguous && gemm_is_skinny(p.M, p.N, p.K, p.batches)) {
+        SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
+        return gemm_skinny_run(!TB, few, stream, who);
+    }
+    const int64_t cu = compute_units(), rows = TA ? p.M : rows_hint;
+    // (row counts from the device: an expectation, and a batch may have a standard deviation more)
+    const int64_t most = !TA && p.live ? rows + (int64_t)std::sqrt((double)rows) : rows;
+    const double kt = (double)((TA ? rows_hint : p.K) + 63) / 64;
+    const int64_t big = (most + 255) / 256 * (((int64_t)p.N + 255) / 256) * p.batches, small = (most + 127) / 128 * (((int64_t)p.N + 127) / 128) * p.batches;
+    const int64_t last = big % cu;
+    const double t_big = (double)(big / cu) * (1.3 * kt + 10) +
+                         (last == 0 ? 0. : 2 * last <= cu ? gemm_cost_small(4 * last, kt, cu) + 3 : (1.0 + 0.3 * (double)last / (double)cu) * kt + 10);
+    if (gemm_cost_small(small, kt, cu) < t_big) return gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who);
+    p.stay = (int)(cu / 8 * 8);
+    // (with many rounds the last one hardly counts, and a launch that may find nothing to do costs 3 us)
+    p.split = big < 6 * cu && (p.live ? true : gemm_last_round((int)big, p.stay) > 0);
+    if (gemm_launch<2, 2, TA, TB, GRAD>(p, stream, who)) return 1;
+    if (!p.split) return 0;
+    p.split = 2;
+    return gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who);
 }
 
 // what the buffer descriptors cover: from a tile's corner, a tile of a k-fast operand and 64 rows of a k-slow one
@@ -623,7 +683,7 @@ extern "C" int planmoe_gemm_nt_bf16(const void *a, const void *b, const void *bi
                "planmoe_gemm_nt_bf16: operands must be 16-byte aligned");
     PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_nt_bf16: 256 rows of an operand must stay under 2 GiB");
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
-               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, !aligned16(bias)};
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, 0, 0, !aligned16(bias)};
     return gemm_run<false, false, false>(p, m, (hipStream_t)stream, "planmoe_gemm_nt_bf16");
 }
 
@@ -642,7 +702,7 @@ extern "C" int planmoe_gemm_nn_bf16(const void *a, const void *b, const void *bi
                "planmoe_gemm_nn_bf16: operands must be 16-byte aligned");
     PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_nn_bf16: 256 rows of an operand must stay under 2 GiB");
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
-               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, !aligned16(bias)};
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, activation, 0, 0, !aligned16(bias)};
     return gemm_run<false, true, false>(p, m, (hipStream_t)stream, "planmoe_gemm_nn_bf16");
 }
 
@@ -660,7 +720,7 @@ extern "C" int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, i
                "planmoe_gemm_tn_bf16: operands must be 16-byte aligned");
     PM_REQUIRE(gemm_pitch_fits(lda) && gemm_pitch_fits(ldb) && gemm_pitch_fits(ldc), "planmoe_gemm_tn_bf16: 256 rows of an operand must stay under 2 GiB");
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, nullptr, (uint16_t *)c, nullptr, nullptr, 0, 1, m, n, k,
-               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, 0, false};
+               lda, ldb, ldc, batch_stride_a, batch_stride_b, batch_stride_c, batches, 0, 0, 0, false};
     return gemm_run<true, true, false>(p, k, (hipStream_t)stream, "planmoe_gemm_tn_bf16");
 }
 
@@ -693,11 +753,12 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, (const float *)bias, nullptr, (float *)c, nullptr, live, live_planes, live_round,
                      m, n, k, batches, activation};
-        return gemm_f32_run(form, p, st, who);
+        const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
+        return gemm_f32_run(form, p, gemm_f32_tile(form, p, hint), st, who);
     }
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n, most = form == 2 ? k : m;
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, live, live_planes,
-               live_round, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, activation, !aligned16(bias)};
+               live_round, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, activation, 0, 0, !aligned16(bias)};
     const int64_t hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
     if (form == 0) return gemm_run<false, true, false>(p, hint, st, who);
     if (form == 1) return gemm_run<false, false, false>(p, hint, st, who);
@@ -707,7 +768,7 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
 extern "C" size_t planmoe_expert_gemm_relu_bwd_workspace_bytes(int batches, int m, int n)
 {
     if (batches < 1 || m < 1 || n < 1) return 16;
-    return (size_t)batches * 2 * ((m + 127) / 128) * n * 4;
+    return (size_t)batches * 2 * ((m + 63) / 64) * n * 4;      // (fp32 tiles may have 64 rows)
 }
 
 extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void *b, const void *h, int batches, int m, int n,
@@ -721,19 +782,24 @@ extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void
     PM_REQUIRE(batches <= 65535, "%s: too many batches", who);
     hipStream_t st = (hipStream_t)stream;
     float *parts = dbias ? (float *)workspace : nullptr;
-    int tile_rows = G32_B;
+    const int hint = rows_hint >= 1 && rows_hint < m ? rows_hint : m;
+    int tile_rows, slots;
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
-        if (gemm_f32_run(1, p, st, who)) return 1;
+        tile_rows = gemm_f32_tile(1, p, hint);
+        slots = (m + tile_rows - 1) / tile_rows * 2;
+        if (gemm_f32_run(1, p, tile_rows, st, who)) return 1;
     } else {
         GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
-                   m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, false};
-        if (gemm_run<false, false, true>(p, rows_hint >= 1 && rows_hint < m ? rows_hint : m, st, who, &tile_rows)) return 1;
+                   m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};
+        if (gemm_run<false, false, true>(p, hint, st, who)) return 1;
+        tile_rows = 128;
+        slots = gemm_is_skinny(m, n, k, batches) ? 1 : (m + 127) / 128 * 2;       // (few rows altogether: one slot holds everything)
     }
     if (dbias) {
-        const dim3 grid((unsigned)((n + 255) / 256), (unsigned)batches);
-        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, dbias);
-        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, dbias);
+        const dim3 grid((unsigned)((n + 63) / 64), (unsigned)batches);
+        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, slots, dbias);
+        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, slots, dbias);
         PM_LAUNCH_CHECK(who);
     }
     return 0;

@@ -4,11 +4,12 @@
 // with either operand stored k fast or k slow, as planmoe_gemm_*_bf16.
 //
 // A 32 x 32 x 2 MFMA takes 64 clocks, so unlike bf16 nothing here is bound by operand traffic: a 128 x 128
-// tile reads 32 KB per k-tile of 32 for 4096 clocks of matrix core.  Four waves of 64 x 64, operands straight
-// into LDS (buffer_load ... lds), the next k-tile in flight during the MFMAs of this one, two work-groups
+// tile reads 32 KB per k-tile of 32 for 4096 clocks of matrix core.  Four waves of 64 x 64 (32 x 32 in the small
+// tile), operands straight into LDS (buffer_load ... lds), the next k-tile in flight during the MFMAs of this one, two work-groups
 // per compute unit so that one's barrier and epilogue fall under the other's MFMAs.  A k-fast operand is
-// read four k at a time (16 bytes per lane); which k a lane holds does not matter to the sum as long as
-// both operands agree, so step q of eight k takes k = q from lanes 0 .. 31 and k = 4 + q from lanes 32 .. 63.
+// read four k at a time (16 bytes per lane), sixteen k are two reads, and the sums take them in the order
+// 0 4 8 12, 1 5 9 13, ..: the order of a product made of 16 x 16 x 4 instructions whose lanes read 16 bytes, so what such
+// a product (the fp32 library's) gives, this one gives bit for bit, and a relu behind it cuts the same elements.
 #include "gemm_f32.hpp"
 
 namespace pm {
@@ -18,8 +19,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t g32_u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int G32_BK = 32;
-constexpr int G32_OPERAND = G32_B * G32_BK * 4;             // one operand's k-tile in LDS
-constexpr int G32_LDS = 4 * G32_OPERAND;                    // A0 A1 B0 B1
 
 __device__ __forceinline__ g32_u32x4 g32_desc(const void *base, int64_t bytes)
 {
@@ -32,9 +31,11 @@ __device__ __forceinline__ void g32_dma16(g32_u32x4 desc, uint32_t voff, uint32_
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
 }
 
-template <bool TA, bool TB>
+// F: 32 x 32 fragments of a wave on a side; the tile is 64 F x 64 F
+template <int F, bool TA, bool TB>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
 {
+    constexpr int G32_B = 64 * F, G32_OPERAND = G32_B * G32_BK * 4;         // tile side; one operand's k-tile in LDS (A0 A1 B0 B1)
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -69,11 +70,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     const int64_t step_a = TA ? (int64_t)G32_BK * lda * 4 : G32_BK * 4, step_b = TB ? (int64_t)G32_BK * ldb * 4 : G32_BK * 4;
     const int KT = (K + G32_BK - 1) / G32_BK, k_tail = K % G32_BK ? K % G32_BK : G32_BK;
 
-    // k fast: 128 rows of 128 bytes, a load fills eight, chunk c of row r at unit c ^ (r >> 1) & 7.
-    // k slow: 32 rows of 512 bytes, a load fills two.
+    // k fast: 64 F rows of 128 bytes, a load fills eight, chunk c of row r at unit c ^ (r >> 1) & 7.
+    // k slow: 32 rows of 256 F bytes, a load fills 4 / F.
     auto fetch = [&](bool T, int i, int ld) -> uint32_t {
-        if (T) return (uint32_t)(8 * wave + (lane >> 5)) * (uint32_t)ld * 4u + (uint32_t)(lane & 31) * 16u;
-        const int row = 32 * wave + 8 * i + (lane >> 3);
+        if (T) return (uint32_t)(8 * wave + lane / (16 * F)) * (uint32_t)ld * 4u + (uint32_t)(lane % (16 * F)) * 16u;
+        const int row = 16 * F * wave + 8 * i + (lane >> 3);
         return (uint32_t)row * (uint32_t)ld * 4u + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
     };
     const uint32_t va[2] = {fetch(TA, 0, lda), fetch(TA, TA ? 0 : 1, lda)}, vb[2] = {fetch(TB, 0, ldb), fetch(TB, TB ? 0 : 1, ldb)};
@@ -83,37 +84,38 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     auto load_tile = [&](int kt) {
         if (kt >= KT) return;
         const g32_u32x4 da = g32_desc(A + kt * step_a, ra - kt * step_a), db = g32_desc(B + kt * step_b, rb - kt * step_b);
-        const uint32_t sa = lds0 + (kt & 1) * G32_OPERAND + wave * 4096, sb = sa + 2 * G32_OPERAND;
+        const uint32_t sa = lds0 + (kt & 1) * G32_OPERAND + wave * (2048 * F), sb = sa + 2 * G32_OPERAND;
         const bool last = kt == KT - 1 && k_tail != G32_BK;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            g32_dma16(da, va[i & 1] | (!TA && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)lda * 4u * (TA ? 2 * i : 8 * (i & ~1)), sa + i * 1024);
+        for (int i = 0; i < 2 * F; ++i)
+            g32_dma16(da, va[i & 1] | (!TA && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)lda * 4u * (uint32_t)(TA ? 4 / F * i : 8 * (i & ~1)), sa + i * 1024);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            g32_dma16(db, vb[i & 1] | (!TB && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)ldb * 4u * (TB ? 2 * i : 8 * (i & ~1)), sb + i * 1024);
+        for (int i = 0; i < 2 * F; ++i)
+            g32_dma16(db, vb[i & 1] | (!TB && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)ldb * 4u * (uint32_t)(TB ? 4 / F * i : 8 * (i & ~1)), sb + i * 1024);
     };
 
-    f32x16 acc[2][2];
+    f32x16 acc[F][F];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < F; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < F; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
     const int fr = lane & 31, fc = lane >> 5;
-    // eight k of a side's two 32-row fragments: element q of fragment i
-    auto read8 = [&](bool T, const uint8_t *base, int w, int s, f32x4 (&f)[2]) {
-        if (T) {
+    // sixteen k of a side's 32-row fragments: element q of half h of fragment i is k = 8 h + 4 fc + q
+    auto read16 = [&](bool T, const uint8_t *base, int w, int s, f32x4 (&f)[F][2]) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < F; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    f[i][q] = *reinterpret_cast<const float *>(base + (8 * s + 4 * fc + q) * 512 + (64 * w + 32 * i + fr) * 4);
-        } else {
+            for (int h = 0; h < 2; ++h) {
+                if (T) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-                f[i] = *reinterpret_cast<const f32x4 *>(base + (64 * w + 32 * i + fr) * 128 + (((2 * s + fc) ^ ((fr >> 1) & 7)) * 16));
-        }
+                    for (int q = 0; q < 4; ++q)
+                        f[i][h][q] = *reinterpret_cast<const float *>(base + (16 * s + 8 * h + 4 * fc + q) * (256 * F) + (32 * F * w + 32 * i + fr) * 4);
+                } else {
+                    f[i][h] = *reinterpret_cast<const f32x4 *>(base + (32 * F * w + 32 * i + fr) * 128 + (((4 * s + 2 * h + fc) ^ ((fr >> 1) & 7)) * 16));
+                }
+            }
     };
 
     load_tile(0);
@@ -122,32 +124,34 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         load_tile(kt + 1);
         const uint8_t *a = lds + (kt & 1) * G32_OPERAND, *b = a + 2 * G32_OPERAND;
-        f32x4 fa[2][2], fb[2][2];
-        read8(TA, a, wm, 0, fa[0]);
-        read8(TB, b, wn, 0, fb[0]);
+        f32x4 fa[2][F][2], fb[2][F][2];
+        read16(TA, a, wm, 0, fa[0]);
+        read16(TB, b, wn, 0, fb[0]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s < 3) { read8(TA, a, wm, s + 1, fa[(s + 1) & 1]); read8(TB, b, wn, s + 1, fb[(s + 1) & 1]); }
+        for (int s = 0; s < 2; ++s) {
+            if (s == 0) { read16(TA, a, wm, 1, fa[1]); read16(TB, b, wn, 1, fb[1]); }
             // (the second operand first: a lane then holds four consecutive columns of one row)
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int h = 0; h < 2; ++h)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[s & 1][j][q], fa[s & 1][i][q], acc[i][j], 0, 0, 0);
+                    for (int i = 0; i < F; ++i)
+#pragma unroll
+                        for (int j = 0; j < F; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[s][j][h][q], fa[s][i][h][q], acc[i][j], 0, 0, 0);
         }
     }
 
     const int64_t corner = (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0;
     const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - m0 - 1) * p.N + (p.N - n0)) * 4);
     const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
-    float sums[2][4][4];
+    float sums[F][4][4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < F; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int col = wn * 64 + 32 * j + 8 * q + 4 * fc;
+            const int col = wn * 32 * F + 32 * j + 8 * q + 4 * fc;
             const bool in_n = n0 + col < p.N;
             f32x4 add = {0.f, 0.f, 0.f, 0.f};
             if (p.bias && in_n) {
@@ -157,8 +161,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
 #pragma unroll
             for (int x = 0; x < 4; ++x) sums[j][q][x] = 0.f;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int row = wm * 64 + 32 * i + fr;
+            for (int i = 0; i < F; ++i) {
+                const int row = wm * 32 * F + 32 * i + fr;
                 f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
                 if (p.bias) v += add;
                 if (p.relu) {
@@ -179,45 +183,64 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
         const int slots = tiles_m * 2;
         float *to = p.colsum + ((int64_t)e * slots + m0 / G32_B * 2 + wm) * p.N + n0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < F; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
 #pragma unroll
                 for (int x = 0; x < 4; ++x)
 #pragma unroll
                     for (int d = 1; d < 32; d <<= 1) sums[j][q][x] += __shfl_xor(sums[j][q][x], d);
-                const int col = wn * 64 + 32 * j + 8 * q + 4 * fc;
+                const int col = wn * 32 * F + 32 * j + 8 * q + 4 * fc;
                 if (fr == 0 && n0 + col < p.N) *reinterpret_cast<float4 *>(to + col) = make_float4(sums[j][q][0], sums[j][q][1], sums[j][q][2], sums[j][q][3]);
             }
     }
 }
 
-template <bool TA, bool TB>
+template <int F, bool TA, bool TB>
 static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
 {
-    const auto kernel = gemm_f32_kernel<TA, TB>;
+    constexpr int LDS = 4 * 64 * F * G32_BK * 4, SIDE = 64 * F;
+    const auto kernel = gemm_f32_kernel<F, TA, TB>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
     if (dev >= 64 || !ready[dev]) {
-        PM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G32_LDS) == hipSuccess,
-                   "%s: the kernel needs %d bytes of LDS", who, G32_LDS);
+        PM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess,
+                   "%s: the kernel needs %d bytes of LDS", who, LDS);
         if (dev < 64) ready[dev] = true;
     }
-    const int64_t tiles = ((int64_t)p.M + G32_B - 1) / G32_B * (((int64_t)p.N + G32_B - 1) / G32_B) * p.batches;
+    const int64_t tiles = ((int64_t)p.M + SIDE - 1) / SIDE * (((int64_t)p.N + SIDE - 1) / SIDE) * p.batches;
     PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
-    kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, G32_LDS, stream>>>(p);
+    kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, LDS, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
 
-int gemm_f32_run(int form, const Gemm32Args &p, hipStream_t stream, const char *who)
+// The tile's side: a compute unit's matrix cores take 1.7 us for a k-tile of 128 x 128 and a quarter of that, and
+// a tenth, for one of 64 x 64; what counts is the fullest compute unit (4 x 300 x 512 x 1024: 64 tiles of 128, 57 us).
+int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
+{
+    const int64_t m = form == 2 ? p.M : rows_hint;
+    const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
+    auto cost = [&](int64_t side, double us) {
+        const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
+        return (double)((tiles + 255) / 256) * (us * kt + 2);
+    };
+    return cost(64, 0.47) < cost(128, 1.7) ? 64 : 128;
+}
+
+int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who)
 {
     PM_REQUIRE((int64_t)p.K * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.M * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.N * 4 * 128 < ((int64_t)1 << 31),
                "%s: 128 rows of an operand must stay under 2 GiB", who);
-    if (form == 0) return gemm_f32_launch<false, true>(p, stream, who);
-    if (form == 1) return gemm_f32_launch<false, false>(p, stream, who);
-    return gemm_f32_launch<true, true>(p, stream, who);
+    if (side == 64) {
+        if (form == 0) return gemm_f32_launch<1, false, true>(p, stream, who);
+        if (form == 1) return gemm_f32_launch<1, false, false>(p, stream, who);
+        return gemm_f32_launch<1, true, true>(p, stream, who);
+    }
+    if (form == 0) return gemm_f32_launch<2, false, true>(p, stream, who);
+    if (form == 1) return gemm_f32_launch<2, false, false>(p, stream, who);
+    return gemm_f32_launch<2, true, true>(p, stream, who);
 }
 
 } // namespace pm

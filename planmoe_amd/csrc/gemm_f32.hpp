@@ -11,9 +11,10 @@ struct Gemm32Args {
     int live_planes, live_round;
     int M, N, K, batches, relu;            // operands and result contiguous
 };
-constexpr int G32_B = 128;                 // rows and columns of a tile
 
-// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment
-int gemm_f32_run(int form, const Gemm32Args &p, hipStream_t stream, const char *who);
+// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  side: rows and columns of a tile, 64 or 128
+// (gemm_f32_tile picks it for a number of rows in use)
+int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint);
+int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who);
 
 } // namespace pm

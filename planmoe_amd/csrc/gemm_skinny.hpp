@@ -1,0 +1,22 @@
+// The experts' product for few rows, as the expert GEMM entry points call it.
+#pragma once
+#include "common.hpp"
+
+namespace pm {
+
+constexpr int SKINNY_ROWS = 64;                             // the most rows of an expert it takes
+
+struct SkinnyArgs {
+    const uint16_t *A, *B, *bias;
+    const uint16_t *mask;         // relu's backward (nt): c is kept where mask > 0, NULL: none
+    uint16_t *C;
+    float *colsum;                // with mask: column sums of what was stored, [batches][N], NULL: none
+    const int *live;              // [live_planes][batches]: rows in use, NULL: all
+    int live_planes, live_round;
+    int M, N, K, batches, relu;   // operands and result contiguous
+};
+
+// nt: b is [batches, N, K], else [batches, K, N]; the caller has checked shape and alignment
+int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who);
+
+} // namespace pm

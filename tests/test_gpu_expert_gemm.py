@@ -98,6 +98,70 @@ def test_expert_gemm_relu_backward_and_its_bias_gradient(B, m, n, k, counted, dt
         assert bool(((db[e].double() - stored.sum(0)).abs() <= tol).all())
 
 
+# few rows per expert against a whole weight: one row, either side of 16, 32 and 64 rows; columns and reduction lengths that
+# are and are not whole steps of the waves that share a reduction
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(8, 8), (136, 520), (264, 1032), (64, 4096)])
+def test_expert_gemm_with_few_rows(m, n, k):
+    from planmoe_amd import ops
+    print("case", m, n, k, flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    B, dtype = 3, torch.bfloat16
+    live = torch.tensor([[m, 0, max(m // 2, 1)]], dtype=torch.int32)
+    a, bias = torch.randn(B, m, k, generator=g).to(dtype), torch.randn(B, n, generator=g).to(dtype)
+    w, h = torch.randn(B, k, n, generator=g).to(dtype), torch.randn(B, m, n, generator=g).clamp(min=0).to(dtype)
+    for e in range(B):
+        a[e, int(live[0, e]):] = float("nan")
+    wt = w.transpose(1, 2).contiguous()
+    nn = torch.full((B, m, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    ops.expert_gemm("nn", a.to(DEV), w.to(DEV), bias.to(DEV), relu=True, live=live.to(DEV), out=nn)
+    ops.expert_gemm("nt", a.to(DEV), wt.to(DEV), live=live.to(DEV), out=nt)
+    _, db = ops.expert_gemm_relu_bwd(a.to(DEV), wt.to(DEV), h.to(DEV), live=live.to(DEV), out=masked)
+    torch.cuda.synchronize()
+    nn, nt, masked, db = nn.cpu().double(), nt.cpu().double(), masked.cpu().double(), db.cpu().double()
+    for e in range(B):
+        r = int(live[0, e])
+        ref, mag = a[e, :r].double() @ w[e].double(), a[e, :r].double().abs() @ w[e].double().abs()
+        tol = _bound(ref, mag, k, dtype)
+        biased = ref + bias[e].double()
+        assert bool(((nn[e, :r] - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all())
+        assert bool(((nt[e, :r] - ref).abs() <= tol).all())
+        assert bool(((masked[e, :r] - ref * (h[e, :r] > 0)).abs() <= tol).all())
+        assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all())
+        stored = masked[e, :r]
+        assert bool(((db[e] - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all())
+
+
+# 256 work-groups that stay take 256 x 256 tiles, four to a tile row here; what is left for a last round is a launch of
+# quarters up to 128 tiles.  Rows in use that leave 0, 4 (one row of the last tile), 128 and 132 tiles, and fewer than one round
+@pytest.mark.parametrize("rows", [16384, 16385, 24576, 24577, 300])
+def test_expert_gemm_last_round(rows):
+    from planmoe_amd import ops
+    print("case", rows, flush=True)
+    cap, n, k, dtype = 24832, 1024, 512, torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    a, w = torch.randn(2, cap // 2, k, device=DEV, generator=g).to(dtype), torch.randn(2, k, n, device=DEV, generator=g).to(dtype)
+    first = 0 if rows < 512 else rows // 512 * 256          # (the odd row is the second batch's)
+    live = torch.tensor([[first, rows - first]], dtype=torch.int32, device=DEV)
+    h = torch.randn(2, cap // 2, n, device=DEV, generator=g).clamp(min=0).to(dtype)
+    out = torch.full((2, cap // 2, n), 7.0, dtype=dtype, device=DEV)
+    masked = out.clone()
+    ops.expert_gemm("nn", a, w, live=live, out=out, rows_hint=rows // 2)
+    _, db = ops.expert_gemm_relu_bwd(a, w.transpose(1, 2).contiguous(), h, live=live, out=masked, rows_hint=rows // 2)
+    torch.cuda.synchronize()
+    for e in range(2):
+        r = int(live[0, e])
+        ref, mag = a[e, :r].double() @ w[e].double(), a[e, :r].double().abs() @ w[e].double().abs()
+        tol = _bound(ref, mag, k, dtype)
+        assert bool(((out[e, :r].double() - ref).abs() <= tol).all()), e
+        assert bool((out[e, r:] == 7.0).all()), e
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all()), e
+        assert bool((masked[e, r:] == 7.0).all()), e
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, dtype)).all()), e
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T,M,E", [(1, 8, 1), (33, 520, 3), (1000, 264, 9), (517, 2056, 16)])
 def test_gate_weight_gradient_and_row_sums(T, M, E, dtype):
