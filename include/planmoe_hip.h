@@ -172,6 +172,15 @@ int planmoe_bwd_gate(const void *x, const void *dispatched, int dtype, const int
                      const int32_t *locations, int64_t plane_stride, int top_k, int samples,
                      int model_dim, int capacity, float *grad_gates, void *stream);
 
+/* Backward of planmoe_combine_fwd in one pass over grad [samples, model_dim] (GatingDecoder.backward,
+ * fast_dispatch.py:62-79): grad_dispatched = planmoe_dispatch_fwd of grad with `gates`, grad_gates =
+ * planmoe_bwd_gate of grad and `dispatched`.  samples, capacity >= 1; workspace of
+ * planmoe_dispatch_workspace_bytes. */
+int planmoe_combine_bwd(const void *grad, const void *dispatched, int dtype, const float *gates,
+                        const int32_t *indices, const int32_t *locations, int64_t plane_stride, int top_k,
+                        int samples, int model_dim, int experts, int capacity, void *grad_dispatched,
+                        float *grad_gates, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------- "int8" codec
  * Replaces Int8Compressor::compress / ::decompress (custom/compressor/int8.cpp:7-60).
  * Per row of row_len elements: bias = min, scale = max - min,

@@ -40,6 +40,8 @@ SIGNATURES = {
                                     c_int, c_int, c_int, c_void_p, c_void_p]),
     "planmoe_bwd_gate": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int,
                                  c_int, c_int, c_int, c_void_p, c_void_p]),
+    "planmoe_combine_bwd": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
+                                    c_int, c_int, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "planmoe_int8_compress": (c_int, [c_void_p, c_int, c_int64, c_int, c_void_p, c_void_p, c_void_p,
                                       c_void_p]),
     "planmoe_int8_decompress": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int,

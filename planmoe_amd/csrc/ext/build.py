@@ -1,5 +1,5 @@
-"""Builds schemoe_custom_kernel*.so (the reference's pybind module name) and _planmoe_layer*.so (the layer's
-host side) in planmoe_amd/csrc/ext with g++ against torch's headers and libplanmoe_hip.so.  Run by
+"""Builds schemoe_custom_kernel*.so (the reference's pybind module name) and _planmoe_layer*.so (the host
+side of the layer and of the routing API) in planmoe_amd/csrc/ext with g++ against torch's headers and libplanmoe_hip.so.  Run by
 __graft_entry__.build()."""
 import os
 import subprocess
@@ -30,7 +30,8 @@ def _flags(name):
 def _objects():
     return [(NAME, os.path.join(HERE, NAME + ".cpp"), os.path.join(HERE, NAME + ".o")),
             (NAME, os.path.join(HERE, "example_third_party_compressor.cpp"), os.path.join(HERE, "example_third_party_compressor.o")),
-            (LAYER, os.path.join(HERE, "layer.cpp"), os.path.join(HERE, LAYER + ".o"))]
+            (LAYER, os.path.join(HERE, "layer.cpp"), os.path.join(HERE, LAYER + ".o")),
+            (LAYER, os.path.join(HERE, "routing.cpp"), os.path.join(HERE, "routing.o"))]
 
 
 def compile_objects():
@@ -43,11 +44,11 @@ def compile_objects():
 
 def link():
     csrc = os.path.join(ROOT, "planmoe_amd", "csrc")
-    (_, _, module_obj), (_, _, example_obj), (_, _, layer_obj) = _objects()
+    (_, _, module_obj), (_, _, example_obj), (_, _, layer_obj), (_, _, routing_obj) = _objects()
     libs = ["-L" + p for p in ce.library_paths()] + ["-L/opt/rocm/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
             "-ltorch", "-ltorch_python", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"] + ["-Wl,-rpath," + p for p in ce.library_paths()]
     subprocess.check_call(["g++", "-shared", module_obj, "-o", target(), "-L" + csrc, "-lplanmoe_hip", "-Wl,-rpath," + csrc] + libs)
-    subprocess.check_call(["g++", "-shared", layer_obj, "-o", target(LAYER), "-L" + csrc, "-lplanmoe_hip", "-Wl,-rpath," + csrc] + libs)
+    subprocess.check_call(["g++", "-shared", layer_obj, routing_obj, "-o", target(LAYER), "-L" + csrc, "-lplanmoe_hip", "-Wl,-rpath," + csrc] + libs)
     # the example plug-in: a compressor compiled against include/planmoe/compressor/abstract.h with the
     # same flags and linked against the module just built
     subprocess.check_call(["g++", "-shared", example_obj, "-o", example_target(), target(), "-Wl,-rpath," + HERE] + libs)

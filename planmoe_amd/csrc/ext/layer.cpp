@@ -9,32 +9,14 @@
 // With one rank the exchange delivers what was sent, so the "int8" codec is applied to rows in registers
 // (planmoe_layer_dispatch, planmoe_layer_combine, planmoe_layer_combine_bwd) and the rows of empty capacity
 // slots are neither written nor multiplied: the products get the number of rows in use of every expert.
-#include "planmoe_hip.h"
-
-#include <ATen/hip/HIPEvent.h>
-#include <hip/hip_runtime_api.h>
-#include <torch/extension.h>
-
-#include <algorithm>
+#include "host.hpp"
 
 namespace {
 
-using torch::Tensor;
+using namespace planmoe_host;
 
 enum Codec { CODEC_NONE = 0, CODEC_INT8 = 1, CODEC_ZFP = 2, CODEC_LZ = 3 };
 constexpr double ZFP_RATE = 8.0;             // zfpc.h:17
-
-void *current_stream() { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
-#define PM_CALL(expr) TORCH_CHECK((expr) == 0, planmoe_last_error())
-
-int pm_dtype(at::ScalarType t)
-{
-    TORCH_CHECK(t == at::kFloat || t == at::kBFloat16 || t == at::kHalf, "planmoe: unsupported dtype (float32, bfloat16 or float16)");
-    return t == at::kFloat ? PLANMOE_F32 : t == at::kBFloat16 ? PLANMOE_BF16 : PLANMOE_F16;
-}
-const int32_t *ints(const Tensor &t) { return t.data_ptr<int32_t>(); }
-const float *floats(const Tensor &t) { return t.data_ptr<float>(); }
-void *raw(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 struct Shape {
     int T, M, E, H, k, cap, dt;
@@ -53,8 +35,6 @@ struct Live {
 struct Pass {
     Tensor y, l_aux, gates, indices, locations, counts, scores, xe, h, ye, stream;
 };
-
-Tensor bytes(int64_t n, const Tensor &like) { return at::empty({std::max<int64_t>(n, 16)}, like.options().dtype(at::kByte)); }
 
 Tensor lz_round_trip(const Tensor &buf, void *st)
 {
@@ -90,15 +70,6 @@ Tensor zfp_combine(const Tensor &stream, const float *gates, const Pass &p, cons
     Tensor out = at::empty({s.T, s.M}, stream.options().dtype(at::kFloat)), ws = bytes((int64_t)planmoe_combine_zfp_workspace_bytes(s.E, s.cap), stream);
     PM_CALL(planmoe_combine_zfp(stream.data_ptr(), ZFP_RATE, gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap,
                                 out.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
-    return out;
-}
-
-// fast_encode's buffer with zeros in the empty slots
-Tensor dispatch_rows(const Tensor &x, const float *gates, const Pass &p, const Shape &s, void *st)
-{
-    Tensor out = at::empty({s.rows(), s.M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(s.E, s.cap), x);
-    PM_CALL(planmoe_dispatch_fwd(x.data_ptr(), s.dt, gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap,
-                                 out.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), st));
     return out;
 }
 
@@ -200,6 +171,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         ctx->saved_data["cap"] = cap;
         ctx->saved_data["normalize"] = normalize;
         ctx->saved_data["codec"] = codec;
+        ctx->set_materialize_grads(false);
         return {p.y, p.l_aux};
     }
 
@@ -236,8 +208,10 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                 PM_CALL(planmoe_bwd_gate_zfp(ye.data_ptr(), ZFP_RATE, floats(grad), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
                                              grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
             } else if (codec == CODEC_LZ) {
-                gye = lz_round_trip(dispatch_rows(grad, floats(gates), p, s, st), st);
-                PM_CALL(planmoe_bwd_gate(grad.data_ptr(), ye.data_ptr(), s.dt, idx, loc, s.T, s.k, s.T, s.M, s.cap, grad_gates.data_ptr<float>(), st));
+                Tensor buf = at::empty({s.rows(), s.M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(s.E, s.cap), x);
+                PM_CALL(planmoe_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, buf.data_ptr(),
+                                            grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
+                gye = lz_round_trip(buf, st);
             } else {
                 gye = at::empty({s.rows(), s.M}, x.options());
                 PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, codec == CODEC_INT8, floats(gates), idx, loc, s.T, s.k, s.T, s.M,
@@ -332,5 +306,13 @@ std::tuple<Tensor, Tensor> ffn_layer(const Tensor &x, const Tensor &wg, const Te
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    pybind11::register_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (const Failure &e) {
+            PyErr_SetString(pybind11::module_::import("planmoe_amd._lib").attr("PlanMoEError").ptr(), e.what());
+        }
+    });
+    def_routing(m);
     m.def("ffn_layer", &ffn_layer, pybind11::call_guard<pybind11::gil_scoped_release>(), "the layer with its built-in experts, forward (and its autograd node)");
 }

@@ -7,6 +7,8 @@
 // moves it with 16-byte accesses, all k choices of the token in the same pass.
 #include "rows.hpp"
 
+#include <algorithm>
+
 namespace pm {
 
 // ------------------------------------------------------------------ slot occupancy flags
@@ -32,16 +34,16 @@ __global__ __launch_bounds__(256) void slot_flags_mark(uint32_t *flags, const in
 // ------------------------------------------------------------------ dispatch (scatter rows)
 // Blocks [0, token_blocks) move token rows: dispatched[slot] = 0 + gate * x[t].
 // Blocks [token_blocks, gridDim.x) write zero rows into the slots no live pair addresses.
-template <int DT, bool VECTOR>
+template <int DT, int MODE>
 __global__ __launch_bounds__(256) void dispatch_kernel(
     const void *__restrict__ x, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
     void *__restrict__ dispatched, const uint32_t *__restrict__ flags, int token_blocks)
 {
-    using IO = RowIO<DT, VECTOR>;
+    using IO = RowIO<DT, MODE>;
     const int wave = threadIdx.x >> 6, lane = lane_id();
-    const int units = model_dim / IO::U;
+    const int units = IO::units(model_dim);
     const int64_t row_bytes = (int64_t)model_dim * sizeof(typename Elem<DT>::store_t);
 
     if ((int)blockIdx.x >= token_blocks) {
@@ -50,7 +52,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
         for (int s = (blockIdx.x - token_blocks) * 4 + wave; s < slots; s += nwaves) {
             if (flags[s]) continue;
             char *row = (char *)dispatched + (int64_t)s * row_bytes;
-            for (int u = lane; u < units; u += WAVE) IO::store_zero(row, u);
+            for (int u = lane; u < units; u += WAVE) IO::store_zero(row, IO::at(u, (int)row_bytes));
         }
         return;
     }
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
         if (__ballot(slot >= 0) == 0) continue;          // every choice of this pass dropped: the row is not read
         for (int u = lane; u < units; u += WAVE) {
             float v[IO::U];
-            IO::load(src, u, v);
+            IO::load(src, IO::at(u, (int)row_bytes), v);
             for (int j = 0; j < np; ++j) {
                 const int s = rl_i(slot, j);
                 if (s < 0) continue;
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
                 float o[IO::U];
 #pragma unroll
                 for (int i = 0; i < IO::U; ++i) o[i] = 0.f + g * v[i];
-                IO::store((char *)dispatched + (int64_t)s * row_bytes, u, o);
+                IO::store((char *)dispatched + (int64_t)s * row_bytes, IO::at(u, (int)row_bytes), o);
             }
         }
     }
@@ -82,15 +84,15 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
 
 // ------------------------------------------------------------------ combine (gather rows)
 // out[t] = sum_j (live_j ? gate_j * dispatched[slot_j] : 0), planes added left to right.
-template <int DT, bool VECTOR>
+template <int DT, int MODE>
 __global__ __launch_bounds__(256) void combine_kernel(
     const void *__restrict__ dispatched, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int capacity, void *__restrict__ out)
 {
-    using IO = RowIO<DT, VECTOR>;
+    using IO = RowIO<DT, MODE>;
     const int wave = threadIdx.x >> 6, lane = lane_id();
-    const int units = model_dim / IO::U;
+    const int units = IO::units(model_dim);
     const int64_t row_bytes = (int64_t)model_dim * sizeof(typename Elem<DT>::store_t);
     const int t = blockIdx.x * 4 + wave;
     if (t >= samples) return;
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(256) void combine_kernel(
                 const char *row = (const char *)dispatched + (int64_t)max(s, 0) * row_bytes;
                 float term[B][IO::U];
 #pragma unroll
-                for (int b = 0; b < B; ++b) IO::load(row, min(u0 + b * WAVE, units - 1), term[b]);
+                for (int b = 0; b < B; ++b) IO::load(row, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes), term[b]);
 #pragma unroll
                 for (int b = 0; b < B; ++b) {
 #pragma unroll
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(256) void combine_kernel(
             }
 #pragma unroll
             for (int b = 0; b < B; ++b)
-                if (u0 + b * WAVE < units) IO::store(dst, u0 + b * WAVE, acc[b]);
+                if (u0 + b * WAVE < units) IO::store(dst, IO::at(u0 + b * WAVE, (int)row_bytes), acc[b]);
         }
     } else {
         // more planes than lanes: walk the planes straight from memory
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(256) void combine_kernel(
                 const float g = gates ? gates[o] : 1.f;
                 float term[IO::U];
                 if (e >= 0 && l >= 0 && l < capacity) {
-                    IO::load((const char *)dispatched + ((int64_t)e * capacity + l) * row_bytes, u, term);
+                    IO::load((const char *)dispatched + ((int64_t)e * capacity + l) * row_bytes, IO::at(u, (int)row_bytes), term);
 #pragma unroll
                     for (int i = 0; i < IO::U; ++i) term[i] = g * term[i];
                 } else {
@@ -145,34 +147,37 @@ __global__ __launch_bounds__(256) void combine_kernel(
 #pragma unroll
                 for (int i = 0; i < IO::U; ++i) acc[i] = (j == 0) ? term[i] : acc[i] + term[i];
             }
-            IO::store(dst, u, acc);
+            IO::store(dst, IO::at(u, (int)row_bytes), acc);
         }
     }
 }
 
-template <int DT, bool VECTOR>
+template <int DT, int MODE>
 __global__ __launch_bounds__(256) void zero_rows_kernel(void *__restrict__ out, int samples, int model_dim)
 {
-    using IO = RowIO<DT, VECTOR>;
+    using IO = RowIO<DT, MODE>;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= samples) return;
-    char *dst = (char *)out + (int64_t)t * model_dim * (int64_t)sizeof(typename Elem<DT>::store_t);
-    for (int u = lane_id(); u < model_dim / IO::U; u += WAVE) IO::store_zero(dst, u);
+    const int row_bytes = model_dim * (int)sizeof(typename Elem<DT>::store_t);
+    char *dst = (char *)out + (int64_t)t * row_bytes;
+    for (int u = lane_id(); u < IO::units(model_dim); u += WAVE) IO::store_zero(dst, IO::at(u, row_bytes));
 }
 
 // ------------------------------------------------------------------ gate gradient
 // grad_gates[j][t] = <dispatched[slot_j], x[t]> (0 for a dropped pair).  One wave per token;
-// planes are taken four at a time so the token row is read once per group.
-template <int DT, bool VECTOR>
+// planes are taken four at a time so the token row is read once per group.  Rows that are not 16-byte aligned go
+// element by element, also where they could be read as dwords: where a token's choices hold the same row, what
+// the normalised gates pass on is the rounding of these sums alone, and their order stays what it is.
+template <int DT, int MODE>
 __global__ __launch_bounds__(256) void bwd_gate_kernel(
     const void *__restrict__ x, const void *__restrict__ dispatched,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int capacity, float *__restrict__ grad_gates)
 {
-    using IO = RowIO<DT, VECTOR>;
+    using IO = RowIO<DT, MODE>;
     constexpr int G = 4;
     const int wave = threadIdx.x >> 6, lane = lane_id();
-    const int units = model_dim / IO::U;
+    const int units = IO::units(model_dim);
     const int64_t row_bytes = (int64_t)model_dim * sizeof(typename Elem<DT>::store_t);
     const int t = blockIdx.x * 4 + wave;
     if (t >= samples) return;
@@ -186,21 +191,21 @@ __global__ __launch_bounds__(256) void bwd_gate_kernel(
 #pragma unroll
         for (int j = 0; j < G; ++j) s[j] = (j < np) ? rl_i(slot, j) : -1;
         float acc[G] = {0.f, 0.f, 0.f, 0.f};
-        // two units of the row per lane and pass; the slot rows of all choices are requested with
+        // two vectors or eight elements of the row per lane and pass; the slot rows of all choices are requested with
         // straight-line loads at clamped addresses (a dropped choice reads slot 0 and is left out
         // of the sum; the caller guarantees a slot 0 to read: capacity >= 1)
-        constexpr int B = 2;
+        constexpr int B = MODE == ROWS_16 ? 2 : 8;
         for (int u0 = lane; u0 < units; u0 += B * WAVE) {
             float a[B][IO::U];
 #pragma unroll
-            for (int b = 0; b < B; ++b) IO::load_stream(xr, min(u0 + b * WAVE, units - 1), a[b]);
+            for (int b = 0; b < B; ++b) IO::load_stream(xr, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes), a[b]);
 #pragma unroll
             for (int j = 0; j < G; ++j) {
                 if (j < np) {
                     const char *row = (const char *)dispatched + (int64_t)max(s[j], 0) * row_bytes;
                     float d[B][IO::U];
 #pragma unroll
-                    for (int b = 0; b < B; ++b) IO::load_stream(row, min(u0 + b * WAVE, units - 1), d[b]);
+                    for (int b = 0; b < B; ++b) IO::load_stream(row, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes), d[b]);
 #pragma unroll
                     for (int b = 0; b < B; ++b) {
                         const bool live = s[j] >= 0 && u0 + b * WAVE < units;
@@ -208,6 +213,122 @@ __global__ __launch_bounds__(256) void bwd_gate_kernel(
                         for (int i = 0; i < IO::U; ++i) acc[j] = live ? fmaf(d[b][i], a[b][i], acc[j]) : acc[j];
                     }
                 }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+            if (j >= np) break;
+            const float r = wave_sum(acc[j]);
+            if (lane == 0) grad_gates[(int64_t)(j0 + j) * stride + t] = r;
+        }
+    }
+}
+
+// ------------------------------------------------------------------ combine's backward pass
+// dispatch_kernel's scatter of the gated gradient and bwd_gate_kernel's products in one pass over the gradient:
+// grad_rows[slot_j] = 0 + gate_j * grad[t], grad_gates[j][t] = <rows[slot_j], grad[t]>.  Bound by memory (8192 x
+// 2048 fp32, two choices: 335 MB where the two launches move 402).
+template <int DT, int MODE>
+__global__ __launch_bounds__(256) void combine_bwd_kernel(
+    const void *__restrict__ grad, const void *__restrict__ rows, const float *__restrict__ gates,
+    const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
+    int top_k, int samples, int model_dim, int experts, int capacity,
+    void *__restrict__ grad_rows, float *__restrict__ grad_gates, const uint32_t *__restrict__ flags, int token_blocks)
+{
+    using IO = RowIO<DT, MODE>;
+    constexpr int G = 4, B = 2;
+    const int wave = threadIdx.x >> 6, lane = lane_id();
+    const int units = IO::units(model_dim);
+    const int row_bytes = model_dim * (int)sizeof(typename Elem<DT>::store_t);
+
+    if ((int)blockIdx.x >= token_blocks) {
+        const int slots = experts * capacity;
+        const int nwaves = (gridDim.x - token_blocks) * 4;
+        for (int s = (blockIdx.x - token_blocks) * 4 + wave; s < slots; s += nwaves) {
+            if (flags[s]) continue;
+            char *row = (char *)grad_rows + (int64_t)s * row_bytes;
+            for (int u = lane; u < units; u += WAVE) IO::store_zero(row, IO::at(u, row_bytes));
+        }
+        return;
+    }
+
+    const int t = blockIdx.x * 4 + wave;
+    if (t >= samples) return;
+    const char *gr = (const char *)grad + (int64_t)t * row_bytes;
+    for (int j0 = 0; j0 < top_k; j0 += G) {
+        const int np = min(G, top_k - j0);
+        int slot; float gate;
+        fetch_planes(gates, indices, locations, stride, t, j0, np, experts, capacity, slot, gate);
+        int s[G];
+        float g[G], acc[G];
+#pragma unroll
+        for (int j = 0; j < G; ++j) { s[j] = j < np ? rl_i(slot, j) : -1; g[j] = rl_f(gate, j); acc[j] = 0.f; }
+        if constexpr (MODE == ROWS_16) {
+            for (int u0 = lane; u0 < units; u0 += B * WAVE) {
+                int off[B];
+                float a[B][IO::U];
+#pragma unroll
+                for (int b = 0; b < B; ++b) {
+                    off[b] = IO::at(min(u0 + b * WAVE, units - 1), row_bytes);
+                    IO::load(gr, off[b], a[b]);
+                }
+                // every choice's row is requested before the first is used (a dropped choice reads slot 0, unused: capacity >= 1)
+                float d[G][B][IO::U];
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    if (j < np) {
+#pragma unroll
+                        for (int b = 0; b < B; ++b) IO::load((const char *)rows + (int64_t)max(s[j], 0) * row_bytes, off[b], d[j][b]);
+                    }
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    if (s[j] < 0) continue;
+                    char *to = (char *)grad_rows + (int64_t)s[j] * row_bytes;
+#pragma unroll
+                    for (int b = 0; b < B; ++b) {
+                        const bool live = u0 + b * WAVE < units;
+                        float o[IO::U];
+#pragma unroll
+                        for (int i = 0; i < IO::U; ++i) {
+                            acc[j] = live ? fmaf(d[j][b][i], a[b][i], acc[j]) : acc[j];
+                            o[i] = 0.f + g[j] * a[b][i];
+                        }
+                        if (live) IO::store(to, off[b], o);
+                    }
+                }
+            }
+        } else {
+            // rows as dwords for the scatter, then (from the caches) element by element for the sums, as bwd_gate_kernel
+            for (int u = lane; u < units; u += WAVE) {
+                const int off = IO::at(u, row_bytes);
+                float a[IO::U];
+                IO::load(gr, off, a);
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    if (s[j] < 0) continue;
+                    float o[IO::U];
+#pragma unroll
+                    for (int i = 0; i < IO::U; ++i) o[i] = 0.f + g[j] * a[i];
+                    IO::store((char *)grad_rows + (int64_t)s[j] * row_bytes, off, o);
+                }
+            }
+            using E = Elem<DT>;
+            constexpr int S = 8;
+            for (int u0 = lane; u0 < model_dim; u0 += S * WAVE) {
+                float a[S], d[G][S];
+#pragma unroll
+                for (int b = 0; b < S; ++b) a[b] = E::load(gr, min(u0 + b * WAVE, model_dim - 1));
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    if (j < np) {
+#pragma unroll
+                        for (int b = 0; b < S; ++b)
+                            d[j][b] = E::load((const char *)rows + (int64_t)max(s[j], 0) * row_bytes, min(u0 + b * WAVE, model_dim - 1));
+                    }
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+#pragma unroll
+                    for (int b = 0; b < S; ++b) acc[j] = s[j] >= 0 && u0 + b * WAVE < model_dim ? fmaf(d[j][b], a[b], acc[j]) : acc[j];
             }
         }
 #pragma unroll
@@ -274,17 +395,11 @@ extern "C" int planmoe_dispatch_fwd(const void *x, int dtype, const float *gates
     launch_slot_flags(flags, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
     const int token_blocks = (samples + 3) / 4;
     const int fill_blocks = min((slots + 3) / 4, 2048);
-    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
-    const bool vector = (model_dim % vec == 0) && aligned16(x) && aligned16(dispatched);
+    const int mode = rows_mode(dtype, model_dim, x, dispatched);
     PM_DTYPE_SWITCH(dtype, DT, {
-        if (vector)
-            dispatch_kernel<DT, true><<<token_blocks + fill_blocks, 256, 0, st>>>(
-                x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts,
-                capacity, dispatched, flags, token_blocks);
-        else
-            dispatch_kernel<DT, false><<<token_blocks + fill_blocks, 256, 0, st>>>(
-                x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts,
-                capacity, dispatched, flags, token_blocks);
+        PM_ROWS_SWITCH(mode, MODE, (dispatch_kernel<DT, MODE><<<token_blocks + fill_blocks, 256, 0, st>>>(
+            x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, dispatched, flags,
+            token_blocks)));
     });
     PM_LAUNCH_CHECK("planmoe_dispatch_fwd");
     return 0;
@@ -302,28 +417,20 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     PM_REQUIRE(out, "planmoe_combine_fwd: out is NULL");
     PM_REQUIRE(dispatched || capacity == 0, "planmoe_combine_fwd: dispatched is NULL");
     hipStream_t st = (hipStream_t)stream;
-    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
-    const bool vector = (model_dim % vec == 0) && aligned16(out) && aligned16(dispatched);
+    const int mode = rows_mode(dtype, model_dim, out, dispatched);
     const int blocks = (samples + 3) / 4;
     if (capacity == 0) {
         // no slot exists, every choice is dropped: zero rows.  (combine_kernel fetches rows with
         // unconditional loads at clamped slots and must not run without a row to read.)
         PM_DTYPE_SWITCH(dtype, DT, {
-            if (vector) zero_rows_kernel<DT, true><<<blocks, 256, 0, st>>>(out, samples, model_dim);
-            else zero_rows_kernel<DT, false><<<blocks, 256, 0, st>>>(out, samples, model_dim);
+            PM_ROWS_SWITCH(mode, MODE, (zero_rows_kernel<DT, MODE><<<blocks, 256, 0, st>>>(out, samples, model_dim)));
         });
         PM_LAUNCH_CHECK("planmoe_combine_fwd");
         return 0;
     }
     PM_DTYPE_SWITCH(dtype, DT, {
-        if (vector)
-            combine_kernel<DT, true><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations,
-                                                            plane_stride, top_k, samples, model_dim,
-                                                            capacity, out);
-        else
-            combine_kernel<DT, false><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations,
-                                                             plane_stride, top_k, samples, model_dim,
-                                                             capacity, out);
+        PM_ROWS_SWITCH(mode, MODE, (combine_kernel<DT, MODE><<<blocks, 256, 0, st>>>(
+            dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out)));
     });
     PM_LAUNCH_CHECK("planmoe_combine_fwd");
     return 0;
@@ -346,19 +453,45 @@ extern "C" int planmoe_bwd_gate(const void *x, const void *dispatched, int dtype
         PM_LAUNCH_CHECK("planmoe_bwd_gate");
         return 0;
     }
-    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
-    const bool vector = (model_dim % vec == 0) && aligned16(x) && aligned16(dispatched);
+    const int mode = rows_mode(dtype, model_dim, x, dispatched);
     const int blocks = (samples + 3) / 4;
     PM_DTYPE_SWITCH(dtype, DT, {
-        if (vector)
-            bwd_gate_kernel<DT, true><<<blocks, 256, 0, st>>>(x, dispatched, indices, locations,
-                                                             plane_stride, top_k, samples,
-                                                             model_dim, capacity, grad_gates);
+        if (mode == ROWS_16)
+            bwd_gate_kernel<DT, ROWS_16><<<blocks, 256, 0, st>>>(
+                x, dispatched, indices, locations, plane_stride, top_k, samples, model_dim, capacity, grad_gates);
         else
-            bwd_gate_kernel<DT, false><<<blocks, 256, 0, st>>>(x, dispatched, indices, locations,
-                                                              plane_stride, top_k, samples,
-                                                              model_dim, capacity, grad_gates);
+            bwd_gate_kernel<DT, ROWS_1><<<blocks, 256, 0, st>>>(
+                x, dispatched, indices, locations, plane_stride, top_k, samples, model_dim, capacity, grad_gates);
     });
     PM_LAUNCH_CHECK("planmoe_bwd_gate");
+    return 0;
+}
+
+extern "C" int planmoe_combine_bwd(const void *grad, const void *dispatched, int dtype, const float *gates,
+                                   const int32_t *indices, const int32_t *locations, int64_t plane_stride,
+                                   int top_k, int samples, int model_dim, int experts, int capacity,
+                                   void *grad_dispatched, float *grad_gates, void *workspace,
+                                   size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_combine_bwd";
+    if (check_planes(who, indices, locations, plane_stride, top_k, samples)) return 1;
+    PM_REQUIRE(dtype_ok(dtype), "%s: bad dtype %d", who, dtype);
+    PM_REQUIRE(model_dim >= 1 && experts >= 1 && capacity >= 1 && samples >= 1, "%s: bad shape", who);
+    PM_REQUIRE((int64_t)experts * capacity < (1ll << 31), "%s: experts*capacity overflows int32", who);
+    PM_REQUIRE((int64_t)samples * top_k < (1ll << 31), "%s: samples*top_k overflows int32", who);
+    PM_REQUIRE(grad && dispatched && grad_dispatched && grad_gates, "%s: NULL argument", who);
+    PM_REQUIRE(workspace && workspace_bytes >= planmoe_dispatch_workspace_bytes(experts, capacity), "%s: workspace too small", who);
+    hipStream_t st = (hipStream_t)stream;
+    uint32_t *flags = (uint32_t *)workspace;
+    const int slots = experts * capacity;
+    launch_slot_flags(flags, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const int token_blocks = (samples + 3) / 4, fill_blocks = min((slots + 3) / 4, 2048);
+    const int mode = std::min(rows_mode(dtype, model_dim, grad, dispatched), rows_mode(dtype, model_dim, grad_dispatched, grad_dispatched));
+    PM_DTYPE_SWITCH(dtype, DT, {
+        PM_ROWS_SWITCH(mode, MODE, (combine_bwd_kernel<DT, MODE><<<token_blocks + fill_blocks, 256, 0, st>>>(
+            grad, dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity,
+            grad_dispatched, grad_gates, flags, token_blocks)));
+    });
+    PM_LAUNCH_CHECK(who);
     return 0;
 }

@@ -1,10 +1,12 @@
 """Routing and dispatch/combine API -- mirror of the reference's impls/fast_dispatch.py.
 
 Same names, arguments, defaults and return structure; the work is done by libplanmoe_hip
-(one launch for all k choices instead of one JIT kernel launch per choice)."""
+(one launch for all k choices instead of one JIT kernel launch per choice).  On the GPU the host side is
+csrc/ext/routing.cpp; what it does not take as it is (no tokens, no slots, planes of other types, host
+tensors) goes through the classes below."""
 import torch
 
-from . import host_route, losses, ops
+from . import ext, host_route, losses, ops
 from ._lib import PlanMoEError
 from .gating import fast_cumsum_sub_one  # noqa: F401  (re-exported like the reference)
 
@@ -107,6 +109,10 @@ class TutelMoeFastDispatcher:
             out = GatingEncoder.apply(self, host) if self.is_postscore else GatingEncoder.apply(self, host, *self.gates_)
             return out.to(self.original_dtype)
         data = data.to(self.original_dtype).contiguous()
+        out = ext.layer().encode(data, [] if self.is_postscore else self.gates_, self.indices_, self.locations_,
+                                 self.num_global_experts, self.capacity)
+        if out is not None:
+            return out.view(-1, data.size(-1))
         if self.is_postscore:
             return GatingEncoder.apply(self, data)
         return GatingEncoder.apply(self, data, *self.gates_)
@@ -117,6 +123,10 @@ class TutelMoeFastDispatcher:
             out = GatingDecoder.apply(self, host, *self.gates_) if self.is_postscore else GatingDecoder.apply(self, host)
             return out.to(self.original_dtype)
         data = data.to(self.original_dtype).contiguous()
+        out = ext.layer().decode(data, self.gates_ if self.is_postscore else [], self.indices_, self.locations_,
+                                 self.num_global_experts, self.capacity)
+        if out is not None:
+            return out
         if self.is_postscore:
             return GatingDecoder.apply(self, data, *self.gates_)
         return GatingDecoder.apply(self, data)
@@ -137,6 +147,7 @@ class _Route(torch.autograd.Function):
         scores = r["scores"] if is_logits else inp.detach().contiguous()
         ctx.save_for_backward(scores, r["indices"], r["counts"])
         ctx.normalize_gate, ctx.is_logits, ctx.want_l_aux = normalize_gate, is_logits, want_l_aux
+        ctx.set_materialize_grads(False)         # (three integer outputs: no zeros in place of their gradients)
         l_aux = r["l_aux"] if want_l_aux else inp.new_zeros(())
         ctx.mark_non_differentiable(r["indices"], r["locations"], r["counts"])
         return r["gates"], l_aux, r["indices"], r["locations"], r["counts"]
@@ -144,6 +155,8 @@ class _Route(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_gates, grad_l_aux, *unused):
         scores, indices, counts = ctx.saved_tensors
+        if grad_gates is None and grad_l_aux is None:
+            return None, None, None, None, None
         if grad_gates is None:
             grad_gates = torch.zeros((indices.shape[0], scores.shape[0]), dtype=scores.dtype, device=scores.device)
         dl = grad_l_aux if (ctx.want_l_aux and grad_l_aux is not None) else None
@@ -171,8 +184,13 @@ def extract_critical(scores, top_k, loss_fn=losses.gshard_loss, capacity_factor=
         return host_route.extract_critical(scores, top_k, loss_fn, capacity_factor, batch_prioritized_routing,
                                            normalize_gate, alignment)
     num_global_experts = int(scores.size(1))
-    top_k = min(top_k, num_global_experts)
     want_kernel_loss = loss_fn is losses.gshard_loss
+    if not batch_prioritized_routing and capacity_factor > 0 and (want_kernel_loss or loss_fn is None):
+        out = ext.layer().extract_critical(scores, top_k, want_kernel_loss, capacity_factor, normalize_gate, alignment)
+        if out is not None:
+            indices_s, locations_s, gates_s, capacity, l_loss = out
+            return (num_global_experts, indices_s, locations_s, gates_s, capacity), l_loss
+    top_k = min(top_k, num_global_experts)
     gates, l_aux, indices, locations, _ = route(scores, top_k, False, normalize_gate, want_kernel_loss)
     if batch_prioritized_routing:
         importance_scores = -1 * scores.detach().max(dim=1)[0]
@@ -207,7 +225,11 @@ def extract_critical(scores, top_k, loss_fn=losses.gshard_loss, capacity_factor=
 
 def fast_encode(data, critial_data, is_postscore=True):
     # fast_dispatch.py:197-201
-    num_global_experts = critial_data[0]
+    num_global_experts, indices_s, locations_s, gates_s, capacity = critial_data
+    if data.is_cuda:
+        out = ext.layer().encode(data, [] if is_postscore else gates_s, indices_s, locations_s, num_global_experts, capacity)
+        if out is not None:
+            return out
     dispatcher = TutelMoeFastDispatcher(num_global_experts, 0, data.size(-1), data.dtype)
     dispatcher.update(*critial_data[1:], is_postscore=is_postscore)
     return dispatcher.encode(data).view(num_global_experts, -1, data.size(-1))
@@ -215,7 +237,11 @@ def fast_encode(data, critial_data, is_postscore=True):
 
 def fast_decode(data, critial_data, is_postscore=True):
     # fast_dispatch.py:203-207
-    num_global_experts = critial_data[0]
+    num_global_experts, indices_s, locations_s, gates_s, capacity = critial_data
+    if data.is_cuda:
+        out = ext.layer().decode(data, gates_s if is_postscore else [], indices_s, locations_s, num_global_experts, capacity)
+        if out is not None:
+            return out
     dispatcher = TutelMoeFastDispatcher(num_global_experts, 0, data.size(-1), data.dtype)
     dispatcher.update(*critial_data[1:], is_postscore=is_postscore)
     return dispatcher.decode(data.reshape(-1, data.size(-1))).view(-1, data.size(-1))
