@@ -329,6 +329,11 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 
     int j = blockIdx.x / 8;
     if (!in_range(j)) return;
+    // a quarter may lie behind the rows or columns in use (a work-group has one quarter at most): nothing to read or store
+    if (p.split == 2) {
+        const Where w = locate(j);
+        if (w.m0 >= (TA ? p.M : w.rows) || w.n0 >= p.N) return;
+    }
     Cursor c0, c1, c2, c3;                        // k-tiles 0 .. 3 from here
     c0.j = j;
     seek(c0);
@@ -385,7 +390,7 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         const uint32_t put = ((uint32_t)(wm * 32 * I + l / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
         const int M = TA ? p.M : here.rows;
         const int64_t corner = (int64_t)here.e * p.sC + (int64_t)here.m0 * p.ldc + here.n0;
-        const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2);
+        const int bytes = (int)max((int64_t)0, min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2));
         const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t mask = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(GRAD ? p.mask + corner : p.C), 0, GRAD ? bytes : 0, 0x00020000);
 #pragma unroll

@@ -184,3 +184,30 @@ def test_gate_weight_gradient_and_row_sums(T, M, E, dtype):
     assert bool(((dw.double().cpu() - ref).abs() <= (T + 2) * 2.0 ** -24 * mag + half * ref.abs() + 1e-30).all())
     rows = x[:min(T, (T - T // 3 + 3) // 4 * 4)].double()
     assert bool(((out[0].double().cpu() - rows.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * rows.abs().sum(0) + half * rows.sum(0).abs() + 1e-30).all())
+
+
+# Rows that end on a tile of 256 or 128 and just behind one, batches of less than a tile and of no rows: a quarter of the last
+# round that has no rows stores nothing; several tiles for a work-group; the last one has no row counts
+@pytest.mark.parametrize("n,k,hint,counts", [(1024, 512, 4096, [4096, 4097, 4160, 4161]), (1024, 512, 4096, [4224, 4225, 128, 1]),
+                                             (2048, 2048, 500, [512, 513, 576, 577, 500, 64, 1, 0]), (1024, 1024, 0, [4160] * 4)])
+def test_expert_gemm_rows_around_a_tile(n, k, hint, counts):
+    from planmoe_amd import ops
+    print("case", n, k, counts, flush=True)
+    B, cap, dtype = len(counts), max(counts) + (64 if hint else 0), torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(sum(counts))
+    a, w = torch.randn(B, cap, k, device=DEV, generator=g).to(dtype), torch.randn(B, k, n, device=DEV, generator=g).to(dtype)
+    bias, h = torch.randn(B, n, device=DEV, generator=g).to(dtype), torch.randn(B, cap, n, device=DEV, generator=g).clamp(min=0).to(dtype)
+    live = torch.tensor([counts], dtype=torch.int32, device=DEV) if hint else None
+    out = torch.full((B, cap, n), 7.0, dtype=dtype, device=DEV)
+    masked = out.clone()
+    ops.expert_gemm("nn", a, w, bias, relu=True, live=live, out=out, rows_hint=hint)
+    _, db = ops.expert_gemm_relu_bwd(a, w.transpose(1, 2).contiguous(), h, live=live, out=masked, rows_hint=hint)
+    torch.cuda.synchronize()
+    for e, r in enumerate(counts):
+        ref, mag = a[e, :r].double() @ w[e].double(), a[e, :r].double().abs() @ w[e].double().abs()
+        tol, biased = _bound(ref, mag, k, dtype), ref + bias[e].double()
+        assert bool(((out[e, :r].double() - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all()), e
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all()), e
+        assert bool((out[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all()), e
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), e
