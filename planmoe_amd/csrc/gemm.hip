@@ -393,6 +393,17 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         const int bytes = (int)max((int64_t)0, min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2));
         const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t mask = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(GRAD ? p.mask + corner : p.C), 0, GRAD ? bytes : 0, 0x00020000);
+        // GRAD: a piece's masks are asked for while the piece before is worked on and ahead of its stores (asked for when
+        // they were wanted, each piece waited for memory and for the stores before it: 337 us at 8 x 4096 x 4096 x 1024)
+        pm_u32x4 keep[2][2 * J];
+        auto ask = [&](int n) {                   // piece n: half b of the columns, half a of the rows, fragment i
+            const int b = n / (2 * I), a = n / I % 2, i = n % I;
+            const uint32_t at = here.n0 + 64 * J * b + put_col < p.N ? put : GEMM_NOWHERE;
+#pragma unroll
+            for (int t = 0; t < 2 * J; ++t)
+                keep[n & 1][t] = __builtin_amdgcn_raw_buffer_load_b128(mask, at, ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u, 0);
+        };
+        if (GRAD) ask(0);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             const uint32_t put_b = here.n0 + 64 * J * b + put_col < p.N ? put : GEMM_NOWHERE;
@@ -412,10 +423,8 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 #pragma unroll
                 for (int i = 0; i < I; ++i) {
                     auto so = [&](int t) { return ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u; };
-                    pm_u32x4 keep[2 * J];
-                    if (GRAD)
-#pragma unroll
-                        for (int t = 0; t < 2 * J; ++t) keep[t] = __builtin_amdgcn_raw_buffer_load_b128(mask, put_b, so(t), 0);
+                    const int n = (2 * b + a) * I + i;
+                    if (GRAD && n + 1 < 4 * I) ask(n + 1);
 #pragma unroll
                     for (int jj = 0; jj < J; ++jj)
                         asm volatile("" : "+a"(acc[a][b][i][jj]));      // (in the accumulator registers until here: copied all at once they would not fit)
@@ -446,7 +455,7 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
                         if (GRAD) {               // relu's backward: kept where its output was positive
 #pragma unroll
                             for (int x = 0; x < 4; ++x) {
-                                const uint32_t k = keep[t][x];
+                                const uint32_t k = keep[n & 1][t][x];
                                 v[x] &= ((int)(k << 16) > 0 ? 0xffffu : 0u) | ((int)k >= 0x10000 ? 0xffff0000u : 0u);
                                 add[2 * x] += __uint_as_float(v[x] << 16);
                                 add[2 * x + 1] += __uint_as_float(v[x] & 0xffff0000u);
@@ -455,6 +464,10 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
                             }
                         }
                         __builtin_amdgcn_raw_buffer_store_b128(v, out, put_b, so(t), 0);
+                        // A vector instruction that writes the first register of a 16-byte store right behind it can reach
+                        // the stored value (seen with a scalar offset, where the compiler leaves no gap): results of one
+                        // column in eight were the next address.  The value is held over a gap.
+                        asm volatile("s_nop 1" :: "v"(v));
                         if (GRAD) __builtin_amdgcn_sched_barrier(0);         // (one piece's temporaries at a time: the registers are full)
                     }
                     __builtin_amdgcn_wave_barrier();
@@ -661,8 +674,9 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who)
                          (last == 0 ? 0. : 2 * last <= cu ? gemm_cost_small(4 * last, kt, cu) + 3 : (1.0 + 0.3 * (double)last / (double)cu) * kt + 10);
     if (gemm_cost_small(small, kt, cu) < t_big) return gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who);
     p.stay = (int)(cu / 8 * 8);
-    // (with many rounds the last one hardly counts, and a launch that may find nothing to do costs 3 us)
-    p.split = big < 6 * cu && (p.live ? true : gemm_last_round((int)big, p.stay) > 0);
+    // (with many rounds the last one hardly counts, and a launch that may find nothing to do costs 3 us; a weight
+    // gradient's tiles are known here)
+    p.split = big < 6 * cu && (p.live && !TA ? true : gemm_last_round((int)big, p.stay) > 0);
     if (gemm_launch<2, 2, TA, TB, GRAD>(p, stream, who)) return 1;
     if (!p.split) return 0;
     p.split = 2;
