@@ -805,9 +805,10 @@ extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void
     int tile_rows, slots;
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
-        tile_rows = gemm_f32_tile(1, p, hint);
+        const int side = gemm_f32_tile(1, p, hint);
+        tile_rows = side ? side : 64;
         slots = (m + tile_rows - 1) / tile_rows * 2;
-        if (gemm_f32_run(1, p, tile_rows, st, who)) return 1;
+        if (gemm_f32_run(1, p, side, st, who)) return 1;
     } else {
         GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
                    m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};

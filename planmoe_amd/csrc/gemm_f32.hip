@@ -196,6 +196,118 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     }
 }
 
+// Few rows: a wave on its own, 16 MF rows by 16 columns, operands from memory straight into registers
+// (no LDS, no barrier), 2 U steps of 16 k in flight.  v_mfma_f32_16x16x4_f32 with lane group g at k = 4 g + q: the sums
+// take the k in the same order as the tiles do, so which kernel serves a shape does not show in the result.
+// Bound by reading the weight (tiles of 64 x 64 wait a trip to memory for every 32 k and there are few of them: 8 experts
+// of 2 rows, 4096 -> 1024, 134 MB: 90 us, here 39).  U: nn reads a k at a time, 64 bytes of a row, and takes twice
+// the steps in flight that nt does (nn with 8: 90 us; nt with 16: 40 us, and 26 in place of 23 at 1024 -> 4096).
+template <int MF, int U, bool TB>
+__global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args p)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
+    const int e = blockIdx.z, m0 = blockIdx.y * 16 * MF, n0 = (blockIdx.x * 4 + wave) * 16;
+    int M = p.M;
+    if (p.live) {
+        int n = 0;
+        for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
+        M = min(M, (n + p.live_round - 1) / p.live_round * p.live_round);
+    }
+    // (column sums have two slots for every 64 rows in use: the second of them may have no rows)
+    if (m0 >= (p.colsum ? (M + 63) / 64 * 64 : M) || n0 >= p.N) return;
+    const float *A = p.A + (int64_t)e * p.M * p.K, *B = p.B + (int64_t)e * p.N * p.K;
+    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, M * p.K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, p.N * p.K * 4, 0x00020000);
+    constexpr uint32_t NOWHERE = 0x80000000u;
+    const int steps = (p.K + 15) / 16, col = n0 + l16;
+
+    f32x4 acc[MF], fa[2][U][MF], fb[2][U];
+#pragma unroll
+    for (int m = 0; m < MF; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // rows and columns past the end, and k past the end, read as zero
+    auto load = [&](f32x4 (&a)[U][MF], f32x4 (&b)[U], int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = 16 * (s0 + u) + 4 * g;
+            const bool in_k = k < p.K;
+#pragma unroll
+            for (int m = 0; m < MF; ++m) {
+                const int row = m0 + 16 * m + l16;
+                a[u][m] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(da, in_k && row < M ? ((uint32_t)row * (uint32_t)p.K + (uint32_t)k) * 4u : NOWHERE, 0, 0));
+            }
+            if (TB) {
+                const uint32_t at = in_k && col < p.N ? ((uint32_t)k * (uint32_t)p.N + (uint32_t)col) * 4u : NOWHERE;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) b[u][q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(db, at, (uint32_t)(q * 4) * (uint32_t)p.N, 0));
+            } else {
+                b[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(db, in_k && col < p.N ? ((uint32_t)col * (uint32_t)p.K + (uint32_t)k) * 4u : NOWHERE, 0, 0));
+            }
+        }
+    };
+    // (the second operand first: a lane then holds four consecutive columns of one row)
+    auto multiply = [&](const f32x4 (&a)[U][MF], const f32x4 (&b)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int m = 0; m < MF; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][q], a[u][m][q], acc[m], 0, 0, 0);
+    };
+    load(fa[0], fb[0], 0);
+    for (int s = 0; s < steps; s += 2 * U) {
+        // (held in this order: moved behind the products to save registers, the loads would be waited for)
+        load(fa[1], fb[1], s + U);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fa[0], fb[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(fa[0], fb[0], s + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fa[1], fb[1]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    const int c = n0 + 4 * g;                    // (N is a multiple of 4: a lane's columns are in or out together)
+    const bool in_n = c < p.N;
+    f32x4 add = {0.f, 0.f, 0.f, 0.f}, sums = add;
+    if (p.bias && in_n)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) add[x] = p.bias[(int64_t)e * p.N + c + x];
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+        const int row = m0 + 16 * m + l16;
+        const int64_t at = ((int64_t)e * p.M + row) * p.N + c;
+        const bool inside = in_n && row < M;
+        f32x4 v = acc[m];
+        if (p.bias) v += add;
+        if (p.relu)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) v[x] = v[x] < 0.f ? 0.f : v[x];
+        if (p.mask) {
+            f32x4 k = {0.f, 0.f, 0.f, 0.f};
+            if (inside) k = *reinterpret_cast<const f32x4 *>(p.mask + at);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) { v[x] = k[x] > 0.f ? v[x] : 0.f; sums[x] += v[x]; }
+        }
+        if (inside) *reinterpret_cast<f32x4 *>(p.C + at) = v;
+    }
+    if (p.colsum) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int d = 1; d < 16; d <<= 1) sums[x] += __shfl_xor(sums[x], d);
+        if (l16 == 0 && in_n) *reinterpret_cast<f32x4 *>(p.colsum + ((int64_t)e * ((p.M + 63) / 64 * 2) + m0 / 32) * p.N + c) = sums;
+    }
+}
+
+template <int MF, int U, bool TB>
+static int gemm_f32_wave_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
+{
+    const int rows = p.colsum ? (p.M + 63) / 64 * 64 : p.M;
+    gemm_f32_wave_kernel<MF, U, TB><<<dim3((unsigned)((p.N + 63) / 64), (unsigned)((rows + 16 * MF - 1) / (16 * MF)), (unsigned)p.batches), 256, 0, stream>>>(p);
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
 template <int F, bool TA, bool TB>
 static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
 {
@@ -218,8 +330,13 @@ static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *
 
 // The tile's side: a compute unit's matrix cores take 1.7 us for a k-tile of 128 x 128 and a quarter of that, and
 // a tenth, for one of 64 x 64; what counts is the fullest compute unit (4 x 300 x 512 x 1024: 64 tiles of 128, 57 us).
+// 0, waves on their own, up to 32 rows, where they read the weight once (8 experts, 2 rows each: nn 1024 -> 4096 44 -> 27 us,
+// nt 41 -> 23, 4096 -> 1024 90 -> 39; 60 rows, nt 512 -> 2048: 23 -> 31).
 int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
 {
+    if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && p.batches <= 65535 &&
+        p.M <= 32 * 65535)
+        return 0;
     const int64_t m = form == 2 ? p.M : rows_hint;
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
     auto cost = [&](int64_t side, double us) {
@@ -233,6 +350,10 @@ int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, co
 {
     PM_REQUIRE((int64_t)p.K * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.M * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.N * 4 * 128 < ((int64_t)1 << 31),
                "%s: 128 rows of an operand must stay under 2 GiB", who);
+    if (side == 0) {
+        if (p.M <= 16 && !p.colsum) return form == 0 ? gemm_f32_wave_launch<1, 16, true>(p, stream, who) : gemm_f32_wave_launch<1, 8, false>(p, stream, who);
+        return form == 0 ? gemm_f32_wave_launch<2, 8, true>(p, stream, who) : gemm_f32_wave_launch<2, 4, false>(p, stream, who);
+    }
     if (side == 64) {
         if (form == 0) return gemm_f32_launch<1, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<1, false, false>(p, stream, who);

@@ -12,8 +12,8 @@ struct Gemm32Args {
     int M, N, K, batches, relu;            // operands and result contiguous
 };
 
-// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  side: rows and columns of a tile, 64 or 128
-// (gemm_f32_tile picks it for a number of rows in use)
+// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  side: rows and columns of a tile, 64 or 128, or 0:
+// no tiles, waves on their own (gemm_f32_tile picks it for a number of rows in use); column sums then have two slots for 64 rows
 int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint);
 int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who);
 

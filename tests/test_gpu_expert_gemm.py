@@ -211,3 +211,34 @@ def test_expert_gemm_rows_around_a_tile(n, k, hint, counts):
         assert bool((out[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all()), e
         stored = masked[e, :r].double()
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), e
+
+
+# fp32: few rows are served by waves on their own, whose sums take the reduction in the tiles' order: the first
+# rows of a product do not depend on how many rows there are.  Either side of 16 and 32 rows, k steps and columns that are not whole
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33])
+@pytest.mark.parametrize("n,k", [(4, 4), (68, 20), (136, 520), (1104, 132)])
+def test_expert_gemm_fp32_does_not_depend_on_the_number_of_rows(m, n, k):
+    from planmoe_amd import ops
+    print("case", m, n, k, flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    B, many = 2, 16384                           # (the many rows: 128 x 128 tiles)
+    live = torch.tensor([[m, m // 2]], dtype=torch.int32)
+    a, w, bias = torch.randn(B, many, k, generator=g).to(DEV), torch.randn(B, k, n, generator=g), torch.randn(B, n, generator=g).to(DEV)
+    wt, w, few = w.transpose(1, 2).contiguous().to(DEV), w.to(DEV), a[:, :m].clone()
+    h = torch.randn(B, m, n, generator=g).clamp(min=0)
+    for e in range(B):
+        few[e, int(live[0, e]):] = float("nan")
+    nn, nt = torch.full((B, m, n), 7.0, device=DEV), torch.full((B, m, n), 7.0, device=DEV)
+    masked = nn.clone()
+    ops.expert_gemm("nn", few, w, bias, relu=True, live=live.to(DEV), out=nn)
+    ops.expert_gemm("nt", few, wt, live=live.to(DEV), out=nt)
+    _, db = ops.expert_gemm_relu_bwd(few, wt, h.to(DEV), live=live.to(DEV), out=masked)
+    want_nn, want_nt = ops.expert_gemm("nn", a, w, bias, relu=True), ops.expert_gemm("nt", a, wt)
+    torch.cuda.synchronize()
+    for e in range(B):
+        r = int(live[0, e])
+        assert torch.equal(nn[e, :r], want_nn[e, :r]) and torch.equal(nt[e, :r], want_nt[e, :r])
+        assert torch.equal(masked[e, :r], torch.where(h[e, :r].to(DEV) > 0, want_nt[e, :r], torch.zeros((), device=DEV)))
+        assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all())
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all())
