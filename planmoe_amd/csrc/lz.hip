@@ -18,7 +18,8 @@
 // The launches: sizes of every block (match + parse, nothing written but two integers and a
 // class byte per block), an in-place exclusive scan of the sizes (chunks, then chunk totals),
 // placement (stored blocks are copied straight through, the others analysed again and packed at
-// their final offset), and a launch that zeroes what lies beyond the totals.  The reference
+// their final offset), and a launch that zeroes what lies beyond the totals.  Up to 16 MB there is one
+// chunk: no totals to scan, and the placement's spare work-groups do the zeroing.  The reference
 // stages every block at a fixed stride in a buffer as large as the input, scans with a library
 // call and copies everything once more (gpulz.cu:148-211, 460-494, 220-258); here no
 // full-size temporary exists and no work-group ever waits for another.
@@ -154,44 +155,50 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
         b.data_bytes = LZ_BLOCK_BYTES;
         return LZ_STORED;
     }
-    uint32_t any = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) any |= (uint32_t)((hit[i] >> lane) & 1u) << i;
-
-    // ---- hit masks: bit j of hits[i] = symbol 8l+i equals window symbol 8l+i-32+j.
-    // They hold all the matcher needs: while symbol p+r still equals window symbol w+r, bit
-    // (w - p + 32) of the mask of position p+r is set.
-    uint32_t hits[8];
+    uint32_t any = 0, live = 0;                         // live: positions that some lane has a hit at
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        hits[i] = 0;
-        if (hit[i] == 0) continue;
-        const uint32_t k = ahead_key(own[i]);
-        uint32_t m = 0;
-#pragma unroll
-        for (int j = LZ_WINDOW - 1; j >= 0; --j) m = shift_in_equal(m, k, win[i + j]);
-        hits[i] = m;
+        any |= (uint32_t)((hit[i] >> lane) & 1u) << i;
+        live |= hit[i] != 0 ? 1u << i : 0u;
     }
+
+    // ---- hit masks: bit j of position 8l+i's = symbol 8l+i equals window symbol 8l+i-32+j.
+    // They hold all the matcher needs: while symbol p+r still equals window symbol w+r, bit
+    // (w - p + 32) of the mask of position p+r is set.
+    // (The positions are a loop, here and in the matcher: written out eight times the code was 15 KB walked once,
+    // and a wave alone on its compute unit waited for instructions most of its time.)
     uint32_t *hmask = keys;                             // the keys are all in registers by now
     wave_sync();
-    *reinterpret_cast<uint4 *>(hmask + 8 * lane) = make_uint4(hits[0], hits[1], hits[2], hits[3]);
-    *reinterpret_cast<uint4 *>(hmask + 8 * lane + 4) = make_uint4(hits[4], hits[5], hits[6], hits[7]);
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+        uint32_t m = 0;
+        if ((live >> i) & 1u) {
+            const uint32_t k = ahead_key(win[LZ_WINDOW]);
+#pragma unroll
+            for (int j = LZ_WINDOW - 1; j >= 0; --j) m = shift_in_equal(m, k, win[j]);
+        }
+        hmask[8 * lane + i] = m;
+#pragma unroll
+        for (int j = 0; j < 39; ++j) win[j] = win[j + 1];          // the next position's window and symbol
+    }
     wave_sync();
 
     // ---- the reference's matcher (gpulz.cu:46-85) on the masks: a run starts at the next hit,
     // grows while the following positions hit at the same distance, and the window symbol after
     // a run is consumed by the comparison that ended it
-    b.lens_lo = b.lens_hi = b.offs_lo = b.offs_hi = b.match_mask = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        if (hit[i] == 0) continue;
+    uint64_t lens = 0, offs = 0;
+    b.match_mask = 0;
+#pragma unroll 1
+    for (uint32_t todo = live; todo != 0; todo &= todo - 1) {
+        const int i = __builtin_ctz(todo);
         uint32_t len = 0, off = 0;
         if ((any >> i) & 1) {
             const int p = 8 * lane + i;
             const uint32_t room = (uint32_t)(LZ_SYMS - p);              // symbols left in the block
+            const uint32_t mask = hmask[p];
             uint32_t j = 0;
             while (j < (uint32_t)LZ_WINDOW) {
-                const uint32_t rest = hits[i] & (0xffffffffu << j);
+                const uint32_t rest = mask & (0xffffffffu << j);
                 if (rest == 0) break;
                 const uint32_t j0 = __builtin_ctz(rest);
                 // the run ends with the window (32 - j0 symbols from its start) or the block
@@ -211,10 +218,12 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
                 j = j0 + r + 1;
             }
         }
-        if (i < 4) { b.lens_lo |= len << (8 * i); b.offs_lo |= off << (8 * i); }
-        else       { b.lens_hi |= len << (8 * (i - 4)); b.offs_hi |= off << (8 * (i - 4)); }
+        lens |= (uint64_t)len << (8 * i);
+        offs |= (uint64_t)off << (8 * i);
         b.match_mask |= (uint32_t)(len != 0) << i;
     }
+    b.lens_lo = (uint32_t)lens; b.lens_hi = (uint32_t)(lens >> 32);
+    b.offs_lo = (uint32_t)offs; b.offs_hi = (uint32_t)(offs >> 32);
     wave_sync();                                        // hmask is the key area of the next block
 
     // ---- greedy parse: [cur, nxt) is a run of literals, nxt the next position with a match
@@ -279,9 +288,10 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
 // ---- launch 2: both tables, in place: exclusive sums inside chunks of 8192 entries, chunk totals
 __global__ __launch_bounds__(256) void lz_scan_chunks_kernel(int32_t *__restrict__ flag_off,
                                                             int32_t *__restrict__ data_off, int64_t entries,
-                                                            uint32_t *__restrict__ totals)
+                                                            uint32_t *__restrict__ totals, uint32_t *__restrict__ bases)
 {
     __shared__ uint32_t wave_tot[4];
+    if (gridDim.x == 1 && threadIdx.x < 2) bases[threadIdx.x] = 0;       // (no chunks before it: launch 3 is left out)
     constexpr int PER = LZ_SCAN_CHUNK / 256;            // 32 entries per thread, contiguous
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
     const int64_t e0 = (int64_t)blockIdx.x * LZ_SCAN_CHUNK + (int64_t)threadIdx.x * PER;
@@ -349,6 +359,26 @@ __global__ __launch_bounds__(LZ_MAX_CHUNKS) void lz_scan_totals_kernel(const uin
     }
 }
 
+// zero flags[flag_total ..) and data[data_total ..): 16 bytes per lane and step, neighbouring lanes at
+// neighbouring addresses (the piece the used part ends in byte by byte)
+__device__ __forceinline__ void lz_clear_slack(int64_t tid, int64_t nthreads, int32_t flag_total, int32_t data_total,
+                                               int64_t blocks, uint8_t *__restrict__ flags, uint8_t *__restrict__ data)
+{
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        uint8_t *buf = a ? data : flags;
+        const int64_t size = a ? blocks * LZ_BLOCK_BYTES : blocks * (LZ_SYMS / 8);     // multiples of 64
+        const int64_t used = min(max((int64_t)(a ? data_total : flag_total), (int64_t)0), size);
+        for (int64_t lo = (used / 16 + tid) * 16; lo < size; lo += nthreads * 16) {
+            if (lo >= used) {
+                *reinterpret_cast<uint4 *>(buf + lo) = make_uint4(0, 0, 0, 0);
+            } else {
+                for (int64_t q = used; q < lo + 16; ++q) buf[q] = 0;
+            }
+        }
+    }
+}
+
 struct __attribute__((aligned(16))) LzPlaceShared {
     uint32_t keys[LZ_WAVES][LZ_WINDOW + LZ_SYMS];
     uint16_t stage[LZ_WAVES][LZ_BLOCK_BYTES / 2];   // token bytes of the block
@@ -362,6 +392,14 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     uint8_t *__restrict__ flags, uint8_t *__restrict__ data)
 {
     __shared__ LzPlaceShared sh;
+    // With one chunk the totals are there already (their base is zero: the wave of the last block writes back what it
+    // read), and the work-groups behind the blocks' clear what lies beyond them: no launch 5.
+    const int64_t groups = (blocks + LZ_WAVES - 1) / LZ_WAVES;
+    if (blockIdx.x >= groups) {
+        lz_clear_slack(((int64_t)blockIdx.x - groups) * LZ_WAVES * WAVE + threadIdx.x, ((int64_t)gridDim.x - groups) * LZ_WAVES * WAVE,
+                       flag_off[blocks], data_off[blocks], blocks, flags, data);
+        return;
+    }
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
     const int64_t block = (int64_t)blockIdx.x * LZ_WAVES + wave;
@@ -454,27 +492,13 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
         *reinterpret_cast<uint16_t *>(dst + data_bytes - 2) = stage[data_bytes / 2 - 1];
 }
 
-// ---- launch 5: zero flags[flag_off[blocks] ..) and data[data_off[blocks] ..): 16 bytes per lane and step,
-// neighbouring lanes at neighbouring addresses (the piece the used part ends in byte by byte)
+// ---- launch 5: what lies beyond the totals
 __global__ __launch_bounds__(256) void lz_clear_slack_kernel(const int32_t *__restrict__ flag_off,
                                                             const int32_t *__restrict__ data_off,
                                                             int64_t blocks, uint8_t *__restrict__ flags,
                                                             uint8_t *__restrict__ data)
 {
-    const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x, nthreads = (int64_t)gridDim.x * 256;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        uint8_t *buf = a ? data : flags;
-        const int64_t size = a ? blocks * LZ_BLOCK_BYTES : blocks * (LZ_SYMS / 8);     // multiples of 64
-        const int64_t used = min(max((int64_t)(a ? data_off[blocks] : flag_off[blocks]), (int64_t)0), size);
-        for (int64_t lo = (used / 16 + tid) * 16; lo < size; lo += nthreads * 16) {
-            if (lo >= used) {
-                *reinterpret_cast<uint4 *>(buf + lo) = make_uint4(0, 0, 0, 0);
-            } else {
-                for (int64_t q = used; q < lo + 16; ++q) buf[q] = 0;
-            }
-        }
-    }
+    lz_clear_slack((int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256, flag_off[blocks], data_off[blocks], blocks, flags, data);
 }
 
 struct LzDecodeShared {
@@ -641,19 +665,30 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_decompress_kernel(
         va[u] = src[lane];                             // 1 KB per instruction
         vb[u] = src[lane + WAVE];
     }
+    uint32_t rest = 0;
 #pragma unroll
     for (int u = 0; u < LZ_DEC_PER; ++u) {
         const int64_t block = first + u;
         if (block >= blocks) break;
-        const uint32_t mine = (uint32_t)lane < nflag[u] ? fb[u] : 0u;
-        if (direct[u] && __ballot(mine != 0) == 0) {
+        if (direct[u] && __ballot((uint32_t)lane < nflag[u] && fb[u] != 0) == 0) {
             pm_u32x4 *dst = reinterpret_cast<pm_u32x4 *>(out + block * LZ_SYMS);
             __builtin_nontemporal_store(va[u], dst + lane);
             __builtin_nontemporal_store(vb[u], dst + lane + WAVE);
         } else {
-            lz_decode_block(out, nsym, block, lane, mine, nflag[u], d0[u], nbytes[u], data, sh.bytes[wave], sh.out[wave]);
-            wave_sync();                               // the LDS of the wavefront serves the next block
+            rest |= 1u << u;
         }
+    }
+    // (one copy of the decoder's code: four, each walked once, were 24 KB of instructions to wait for)
+#pragma unroll 1
+    for (; rest != 0; rest &= rest - 1) {
+        const int u = __builtin_ctz(rest);
+        int64_t d = d0[0];
+        uint32_t nf = nflag[0], nb = nbytes[0], bits = fb[0];
+#pragma unroll
+        for (int w = 1; w < LZ_DEC_PER; ++w)
+            if (u == w) { d = d0[w]; nf = nflag[w]; nb = nbytes[w]; bits = fb[w]; }
+        lz_decode_block(out, nsym, first + u, lane, (uint32_t)lane < nf ? bits : 0u, nf, d, nb, data, sh.bytes[wave], sh.out[wave]);
+        wave_sync();                                   // the LDS of the wavefront serves the next block
     }
 }
 
@@ -713,13 +748,14 @@ extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *f
     const int chunks = (int)((entries + LZ_SCAN_CHUNK - 1) / LZ_SCAN_CHUNK);      // <= 128 below 2^31 bytes
     lz_sizes_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
                                                                 flag_offsets, data_offsets, cls);
-    lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals);
-    lz_scan_totals_kernel<<<1, LZ_MAX_CHUNKS, 0, st>>>(totals, chunks, bases);
-    lz_place_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
-                                                                flag_offsets, data_offsets, cls, bases, flags, data);
+    lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals, bases);
+    if (chunks > 1) lz_scan_totals_kernel<<<1, LZ_MAX_CHUNKS, 0, st>>>(totals, chunks, bases);
     const int64_t slack_chunks = (blocks * LZ_BLOCK_BYTES / 16 + 255) / 256;          // enough for all of data
-    lz_clear_slack_kernel<<<(unsigned)min(slack_chunks, (int64_t)4096), 256, 0, st>>>(flag_offsets, data_offsets,
-                                                                                   blocks, flags, data);
+    const int64_t clear_groups = chunks > 1 ? 0 : min((slack_chunks + 1) / 2, (int64_t)256);
+    lz_place_kernel<<<(unsigned)(groups + clear_groups), LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks, flag_offsets,
+                                                                                 data_offsets, cls, bases, flags, data);
+    if (chunks > 1)
+        lz_clear_slack_kernel<<<(unsigned)min(slack_chunks, (int64_t)4096), 256, 0, st>>>(flag_offsets, data_offsets, blocks, flags, data);
     PM_LAUNCH_CHECK("planmoe_lz_compress");
     return 0;
 }
