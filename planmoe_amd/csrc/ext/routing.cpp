@@ -32,10 +32,19 @@ int64_t spacing(const std::vector<Tensor> &t)
     return d / size;
 }
 
+bool flat(const std::vector<Tensor> &t, size_t k, int64_t n, at::ScalarType type, const Tensor &data)
+{
+    if (t.size() != k) return false;
+    for (const Tensor &v : t)
+        if (!v.is_cuda() || v.device() != data.device() || v.dim() != 1 || v.numel() != n || v.scalar_type() != type || !v.is_contiguous()) return false;
+    return true;
+}
+
 struct Planes {
     std::vector<Tensor> idx, loc, gates;         // (what keeps the memory)
-    const int32_t *i, *l;
-    const float *g;
+    const int32_t *i() const { return ints(idx[0]); }
+    const int32_t *l() const { return ints(loc[0]); }
+    const float *g() const { return gates.empty() ? nullptr : floats(gates[0]); }
     int64_t stride, samples;
     int k, experts, capacity;
 };
@@ -55,9 +64,6 @@ Planes planes_of(std::vector<Tensor> idx, std::vector<Tensor> loc, std::vector<T
         if (!gates.empty()) gates = {at::stack(gates)};
     }
     p.stride = a > 0 && a == b && a == c ? a : p.samples;
-    p.i = ints(idx[0]);
-    p.l = ints(loc[0]);
-    p.g = gates.empty() ? nullptr : floats(gates[0]);
     p.idx = std::move(idx);
     p.loc = std::move(loc);
     p.gates = std::move(gates);
@@ -68,7 +74,7 @@ Tensor scatter(const Tensor &x, const float *gates, const Planes &p)
 {
     const int64_t M = x.size(-1);
     Tensor out = at::empty({p.experts, p.capacity, M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(p.experts, p.capacity), x);
-    PM_CALL(planmoe_dispatch_fwd(x.data_ptr(), pm_dtype(x.scalar_type()), gates, p.i, p.l, p.stride, p.k, (int)p.samples, (int)M, p.experts, p.capacity,
+    PM_CALL(planmoe_dispatch_fwd(x.data_ptr(), pm_dtype(x.scalar_type()), gates, p.i(), p.l(), p.stride, p.k, (int)p.samples, (int)M, p.experts, p.capacity,
                                  out.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), current_stream()));
     return out;
 }
@@ -77,7 +83,7 @@ Tensor gather(const Tensor &slots, const float *gates, const Planes &p)
 {
     const int64_t M = slots.size(-1);
     Tensor out = at::empty({p.samples, M}, slots.options());
-    PM_CALL(planmoe_combine_fwd(slots.data_ptr(), pm_dtype(slots.scalar_type()), gates, p.i, p.l, p.stride, p.k, (int)p.samples, (int)M, p.capacity,
+    PM_CALL(planmoe_combine_fwd(slots.data_ptr(), pm_dtype(slots.scalar_type()), gates, p.i(), p.l(), p.stride, p.k, (int)p.samples, (int)M, p.capacity,
                                 out.data_ptr(), current_stream()));
     return out;
 }
@@ -93,7 +99,7 @@ std::vector<Tensor> planes_as_tensors(const Tensor &buffer, const Planes &p)
 std::vector<Tensor> gate_gradients(const Tensor &x, const Tensor &slots, const Planes &p)
 {
     Tensor out = at::empty({p.k * p.stride}, x.options().dtype(at::kFloat));
-    PM_CALL(planmoe_bwd_gate(x.data_ptr(), slots.data_ptr(), pm_dtype(x.scalar_type()), p.i, p.l, p.stride, p.k, (int)p.samples, (int)x.size(-1),
+    PM_CALL(planmoe_bwd_gate(x.data_ptr(), slots.data_ptr(), pm_dtype(x.scalar_type()), p.i(), p.l(), p.stride, p.k, (int)p.samples, (int)x.size(-1),
                              p.capacity, out.data_ptr<float>(), current_stream()));
     return planes_as_tensors(out, p);
 }
@@ -104,7 +110,7 @@ std::tuple<Tensor, std::vector<Tensor>> gather_backward(const Tensor &grad, cons
     const int64_t M = grad.size(-1);
     Tensor out = at::empty({p.experts, p.capacity, M}, grad.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(p.experts, p.capacity), grad);
     Tensor gg = at::empty({p.k * p.stride}, grad.options().dtype(at::kFloat));
-    PM_CALL(planmoe_combine_bwd(grad.data_ptr(), slots.data_ptr(), pm_dtype(grad.scalar_type()), p.g, p.i, p.l, p.stride, p.k, (int)p.samples, (int)M,
+    PM_CALL(planmoe_combine_bwd(grad.data_ptr(), slots.data_ptr(), pm_dtype(grad.scalar_type()), p.g(), p.i(), p.l(), p.stride, p.k, (int)p.samples, (int)M,
                                 p.experts, p.capacity, out.data_ptr(), gg.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), current_stream()));
     return {out, planes_as_tensors(gg, p)};
 }
@@ -112,23 +118,27 @@ std::tuple<Tensor, std::vector<Tensor>> gather_backward(const Tensor &grad, cons
 // encode (tokens to slots) and decode (slots to tokens); each is the other's backward pass
 template <bool ENCODE>
 struct Move : public torch::autograd::Function<Move<ENCODE>> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &data, at::TensorList gates, Planes *planes)
+    static Tensor forward(AutogradContext *ctx, const Tensor &data, at::TensorList gates, Planes *planes, Planes *given)
     {
         ctx->set_materialize_grads(false);
-        ctx->saved_data["planes"] = c10::IValue::make_capsule(c10::make_intrusive<Held>(*planes));
+        ctx->saved_data["planes"] = c10::IValue::make_capsule(c10::make_intrusive<Held>(*given));
         if (!gates.empty()) ctx->saved_data["data"] = data;         // (for the gates' gradient)
         ctx->saved_data["sizes"] = data.sizes().vec();
-        return ENCODE ? scatter(data, planes->g, *planes) : gather(data, planes->g, *planes);
+        return ENCODE ? scatter(data, planes->g(), *planes) : gather(data, planes->g(), *planes);
     }
 
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        const Planes &p = static_cast<Held *>(ctx->saved_data["planes"].toCapsule().get())->planes;
-        const int gates = (int)(p.g ? p.k : 0);
-        variable_list out(2 + gates);
+        const Planes &kept = static_cast<Held *>(ctx->saved_data["planes"].toCapsule().get())->planes;
+        const int gates = (int)kept.gates.size();
+        variable_list out(3 + gates);
         if (!grads[0].defined()) return out;
         const Tensor grad = grads[0].contiguous();
         const c10::DeviceGuard guard(grad.device());
+        // (looked at again: what the planes lie in may have been exchanged since the forward pass)
+        TORCH_CHECK(flat(kept.idx, kept.k, kept.samples, at::kInt, grad) && flat(kept.loc, kept.k, kept.samples, at::kInt, grad) &&
+                    (gates == 0 || flat(kept.gates, kept.k, kept.samples, at::kFloat, grad)), "the routing's tensors have changed their shape, type or device");
+        const Planes p = planes_of(kept.idx, kept.loc, kept.gates, kept.experts, kept.capacity);
         bool to_gates = false;
         for (int j = 0; j < gates; ++j) to_gates |= ctx->needs_input_grad(1 + j);
         const Tensor data = to_gates ? ctx->saved_data["data"].toTensor() : Tensor();
@@ -137,7 +147,7 @@ struct Move : public torch::autograd::Function<Move<ENCODE>> {
         if (!ENCODE && to_gates && ctx->needs_input_grad(0)) {
             std::tie(d, g) = gather_backward(grad, data, p);
         } else {
-            if (ctx->needs_input_grad(0)) d = ENCODE ? gather(grad, p.g, p) : scatter(grad, p.g, p);
+            if (ctx->needs_input_grad(0)) d = ENCODE ? gather(grad, p.g(), p) : scatter(grad, p.g(), p);
             if (to_gates) g = ENCODE ? gate_gradients(data, grad, p) : gate_gradients(grad, data, p);
         }
         if (d.defined()) out[0] = d.view(ctx->saved_data["sizes"].toIntVector());
@@ -150,14 +160,6 @@ struct Move : public torch::autograd::Function<Move<ENCODE>> {
         Planes planes;
     };
 };
-
-bool flat(const std::vector<Tensor> &t, size_t k, int64_t n, at::ScalarType type, const Tensor &data)
-{
-    if (t.size() != k) return false;
-    for (const Tensor &v : t)
-        if (!v.is_cuda() || v.device() != data.device() || v.dim() != 1 || v.numel() != n || v.scalar_type() != type || !v.is_contiguous()) return false;
-    return true;
-}
 
 // None where the arguments are not what the kernels take as they are (the caller converts them, or says what is wrong)
 template <bool ENCODE>
@@ -172,8 +174,11 @@ std::optional<Tensor> move(const Tensor &data_, const std::vector<Tensor> &gates
     if (!flat(idx, k, n, at::kInt, data_) || !flat(loc, k, n, at::kInt, data_) || !(gates.empty() || flat(gates, k, n, at::kFloat, data_))) return std::nullopt;
     const c10::DeviceGuard guard(data_.device());
     const Tensor data = data_.contiguous();
-    Planes p = planes_of(idx, loc, gates, (int)experts, (int)capacity);
-    return Move<ENCODE>::apply(data, at::TensorList(gates), &p);
+    Planes p = planes_of(idx, loc, gates, (int)experts, (int)capacity), given = p;
+    given.idx = idx;
+    given.loc = loc;
+    given.gates = gates;
+    return Move<ENCODE>::apply(data, at::TensorList(gates), &p, &given);
 }
 
 // ------------------------------------------------------------------ routing

@@ -69,3 +69,25 @@ def test_gradients_that_are_not_asked_for():
     gates[1].sum().backward()
     torch.cuda.synchronize()
     assert torch.equal(want, s2.grad)
+
+
+def test_the_backward_pass_reads_the_planes_where_they_are_then():
+    """A choice's indices exchanged for a copy elsewhere (as an optimizer or a memory saver does with .data) between the
+    forward and the backward pass: the planes are not where the forward pass found them, nor equally far apart."""
+    import planmoe_amd
+    g = torch.Generator().manual_seed(5)
+    scores = torch.softmax(torch.randn(70, 6, generator=g), 1).to(DEV)
+    x, grad = torch.randn(70, 40, generator=g).to(DEV), torch.randn(70, 40, generator=g).to(DEV)
+
+    def run(exchange):
+        xs = x.clone().requires_grad_(True)
+        crit, _ = planmoe_amd.extract_critical(scores, 2, capacity_factor=1.0, alignment=4)
+        y = planmoe_amd.fast_decode(planmoe_amd.fast_encode(xs, crit), crit)
+        if exchange:
+            crit[1][0].data = crit[1][0].data.clone()
+        y.backward(grad)
+        torch.cuda.synchronize()
+        return y.detach(), xs.grad
+
+    (y0, g0), (y1, g1) = run(False), run(True)
+    assert torch.equal(y0, y1) and torch.equal(g0, g1)
