@@ -290,9 +290,9 @@ std::tuple<Tensor, Tensor> ffn_layer(const Tensor &x, const Tensor &wg, const Te
 {
     check(x, wg, w1, b1, w2, b2, k, cap);
     const c10::DeviceGuard guard(x.device());
+    // (a forward-mode tangent goes to the node as well, which refuses it: it would be lost here without a word)
     bool grad = false;
-    if (at::GradMode::is_enabled())
-        for (const Tensor *t : {&x, &wg, &w1, &b1, &w2, &b2}) grad |= t->requires_grad();
+    for (const Tensor *t : {&x, &wg, &w1, &b1, &w2, &b2}) grad |= (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined();
     if (!grad) {
         const at::NoGradGuard no_grad;
         Pass p = forward_pass(x, wg, w1, b1, w2, b2, shape_of(x, wg, w1, k, cap), fp32_gate, normalize, (int)codec, false);

@@ -4,6 +4,7 @@ One GPU: the comm step is a copy on the device's comm stream between two events
 (compressor.comm_operation), so with a2a_ffn_overlap_degree > 1 a chunk's copy runs beside the
 next chunk's compress; the fused int8 / zfp paths below collapse the steps either side of it."""
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import compressor as _ck
 from . import ops
@@ -175,7 +176,7 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     for p in (gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias):
         if p.dtype != dtype or not p.is_contiguous():
             return None
-    if _hooked(experts) or _hooked(gate) or torch.is_autocast_enabled(x.device.type):
+    if _hooked(experts) or _hooked(gate) or _hooked(gate.wg) or _has_any_global_hook() or torch.is_autocast_enabled(x.device.type):
         return None
     codec = _NATIVE_CODECS.get(layer.compress_name, 0)
     if codec == 2 and not fused_zfp_eligible(x, 'zfp', degree, True, layer.num_global_experts, capacity):

@@ -84,3 +84,22 @@ def test_native_layer_leaves_hooks_and_frozen_parameters_to_autograd():
     layer(x).float().sum().backward()
     torch.cuda.synchronize()
     assert x.grad is not None and all(p.grad is None for p in layer.parameters())
+
+
+def test_native_layer_refuses_tangents_and_leaves_global_hooks_to_the_steps():
+    import planmoe_amd
+    torch.manual_seed(3)
+    layer = planmoe_amd.moe_layer({"type": "top", "k": 2, "fp32_gate": True}, 64,
+                                  experts={"type": "ffn", "count_per_node": 4, "hidden_size_per_expert": 64}).to(DEV).bfloat16()
+    x = torch.randn(40, 64, device=DEV).bfloat16()
+    import torch.autograd.forward_ad as fw
+    with fw.dual_level(), torch.no_grad(), pytest.raises((RuntimeError, NotImplementedError)):
+        layer(fw.make_dual(x, torch.ones_like(x)))
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(m))
+    try:
+        layer(x)
+    finally:
+        handle.remove()
+    torch.cuda.synchronize()
+    assert layer.experts in seen
