@@ -31,6 +31,7 @@ namespace {
 constexpr int LZ_SYMS = 512;             // symbols per block (gpulz.cu:6 / sizeof(float))
 constexpr int LZ_WINDOW = 32;            // gpulz.cu:12
 constexpr int LZ_BLOCK_BYTES = 2048;
+constexpr int LZ_PITCH = WAVE + 4;        // words between a position's masks and the next one's of a lane
 constexpr int LZ_WAVES = 8;              // blocks per work-group
 constexpr int LZ_SCAN_CHUNK = 8192;      // table entries scanned by one work-group
 constexpr int LZ_MAX_CHUNKS = 256;       // (2^31 / 2048 + 1) / 8192 rounded up to the scan's width
@@ -155,20 +156,20 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
         b.data_bytes = LZ_BLOCK_BYTES;
         return LZ_STORED;
     }
-    uint32_t any = 0, live = 0;                         // live: positions that some lane has a hit at
+    uint32_t live = 0;                                  // positions that some lane has a hit at
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        any |= (uint32_t)((hit[i] >> lane) & 1u) << i;
-        live |= hit[i] != 0 ? 1u << i : 0u;
-    }
+    for (int i = 0; i < 8; ++i) live |= hit[i] != 0 ? 1u << i : 0u;
 
     // ---- hit masks: bit j of position 8l+i's = symbol 8l+i equals window symbol 8l+i-32+j.
     // They hold all the matcher needs: while symbol p+r still equals window symbol w+r, bit
     // (w - p + 32) of the mask of position p+r is set.
     // (The positions are a loop, here and in the matcher: written out eight times the code was 15 KB walked once,
     // and a wave alone on its compute unit waited for instructions most of its time.)
+    static_assert(8 * LZ_PITCH <= LZ_WINDOW + LZ_SYMS, "the masks take the keys' place");
     uint32_t *hmask = keys;                             // the keys are all in registers by now
     wave_sync();
+    // position 8 q + i lies at i * LZ_PITCH + q: the lanes' reads at one distance are neighbours.  Zero behind the block.
+    if (lane < 32) hmask[(lane >> 2) * LZ_PITCH + WAVE + (lane & 3)] = 0;
 #pragma unroll 1
     for (int i = 0; i < 8; ++i) {
         uint32_t m = 0;
@@ -177,7 +178,7 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
 #pragma unroll
             for (int j = LZ_WINDOW - 1; j >= 0; --j) m = shift_in_equal(m, k, win[j]);
         }
-        hmask[8 * lane + i] = m;
+        hmask[i * LZ_PITCH + lane] = m;
 #pragma unroll
         for (int j = 0; j < 39; ++j) win[j] = win[j + 1];          // the next position's window and symbol
     }
@@ -185,38 +186,51 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
 
     // ---- the reference's matcher (gpulz.cu:46-85) on the masks: a run starts at the next hit,
     // grows while the following positions hit at the same distance, and the window symbol after
-    // a run is consumed by the comparison that ended it
+    // a run is consumed by the comparison that ended it.
+    // The lengths of the runs that start at any bit come first, all bits at once: bit j is alive after k steps
+    // if positions p .. p+k-1 hit at it, and when it dies k goes into the bit's place of six words.  (Run by run,
+    // with a read of the following masks for each, a block whose first 64 symbols are zero took 45 us.)
     uint64_t lens = 0, offs = 0;
     b.match_mask = 0;
 #pragma unroll 1
     for (uint32_t todo = live; todo != 0; todo &= todo - 1) {
         const int i = __builtin_ctz(todo);
-        uint32_t len = 0, off = 0;
-        if ((any >> i) & 1) {
-            const int p = 8 * lane + i;
-            const uint32_t room = (uint32_t)(LZ_SYMS - p);              // symbols left in the block
-            const uint32_t mask = hmask[p];
-            uint32_t j = 0;
-            while (j < (uint32_t)LZ_WINDOW) {
-                const uint32_t rest = mask & (0xffffffffu << j);
-                if (rest == 0) break;
-                const uint32_t j0 = __builtin_ctz(rest);
-                // the run ends with the window (32 - j0 symbols from its start) or the block
-                const uint32_t limit = min((uint32_t)LZ_WINDOW - j0, room);
-                uint32_t r = 1;
-                while (r < limit) {                     // 8 positions per step; words past the block are cut off by limit
-                    uint32_t ones = 0;
+        const uint32_t room = (uint32_t)(LZ_SYMS - 8 * lane - i);       // symbols left in the block
+        const uint32_t mask = hmask[i * LZ_PITCH + lane];
+        uint32_t alive = mask, runs[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 1
+        for (int k0 = 0; k0 < LZ_WINDOW; k0 += 8) {
+            if (__ballot(alive != 0) == 0) break;
+            uint32_t next[8];
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) ones |= ((hmask[p + r + t] >> j0) & 1u) << t;
-                    const uint32_t cnt = __builtin_ctz(~ones);
-                    r += cnt;
-                    if (cnt < 8) break;
-                }
-                r = min(r, limit);
-                if (r > len) { len = r; off = LZ_WINDOW - j0; }
-                if (r >= room) break;                   // the look-ahead reached the end of the block
-                j = j0 + r + 1;
+            for (int t = 0; t < 8; ++t) {
+                const int at = i + k0 + t + 1;
+                next[t] = hmask[(at & 7) * LZ_PITCH + lane + (at >> 3)];
             }
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const int k = k0 + t + 1;               // a run of k ends here, or (32 - j symbols from bit j on) with the window
+                const uint32_t on = alive & next[t] & (0x7fffffffu >> (k - 1)), dead = alive & ~on;
+#pragma unroll
+                for (int q = 0; q < 6; ++q) runs[q] |= dead & (0u - (((uint32_t)k >> q) & 1u));
+                alive = on;
+            }
+        }
+        uint32_t longest = 0, with = mask;              // of all runs, whether the walk gets to them or not
+#pragma unroll
+        for (int q = 5; q >= 0; --q)
+            if (with & runs[q]) { with &= runs[q]; longest |= 1u << q; }
+        uint32_t len = 0, off = 0, j = 0;
+        while (len < longest && j + len < (uint32_t)LZ_WINDOW) {         // (no longer run to come)
+            const uint32_t rest = mask & (0xffffffffu << j);
+            if (rest == 0) break;
+            const uint32_t j0 = __builtin_ctz(rest);
+            uint32_t r = 0;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) r |= ((runs[q] >> j0) & 1u) << q;
+            if (r > len) { len = r; off = LZ_WINDOW - j0; }
+            if (r >= room) break;                       // the look-ahead reached the end of the block
+            j = j0 + r + 1;
         }
         lens |= (uint64_t)len << (8 * i);
         offs |= (uint64_t)off << (8 * i);
