@@ -692,6 +692,29 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_decompress_kernel(
             rest |= 1u << u;
         }
     }
+    // Blocks of one repeated value (empty capacity slots): this coder's 44 bytes for it -- the value, (1,1) (2,2) (4,4) (8,8)
+    // (16,16) and (32,32) to the end -- are recognised as a whole and not walked match by match.  All four blocks' bytes are
+    // asked for together.  (134 MB with 30 % of its slots empty: decompress 70 us when they were walked, 50 now.)
+    uint32_t token[LZ_DEC_PER];
+#pragma unroll
+    for (int u = 0; u < LZ_DEC_PER; ++u) token[u] = 0;
+    if (rest != 0) {
+#pragma unroll
+        for (int u = 0; u < LZ_DEC_PER; ++u)
+            token[u] = *reinterpret_cast<const uint16_t *>(data + min(d0[u] + 2 * min(lane, 21), dcap - 2));
+        const uint32_t n = lane < 7 ? 1u << max(lane - 2, 0) : 32u, flag = lane == 0 ? 0xfeu : lane == 1 ? 0xffu : 0x1fu;
+#pragma unroll
+        for (int u = 0; u < LZ_DEC_PER; ++u) {
+            const int64_t block = first + u;
+            const bool odd = (lane >= 2 && lane < 22 && token[u] != (n | (n << 8))) || (lane < 3 && fb[u] != flag);
+            if (!((rest >> u) & 1u) || nflag[u] != 3 || nbytes[u] != 44 || block * LZ_SYMS + LZ_SYMS > nsym || __ballot(odd) != 0) continue;
+            const uint32_t v = __builtin_amdgcn_readlane(token[u], 0) | (__builtin_amdgcn_readlane(token[u], 1) << 16);
+            pm_u32x4 *dst = reinterpret_cast<pm_u32x4 *>(out + block * LZ_SYMS);
+            __builtin_nontemporal_store(pm_u32x4{v, v, v, v}, dst + lane);
+            __builtin_nontemporal_store(pm_u32x4{v, v, v, v}, dst + lane + WAVE);
+            rest &= ~(1u << u);
+        }
+    }
     // (one copy of the decoder's code: four, each walked once, were 24 KB of instructions to wait for)
 #pragma unroll 1
     for (; rest != 0; rest &= rest - 1) {
