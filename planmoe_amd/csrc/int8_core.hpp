@@ -152,6 +152,15 @@ struct RowEncoder {
         for (int i = 0; i < E::VEC / 4; ++i)
             w[i] = rq(0.f + f[4 * i]) | (rq(0.f + f[4 * i + 1]) << 8) | (rq(0.f + f[4 * i + 2]) << 16) | (rq(0.f + f[4 * i + 3]) << 24);
     }
+    // the codes of one vector, one by one
+    template <bool FAST>
+    __device__ __forceinline__ void codes(const uint4 &raw, uint32_t (&c)[E::VEC]) const
+    {
+        float f[E::VEC];
+        E::unpack(raw, f);
+#pragma unroll
+        for (int i = 0; i < E::VEC; ++i) c[i] = rq(0.f + f[i]);
+    }
     // the row scaled by its gate first, as the dispatcher stores it: round(0 + g * x)
     template <bool FAST>
     __device__ __forceinline__ void encode_gated(const uint4 &raw, float g, uint32_t *w) const
@@ -245,7 +254,18 @@ struct RowEncoder<PLANMOE_BF16> {
     template <bool FAST>
     __device__ __forceinline__ uint32_t pair_values(float f0, float f1) const
     {
-        if constexpr (!FAST) return quantise<PLANMOE_BF16>(0.f + f0, rq.bias, rq.scale) | (quantise<PLANMOE_BF16>(0.f + f1, rq.bias, rq.scale) << 8);
+        uint32_t c0, c1;
+        codes_of<FAST>(f0, f1, c0, c1);
+        return c0 | (c1 << 8);
+    }
+    template <bool FAST>
+    __device__ __forceinline__ void codes_of(float f0, float f1, uint32_t &c0, uint32_t &c1) const
+    {
+        if constexpr (!FAST) {
+            c0 = quantise<PLANMOE_BF16>(0.f + f0, rq.bias, rq.scale);
+            c1 = quantise<PLANMOE_BF16>(0.f + f1, rq.bias, rq.scale);
+            return;
+        }
         // (each difference rounded on its own, into the upper half of a word with zeros below: the
         // rounded value is a float right away, one conversion per value instead of one per pair
         // and an unpacking of both)
@@ -263,7 +283,16 @@ struct RowEncoder<PLANMOE_BF16> {
         // truncation does not see them)
         const float m0 = __uint_as_float(pk << 16), m1 = __uint_as_float(pk);
         // truncation; the conversion saturates NaN (0/0 rows) and negatives to 0, m <= 255
-        return __float2uint_rz(m0) | (__float2uint_rz(m1) << 8);
+        c0 = __float2uint_rz(m0);
+        c1 = __float2uint_rz(m1);
+    }
+    // the codes of one vector, one by one
+    template <bool FAST>
+    __device__ __forceinline__ void codes(const uint4 &raw, uint32_t (&c)[8]) const
+    {
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) codes_of<FAST>(__uint_as_float(w[i] << 16), __uint_as_float(w[i] & 0xffff0000u), c[2 * i], c[2 * i + 1]);
     }
     template <bool FAST>
     __device__ __forceinline__ void encode(const uint4 &raw, uint32_t *w) const

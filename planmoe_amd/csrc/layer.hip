@@ -41,11 +41,51 @@ __device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
     if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
 }
 
+// The same with the decoder as a table: a row has 256 codes, so a wave works out gate * decoded(code) for four codes a
+// lane, into LDS, and a value is a lookup by its code.  (Decoding value by value, the 35 vector instructions of a pair
+// of bf16 values took as long as its bytes.  Combine at 16384 x 4096, top-2, 113 -> 81 us,
+// at 16384 x 1024 35 -> 27, its backward pass there 64 -> 48.)
+template <int DT>
+struct RowTable {
+    RowEncoder<DT> enc;
+    const float *tab;                            // 256 values, the wave's own
+    template <int CACHE>
+    __device__ __forceinline__ RowTable(const uint4 (&row)[CACHE], float gate, float *table) : enc(0.f, 0.f), tab(table)
+    {
+        using E = Elem<DT>;
+        RowStats<DT, false> stats;
+        stats.init();
+#pragma unroll
+        for (int c = 0; c < CACHE; ++c) stats.add(row[c]);
+        float mn, mx, f[4];
+        stats.finish(mn, mx);
+        const float scale = E::round(mx - mn);
+        enc = RowEncoder<DT>(mn, scale);
+        RowDecoder<DT>(mn, scale).word(0x03020100u + 0x04040404u * (uint32_t)lane_id(), f);
+        *reinterpret_cast<float4 *>(table + 4 * lane_id()) = make_float4(gate * f[0], gate * f[1], gate * f[2], gate * f[3]);
+    }
+    template <bool FAST>
+    __device__ __forceinline__ void values(const uint4 &raw, float (&f)[Elem<DT>::VEC]) const
+    {
+        uint32_t c[Elem<DT>::VEC];
+        enc.template codes<FAST>(raw, c);
+#pragma unroll
+        for (int i = 0; i < Elem<DT>::VEC; ++i) f[i] = tab[c[i]];
+    }
+};
+// what a wave's lanes wrote to its LDS is there for all of them, and what they read has been read
+__device__ __forceinline__ void table_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // out[t] = sum_j gate_j * codec(rows[slot_j]), planes left to right, one rounding at the end.
 // One wave per token; the rows of two choices are requested before either is used and stay as they lie in
-// memory until both have been through the codec (two 8 KB rows and their sum in fp32 took 230 registers
-// and left two waves per SIMD: 112 us at 16384 x 4096 bf16, top-2, for 403 MB).  More than two choices
-// keep their sum in fp32.
+// memory until their values are looked up, vector by vector (two 8 KB rows and their sum in fp32 took 230
+// registers and left two waves per SIMD).  16384 x 4096 bf16, top-2, 403 MB: 81 us = 5.0 TB/s.  More than two
+// choices keep their sum in fp32.
 template <int DT, int CACHE, bool TWO>
 __global__ __launch_bounds__(256) void layer_combine_kernel(
     const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
@@ -54,9 +94,10 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
+    __shared__ __align__(16) float s_table[4][2][256];
     const int lane = lane_id(), units = model_dim / V;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= samples) return;
+    if (t >= samples) return;                    // (no work-group barrier below)
     const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
     uint4 *dst = reinterpret_cast<uint4 *>((char *)out + (int64_t)t * row_bytes);
     auto request = [&](int s, uint4 (&r)[CACHE]) {
@@ -72,26 +113,31 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
         const float g0 = rl_f(gate, 0), g1 = rl_f(gate, 1);
         request(s0, r0);
         if (s1 >= 0) request(s1, r1);
-        if (s0 >= 0) through_int8<DT, CACHE, false>(r0);
-        if (s1 >= 0) through_int8<DT, CACHE, false>(r1);
+        const RowTable<DT> t0(r0, g0, s_table[threadIdx.x >> 6][0]);
+        // (a choice without a slot has no row: row 0 stands for it above, what is looked up is not used)
+        const RowTable<DT> t1(s1 >= 0 ? r1 : r0, g1, s_table[threadIdx.x >> 6][1]);
+        table_sync();
+        auto body = [&](auto mode) {
 #pragma unroll
-        for (int c = 0; c < CACHE; ++c) {
-            float f[V], h[V];
-            E::unpack(r0[c], f);
+            for (int c = 0; c < CACHE; ++c) {
+                float f[V], h[V];
+                t0.template values<decltype(mode)::value>(r0[c], f);
 #pragma unroll
-            for (int i = 0; i < V; ++i) f[i] = s0 >= 0 ? g0 * f[i] : 0.f;
-            if (top_k > 1) {
-                if (s1 >= 0) {
-                    E::unpack(r1[c], h);
+                for (int i = 0; i < V; ++i) f[i] = s0 >= 0 ? f[i] : 0.f;
+                if (top_k > 1) {
+                    if (s1 >= 0) {
+                        t1.template values<decltype(mode)::value>(r1[c], h);
 #pragma unroll
-                    for (int i = 0; i < V; ++i) f[i] += g1 * h[i];
-                } else {
+                        for (int i = 0; i < V; ++i) f[i] += h[i];
+                    } else {
 #pragma unroll
-                    for (int i = 0; i < V; ++i) f[i] += 0.f;
+                        for (int i = 0; i < V; ++i) f[i] += 0.f;
+                    }
                 }
+                if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(f));
             }
-            if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(f));
-        }
+        };
+        if (t0.enc.fast() && t1.enc.fast()) body(std::true_type{}); else body(std::false_type{});
         return;
     }
     float acc[CACHE][V];
@@ -132,9 +178,10 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
+    __shared__ __align__(16) float s_table[4][256];
     const int lane = lane_id(), units = model_dim / V;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= samples) return;
+    if (t >= samples) return;                    // (no work-group barrier below)
     const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
     uint4 g_row[CACHE];
     {
@@ -163,16 +210,35 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
             for (int c = 0; c < CACHE; ++c) r[c] = next[c];
             if (j + 1 < np) request(j + 1);
             if (s < 0) continue;
-            if constexpr (INT8) through_int8<DT, CACHE, false>(r);
             float acc = 0.f;
-#pragma unroll
-            for (int c = 0; c < CACHE; ++c) {
-                float a[V], b[V];
+            auto dot = [&](int c, const float (&b)[V]) {
+                float a[V];
                 E::unpack(g_row[c], a);
-                E::unpack(r[c], b);
                 if (c * WAVE + lane < units) {
 #pragma unroll
                     for (int i = 0; i < V; ++i) acc = fmaf(b[i], a[i], acc);
+                }
+            };
+            if constexpr (INT8) {
+                float *table = s_table[threadIdx.x >> 6];
+                const RowTable<DT> tab(r, 1.f, table);
+                table_sync();
+                auto body = [&](auto mode) {
+#pragma unroll
+                    for (int c = 0; c < CACHE; ++c) {
+                        float b[V];
+                        tab.template values<decltype(mode)::value>(r[c], b);
+                        dot(c, b);
+                    }
+                };
+                if (tab.enc.fast()) body(std::true_type{}); else body(std::false_type{});
+                table_sync();
+            } else {
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) {
+                    float b[V];
+                    E::unpack(r[c], b);
+                    dot(c, b);
                 }
             }
             acc = wave_sum(acc);
@@ -186,10 +252,24 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
                 for (int i = 0; i < V; ++i) a[i] = E::round(0.f + g * a[i]);
                 r[c] = E::pack(a);
             }
-            if constexpr (INT8) through_int8<DT, CACHE, false>(r);
             uint4 *dst = reinterpret_cast<uint4 *>((char *)grad_rows + (int64_t)s * row_bytes);
+            if constexpr (INT8) {
+                const RowTable<DT> tab(r, 1.f, s_table[threadIdx.x >> 6]);
+                table_sync();
+                auto body = [&](auto mode) {
 #pragma unroll
-            for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, r[c]);
+                    for (int c = 0; c < CACHE; ++c) {
+                        float b[V];
+                        tab.template values<decltype(mode)::value>(r[c], b);
+                        if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, E::pack(b));
+                    }
+                };
+                if (tab.enc.fast()) body(std::true_type{}); else body(std::false_type{});
+                table_sync();                    // (the next choice's table takes this one's place)
+            } else {
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) stream_store(dst + c * WAVE + lane, r[c]);
+            }
         }
     }
 }

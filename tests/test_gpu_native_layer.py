@@ -103,3 +103,51 @@ def test_native_layer_refuses_tangents_and_leaves_global_hooks_to_the_steps():
         handle.remove()
     torch.cuda.synchronize()
     assert layer.experts in seen
+
+
+# the codec on rows in registers against compress, then combine from the codes: bit for bit.  Rows of one piece, of no whole
+# number of waves' pieces, of the longest kind; rows of one value, with NaN, infinities, negative zeros; choices without a slot
+@pytest.mark.parametrize("M", [8, 520, 4096])
+@pytest.mark.parametrize("k", [1, 2, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_layer_combine_equals_compress_and_combine(M, k, dtype):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", M, k, dtype, flush=True)
+    T, E, cap = 37, 4, 12
+    g = torch.Generator().manual_seed(M + k)
+    rows = torch.randn(E * cap, M, generator=g)
+    rows[3] = 0.25
+    rows[7, M // 2] = float("nan")
+    rows[9, 0] = float("inf")
+    rows[11, ::2] = -0.0
+    rows[13] *= 1e-30 if dtype != torch.float16 else 1e-6
+    rows = rows.to(dtype).to(DEV)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)], 1).int().contiguous().to(DEV)
+    loc = torch.randint(0, cap + 3, (k, T), generator=g, dtype=torch.int32).to(DEV)
+    gates, grad = torch.rand(k, T, generator=g).to(DEV), torch.randn(T, M, generator=g).to(dtype).to(DEV)
+    out = torch.empty(T, M, dtype=dtype, device=DEV)
+    check(lib.planmoe_layer_combine(ops._ptr(rows), ops._dt(rows, "t"), 1, ops._ptr(gates), ops._ptr(idx), ops._ptr(loc), T, k, T, M, E, cap,
+                                    ops._ptr(out), ops._stream(rows)))
+    codes, bias, scale = ops.int8_compress(rows)
+    want = ops.combine_int8(codes, bias, scale, list(idx), list(loc), list(gates), T, cap)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    same = (out.view(bits) == want.view(bits)) | (out.isnan() & want.isnan())
+    torch.cuda.synchronize()
+    assert bool(same.all())
+    # the backward pass: gate gradients, and rows by their slots (unique slots only: two tokens on one slot would race)
+    if k == 1:
+        loc, idx = (torch.arange(T) // E).int()[None].contiguous().to(DEV), (torch.arange(T) % E).int()[None].contiguous().to(DEV)
+        grad_rows, gg = torch.zeros_like(rows), torch.empty(k, T, device=DEV)
+        check(lib.planmoe_layer_combine_bwd(ops._ptr(grad), ops._ptr(rows), ops._dt(rows, "t"), 1, ops._ptr(gates), ops._ptr(idx), ops._ptr(loc), T, k, T, M,
+                                            E, cap, ops._ptr(grad_rows), ops._ptr(gg), ops._stream(rows)))
+        seen = ops.int8_decompress(codes, bias, scale)
+        slot = (idx[0] * cap + loc[0]).long()
+        gated = (gates[0][:, None] * grad.float()).to(dtype)
+        c2 = ops.int8_compress(gated)
+        wanted = ops.int8_decompress(*c2)
+        dots, mag = (seen[slot].double() * grad.double()).sum(1), (seen[slot].double() * grad.double()).abs().sum(1)
+        torch.cuda.synchronize()
+        assert torch.equal(grad_rows[slot].view(bits), wanted.view(bits))
+        fine = torch.isfinite(dots)
+        assert bool(((gg[0].double() - dots).abs() <= (M + 2) * 2.0 ** -24 * mag + 1e-30)[fine].all())
