@@ -14,7 +14,8 @@ using namespace planmoe_host;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// part of a buffer as a tensor of its own (no view in autograd's sense: an output of a node may be one)
+// part of a buffer as a tensor of its own: no view in autograd's sense (an output of a node may be one), its in-place
+// changes are counted apart from the buffer's
 Tensor piece(const Tensor &base, int64_t first, at::IntArrayRef sizes)
 {
     const at::AutoDispatchBelowADInplaceOrView guard;
@@ -185,7 +186,8 @@ std::optional<Tensor> move(const Tensor &data_, const std::vector<Tensor> &gates
 struct Routed {
     int T, E, k;
     bool normalize, want_loss;
-    std::vector<Tensor> indices, locations;
+    Tensor indices;                              // [k T]
+    std::vector<Tensor> locations;
 };
 
 struct Route : public torch::autograd::Function<Route> {
@@ -201,14 +203,15 @@ struct Route : public torch::autograd::Function<Route> {
                                    gates.data_ptr(), r->T, nullptr, loss.defined() ? loss.data_ptr<float>() : nullptr, i + 2 * plane, ws.data_ptr(),
                                    (size_t)ws.numel(), current_stream()));
         variable_list out;
+        r->indices = piece(ints_, 0, {plane});
         for (int j = 0; j < r->k; ++j) {
-            r->indices.push_back(piece(ints_, (int64_t)j * r->T, {r->T}));
             r->locations.push_back(piece(ints_, plane + (int64_t)j * r->T, {r->T}));
             out.push_back(piece(gates, (int64_t)j * r->T, {r->T}));
         }
         if (r->want_loss) out.push_back(loss);
-        ctx->save_for_backward({scores});
-        ctx->saved_data["ints"] = ints_;
+        // (as variables: the gradient is that of these indices, and an index plane edited in place until then is refused.
+        // The locations are not read again and are edited at will)
+        ctx->save_for_backward({scores, r->indices, piece(ints_, 2 * plane, {(int64_t)r->k * r->E})});
         ctx->saved_data["k"] = (int64_t)r->k;
         ctx->saved_data["normalize"] = r->normalize;
         return out;
@@ -216,7 +219,8 @@ struct Route : public torch::autograd::Function<Route> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        const Tensor scores = ctx->get_saved_variables()[0], ints_ = ctx->saved_data["ints"].toTensor();
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &scores = saved[0], &indices = saved[1], &counts = saved[2];
         const c10::DeviceGuard guard(scores.device());
         const int k = (int)ctx->saved_data["k"].toInt(), T = (int)scores.size(0), E = (int)scores.size(1);
         std::vector<Tensor> gg(grads.begin(), grads.begin() + k);
@@ -230,9 +234,8 @@ struct Route : public torch::autograd::Function<Route> {
         if (!any) return {Tensor(), Tensor()};
         if (spacing(gg) != T && k > 1) gg = {at::stack(gg)};        // (the indices' planes are T apart)
         Tensor out = at::empty_like(scores);
-        const int32_t *i = ints(ints_);
-        PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), i, gg[0].data_ptr(), stride, T, E, k,
-                                  ctx->saved_data["normalize"].toBool(), dl.defined() ? floats(dl) : nullptr, dl.defined() ? i + 2 * (int64_t)k * T : nullptr,
+        PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), ints(indices), gg[0].data_ptr(), stride, T, E, k,
+                                  ctx->saved_data["normalize"].toBool(), dl.defined() ? floats(dl) : nullptr, dl.defined() ? ints(counts) : nullptr,
                                   0, out.data_ptr(), current_stream()));
         return {out, Tensor()};
     }
@@ -262,7 +265,10 @@ std::optional<Critical> extract_critical(const Tensor &scores_, int64_t top_k, b
     }
     int capacity = 0;
     PM_CALL(planmoe_capacity(r.T, r.E, r.k, capacity_factor, (int)alignment, &capacity));
-    return Critical(std::move(r.indices), std::move(r.locations), std::move(out), capacity, loss);
+    // (views of what the node has saved: their in-place changes are its)
+    std::vector<Tensor> indices;
+    for (int j = 0; j < r.k; ++j) indices.push_back(r.indices.narrow(0, (int64_t)j * r.T, r.T));
+    return Critical(std::move(indices), std::move(r.locations), std::move(out), capacity, loss);
 }
 
 } // namespace

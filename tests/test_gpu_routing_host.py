@@ -91,3 +91,26 @@ def test_the_backward_pass_reads_the_planes_where_they_are_then():
 
     (y0, g0), (y1, g1) = run(False), run(True)
     assert torch.equal(y0, y1) and torch.equal(g0, g1)
+
+
+@pytest.mark.parametrize("k", [1, 2])
+def test_index_planes_edited_in_place_are_refused(k):
+    """The gradient reads the indices again, so a plane edited between the forward and the backward pass would change it
+    without a word: autograd refuses it (the edits here stay in range).  The slots are not read: they may be edited."""
+    import planmoe_amd
+    g = torch.Generator().manual_seed(11)
+    scores = torch.softmax(torch.randn(50, 6, generator=g), 1).to(DEV)
+
+    def run(plane):
+        s = scores.clone().requires_grad_(True)
+        crit, loss = planmoe_amd.extract_critical(s, k, alignment=4)
+        if plane is not None:
+            crit[plane][-1].zero_()
+        (crit[3][0].sum() + loss).backward()
+        torch.cuda.synchronize()
+        return s.grad
+
+    want = run(None)
+    assert torch.equal(run(2), want)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        run(1)
