@@ -111,6 +111,7 @@ int planmoe_route_locations(const int32_t *indices, int64_t plane_stride, int sa
  * divided by their clamped sum) and of gshard_loss (losses.py:12-19: me depends on the scores,
  * ce does not).
  *   scores        [samples, experts] `dtype`, the scores routing ran on (scores_out)
+ *   indices       a choice outside [0, experts) counts as not there: it has no share in the gates' sum
  *   grad_gates    `dtype` k planes: gradient arriving at the gates
  *   grad_l_aux    optional fp32 scalar: gradient arriving at l_aux (needs first_choice_counts =
  *                 row 0 of expert_counts)

@@ -327,8 +327,10 @@ __global__ __launch_bounds__(256) void route_bwd_kernel(
     const float lscale = dl * ((float)experts / (float)samples) / (float)samples;
     float sum = 0.f, dot = 0.f;
     for (int j = 0; j < k; ++j) {
-        const float sj = E::load(scores, base + indices[(int64_t)j * stride + t]);
-        sum = (j == 0) ? sj : E::round(sum + sj);
+        const int e = indices[(int64_t)j * stride + t];
+        if (e < 0 || e >= experts) continue;             // (no expert: the choice is not there)
+        const float sj = E::load(scores, base + e);
+        sum = E::round(sum + sj);
         dot += E::load(dgates, (int64_t)j * stride + t) * sj;
     }
     const float eps = DT == PLANMOE_F32 ? 1.1920928955078125e-07f : DT == PLANMOE_BF16 ? 0.0078125f : 0.0009765625f;

@@ -194,6 +194,28 @@ def test_routing_gradients_match_autograd(T, E, k, normalize):
     assert torch.allclose(s_dev.grad.cpu().double(), s64.grad, rtol=1e-5, atol=1e-7)
 
 
+def test_routing_gradients_of_choices_without_an_expert():
+    """Indices outside the experts (a caller's mark for padding tokens) read no score and have no share in the sum."""
+    from planmoe_amd import ops
+    T, E, k = 70, 6, 3
+    g = torch.Generator().manual_seed(2)
+    scores, dg = torch.softmax(torch.randn(T, E, generator=g), 1), torch.randn(k, T, generator=g)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)], 1).int()
+    idx[0, :20] = -1
+    idx[1, 10:30] = E
+    idx[2, :12] = -(1 << 30)
+    s = scores.double().requires_grad_(True)
+    there = (idx >= 0) & (idx < E)
+    picked = s.gather(1, idx.t().long().clamp(0, E - 1)).t() * there
+    (picked / picked.sum(0).clamp(min=torch.finfo(torch.float32).eps) * dg.double() * there).sum().backward()
+    got = ops.route_bwd(scores.to(DEV), idx.contiguous().to(DEV), dg.to(DEV))
+    torch.cuda.synchronize()
+    # (dg_j - sum_i dg_i g_i) / D: a few fp32 roundings of terms of at most max |dg| / D
+    tol = 16 * 2.0 ** -24 * float(dg.abs().max()) / picked.detach().sum(0).clamp(min=1e-6)[:, None]
+    assert bool(((got.double().cpu() - s.grad).abs() <= tol).all())
+    assert bool((got[10:12].cpu() == 0).all())        # (tokens 10, 11 have no choice left)
+
+
 def test_routing_gradients_through_the_fused_softmax():
     from planmoe_amd.fast_dispatch import route
     T, E, k = 400, 8, 2
