@@ -281,4 +281,17 @@ class MOELayer(torch.nn.Module):
                                     normalize_gate=self.normalize_gate, group=self.group, alignment=alignment)
 
 
+# the way from the layer into its built-in experts and through them, as defined here
+_EXPERT_LOCAL = MOELayer.expert_local
+_EXPERTS_FORWARD, _EXPERTS_LINEAR = _experts.FusedExpertsNetwork.forward, _experts.FusedExpertsNetwork._linear
+
+
+def runs_built_in_experts(layer):
+    """Whether a layer over a FusedExpertsNetwork has that way: no part of it replaced on the objects, in a subclass or
+    in the classes."""
+    return all(getattr(type(owner), name) is method and name not in owner.__dict__ for owner, name, method in (
+        (layer, 'expert_local', _EXPERT_LOCAL), (layer.experts, 'forward', _EXPERTS_FORWARD),
+        (layer.experts, '_linear', _EXPERTS_LINEAR)))
+
+
 moe_layer = MOELayer

@@ -157,16 +157,18 @@ def _hooked(module):
 
 def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     """The codec number for csrc/ext/layer.cpp when the whole layer is its business, else None.  What is left to
-    the steps below: experts or gates that are not the built-in ones or carry hooks, other dtypes (a gate in
+    the steps below: experts or gates that are not the built-in ones, have a method replaced (on the object,
+    as adapters and offloading wrappers do, in a subclass or in the class) or carry hooks, other dtypes (a gate in
     fp32 next to 16-bit rows among them), overlap slices, autocast, and every option that asks for the
     reference's structure."""
     from .experts import FusedExpertsNetwork
     from .gates import LinearTopKGate
+    from .moe_layer import runs_built_in_experts
     experts = layer.experts
     if not (NATIVE_LAYER and FUSE_GATE and FUSE_INT8 and FUSE_ZFP and not FFN_FROM_CODES and not _ck.SINGLE_RANK_COMM_COPIES and
             degree == 1 and reserve_dims == 1 and layer.is_postscore and x.is_cuda and capacity >= 1 and x.shape[0] >= 1 and
             type(experts) is FusedExpertsNetwork and experts._relu and type(gate) is LinearTopKGate and
-            layer.num_global_experts <= 64):
+            layer.num_global_experts <= 64 and runs_built_in_experts(layer)):
         return None
     dtype, M, H = x.dtype, x.shape[1], experts.hidden_size_per_expert
     vec = 8 if dtype == torch.bfloat16 else 4

@@ -151,3 +151,50 @@ def test_layer_combine_equals_compress_and_combine(M, k, dtype):
         assert torch.equal(grad_rows[slot].view(bits), wanted.view(bits))
         fine = torch.isfinite(dots)
         assert bool(((gg[0].double() - dots).abs() <= (M + 2) * 2.0 ** -24 * mag + 1e-30)[fine].all())
+
+
+def _layer(dtype, codec="no", M=64, H=72, E=4, k=2, cf=1.25, cls=None):
+    import planmoe_amd
+    torch.manual_seed(3)
+    return (cls or planmoe_amd.moe_layer)({"type": "top", "k": k, "capacity_factor": cf, "fp32_gate": True}, M,
+                                          experts={"type": "ffn", "count_per_node": E, "hidden_size_per_expert": H},
+                                          compress_name=codec).to(DEV).to(dtype)
+
+
+def test_replaced_methods_are_called(monkeypatch):
+    """The forward of the experts replaced on the object or in the class, expert_local overridden or replaced: the layer goes
+    through them."""
+    from planmoe_amd.experts import FusedExpertsNetwork
+    from planmoe_amd.moe_layer import MOELayer
+    x = torch.randn(40, 64, device=DEV).bfloat16()
+    seen = []
+
+    def twice(inner):
+        def call(*args):
+            seen.append(1)
+            return inner(*args) * 2
+        return call
+
+    with torch.no_grad():
+        plain = _layer(torch.bfloat16)(x)
+        layer = _layer(torch.bfloat16)
+        layer.experts.forward = twice(layer.experts.forward)
+        got = [layer(x)]
+        layer = _layer(torch.bfloat16)
+        layer.expert_local = twice(layer.expert_local)
+        got.append(layer(x))
+
+        class Mine(MOELayer):
+            def expert_local(self, *args):
+                return twice(super().expert_local)(*args)
+
+        got.append(_layer(torch.bfloat16, cls=Mine)(x))
+        layer = _layer(torch.bfloat16)
+        for cls, name in ((FusedExpertsNetwork, "forward"), (MOELayer, "expert_local")):
+            with monkeypatch.context() as m:
+                m.setattr(cls, name, twice(getattr(cls, name)))
+                got.append(layer(x))
+    torch.cuda.synchronize()
+    assert len(seen) == 5
+    for y in got:                                # (the products of the steps sum in another order: bf16 roundings)
+        assert float((y.double() - 2 * plain.double()).norm()) <= 1e-2 * float(2 * plain.double().norm())
