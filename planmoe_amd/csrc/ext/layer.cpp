@@ -79,6 +79,14 @@ Live live_rows(const Pass &p, const Shape &s, int codec)
     return Live{ints(p.counts), s.k, codec == CODEC_ZFP ? 4 : 1};
 }
 
+// a gradient as the kernels read rows: contiguous and 16-byte aligned (what comes back through torch.cat is contiguous,
+// but begins anywhere)
+Tensor as_rows(const Tensor &grad)
+{
+    const Tensor t = grad.contiguous();
+    return (uintptr_t)t.data_ptr() % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
 
 Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, const Shape &s,
@@ -197,7 +205,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                    need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
         Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates;
         if (grads[0].defined()) {
-            const Tensor grad = grads[0].contiguous();
+            const Tensor grad = as_rows(grads[0]);
             const Tensor gates = float_gates(p.gates);
             const Live live = live_rows(p, s, codec);
             grad_gates = at::empty({s.k, s.T}, x.options().dtype(at::kFloat));

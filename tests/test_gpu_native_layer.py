@@ -198,3 +198,25 @@ def test_replaced_methods_are_called(monkeypatch):
     assert len(seen) == 5
     for y in got:                                # (the products of the steps sum in another order: bf16 roundings)
         assert float((y.double() - 2 * plain.double()).norm()) <= 1e-2 * float(2 * plain.double().norm())
+
+
+def _pass(layer, x, gy):
+    layer.zero_grad()
+    x = x.clone().requires_grad_(True)
+    y = layer(x)
+    y.backward(gy)
+    torch.cuda.synchronize()
+    return {"y": y.detach(), "dx": x.grad, **{n: p.grad for n, p in layer.named_parameters()}}
+
+
+@pytest.mark.parametrize("codec,dtype", [("no", torch.bfloat16), ("no", torch.float32), ("int8", torch.bfloat16), ("int8", torch.float32),
+                                         ("zfp", torch.float32), ("lz", torch.float32)])
+def test_gradient_that_is_not_aligned(codec, dtype):
+    """What torch.cat sends back to a part of its result is contiguous and begins anywhere."""
+    layer = _layer(dtype, codec)
+    x, gy = torch.randn(40, 64, device=DEV).to(dtype), torch.randn(40, 64, device=DEV).to(dtype)
+    off = torch.cat([gy.new_zeros(1), gy.flatten()])[1:].view_as(gy)
+    assert off.is_contiguous() and off.data_ptr() % 16 != 0
+    want, got = _pass(layer, x, gy), _pass(layer, x, off)
+    for name in want:
+        assert torch.equal(want[name], got[name]), name
