@@ -14,6 +14,13 @@ def _kernel_serves(x, w):
             not torch.is_autocast_enabled(x.device.type))
 
 
+def aligned(t):
+    """t as the kernels read it: contiguous, 16-byte aligned.  (A view of a flat buffer of parameters or rows begins
+    anywhere; it is copied for the product.)"""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _BatchedLinear(torch.autograd.Function):
     """y = act(x @ w + bias) over experts: x [E, R, in], w [E, in, out] (as the reference stores it),
     bias [E, out], act = relu or nothing; torch.add(torch.matmul(x, w), bias.unsqueeze(1)) of
@@ -24,7 +31,7 @@ class _BatchedLinear(torch.autograd.Function):
     def forward(ctx, x, w, bias, relu):
         from . import ops
         x, w = x.contiguous(), w.contiguous()
-        y = ops.expert_gemm('nn', x, w, bias, relu=relu)
+        y = ops.expert_gemm('nn', aligned(x), aligned(w), None if bias is None else bias.contiguous(), relu=relu)
         ctx.save_for_backward(x, w, y if relu else None)
         ctx.relu, ctx.has_bias = relu, bias is not None
         return y
@@ -33,14 +40,14 @@ class _BatchedLinear(torch.autograd.Function):
     def backward(ctx, gy):
         from . import ops
         x, w, y = ctx.saved_tensors
-        gy = gy.contiguous()
         if ctx.relu:
-            gy = torch.ops.aten.threshold_backward(gy, y, 0.0)      # relu's own backward: one pass over dy and y
+            gy = torch.ops.aten.threshold_backward(gy.contiguous(), y, 0.0)      # relu's own backward: one pass over dy and y
+        gy = aligned(gy)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = ops.expert_gemm('nt', gy, w)                       # [E, R, out] x [E, in, out]^T
+            dx = ops.expert_gemm('nt', gy, aligned(w))              # [E, R, out] x [E, in, out]^T
         if ctx.needs_input_grad[1]:
-            dw = ops.expert_gemm('tn', x, gy)                       # x^T dy
+            dw = ops.expert_gemm('tn', aligned(x), gy)              # x^T dy
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = gy.sum(dim=1, dtype=torch.float32).to(gy.dtype)
         return dx, dw, db, None

@@ -160,7 +160,7 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     the steps below: experts or gates that are not the built-in ones, have a method replaced (on the object,
     as adapters and offloading wrappers do, in a subclass or in the class) or carry hooks, other dtypes (a gate in
     fp32 next to 16-bit rows among them), overlap slices, autocast, and every option that asks for the
-    reference's structure."""
+    reference's structure; weights that are not 16-byte aligned."""
     from .experts import FusedExpertsNetwork
     from .gates import LinearTopKGate
     from .moe_layer import runs_built_in_experts
@@ -178,6 +178,9 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     for p in (gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias):
         if p.dtype != dtype or not p.is_contiguous():
             return None
+    # (weights that are views of a flat buffer: the steps copy them for their products)
+    if (experts.batched_fc1_w.data_ptr() | experts.batched_fc2_w.data_ptr()) % 16:
+        return None
     if _hooked(experts) or _hooked(gate) or _hooked(gate.wg) or _has_any_global_hook() or torch.is_autocast_enabled(x.device.type):
         return None
     codec = _NATIVE_CODECS.get(layer.compress_name, 0)

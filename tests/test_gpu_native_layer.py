@@ -220,3 +220,37 @@ def test_gradient_that_is_not_aligned(codec, dtype):
     want, got = _pass(layer, x, gy), _pass(layer, x, off)
     for name in want:
         assert torch.equal(want[name], got[name]), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weights_that_are_not_aligned(dtype):
+    """Parameters that are views of a flat buffer, biases that are columns of one."""
+    layer = _layer(dtype)
+    x, gy = torch.randn(40, 64, device=DEV).to(dtype), torch.randn(40, 64, device=DEV).to(dtype)
+    want = _pass(layer, x, gy)
+    experts = layer.experts
+    flat = torch.cat([torch.zeros(1, dtype=dtype, device=DEV)] + [p.detach().flatten() for p in experts.parameters()])
+    at = 1
+    for name, p in list(experts.named_parameters()):
+        view = flat[at:at + p.numel()].view(p.shape)
+        assert view.data_ptr() % 16 != 0
+        setattr(experts, name, torch.nn.Parameter(view))
+        at += p.numel()
+    # (the products now run over whole buffers: bf16 roundings, and sums of up to 72 terms in another order)
+    _compare(_pass(layer, x, gy), want, 1e-2 if dtype == torch.bfloat16 else 2e-5)
+    # the experts alone, with rows and a gradient that are not aligned either, a bias with gaps between its values
+    whole = experts(rows.clone(), layer).detach()
+    experts.batched_fc1_bias = torch.nn.Parameter(experts.batched_fc1_bias.detach()[..., None].repeat(1, 1, 3)[..., 1])
+    rows = torch.randn(1 + 4 * 20 * 64, device=DEV).to(dtype)[1:].view(4, 20, 64)
+    got = []
+    for off in (True, False):
+        r = (rows if off else rows.clone()).detach().requires_grad_(True)
+        g = rows if off else rows.clone()
+        layer.zero_grad()
+        y = experts(r, layer)
+        y.backward(g)
+        got.append([y.detach(), r.grad] + [p.grad for p in experts.parameters()])
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], whole)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
