@@ -239,9 +239,9 @@ def test_weights_that_are_not_aligned(dtype):
     # (the products now run over whole buffers: bf16 roundings, and sums of up to 72 terms in another order)
     _compare(_pass(layer, x, gy), want, 1e-2 if dtype == torch.bfloat16 else 2e-5)
     # the experts alone, with rows and a gradient that are not aligned either, a bias with gaps between its values
+    rows = torch.randn(1 + 4 * 20 * 64, device=DEV).to(dtype)[1:].view(4, 20, 64)
     whole = experts(rows.clone(), layer).detach()
     experts.batched_fc1_bias = torch.nn.Parameter(experts.batched_fc1_bias.detach()[..., None].repeat(1, 1, 3)[..., 1])
-    rows = torch.randn(1 + 4 * 20 * 64, device=DEV).to(dtype)[1:].view(4, 20, 64)
     got = []
     for off in (True, False):
         r = (rows if off else rows.clone()).detach().requires_grad_(True)
