@@ -755,8 +755,10 @@ static int expert_gemm_check(const char *who, int form, int dtype, const void *a
     // (what is read and stored in 16-byte pieces: the fast index of every operand and of the result)
     PM_REQUIRE(n % vec == 0 && (form == 2 ? m : k) % vec == 0, "%s: the fast index of every operand must be a multiple of %d", who, vec);
     PM_REQUIRE(!live || (batches <= 64 && live_planes >= 1 && live_round >= 1), "%s: row counts for up to 64 batches", who);
-    const int widest = n > k ? (n > m ? n : m) : (k > m ? k : m);
-    PM_REQUIRE((int64_t)widest * 2 * 256 * (dtype == PLANMOE_F32 ? 2 : 1) < ((int64_t)1 << 31), "%s: 256 rows of an operand must stay under 2 GiB", who);
+    // row lengths: a's, and the longer of b's and c's (n, or with b^T: k and n).  How many rows there are is no row length: the
+    // kernels' offsets start at a tile's corner
+    const int pitch_a = form == 2 ? m : k, pitch = n > pitch_a ? n : pitch_a;
+    PM_REQUIRE((int64_t)pitch * 2 * 256 * (dtype == PLANMOE_F32 ? 2 : 1) < ((int64_t)1 << 31), "%s: 256 rows of an operand must stay under 2 GiB", who);
     return 0;
 }
 

@@ -348,8 +348,6 @@ int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
 
 int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who)
 {
-    PM_REQUIRE((int64_t)p.K * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.M * 4 * 128 < ((int64_t)1 << 31) && (int64_t)p.N * 4 * 128 < ((int64_t)1 << 31),
-               "%s: 128 rows of an operand must stay under 2 GiB", who);
     if (side == 0) {
         if (p.M <= 16 && !p.colsum) return form == 0 ? gemm_f32_wave_launch<1, 16, true>(p, stream, who) : gemm_f32_wave_launch<1, 8, false>(p, stream, who);
         return form == 0 ? gemm_f32_wave_launch<2, 8, true>(p, stream, who) : gemm_f32_wave_launch<2, 4, false>(p, stream, who);

@@ -6,12 +6,18 @@ buffer straight into the first GEMM."""
 import torch
 
 
+def row_fits(length, dtype):
+    """256 rows of an operand of planmoe_expert_gemm stay under 2 GiB.  (Longer fp32 rows are the library's; bf16 rows
+    are refused: the library's batched bf16 products are kept away from transposed operands.)"""
+    return dtype != torch.float32 or length * 4 * 256 < 1 << 31
+
+
 def _kernel_serves(x, w):
     """planmoe_expert_gemm takes bf16 / fp32 operands on the GPU whose row lengths are whole 16-byte pieces."""
     vec = 8 if x.dtype == torch.bfloat16 else 4
     return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and x.dim() == 3 and x.numel() > 0 and
             w.shape[1] % vec == 0 and w.shape[2] % vec == 0 and x.shape[0] == w.shape[0] and x.shape[2] == w.shape[1] and
-            not torch.is_autocast_enabled(x.device.type))
+            row_fits(max(w.shape[1:]), x.dtype) and not torch.is_autocast_enabled(x.device.type))
 
 
 def aligned(t):

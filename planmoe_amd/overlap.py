@@ -161,7 +161,7 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     as adapters and offloading wrappers do, in a subclass or in the class) or carry hooks, other dtypes (a gate in
     fp32 next to 16-bit rows among them), overlap slices, autocast, and every option that asks for the
     reference's structure; weights that are not 16-byte aligned."""
-    from .experts import FusedExpertsNetwork
+    from .experts import FusedExpertsNetwork, row_fits
     from .gates import LinearTopKGate
     from .moe_layer import runs_built_in_experts
     experts = layer.experts
@@ -173,7 +173,7 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     dtype, M, H = x.dtype, x.shape[1], experts.hidden_size_per_expert
     vec = 8 if dtype == torch.bfloat16 else 4
     if not ((dtype == torch.bfloat16 or dtype == torch.float32) and M % vec == 0 and H % vec == 0 and M <= 1024 * vec and
-            experts.output_dim in (None, M)):
+            row_fits(H, dtype) and experts.output_dim in (None, M)):
         return None
     for p in (gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias):
         if p.dtype != dtype or not p.is_contiguous():

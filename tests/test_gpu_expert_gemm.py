@@ -242,3 +242,33 @@ def test_expert_gemm_fp32_does_not_depend_on_the_number_of_rows(m, n, k):
         assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all())
         stored = masked[e, :r].double()
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all())
+
+
+# more rows than 256 (or 128) of them would fit in 2 GiB if they were as long: rows are no row length.  nn and nt rows,
+# a tn product's reduction, the masked product
+@pytest.mark.parametrize("dtype,rows", [(torch.float32, 2097160), (torch.float32, 4194312), (torch.bfloat16, 4194312)])
+def test_expert_gemm_takes_millions_of_rows(dtype, rows):
+    from planmoe_amd import ops
+    print("case", dtype, rows, flush=True)
+    n = k = 8
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    a, dy = torch.randn(1, rows, k, device=DEV, generator=g).to(dtype), torch.randn(1, rows, n, device=DEV, generator=g).to(dtype)
+    w, h = torch.randn(1, k, n, device=DEV, generator=g).to(dtype), torch.randn(1, rows, n, device=DEV, generator=g).clamp(min=0).to(dtype)
+    ref, mag = a[0].double() @ w[0].double(), a[0].double().abs() @ w[0].double().abs()
+    tol, wt = _bound(ref, mag, k, dtype), w.transpose(1, 2).contiguous()
+    assert bool(((ops.expert_gemm("nn", a, w)[0].double() - ref).abs() <= tol).all())
+    assert bool(((ops.expert_gemm("nt", a, wt)[0].double() - ref).abs() <= tol).all())
+    masked, db = ops.expert_gemm_relu_bwd(a, wt, h)
+    assert bool(((masked[0].double() - ref * (h[0] > 0)).abs() <= tol).all())
+    stored = masked[0].double()
+    assert bool(((db[0].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), rows, dtype)).all())
+    got = ops.expert_gemm("tn", a, dy)[0].double()
+    ref, mag = a[0].double().t() @ dy[0].double(), a[0].double().abs().t() @ dy[0].double().abs()
+    assert bool(((got - ref).abs() <= _bound(ref, mag, rows, dtype)).all())
+    # a few rows in use of many
+    live = torch.tensor([[3]], dtype=torch.int32, device=DEV)
+    out = torch.full((1, rows, n), 7.0, dtype=dtype, device=DEV)
+    ops.expert_gemm("nn", a, w, live=live, rows_hint=3, out=out)
+    ref = a[0, :3].double() @ w[0].double()
+    torch.cuda.synchronize()
+    assert bool(((out[0, :3].double() - ref).abs() <= tol[:3]).all()) and bool((out[0, 3:] == 7.0).all())

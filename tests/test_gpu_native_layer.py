@@ -254,3 +254,10 @@ def test_weights_that_are_not_aligned(dtype):
     assert torch.equal(got[0][0], whole)
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_fp32_layer_with_two_million_slots_an_expert():
+    """The number of slots is no row length: it has no bound but the slots' numbers (int32)."""
+    T, cf = 8, 524290.0                          # capacity 4 cf: 2097160, 2 GiB over 256 rows of 4-byte values and 8
+    args = ("no", torch.float32, T, 8, 8, 2, 1, cf, True)
+    _compare(_run(True, *args), _run(False, *args), 2e-5)
