@@ -478,12 +478,27 @@ int planmoe_layer_combine(const void *rows, int dtype, int codec, const float *g
                           const int32_t *locations, int64_t plane_stride, int top_k, int samples,
                           int model_dim, int experts, int capacity, void *out, void *stream);
 
+/* The same with codec = 1, and the codes [experts * capacity, model_dim], minima and scales [experts * capacity] (`dtype`) of the
+ * rows that hold a token kept as Int8Compressor::compress leaves them (int8.cpp:10-24): a byte a value for the backward
+ * pass to read in place of the rows.  codes 16-byte aligned. */
+int planmoe_layer_combine_keep(const void *rows, int dtype, const float *gates, const int32_t *indices,
+                               const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                               int model_dim, int experts, int capacity, void *out, uint8_t *codes,
+                               void *bias, void *scale, void *stream);
+
 /* Its backward pass (GatingDecoder.backward, fast_dispatch.py:62-79): grad_gates[j][t] = <grad[t],
  * codec(rows[slot])> and grad_rows[slot] = codec(gate * grad[t]); rows of empty slots are not written. */
 int planmoe_layer_combine_bwd(const void *grad, const void *rows, int dtype, int codec, const float *gates,
                               const int32_t *indices, const int32_t *locations, int64_t plane_stride,
                               int top_k, int samples, int model_dim, int experts, int capacity,
                               void *grad_rows, float *grad_gates, void *stream);
+
+/* The same with codec = 1 from what planmoe_layer_combine_keep kept: same bits as from the rows. */
+int planmoe_layer_combine_bwd_codes(const void *grad, const uint8_t *codes, const void *bias, const void *scale,
+                                    int dtype, const float *gates, const int32_t *indices,
+                                    const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                                    int model_dim, int experts, int capacity, void *grad_rows,
+                                    float *grad_gates, void *stream);
 
 /* out[e][c] = sum over the rows in use of a[e] (live as planmoe_expert_gemm): a bias gradient of
  * experts/ffn.py:77-79.  fp32 sums, one rounding. */

@@ -13,9 +13,19 @@
 
 namespace pm {
 
-// decompress(compress(row)) of a row held as CACHE vectors per lane (vectors past the end: copies of the last)
-template <int DT, int CACHE, bool CANON>
-__device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
+// a vector's codes as they are kept, one byte a value
+template <int DT> struct CodeWords { uint32_t w[Elem<DT>::VEC / 4]; };
+template <int DT>
+__device__ __forceinline__ void store_codes(uint8_t *to, const CodeWords<DT> &v)
+{
+    if constexpr (Elem<DT>::VEC == 8) stream_store(reinterpret_cast<uint2 *>(to), make_uint2(v.w[0], v.w[1]));
+    else stream_store(reinterpret_cast<uint32_t *>(to), v.w[0]);
+}
+
+// decompress(compress(row)) of a row held as CACHE vectors per lane (vectors past the end: copies of the last);
+// keep(c, codes) sees the codes of vector c.  Returns the row's minimum and scale.
+template <int DT, int CACHE, bool CANON, typename Keep>
+__device__ __forceinline__ float2 through_int8(uint4 (&row)[CACHE], Keep keep)
 {
     using E = Elem<DT>;
     RowStats<DT, CANON> stats;
@@ -30,15 +40,17 @@ __device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
     auto body = [&](auto mode) {
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) {
-            uint32_t w[2];
+            CodeWords<DT> code;
             float f[E::VEC];
-            enc.template encode<decltype(mode)::value>(row[c], w);
+            enc.template encode<decltype(mode)::value>(row[c], code.w);
+            keep(c, code);
 #pragma unroll
-            for (int q = 0; q < E::VEC / 4; ++q) dec.word(w[q], f + 4 * q);
+            for (int q = 0; q < E::VEC / 4; ++q) dec.word(code.w[q], f + 4 * q);
             row[c] = E::pack(f);
         }
     };
     if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
+    return make_float2(mn, scale);
 }
 
 // The same with the decoder as a table: a row has 256 codes, so a wave works out gate * decoded(code) for four codes a
@@ -46,9 +58,17 @@ __device__ __forceinline__ void through_int8(uint4 (&row)[CACHE])
 // of bf16 values took as long as its bytes.  Combine at 16384 x 4096, top-2, 113 -> 81 us,
 // at 16384 x 1024 35 -> 27, its backward pass there 64 -> 48.)
 template <int DT>
+__device__ __forceinline__ void fill_table(float mn, float scale, float gate, float *table)
+{
+    float f[4];
+    RowDecoder<DT>(mn, scale).word(0x03020100u + 0x04040404u * (uint32_t)lane_id(), f);
+    *reinterpret_cast<float4 *>(table + 4 * lane_id()) = make_float4(gate * f[0], gate * f[1], gate * f[2], gate * f[3]);
+}
+template <int DT>
 struct RowTable {
     RowEncoder<DT> enc;
     const float *tab;                            // 256 values, the wave's own
+    float mn, scale;
     template <int CACHE>
     __device__ __forceinline__ RowTable(const uint4 (&row)[CACHE], float gate, float *table) : enc(0.f, 0.f), tab(table)
     {
@@ -57,20 +77,28 @@ struct RowTable {
         stats.init();
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) stats.add(row[c]);
-        float mn, mx, f[4];
+        float mx;
         stats.finish(mn, mx);
-        const float scale = E::round(mx - mn);
+        scale = E::round(mx - mn);
         enc = RowEncoder<DT>(mn, scale);
-        RowDecoder<DT>(mn, scale).word(0x03020100u + 0x04040404u * (uint32_t)lane_id(), f);
-        *reinterpret_cast<float4 *>(table + 4 * lane_id()) = make_float4(gate * f[0], gate * f[1], gate * f[2], gate * f[3]);
+        fill_table<DT>(mn, scale, gate, table);
+    }
+    template <bool FAST, typename Keep>
+    __device__ __forceinline__ void values(const uint4 &raw, float (&f)[Elem<DT>::VEC], Keep keep) const
+    {
+        uint32_t c[Elem<DT>::VEC];
+        enc.template codes<FAST>(raw, c);
+        CodeWords<DT> code;
+#pragma unroll
+        for (int q = 0; q < Elem<DT>::VEC / 4; ++q) code.w[q] = c[4 * q] | (c[4 * q + 1] << 8) | (c[4 * q + 2] << 16) | (c[4 * q + 3] << 24);
+        keep(code);
+#pragma unroll
+        for (int i = 0; i < Elem<DT>::VEC; ++i) f[i] = tab[c[i]];
     }
     template <bool FAST>
     __device__ __forceinline__ void values(const uint4 &raw, float (&f)[Elem<DT>::VEC]) const
     {
-        uint32_t c[Elem<DT>::VEC];
-        enc.template codes<FAST>(raw, c);
-#pragma unroll
-        for (int i = 0; i < Elem<DT>::VEC; ++i) f[i] = tab[c[i]];
+        values<FAST>(raw, f, [](const CodeWords<DT> &) {});
     }
 };
 // what a wave's lanes wrote to its LDS is there for all of them, and what they read has been read
@@ -85,12 +113,13 @@ __device__ __forceinline__ void table_sync()
 // One wave per token; the rows of two choices are requested before either is used and stay as they lie in
 // memory until their values are looked up, vector by vector (two 8 KB rows and their sum in fp32 took 230
 // registers and left two waves per SIMD).  16384 x 4096 bf16, top-2, 403 MB: 81 us = 5.0 TB/s.  More than two
-// choices keep their sum in fp32.
-template <int DT, int CACHE, bool TWO>
+// choices keep their sum in fp32.  KEEP: the rows' codes, minima and scales are stored as well, by slot (what a backward
+// pass reads in place of the rows: a byte a value to hold between the passes).
+template <int DT, int CACHE, bool TWO, bool KEEP>
 __global__ __launch_bounds__(256) void layer_combine_kernel(
     const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
     const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples, int model_dim, int capacity,
-    void *__restrict__ out)
+    void *__restrict__ out, uint8_t *__restrict__ codes, void *__restrict__ bias, void *__restrict__ scales)
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
@@ -105,6 +134,12 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
     };
+    auto keep_codes = [&](int s, int c, const CodeWords<DT> &code) {
+        if (KEEP && s >= 0 && c * WAVE + lane < units) store_codes<DT>(codes + (int64_t)s * model_dim + (c * WAVE + lane) * V, code);
+    };
+    auto keep_row = [&](int s, float mn, float scale) {
+        if (KEEP && s >= 0 && lane == 0) { E::store(bias, s, mn); E::store(scales, s, scale); }
+    };
     if constexpr (TWO) {
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, 0, top_k, 0x7fffffff, capacity, slot, gate);
@@ -117,16 +152,18 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
         // (a choice without a slot has no row: row 0 stands for it above, what is looked up is not used)
         const RowTable<DT> t1(s1 >= 0 ? r1 : r0, g1, s_table[threadIdx.x >> 6][1]);
         table_sync();
+        keep_row(s0, t0.mn, t0.scale);
+        keep_row(s1, t1.mn, t1.scale);
         auto body = [&](auto mode) {
 #pragma unroll
             for (int c = 0; c < CACHE; ++c) {
                 float f[V], h[V];
-                t0.template values<decltype(mode)::value>(r0[c], f);
+                t0.template values<decltype(mode)::value>(r0[c], f, [&](const CodeWords<DT> &code) { keep_codes(s0, c, code); });
 #pragma unroll
                 for (int i = 0; i < V; ++i) f[i] = s0 >= 0 ? f[i] : 0.f;
                 if (top_k > 1) {
                     if (s1 >= 0) {
-                        t1.template values<decltype(mode)::value>(r1[c], h);
+                        t1.template values<decltype(mode)::value>(r1[c], h, [&](const CodeWords<DT> &code) { keep_codes(s1, c, code); });
 #pragma unroll
                         for (int i = 0; i < V; ++i) f[i] += h[i];
                     } else {
@@ -150,7 +187,10 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
             const int s = rl_i(slot, j);
             const float g = rl_f(gate, j);
             request(s, r);
-            if (s >= 0) through_int8<DT, CACHE, false>(r);
+            if (s >= 0) {
+                const float2 row = through_int8<DT, CACHE, false>(r, [&](int c, const CodeWords<DT> &code) { keep_codes(s, c, code); });
+                keep_row(s, row.x, row.y);
+            }
 #pragma unroll
             for (int c = 0; c < CACHE; ++c) {
                 float f[V];
@@ -169,12 +209,14 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
 
 // Backward of the combine: grad_gates_j = <grad[t], codec(rows[slot_j])> and grad_rows[slot_j] =
 // codec(round(gate_j * grad[t])) (GatingDecoder.backward, fast_dispatch.py:62-79, with the two codec
-// passes around it, overlap.py:19-34).
-template <int DT, int CACHE, bool INT8>
+// passes around it, overlap.py:19-34).  The rows come as they are (SEEN_ROWS without a codec, SEEN_INT8 with), or as the codes,
+// minima and scales that the forward pass kept (SEEN_CODES): half or a quarter of the bytes, and no codes to work out.
+enum { SEEN_ROWS, SEEN_INT8, SEEN_CODES };
+template <int DT, int CACHE, int SEEN>
 __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
-    const void *__restrict__ grad, const void *__restrict__ rows, const float *__restrict__ gates,
-    const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples,
-    int model_dim, int capacity, void *__restrict__ grad_rows, float *__restrict__ grad_gates)
+    const void *__restrict__ grad, const void *__restrict__ rows, const void *__restrict__ bias, const void *__restrict__ scales,
+    const float *__restrict__ gates, const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
+    int top_k, int samples, int model_dim, int capacity, void *__restrict__ grad_rows, float *__restrict__ grad_gates)
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
@@ -183,6 +225,8 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= samples) return;                    // (no work-group barrier below)
     const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
+    constexpr bool INT8 = SEEN != SEEN_ROWS;
+    using seen_t = std::conditional_t<SEEN == SEEN_CODES, CodeWords<DT>, uint4>;       // a lane's vector of a row
     uint4 g_row[CACHE];
     {
         const uint4 *src = reinterpret_cast<const uint4 *>((const char *)grad + (int64_t)t * row_bytes);
@@ -194,10 +238,12 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
         if (lane < np && slot < 0) grad_gates[(int64_t)(j0 + lane) * stride + t] = 0.f;
+        float mn = 0.f, scale = 0.f;
+        if (SEEN == SEEN_CODES && lane < np && slot >= 0) { mn = E::load(bias, slot); scale = E::load(scales, slot); }
         // the next choice's row is on its way while this one's is worked on (a dropped choice reads slot 0, unused)
-        uint4 next[CACHE];
+        seen_t next[CACHE];
         auto request = [&](int j) {
-            const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)max(rl_i(slot, j), 0) * row_bytes);
+            const seen_t *src = reinterpret_cast<const seen_t *>(rows) + (int64_t)max(rl_i(slot, j), 0) * units;
 #pragma unroll
             for (int c = 0; c < CACHE; ++c) next[c] = src[min(c * WAVE + lane, units - 1)];
         };
@@ -205,9 +251,9 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
         for (int j = 0; j < np; ++j) {
             const int s = rl_i(slot, j);
             const float g = rl_f(gate, j);
-            uint4 r[CACHE];
+            seen_t seen[CACHE];
 #pragma unroll
-            for (int c = 0; c < CACHE; ++c) r[c] = next[c];
+            for (int c = 0; c < CACHE; ++c) seen[c] = next[c];
             if (j + 1 < np) request(j + 1);
             if (s < 0) continue;
             float acc = 0.f;
@@ -219,15 +265,27 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
                     for (int i = 0; i < V; ++i) acc = fmaf(b[i], a[i], acc);
                 }
             };
-            if constexpr (INT8) {
+            if constexpr (SEEN == SEEN_CODES) {
                 float *table = s_table[threadIdx.x >> 6];
-                const RowTable<DT> tab(r, 1.f, table);
+                fill_table<DT>(rl_f(mn, j), rl_f(scale, j), 1.f, table);
+                table_sync();
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) {
+                    float b[V];
+#pragma unroll
+                    for (int i = 0; i < V; ++i) b[i] = table[(seen[c].w[i / 4] >> (8 * (i % 4))) & 0xffu];
+                    dot(c, b);
+                }
+                table_sync();
+            } else if constexpr (SEEN == SEEN_INT8) {
+                float *table = s_table[threadIdx.x >> 6];
+                const RowTable<DT> tab(seen, 1.f, table);
                 table_sync();
                 auto body = [&](auto mode) {
 #pragma unroll
                     for (int c = 0; c < CACHE; ++c) {
                         float b[V];
-                        tab.template values<decltype(mode)::value>(r[c], b);
+                        tab.template values<decltype(mode)::value>(seen[c], b);
                         dot(c, b);
                     }
                 };
@@ -237,13 +295,14 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
 #pragma unroll
                 for (int c = 0; c < CACHE; ++c) {
                     float b[V];
-                    E::unpack(r[c], b);
+                    E::unpack(seen[c], b);
                     dot(c, b);
                 }
             }
             acc = wave_sum(acc);
             if (lane == 0) grad_gates[(int64_t)(j0 + j) * stride + t] = acc;
             // the gradient row as the dispatcher stores it for this gate: round(0 + g * x)
+            uint4 r[CACHE];
 #pragma unroll
             for (int c = 0; c < CACHE; ++c) {
                 float a[V];
@@ -429,6 +488,29 @@ int rows_check(const char *who, int dtype, const void *rows, const int32_t *indi
         else CALL(16);                                        \
     } while (0)
 
+// codes NULL: none are kept
+static int combine_int8_rows(const char *who, const void *rows, int dtype, const float *gates, const int32_t *indices, const int32_t *locations,
+                             int64_t plane_stride, int top_k, int samples, int model_dim, int capacity, void *out, uint8_t *codes, void *bias,
+                             void *scale, void *stream)
+{
+    if (samples == 0) return 0;
+    PM_REQUIRE(out && aligned16(out), "%s: NULL or unaligned output", who);
+    const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
+    hipStream_t st = (hipStream_t)stream;
+#define PM_LC_(CACHE, TWO, KEEP) (layer_combine_kernel<DT, CACHE, TWO, KEEP><<<(samples + 3) / 4, 256, 0, st>>>(rows, gates, indices, locations, \
+        plane_stride, top_k, samples, model_dim, capacity, out, codes, bias, scale))
+#define PM_LC(CACHE)                                                                          \
+    do {                                                                                      \
+        if (top_k <= 2) { if (codes) PM_LC_(CACHE, true, true); else PM_LC_(CACHE, true, false); }     \
+        else { if (codes) PM_LC_(CACHE, false, true); else PM_LC_(CACHE, false, false); }     \
+    } while (0)
+    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LC));
+#undef PM_LC
+#undef PM_LC_
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
 extern "C" int planmoe_layer_combine(const void *rows, int dtype, int codec, const float *gates, const int32_t *indices,
                                      const int32_t *locations, int64_t plane_stride, int top_k, int samples, int model_dim,
                                      int experts, int capacity, void *out, void *stream)
@@ -436,16 +518,41 @@ extern "C" int planmoe_layer_combine(const void *rows, int dtype, int codec, con
     const char *who = "planmoe_layer_combine";
     if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
     if (codec == 0) return planmoe_combine_fwd(rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, stream);
+    return combine_int8_rows(who, rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, nullptr, nullptr,
+                             nullptr, stream);
+}
+
+extern "C" int planmoe_layer_combine_keep(const void *rows, int dtype, const float *gates, const int32_t *indices, const int32_t *locations,
+                                          int64_t plane_stride, int top_k, int samples, int model_dim, int experts, int capacity,
+                                          void *out, uint8_t *codes, void *bias, void *scale, void *stream)
+{
+    const char *who = "planmoe_layer_combine_keep";
+    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
+    PM_REQUIRE(codes && bias && scale && aligned16(codes), "%s: NULL output, or codes not 16-byte aligned", who);
+    return combine_int8_rows(who, rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, codes, bias, scale,
+                             stream);
+}
+
+// seen: SEEN_ROWS, SEEN_INT8 or SEEN_CODES (bias and scale are read with the last only)
+static int combine_bwd_rows(const char *who, int seen, const void *grad, const void *rows, const void *bias, const void *scale, int dtype,
+                            const float *gates, const int32_t *indices, const int32_t *locations, int64_t plane_stride, int top_k,
+                            int samples, int model_dim, int capacity, void *grad_rows, float *grad_gates, void *stream)
+{
     if (samples == 0) return 0;
-    PM_REQUIRE(out && aligned16(out), "%s: NULL or unaligned output", who);
+    PM_REQUIRE(grad && grad_rows && grad_gates && gates && aligned16(grad) && aligned16(grad_rows), "%s: NULL or unaligned argument", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
     hipStream_t st = (hipStream_t)stream;
-#define PM_LC_(CACHE, TWO) (layer_combine_kernel<DT, CACHE, TWO><<<(samples + 3) / 4, 256, 0, st>>>(rows, gates, indices, locations, \
-        plane_stride, top_k, samples, model_dim, capacity, out))
-#define PM_LC(CACHE) do { if (top_k <= 2) PM_LC_(CACHE, true); else PM_LC_(CACHE, false); } while (0)
-    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LC));
-#undef PM_LC
-#undef PM_LC_
+#define PM_LB_(CACHE, SEEN) (layer_combine_bwd_kernel<DT, CACHE, SEEN><<<(samples + 3) / 4, 256, 0, st>>>(grad, rows, bias, scale, gates, indices, \
+        locations, plane_stride, top_k, samples, model_dim, capacity, grad_rows, grad_gates))
+#define PM_LB(CACHE)                                                                          \
+    do {                                                                                      \
+        if (seen == SEEN_CODES) PM_LB_(CACHE, SEEN_CODES);                                    \
+        else if (seen == SEEN_INT8) PM_LB_(CACHE, SEEN_INT8);                                 \
+        else PM_LB_(CACHE, SEEN_ROWS);                                                        \
+    } while (0)
+    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LB));
+#undef PM_LB
+#undef PM_LB_
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -457,18 +564,20 @@ extern "C" int planmoe_layer_combine_bwd(const void *grad, const void *rows, int
 {
     const char *who = "planmoe_layer_combine_bwd";
     if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
-    if (samples == 0) return 0;
-    PM_REQUIRE(grad && grad_rows && grad_gates && gates && aligned16(grad) && aligned16(grad_rows), "%s: NULL or unaligned argument", who);
-    const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
-    hipStream_t st = (hipStream_t)stream;
-#define PM_LB_(CACHE, INT8) (layer_combine_bwd_kernel<DT, CACHE, INT8><<<(samples + 3) / 4, 256, 0, st>>>(grad, rows, gates, indices, \
-        locations, plane_stride, top_k, samples, model_dim, capacity, grad_rows, grad_gates))
-#define PM_LB(CACHE) do { if (codec) PM_LB_(CACHE, true); else PM_LB_(CACHE, false); } while (0)
-    PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LB));
-#undef PM_LB
-#undef PM_LB_
-    PM_LAUNCH_CHECK(who);
-    return 0;
+    return combine_bwd_rows(who, codec ? SEEN_INT8 : SEEN_ROWS, grad, rows, nullptr, nullptr, dtype, gates, indices, locations, plane_stride, top_k,
+                            samples, model_dim, capacity, grad_rows, grad_gates, stream);
+}
+
+extern "C" int planmoe_layer_combine_bwd_codes(const void *grad, const uint8_t *codes, const void *bias, const void *scale, int dtype,
+                                               const float *gates, const int32_t *indices, const int32_t *locations,
+                                               int64_t plane_stride, int top_k, int samples, int model_dim, int experts,
+                                               int capacity, void *grad_rows, float *grad_gates, void *stream)
+{
+    const char *who = "planmoe_layer_combine_bwd_codes";
+    if (rows_check(who, dtype, codes, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
+    PM_REQUIRE((bias && scale) || samples == 0, "%s: NULL argument", who);
+    return combine_bwd_rows(who, SEEN_CODES, grad, codes, bias, scale, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim,
+                            capacity, grad_rows, grad_gates, stream);
 }
 
 // how many shares a reduction over `rows` is cut into for `blocks` column blocks: enough work-groups for the GPU, at least 32 rows each

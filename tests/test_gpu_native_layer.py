@@ -261,3 +261,82 @@ def test_fp32_layer_with_two_million_slots_an_expert():
     T, cf = 8, 524290.0                          # capacity 4 cf: 2097160, 2 GiB over 256 rows of 4-byte values and 8
     args = ("no", torch.float32, T, 8, 8, 2, 1, cf, True)
     _compare(_run(True, *args), _run(False, *args), 2e-5)
+
+
+# the codes kept for the backward pass: what the codec gives for the rows that hold a token, and nothing else written; the
+# output, the gradients of the gates and of the rows are the same bits as with the rows themselves
+@pytest.mark.parametrize("M", [8, 520, 4096])
+@pytest.mark.parametrize("k", [1, 2, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_layer_combine_from_kept_codes(M, k, dtype):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", M, k, dtype, flush=True)
+    T, E, cap = 37, 4, 29
+    g = torch.Generator().manual_seed(M + k)
+    rows = torch.randn(E * cap, M, generator=g)
+    rows[3] = 0.25
+    rows[7, M // 2] = float("nan")
+    rows[9, 0] = float("inf")
+    rows[11, ::2] = -0.0
+    rows[13] *= 1e-30 if dtype != torch.float16 else 1e-6
+    rows = rows.to(dtype).to(DEV)
+    # pair n of a token and a choice has slot n % (cap + 3) of expert n / (cap + 3): every slot once, some behind the capacity
+    n = torch.arange(T * k).view(T, k).t()
+    idx, loc = (n // (cap + 3)).int().contiguous().to(DEV), (n % (cap + 3)).int().contiguous().to(DEV)
+    gates, grad = torch.rand(k, T, generator=g).to(DEV), torch.randn(T, M, generator=g).to(dtype).to(DEV)
+    out, want = (torch.empty(T, M, dtype=dtype, device=DEV) for _ in range(2))
+    codes = torch.full((E * cap, M), 77, dtype=torch.uint8, device=DEV)
+    bias, scale = (torch.full((E * cap,), 5.0, dtype=dtype, device=DEV) for _ in range(2))
+    planes = (ops._ptr(gates), ops._ptr(idx), ops._ptr(loc), T, k, T, M, E, cap)
+    check(lib.planmoe_layer_combine(ops._ptr(rows), ops._dt(rows, "t"), 1, *planes, ops._ptr(want), ops._stream(rows)))
+    check(lib.planmoe_layer_combine_keep(ops._ptr(rows), ops._dt(rows, "t"), *planes, ops._ptr(out), ops._ptr(codes), ops._ptr(bias),
+                                         ops._ptr(scale), ops._stream(rows)))
+    all_codes, all_bias, all_scale = ops.int8_compress(rows)
+    grad_rows, wanted_rows = torch.full_like(rows, 7.0), torch.full_like(rows, 7.0)
+    gg, wanted_gates = torch.empty(k, T, device=DEV), torch.empty(k, T, device=DEV)
+    check(lib.planmoe_layer_combine_bwd(ops._ptr(grad), ops._ptr(rows), ops._dt(rows, "t"), 1, *planes, ops._ptr(wanted_rows), ops._ptr(wanted_gates),
+                                        ops._stream(rows)))
+    check(lib.planmoe_layer_combine_bwd_codes(ops._ptr(grad), ops._ptr(codes), ops._ptr(bias), ops._ptr(scale), ops._dt(rows, "t"), *planes,
+                                              ops._ptr(grad_rows), ops._ptr(gg), ops._stream(rows)))
+    torch.cuda.synchronize()
+    live = loc < cap
+    used = torch.zeros(E * cap, dtype=torch.bool, device=DEV)
+    used[(idx * cap + loc).long()[live]] = True
+    assert int(used.sum()) == int(live.sum()) and int((~live).sum()) > 0
+
+    def same(a, b):
+        bits = torch.int32 if dtype == torch.float32 else torch.int16
+        return bool(((a.view(bits) == b.view(bits)) | (a.isnan() & b.isnan())).all())
+    assert torch.equal(codes[used], all_codes.view(E * cap, M)[used]) and bool((codes[~used] == 77).all())
+    assert same(bias[used], all_bias.view(-1)[used]) and same(scale[used], all_scale.view(-1)[used])
+    assert bool((bias[~used] == 5.0).all()) and bool((scale[~used] == 5.0).all())
+    assert same(out, want) and same(grad_rows, wanted_rows)
+    assert bool(((gg == wanted_gates) | (gg.isnan() & wanted_gates.isnan())).all())
+
+
+def test_int8_training_holds_no_more_than_its_steps():
+    """Between the passes the second product's output is held as codes, a byte a value, as the steps hold it."""
+    from planmoe_amd import overlap
+
+    def held(native, dtype):
+        overlap.NATIVE_LAYER = native
+        kept = {}
+
+        def pack(t):
+            kept[t.untyped_storage().data_ptr()] = t.untyped_storage().nbytes()
+            return t
+        try:
+            layer, x = _layer(dtype, "int8", M=256, H=64), torch.randn(512, 256, device=DEV).to(dtype).requires_grad_(True)
+            with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+                y = layer(x)
+            y.float().sum().backward()
+            torch.cuda.synchronize()
+        finally:
+            overlap.NATIVE_LAYER = True
+        return sum(kept.values())
+
+    for dtype in (torch.bfloat16, torch.float32):
+        native, steps = held(True, dtype), held(False, dtype)
+        print("held", dtype, native, steps, flush=True)
+        assert native <= steps + 4096            # (a plane or a scalar that the steps take apart)
