@@ -14,12 +14,12 @@ using namespace planmoe_host;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// part of a buffer as a tensor of its own: no view in autograd's sense (an output of a node may be one), its in-place
+// part of a flat buffer as a tensor of its own: no view in autograd's sense (an output of a node may be one), its in-place
 // changes are counted apart from the buffer's
-Tensor piece(const Tensor &base, int64_t first, at::IntArrayRef sizes)
+Tensor piece(const Tensor &base, int64_t first, int64_t size)
 {
     const at::AutoDispatchBelowADInplaceOrView guard;
-    return base.narrow(0, first, c10::multiply_integers(sizes)).view(sizes);
+    return base.narrow(0, first, size);
 }
 
 // k flat tensors as planes of one buffer, equally far apart: the distance in elements (0: any, one plane), or -1
@@ -92,7 +92,7 @@ Tensor gather(const Tensor &slots, const float *gates, const Planes &p)
 std::vector<Tensor> planes_as_tensors(const Tensor &buffer, const Planes &p)
 {
     std::vector<Tensor> parts;
-    for (int j = 0; j < p.k; ++j) parts.push_back(piece(buffer, j * p.stride, {p.samples}));
+    for (int j = 0; j < p.k; ++j) parts.push_back(piece(buffer, j * p.stride, p.samples));
     return parts;
 }
 
@@ -186,7 +186,7 @@ std::optional<Tensor> move(const Tensor &data_, const std::vector<Tensor> &gates
 struct Routed {
     int T, E, k;
     bool normalize, want_loss;
-    Tensor indices;                              // [k T]
+    Tensor read;                                 // what the backward pass reads: indices [k T], counts [k E]
     std::vector<Tensor> locations;
 };
 
@@ -194,24 +194,24 @@ struct Route : public torch::autograd::Function<Route> {
     static variable_list forward(AutogradContext *ctx, const Tensor &scores, Routed *r)
     {
         ctx->set_materialize_grads(false);
-        const int64_t plane = (int64_t)r->k * r->T;
-        Tensor ints_ = at::empty({2 * plane + (int64_t)r->k * r->E}, scores.options().dtype(at::kInt)), gates = at::empty({plane}, scores.options());
+        const int64_t plane = (int64_t)r->k * r->T, read = plane + (int64_t)r->k * r->E;
+        Tensor ints_ = at::empty({read + plane}, scores.options().dtype(at::kInt)), gates = at::empty({plane}, scores.options());
         Tensor loss = r->want_loss ? at::empty({}, scores.options().dtype(at::kFloat)) : Tensor();
         Tensor ws = bytes((int64_t)planmoe_route_workspace_bytes(r->T, r->E, r->k), scores);
         int32_t *i = ints_.data_ptr<int32_t>();
-        PM_CALL(planmoe_route_topk(scores.data_ptr(), pm_dtype(scores.scalar_type()), 0, nullptr, r->T, r->E, r->k, r->normalize, i, i + plane,
-                                   gates.data_ptr(), r->T, nullptr, loss.defined() ? loss.data_ptr<float>() : nullptr, i + 2 * plane, ws.data_ptr(),
+        PM_CALL(planmoe_route_topk(scores.data_ptr(), pm_dtype(scores.scalar_type()), 0, nullptr, r->T, r->E, r->k, r->normalize, i, i + read,
+                                   gates.data_ptr(), r->T, nullptr, loss.defined() ? loss.data_ptr<float>() : nullptr, i + plane, ws.data_ptr(),
                                    (size_t)ws.numel(), current_stream()));
         variable_list out;
-        r->indices = piece(ints_, 0, {plane});
         for (int j = 0; j < r->k; ++j) {
-            r->locations.push_back(piece(ints_, plane + (int64_t)j * r->T, {r->T}));
-            out.push_back(piece(gates, (int64_t)j * r->T, {r->T}));
+            r->locations.push_back(piece(ints_, read + (int64_t)j * r->T, r->T));
+            out.push_back(piece(gates, (int64_t)j * r->T, r->T));
         }
         if (r->want_loss) out.push_back(loss);
-        // (as variables: the gradient is that of these indices, and an index plane edited in place until then is refused.
+        // (as a variable: the gradient is that of these indices, and an index plane edited in place until then is refused.
         // The locations are not read again and are edited at will)
-        ctx->save_for_backward({scores, r->indices, piece(ints_, 2 * plane, {(int64_t)r->k * r->E})});
+        r->read = piece(ints_, 0, read);
+        ctx->save_for_backward({scores, r->read});
         ctx->saved_data["k"] = (int64_t)r->k;
         ctx->saved_data["normalize"] = r->normalize;
         return out;
@@ -220,7 +220,8 @@ struct Route : public torch::autograd::Function<Route> {
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &scores = saved[0], &indices = saved[1], &counts = saved[2];
+        const Tensor &scores = saved[0];
+        const int32_t *i = ints(saved[1]);
         const c10::DeviceGuard guard(scores.device());
         const int k = (int)ctx->saved_data["k"].toInt(), T = (int)scores.size(0), E = (int)scores.size(1);
         std::vector<Tensor> gg(grads.begin(), grads.begin() + k);
@@ -234,8 +235,8 @@ struct Route : public torch::autograd::Function<Route> {
         if (!any) return {Tensor(), Tensor()};
         if (spacing(gg) != T && k > 1) gg = {at::stack(gg)};        // (the indices' planes are T apart)
         Tensor out = at::empty_like(scores);
-        PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), ints(indices), gg[0].data_ptr(), stride, T, E, k,
-                                  ctx->saved_data["normalize"].toBool(), dl.defined() ? floats(dl) : nullptr, dl.defined() ? ints(counts) : nullptr,
+        PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), i, gg[0].data_ptr(), stride, T, E, k,
+                                  ctx->saved_data["normalize"].toBool(), dl.defined() ? floats(dl) : nullptr, dl.defined() ? i + (int64_t)k * T : nullptr,
                                   0, out.data_ptr(), current_stream()));
         return {out, Tensor()};
     }
@@ -267,7 +268,7 @@ std::optional<Critical> extract_critical(const Tensor &scores_, int64_t top_k, b
     PM_CALL(planmoe_capacity(r.T, r.E, r.k, capacity_factor, (int)alignment, &capacity));
     // (views of what the node has saved: their in-place changes are its)
     std::vector<Tensor> indices;
-    for (int j = 0; j < r.k; ++j) indices.push_back(r.indices.narrow(0, (int64_t)j * r.T, r.T));
+    for (int j = 0; j < r.k; ++j) indices.push_back(r.read.narrow(0, (int64_t)j * r.T, r.T));
     return Critical(std::move(indices), std::move(r.locations), std::move(out), capacity, loss);
 }
 

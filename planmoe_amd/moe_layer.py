@@ -150,6 +150,8 @@ class MOELayer(torch.nn.Module):
         self.protected_shape = y.shape
         return y.reshape(y.size(0), y.size(1), -1)
 
+    _own_expert_local = expert_local            # (as defined here: overlap.native_codec asks whether it still is)
+
     # ------------------------------------------------------------------ forward
     def _deliver(self, y, l_aux, shape, dtype):
         """Common tail of every path (moe_layer.py:306-311)."""
@@ -279,19 +281,6 @@ class MOELayer(torch.nn.Module):
             return extract_critical(scores, top_k=k, loss_fn=loss_fn, capacity_factor=cf,
                                     batch_prioritized_routing=self.batch_prioritized_routing,
                                     normalize_gate=self.normalize_gate, group=self.group, alignment=alignment)
-
-
-# the way from the layer into its built-in experts and through them, as defined here
-_EXPERT_LOCAL = MOELayer.expert_local
-_EXPERTS_FORWARD, _EXPERTS_LINEAR = _experts.FusedExpertsNetwork.forward, _experts.FusedExpertsNetwork._linear
-
-
-def runs_built_in_experts(layer):
-    """Whether a layer over a FusedExpertsNetwork has that way: no part of it replaced on the objects, in a subclass or
-    in the classes."""
-    return all(getattr(type(owner), name) is method and name not in owner.__dict__ for owner, name, method in (
-        (layer, 'expert_local', _EXPERT_LOCAL), (layer.experts, 'forward', _EXPERTS_FORWARD),
-        (layer.experts, '_linear', _EXPERTS_LINEAR)))
 
 
 moe_layer = MOELayer

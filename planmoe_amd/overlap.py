@@ -8,7 +8,8 @@ from torch.nn.modules.module import _has_any_global_hook
 
 from . import compressor as _ck
 from . import ops
-from .gates import weight_grad
+from .experts import FusedExpertsNetwork, row_fits
+from .gates import LinearTopKGate, weight_grad
 
 MAX_NUM_SPLIT = 32     # AllToAllStatus.max_num_split of the reference (communicate.py)
 
@@ -134,7 +135,6 @@ FFN_FROM_CODES_AFFINE = False
 def ffn_from_codes_fn(module, x, degree, reserve_dims):
     """The experts as a function of (codes, bias, scale) [E, C, ...] when the layer's receive side
     may skip the decompress, else None."""
-    from .experts import FusedExpertsNetwork
     if not (FFN_FROM_CODES and not torch.is_grad_enabled() and type(module) is FusedExpertsNetwork and degree == 1 and
             reserve_dims == 1 and x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 64 == 0 and
             module.hidden_size_per_expert % 128 == 0 and module.batched_fc1_w.dtype == torch.bfloat16 and
@@ -155,31 +155,35 @@ def _hooked(module):
     return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
 
 
+def _replaced(layer, experts):
+    """Whether a method on the way from the layer into its built-in experts and through them is not the one defined here:
+    replaced on the object (as adapters and offloading wrappers do), in a subclass or in the class."""
+    own, cls, theirs, inner = layer.__dict__, type(layer), experts.__dict__, type(experts)
+    return (cls.expert_local is not cls._own_expert_local or inner.forward is not inner._own_forward or
+            inner._linear is not inner._own_linear or 'expert_local' in own or 'forward' in theirs or '_linear' in theirs)
+
+
 def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     """The codec number for csrc/ext/layer.cpp when the whole layer is its business, else None.  What is left to
-    the steps below: experts or gates that are not the built-in ones, have a method replaced (on the object,
-    as adapters and offloading wrappers do, in a subclass or in the class) or carry hooks, other dtypes (a gate in
-    fp32 next to 16-bit rows among them), overlap slices, autocast, and every option that asks for the
-    reference's structure; weights that are not 16-byte aligned."""
-    from .experts import FusedExpertsNetwork, row_fits
-    from .gates import LinearTopKGate
-    from .moe_layer import runs_built_in_experts
+    the steps below: experts or gates that are not the built-in ones or carry hooks, replaced methods, other dtypes (a
+    gate in fp32 next to 16-bit rows among them), overlap slices, autocast, every option that asks for the
+    reference's structure, and weights that are not 16-byte aligned (views of a flat buffer: the steps copy them)."""
     experts = layer.experts
     if not (NATIVE_LAYER and FUSE_GATE and FUSE_INT8 and FUSE_ZFP and not FFN_FROM_CODES and not _ck.SINGLE_RANK_COMM_COPIES and
             degree == 1 and reserve_dims == 1 and layer.is_postscore and x.is_cuda and capacity >= 1 and x.shape[0] >= 1 and
             type(experts) is FusedExpertsNetwork and experts._relu and type(gate) is LinearTopKGate and
-            layer.num_global_experts <= 64 and runs_built_in_experts(layer)):
+            layer.num_global_experts <= 64 and not _replaced(layer, experts)):
         return None
     dtype, M, H = x.dtype, x.shape[1], experts.hidden_size_per_expert
     vec = 8 if dtype == torch.bfloat16 else 4
     if not ((dtype == torch.bfloat16 or dtype == torch.float32) and M % vec == 0 and H % vec == 0 and M <= 1024 * vec and
             row_fits(H, dtype) and experts.output_dim in (None, M)):
         return None
-    for p in (gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias):
+    w1, w2 = experts.batched_fc1_w, experts.batched_fc2_w
+    for p in (gate.wg.weight, w1, experts.batched_fc1_bias, w2, experts.batched_fc2_bias):
         if p.dtype != dtype or not p.is_contiguous():
             return None
-    # (weights that are views of a flat buffer: the steps copy them for their products)
-    if (experts.batched_fc1_w.data_ptr() | experts.batched_fc2_w.data_ptr()) % 16:
+    if (w1.data_ptr() | w2.data_ptr()) % 16:
         return None
     if _hooked(experts) or _hooked(gate) or _hooked(gate.wg) or _has_any_global_hook() or torch.is_autocast_enabled(x.device.type):
         return None
@@ -379,7 +383,6 @@ def gate_weight_fits(gate, x):
 
 def gate_route_eligible(x, gate, experts, is_postscore):
     """Gate, routing and encode as one call chain (planmoe_gate_route) for any compressor."""
-    from .gates import LinearTopKGate
     vec = 4 if x.dtype == torch.float32 else 8
     return (FUSE_GATE and is_postscore and type(gate) is LinearTopKGate and experts <= 64 and x.is_cuda and
             x.dtype in (torch.float32, torch.bfloat16, torch.float16) and x.shape[-1] % vec == 0 and
@@ -397,7 +400,6 @@ def gate_route_encode(x, gate, top_k, capacity, normalize_gate, codec):
 
 def fused_gate_eligible(x, gate, experts, compress_name, degree, is_postscore):
     """The whole send side (gate, routing, encode, compress) as planmoe_forward_int8."""
-    from .gates import LinearTopKGate
     return (fused_int8_eligible(x, compress_name, degree, is_postscore) and type(gate) is LinearTopKGate and
             experts <= 64 and x.shape[0] >= 1 and gate_weight_fits(gate, x))
 
