@@ -29,6 +29,17 @@ int  fail(const char *fmt, ...);          // sets the error text, returns 1
 void fill_u32(uint32_t *p, size_t n, uint32_t value, hipStream_t stream);
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// of the current device
+inline int compute_units()
+{
+    static int known[64];                        // (written once per device, with the same value by whoever is first)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev < 64 && known[dev]) return known[dev];
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
+    if (dev < 64) known[dev] = n;
+    return n;
+}
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 inline int dtype_bytes(int dt) { return dt == PLANMOE_F32 ? 4 : 2; }
 inline bool dtype_ok(int dt) { return dt == PLANMOE_F32 || dt == PLANMOE_BF16 || dt == PLANMOE_F16; }

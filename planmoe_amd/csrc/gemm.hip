@@ -599,17 +599,6 @@ using namespace pm;
 
 namespace {
 
-int compute_units()
-{
-    static int known[64];                        // (written once per device, with the same value by whoever is first)
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (dev < 64 && known[dev]) return known[dev];
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
-    if (dev < 64) known[dev] = n;
-    return n;
-}
-
 template <int I, int J, bool TA, bool TB, bool GRAD>
 int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 {

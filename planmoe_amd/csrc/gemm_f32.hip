@@ -337,11 +337,11 @@ int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
     if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && p.batches <= 65535 &&
         p.M <= 32 * 65535)
         return 0;
-    const int64_t m = form == 2 ? p.M : rows_hint;
+    const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
     auto cost = [&](int64_t side, double us) {
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
-        return (double)((tiles + 255) / 256) * (us * kt + 2);
+        return (double)((tiles + cu - 1) / cu) * (us * kt + 2);
     };
     return cost(64, 0.47) < cost(128, 1.7) ? 64 : 128;
 }

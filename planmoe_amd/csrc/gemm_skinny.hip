@@ -199,7 +199,7 @@ int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
     (!nt ? skinny_launch<false, MF, C, U_NN, WAVES_NN, false>(p, stream, who)            \
      : grad ? skinny_launch<true, MF, C, U_NT, WAVES_NT, true>(p, stream, who)           \
             : skinny_launch<true, MF, C, U_NT, WAVES_NT, false>(p, stream, who))
-    const bool narrow = (int64_t)((p.N + 127) / 128) * p.batches < 256;
+    const bool narrow = (int64_t)((p.N + 127) / 128) * p.batches < compute_units();
     if (p.M <= 16) return narrow ? PM_SK(1, 4, 4, 16, 2, 16) : PM_SK(1, 8, 1, 16, 1, 16);
     if (p.M <= 32) return narrow && nt ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);        // (nt holds 16 KB of weight per step: 8 waves' registers)
     return narrow ? PM_SK(4, 4, 5, 8, 2, 8) : PM_SK(4, 8, 1, 8, 1, 8);
