@@ -206,15 +206,37 @@ template <int MF, int U, bool TB>
 __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args p)
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
-    const int e = blockIdx.z, m0 = blockIdx.y * 16 * MF, n0 = (blockIdx.x * 4 + wave) * 16;
-    int M = p.M;
-    if (p.live) {
+    // The pieces of 16 MF rows by 64 columns that hold rows in use, batch by batch, the row blocks of a column next to each other
+    // (they read the same weight); what is left of the grid has nothing to do.  (A grid over the capacity, with empty row
+    // blocks between full ones, leaves whole groups of compute units with the empty ones, since work is handed to them in
+    // turn: 64 experts of 32 rows, 4096 -> 1024, took 402 us at a capacity of 32 and 751 at 36, here 402 at both.)
+    // Column sums have two slots for every 64 rows in use: the second of them may have no rows.
+    auto blocks_of = [&](int rows) { return ((p.colsum ? (rows + 63) / 64 * 64 : rows) + 16 * MF - 1) / (16 * MF); };
+    auto round_up = [&](int n) { return min(p.M, (n + p.live_round - 1) / p.live_round * p.live_round); };
+    const int number = blockIdx.x, cols = (p.N + 63) / 64, most = blocks_of(p.M);
+    int e = number / (most * cols), M = p.M, blocks = most, piece = number - e * most * cols;
+    if (p.live && most == 1) {                   // (a batch is a row block at most)
         int n = 0;
         for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
-        M = min(M, (n + p.live_round - 1) / p.live_round * p.live_round);
+        M = round_up(n);
+    } else if (p.live) {                         // (lane = batch)
+        int n = 0;
+        if (lane < p.batches)
+            for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + lane];
+        const int rows = round_up(n);
+        int ends = lane < p.batches ? blocks_of(rows) * cols : 0;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(ends, d);
+            if (lane >= d) ends += o;
+        }
+        if (number >= __builtin_amdgcn_readlane(ends, 63)) return;
+        e = __builtin_amdgcn_readfirstlane(__popcll(__ballot(ends <= number)));        // (so many batches end before)
+        M = __builtin_amdgcn_readlane(rows, e);
+        blocks = blocks_of(M);
+        piece = number - (e > 0 ? __builtin_amdgcn_readlane(ends, e - 1) : 0);
     }
-    // (column sums have two slots for every 64 rows in use: the second of them may have no rows)
-    if (m0 >= (p.colsum ? (M + 63) / 64 * 64 : M) || n0 >= p.N) return;
+    const int m0 = piece % blocks * 16 * MF, n0 = (piece / blocks * 4 + wave) * 16;
+    if (M == 0 || n0 >= p.N) return;
     const float *A = p.A + (int64_t)e * p.M * p.K, *B = p.B + (int64_t)e * p.N * p.K;
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, M * p.K * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, p.N * p.K * 4, 0x00020000);
@@ -299,11 +321,17 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
     }
 }
 
+// how many pieces of `rows` by 64 columns the products have at most
+static int64_t gemm_f32_wave_pieces(const Gemm32Args &p, int rows)
+{
+    const int64_t m = p.colsum ? ((int64_t)p.M + 63) / 64 * 64 : p.M;
+    return (m + rows - 1) / rows * (((int64_t)p.N + 63) / 64) * p.batches;
+}
+
 template <int MF, int U, bool TB>
 static int gemm_f32_wave_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
 {
-    const int rows = p.colsum ? (p.M + 63) / 64 * 64 : p.M;
-    gemm_f32_wave_kernel<MF, U, TB><<<dim3((unsigned)((p.N + 63) / 64), (unsigned)((rows + 16 * MF - 1) / (16 * MF)), (unsigned)p.batches), 256, 0, stream>>>(p);
+    gemm_f32_wave_kernel<MF, U, TB><<<dim3((unsigned)gemm_f32_wave_pieces(p, 16 * MF)), 256, 0, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -331,11 +359,17 @@ static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *
 // The tile's side: a compute unit's matrix cores take 1.7 us for a k-tile of 128 x 128 and a quarter of that, and
 // a tenth, for one of 64 x 64; what counts is the fullest compute unit (4 x 300 x 512 x 1024: 64 tiles of 128, 57 us).
 // 0, waves on their own, up to 32 rows, where they read the weight once (8 experts, 2 rows each: nn 1024 -> 4096 44 -> 27 us,
-// nt 41 -> 23, 4096 -> 1024 90 -> 39; 60 rows, nt 512 -> 2048: 23 -> 31).
+// nt 41 -> 23, 4096 -> 1024 90 -> 39; 60 rows, nt 512 -> 2048: 23 -> 31).  The rows are those expected: with skewed routing an
+// expert has more, and its weight is read once for every 32 of them, but all experts together have as many rows as before,
+// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves and in tiles, nn, nt:
+//   8 experts, 256 rows, 4096 -> 1024    even 69, 86 and 90, 89;     128 of the rows on one 70, 88 and 91, 90
+//   8 experts, 128 rows, 1024 -> 4096    even 31, 32 and 43, 42;     64 on one 44, 52 and 42, 42
+//   16 experts, 256 rows, 4096 -> 1024   even 55, 60 and 93, 97;     128 on one 123, 140 and 152, 155
+//   64 experts, 2048 rows, 1024 -> 4096  even 388, 361 and 305, 303; by Zipf's law (1.2) 531, 525 and 918, 912
 int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
 {
-    if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && p.batches <= 65535 &&
-        p.M <= 32 * 65535)
+    if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
+        gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
         return 0;
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;

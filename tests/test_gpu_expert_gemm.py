@@ -272,3 +272,40 @@ def test_expert_gemm_takes_millions_of_rows(dtype, rows):
     ref = a[0, :3].double() @ w[0].double()
     torch.cuda.synchronize()
     assert bool(((out[0, :3].double() - ref).abs() <= tol[:3]).all()) and bool((out[0, 3:] == 7.0).all())
+
+
+# few rows expected, many of an expert: the waves on their own find the row blocks in use among all batches.  Batches without
+# rows first, last and in between, with one row, with a whole capacity; 64 batches; and no row counts at all
+@pytest.mark.parametrize("B,cap,n,k,counted", [(5, 300, 68, 20, True), (64, 100, 132, 64, True), (3, 100, 260, 36, False), (1, 65, 64, 16, True)])
+def test_expert_gemm_fp32_few_rows_expected_and_many_there(B, cap, n, k, counted):
+    from planmoe_amd import ops
+    print("case", B, cap, n, k, counted, flush=True)
+    g = torch.Generator().manual_seed(B + cap)
+    live = torch.randint(0, cap // 2, (2, B), generator=g, dtype=torch.int32)
+    if B > 3:
+        live[:, 0] = live[:, -1] = live[:, 2] = 0
+        live[:, 1] = cap
+        live[:, 3] = torch.tensor([0, 1])
+    rows = [min(cap, int(c)) for c in live.sum(0)] if counted else [cap] * B
+    a, h = torch.randn(B, cap, k, generator=g), torch.randn(B, cap, n, generator=g).clamp(min=0)
+    w, bias = torch.randn(B, k, n, generator=g), torch.randn(B, n, generator=g)
+    for e, r in enumerate(rows):
+        a[e, r:] = float("nan")
+    ad, wd, wt = a.to(DEV), w.to(DEV), w.transpose(1, 2).contiguous().to(DEV)
+    kw = dict(live=live.to(DEV) if counted else None, rows_hint=3)
+    nn = torch.full((B, cap, n), 7.0, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    ops.expert_gemm("nn", ad, wd, bias.to(DEV), relu=True, out=nn, **kw)
+    ops.expert_gemm("nt", ad, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(ad, wt, h.to(DEV), out=masked, **kw)
+    torch.cuda.synchronize()
+    nn, nt, masked, db = nn.cpu().double(), nt.cpu().double(), masked.cpu().double(), db.cpu().double()
+    for e, r in enumerate(rows):
+        ref, mag = a[e, :r].double() @ w[e].double(), a[e, :r].double().abs() @ w[e].double().abs()
+        tol, biased = _bound(ref, mag, k, torch.float32), ref + bias[e].double()
+        assert bool(((nn[e, :r] - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, torch.float32)).all()), e
+        assert bool(((nt[e, :r] - ref).abs() <= tol).all()), e
+        assert bool(((masked[e, :r] - ref * (h[e, :r] > 0)).abs() <= tol).all()), e
+        assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all()), e
+        stored = masked[e, :r]
+        assert bool(((db[e] - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all()), e
