@@ -33,7 +33,7 @@ struct Live {
 };
 
 struct Pass {
-    Tensor y, l_aux, gates, indices, locations, counts, scores, xe, h, ye, stream, codes, ranges;       // ranges: [2, rows] minima and scales of the codes
+    Tensor y, l_aux, gates, indices, locations, counts, scores, xe, h, ye, stream, codes;
 };
 
 Tensor lz_round_trip(const Tensor &buf, void *st)
@@ -87,7 +87,14 @@ Tensor as_rows(const Tensor &grad)
     return (uintptr_t)t.data_ptr() % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
-void *second_half(const Tensor &t) { return (char *)t.data_ptr() + t.nbytes() / 2; }
+// the codes of the experts' rows [rows, M], behind them the rows' minima and scales in x's dtype
+struct Kept {
+    Kept(const Tensor &buffer, const Shape &s, int64_t size)
+        : codes(buffer.data_ptr<uint8_t>()), bias(codes + s.rows() * s.M), scale(codes + s.rows() * (s.M + size)) {}
+    static int64_t bytes(const Shape &s, int64_t size) { return s.rows() * (s.M + 2 * size); }
+    uint8_t *codes;
+    void *bias, *scale;
+};
 
 Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
 
@@ -142,10 +149,10 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     p.y = at::empty({s.T, s.M}, x.options());
     if (codec == CODEC_INT8 && keep) {
         // (the backward pass reads the codes: a byte a value is held until then, as between Compress and its backward)
-        p.codes = bytes(s.rows() * s.M, x);
-        p.ranges = at::empty({2, s.rows()}, x.options());
-        PM_CALL(planmoe_layer_combine_keep(p.ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(),
-                                           p.codes.data_ptr<uint8_t>(), p.ranges.data_ptr(), second_half(p.ranges), st));
+        p.codes = bytes(Kept::bytes(s, x.element_size()), x);
+        const Kept kept(p.codes, s, x.element_size());
+        PM_CALL(planmoe_layer_combine_keep(p.ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), kept.codes,
+                                           kept.bias, kept.scale, st));
         p.ye = Tensor();
         return p;
     }
@@ -186,7 +193,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         const Shape s = shape_of(x, wg, w1, k, cap);
         Pass p = forward_pass(x, wg, w1, b1, w2, b2, s, fp32_gate, normalize, (int)codec, true);
         ctx->save_for_backward({x, wg, w1, w2, p.scores, p.gates, p.indices, p.locations, p.counts, p.xe, p.h,
-                                codec == CODEC_ZFP ? p.stream : codec == CODEC_INT8 ? p.codes : p.ye, p.ranges});
+                                codec == CODEC_ZFP ? p.stream : codec == CODEC_INT8 ? p.codes : p.ye});
         ctx->saved_data["k"] = k;
         ctx->saved_data["cap"] = cap;
         ctx->saved_data["normalize"] = normalize;
@@ -211,7 +218,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         p.counts = saved[8];
         p.xe = saved[9];
         p.h = saved[10];
-        const Tensor &ye = saved[11], &ranges = saved[12];       // (rows; zfp: their stream; int8: their codes)
+        const Tensor &ye = saved[11];                // (the rows; zfp: their stream; int8: their codes)
         const int32_t *idx = ints(p.indices), *loc = ints(p.locations);
         const bool need_x = ctx->needs_input_grad(0), need_gate = ctx->needs_input_grad(1), need_w1 = ctx->needs_input_grad(2),
                    need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
@@ -234,13 +241,14 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                 gye = lz_round_trip(buf, st);
             } else {
                 gye = at::empty({s.rows(), s.M}, x.options());
-                if (codec == CODEC_INT8)
-                    PM_CALL(planmoe_layer_combine_bwd_codes(grad.data_ptr(), ye.data_ptr<uint8_t>(), ranges.data_ptr(), second_half(ranges), s.dt,
-                                                            floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, gye.data_ptr(),
-                                                            grad_gates.data_ptr<float>(), st));
-                else
+                if (codec == CODEC_INT8) {
+                    const Kept kept(ye, s, x.element_size());
+                    PM_CALL(planmoe_layer_combine_bwd_codes(grad.data_ptr(), kept.codes, kept.bias, kept.scale, s.dt, floats(gates), idx, loc, s.T, s.k,
+                                                            s.T, s.M, s.E, s.cap, gye.data_ptr(), grad_gates.data_ptr<float>(), st));
+                } else {
                     PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, 0, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
                                                       gye.data_ptr(), grad_gates.data_ptr<float>(), st));
+                }
             }
             auto colsum = [&](const Tensor &a, int cols) {
                 Tensor out = at::empty({s.E, cols}, x.options()), ws = bytes((int64_t)planmoe_rows_colsum_workspace_bytes(s.E, s.cap, cols), x);
