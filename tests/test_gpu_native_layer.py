@@ -340,3 +340,28 @@ def test_int8_training_holds_no_more_than_its_steps():
         native, steps = held(True, dtype), held(False, dtype)
         print("held", dtype, native, steps, flush=True)
         assert native <= steps + 4096            # (a plane or a scalar that the steps take apart)
+
+
+@pytest.mark.parametrize("codec,dtype", [("no", torch.bfloat16), ("int8", torch.bfloat16), ("no", torch.float32), ("zfp", torch.float32),
+                                         ("lz", torch.float32)])
+def test_native_layer_on_a_stream_of_its_own(codec, dtype):
+    """The forward pass on another stream, behind work that is still running there; the backward pass asked for from the
+    stream that was current before: everything is launched, and its memory used, on the forward pass's stream."""
+    layer = _layer(dtype, codec)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, gy = (torch.randn(300, 64, device=DEV, generator=g).to(dtype) for _ in range(2))
+    want = _pass(layer, x, gy)
+    layer.zero_grad()
+    v, stream = torch.zeros_like(x).requires_grad_(True), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(20_000_000)            # (about 10 ms: what does not wait for the copy below sees other values)
+        with torch.no_grad():
+            v.copy_(x)
+        y = layer(v)
+    y.backward(gy)
+    torch.cuda.current_stream().wait_stream(stream)
+    got = {"y": y.detach(), "dx": v.grad, **{n: p.grad for n, p in layer.named_parameters()}}
+    torch.cuda.synchronize()
+    for name in want:
+        assert torch.equal(want[name], got[name]), name

@@ -114,3 +114,35 @@ def test_index_planes_edited_in_place_are_refused(k):
     assert torch.equal(run(2), want)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         run(1)
+
+
+@pytest.mark.parametrize("postscore", [True, False])
+def test_nodes_on_a_stream_of_their_own(postscore):
+    """The forward pass on another stream, behind work that is still running there; the backward pass asked for from the
+    stream that was current before."""
+    import planmoe_amd as pm
+    g = torch.Generator().manual_seed(9)
+    scores = torch.softmax(torch.randn(300, 6, generator=g), 1).to(DEV)
+    x, gy = torch.randn(300, 40, generator=g).to(DEV), torch.randn(300, 40, generator=g).to(DEV)
+
+    def run(s, v):
+        crit, loss = pm.extract_critical(s, 2, alignment=4)
+        return pm.fast_decode(pm.fast_encode(v, crit, is_postscore=postscore), crit, is_postscore=postscore), loss
+
+    s, v = _fresh(scores, x)
+    y, loss = run(s, v)
+    torch.autograd.backward([y, loss], [gy, torch.full_like(loss, 0.5)])
+    want = [y.detach(), loss.detach(), s.grad, v.grad]
+    s, v, stream = torch.zeros_like(scores).requires_grad_(True), torch.zeros_like(x).requires_grad_(True), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(20_000_000)            # (about 10 ms: what does not wait for the copies below sees other values)
+        with torch.no_grad():
+            s.copy_(scores)
+            v.copy_(x)
+        y, loss = run(s, v)
+    torch.autograd.backward([y, loss], [gy, torch.full_like(loss, 0.5)])
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    for a, b in zip(want, [y.detach(), loss.detach(), s.grad, v.grad]):
+        assert torch.equal(a, b)
