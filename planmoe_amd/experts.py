@@ -4,6 +4,14 @@ backward pass, are planmoe_expert_gemm (hand-written kernels for the matrix core
 either way round; no library GEMM is called); forward_from_codes() takes the int8 codes of the receive
 buffer straight into the first GEMM."""
 import torch
+from torch.autograd import forward_ad
+
+
+def _transformed(*tensors):
+    """Whether a tensor is under vmap, a functional gradient or forward-mode differentiation: a node of autograd with
+    raw pointers behind it cannot follow those."""
+    return any(torch._C._functorch.is_functorch_wrapped_tensor(t) or forward_ad.unpack_dual(t).tangent is not None
+               for t in tensors)
 
 
 def row_fits(length, dtype):
@@ -46,6 +54,14 @@ class _BatchedLinear(torch.autograd.Function):
     def backward(ctx, gy):
         from . import ops
         x, w, y = ctx.saved_tensors
+        if torch.is_grad_enabled() and gy.dtype == torch.float32:
+            # a gradient that is differentiated in turn: the same products where autograd sees them.  (Not in 16 bits: the
+            # library's batched products of that kind are kept away from transposed operands)
+            if ctx.relu:
+                gy = gy * (y > 0)
+            return (torch.matmul(gy, w.transpose(1, 2)) if ctx.needs_input_grad[0] else None,
+                    torch.matmul(x.transpose(1, 2), gy) if ctx.needs_input_grad[1] else None,
+                    gy.sum(dim=1) if ctx.has_bias and ctx.needs_input_grad[2] else None, None)
         if ctx.relu:
             gy = torch.ops.aten.threshold_backward(gy.contiguous(), y, 0.0)      # relu's own backward: one pass over dy and y
         gy = aligned(gy)
@@ -102,7 +118,7 @@ class FusedExpertsNetwork(torch.nn.Module):
     LIBRARY_BATCHED_LIMIT = 1 << 32
 
     def _linear(self, x, w, bias, relu):
-        if _kernel_serves(x, w):
+        if _kernel_serves(x, w) and not (x.dtype == torch.float32 and _transformed(x, w, bias)):
             return _BatchedLinear.apply(x, w, bias, relu)
         if x.is_cuda and x.shape[0] > 1 and x.shape[0] * x.shape[1] * w.shape[1] * w.shape[2] > self.LIBRARY_BATCHED_LIMIT:
             y = torch.stack([torch.addmm(bias[e], x[e], w[e]) for e in range(x.shape[0])])

@@ -316,3 +316,40 @@ def test_layer_with_the_builtin_ffn_at_config2_size():
     with torch.no_grad():
         y2 = layer(x)
     assert torch.allclose(y2.float(), y.detach().float(), rtol=2e-2, atol=2e-2 * float(y.detach().float().abs().max()))
+
+
+def test_fp32_experts_under_transforms_and_twice_differentiated():
+    """The experts alone in fp32: vmap, a functional gradient, forward mode and a gradient of a gradient, as products of the
+    library allow them; against the same in fp64 without the kernels."""
+    import torch.autograd.forward_ad as fw
+    from planmoe_amd.experts import FusedExpertsNetwork
+
+    class Ctx:
+        model_dim, num_local_experts = 16, 3
+
+    torch.manual_seed(0)
+    experts = FusedExpertsNetwork(hidden_size_per_expert=24)
+    experts.update(Ctx)
+    experts = experts.to(DEV)
+    w1, b1, w2, b2 = (p.detach().double() for p in (experts.batched_fc1_w, experts.batched_fc1_bias, experts.batched_fc2_w, experts.batched_fc2_bias))
+
+    def exact(v):
+        return torch.matmul(torch.relu(torch.matmul(v, w1) + b1[:, None]), w2) + b2[:, None]
+
+    def close(a, b):                             # sums of at most 24 products, a few deep
+        assert float((a.double() - b).norm()) <= 1e-5 * float(b.norm())
+
+    x, t = torch.randn(4, 3, 5, 16, device=DEV), torch.randn(3, 5, 16, device=DEV)
+    close(torch.vmap(lambda v: experts(v, Ctx))(x), exact(x.double()))
+    close(torch.func.grad(lambda v: experts(v, Ctx).square().sum())(x[0]), torch.func.grad(lambda v: exact(v).square().sum())(x[0].double()))
+    with fw.dual_level():
+        got = fw.unpack_dual(experts(fw.make_dual(x[0], t), Ctx)).tangent
+        close(got, fw.unpack_dual(exact(fw.make_dual(x[0].double(), t.double()))).tangent)
+
+    def penalty(f, v):
+        v = v.clone().requires_grad_(True)
+        (g,) = torch.autograd.grad(f(v).square().sum(), v, create_graph=True)
+        (h,) = torch.autograd.grad(g.square().sum(), v)
+        return g.detach(), h
+    for a, b in zip(penalty(lambda v: experts(v, Ctx), x[0]), penalty(exact, x[0].double())):
+        close(a, b)
