@@ -114,7 +114,8 @@ __device__ __forceinline__ void table_sync()
 // memory until their values are looked up, vector by vector (two 8 KB rows and their sum in fp32 took 230
 // registers and left two waves per SIMD).  16384 x 4096 bf16, top-2, 403 MB: 81 us = 5.0 TB/s.  More than two
 // choices keep their sum in fp32.  KEEP: the rows' codes, minima and scales are stored as well, by slot (what a backward
-// pass reads in place of the rows: a byte a value to hold between the passes).
+// pass reads in place of the rows: a byte a value to hold between the passes; 16384 x 1024 bf16, top-2: 26.5 -> 32 us, and the
+// backward pass 48 -> 38).
 template <int DT, int CACHE, bool TWO, bool KEEP>
 __global__ __launch_bounds__(256) void layer_combine_kernel(
     const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
@@ -211,6 +212,7 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
 // codec(round(gate_j * grad[t])) (GatingDecoder.backward, fast_dispatch.py:62-79, with the two codec
 // passes around it, overlap.py:19-34).  The rows come as they are (SEEN_ROWS without a codec, SEEN_INT8 with), or as the codes,
 // minima and scales that the forward pass kept (SEEN_CODES): half or a quarter of the bytes, and no codes to work out.
+// 16384 x 1024 bf16, top-2: 48 us from the rows, 38 from the codes (33 MB of the gradient in, 34 of codes, 67 out).
 enum { SEEN_ROWS, SEEN_INT8, SEEN_CODES };
 template <int DT, int CACHE, int SEEN>
 __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
