@@ -445,7 +445,8 @@ int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int 
  * min(sum of its entries rounded up to live_round, m) rows (form 2: that many k) in use; rows of c beyond
  * them are not written, rows of a and b beyond them are not read (up to 64 batches).  rows_hint: the number
  * of rows in use to expect (what the tile is picked by; 0: all).  n, and k (form 2: m), multiples of 8
- * (fp32: 4). */
+ * (fp32: 4); a, b and c 16-byte aligned, 256 of their rows under 2 GiB (how many rows there are has no such
+ * bound). */
 int planmoe_expert_gemm(int form, int dtype, const void *a, const void *b, const void *bias, int activation,
                         int batches, int m, int n, int k, const int32_t *live, int live_planes,
                         int live_round, int rows_hint, void *c, void *stream);
