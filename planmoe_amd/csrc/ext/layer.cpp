@@ -133,7 +133,8 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     }
     const Live live = live_rows(p, s, codec);
     p.h = at::empty({s.rows(), s.H}, x.options());
-    PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
+    // (which elements a relu cut is asked by a backward pass only)
+    PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), keep ? 1 : 2, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
                                 s.hint(), p.h.data_ptr(), st));
     p.ye = at::empty({s.rows(), s.M}, x.options());
     PM_CALL(planmoe_expert_gemm(0, s.dt, p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,

@@ -757,14 +757,14 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
 {
     const char *who = "planmoe_expert_gemm";
     if (expert_gemm_check(who, form, dtype, a, b, batches, m, n, k, live, live_planes, live_round, c)) return 1;
-    PM_REQUIRE(activation == 0 || activation == 1, "%s: activation is 0 (none) or 1 (relu)", who);
+    PM_REQUIRE(activation >= 0 && activation <= 2, "%s: activation is 0 (none), 1 (relu) or 2 (relu without a backward pass)", who);
     PM_REQUIRE(!bias || form != 2, "%s: a weight gradient has no bias", who);
     hipStream_t st = (hipStream_t)stream;
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, (const float *)bias, nullptr, (float *)c, nullptr, live, live_planes, live_round,
                      m, n, k, batches, activation};
         const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
-        return gemm_f32_run(form, p, gemm_f32_tile(form, p, hint), st, who);
+        return gemm_f32_run(form, p, gemm_f32_pick(form, p, hint), st, who);
     }
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n, most = form == 2 ? k : m;
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, live, live_planes,
@@ -796,10 +796,10 @@ extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void
     int tile_rows, slots;
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
-        const int side = gemm_f32_tile(1, p, hint);
-        tile_rows = side ? side : 64;
+        const Gemm32Kernel kernel = gemm_f32_pick(1, p, hint);
+        tile_rows = gemm_f32_slot_rows(kernel);
         slots = (m + tile_rows - 1) / tile_rows * 2;
-        if (gemm_f32_run(1, p, side, st, who)) return 1;
+        if (gemm_f32_run(1, p, kernel, st, who)) return 1;
     } else {
         GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
                    m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};

@@ -10,26 +10,12 @@
 // read four k at a time (16 bytes per lane), sixteen k are two reads, and the sums take them in the order
 // 0 4 8 12, 1 5 9 13, ..: the order of a product made of 16 x 16 x 4 instructions whose lanes read 16 bytes, so what such
 // a product (the fp32 library's) gives, this one gives bit for bit, and a relu behind it cuts the same elements.
-#include "gemm_f32.hpp"
+// (Larger products that no such relu follows are gemm_f32_split.hip's.)
+#include "gemm_f32_core.hpp"
+#include <algorithm>
+#include <cmath>
 
 namespace pm {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t g32_u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int G32_BK = 32;
-
-__device__ __forceinline__ g32_u32x4 g32_desc(const void *base, int64_t bytes)
-{
-    const uint64_t a = (uint64_t)base;
-    const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffff ? 0x7fffffffu : (uint32_t)bytes;
-    return g32_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, n, 0x00020000u};
-}
-__device__ __forceinline__ void g32_dma16(g32_u32x4 desc, uint32_t voff, uint32_t soff, uint32_t lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
-}
 
 // F: 32 x 32 fragments of a wave on a side; the tile is 64 F x 64 F
 template <int F, bool TA, bool TB>
@@ -143,57 +129,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
         }
     }
 
-    const int64_t corner = (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0;
-    const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - m0 - 1) * p.N + (p.N - n0)) * 4);
-    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
-    float sums[F][4][4];
-#pragma unroll
-    for (int j = 0; j < F; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int col = wn * 32 * F + 32 * j + 8 * q + 4 * fc;
-            const bool in_n = n0 + col < p.N;
-            f32x4 add = {0.f, 0.f, 0.f, 0.f};
-            if (p.bias && in_n) {
-#pragma unroll
-                for (int x = 0; x < 4; ++x) add[x] = p.bias[(int64_t)e * p.N + n0 + col + x];
-            }
-#pragma unroll
-            for (int x = 0; x < 4; ++x) sums[j][q][x] = 0.f;
-#pragma unroll
-            for (int i = 0; i < F; ++i) {
-                const int row = wm * 32 * F + 32 * i + fr;
-                f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                if (p.bias) v += add;
-                if (p.relu) {
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = v[x] < 0.f ? 0.f : v[x];
-                }
-                const bool inside = in_n && m0 + row < M;
-                if (p.mask) {
-                    f32x4 k = {0.f, 0.f, 0.f, 0.f};
-                    if (inside) k = *reinterpret_cast<const f32x4 *>(p.mask + corner + (int64_t)row * p.N + col);
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) { v[x] = k[x] > 0.f ? v[x] : 0.f; sums[j][q][x] += inside ? v[x] : 0.f; }
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(pm_u32x4, v), out, in_n ? ((uint32_t)row * (uint32_t)p.N + (uint32_t)col) * 4u : 0x80000000u, 0, 0);
-            }
-        }
-    if (p.colsum) {
-        const int slots = tiles_m * 2;
-        float *to = p.colsum + ((int64_t)e * slots + m0 / G32_B * 2 + wm) * p.N + n0;
-#pragma unroll
-        for (int j = 0; j < F; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-#pragma unroll
-                for (int x = 0; x < 4; ++x)
-#pragma unroll
-                    for (int d = 1; d < 32; d <<= 1) sums[j][q][x] += __shfl_xor(sums[j][q][x], d);
-                const int col = wn * 32 * F + 32 * j + 8 * q + 4 * fc;
-                if (fr == 0 && n0 + col < p.N) *reinterpret_cast<float4 *>(to + col) = make_float4(sums[j][q][0], sums[j][q][1], sums[j][q][2], sums[j][q][3]);
-            }
-    }
+    g32_store<F, F>(p, acc, e, m0, n0, M, wm, wn, m0 / G32_B * 2 + wm, tiles_m * 2);
 }
 
 // Few rows: a wave on its own, 16 MF rows by 16 columns, operands from memory straight into registers
@@ -366,34 +302,69 @@ static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *
 //   8 experts, 128 rows, 1024 -> 4096    even 31, 32 and 43, 42;     64 on one 44, 52 and 42, 42
 //   16 experts, 256 rows, 4096 -> 1024   even 55, 60 and 93, 97;     128 on one 123, 140 and 152, 155
 //   64 experts, 2048 rows, 1024 -> 4096  even 388, 361 and 305, 303; by Zipf's law (1.2) 531, 525 and 918, 912
-int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint)
+//
+// On the bf16 matrix cores, in three parts a value (gemm_f32_split.hip), where there is more than one tile of 64 x 64 for a compute
+// unit; one tile on its own is bound by issuing the splits (8 experts, 128 rows, 1024 -> 1024: 25 us in fp32, 28 in parts) and stays here.
+// A launch takes its rounds; us for a k-tile with few and with all compute units at work, and once for a tile, fitted to 60 shapes
+// (within 7 %): 64 x 64 0.6 alone, 0.44 each of several on a compute unit, + 6; 128 x 128 1.1 - 1.4, + 6; 256 x 128 1.9 - 2.5, + 7.
+//   experts x rows, in, out       fp32 tiles    64     128    256 x 128
+//   16 x 512, 1024, 1024 nn          147        126     102     88
+//   16 x 512, 1024, 1024 tn          133        131     114     98
+//   2 x 4096, 4096, 4096 nt         2005       1727    1434   1259
+//   4 x 1000, 512, 2048 tn            75         66      52     76
+//   8 x 300, 712, 712 nn              30         26      32     50
+// Not under a relu whose backward pass asks which elements it cut: one within rounding of zero that is cut here and kept there
+// changes a weight gradient by 1e-3 of itself at 2^20 elements, so that product keeps the library's order of sums.  Not up to
+// 64 rows, where reading the weight takes as long as the fp32 matrix cores do (16 x 56, 1792 -> 1992 and back: 201 us in fp32, 205 in parts).  And not
+// with rows or columns of less than 256 values, where a product of few rows on waves has the same sums as one of many.
+static Gemm32Kernel gemm_f32_pick_split(int form, const Gemm32Args &p, int rows_hint)
+{
+    const double cu = compute_units(), kt = (double)(((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK);
+    // (row counts from the device: an expectation, and a batch may have a standard deviation more)
+    const int64_t m = form == 2 ? p.M : p.live ? std::min<int64_t>(p.M, rows_hint + (int64_t)std::sqrt((double)rows_hint)) : rows_hint;
+    auto tiles = [&](int64_t bm, int64_t bn) { return (double)((m + bm - 1) / bm * ((p.N + bn - 1) / bn) * p.batches); };
+    auto rounds = [&](double t, double low, double high, double once) {
+        const double full = std::floor(t / cu), rest = t - full * cu;
+        return full * (high * kt + once) + (rest > 0 ? (low + (high - low) * rest / cu) * kt + once : 0.);
+    };
+    const double small = std::ceil(tiles(64, 64) / cu), t64 = (small <= 1 ? 0.6 : 0.44 * small) * kt + 6;
+    const double t128 = rounds(tiles(128, 128), 1.1, 1.4, 6), t256 = rounds(tiles(256, 128), 1.9, 2.5, 7);
+    if (t64 <= t128 && t64 <= t256) return small <= 1 ? G32_TILE_64 : G32_SPLIT_64;
+    return t128 <= t256 ? G32_SPLIT_128 : G32_SPLIT_256;
+}
+
+Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
 {
     if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
         gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
-        return 0;
+        return G32_WAVES;
+    if (p.relu != 1 && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
     auto cost = [&](int64_t side, double us) {
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
         return (double)((tiles + cu - 1) / cu) * (us * kt + 2);
     };
-    return cost(64, 0.47) < cost(128, 1.7) ? 64 : 128;
+    return cost(64, 0.47) < cost(128, 1.7) ? G32_TILE_64 : G32_TILE_128;
 }
 
-int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who)
+int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who)
 {
-    if (side == 0) {
+    switch (kernel) {
+    case G32_WAVES:
         if (p.M <= 16 && !p.colsum) return form == 0 ? gemm_f32_wave_launch<1, 16, true>(p, stream, who) : gemm_f32_wave_launch<1, 8, false>(p, stream, who);
         return form == 0 ? gemm_f32_wave_launch<2, 8, true>(p, stream, who) : gemm_f32_wave_launch<2, 4, false>(p, stream, who);
-    }
-    if (side == 64) {
+    case G32_TILE_64:
         if (form == 0) return gemm_f32_launch<1, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<1, false, false>(p, stream, who);
         return gemm_f32_launch<1, true, true>(p, stream, who);
+    case G32_TILE_128:
+        if (form == 0) return gemm_f32_launch<2, false, true>(p, stream, who);
+        if (form == 1) return gemm_f32_launch<2, false, false>(p, stream, who);
+        return gemm_f32_launch<2, true, true>(p, stream, who);
+    default:
+        return gemm_f32_split_run(form, p, kernel, stream, who);
     }
-    if (form == 0) return gemm_f32_launch<2, false, true>(p, stream, who);
-    if (form == 1) return gemm_f32_launch<2, false, false>(p, stream, who);
-    return gemm_f32_launch<2, true, true>(p, stream, who);
 }
 
 } // namespace pm

@@ -9,12 +9,19 @@ struct Gemm32Args {
     float *C, *colsum;                     // colsum: [batches][2 tile rows][N] column sums of what was stored, NULL: none
     const int *live;                       // [live_planes][batches]: rows in use (k of a tn product), NULL: all
     int live_planes, live_round;
-    int M, N, K, batches, relu;            // operands and result contiguous
+    int M, N, K, batches;                  // operands and result contiguous
+    int relu;                              // 1; 2: and no backward pass asks which elements it cut
 };
 
-// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  side: rows and columns of a tile, 64 or 128, or 0:
-// no tiles, waves on their own (gemm_f32_tile picks it for a number of rows in use); column sums then have two slots for 64 rows
-int gemm_f32_tile(int form, const Gemm32Args &p, int rows_hint);
-int gemm_f32_run(int form, const Gemm32Args &p, int side, hipStream_t stream, const char *who);
+// Kernels: waves on their own; tiles of 64 x 64 and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128
+// on the bf16 matrix cores, the operands in three parts
+enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_TILE_128, G32_SPLIT_64, G32_SPLIT_128, G32_SPLIT_256 };
+
+// form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  rows_hint: rows in use
+Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint);
+int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who);
+int gemm_f32_split_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who);
+// column sums have two slots for so many rows
+inline int gemm_f32_slot_rows(Gemm32Kernel kernel) { return kernel == G32_TILE_128 || kernel == G32_SPLIT_128 || kernel == G32_SPLIT_256 ? 128 : 64; }
 
 } // namespace pm

@@ -309,3 +309,73 @@ def test_expert_gemm_fp32_few_rows_expected_and_many_there(B, cap, n, k, counted
         assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all()), e
         stored = masked[e, :r]
         assert bool(((db[e] - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all()), e
+
+
+def _fp64(form, a, b):
+    a, b = a.double(), b.double()
+    a, b = (a.transpose(1, 2).contiguous() if form == "tn" else a), (b.transpose(1, 2).contiguous() if form == "nt" else b)
+    return a @ b, a.abs() @ b.abs()
+
+
+# fp32 on the bf16 matrix cores in three parts a value: one shape for each tile (64, 128 and 256 rows; 256 compute units pick
+# them by the number of tiles), rows, columns and reductions that are no multiple of anything but 4, one past a tile and one
+# k-tile's edge.  A k-slow operand's rows need not be a multiple of 4.
+@pytest.mark.parametrize("form,B,m,n,k", [("nn", 8, 301, 712, 712), ("nt", 8, 299, 708, 700), ("tn", 8, 712, 716, 301), ("nn", 4, 999, 1004, 300),
+                                          ("nt", 4, 1000, 1004, 292), ("tn", 4, 516, 2048, 1001), ("nn", 4, 2041, 1004, 260), ("nt", 16, 257, 1036, 1028),
+                                          ("tn", 8, 1028, 1004, 129), ("tn", 8, 1028, 1024, 1)])
+def test_expert_gemm_fp32_in_parts(form, B, m, n, k):
+    from planmoe_amd import ops
+    print("case", form, B, m, n, k, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = torch.randn(*((B, k, m) if form == "tn" else (B, m, k)), device=DEV, generator=g)
+    b = torch.randn(*((B, n, k) if form == "nt" else (B, k, n)), device=DEV, generator=g)
+    got, (ref, mag) = ops.expert_gemm(form, a, b), _fp64(form, a, b)
+    # six products of parts leave 2^-26 of a product out and are six sums for 16 k: inside the bound of k fp32 products and sums
+    assert bool(((got.double() - ref).abs() <= _bound(ref, mag, k, torch.float32)).all())
+    # parts of the smallest values are no subnormal bf16 values; sums that the scaled parts overflow are made again
+    for scale_a, scale_b in ((2.0 ** -126, 1.0), (2.0 ** -63, 2.0 ** -62), (2.0 ** 100, 2.0 ** -100), (2.0 ** 60, 2.0 ** 55), (2.0 ** 125, 2.0 ** -120)):
+        got, (ref, mag) = ops.expert_gemm(form, a * scale_a, b * scale_b), _fp64(form, a * scale_a, b * scale_b)
+        # (a result below the normal range is rounded to 2^-149 in every sum)
+        assert bool(((got.double() - ref).abs() <= _bound(ref, mag, k, torch.float32) - 1e-30 + (k + 2) * 2.0 ** -149).all()), (scale_a, scale_b)
+    # infinities and NaN reach the results they belong to and no others
+    a[0, 0, 7], a[B - 1, 0, 1] = float("inf"), float("nan")
+    if k > 3:
+        b[0, 2, 3], b[B - 1, 3, 2] = float("-inf"), 3.4e38
+    got, (ref, mag) = ops.expert_gemm(form, a, b), _fp64(form, a, b)
+    torch.cuda.synchronize()
+    finite = ref.abs() < 3.4028235e38
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[got.isinf()], ref[got.isinf()].float()) and bool(got[finite].isfinite().all())
+    assert bool(((got.double() - ref).abs()[finite] <= _bound(ref, mag, k, torch.float32)[finite]).all())
+
+
+# the same with row counts: batches without rows and with a capacity's, rows beyond those in use hold NaN; the masked product and its sums
+@pytest.mark.parametrize("B,cap,n,k,hint", [(16, 520, 1036, 1028, 500), (8, 320, 712, 716, 290), (4, 1100, 1004, 300, 980)])
+def test_expert_gemm_fp32_in_parts_takes_the_rows_in_use_only(B, cap, n, k, hint):
+    from planmoe_amd import ops
+    print("case", B, cap, n, k, hint, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(B + cap)
+    counts = [0, cap, 1, hint] + [cap // 2 + 7 * e for e in range(4, B)]
+    live = torch.tensor([counts], dtype=torch.int32, device=DEV)
+    a, dy = torch.randn(B, cap, k, device=DEV, generator=g), torch.randn(B, cap, n, device=DEV, generator=g)
+    w, bias, h = torch.randn(B, k, n, device=DEV, generator=g), torch.randn(B, n, device=DEV, generator=g), torch.randn(B, cap, n, device=DEV, generator=g).clamp(min=0)
+    rows = [min(cap, c) for c in counts]
+    for e, r in enumerate(rows):
+        a[e, r:] = dy[e, r:] = float("nan")
+    nn = torch.full((B, cap, n), 7.0, device=DEV)
+    masked = nn.clone()
+    kw = dict(live=live, rows_hint=hint)
+    ops.expert_gemm("nn", a, w, bias, out=nn, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, w.transpose(1, 2).contiguous(), h, out=masked, **kw)
+    dw = ops.expert_gemm("tn", a, dy, **kw)
+    torch.cuda.synchronize()
+    for e, r in enumerate(rows):
+        x, wd = a[e, :r].double(), w[e].double()
+        ref, mag = x @ wd, x.abs() @ wd.abs()
+        tol, biased = _bound(ref, mag, k, torch.float32), ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - biased).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, torch.float32)).all()), e
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all()), e
+        assert bool((nn[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all()), e
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all()), e
+        d = dy[e, :r].double()
+        assert bool(((dw[e].double() - x.t() @ d).abs() <= _bound(d, x.abs().t() @ d.abs(), cap, torch.float32)).all()), e
