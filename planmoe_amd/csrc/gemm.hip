@@ -13,6 +13,7 @@
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
 #include "gemm_skinny.hpp"
+#include <algorithm>
 #include <cmath>
 
 namespace pm {
@@ -36,9 +37,9 @@ __device__ __forceinline__ gemm_bf16x8 gemm_read_tr(gemm_lds_ptr lo, gemm_lds_pt
 }
 
 // ---------------------------------------------------------------- the kernel
-// Tiles of 256 x 256 (or 128 on a side), k-tiles of 64, four waves.  Each side of a tile is two halves;
-// a wave has 32 I rows of either A half and 32 J columns of either B half, so its share of the tile is
-// four quadrants and a k-tile is four phases, one quadrant each: 4 I J v_mfma_f32_32x32x16_bf16.
+// Tiles of 256 x 256 (128 x 128; 128, 160 or 192 x 256), k-tiles of 64, four waves, two by two (or side by side, each with
+// all rows).  Each side of a tile is two halves; a wave has 32 I rows of an A half and 32 J columns of either B half, so
+// its share of the tile is four quadrants and a k-tile is four phases, one quadrant each: 4 I J v_mfma_f32_32x32x16_bf16.
 // During a phase the wave reads from LDS the one half of an operand that the next phase needs and has
 // not got (the quadrants of successive k-tiles are walked so that this is always one half), and asks
 // for one half of a k-tile two further on, straight into LDS (buffer_load ... lds), into the space
@@ -67,7 +68,7 @@ struct GemmArgs {
     const uint16_t *A, *B, *bias;
     const uint16_t *mask;         // GRAD: c is kept where mask > 0 (c's shape and pitches), else zero
     uint16_t *C;
-    float *colsum;                // GRAD: [batches][2 ceil(M / 128)][N] column sums of what was stored, by 128 rows and wave row, NULL: none
+    float *colsum;                // GRAD: [batches][slots][N] column sums of what was stored, NULL: none; a slot for 128 rows and wave row (one wave row: a tile)
     const int *live;              // [live_planes][batches]: rows in use per batch (k of a tn product), NULL: all
     int live_planes, live_round;
     int M, N, K;
@@ -102,51 +103,62 @@ template <int N> __device__ __forceinline__ void gemm_phase_wait()
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
-// I, J: a tile is 128 I rows by 128 J columns
-template <int I, int J>
+// WM x 4 / WM waves; in the halves of A a wave has I0 and I1 fragments of 32 rows, in those of B J fragments each of 32 columns
+template <int WM_, int I0, int I1, int J_>
 struct GemmShape {
-    static constexpr int BM = 128 * I, BN = 128 * J;
+    static constexpr int WM = WM_, WN = 4 / WM_, J = J_;
+    static constexpr int I(int h) { return h ? I1 : I0; }
+    static constexpr int IMAX = I0 > I1 ? I0 : I1;
+    static constexpr int BM = 32 * WM * (I0 + I1), BN = 64 * WN * J;
+    static constexpr int half(int o, int h) { return o == 0 ? 32 * WM * I(h) : 32 * WN * J; }        // rows (columns) of a half
     // LDS: both stages of A, both stages of B (so that an operand's halves are all within the 64 KB that an
     // LDS instruction's offset covers), the waves' output pieces (32 rows of 32 J values each), tables
     static constexpr int half_at(int o, int stage, int h)
     {
-        return o == 0 ? (2 * stage + h) * 8192 * I : 4 * 8192 * I + (2 * stage + h) * 8192 * J;
+        return o == 0 ? stage * BM * 128 + h * half(0, 0) * 128 : 2 * BM * 128 + (2 * stage + h) * half(1, 0) * 128;
     }
-    static constexpr int OPERANDS = 4 * 8192 * (I + J);
+    static constexpr int OPERANDS = 256 * (BM + BN);
     static constexpr int PITCH = 64 * J + 16;               // bytes between rows of an output piece
     static constexpr int TABLE = OPERANDS + 4 * 32 * PITCH, BIAS = TABLE + GEMM_TABLE_BYTES;
     static constexpr int LDS = BIAS + GEMM_BIAS_BYTES;
-    static constexpr int STORES = 8 * I * J;                // 16-byte stores of a lane per tile
-    // loads a wave issues in phase p, and how many of them may be outstanding at its end: the half that
-    // phase p + 1 reads was asked for six phases before p, what is younger is not needed yet
-    static constexpr int loads(int p) { return (p & 3) < 2 ? 2 * J : 2 * I; }
+    static constexpr int STORES = 2 * (I0 + I1) * 2 * J;    // 16-byte stores of a lane per tile
+    // loads a wave issues in phase p (the halves B B A1 A0), and how many of them may be outstanding at its end: the half that
+    // phase p + 1 reads was asked for six phases before p, what is younger is not needed yet.  One wave row reads
+    // the first pieces of A1 a phase ahead of the others (EARLY of them, with A's fragments read by all four waves a
+    // phase would otherwise have more LDS reads than the products of a phase cover), so that half is there a phase earlier.
+    static constexpr int EARLY = WM == 1 ? 4 * (I1 - 2) : 0;
+    static constexpr int half_loads(int o, int h) { return half(o, h) / 32; }
+    static constexpr int loads(int p) { return (p & 3) < 2 ? half_loads(1, 0) : half_loads(0, (p & 3) == 2); }
     static constexpr int wait(int p)
     {
         int s = 0;
-        for (int j = 0; j < 6; ++j) s += loads(p - j + 8);
+        for (int j = 0; j < (EARLY > 0 && (p & 3) == 3 ? 5 : 6); ++j) s += loads(p - j + 8);
         return s;
     }
     static_assert(wait(3) + STORES < 64 && wait(1) + STORES < 64, "the counter of outstanding loads and stores has six bits");
     static constexpr int WAVES_PER_SIMD = LDS * 2 <= 160 * 1024 ? 2 : 1;     // (= work-groups per compute unit)
 };
+typedef GemmShape<2, 2, 2, 2> Gemm256;        // 256 x 256
+typedef GemmShape<2, 1, 1, 1> Gemm128;        // 128 x 128
+template <int I0, int I1> using GemmFlat = GemmShape<1, I0, I1, 1>;        // 32 (I0 + I1) x 256
 
-template <int I, int J, bool TA, bool TB, bool GRAD>
-__global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void gemm_bf16_kernel(const GemmArgs p)
+template <class S, bool TA, bool TB, bool GRAD>
+__global__ __launch_bounds__(GEMM_WG, S::WAVES_PER_SIMD) void gemm_bf16_kernel(const GemmArgs p)
 {
-    using S = GemmShape<I, J>;
+    constexpr int J = S::J;
+    static_assert(!TA || S::WM == 2, "a k-slow A: two wave rows");
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / S::WN, wn = wave % S::WN;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
 
     // ---- the tiles: work-groups go to the 8 XCDs in turn, each XCD (with an L2 of its own) takes an
     // eighth of the tiles in a row, in the order batch, panel of 8 tile columns, tile row, column, so
     // that the tiles it works on at a time share operands (12 operand tiles for 32 products at 256 x 256).
     // With `live` the tiles of a batch are those of its rows in use: table[e] is the number before batch e.
-    static_assert(I == J, "square tiles");
-    const int side = p.split == 2 ? 256 : S::BM;            // (of the tiles that are counted)
-    const int tiles_n = (p.N + side - 1) / side;
+    const int side = p.split == 2 ? 256 : S::BM, side_n = p.split == 2 ? 256 : S::BN;        // (of the tiles that are counted)
+    const int tiles_n = (p.N + side_n - 1) / side_n;
     int total, base = 0;
     int *table = reinterpret_cast<int *>(lds + S::TABLE);
     if (p.live) {
@@ -198,7 +210,7 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         in -= panel * tm * 8;
         const int width = min(8, tiles_n - panel * 8);
         w.m0 = in / width * side + (p.split == 2 ? (number & 2) * 64 : 0);
-        w.n0 = (panel * 8 + in % width) * side + (p.split == 2 ? (number & 1) * 128 : 0);
+        w.n0 = (panel * 8 + in % width) * side_n + (p.split == 2 ? (number & 1) * 128 : 0);
         return w;
     };
     auto in_range = [&](int j) { return j < per_xcd && first_tile + j < total; };
@@ -227,91 +239,100 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         if (--c.real <= 0) c.ra = c.rb = 0;
     };
 
-    // ---- which 16 bytes of a half a lane fetches.  k fast: 64 X rows of 128 bytes, a load fills eight of
+    // ---- which 16 bytes of a half a lane fetches.  k fast: rows of 128 bytes, a load fills eight of
     // them, chunk c of row r lies at unit c ^ (r >> 1) & 7 (the 16 rows that one pass of a fragment read
     // touches then lie two by two in the halves of the LDS's 256 bytes, at eight different units).  k slow:
-    // 64 rows of 128 X bytes, chunk c of row k at unit c ^ (k & 3) << 2 (128-byte rows: c ^ (k >> 1 & 1) << 2),
-    // so that the 4 rows of a transposing read's patch lie in different quarters of the 256 bytes.
+    // 64 rows of 128 X bytes (64 X rows or columns a half), chunk c of row k at unit c ^ (k & 3) << 2 (128-byte rows:
+    // c ^ (k >> 1 & 1) << 2), so that the 4 rows of a transposing read's patch lie in different quarters of the 256 bytes.
     // Load i of a half: k fast, rows 8 i on (the swizzle turns with the parity of i); k slow, rows 8 / X i on.
-    auto fetch = [&](bool T, int X, int i, int ld) -> uint32_t {
+    auto fetch = [&](bool T, int half, int i, int ld) -> uint32_t {
         if (T) {
-            const int kr = 16 * wave + lane / (8 * X), u = lane % (8 * X);
+            const int X = half / 64, kr = 16 * wave + lane / (8 * X), u = lane % (8 * X);
             return (uint32_t)kr * (uint32_t)ld * 2u + (uint32_t)(X == 2 ? u ^ ((kr & 3) << 2) : u ^ (((kr >> 1) & 1) << 2)) * 16u;
         }
-        const int row = 16 * X * wave + 8 * i + (lane >> 3);
+        const int row = half / 4 * wave + 8 * i + (lane >> 3);
         return (uint32_t)row * (uint32_t)ld * 2u + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
     };
-    uint32_t va[2], vb[2];
-    va[0] = fetch(TA, I, 0, p.lda); va[1] = TA ? va[0] : fetch(TA, I, 1, p.lda);
-    vb[0] = fetch(TB, J, 0, p.ldb); vb[1] = TB ? vb[0] : fetch(TB, J, 1, p.ldb);
+    uint32_t va[2][2], vb[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) { va[h][0] = fetch(TA, S::half(0, h), 0, p.lda); va[h][1] = TA ? va[h][0] : fetch(TA, S::half(0, h), 1, p.lda); }
+    vb[0] = fetch(TB, S::half(1, 0), 0, p.ldb); vb[1] = TB ? vb[0] : fetch(TB, S::half(1, 0), 1, p.ldb);
     // a reduction length that is no multiple of 64: the chunks of a k-fast row past its end are asked for
-    // out of range in a tile's last k-tile.  Chunk of a lane in load i: (lane & 7) ^ (4 i + (lane >> 4) & 7)
+    // out of range in a tile's last k-tile.  Chunk of a lane in load i: (lane & 7) ^ (4 (n + i) + (lane >> 4) & 7), n the
+    // eights of rows of the half that lie before this wave's
     const int k_tail = TA || p.K % GEMM_BK == 0 ? GEMM_BK : p.K % GEMM_BK;      // (tn: both operands are k-slow)
     auto past = [&](int i) -> uint32_t {
         return (int)(((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 8) >= k_tail ? GEMM_NOWHERE : 0u;
     };
-    const uint32_t past0 = past(0), past1 = past(1);
+    const uint32_t past0 = past(0), past1 = past(1);      // (n + i even, odd)
     auto load = [&](int stage, int o, int h, int i, const Cursor &c) {
-        const int X = o == 0 ? I : J;
+        const int half = S::half(o, h), each = S::half_loads(o, h), X = half / 64;
         const bool T = o == 0 ? TA : TB;
-        const uint32_t dst = lds0 + S::half_at(o, stage, h) + wave * (2048 * X) + i * 1024;
-        const uint32_t ld = (uint32_t)(o == 0 ? p.lda : p.ldb), first = h ? 64u * X : 0u;
-        const uint32_t soff = T ? ld * 2u * (uint32_t)(8 / X * i) + first * 2u : ld * 2u * ((uint32_t)(8 * (i & ~1)) + first);
-        uint32_t v = o == 0 ? va[i & 1] : vb[i & 1];
-        if (!T && k_tail != GEMM_BK) v |= c.real == 1 ? ((i & 1) ? past1 : past0) : 0u;
+        const uint32_t dst = lds0 + S::half_at(o, stage, h) + wave * (each * 1024) + i * 1024;
+        const uint32_t ld = (uint32_t)(o == 0 ? p.lda : p.ldb), first = h ? (uint32_t)S::half(o, 0) : 0u;
+        const uint32_t soff = T ? ld * 2u * (uint32_t)(8 / (X > 0 ? X : 1) * i) + first * 2u : ld * 2u * ((uint32_t)(8 * (i & ~1)) + first);
+        uint32_t v = o == 0 ? va[h][i & 1] : vb[i & 1];
+        if (!T && k_tail != GEMM_BK) v |= c.real == 1 ? (((each & wave) + i) & 1 ? past1 : past0) : 0u;
         gemm_dma16(o == 0 ? gemm_desc(c.a, c.ra) : gemm_desc(c.b, c.rb), v, soff, dst);
     };
 
     // ---- fragments: 32 rows (columns) x 16 k; lane = row l % 32, k-chunk l / 32.  Where a lane's piece of the
     // first fragment of a half lies: k fast, one place for each of the four steps (the swizzle); k slow, one
     // for each fragment of the half
-    gemm_bf16x8 fa[2][I][4], fb[2][J][4];
+    gemm_bf16x8 fa[2][S::IMAX][4], fb[2][J][4];
     const int fr = lane & 31, fc = lane >> 5, tg = lane >> 4, ts = lane & 15;
-    uint32_t ra[4], rb[4];
-    auto place = [&](bool T, int X, int n, int w) -> uint32_t {
+    uint32_t ra[2][4], rb[4];                     // (A: by half, where the waves' shares differ)
+    auto place = [&](bool T, int X, int share, int n, int w) -> uint32_t {        // share: fragments of a wave in the half
         if (T) {
             // lane = (group of 16 lanes, s): k row 8 (g / 2) + s / 4 of the step's 16, 8 bytes s % 4 of the 32 that columns
             // 16 (g % 2) .. + 15 of the fragment take
-            const int row = 8 * (tg >> 1) + (ts >> 2), c = 4 * X * w + 4 * n + 2 * (tg & 1) + ((ts & 3) >> 1);
+            const int row = 8 * (tg >> 1) + (ts >> 2), c = 4 * share * w + 4 * n + 2 * (tg & 1) + ((ts & 3) >> 1);
             const int u = X == 2 ? c ^ ((ts >> 2) << 2) : c ^ ((ts >> 3) << 2);
             return row * (128 * X) + u * 16 + 8 * (ts & 1);
         }
-        return (32 * X * w + fr) * 128 + (((2 * n + fc) ^ ((fr >> 1) & 7)) * 16);
+        return (32 * share * w + fr) * 128 + (((2 * n + fc) ^ ((fr >> 1) & 7)) * 16);
     };
 #pragma unroll
-    for (int n = 0; n < (TA ? I : 4); ++n) ra[n] = lds0 + place(TA, I, n, wm);
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int n = 0; n < (TB ? J : 4); ++n) rb[n] = lds0 + S::half_at(1, 0, 0) + place(TB, J, n, wn);
+        for (int n = 0; n < (TA ? S::I(h) : 4); ++n) ra[h][n] = lds0 + place(TA, S::half(0, h) / 64, S::I(h), n, wm);
+#pragma unroll
+    for (int n = 0; n < (TB ? J : 4); ++n) rb[n] = lds0 + S::half_at(1, 0, 0) + place(TB, S::half(1, 0) / 64, J, n, wn);
     auto read = [&](int stage, int o, int h, int r) {
-        const int X = o == 0 ? I : J, ks = r / X, i = r % X;
+        const int share = o == 0 ? S::I(h) : J, X = S::half(o, h) / 64, ks = r / share, i = r % share;
         const uint32_t at = (uint32_t)(S::half_at(o, stage, h) - S::half_at(o, 0, 0));
         gemm_bf16x8 f;
         if (o == 0 ? TA : TB) {
-            const gemm_lds_ptr q = (gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[i] : rb[i]) + at + ks * (16 * 128 * X);
+            const gemm_lds_ptr q = (gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[h][i] : rb[i]) + at + ks * (16 * 128 * X);
             f = gemm_read_tr(q, q + 4 * 128 * X);
         } else {
-            f = *(const gemm_bf16x8 __attribute__((address_space(3))) *)((gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[ks] : rb[ks]) + at + i * 4096);
+            f = *(const gemm_bf16x8 __attribute__((address_space(3))) *)((gemm_lds_ptr)(uintptr_t)(o == 0 ? ra[h][ks] : rb[ks]) + at + i * 4096);
         }
         if (o == 0) fa[h][i][ks] = f; else fb[h][i][ks] = f;
     };
 
-    f32x16 acc[2][2][I][J];
+    f32x16 acc[2][2][S::IMAX][J];
     int fresh = 0;                                // the stores of the tile before have just gone out
 
     // one phase: quadrant (qa, qb); read half (ro, rh) of stage rs; ask for half (lo, lh) into stage lst
     // (the second operand first in the MFMA: a lane then holds four consecutive columns of one row)
-#define PM_PHASE(P, qa, qb, rs, ro, rh, lst, lo, lh, cur)                                                            \
+    // (r0, r1: which of the half's fragments, x0 of half (xo, xh) of the stage on top)
+#define PM_PHASE(P, qa, qb, rs, ro, rh, r0, xs, xn, lst, lo, lh, cur)                                                \
     do {                                                                                                             \
-        constexpr int n_ = 4 * I * J, half_ = n_ / 2, reads_ = 4 * ((ro) == 0 ? I : J), loads_ = S::loads(P);         \
+        constexpr int share_ = S::I(qa), n_ = 4 * share_ * J, half_ = n_ / 2;                                         \
+        constexpr int own_ = 4 * ((ro) == 0 ? S::I(rh) : J) - (r0), reads_ = own_ + (xn), loads_ = S::loads(P);       \
         constexpr int rper_ = (reads_ + half_ - 1) / half_, lper_ = (loads_ + half_ - 1) / half_;                     \
         constexpr int lgap_ = half_ / loads_ > 0 ? half_ / loads_ : 1;                                               \
         _Pragma("unroll") for (int s_ = 0; s_ < n_; ++s_) {                                                          \
-            const int ks_ = s_ / (I * J), i_ = s_ / J % I, j_ = s_ % J;                                              \
+            const int ks_ = s_ / (share_ * J), i_ = s_ / J % share_, j_ = s_ % J;                                    \
             acc[qa][qb][i_][j_] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[qb][j_][ks_], fa[qa][i_][ks_], acc[qa][qb][i_][j_], 0, 0, 0); \
             __builtin_amdgcn_sched_barrier(0);                                                                       \
             if (s_ < half_) {                                                                                        \
-                _Pragma("unroll") for (int x_ = 0; x_ < rper_; ++x_)                                                 \
-                    if (s_ * rper_ + x_ < reads_) read(rs, ro, rh, s_ * rper_ + x_);                                 \
+                _Pragma("unroll") for (int x_ = 0; x_ < rper_; ++x_) {                                               \
+                    const int r_ = s_ * rper_ + x_;                                                                  \
+                    if (r_ < own_) read(rs, ro, rh, (r0) + r_);                                                      \
+                    else if (r_ < reads_) read(xs, 0, 1, r_ - own_);                                                 \
+                }                                                                                                    \
                 __builtin_amdgcn_sched_barrier(0);                                                                   \
             } else if ((s_ - half_) % lgap_ == 0) {                                                                  \
                 _Pragma("unroll") for (int x_ = 0; x_ < lper_; ++x_) {                                               \
@@ -340,31 +361,26 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
     c1 = c0; advance(c1);
     c2 = c1; advance(c2);
     c3 = c2; advance(c3);
+    auto ask = [&](int stage, int o, int h, const Cursor &c) {
 #pragma unroll
-    for (int i = 0; i < 2 * I; ++i) load(0, 0, 0, i, c0);
+        for (int i = 0; i < S::half_loads(o, h); ++i) load(stage, o, h, i, c);
+    };
+    ask(0, 0, 0, c0);
+    ask(0, 1, 0, c0);
+    ask(0, 1, 1, c0);
+    ask(0, 0, 1, c0);
+    ask(1, 0, 0, c1);
+    ask(1, 1, 1, c1);
+    ask(1, 1, 0, c1);
+    ask(1, 0, 1, c1);
+    gemm_phase_wait<3 * S::half_loads(1, 0) + 2 * S::half_loads(0, 1) + S::half_loads(0, 0)>();
 #pragma unroll
-    for (int i = 0; i < 2 * J; ++i) load(0, 1, 0, i, c0);
-#pragma unroll
-    for (int i = 0; i < 2 * J; ++i) load(0, 1, 1, i, c0);
-#pragma unroll
-    for (int i = 0; i < 2 * I; ++i) load(0, 0, 1, i, c0);
-#pragma unroll
-    for (int i = 0; i < 2 * I; ++i) load(1, 0, 0, i, c1);
-#pragma unroll
-    for (int i = 0; i < 2 * J; ++i) load(1, 1, 1, i, c1);
-#pragma unroll
-    for (int i = 0; i < 2 * J; ++i) load(1, 1, 0, i, c1);
-#pragma unroll
-    for (int i = 0; i < 2 * I; ++i) load(1, 0, 1, i, c1);
-    gemm_phase_wait<6 * (I + J)>();
-#pragma unroll
-    for (int r = 0; r < 4 * I; ++r) read(0, 0, 0, r);
+    for (int r = 0; r < 4 * S::I(0); ++r) read(0, 0, 0, r);
 #pragma unroll
     for (int r = 0; r < 4 * J; ++r) read(0, 1, 0, r);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < 2 * I; ++i) load(0, 0, 0, i, c2);
+    ask(0, 0, 0, c2);
     gemm_phase_wait<S::wait(7)>();
     __builtin_amdgcn_sched_barrier(0);
 
@@ -387,7 +403,8 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         uint8_t *lay = piece + (l & 31) * S::PITCH + (l >> 5) * 8;
         // where a lane's 16-byte pieces go, from the tile's corner; the uniform part of a piece's place is the store's scalar offset
         const int put_col = wn * 32 * J + l % (4 * J) * 8;
-        const uint32_t put = ((uint32_t)(wm * 32 * I + l / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
+        const uint32_t put = ((uint32_t)(l / (4 * J)) * (uint32_t)p.ldc + (uint32_t)put_col) * 2u;
+        auto row_of = [&](int a, int i) { return S::half(0, 0) * a + 32 * (S::I(a) * wm + i); };      // first row of a wave's fragment in the tile
         const int M = TA ? p.M : here.rows;
         const int64_t corner = (int64_t)here.e * p.sC + (int64_t)here.m0 * p.ldc + here.n0;
         const int bytes = (int)max((int64_t)0, min((int64_t)0x7fffffff, ((int64_t)(M - here.m0 - 1) * p.ldc + (p.N - here.n0)) * 2));
@@ -396,35 +413,36 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
         // GRAD: a piece's masks are asked for while the piece before is worked on and ahead of its stores (asked for when
         // they were wanted, each piece waited for memory and for the stores before it: 337 us at 8 x 4096 x 4096 x 1024)
         pm_u32x4 keep[2][2 * J];
+        constexpr int PIECES = S::I(0) + S::I(1);
         auto ask = [&](int n) {                   // piece n: half b of the columns, half a of the rows, fragment i
-            const int b = n / (2 * I), a = n / I % 2, i = n % I;
-            const uint32_t at = here.n0 + 64 * J * b + put_col < p.N ? put : GEMM_NOWHERE;
+            const int b = n / PIECES, a = n % PIECES >= S::I(0), i = n % PIECES - a * S::I(0);
+            const uint32_t at = here.n0 + S::half(1, 0) * b + put_col < p.N ? put : GEMM_NOWHERE;
 #pragma unroll
             for (int t = 0; t < 2 * J; ++t)
-                keep[n & 1][t] = __builtin_amdgcn_raw_buffer_load_b128(mask, at, ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u, 0);
+                keep[n & 1][t] = __builtin_amdgcn_raw_buffer_load_b128(mask, at, ((uint32_t)(row_of(a, i) + 16 / J * t) * (uint32_t)p.ldc + S::half(1, 0) * b) * 2u, 0);
         };
         if (GRAD) ask(0);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const uint32_t put_b = here.n0 + 64 * J * b + put_col < p.N ? put : GEMM_NOWHERE;
+            const uint32_t put_b = here.n0 + S::half(1, 0) * b + put_col < p.N ? put : GEMM_NOWHERE;
             float add[8];                         // bias of the lane's columns (GRAD: their sums)
 #pragma unroll
             for (int x = 0; x < 8; ++x) add[x] = 0.f;
             if (!GRAD && p.bias) {
                 if (p.bias_by_value) {
 #pragma unroll
-                    for (int x = 0; x < 8; ++x) add[x] = bf16_to_f32(p.bias[(int64_t)here.e * p.N + min(here.n0 + 64 * J * b + put_col + x, p.N - 1)]);
+                    for (int x = 0; x < 8; ++x) add[x] = bf16_to_f32(p.bias[(int64_t)here.e * p.N + min(here.n0 + S::half(1, 0) * b + put_col + x, p.N - 1)]);
                 } else {
-                    Elem<PLANMOE_BF16>::unpack(*reinterpret_cast<const uint4 *>(lds + S::BIAS + turn * 1024 + (64 * J * b + put_col) * 2), add);
+                    Elem<PLANMOE_BF16>::unpack(*reinterpret_cast<const uint4 *>(lds + S::BIAS + turn * 1024 + (S::half(1, 0) * b + put_col) * 2), add);
                 }
             }
 #pragma unroll
             for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int i = 0; i < I; ++i) {
-                    auto so = [&](int t) { return ((uint32_t)(64 * I * a + 32 * i + 16 / J * t) * (uint32_t)p.ldc + 64 * J * b) * 2u; };
-                    const int n = (2 * b + a) * I + i;
-                    if (GRAD && n + 1 < 4 * I) ask(n + 1);
+                for (int i = 0; i < S::I(a); ++i) {
+                    auto so = [&](int t) { return ((uint32_t)(row_of(a, i) + 16 / J * t) * (uint32_t)p.ldc + S::half(1, 0) * b) * 2u; };
+                    const int n = PIECES * b + S::I(0) * a + i;
+                    if (GRAD && n + 1 < 2 * PIECES) ask(n + 1);
 #pragma unroll
                     for (int jj = 0; jj < J; ++jj)
                         asm volatile("" : "+a"(acc[a][b][i][jj]));      // (in the accumulator registers until here: copied all at once they would not fit)
@@ -483,11 +501,12 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
                 const int c = l % (32 * J);
 #pragma unroll
                 for (int r = 0; r < 16 / J; ++r) s += sums[(c / 8 + 4 * J * r) * 8 + c % 8];
-                const int col = here.n0 + 64 * J * b + wn * 32 * J + c, slots = (p.M + 127) / 128 * 2, slot = here.m0 / 128 * 2 + wm;
+                const int col = here.n0 + S::half(1, 0) * b + wn * 32 * J + c;
+                const int each = S::WM == 2 ? 128 : S::BM, slots = (p.M + each - 1) / each * S::WM, slot = here.m0 / each * S::WM + wm;
                 if (l < 32 * J && col < p.N && slot < slots) {
                     float *to = p.colsum + ((int64_t)here.e * slots + slot) * p.N + col;
                     to[0] = s;
-                    if (I == 2 && slot + 2 < slots) to[2 * (int64_t)p.N] = 0.f;        // (a tile of 256 rows: all in the first slot)
+                    if (S::WM == 2 && S::BM == 256 && slot + 2 < slots) to[2 * (int64_t)p.N] = 0.f;        // (a tile of 256 rows: all in the first slot)
                 }
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_sched_barrier(0);
@@ -501,21 +520,21 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 #pragma unroll
             for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int i = 0; i < I; ++i)
+                for (int i = 0; i < S::I(a); ++i)
 #pragma unroll
                     for (int jj = 0; jj < J; ++jj)
 #pragma unroll
                         for (int q = 0; q < 16; ++q) acc[a][b][i][jj][q] = 0.f;
         do {
-            PM_PHASE(0, 0, 0, 0, 1, 1, 0, 1, 0, c2);
-            PM_PHASE(1, 0, 1, 0, 0, 1, 0, 1, 1, c2);
-            PM_PHASE(2, 1, 1, 1, 0, 0, 0, 0, 1, c2);
-            PM_PHASE(3, 1, 0, 1, 1, 1, 1, 0, 0, c3);
+            PM_PHASE(0, 0, 0, 0, 1, 1, 0, 0, S::EARLY, 0, 1, 0, c2);
+            PM_PHASE(1, 0, 1, 0, 0, 1, S::EARLY, 0, 0, 0, 1, 1, c2);
+            PM_PHASE(2, 1, 1, 1, 0, 0, 0, 0, 0, 0, 0, 1, c2);
+            PM_PHASE(3, 1, 0, 1, 1, 1, 0, 0, 0, 1, 0, 0, c3);
             c2 = c3; advance(c3);
-            PM_PHASE(4, 0, 1, 1, 1, 0, 1, 1, 1, c2);
-            PM_PHASE(5, 0, 0, 1, 0, 1, 1, 1, 0, c2);
-            PM_PHASE(6, 1, 0, 0, 0, 0, 1, 0, 1, c2);
-            PM_PHASE(7, 1, 1, 0, 1, 0, 0, 0, 0, c3);
+            PM_PHASE(4, 0, 1, 1, 1, 0, 0, 1, S::EARLY, 1, 1, 1, c2);
+            PM_PHASE(5, 0, 0, 1, 0, 1, S::EARLY, 0, 0, 1, 1, 0, c2);
+            PM_PHASE(6, 1, 0, 0, 0, 0, 0, 0, 0, 1, 0, 1, c2);
+            PM_PHASE(7, 1, 1, 0, 1, 0, 0, 0, 0, 0, 0, 0, c3);
             c2 = c3; advance(c3);
             fresh = 0;
         } while (--left);
@@ -537,7 +556,7 @@ __global__ __launch_bounds__(GEMM_WG, (GemmShape<I, J>::WAVES_PER_SIMD)) void ge
 // work-group, its waves every fourth slot, eight loads in flight
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restrict__ parts, const int *__restrict__ live, int live_planes,
-                                                          int live_round, int batches, int M, int N, int BM, int slots,
+                                                          int live_round, int batches, int M, int N, int BM, int per_tile, int slots,
                                                           void *__restrict__ out)
 {
     __shared__ float s_sum[4][64];
@@ -548,7 +567,7 @@ __global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restric
         for (int j = 0; j < live_planes; ++j) c += live[j * batches + e];
         rows = min(M, (c + live_round - 1) / live_round * live_round);
     }
-    const int used = min(slots, (rows + BM - 1) / BM * 2);
+    const int used = min(slots, (rows + BM - 1) / BM * per_tile);
     const float *from = parts + (int64_t)e * slots * N + min(n, N - 1);
     float s = 0.f;
     for (int i0 = wave * 8; i0 < used; i0 += 32) {
@@ -599,11 +618,10 @@ using namespace pm;
 
 namespace {
 
-template <int I, int J, bool TA, bool TB, bool GRAD>
+template <class S, bool TA, bool TB, bool GRAD>
 int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 {
-    using S = GemmShape<I, J>;
-    const auto kernel = gemm_bf16_kernel<I, J, TA, TB, GRAD>;
+    const auto kernel = gemm_bf16_kernel<S, TA, TB, GRAD>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -612,8 +630,8 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
                    "%s: the kernel needs %d bytes of LDS", who, S::LDS);
         if (dev < 64) ready[dev] = true;
     }
-    const int64_t side = p.split == 2 ? 256 : S::BM;
-    int64_t tiles = ((int64_t)p.M + side - 1) / side * (((int64_t)p.N + side - 1) / side) * p.batches;
+    const int64_t side = p.split == 2 ? 256 : S::BM, side_n = p.split == 2 ? 256 : S::BN;
+    int64_t tiles = ((int64_t)p.M + side - 1) / side * (((int64_t)p.N + side_n - 1) / side_n) * p.batches;
     PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
     if (p.split == 2) tiles = 4 * (tiles < p.stay / 2 ? tiles : p.stay / 2);
     const int64_t stay = (int64_t)compute_units() * S::WAVES_PER_SIMD / 8 * 8;
@@ -624,19 +642,64 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 
 // Which tile: 256 x 256 moves the fewest operand bytes per product, 128 x 128 (two work-groups per compute
 // unit) leaves fewer compute units idle where there are few tiles and loses less in a last round that is
-// not full.  A launch takes its rounds; a round takes its k-tiles and what a tile costs once (start,
-// results).  Microseconds, fitted to 22 shapes from 8 x 4 x 4096 x 1024 to 8 x 4928 x 4096 x 1024 (within 10 % there):
-// a k-tile of 256 x 256 takes 1.0 us with few compute units at work and 1.3 with all of them (the clock sinks
-// under the matrix cores), one of 128 x 128 takes 0.45 alone on its compute unit and 0.8 for two at a time.
-// Example: 8 x 512 x 2048 x 2048 takes 37 us in the small tiles and 49 in the large, 8 x 1024 x 2048 x 2048 69 and 59.
+// not full.  Between them 128, 160 and 192 rows by 256 columns, where the tiles of 256 rows leave compute units idle and 128 x 128
+// is bound by its operands: the height whose tiles fill the rounds best.  A launch takes its rounds; a round takes its k-tiles,
+// each faster with few compute units at work than with all of them (the clock sinks under the matrix cores), and what a tile
+// costs once; reading the weights is a floor (4.6 TB/s in tiles of 256 columns that are low, 3.3 otherwise).  Fitted to 42
+// timings of 14 shapes: what it picks takes 0.8 % longer than the best (1.10 times the best without the low tiles).
+// us in one launch, rows +- sqrt(rows) in use, nn:
+//   experts x rows, in, out      128 x 128    256    128    160    192 x 256
+//   8 x 500, 2048, 2048             49         48     57     42     42     (54 in 256 and a launch of quarters)
+//   8 x 128, 4096, 4096             84         80     64     64     66
+//   16 x 512, 1024, 1024            29         31     34     25     26
+//   8 x 250, 2048, 2048             31         43     29     32     35
+//   8 x 2000, 4096, 1024           142        171    158    129    140
+//   8 x 4096, 4096, 4096          1125        846    987    968    930
 //
-// A last round of large tiles that is at most half full is a launch of its own, in quarters (8 experts of 4096 +- 100
+// A last round of large tiles that is at most half full may be a launch of its own, in quarters (8 experts of 4096 +- 100
 // rows by 1024 columns: 512 tiles and a few, whose third round would take half as long again as the other two).
-double gemm_cost_small(int64_t tiles, double kt, int64_t cu)
-{
-    const int64_t rest = tiles % (2 * cu);
-    return (double)(tiles / (2 * cu)) * (0.8 * kt + 5) + (rest == 0 ? 0. : rest <= cu ? 0.45 * kt + 5 : 0.8 * kt + 5);
-}
+struct GemmCost {
+    double rows, kt, cu;                         // rows expected of a batch; k-tiles
+    int64_t most, n, batches, weight_bytes;      // rows at most
+    bool counted;                                // the rows are an expectation: of many batches, with a standard deviation of its root
+
+    double tiles(int64_t bm, int64_t bn) const
+    {
+        double t = 0;
+        for (const double q : {-1.5, -0.5, 0.5, 1.5}) {
+            const int64_t r = counted ? std::min(most, std::max<int64_t>(1, (int64_t)(rows + q * std::sqrt(rows)))) : (int64_t)rows;
+            t += 0.25 * (double)((r + bm - 1) / bm);
+        }
+        return t * (double)((n + bn - 1) / bn * batches);
+    }
+    double rounds(double t, double low, double high, double once) const
+    {
+        const double full = std::floor(t / cu), rest = t - full * cu;
+        return full * (high * kt + once) + (rest > 0.01 ? (low + (high - low) * rest / cu) * kt + once : 0.);
+    }
+    double quarters(double t) const              // tiles of 128 x 128, two work-groups per compute unit
+    {
+        const double full = std::floor(t / (2 * cu)), rest = t - full * 2 * cu;
+        return full * (kt + 2) + (rest <= 0.01 ? 0. : rest <= cu ? (0.41 + 0.19 * rest / cu) * kt + 2 : (0.6 + 0.4 * (rest - cu) / cu) * kt + 2);
+    }
+    double floor(double rate) const { return (double)weight_bytes * 1e-6 / rate + 6; }
+    double small() const { return std::max(quarters(tiles(128, 128)) + 7, floor(3.3)); }
+    double big() const { return std::max(rounds(tiles(256, 256), 1.0, 1.4, 3) + 6, floor(3.3)); }
+    // the last round as a launch of quarters; with many rounds it hardly counts
+    double big_and_quarters() const
+    {
+        const double t = tiles(256, 256), full = std::floor(t / cu), last = t - full * cu;
+        return t < 6 * cu && full > 0 && last > 0.01 && 2 * last <= cu ? std::max(full * (1.4 * kt + 3) + 6 + quarters(4 * last) + 10, floor(3.3)) : 1e30;
+    }
+    double low(int height) const                 // height: 128, 160, 192
+    {
+        const double t = tiles(height, 256), us = height == 128 ? rounds(t, 0.58, 0.9, 2) : height == 160 ? rounds(t, 0.7, 1.07, 2) : rounds(t, 0.79, 1.25, 2);
+        return std::max(us + 6, floor(4.6));
+    }
+};
+
+// The column sums of a masked product: a tile of so many rows has so many slots (0 rows: one slot for everything)
+struct GemmSlots { int rows, per_tile; };
 
 // few rows per batch against a whole weight
 bool gemm_is_skinny(int64_t m, int64_t n, int64_t k, int64_t batches)
@@ -645,31 +708,37 @@ bool gemm_is_skinny(int64_t m, int64_t n, int64_t k, int64_t batches)
 }
 
 template <bool TA, bool TB, bool GRAD>
-int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who)
+int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who, GemmSlots *sums = nullptr)
 {
+    if (sums) *sums = GemmSlots{128, 2};
     const bool contiguous = p.lda == p.K && p.ldb == (TB ? p.N : p.K) && p.ldc == p.N && p.sB == (int64_t)p.N * p.K && p.sA == (int64_t)p.M * p.K &&
                             p.sC == (int64_t)p.M * p.N;
     if (!TA && contiguous && gemm_is_skinny(p.M, p.N, p.K, p.batches)) {
+        if (sums) *sums = GemmSlots{0, 1};
         SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
         return gemm_skinny_run(!TB, few, stream, who);
     }
-    const int64_t cu = compute_units(), rows = TA ? p.M : rows_hint;
-    // (row counts from the device: an expectation, and a batch may have a standard deviation more)
-    const int64_t most = !TA && p.live ? rows + (int64_t)std::sqrt((double)rows) : rows;
-    const double kt = (double)((TA ? rows_hint : p.K) + 63) / 64;
-    const int64_t big = (most + 255) / 256 * (((int64_t)p.N + 255) / 256) * p.batches, small = (most + 127) / 128 * (((int64_t)p.N + 127) / 128) * p.batches;
-    const int64_t last = big % cu;
-    const double t_big = (double)(big / cu) * (1.3 * kt + 10) +
-                         (last == 0 ? 0. : 2 * last <= cu ? gemm_cost_small(4 * last, kt, cu) + 3 : (1.0 + 0.3 * (double)last / (double)cu) * kt + 10);
-    if (gemm_cost_small(small, kt, cu) < t_big) return gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who);
+    const int64_t cu = compute_units();
+    const GemmCost cost{(double)(TA ? p.M : rows_hint), (double)(((TA ? rows_hint : p.K) + 63) / 64), (double)cu, p.M, p.N, p.batches,
+                        TA ? 0 : (int64_t)p.N * p.K * p.batches * 2, !TA && p.live};
+    const double small = cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
+    if constexpr (!TA) {
+        const double low[3] = {cost.low(128), cost.low(160), cost.low(192)};
+        const int f = low[0] <= low[1] && low[0] <= low[2] ? 0 : low[1] <= low[2] ? 1 : 2;
+        if (low[f] < small && low[f] < big) {
+            if (sums) *sums = GemmSlots{128 + 32 * f, 1};
+            if (f == 0) return gemm_launch<GemmFlat<2, 2>, TA, TB, GRAD>(p, stream, who);
+            if (f == 1) return gemm_launch<GemmFlat<2, 3>, TA, TB, GRAD>(p, stream, who);
+            return gemm_launch<GemmFlat<3, 3>, TA, TB, GRAD>(p, stream, who);
+        }
+    }
+    if (small < big) return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
     p.stay = (int)(cu / 8 * 8);
-    // (with many rounds the last one hardly counts, and a launch that may find nothing to do costs 3 us; a weight
-    // gradient's tiles are known here)
-    p.split = big < 6 * cu && (p.live && !TA ? true : gemm_last_round((int)big, p.stay) > 0);
-    if (gemm_launch<2, 2, TA, TB, GRAD>(p, stream, who)) return 1;
+    p.split = big == split;
+    if (gemm_launch<Gemm256, TA, TB, GRAD>(p, stream, who)) return 1;
     if (!p.split) return 0;
     p.split = 2;
-    return gemm_launch<1, 1, TA, TB, GRAD>(p, stream, who);
+    return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
 }
 
 // what the buffer descriptors cover: from a tile's corner, a tile of a k-fast operand and 64 rows of a k-slow one
@@ -793,24 +862,23 @@ extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void
     hipStream_t st = (hipStream_t)stream;
     float *parts = dbias ? (float *)workspace : nullptr;
     const int hint = rows_hint >= 1 && rows_hint < m ? rows_hint : m;
-    int tile_rows, slots;
+    GemmSlots sums;
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
         const Gemm32Kernel kernel = gemm_f32_pick(1, p, hint);
-        tile_rows = gemm_f32_slot_rows(kernel);
-        slots = (m + tile_rows - 1) / tile_rows * 2;
+        sums = GemmSlots{gemm_f32_slot_rows(kernel), 2};
         if (gemm_f32_run(1, p, kernel, st, who)) return 1;
     } else {
         GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
                    m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};
-        if (gemm_run<false, false, true>(p, hint, st, who)) return 1;
-        tile_rows = 128;
-        slots = gemm_is_skinny(m, n, k, batches) ? 1 : (m + 127) / 128 * 2;       // (few rows altogether: one slot holds everything)
+        if (gemm_run<false, false, true>(p, hint, st, who, &sums)) return 1;
     }
     if (dbias) {
+        if (sums.rows == 0) sums.rows = m;
+        const int slots = (m + sums.rows - 1) / sums.rows * sums.per_tile;
         const dim3 grid((unsigned)((n + 63) / 64), (unsigned)batches);
-        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, slots, dbias);
-        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, tile_rows, slots, dbias);
+        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, sums.rows, sums.per_tile, slots, dbias);
+        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, sums.rows, sums.per_tile, slots, dbias);
         PM_LAUNCH_CHECK(who);
     }
     return 0;

@@ -379,3 +379,39 @@ def test_expert_gemm_fp32_in_parts_takes_the_rows_in_use_only(B, cap, n, k, hint
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), torch.float32)).all()), e
         d = dy[e, :r].double()
         assert bool(((dw[e].double() - x.t() @ d).abs() <= _bound(d, x.abs().t() @ d.abs(), cap, torch.float32)).all()), e
+
+
+# bf16 tiles of 128, 160 and 192 rows by 256 columns: rows that end on such a tile, one before and one behind, of one row and none;
+# columns around a multiple of 256, reductions of an odd and an even number of k-tiles with 8 k in the last one, of two k-tiles; no row counts
+@pytest.mark.parametrize("cap,n,k,hint,counts", [(400, 2040, 136, 290, [256, 257, 255, 0, 1, 128, 384, 400]), (160, 4000, 520, 120, [128, 129, 127, 160, 1, 0, 64, 33]),
+                                                 (620, 2056, 200, 490, [480, 481, 479, 620, 0, 1, 160, 161]), (620, 2048, 520, 500, [320, 640, 159, 97, 96, 95, 64, 65]),
+                                                 (1100, 1032, 520, 1000, [960, 961, 959, 1100, 1, 192, 193, 97]), (2500, 2048, 72, 2000, [1920, 1921, 1919, 2500, 0, 1, 288, 289]),
+                                                 (768, 1000, 520, 0, [768] * 8), (384, 4088, 200, 0, [384] * 8)])
+def test_expert_gemm_low_tiles(cap, n, k, hint, counts):
+    from planmoe_amd import ops
+    print("case", cap, n, k, hint, flush=True)
+    B, dtype = 8, torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(cap + n)
+    a, w = torch.randn(B, cap, k, device=DEV, generator=g).to(dtype), torch.randn(B, k, n, device=DEV, generator=g).to(dtype)
+    bias, h = torch.randn(B, n, device=DEV, generator=g).to(dtype), torch.randn(B, cap, n, device=DEV, generator=g).clamp(min=0).to(dtype)
+    rows = [min(cap, c) for c in counts]
+    for e, r in enumerate(rows):
+        a[e, r:] = float("nan")
+    wt, live = w.transpose(1, 2).contiguous(), torch.tensor([counts], dtype=torch.int32, device=DEV) if hint else None
+    nn = torch.full((B, cap, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    kw = dict(live=live, rows_hint=hint)
+    ops.expert_gemm("nn", a, w, bias, relu=True, out=nn, **kw)
+    ops.expert_gemm("nt", a, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, out=masked, **kw)
+    torch.cuda.synchronize()
+    for e, r in enumerate(rows):
+        ref, mag = a[e, :r].double() @ w[e].double(), a[e, :r].double().abs() @ w[e].double().abs()
+        tol, biased = _bound(ref, mag, k, dtype), ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all()), e
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all()), e
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all()), e
+        for out in (nn, nt, masked):
+            assert bool((out[e, r:] == 7.0).all()), e
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), e
