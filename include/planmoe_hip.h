@@ -504,6 +504,31 @@ int planmoe_layer_combine_bwd_codes(const void *grad, const uint8_t *codes, cons
                                     int model_dim, int experts, int capacity, void *grad_rows,
                                     float *grad_gates, void *stream);
 
+/* The zfp codec at rate 8 on the layer's fp32 rows (what Compress and Decompress of "zfp" do around a one-rank
+ * exchange, zfpc.cpp:23-86): same bits as planmoe_zfp_compress and planmoe_zfp_decompress of the buffer whose empty
+ * slots are zeros, without the stream in between.  expert_counts [top_k][experts] from the routing that made
+ * indices and locations: slots from min(sum of an expert's counts, capacity) on, rounded up to 4, are neither read nor
+ * written.  model_dim and capacity multiples of 4.
+ *   _dispatch     rows[slot] = codec(x[token])
+ *   _rows         rows = codec(rows) in place (rows between the count and its multiple of 4 are part of their
+ *                 blocks); stream_out, if not NULL, gets the rows' stream (planmoe_zfp_stream_bytes; blocks without a
+ *                 row in use are left as they are)
+ *   _combine_bwd  grad_rows[slot] = codec(gate * grad[token]); grad_gates [top_k][plane_stride] = <grad[token], row> with
+ *                 the rows decoded from the stream that _rows wrote, 0 for a choice without a slot
+ * Workspace: planmoe_layer_zfp_workspace_bytes, 16-byte aligned. */
+size_t planmoe_layer_zfp_workspace_bytes(int experts, int capacity);
+int planmoe_layer_zfp_dispatch(const float *x, const int32_t *indices, const int32_t *locations, int64_t plane_stride,
+                               int top_k, int samples, int model_dim, int experts, int capacity,
+                               const int32_t *expert_counts, float *rows, void *workspace,
+                               size_t workspace_bytes, void *stream);
+int planmoe_layer_zfp_rows(float *rows, int model_dim, int experts, int capacity, const int32_t *expert_counts,
+                           int planes, void *stream_out, size_t stream_capacity, void *stream);
+int planmoe_layer_zfp_combine_bwd(const void *stream_in, const float *grad, const float *gates, const int32_t *indices,
+                                  const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                                  int model_dim, int experts, int capacity, const int32_t *expert_counts,
+                                  float *grad_rows, float *grad_gates, void *workspace, size_t workspace_bytes,
+                                  void *stream);
+
 /* out[e][c] = sum over the rows in use of a[e] (live as planmoe_expert_gemm): a bias gradient of
  * experts/ffn.py:77-79.  fp32 sums, one rounding. */
 size_t planmoe_rows_colsum_workspace_bytes(int batches, int rows, int cols);

@@ -96,6 +96,12 @@ SIGNATURES = {
                                           c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "planmoe_layer_combine_keep": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
                                            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "planmoe_layer_zfp_workspace_bytes": (c_size_t, [c_int, c_int]),
+    "planmoe_layer_zfp_dispatch": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                                           c_void_p, c_size_t, c_void_p]),
+    "planmoe_layer_zfp_rows": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
+    "planmoe_layer_zfp_combine_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                              c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "planmoe_layer_combine_bwd_codes": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64,
                                                 c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "planmoe_rows_colsum_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),

@@ -48,30 +48,14 @@ Tensor lz_round_trip(const Tensor &buf, void *st)
     return out;
 }
 
-Tensor zfp_stream_of(const Tensor &rows, const Shape &s, void *st)
+Tensor zfp_stream(const Shape &s, const Tensor &like) { return bytes((int64_t)planmoe_zfp_stream_bytes(2, s.M, s.rows(), ZFP_RATE), like); }
+
+void zfp_rows(const Tensor &rows, const Tensor &stream, const Pass &p, const Shape &s, void *st)
 {
-    Tensor out = bytes((int64_t)planmoe_zfp_max_bytes(2, s.M, s.rows(), ZFP_RATE), rows);
-    PM_CALL(planmoe_zfp_compress(floats(rows), 2, s.M, s.rows(), ZFP_RATE, out.data_ptr(), (size_t)out.numel(), st));
-    return out;
+    PM_CALL(planmoe_layer_zfp_rows(rows.data_ptr<float>(), s.M, s.E, s.cap, ints(p.counts), s.k, raw(stream), stream.defined() ? (size_t)stream.numel() : 0, st));
 }
 
-Tensor zfp_dispatch(const Tensor &x, const float *gates, const Pass &p, const Shape &s, void *st)
-{
-    Tensor coded = bytes((int64_t)planmoe_zfp_max_bytes(2, s.M, s.rows(), ZFP_RATE), x);
-    Tensor ws = bytes((int64_t)planmoe_dispatch_zfp_workspace_bytes(s.E, s.cap), x), out = at::empty({s.rows(), s.M}, x.options());
-    PM_CALL(planmoe_dispatch_zfp(floats(x), gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap, ZFP_RATE,
-                                 coded.data_ptr(), (size_t)coded.numel(), ws.data_ptr(), (size_t)ws.numel(), st));
-    PM_CALL(planmoe_zfp_decompress(coded.data_ptr(), 2, s.M, s.rows(), ZFP_RATE, out.data_ptr<float>(), st));
-    return out;
-}
-
-Tensor zfp_combine(const Tensor &stream, const float *gates, const Pass &p, const Shape &s, void *st)
-{
-    Tensor out = at::empty({s.T, s.M}, stream.options().dtype(at::kFloat)), ws = bytes((int64_t)planmoe_combine_zfp_workspace_bytes(s.E, s.cap), stream);
-    PM_CALL(planmoe_combine_zfp(stream.data_ptr(), ZFP_RATE, gates, ints(p.indices), ints(p.locations), s.T, s.k, s.T, s.M, s.E, s.cap,
-                                out.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
-    return out;
-}
+Tensor zfp_workspace(const Shape &s, const Tensor &like) { return bytes((int64_t)planmoe_layer_zfp_workspace_bytes(s.E, s.cap), like); }
 
 Live live_rows(const Pass &p, const Shape &s, int codec)
 {
@@ -118,7 +102,10 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     if (codec == CODEC_ZFP) {
         PM_CALL(planmoe_gate_route(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, idx, loc, raw(p.gates),
                                    s.T, nullptr, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, ws.data_ptr(), (size_t)ws.numel(), st));
-        p.xe = zfp_dispatch(x, nullptr, p, s, st);
+        p.xe = at::empty({s.rows(), s.M}, x.options());
+        ws = zfp_workspace(s, x);
+        PM_CALL(planmoe_layer_zfp_dispatch(floats(x), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt, p.xe.data_ptr<float>(), ws.data_ptr(),
+                                           (size_t)ws.numel(), st));
     } else if (codec == CODEC_LZ) {
         p.xe = at::empty({s.rows(), s.M}, x.options());
         PM_CALL(planmoe_forward_plain(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, idx, loc,
@@ -141,10 +128,8 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
                                 s.hint(), p.ye.data_ptr(), st));
     const Tensor gates = float_gates(p.gates);
     if (codec == CODEC_ZFP) {
-        p.stream = zfp_stream_of(p.ye, s, st);
-        p.ye = Tensor();                     // (the backward pass reads the stream)
-        p.y = zfp_combine(p.stream, floats(gates), p, s, st);
-        return p;
+        if (keep) p.stream = zfp_stream(s, x);
+        zfp_rows(p.ye, p.stream, p, s, st);
     }
     if (codec == CODEC_LZ) p.ye = lz_round_trip(p.ye, st);
     p.y = at::empty({s.T, s.M}, x.options());
@@ -158,6 +143,7 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
         return p;
     }
     PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, codec == CODEC_INT8, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
+    if (p.stream.defined()) p.ye = Tensor();         // (the backward pass reads the stream)
     return p;
 }
 
@@ -231,10 +217,10 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
             grad_gates = at::empty({s.k, s.T}, x.options().dtype(at::kFloat));
             Tensor gye;
             if (codec == CODEC_ZFP) {
-                gye = zfp_dispatch(grad, floats(gates), p, s, st);
-                Tensor ws = bytes((int64_t)planmoe_combine_zfp_workspace_bytes(s.E, s.cap), x);
-                PM_CALL(planmoe_bwd_gate_zfp(ye.data_ptr(), ZFP_RATE, floats(grad), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
-                                             grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
+                gye = at::empty({s.rows(), s.M}, x.options());
+                Tensor ws = zfp_workspace(s, x);
+                PM_CALL(planmoe_layer_zfp_combine_bwd(ye.data_ptr(), floats(grad), floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, ints(p.counts),
+                                                      gye.data_ptr<float>(), grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
             } else if (codec == CODEC_LZ) {
                 Tensor buf = at::empty({s.rows(), s.M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(s.E, s.cap), x);
                 PM_CALL(planmoe_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, buf.data_ptr(),
@@ -280,14 +266,11 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                     Tensor gxe = at::empty({s.rows(), s.M}, x.options());
                     PM_CALL(planmoe_expert_gemm(1, s.dt, gh.data_ptr(), w1.data_ptr(), nullptr, 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
                                                 s.hint(), gxe.data_ptr(), st));
-                    if (codec == CODEC_ZFP) {
-                        dx = zfp_combine(zfp_stream_of(gxe, s, st), nullptr, p, s, st);
-                    } else {
-                        if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
-                        dx = at::empty_like(x);
-                        PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
-                                                      dx.data_ptr(), st));
-                    }
+                    if (codec == CODEC_ZFP) zfp_rows(gxe, Tensor(), p, s, st);
+                    if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
+                    dx = at::empty_like(x);
+                    PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                                                  dx.data_ptr(), st));
                 }
             }
         }

@@ -365,3 +365,74 @@ def test_native_layer_on_a_stream_of_its_own(codec, dtype):
     torch.cuda.synchronize()
     for name in want:
         assert torch.equal(want[name], got[name]), name
+
+
+# the zfp codec as it reaches the layer's rows against the coder and the decoder, bit for bit: fields that spend their bits on few
+# planes and on many, whose budget ends in and between planes and that never reach it, zeros, subnormals, infinities, NaN, the largest values
+@pytest.mark.parametrize("M", [4, 64, 1028])
+def test_layer_zfp_rows_equal_compress_and_decompress(M):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", M, flush=True)
+    E, cap = 8, 64
+    g = torch.Generator().manual_seed(M)
+    rows = torch.randn(E, cap, M, generator=g)
+    at = torch.arange(M) / M
+    rows[1] = torch.sin(at * torch.randint(1, 9, (cap, 1), generator=g)) + 1e-3 * rows[1]
+    rows[2] = torch.exp(20 * rows[2])                                                         # a few values tell
+    rows[3] *= torch.rand(cap, M, generator=g) < 0.1
+    rows[4] = rows[4].sign() * 2.0 ** torch.randint(-149, 128, (cap, M), generator=g).float()
+    rows[5, :16], rows[5, 16:32], rows[5, 32:48] = 0.75, torch.randint(-4, 5, (16, M), generator=g).float(), rows[5, 32:48] * 1e-42
+    rows[5, 48:52], rows[5, 52:56], rows[5, 56:] = 0.0, 3.4e38, rows[5, 56:] * 2.0 ** -126
+    special = torch.tensor([float("inf"), float("-inf"), float("nan"), -0.0, 1.0, 3e38, 1e-40])
+    rows[6] = torch.where(torch.rand(cap, M, generator=g) < 0.05, special[torch.randint(0, 7, (cap, M), generator=g)], rows[6])
+    rows[7] = special[torch.randint(0, 7, (cap, M), generator=g)]
+    counts = torch.tensor([[64, 30, 64, 61, 40, 64, 0, 63], [0, 5, 70, 2, 24, 0, 64, 0]], dtype=torch.int32)
+    rows, counts = rows.to(DEV), counts.to(DEV)
+    stream = ops.zfp_compress(rows.view(E * cap, M), M, E * cap, 2)
+    want = ops.zfp_decompress(stream, M, E * cap, 2).view(E, cap, M)
+    for keep in (False, True):
+        got, kept = rows.clone(), torch.zeros_like(stream)
+        check(lib.planmoe_layer_zfp_rows(ops._ptr(got), M, E, cap, ops._ptr(counts), 2, ops._ptr(kept) if keep else None,
+                                         kept.numel() * kept.element_size() if keep else 0, ops._stream(got)))
+        torch.cuda.synchronize()
+        for e, n in enumerate(counts.sum(0).clamp(max=cap).tolist()):
+            n = (n + 3) // 4 * 4
+            assert torch.equal(got[e, :n].view(torch.int32), want[e, :n].view(torch.int32)), (e, keep)
+            assert torch.equal(got[e, n:].view(torch.int32), rows[e, n:].view(torch.int32)), (e, keep)
+            if keep:
+                size = cap * M                   # (a byte a value)
+                a, b = (t.view(torch.uint8)[e * size:e * size + n * M] for t in (kept, stream))
+                assert torch.equal(a, b) and not kept.view(torch.uint8)[e * size + n * M:(e + 1) * size].any(), e
+
+
+@pytest.mark.parametrize("T,M,E,k,cap", [(1, 4, 4, 1, 4), (333, 520, 4, 2, 100), (100, 1028, 8, 3, 64), (257, 64, 16, 2, 8)])
+def test_layer_zfp_dispatch_and_combine_backward_equal_the_steps(T, M, E, k, cap):
+    """Against planmoe_dispatch_zfp, planmoe_zfp_decompress and planmoe_bwd_gate_zfp, bit for bit; tokens that take no slot."""
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", T, M, E, k, cap, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + M)
+    x, grad = torch.randn(T, M, generator=g, device=DEV), torch.randn(T, M, generator=g, device=DEV)
+    routed = ops.route_topk(torch.softmax(torch.randn(T, E, generator=g, device=DEV), 1), k)
+    idx, loc = (torch.stack(list(routed[n])).int().contiguous() for n in ("indices", "locations"))
+    gates = torch.rand(k, T, generator=g, device=DEV)
+    counts = torch.stack([torch.bincount(i.long(), minlength=E) for i in idx]).int().contiguous()
+    ws = torch.empty(lib.planmoe_layer_zfp_workspace_bytes(E, cap), dtype=torch.uint8, device=DEV).fill_(0x7f)      # (no slot of before helps)
+    rows, grad_rows = torch.full((E, cap, M), 7.0, device=DEV), torch.full((E, cap, M), 7.0, device=DEV)
+    grad_gates = torch.full((k, T), 7.0, device=DEV)
+    check(lib.planmoe_layer_zfp_dispatch(ops._ptr(x), ops._ptr(idx), ops._ptr(loc), T, k, T, M, E, cap, ops._ptr(counts), ops._ptr(rows),
+                                         ops._ptr(ws), ws.numel(), ops._stream(x)))
+    want = ops.zfp_decompress(ops.dispatch_zfp(x, list(idx), list(loc), None, E, cap), M, E * cap, 2).view(E, cap, M)
+    seen = ops.zfp_compress(torch.randn(E * cap, M, generator=g, device=DEV), M, E * cap, 2)
+    ws.fill_(0x7f)
+    check(lib.planmoe_layer_zfp_combine_bwd(ops._ptr(seen), ops._ptr(grad), ops._ptr(gates), ops._ptr(idx), ops._ptr(loc), T, k, T, M, E, cap,
+                                            ops._ptr(counts), ops._ptr(grad_rows), ops._ptr(grad_gates), ops._ptr(ws), ws.numel(), ops._stream(x)))
+    want_rows = ops.zfp_decompress(ops.dispatch_zfp(grad, list(idx), list(loc), list(gates), E, cap), M, E * cap, 2).view(E, cap, M)
+    want_gates = ops.bwd_gate_zfp(seen, grad, list(idx), list(loc), E, cap)
+    torch.cuda.synchronize()
+    assert torch.equal(grad_gates, want_gates.view(k, T))
+    for e, n in enumerate(counts.sum(0).clamp(max=cap).tolist()):
+        n = (n + 3) // 4 * 4
+        assert torch.equal(rows[e, :n], want[e, :n]) and bool((rows[e, n:] == 7.0).all()), e
+        assert torch.equal(grad_rows[e, :n], want_rows[e, :n]) and bool((grad_rows[e, n:] == 7.0).all()), e
