@@ -9,6 +9,7 @@
 //                         from the transposed histograms; token rows go to uint8 codes in their
 //                         slots (x is read a second time), slots past an expert's fill are zero
 //                         rows; one block finishes the GShard loss and the expert counts.
+//                         (planmoe_layer_dispatch of up to 32 tokens and 16 experts: one group, and all of this in one launch)
 //   group_offsets_kernel  only for top_k > 4 and for planmoe_gate_route (routing without
 //                         dispatch, finished by route_offsets_kernel): the prefix over groups as
 //                         a launch of its own.
@@ -95,6 +96,67 @@ __device__ __forceinline__ void wave_sum_n(T (&v)[N])
     for (int i = 0; i < N; ++i) v[i] = wave_allreduce(v[i], [](T a, T b) { return a + b; });
 }
 
+// OUT: what a kept row arrives as.  CODES: codes with bias and scale.  ROWS: no codec -- `codes` is the
+// dispatched buffer in x's dtype and a kept row arrives there as 0 + x (what fast_encode's accumulation
+// into zeros leaves: -0 becomes +0), an empty slot as zeros.  DECODED: the same buffer with what the
+// decompressor makes of the row's codes (the codes stay in registers: one pass where dispatch + int8
+// and the decompressor write and read them).
+enum { OUT_CODES = 0, OUT_ROWS = 1, OUT_DECODED = 2 };
+// A token's row to its slots (lane j holds that of choice j, -1: none).  each(f) calls f(u, vector u) for the lane's
+// vectors; minimum and maximum of the row are not used for ROWS.
+template <int DT, int OUT, typename Each>
+__device__ __forceinline__ void send_row(Each each, int slot, int top_k, int units, uint8_t *__restrict__ codes, void *__restrict__ bias_out,
+                                         void *__restrict__ scale_out, float mn, float mx)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC;
+    if constexpr (OUT == OUT_ROWS) {
+        each([&](int u, const uint4 &raw) {
+            float f[V];
+            E::unpack(raw, f);
+#pragma unroll
+            for (int i = 0; i < V; ++i) f[i] = 0.f + f[i];
+            const uint4 v = E::pack(f);
+            for (int j = 0; j < top_k; ++j) {
+                const int sl = rl_i(slot, j);
+                if (sl >= 0) stream_store(reinterpret_cast<uint4 *>(codes + (int64_t)sl * units * 16) + u, v);
+            }
+        });
+        return;
+    }
+    const float scale = E::round(mx - mn);
+    if constexpr (OUT == OUT_CODES) {
+        if (slot >= 0) { E::store(bias_out, slot, mn); E::store(scale_out, slot, scale); }
+    }
+    const RowEncoder<DT> enc(mn, scale);
+    const RowDecoder<DT> dec(mn, scale);
+    auto body = [&](auto mode) {
+        each([&](int u, const uint4 &raw) {
+            uint32_t w[2];
+            enc.template encode<decltype(mode)::value>(raw, w);
+            if constexpr (OUT == OUT_DECODED) {
+                float f[V];
+#pragma unroll
+                for (int q = 0; q < V / 4; ++q) dec.word(w[q], f + 4 * q);
+                const uint4 v = E::pack(f);
+                for (int j = 0; j < top_k; ++j) {
+                    const int s = rl_i(slot, j);
+                    if (s >= 0) stream_store(reinterpret_cast<uint4 *>(codes + (int64_t)s * units * 16) + u, v);
+                }
+                return;
+            }
+            for (int j = 0; j < top_k; ++j) {
+                const int s = rl_i(slot, j);
+                if (s < 0) continue;
+                uint8_t *row = codes + (int64_t)s * (units * V);
+                if constexpr (V == 8) stream_store(reinterpret_cast<uint2 *>(row) + u, make_uint2(w[0], w[1]));
+                else stream_store(reinterpret_cast<uint32_t *>(row) + u, w[0]);
+            }
+        });
+    };
+    if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
+}
+
 // SDT: dtype of logits / scores / gates (F32 when fp32_gate, else the input dtype)
 // CAP: compile-time bound of the expert count held in registers by the routing epilogue
 // NT == 1: split-K over the 4 waves, weights straight from L2 (up to 16 experts);
@@ -102,15 +164,22 @@ __device__ __forceinline__ void wave_sum_n(T (&v)[N])
 // MODE 0: logits = x . wg^T computed here.  MODE 1 / 2: no GEMM; x holds the [samples, experts]
 // logits / scores in the routing dtype (the stand-alone routing entry point) and only the
 // epilogue runs, on 64-token groups.
-template <int DT, int SDT, int NT, int CAP, bool SPLITK, int GROUP, int MODE = 0>
+// ONE (not ONE_OFF): all tokens are one group, so what the group knows is all there is, and slots, loss and counts are
+// final.  OUT_ROWS / OUT_DECODED: the rows go to their slots as well; every work-group routes all tokens for itself, sends the
+// rows of four, and the first one writes the routing.  (A pass of the layer at 8 tokens x 1024, hidden 4096, 8 experts: 51.0 us
+// with two launches for this, 47.1 with one; the copy itself is 16 KB.)
+enum { ONE_OFF = -1, ONE_ROUTING = 0 };
+template <int DT, int SDT, int NT, int CAP, bool SPLITK, int GROUP, int MODE = 0, int ONE = ONE_OFF>
 __global__ __launch_bounds__(256) void gate_route_kernel(
     const void *__restrict__ x, const void *__restrict__ wg, const float *__restrict__ logit_bias,
     int samples, int model_dim, int experts, int k, int normalize_gate,
     int32_t *__restrict__ indices, int32_t *__restrict__ locations, void *__restrict__ gates,
     int64_t stride, void *__restrict__ logits_out, void *__restrict__ scores_out,
-    float *__restrict__ l_aux, int32_t *__restrict__ counts_out, void *__restrict__ workspace)
+    float *__restrict__ l_aux, int32_t *__restrict__ counts_out, void *__restrict__ workspace,
+    uint8_t *__restrict__ rows, int capacity)
 {
     using S = Elem<SDT>;
+    const bool first = ONE == ONE_OFF || blockIdx.x == 0;        // (of work-groups that route the same tokens)
     static_assert(GROUP == 64 || (SPLITK && GROUP == 32), "the LDS-shared variant is built for 64 tokens");
     constexpr int COLS = 16 * NT + 1;
     // split-K: part[4][GROUP][COLS] floats; else the weight buffers / logits[GROUP][COLS]
@@ -119,9 +188,9 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
     float (*part)[GROUP][COLS] = reinterpret_cast<float (*)[GROUP][COLS]>(smem);
 
     const int tid = threadIdx.x, lane = lane_id();
-    const int groups = gridDim.x;
+    const int groups = ONE == ONE_OFF ? gridDim.x : 1;
     const FwdWs ws = fwd_ws(workspace, groups, k, experts, samples);
-    const int t0 = blockIdx.x * GROUP;
+    const int t0 = ONE == ONE_OFF ? blockIdx.x * GROUP : 0;
     // the additive logit biases of this lane's experts, asked for before the GEMM: read where they are
     // used, their latency would stand in every pass of the epilogue (6.5 -> 2 us per group at 64 experts)
     constexpr int LPT_ = CAP < 16 ? CAP : 16, EPL_ = CAP / LPT_;
@@ -179,7 +248,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
     for (int p = 0; p < TPW4 / TPP; ++p) {
         const int tok = wave * TPW4 + p * TPP + min(tk, TPP - 1);   // lanes past the pass repeat a token
         const int t = t0 + tok;
-        const bool valid = t < samples && tk < TPP;
+        const bool valid = t < samples && tk < TPP, writes = valid && first;
         float sc[EPL];
         float mx = -INFINITY;
 #pragma unroll
@@ -191,7 +260,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
                 else v = part[0][tok][e];
                 v = S::round(v);
                 if constexpr (MODE != 2) {
-                    if (logits_out && valid) S::store(logits_out, (int64_t)t * experts + e, v);
+                    if (logits_out && writes) S::store(logits_out, (int64_t)t * experts + e, v);
                     if (logit_bias) v = S::round(v + lbias[q]);
                 }
             }
@@ -213,7 +282,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
                 const int e = q * LPT + el;
                 if (e < experts) {
                     sc[q] = S::round(sc[q] * inv);
-                    if (scores_out && valid) S::store(scores_out, (int64_t)t * experts + e, sc[q]);
+                    if (scores_out && writes) S::store(scores_out, (int64_t)t * experts + e, sc[q]);
                 } else {
                     sc[q] = -INFINITY;
                 }
@@ -254,14 +323,14 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
             if (el == 0 && tk < TPP) s_best[j][tok] = (uint8_t)bi;
             if (j < LPT) {
                 if (el == j) { my_gate = bv; my_idx = bi; }
-            } else if (valid && el == j % LPT) {
+            } else if (writes && el == j % LPT) {
                 // more planes than lanes per token: index and raw gate go out now, the gate is
                 // normalised below
                 indices[(int64_t)j * stride + t] = bi;
                 S::store(gates, (int64_t)j * stride + t, bv);
             }
         }
-        if (valid) {
+        if (writes) {
             const bool norm = k > 1 && normalize_gate;
             const float d = fmaxf(denom, eps);
             if (el < k) {
@@ -282,6 +351,8 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
     }
     __syncthreads();
 
+    __shared__ int32_t s_slot[ONE > 0 ? 4 : 1][GROUP];
+    __shared__ float s_range[ONE == OUT_DECODED && STATS ? GROUP : 1][2];
     // ---- part 2: wave 0, one lane per token: rank of every token among the group's tokens with
     // the same choice (wave ballots), the group's histograms, row min / max, score column sums
     if (tid < WAVE) {
@@ -299,14 +370,20 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
                 }
                 float lo, hi;
                 RowStats<PLANMOE_BF16, true>::decode(a, b, n, lo, hi);
-                ws.row_min[t] = lo; ws.row_max[t] = hi;
+                if constexpr (ONE == ONE_OFF) { ws.row_min[t] = lo; ws.row_max[t] = hi; }
+                else if constexpr (ONE == OUT_DECODED) { s_range[tid][0] = lo; s_range[tid][1] = hi; }
             }
         }
         if (l_aux && lane < experts) {
             const float v = ((s_me[0][lane] + s_me[1][lane]) + s_me[2][lane]) + s_me[3][lane];
-            ws.me[(int64_t)blockIdx.x * experts + lane] = v;
-            ws.me_t[(int64_t)lane * ws.gstride + blockIdx.x] = v;
+            if constexpr (ONE == ONE_OFF) {
+                ws.me[(int64_t)blockIdx.x * experts + lane] = v;
+                ws.me_t[(int64_t)lane * ws.gstride + blockIdx.x] = v;
+            } else {
+                s_me[0][lane] = v;
+            }
         }
+        int before = 0;                                            // ONE: entries of expert `lane` in the planes before
         for (int j = 0; j < k; ++j) {
             const int best = valid ? (int)s_best[j][tid % GROUP] : -1;
             if (lane < CAP) s_hist[lane] = 0;
@@ -331,9 +408,19 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
                     todo &= ~m;
                 }
             }
-            if (valid) ws.rank[(int64_t)j * samples + t] = rank;
+            if (ONE == ONE_OFF && valid) ws.rank[(int64_t)j * samples + t] = rank;
             __builtin_amdgcn_wave_barrier();
-            if (lane < experts) {
+            if constexpr (ONE != ONE_OFF) {
+                const int l = rank + __shfl(before, max(best, 0));
+                if (valid && first) locations[(int64_t)j * stride + t] = l;
+                if constexpr (ONE > 0) { if (tid < GROUP) s_slot[j][tid] = valid && l < capacity ? best * capacity + l : -1; }
+                const int n = lane < experts ? s_hist[lane] : 0;
+                before += n;
+                if (lane < experts && first) {
+                    if (counts_out) counts_out[j * experts + lane] = n;
+                    if (j == 0 && l_aux) s_me[1][lane] = s_me[0][lane] * ((float)n * ((float)experts / (float)samples));
+                }
+            } else if (lane < experts) {
                 ws.hist[((int64_t)blockIdx.x * k + j) * experts + lane] = s_hist[lane];
                 int32_t *col = ws.hist_t + ((int64_t)j * experts + lane) * ws.gstride;
                 col[blockIdx.x] = s_hist[lane];
@@ -342,6 +429,37 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
             }
             __builtin_amdgcn_wave_barrier();
         }
+        if (ONE != ONE_OFF && l_aux && first && lane == 0) {
+            float a = 0.f;
+            for (int e = 0; e < experts; ++e) a += s_me[1][e];
+            *l_aux = a / (float)samples;
+        }
+    }
+    if constexpr (ONE > 0) {
+        static_assert(MODE == 0, "rows to send");
+        using E = Elem<DT>;
+        __syncthreads();
+        const int t = (int)blockIdx.x * 4 + wave, units = model_dim / E::VEC;
+        if (t >= samples) return;
+        const int slot = lane < k ? s_slot[lane % 4][t] : -1;
+        if (__ballot(slot >= 0) == 0) return;
+        const uint4 *src = reinterpret_cast<const uint4 *>(x) + (int64_t)t * units;
+        auto each = [&](auto f) {
+#pragma unroll 4
+            for (int u = lane; u < units; u += WAVE) f(u, src[u]);
+        };
+        float mn = 0.f, mx = 0.f;
+        if constexpr (ONE == OUT_DECODED) {
+            if constexpr (STATS) {
+                mn = s_range[t][0]; mx = s_range[t][1];
+            } else {
+                RowStats<DT, true> stats;
+                stats.init();
+                for (int u = lane; u < units; u += WAVE) stats.add(src[u]);
+                stats.finish(mn, mx);
+            }
+        }
+        send_row<DT, ONE>(each, slot, k, units, rows, nullptr, nullptr, mn, mx);
     }
 }
 
@@ -480,12 +598,6 @@ __global__ __launch_bounds__(256) void route_locations_merged_kernel(
 // none of its choices leaves without reading its row.  Pays when many tokens are dropped (a
 // capacity factor of 1 with skewed routing drops half of them); otherwise the row is requested
 // first so that it travels while the slots are being worked out.
-// OUT: what a kept row arrives as.  CODES: codes with bias and scale.  ROWS: no codec -- `codes` is the
-// dispatched buffer in x's dtype and a kept row arrives there as 0 + x (what fast_encode's accumulation
-// into zeros leaves: -0 becomes +0), an empty slot as zeros.  DECODED: the same buffer with what the
-// decompressor makes of the row's codes (the codes stay in registers: one pass where dispatch + int8
-// and the decompressor write and read them).
-enum { OUT_CODES = 0, OUT_ROWS = 1, OUT_DECODED = 2 };
 template <int DT, int CACHE, bool MERGED, bool SLOT_FIRST = false, int OUT = OUT_CODES>
 __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
     const void *__restrict__ x, const int32_t *__restrict__ indices, int32_t *__restrict__ locations,
@@ -604,90 +716,55 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
         if (__ballot(slot >= 0) == 0) return;
     }
 
-    if constexpr (OUT == OUT_ROWS) {
-        auto copy = [&](int u, const uint4 &raw) {
-            float f[V];
-            E::unpack(raw, f);
-#pragma unroll
-            for (int i = 0; i < V; ++i) f[i] = 0.f + f[i];
-            const uint4 v = E::pack(f);
-            for (int j = 0; j < top_k; ++j) {
-                const int sl = rl_i(slot, j);
-                if (sl >= 0) stream_store(reinterpret_cast<uint4 *>(codes + (int64_t)sl * units * 16) + u, v);
-            }
-        };
+    auto each = [&](auto f) {
         if constexpr (CACHE > 0) {
 #pragma unroll
-            for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) copy(c * WAVE + lane, cache[c]);
+            for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) f(c * WAVE + lane, cache[c]);
         } else {
-            for (int u = lane; u < units; u += WAVE) copy(u, src[u]);
-        }
-        return;
-    }
-
-    float mn, mx;
-    if (row_min) {                                      // the gate kernel already scanned the row
-        mn = row_min[t]; mx = row_max[t];
-    } else {
-        RowStats<DT, true> stats;
-        stats.init();
-        if constexpr (CACHE > 0) {
-#pragma unroll
-            for (int c = 0; c < CACHE; ++c) stats.add(cache[c]);
-        } else {
-            for (int u = lane; u < units; u += WAVE) stats.add(src[u]);
-        }
-        stats.finish(mn, mx);
-    }
-    const float scale = E::round(mx - mn);
-    if constexpr (OUT == OUT_CODES) {
-        if (slot >= 0) { E::store(bias_out, slot, mn); E::store(scale_out, slot, scale); }
-    }
-    const RowEncoder<DT> enc(mn, scale);
-    const RowDecoder<DT> dec(mn, scale);
-
-    auto body = [&](auto mode) {
-        auto emit = [&](int u, const uint4 &raw) {
-            uint32_t w[2];
-            enc.template encode<decltype(mode)::value>(raw, w);
-            if constexpr (OUT == OUT_DECODED) {
-                float f[V];
-#pragma unroll
-                for (int q = 0; q < V / 4; ++q) dec.word(w[q], f + 4 * q);
-                const uint4 v = E::pack(f);
-                for (int j = 0; j < top_k; ++j) {
-                    const int s = rl_i(slot, j);
-                    if (s >= 0) stream_store(reinterpret_cast<uint4 *>(codes + (int64_t)s * units * 16) + u, v);
-                }
-                return;
-            }
-            for (int j = 0; j < top_k; ++j) {
-                const int s = rl_i(slot, j);
-                if (s < 0) continue;
-                uint8_t *row = codes + (int64_t)s * model_dim;
-                if constexpr (V == 8) stream_store(reinterpret_cast<uint2 *>(row) + u, make_uint2(w[0], w[1]));
-                else stream_store(reinterpret_cast<uint32_t *>(row) + u, w[0]);
-            }
-        };
-        if constexpr (CACHE > 0) {
-#pragma unroll
-            for (int c = 0; c < CACHE; ++c) if (c * WAVE + lane < units) emit(c * WAVE + lane, cache[c]);
-        } else {
-            for (int u = lane; u < units; u += WAVE) emit(u, src[u]);
+            for (int u = lane; u < units; u += WAVE) f(u, src[u]);
         }
     };
-    if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
+    float mn = 0.f, mx = 0.f;
+    if constexpr (OUT != OUT_ROWS) {
+        if (row_min) {                                  // the gate kernel already scanned the row
+            mn = row_min[t]; mx = row_max[t];
+        } else {
+            RowStats<DT, true> stats;
+            stats.init();
+            if constexpr (CACHE > 0) {
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) stats.add(cache[c]);
+            } else {
+                for (int u = lane; u < units; u += WAVE) stats.add(src[u]);
+            }
+            stats.finish(mn, mx);
+        }
+    }
+    send_row<DT, OUT>(each, slot, top_k, units, codes, bias_out, scale_out, mn, mx);
 }
 
 template <int DT, int SDT>
 static void launch_gate_route(int experts, int groups, int group_tokens, hipStream_t st, const void *x, const void *wg,
                               const float *bias, int samples, int model_dim, int k, int normalize,
                               int32_t *indices, int32_t *locations, void *gates, int64_t stride,
-                              void *logits_out, void *scores_out, float *l_aux, int32_t *counts, void *ws)
+                              void *logits_out, void *scores_out, float *l_aux, int32_t *counts, void *ws, int one, void *rows, int capacity)
 {
+#define PM_GR_1(CAP, ONE, WGS)                                                                           \
+    gate_route_kernel<DT, SDT, 1, CAP, true, 32, 0, ONE><<<WGS, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
+        k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws, (uint8_t *)rows, capacity)
+#define PM_GR_ONE(CAP) do { if (one == OUT_ROWS) PM_GR_1(CAP, OUT_ROWS, (samples + 3) / 4);              \
+                            else if (one == OUT_DECODED) PM_GR_1(CAP, OUT_DECODED, (samples + 3) / 4); else PM_GR_1(CAP, ONE_ROUTING, 1); } while (0)
+    if constexpr (DT != PLANMOE_F16) {
+        if (one != ONE_OFF) {
+            if (experts <= 8) PM_GR_ONE(8); else PM_GR_ONE(16);
+            return;
+        }
+    }
+#undef PM_GR_1
+#undef PM_GR_ONE
 #define PM_GR_(NT, CAP, SPLITK, GROUP)                                                                   \
     gate_route_kernel<DT, SDT, NT, CAP, SPLITK, GROUP><<<groups, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
-        k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws)
+        k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws, nullptr, 0)
 #define PM_GR(NT, CAP, SPLITK) do { if (SPLITK && group_tokens == 32) PM_GR_(NT, CAP, SPLITK, (SPLITK ? 32 : 64)); \
                                     else PM_GR_(NT, CAP, SPLITK, 64); } while (0)
     // split-K measured faster than the LDS-shared variant up to 16 experts (30.7 vs 44.4 us at
@@ -750,6 +827,7 @@ static int fused_check(const char *who, const void *x, const void *wg, int dtype
 struct FwdPlan {
     int k, groups, group_tokens, experts_per_block, blocks;
     bool merged;          // the dispatch launch does the prefix over groups itself
+    bool one;             // one group: the gate kernel's slots can be the final ones
     FwdWs ws;
 };
 static void fwd_plan(FwdPlan &plan, void *workspace, int samples, int experts, int top_k)
@@ -760,6 +838,7 @@ static void fwd_plan(FwdPlan &plan, void *workspace, int samples, int experts, i
     plan.experts_per_block = go_experts_per_block(experts, plan.k);
     plan.blocks = (experts + plan.experts_per_block - 1) / plan.experts_per_block;
     plan.merged = plan.k <= 4;
+    plan.one = plan.groups == 1 && plan.merged && plan.group_tokens == 32;
     plan.ws = fwd_ws(workspace, plan.groups, plan.k, experts, samples);
 }
 
@@ -788,14 +867,14 @@ static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t 
 
 // stand-alone routing from logits / scores in memory: the epilogue of gate_route_kernel on 64-token
 // groups, then the prefix over the groups and the final slots
-template <int SDT>
+template <int SDT, int ONE>
 static void launch_route_groups(int experts, int groups, int mode, hipStream_t st, const void *input, const float *bias,
                                 int samples, int k, int normalize, int32_t *indices, int32_t *locations, void *gates,
                                 int64_t stride, void *scores_out, float *l_aux, int32_t *counts, void *ws)
 {
 #define PM_RG_(NT, CAP, MODE)                                                                              \
-    gate_route_kernel<SDT, SDT, NT, CAP, false, 64, MODE><<<groups, 256, 0, st>>>(input, nullptr, bias, samples, 0, \
-        experts, k, normalize, indices, locations, gates, stride, nullptr, scores_out, l_aux, counts, ws)
+    gate_route_kernel<SDT, SDT, NT, CAP, false, 64, MODE, ONE><<<groups, 256, 0, st>>>(input, nullptr, bias, samples, 0, \
+        experts, k, normalize, indices, locations, gates, stride, nullptr, scores_out, l_aux, counts, ws, nullptr, 0)
 #define PM_RG(NT, CAP) do { if (mode == 1) PM_RG_(NT, CAP, 1); else PM_RG_(NT, CAP, 2); } while (0)
     if (experts <= 8) PM_RG(1, 8);
     else if (experts <= 16) PM_RG(1, 16);
@@ -819,9 +898,14 @@ int route_groups(const void *input, int dtype, int is_logits, const float *logit
     workspace = fwd_tables(workspace);
     plan.ws = fwd_ws(workspace, plan.groups, plan.k, experts, samples);
     const int mode = is_logits ? 1 : 2;
-    PM_DTYPE_SWITCH(dtype, SDT, (launch_route_groups<SDT>(experts, plan.groups, mode, st, input, is_logits ? logit_bias : nullptr,
-                                                         samples, plan.k, normalize_gate, indices, locations, gates, stride,
-                                                         is_logits ? scores_out : nullptr, l_aux, counts, workspace)));
+#define PM_ROUTE(ONE) PM_DTYPE_SWITCH(dtype, SDT, (launch_route_groups<SDT, ONE>(experts, plan.groups, mode, st, input, is_logits ? logit_bias : nullptr, \
+                          samples, plan.k, normalize_gate, indices, locations, gates, stride, is_logits ? scores_out : nullptr, l_aux, counts, workspace)))
+    if (plan.groups == 1) {                      // (its slots are the final ones)
+        PM_ROUTE(ONE_ROUTING);
+        return 0;
+    }
+    PM_ROUTE(ONE_OFF);
+#undef PM_ROUTE
     finish_routing(plan, indices, locations, stride, samples, experts, l_aux, counts, st);
     return 0;
 }
@@ -832,22 +916,22 @@ static int run_gate_route(const void *x, const void *wg, int dtype, int fp32_gat
                           int normalize_gate, int32_t *indices, int32_t *locations, void *gates,
                           int64_t stride, void *logits_out, void *scores_out, float *l_aux,
                           int32_t *counts, void *workspace, hipStream_t st, FwdPlan &plan,
-                          bool offsets_follow)
+                          bool offsets_follow, int one = ONE_OFF, void *rows = nullptr, int capacity = 0)
 {
     fwd_plan(plan, workspace, samples, experts, top_k);
     const int k = plan.k, groups = plan.groups;
     if (fp32_gate || dtype == PLANMOE_F32) {
         PM_DTYPE_SWITCH(dtype, DT, (launch_gate_route<DT, PLANMOE_F32>(
             experts, groups, plan.group_tokens, st, x, wg, logit_bias, samples, model_dim, k, normalize_gate, indices,
-            locations, gates, stride, logits_out, scores_out, l_aux, counts, workspace)));
+            locations, gates, stride, logits_out, scores_out, l_aux, counts, workspace, one, rows, capacity)));
     } else if (dtype == PLANMOE_BF16) {
         launch_gate_route<PLANMOE_BF16, PLANMOE_BF16>(experts, groups, plan.group_tokens, st, x, wg, logit_bias, samples,
             model_dim, k, normalize_gate, indices, locations, gates, stride, logits_out, scores_out,
-            l_aux, counts, workspace);
+            l_aux, counts, workspace, one, rows, capacity);
     } else {
         launch_gate_route<PLANMOE_F16, PLANMOE_F16>(experts, groups, plan.group_tokens, st, x, wg, logit_bias, samples,
             model_dim, k, normalize_gate, indices, locations, gates, stride, logits_out, scores_out,
-            l_aux, counts, workspace);
+            l_aux, counts, workspace, one, rows, capacity);
     }
     if (offsets_follow)
         group_offsets_kernel<<<plan.blocks, 256, 0, st>>>(plan.ws.hist, plan.ws.offs, plan.ws.me, groups, k,
@@ -1017,10 +1101,12 @@ extern "C" int planmoe_gate_route(const void *x, const void *wg, int dtype, int 
     workspace = fwd_tables(workspace);
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
+    fwd_plan(plan, workspace, samples, experts, top_k);
+    const bool one = plan.one && dtype != PLANMOE_F16;
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k,
                        normalize_gate, indices, locations, gates, plane_stride, logits_out, scores_out,
-                       l_aux, expert_counts, workspace, st, plan, false)) return 1;
-    finish_routing(plan, indices, locations, plane_stride, samples, experts, l_aux, expert_counts, st);
+                       l_aux, expert_counts, workspace, st, plan, false, one ? ONE_ROUTING : ONE_OFF)) return 1;
+    if (!one) finish_routing(plan, indices, locations, plane_stride, samples, experts, l_aux, expert_counts, st);
     PM_LAUNCH_CHECK("planmoe_gate_route");
     return 0;
 }
@@ -1101,12 +1187,13 @@ extern "C" int planmoe_layer_dispatch(const void *x, const void *wg, int dtype, 
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
     fwd_plan(plan, workspace, samples, experts, top_k);
+    const int out = codec ? OUT_DECODED : OUT_ROWS;
+    const bool one = plan.one && dtype != PLANMOE_F16;
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k, normalize_gate, indices,
                        locations, gates, plane_stride, nullptr, scores_out, l_aux, expert_counts, workspace, st, plan,
-                       !plan.merged)) return 1;
-    if (run_dispatch_routed(x, dtype, samples, model_dim, experts, capacity, indices, locations, plane_stride, l_aux,
-                            expert_counts, (uint8_t *)rows, nullptr, nullptr, plan, st, codec ? OUT_DECODED : OUT_ROWS,
-                            false)) return 1;
+                       !plan.merged, one ? out : ONE_OFF, rows, capacity)) return 1;
+    if (!one && run_dispatch_routed(x, dtype, samples, model_dim, experts, capacity, indices, locations, plane_stride, l_aux,
+                            expert_counts, (uint8_t *)rows, nullptr, nullptr, plan, st, out, false)) return 1;
     PM_LAUNCH_CHECK(who);
     return 0;
 }

@@ -436,3 +436,43 @@ def test_layer_zfp_dispatch_and_combine_backward_equal_the_steps(T, M, E, k, cap
         n = (n + 3) // 4 * 4
         assert torch.equal(rows[e, :n], want[e, :n]) and bool((rows[e, n:] == 7.0).all()), e
         assert torch.equal(grad_rows[e, :n], want_rows[e, :n]) and bool((grad_rows[e, n:] == 7.0).all()), e
+
+
+# up to 32 tokens and 16 experts the gate, the routing and the rows are one launch (33 tokens, 17 experts: two): the same bits as the
+# chain of two launches.  Work-groups of four tokens, rows of one vector and of no whole number of a wave's, capacities that drop choices
+@pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 1, 1, 4), (3, 64, 4, 2, 4), (4, 1032, 8, 4, 2), (5, 520, 9, 3, 4), (31, 256, 16, 2, 4),
+                                         (32, 2048, 8, 2, 12), (32, 64, 2, 2, 8), (33, 256, 16, 2, 4), (8, 64, 17, 1, 4)])
+@pytest.mark.parametrize("codec", [0, 1])
+@pytest.mark.parametrize("dtype,fp32_gate", [(torch.bfloat16, True), (torch.bfloat16, False), (torch.float32, True), (torch.float16, True)])
+def test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec, dtype, fp32_gate):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", T, M, E, k, cap, codec, dtype, fp32_gate, flush=True)
+    g = torch.Generator().manual_seed(T + M + E)
+    x, wg = torch.randn(T, M, generator=g).to(dtype).to(DEV), (torch.randn(E, M, generator=g) * M ** -0.5).to(dtype).to(DEV)
+    x[T // 2] = 0.5                              # (a row of one value: no scale)
+    x[0, 0] = -0.0
+    kw = dict(fp32_gate=fp32_gate, want_scores=True, want_counts=True)
+    if codec:
+        want = ops.forward_int8(x, wg, k, cap, **kw)
+        want["rows"] = ops.int8_decompress(want["codes"], want["bias"], want["scale"])
+    else:
+        want = ops.forward_plain(x, wg, k, cap, **kw)
+        want["rows"] = want["dispatched"]
+    score = torch.float32 if fp32_gate else dtype
+    idx, loc, counts = (torch.full(s, -7, dtype=torch.int32, device=DEV) for s in ((k, T), (k, T), (k, E)))
+    gates, scores = torch.full((k, T), 7.0, dtype=score, device=DEV), torch.full((T, E), 7.0, dtype=score, device=DEV)
+    l_aux, rows = torch.full((), 7.0, device=DEV), torch.full((E * cap, M), 7.0, dtype=dtype, device=DEV)
+    ws = torch.empty(lib.planmoe_forward_workspace_bytes(T, E, k), dtype=torch.uint8, device=DEV).fill_(0x7f)
+    check(lib.planmoe_layer_dispatch(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), int(fp32_gate), None, T, M, E, k, 1, cap, codec, ops._ptr(idx),
+                                     ops._ptr(loc), ops._ptr(gates), T, ops._ptr(scores), ops._ptr(l_aux), ops._ptr(counts), ops._ptr(rows),
+                                     ops._ptr(ws), ws.numel(), ops._stream(x)))
+    alone = ops.gate_route(x, wg, k, **kw)
+    torch.cuda.synchronize()
+    for name, got in (("indices", idx), ("locations", loc), ("gates", gates), ("scores", scores), ("counts", counts), ("l_aux", l_aux)):
+        assert torch.equal(got, want[name].view(got.shape)), name
+        assert torch.equal(alone[name].view(got.shape), got), name
+    used = torch.zeros(E * cap, dtype=torch.bool, device=DEV)
+    used[(idx.long() * cap + loc)[loc < cap]] = True
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    assert torch.equal(rows[used].view(bits), want["rows"].view(E * cap, M)[used].view(bits)) and bool((rows[~used] == 7.0).all())
