@@ -147,6 +147,47 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     return p;
 }
 
+// A pass that nothing is kept of: what only its launches see lies in one buffer (eight allocations take the host 9 us, a third
+// of a decode step's time, three 3).  The lz codec has its own buffers.
+std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2,
+                                          const Shape &s, bool fp32_gate, bool normalize, int codec)
+{
+    void *st = current_stream();
+    const int64_t size = x.element_size();
+    int64_t end = 0;
+    auto piece = [&](int64_t n) { const int64_t at = end; end += (n + 255) / 256 * 256; return at; };
+    const bool bf16_gate = !fp32_gate && s.dt != PLANMOE_F32;
+    const size_t ws_bytes = std::max(planmoe_forward_workspace_bytes(s.T, s.E, s.k), codec == CODEC_ZFP ? planmoe_layer_zfp_workspace_bytes(s.E, s.cap) : 0);
+    const int64_t idx_at = piece((int64_t)s.k * s.T * 4), loc_at = piece((int64_t)s.k * s.T * 4), cnt_at = piece((int64_t)s.k * s.E * 4),
+                  gates_at = piece((int64_t)s.k * s.T * (bf16_gate ? size : 4)), wide_at = bf16_gate ? piece((int64_t)s.k * s.T * 4) : 0,
+                  ws_at = piece((int64_t)ws_bytes), xe_at = piece(s.rows() * s.M * size), h_at = piece(s.rows() * s.H * size), ye_at = piece(s.rows() * s.M * size);
+    const Tensor pool = bytes(end, x);
+    uint8_t *const base = pool.data_ptr<uint8_t>();
+    int32_t *const idx = (int32_t *)(base + idx_at), *const loc = (int32_t *)(base + loc_at), *const cnt = (int32_t *)(base + cnt_at);
+    void *const ws = base + ws_at, *const xe = base + xe_at, *const h = base + h_at, *const ye = base + ye_at;
+    const float *gates = (const float *)(base + gates_at);
+    Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat)), y = at::empty({s.T, s.M}, x.options());
+    if (codec == CODEC_ZFP) {
+        PM_CALL(planmoe_gate_route(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, idx, loc, base + gates_at, s.T, nullptr,
+                                   nullptr, l_aux.data_ptr<float>(), cnt, ws, ws_bytes, st));
+        PM_CALL(planmoe_layer_zfp_dispatch(floats(x), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt, (float *)xe, ws, ws_bytes, st));
+    } else {
+        PM_CALL(planmoe_layer_dispatch(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, codec, idx, loc,
+                                       base + gates_at, s.T, nullptr, l_aux.data_ptr<float>(), cnt, xe, ws, ws_bytes, st));
+    }
+    if (bf16_gate) {
+        at::from_blob(base + wide_at, {s.k, s.T}, x.options().dtype(at::kFloat)).copy_(at::from_blob(base + gates_at, {s.k, s.T}, x.options()));
+        gates = (const float *)(base + wide_at);
+    }
+    const int round = codec == CODEC_ZFP ? 4 : 1;
+    // (which elements a relu cut is asked by a backward pass only)
+    PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 2, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
+    PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, round, s.hint(), ye, st));
+    if (codec == CODEC_ZFP) PM_CALL(planmoe_layer_zfp_rows((float *)ye, s.M, s.E, s.cap, cnt, s.k, nullptr, 0, st));
+    PM_CALL(planmoe_layer_combine(ye, s.dt, codec == CODEC_INT8, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));
+    return {y, l_aux};
+}
+
 Shape shape_of(const Tensor &x, const Tensor &wg, const Tensor &w1, int64_t k, int64_t cap)
 {
     Shape s;
@@ -312,6 +353,7 @@ std::tuple<Tensor, Tensor> ffn_layer(const Tensor &x, const Tensor &wg, const Te
     for (const Tensor *t : {&x, &wg, &w1, &b1, &w2, &b2}) grad |= (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined();
     if (!grad) {
         const at::NoGradGuard no_grad;
+        if (codec != CODEC_LZ) return inference_pass(x, wg, w1, b1, w2, b2, shape_of(x, wg, w1, k, cap), fp32_gate, normalize, (int)codec);
         Pass p = forward_pass(x, wg, w1, b1, w2, b2, shape_of(x, wg, w1, k, cap), fp32_gate, normalize, (int)codec, false);
         return {p.y, p.l_aux};
     }

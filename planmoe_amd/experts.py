@@ -133,7 +133,7 @@ class FusedExpertsNetwork(torch.nn.Module):
             y = self.activation_fn(y)
         return self._linear(y, self.batched_fc2_w, self.batched_fc2_bias, False)
 
-    _own_forward, _own_linear = forward, _linear        # (as defined here: overlap.native_codec asks whether they still are)
+    _own_forward, _own_linear = forward, _linear        # (as defined here: overlap.native_call asks whether they still are)
 
     def forward_from_codes(self, codes, bias, scale, exact=True):
         """The same forward with the int8 codes of the receive buffer as input (inference: no autograd

@@ -32,6 +32,15 @@ def _env_flag(name):
     return int(os.environ.get(name, '0')) != 0
 
 
+def _first_parameter(module):
+    """next(module.parameters(), None), without the walk where the module holds parameters itself."""
+    if type(module).__dict__.get('parameters') is None and isinstance(module, torch.nn.Module) and 'parameters' not in module.__dict__:
+        for p in module._parameters.values():
+            if p is not None:
+                return p
+    return next(module.parameters(), None)
+
+
 class MOELayer(torch.nn.Module):
     # ------------------------------------------------------------------ construction
     @staticmethod
@@ -150,7 +159,7 @@ class MOELayer(torch.nn.Module):
         self.protected_shape = y.shape
         return y.reshape(y.size(0), y.size(1), -1)
 
-    _own_expert_local = expert_local            # (as defined here: overlap.native_codec asks whether it still is)
+    _own_expert_local = expert_local            # (as defined here: overlap.native_call asks whether it still is)
 
     # ------------------------------------------------------------------ forward
     def _deliver(self, y, l_aux, shape, dtype):
@@ -172,11 +181,11 @@ class MOELayer(torch.nn.Module):
         assert len(shape) >= 2, "Input data must be at least 2D tensor: (s)amples, .., (m)odel_dim"
         reserve_shape = shape[-reserve_dims:]
         x = input if len(shape) == 2 and reserve_dims == 1 else input.reshape(-1, reserve_shape.numel())
-        first = next(self.experts.parameters(), None)
+        first = _first_parameter(_overlap.held(self, 'experts'))
         if first is not None and x.dtype != first.dtype:
             x = x.to(first.dtype)
 
-        gate = self.gates[gate_index]
+        gate = _overlap.held(self, 'gates')[gate_index]
         E = self.num_global_experts
         degree = self.a2a_ffn_overlap_degree if a2a_ffn_overlap_degree is None else a2a_ffn_overlap_degree
         k = gate.top_k if top_k is None else top_k
@@ -185,6 +194,19 @@ class MOELayer(torch.nn.Module):
         noisy = self.training and gate.gate_noise > 0
         # "plain" routing: what the routing kernels cover (GShard loss, token order, static capacity)
         plain = self.is_gshard_loss and not self.batch_prioritized_routing and cf > 0
+
+        if plain and not noisy:
+            kk = min(k, E)
+            cap = ops.capacity(x.size(0), E, kk, cf, alignment)
+            loss_dtype = torch.float32 if getattr(gate, 'fp32_gate', False) else x.dtype
+            call = _overlap.native_call(self, gate, x, degree, reserve_dims, cap)
+            if call is not None:
+                # built-in gate and experts: the whole pass as one call and one node of the graph
+                if self.training:
+                    self.save_count = self.save_count + 1
+                y, l_aux = _ext.layer().ffn_layer(x.contiguous(), *call[1:], kk, cap, bool(gate.fp32_gate), bool(self.normalize_gate), call[0])
+                self.protected_shape = torch.Size((E, cap, x.shape[1]))
+                return self._deliver(y, l_aux if l_aux.dtype == loss_dtype else l_aux.to(loss_dtype), shape, dtype)
 
         def expert_fn(expert_input):
             return self.expert_local(expert_input, reserve_shape)
@@ -200,19 +222,6 @@ class MOELayer(torch.nn.Module):
                                                     compress_name=self.compress_name, comm_name=self.comm_name)
 
         if plain and not noisy:
-            kk = min(k, E)
-            cap = ops.capacity(x.size(0), E, kk, cf, alignment)
-            loss_dtype = torch.float32 if getattr(gate, 'fp32_gate', False) else x.dtype
-            codec = _overlap.native_codec(self, gate, x, degree, reserve_dims, cap)
-            if codec is not None:
-                # built-in gate and experts: the whole pass as one call and one node of the graph
-                count_step()
-                experts = self.experts
-                y, l_aux = _ext.layer().ffn_layer(x.contiguous(), gate.wg.weight, experts.batched_fc1_w, experts.batched_fc1_bias,
-                                                  experts.batched_fc2_w, experts.batched_fc2_bias, kk, cap, bool(gate.fp32_gate),
-                                                  bool(self.normalize_gate), codec)
-                self.protected_shape = torch.Size((E, cap, x.shape[1]))
-                return self._deliver(y, l_aux if l_aux.dtype == loss_dtype else l_aux.to(loss_dtype), shape, dtype)
             if _overlap.FUSE_GATE and _overlap.fused_gate_eligible(x, gate, E, self.compress_name, degree,
                                                                    self.is_postscore):
                 # gate GEMM, routing, encode and compress as one call; decompress + decode in one pass

@@ -68,6 +68,13 @@ def planes(tensors, dtype):
 
 # ------------------------------------------------------------------------------ routing
 def capacity(samples, experts, top_k, capacity_factor=1.0, alignment=1):
+    """planmoe_capacity, worked out here (a call of the library takes 1.5 us of every layer call); the library is asked
+    about what it may refuse."""
+    if samples >= 0 and experts >= 1 and top_k >= 1 and 0 < capacity_factor < 1 << 30 and alignment >= 1:
+        out = min(top_k, experts) * int(float(capacity_factor) * -(-samples // experts))
+        out += -out % alignment
+        if out < 1 << 31:
+            return out
     out = ctypes.c_int(0)
     check(lib.planmoe_capacity(samples, experts, top_k, float(capacity_factor), int(alignment),
                                ctypes.byref(out)))

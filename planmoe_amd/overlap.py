@@ -152,7 +152,8 @@ _NATIVE_CODECS = {'int8': 1, 'zfp': 2, 'lz': 3}
 
 
 def _hooked(module):
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+    own = module.__dict__
+    return bool(own['_forward_hooks'] or own['_forward_pre_hooks'] or own['_backward_hooks'] or own['_backward_pre_hooks'])
 
 
 def _replaced(layer, experts):
@@ -163,12 +164,24 @@ def _replaced(layer, experts):
             inner._linear is not inner._own_linear or 'expert_local' in own or 'forward' in theirs or '_linear' in theirs)
 
 
-def native_codec(layer, gate, x, degree, reserve_dims, capacity):
-    """The codec number for csrc/ext/layer.cpp when the whole layer is its business, else None.  What is left to
-    the steps below: experts or gates that are not the built-in ones or carry hooks, replaced methods, other dtypes (a
-    gate in fp32 next to 16-bit rows among them), overlap slices, autocast, every option that asks for the
-    reference's structure, and weights that are not 16-byte aligned (views of a flat buffer: the steps copy them)."""
-    experts = layer.experts
+def held(module, name):
+    """module.name for a parameter or submodule, without nn.Module's search for it (0.1 us instead of 0.6)."""
+    own = module.__dict__
+    if name in own:
+        return own[name]
+    value = own['_parameters'].get(name)
+    if value is None:
+        value = own['_modules'].get(name)
+    return getattr(module, name) if value is None else value
+
+
+def native_call(layer, gate, x, degree, reserve_dims, capacity):
+    """(codec number, gate weight, fc1 weight, bias, fc2 weight, bias) for csrc/ext/layer.cpp when the whole layer is its business,
+    else None.  What is left to the steps below: experts or gates that are not the built-in ones or carry hooks,
+    replaced methods, other dtypes (a gate in fp32 next to 16-bit rows among them), overlap slices, autocast, every
+    option that asks for the reference's structure, and weights that are not 16-byte aligned (views of a flat buffer: the steps
+    copy them)."""
+    experts = held(layer, 'experts')
     if not (NATIVE_LAYER and FUSE_GATE and FUSE_INT8 and FUSE_ZFP and not FFN_FROM_CODES and not _ck.SINGLE_RANK_COMM_COPIES and
             degree == 1 and reserve_dims == 1 and layer.is_postscore and x.is_cuda and capacity >= 1 and x.shape[0] >= 1 and
             type(experts) is FusedExpertsNetwork and experts._relu and type(gate) is LinearTopKGate and
@@ -179,20 +192,28 @@ def native_codec(layer, gate, x, degree, reserve_dims, capacity):
     if not ((dtype == torch.bfloat16 or dtype == torch.float32) and M % vec == 0 and H % vec == 0 and M <= 1024 * vec and
             row_fits(H, dtype) and experts.output_dim in (None, M)):
         return None
-    w1, w2 = experts.batched_fc1_w, experts.batched_fc2_w
-    for p in (gate.wg.weight, w1, experts.batched_fc1_bias, w2, experts.batched_fc2_bias):
+    wg = held(gate, 'wg')
+    weights = (held(wg, 'weight'), held(experts, 'batched_fc1_w'), held(experts, 'batched_fc1_bias'), held(experts, 'batched_fc2_w'),
+               held(experts, 'batched_fc2_bias'))
+    for p in weights:
         if p.dtype != dtype or not p.is_contiguous():
             return None
-    if (w1.data_ptr() | w2.data_ptr()) % 16:
+    if (weights[1].data_ptr() | weights[3].data_ptr()) % 16:
         return None
-    if _hooked(experts) or _hooked(gate) or _hooked(gate.wg) or _has_any_global_hook() or torch.is_autocast_enabled(x.device.type):
+    if _hooked(experts) or _hooked(gate) or _hooked(wg) or _has_any_global_hook() or torch.is_autocast_enabled('cuda'):
         return None
     codec = _NATIVE_CODECS.get(layer.compress_name, 0)
     if codec == 2 and not fused_zfp_eligible(x, 'zfp', degree, True, layer.num_global_experts, capacity):
         return None
     if codec == 3 and (dtype != torch.float32 or 'lz' in _ck.registered()):
         return None
-    return codec
+    return (codec, *weights)
+
+
+def native_codec(layer, gate, x, degree, reserve_dims, capacity):
+    """The codec number of native_call, or None."""
+    call = native_call(layer, gate, x, degree, reserve_dims, capacity)
+    return None if call is None else call[0]
 
 
 class _GaveUp:

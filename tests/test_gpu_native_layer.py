@@ -476,3 +476,22 @@ def test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec
     used[(idx.long() * cap + loc)[loc < cap]] = True
     bits = torch.int32 if dtype == torch.float32 else torch.int16
     assert torch.equal(rows[used].view(bits), want["rows"].view(E * cap, M)[used].view(bits)) and bool((rows[~used] == 7.0).all())
+
+
+# without autograd a pass lies in one buffer: the same bits as the pass that a backward pass may follow, gates in 16 bits among them
+@pytest.mark.parametrize("codec,dtype,fp32_gate", [("no", torch.bfloat16, True), ("no", torch.bfloat16, False), ("int8", torch.bfloat16, False),
+                                                   ("int8", torch.float32, True), ("zfp", torch.float32, True), ("no", torch.float32, False)])
+@pytest.mark.parametrize("T,k", [(1, 1), (19, 2), (300, 3)])
+def test_inference_equals_the_pass_with_autograd(codec, dtype, fp32_gate, T, k):
+    import planmoe_amd
+    torch.manual_seed(T)
+    layer = planmoe_amd.moe_layer({"type": "top", "k": k, "capacity_factor": 1.1, "fp32_gate": fp32_gate}, 136,
+                                  experts={"type": "ffn", "count_per_node": 4, "hidden_size_per_expert": 200}, compress_name=codec).to(DEV).to(dtype)
+    x = torch.randn(T, 136, device=DEV).to(dtype)
+    want = layer(x)
+    with torch.no_grad():
+        got = [layer(x) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert want.requires_grad
+    for y in got:
+        assert torch.equal(y, want) and torch.equal(y.l_aux, want.l_aux) and y.l_aux.dtype == want.l_aux.dtype

@@ -189,3 +189,22 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode != 0
     assert "--gpus 2 is not supported" in (r.stderr + r.stdout)
+
+
+def test_capacity_is_the_librarys():
+    """ops.capacity works it out without the library: the same number over ordinary and odd arguments, the library's errors."""
+    import ctypes
+    import random
+    from planmoe_amd import ops
+    from planmoe_amd._lib import PlanMoEError, lib
+    rng = random.Random(5)
+    for _ in range(2000):
+        args = (rng.randrange(0, 1 << rng.randrange(1, 24)), rng.randrange(1, 70), rng.randrange(1, 80),
+                rng.choice([1.0, 1.1, 1.2, 1.25, 0.3, 2, rng.uniform(1e-9, 9.0)]), rng.choice([1, 4, 8, 12, 64]))
+        out = ctypes.c_int(0)
+        assert lib.planmoe_capacity(*args[:3], ctypes.c_double(args[3]), args[4], ctypes.byref(out)) == 0
+        assert ops.capacity(*args) == out.value, args
+    for args in ((-1, 4, 2, 1.0, 4), (8, 0, 2, 1.0, 4), (8, 4, 0, 1.0, 4), (8, 4, 2, 0.0, 4), (8, 4, 2, float("nan"), 4), (8, 4, 2, 1.0, 0),
+                 (1 << 30, 1, 1, 4.0, 1)):
+        with pytest.raises(PlanMoEError):
+            ops.capacity(*args)
