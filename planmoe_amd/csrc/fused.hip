@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_kernel(
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
     uint8_t *__restrict__ codes, void *__restrict__ bias_out, void *__restrict__ scale_out,
-    const uint32_t *__restrict__ flags, int token_blocks,
+    const SlotFill fill, int token_blocks,
     const void *__restrict__ other, float *__restrict__ grad_gates,
     const void *__restrict__ other_bias, const void *__restrict__ other_scale)
 {
@@ -32,23 +32,21 @@ __global__ __launch_bounds__(256) void dispatch_int8_kernel(
     const int units = model_dim / V;
     __shared__ float s_dtab[CODED ? 4 : 1][CODED ? 256 : 1];         // [wave][code]: decoded values of one row
 
-    if ((int)blockIdx.x >= token_blocks) {
+    const int number = fill.role((int)blockIdx.x, token_blocks);
+    if (number < 0) {
         // slots no live pair addresses: all-zero row -> codes 0, bias 0, scale 0
-        const int slots = experts * capacity;
-        const int nwaves = (gridDim.x - token_blocks) * 4;
-        for (int s = (blockIdx.x - token_blocks) * 4 + wave; s < slots; s += nwaves) {
-            if (flags[s]) continue;
+        fill_empty_slots(fill, ~number, indices, locations, stride, top_k, samples, experts, capacity, [&](int s) {
             uint8_t *row = codes + (int64_t)s * model_dim;
             for (int u = lane; u < units; u += WAVE) {
                 if constexpr (V == 8) stream_store(reinterpret_cast<uint2 *>(row) + u, make_uint2(0u, 0u));
                 else stream_store(reinterpret_cast<uint32_t *>(row) + u, 0u);
             }
             if (lane == 0) { E::store(bias_out, s, 0.f); E::store(scale_out, s, 0.f); }
-        }
+        });
         return;
     }
 
-    const int t = blockIdx.x * 4 + wave;
+    const int t = number * 4 + wave;
     if (t >= samples) return;
     const uint4 *src = reinterpret_cast<const uint4 *>((const char *)x + (int64_t)t * model_dim * (int64_t)sizeof(typename E::store_t));
 
@@ -370,12 +368,12 @@ static void launch_dispatch_int8(int per_lane, unsigned grid, hipStream_t st, co
                                  const float *gates, const int32_t *indices, const int32_t *locations,
                                  int64_t stride, int top_k, int samples, int model_dim, int experts,
                                  int capacity, uint8_t *codes, void *bias, void *scale,
-                                 const uint32_t *flags, int token_blocks, const void *other,
+                                 const SlotFill &fill, int token_blocks, const void *other,
                                  float *grad_gates, const void *other_bias, const void *other_scale)
 {
 #define PM_DI8_(CACHE, GATED, GRAD, CODED)                                                       \
     dispatch_int8_kernel<DT, CACHE, GATED, GRAD, CODED><<<grid, 256, 0, st>>>(x, gates, indices, locations, stride, \
-        top_k, samples, model_dim, experts, capacity, codes, bias, scale, flags, token_blocks,   \
+        top_k, samples, model_dim, experts, capacity, codes, bias, scale, fill, token_blocks,   \
         other, grad_gates, other_bias, other_scale)
 #define PM_DI8(CACHE)                                                                            \
     do {                                                                                         \
@@ -428,15 +426,13 @@ static int run_dispatch_int8(const char *who, const void *x, int dtype, const fl
                "%s: model_dim must be a multiple of %d and buffers 16-byte aligned; "
                "use the unfused entry points otherwise", who, vec);
     hipStream_t st = (hipStream_t)stream;
-    uint32_t *flags = (uint32_t *)workspace;
-    launch_slot_flags(flags, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
     const int token_blocks = (samples + 3) / 4;
-    const int fill_blocks = min((slots + 3) / 4, 2048);
     const int per_lane = (model_dim / vec + WAVE - 1) / WAVE;
     PM_DTYPE_SWITCH(dtype, DT,
-        launch_dispatch_int8<DT>(per_lane, (unsigned)(token_blocks + fill_blocks), st, x, gates, indices,
+        launch_dispatch_int8<DT>(per_lane, (unsigned)(token_blocks + fill.blocks), st, x, gates, indices,
                                  locations, plane_stride, top_k, samples, model_dim, experts, capacity,
-                                 codes, bias, scale, flags, token_blocks, other, grad_gates, other_bias, other_scale));
+                                 codes, bias, scale, fill, token_blocks, other, grad_gates, other_bias, other_scale));
     PM_LAUNCH_CHECK(who);
     return 0;
 }

@@ -98,10 +98,61 @@ __device__ __forceinline__ void fetch_planes(const float *gates, const int32_t *
     }
 }
 
-// occupancy flags of the experts*capacity slots (1 = some live pair addresses the slot)
-void launch_slot_flags(uint32_t *flags, const int32_t *indices, const int32_t *locations,
-                       int64_t stride, int top_k, int samples, int experts, int capacity,
-                       hipStream_t st);
+// Which slots no live pair addresses.  Up to SLOT_FILL_PAIRS pairs the work-groups that write those slots' zero rows find out
+// themselves: there are 2^shift of them, one in 2^shift slots is a work-group's, and it walks the routing planes and keeps a bit
+// a slot in LDS.  They are the first of the grid, so that the walk is beside the rows of the tokens.  (Two small launches in front for flags
+// in memory cost 9 us of 193 in the routing API's pass at 8192 x 2048, and 10 us of host time in any.)  More pairs: flags.
+constexpr int SLOT_FILL_PAIRS = 1 << 17, SLOT_FILL_BITS = 8192;
+struct SlotFill {
+    const uint32_t *flags;                       // NULL: bits in LDS
+    int blocks, shift;                           // work-groups that fill
+    // work-group b of the grid: below zero its number among those that fill is ~b, else its number among those of the tokens
+    __device__ __forceinline__ int role(int b, int token_blocks) const
+    {
+        if (flags) return b >= token_blocks ? ~(b - token_blocks) : b;
+        return b < blocks ? ~b : b - blocks;
+    }
+};
+// zero(slot) for every empty slot of work-group `number`, a wave each
+template <typename Zero>
+__device__ __forceinline__ void fill_empty_slots(const SlotFill &fill, int number, const int32_t *__restrict__ indices,
+                                                 const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples, int experts,
+                                                 int capacity, Zero zero)
+{
+    const int wave = threadIdx.x >> 6, slots = experts * capacity;
+    if (fill.flags) {
+        for (int s = number * 4 + wave; s < slots; s += fill.blocks * 4)
+            if (!fill.flags[s]) zero(s);
+        return;
+    }
+    __shared__ uint32_t s_used[SLOT_FILL_BITS / 32];
+    const int mine = (slots - number + (1 << fill.shift) - 1) >> fill.shift;          // slots number, number + 2^shift, ..
+    for (int i = threadIdx.x; i < (mine + 31) / 32; i += 256) s_used[i] = 0u;
+    __syncthreads();
+    for (int j = 0; j < top_k; ++j) {
+        const int32_t *idx = indices + (int64_t)j * stride, *loc = locations + (int64_t)j * stride;
+        for (int t0 = threadIdx.x; t0 < samples; t0 += 8 * 256) {
+            int e[8], l[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int t = min(t0 + q * 256, samples - 1);      // (the last token again and again: its bit is its own)
+                e[q] = idx[t];
+                l[q] = loc[t];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int s = e[q] * capacity + l[q], at = s >> fill.shift;
+                if (e[q] >= 0 && e[q] < experts && l[q] >= 0 && l[q] < capacity && (s & ((1 << fill.shift) - 1)) == number) atomicOr(&s_used[at >> 5], 1u << (at & 31));
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = wave; i < mine; i += 4)
+        if (!((s_used[i >> 5] >> (i & 31)) & 1u)) zero(number + (i << fill.shift));
+}
+// how the empty slots are found: the flags' launches, or nothing beforehand
+SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locations, int64_t stride, int top_k, int samples, int experts,
+                   int capacity, hipStream_t st);
 int check_planes(const char *who, const int32_t *indices, const int32_t *locations,
                  int64_t stride, int top_k, int samples);
 // routing of up to 64 experts from [samples, experts] logits / scores with the forward chain's

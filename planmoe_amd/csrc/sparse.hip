@@ -32,32 +32,30 @@ __global__ __launch_bounds__(256) void slot_flags_mark(uint32_t *flags, const in
 }
 
 // ------------------------------------------------------------------ dispatch (scatter rows)
-// Blocks [0, token_blocks) move token rows: dispatched[slot] = 0 + gate * x[t].
-// Blocks [token_blocks, gridDim.x) write zero rows into the slots no live pair addresses.
+// token_blocks work-groups move token rows: dispatched[slot] = 0 + gate * x[t]; the others write zero rows into the slots
+// no live pair addresses.
 template <int DT, int MODE>
 __global__ __launch_bounds__(256) void dispatch_kernel(
     const void *__restrict__ x, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
-    void *__restrict__ dispatched, const uint32_t *__restrict__ flags, int token_blocks)
+    void *__restrict__ dispatched, const SlotFill fill, int token_blocks)
 {
     using IO = RowIO<DT, MODE>;
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int units = IO::units(model_dim);
     const int64_t row_bytes = (int64_t)model_dim * sizeof(typename Elem<DT>::store_t);
 
-    if ((int)blockIdx.x >= token_blocks) {
-        const int slots = experts * capacity;
-        const int nwaves = (gridDim.x - token_blocks) * 4;
-        for (int s = (blockIdx.x - token_blocks) * 4 + wave; s < slots; s += nwaves) {
-            if (flags[s]) continue;
+    const int number = fill.role((int)blockIdx.x, token_blocks);
+    if (number < 0) {
+        fill_empty_slots(fill, ~number, indices, locations, stride, top_k, samples, experts, capacity, [&](int s) {
             char *row = (char *)dispatched + (int64_t)s * row_bytes;
             for (int u = lane; u < units; u += WAVE) IO::store_zero(row, IO::at(u, (int)row_bytes));
-        }
+        });
         return;
     }
 
-    const int t = blockIdx.x * 4 + wave;
+    const int t = number * 4 + wave;
     if (t >= samples) return;
     const char *src = (const char *)x + (int64_t)t * row_bytes;
 
@@ -233,7 +231,7 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
     const void *__restrict__ grad, const void *__restrict__ rows, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
-    void *__restrict__ grad_rows, float *__restrict__ grad_gates, const uint32_t *__restrict__ flags, int token_blocks)
+    void *__restrict__ grad_rows, float *__restrict__ grad_gates, const SlotFill fill, int token_blocks)
 {
     using IO = RowIO<DT, MODE>;
     constexpr int G = 4, B = 2;
@@ -241,18 +239,16 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
     const int units = IO::units(model_dim);
     const int row_bytes = model_dim * (int)sizeof(typename Elem<DT>::store_t);
 
-    if ((int)blockIdx.x >= token_blocks) {
-        const int slots = experts * capacity;
-        const int nwaves = (gridDim.x - token_blocks) * 4;
-        for (int s = (blockIdx.x - token_blocks) * 4 + wave; s < slots; s += nwaves) {
-            if (flags[s]) continue;
+    const int number = fill.role((int)blockIdx.x, token_blocks);
+    if (number < 0) {
+        fill_empty_slots(fill, ~number, indices, locations, stride, top_k, samples, experts, capacity, [&](int s) {
             char *row = (char *)grad_rows + (int64_t)s * row_bytes;
             for (int u = lane; u < units; u += WAVE) IO::store_zero(row, IO::at(u, row_bytes));
-        }
+        });
         return;
     }
 
-    const int t = blockIdx.x * 4 + wave;
+    const int t = number * 4 + wave;
     if (t >= samples) return;
     const char *gr = (const char *)grad + (int64_t)t * row_bytes;
     for (int j0 = 0; j0 < top_k; j0 += G) {
@@ -340,15 +336,21 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
     }
 }
 
-void launch_slot_flags(uint32_t *flags, const int32_t *indices, const int32_t *locations,
-                       int64_t stride, int top_k, int samples, int experts, int capacity,
-                       hipStream_t st)
+SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locations, int64_t stride, int top_k, int samples, int experts,
+                   int capacity, hipStream_t st)
 {
     const int slots = experts * capacity;
+    const int64_t pairs = (int64_t)samples * top_k;
+    // as many work-groups as have 16 slots each, fewer where each has more to walk (8 bytes a pair, from the caches)
+    int shift = 0;
+    while (shift < (pairs <= 8192 ? 8 : pairs <= 32768 ? 7 : 6) && (slots >> (shift + 1)) >= 16) ++shift;
+    if (pairs <= SLOT_FILL_PAIRS && (slots >> shift) < SLOT_FILL_BITS) return SlotFill{nullptr, 1 << shift, shift};
+    uint32_t *flags = (uint32_t *)workspace;
     slot_flags_clear<<<(slots + 255) / 256, 256, 0, st>>>(flags, slots);
     if (samples > 0)
         slot_flags_mark<<<(samples * top_k + 255) / 256, 256, 0, st>>>(flags, indices, locations, stride,
                                                                       top_k, samples, experts, capacity);
+    return SlotFill{flags, std::min((slots + 3) / 4, 2048), 0};
 }
 
 int check_planes(const char *who, const int32_t *indices, const int32_t *locations,
@@ -390,15 +392,12 @@ extern "C" int planmoe_dispatch_fwd(const void *x, int dtype, const float *gates
                "planmoe_dispatch_fwd: workspace too small (%zu < %zu)", workspace_bytes,
                planmoe_dispatch_workspace_bytes(experts, capacity));
     hipStream_t st = (hipStream_t)stream;
-    uint32_t *flags = (uint32_t *)workspace;
-
-    launch_slot_flags(flags, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
     const int token_blocks = (samples + 3) / 4;
-    const int fill_blocks = min((slots + 3) / 4, 2048);
     const int mode = rows_mode(dtype, model_dim, x, dispatched);
     PM_DTYPE_SWITCH(dtype, DT, {
-        PM_ROWS_SWITCH(mode, MODE, (dispatch_kernel<DT, MODE><<<token_blocks + fill_blocks, 256, 0, st>>>(
-            x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, dispatched, flags,
+        PM_ROWS_SWITCH(mode, MODE, (dispatch_kernel<DT, MODE><<<token_blocks + fill.blocks, 256, 0, st>>>(
+            x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, dispatched, fill,
             token_blocks)));
     });
     PM_LAUNCH_CHECK("planmoe_dispatch_fwd");
@@ -482,15 +481,13 @@ extern "C" int planmoe_combine_bwd(const void *grad, const void *dispatched, int
     PM_REQUIRE(grad && dispatched && grad_dispatched && grad_gates, "%s: NULL argument", who);
     PM_REQUIRE(workspace && workspace_bytes >= planmoe_dispatch_workspace_bytes(experts, capacity), "%s: workspace too small", who);
     hipStream_t st = (hipStream_t)stream;
-    uint32_t *flags = (uint32_t *)workspace;
-    const int slots = experts * capacity;
-    launch_slot_flags(flags, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
-    const int token_blocks = (samples + 3) / 4, fill_blocks = min((slots + 3) / 4, 2048);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const int token_blocks = (samples + 3) / 4;
     const int mode = std::min(rows_mode(dtype, model_dim, grad, dispatched), rows_mode(dtype, model_dim, grad_dispatched, grad_dispatched));
     PM_DTYPE_SWITCH(dtype, DT, {
-        PM_ROWS_SWITCH(mode, MODE, (combine_bwd_kernel<DT, MODE><<<token_blocks + fill_blocks, 256, 0, st>>>(
+        PM_ROWS_SWITCH(mode, MODE, (combine_bwd_kernel<DT, MODE><<<token_blocks + fill.blocks, 256, 0, st>>>(
             grad, dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity,
-            grad_dispatched, grad_gates, flags, token_blocks)));
+            grad_dispatched, grad_gates, fill, token_blocks)));
     });
     PM_LAUNCH_CHECK(who);
     return 0;

@@ -260,3 +260,40 @@ def test_prescore_mode_gates_at_encode():
     out = planmoe_amd.fast_decode(y.detach(), crit, is_postscore=False)
     want_out = oracle.decode(want, list(idx), list(loc), None, T, C)
     assert np.array_equal(raw(out), want_out.view(np.int32))
+
+
+# empty slots found by the work-groups that fill them, and by flags in memory: pairs either side of 2^17, slots either side of the
+# bits a work-group keeps, one slot, fewer slots than work-groups; pairs outside the experts and the capacity, planes that are not adjacent
+@pytest.mark.parametrize("T,k,E,C", [(1, 1, 1, 1), (5, 2, 3, 5), (2049, 3, 7, 300), (65536, 2, 64, 2052), (65537, 2, 64, 2052), (300, 2, 64, 8180),
+                                     (9000, 1, 60, 2000), (20000, 1, 64, 8000)])
+def test_empty_slots_are_zero_rows(T, k, E, C):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", T, k, E, C, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + C)
+    M, slots = 8, E * C
+    place = torch.randperm(max(slots, T * k), generator=g, device=DEV)[:T * k]         # (distinct; some behind the last slot)
+    idx, loc = (place // C).int(), (place % C).int()
+    drop = torch.rand(T * k, generator=g, device=DEV)
+    idx[drop < 0.1] = -1
+    idx[(drop >= 0.1) & (drop < 0.2)] = E
+    loc[(drop >= 0.2) & (drop < 0.3)] = C
+    loc[(drop >= 0.3) & (drop < 0.4)] = -1
+    live = (idx >= 0) & (idx < E) & (loc >= 0) & (loc < C)
+    x = torch.randn(T, M, generator=g, device=DEV)
+    want = torch.zeros(slots, M, device=DEV)
+    want[(idx.long() * C + loc)[live]] = x.repeat(k, 1)[live]
+    i, l = [p.clone() for p in idx.view(k, T)], [p.clone() for p in loc.view(k, T)]
+    got = ops.dispatch_fwd(x, i, l, None, E, C)
+    codes, bias, scale = ops.dispatch_int8(x, i, l, None, E, C)
+    want_codes, want_bias, want_scale = ops.int8_compress(want)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert torch.equal(codes, want_codes.view(codes.shape)) and torch.equal(bias, want_bias.view(bias.shape)) and torch.equal(scale, want_scale.view(scale.shape))
+    ii, ll, gates = idx.view(k, T), loc.view(k, T), torch.ones(k, T, device=DEV)
+    grad, gg = torch.full((slots, M), 7.0, device=DEV), torch.empty(k, T, device=DEV)
+    ws = torch.empty(lib.planmoe_dispatch_workspace_bytes(E, C), dtype=torch.uint8, device=DEV)
+    check(lib.planmoe_combine_bwd(ops._ptr(x), ops._ptr(want), ops._dt(x, "t"), ops._ptr(gates), ops._ptr(ii), ops._ptr(ll), T, k, T, M, E, C,
+                                  ops._ptr(grad), ops._ptr(gg), ops._ptr(ws), ws.numel(), ops._stream(x)))
+    torch.cuda.synchronize()
+    assert torch.equal(grad, want)
