@@ -504,6 +504,36 @@ int planmoe_layer_combine_bwd_codes(const void *grad, const uint8_t *codes, cons
                                     int model_dim, int experts, int capacity, void *grad_rows,
                                     float *grad_gates, void *stream);
 
+/* Both of them (codec = 0: rows, bias and scale unused; codec = 1: rows are the codes) for up to 64 choices, with
+ * planmoe_route_bwd through the softmax on the gates' gradients in the same launch: grad_logits
+ * [samples][experts] as fp32, rounded to scores_dtype.  The other arguments as there. */
+int planmoe_layer_combine_bwd_logits(const void *grad, const void *rows, const void *bias, const void *scale,
+                                     int dtype, int codec, const float *gates, const int32_t *indices,
+                                     const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                                     int model_dim, int experts, int capacity, void *grad_rows,
+                                     const void *scores, int scores_dtype, int normalize_gate,
+                                     const float *grad_l_aux, const int32_t *first_choice_counts,
+                                     float *grad_logits, void *stream);
+
+/* The second bias's and the gate weight's gradients, beside the products: planmoe_layer_sums leaves shares of
+ * planmoe_rows_colsum (of grad_rows [experts][capacity][model_dim]) and of planmoe_gate_dw in the workspace, and
+ * planmoe_layer_relu_bwd, which is planmoe_expert_gemm_relu_bwd for the same rows, sums them up in its last launch. */
+size_t planmoe_layer_sums_workspace_bytes(int experts, int capacity, int samples, int model_dim);
+int planmoe_layer_sums(const void *grad_rows, int dtype, int experts, int capacity, const int32_t *live,
+                       int live_planes, int live_round, const void *x, const float *grad_logits, int samples,
+                       int model_dim, void *workspace, size_t workspace_bytes, void *stream);
+int planmoe_layer_relu_bwd(int dtype, const void *grad_rows, const void *w2, const void *h, int experts,
+                           int capacity, int hidden, int model_dim, const int32_t *live, int live_planes,
+                           int live_round, int rows_hint, void *grad_h, void *db1, void *workspace,
+                           size_t workspace_bytes, const void *sums, size_t sums_bytes, int samples, void *db2,
+                           void *dwg, void *stream);
+
+/* The gradient of x: planmoe_layer_combine without gates, then planmoe_gate_dx_accumulate (up to 8 experts), the
+ * same roundings, in one pass where a row is at most 8 KB. */
+int planmoe_layer_dx(const void *rows, int dtype, int codec, const int32_t *indices, const int32_t *locations,
+                     int64_t plane_stride, int top_k, int samples, int model_dim, int experts, int capacity,
+                     const float *grad_logits, const void *wg, void *out, void *stream);
+
 /* The zfp codec at rate 8 on the layer's fp32 rows (what Compress and Decompress of "zfp" do around a one-rank
  * exchange, zfpc.cpp:23-86): same bits as planmoe_zfp_compress and planmoe_zfp_decompress of the buffer whose empty
  * slots are zeros, without the stream in between.  expert_counts [top_k][experts] from the routing that made

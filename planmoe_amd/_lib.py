@@ -104,6 +104,16 @@ SIGNATURES = {
                                               c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "planmoe_layer_combine_bwd_codes": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64,
                                                 c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
+    "planmoe_layer_combine_bwd_logits": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64,
+                                                 c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p,
+                                                 c_void_p, c_void_p]),
+    "planmoe_layer_sums_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "planmoe_layer_sums": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_size_t,
+                                   c_void_p]),
+    "planmoe_layer_relu_bwd": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
+                                       c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_size_t, c_int, c_void_p, c_void_p, c_void_p]),
+    "planmoe_layer_dx": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                                 c_void_p, c_void_p]),
     "planmoe_rows_colsum_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "planmoe_rows_colsum": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_size_t,
                                     c_void_p]),

@@ -73,11 +73,12 @@ Tensor as_rows(const Tensor &grad)
 
 // the codes of the experts' rows [rows, M], behind them the rows' minima and scales in x's dtype
 struct Kept {
+    Kept() = default;
     Kept(const Tensor &buffer, const Shape &s, int64_t size)
         : codes(buffer.data_ptr<uint8_t>()), bias(codes + s.rows() * s.M), scale(codes + s.rows() * (s.M + size)) {}
     static int64_t bytes(const Shape &s, int64_t size) { return s.rows() * (s.M + 2 * size); }
-    uint8_t *codes;
-    void *bias, *scale;
+    uint8_t *codes = nullptr;
+    void *bias = nullptr, *scale = nullptr;
 };
 
 Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
@@ -250,13 +251,28 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         const int32_t *idx = ints(p.indices), *loc = ints(p.locations);
         const bool need_x = ctx->needs_input_grad(0), need_gate = ctx->needs_input_grad(1), need_w1 = ctx->needs_input_grad(2),
                    need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
-        Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates;
+        Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates, gf;
+        Tensor gl = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
+        const float *dl = gl.defined() ? floats(gl) : nullptr;
+        const int32_t *count0 = gl.defined() ? ints(p.counts) : nullptr;
+        // the logits' gradient, in the scores' precision
+        auto route_bwd = [&]() {
+            Tensor gg = grad_gates.defined() ? grad_gates.to(scores.scalar_type()) : at::zeros({s.k, s.T}, scores.options());
+            Tensor g = at::empty_like(scores);
+            PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), idx, gg.data_ptr(), s.T, s.T, s.E, s.k, normalize, dl, count0, 1,
+                                      g.data_ptr(), st));
+            return g;
+        };
+        auto as_float = [](const Tensor &g) { return g.scalar_type() == at::kFloat ? g : g.to(at::kFloat); };
+        // everything is asked for, as in a training step: reductions share their launches, and the gate's part of dx is added in the combine
+        const bool whole = grads[0].defined() && need_x && need_gate && need_w1 && need_b1 && need_w2 && need_b2;
         if (grads[0].defined()) {
             const Tensor grad = as_rows(grads[0]);
             const Tensor gates = float_gates(p.gates);
             const Live live = live_rows(p, s, codec);
-            grad_gates = at::empty({s.k, s.T}, x.options().dtype(at::kFloat));
-            Tensor gye;
+            const bool logits = whole && s.k <= 64 && (codec == CODEC_NONE || codec == CODEC_INT8);
+            (logits ? gf : grad_gates) = at::empty({logits ? s.T : s.k, logits ? s.E : s.T}, x.options().dtype(at::kFloat));
+            Tensor gye, sums;
             if (codec == CODEC_ZFP) {
                 gye = at::empty({s.rows(), s.M}, x.options());
                 Tensor ws = zfp_workspace(s, x);
@@ -269,7 +285,13 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                 gye = lz_round_trip(buf, st);
             } else {
                 gye = at::empty({s.rows(), s.M}, x.options());
-                if (codec == CODEC_INT8) {
+                if (logits) {
+                    const bool coded = codec == CODEC_INT8;
+                    const Kept kept = coded ? Kept(ye, s, x.element_size()) : Kept{};
+                    PM_CALL(planmoe_layer_combine_bwd_logits(grad.data_ptr(), coded ? kept.codes : ye.data_ptr(), kept.bias, kept.scale, s.dt, coded,
+                                                             floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, gye.data_ptr(), scores.data_ptr(),
+                                                             pm_dtype(scores.scalar_type()), normalize, dl, count0, gf.data_ptr<float>(), st));
+                } else if (codec == CODEC_INT8) {
                     const Kept kept(ye, s, x.element_size());
                     PM_CALL(planmoe_layer_combine_bwd_codes(grad.data_ptr(), kept.codes, kept.bias, kept.scale, s.dt, floats(gates), idx, loc, s.T, s.k,
                                                             s.T, s.M, s.E, s.cap, gye.data_ptr(), grad_gates.data_ptr<float>(), st));
@@ -277,6 +299,14 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                     PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, 0, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
                                                       gye.data_ptr(), grad_gates.data_ptr<float>(), st));
                 }
+            }
+            if (whole) {
+                if (!gf.defined()) gf = as_float(route_bwd());
+                sums = bytes((int64_t)planmoe_layer_sums_workspace_bytes(s.E, s.cap, s.T, s.M), x);
+                PM_CALL(planmoe_layer_sums(gye.data_ptr(), s.dt, s.E, s.cap, live.counts, live.planes, live.round, x.data_ptr(), floats(gf), s.T, s.M,
+                                           sums.data_ptr(), (size_t)sums.numel(), st));
+                db2 = at::empty({s.E, s.M}, x.options());
+                dwg = at::empty_like(wg);
             }
             auto colsum = [&](const Tensor &a, int cols) {
                 Tensor out = at::empty({s.E, cols}, x.options()), ws = bytes((int64_t)planmoe_rows_colsum_workspace_bytes(s.E, s.cap, cols), x);
@@ -289,15 +319,20 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                 PM_CALL(planmoe_expert_gemm(2, s.dt, p.h.data_ptr(), gye.data_ptr(), nullptr, 0, s.E, s.H, s.M, s.cap, live.counts, live.planes, live.round,
                                             s.hint(), dw2.data_ptr(), st));
             }
-            if (need_b2) db2 = colsum(gye, s.M);
+            if (need_b2 && !whole) db2 = colsum(gye, s.M);
             if (need_x || need_w1 || need_b1) {
                 Tensor gh = at::empty({s.rows(), s.H}, x.options()), ws;
                 if (need_b1) {
                     db1 = at::empty({s.E, s.H}, x.options());
                     ws = bytes((int64_t)planmoe_expert_gemm_relu_bwd_workspace_bytes(s.E, s.cap, s.H), x);
                 }
-                PM_CALL(planmoe_expert_gemm_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
-                                                     live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), ws.defined() ? (size_t)ws.numel() : 0, st));
+                if (whole)
+                    PM_CALL(planmoe_layer_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
+                                                   live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), (size_t)ws.numel(), sums.data_ptr(),
+                                                   (size_t)sums.numel(), s.T, raw(db2), raw(dwg), st));
+                else
+                    PM_CALL(planmoe_expert_gemm_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
+                                                         live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), ws.defined() ? (size_t)ws.numel() : 0, st));
                 if (need_w1) {
                     dw1 = at::empty_like(w1);
                     PM_CALL(planmoe_expert_gemm(2, s.dt, p.xe.data_ptr(), gh.data_ptr(), nullptr, 0, s.E, s.M, s.H, s.cap, live.counts, live.planes,
@@ -310,31 +345,31 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                     if (codec == CODEC_ZFP) zfp_rows(gxe, Tensor(), p, s, st);
                     if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
                     dx = at::empty_like(x);
+                    if (whole && s.E <= 8) {
+                        PM_CALL(planmoe_layer_dx(gxe.data_ptr(), s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
+                                                 wg.data_ptr(), dx.data_ptr(), st));
+                        return {dx, dwg, dw1, db1, dw2, db2, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+                    }
                     PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
                                                   dx.data_ptr(), st));
                 }
             }
         }
         // gates and loss back through the routing into the gate's weight and x
-        if ((grad_gates.defined() || grads[1].defined()) && (need_x || need_gate)) {
-            Tensor gg = grad_gates.defined() ? grad_gates.to(scores.scalar_type()) : at::zeros({s.k, s.T}, scores.options());
-            Tensor gl = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
-            Tensor g = at::empty_like(scores);
-            PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), idx, gg.data_ptr(), s.T, s.T, s.E, s.k, normalize,
-                                      gl.defined() ? floats(gl) : nullptr, gl.defined() ? ints(p.counts) : nullptr, 1, g.data_ptr(), st));
-            const Tensor gf = g.scalar_type() == at::kFloat ? g : g.to(at::kFloat);
-            if (need_gate) {
+        if ((grad_gates.defined() || gf.defined() || grads[1].defined()) && (need_x || need_gate)) {
+            if (!gf.defined()) gf = as_float(route_bwd());
+            if (need_gate && !dwg.defined()) {
                 dwg = at::empty_like(wg);
                 Tensor ws = bytes((int64_t)planmoe_gate_dw_workspace_bytes(s.T, s.M, s.E), x);
                 PM_CALL(planmoe_gate_dw(x.data_ptr(), s.dt, floats(gf), s.T, s.M, s.E, dwg.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), st));
             }
             if (need_x) {
                 if (!dx.defined()) {
-                    dx = at::mm(g.to(x.scalar_type()), wg);
+                    dx = at::mm(gf.to(x.scalar_type()), wg);
                 } else if (s.E <= 8) {
                     PM_CALL(planmoe_gate_dx_accumulate(dx.data_ptr(), s.dt, floats(gf), wg.data_ptr(), s.T, s.M, s.E, st));
                 } else {
-                    dx.addmm_(g.to(x.scalar_type()), wg);
+                    dx.addmm_(gf.to(x.scalar_type()), wg);
                 }
             }
         }

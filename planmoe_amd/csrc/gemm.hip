@@ -13,6 +13,7 @@
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
 #include "gemm_skinny.hpp"
+#include "sums.hpp"
 #include <algorithm>
 #include <cmath>
 
@@ -552,36 +553,6 @@ __global__ __launch_bounds__(GEMM_WG, S::WAVES_PER_SIMD) void gemm_bf16_kernel(c
 #undef PM_PHASE
 }
 
-// the column sums of the tiles of a batch, in order, as the bias gradient: 64 columns per
-// work-group, its waves every fourth slot, eight loads in flight
-template <int DT>
-__global__ __launch_bounds__(256) void gemm_colsum_kernel(const float *__restrict__ parts, const int *__restrict__ live, int live_planes,
-                                                          int live_round, int batches, int M, int N, int BM, int per_tile, int slots,
-                                                          void *__restrict__ out)
-{
-    __shared__ float s_sum[4][64];
-    const int e = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
-    int rows = M;
-    if (live) {
-        int c = 0;
-        for (int j = 0; j < live_planes; ++j) c += live[j * batches + e];
-        rows = min(M, (c + live_round - 1) / live_round * live_round);
-    }
-    const int used = min(slots, (rows + BM - 1) / BM * per_tile);
-    const float *from = parts + (int64_t)e * slots * N + min(n, N - 1);
-    float s = 0.f;
-    for (int i0 = wave * 8; i0 < used; i0 += 32) {
-        float v[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = from[(int64_t)min(i0 + q, used - 1) * N];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s += i0 + q < used ? v[q] : 0.f;
-    }
-    s_sum[wave][lane] = s;
-    __syncthreads();
-    if (wave == 0 && n < N) Elem<DT>::store(out, (int64_t)e * N + n, s_sum[0][lane] + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane]);
-}
-
 // out[e][c][r] = in[e][r][c] for r < rows, zero for rows <= r < rows_out (the padding of a k dimension):
 // 64 x 64 tiles through LDS, 16-byte accesses on both sides
 __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t *__restrict__ in, uint16_t *__restrict__ out,
@@ -850,16 +821,14 @@ extern "C" size_t planmoe_expert_gemm_relu_bwd_workspace_bytes(int batches, int 
     return (size_t)batches * 2 * ((m + 63) / 64) * n * 4;      // (fp32 tiles may have 64 rows)
 }
 
-extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void *b, const void *h, int batches, int m, int n,
-                                            int k, const int32_t *live, int live_planes, int live_round, int rows_hint, void *c,
-                                            void *dbias, void *workspace, size_t workspace_bytes, void *stream)
+int pm::relu_bwd_with(const char *who, int dtype, const void *a, const void *b, const void *h, int batches, int m, int n, int k, const int *live,
+                      int live_planes, int live_round, int rows_hint, void *c, void *dbias, void *workspace, size_t workspace_bytes,
+                      const SumJob *others, int others_n, hipStream_t st)
 {
-    const char *who = "planmoe_expert_gemm_relu_bwd";
     if (expert_gemm_check(who, 1, dtype, a, b, batches, m, n, k, live, live_planes, live_round, c)) return 1;
     PM_REQUIRE(h && aligned16(h), "%s: NULL or unaligned activations", who);
     PM_REQUIRE(!dbias || (workspace && aligned16(workspace) && workspace_bytes >= planmoe_expert_gemm_relu_bwd_workspace_bytes(batches, m, n)), "%s: workspace too small", who);
     PM_REQUIRE(batches <= 65535, "%s: too many batches", who);
-    hipStream_t st = (hipStream_t)stream;
     float *parts = dbias ? (float *)workspace : nullptr;
     const int hint = rows_hint >= 1 && rows_hint < m ? rows_hint : m;
     GemmSlots sums;
@@ -873,15 +842,23 @@ extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void
                    m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};
         if (gemm_run<false, false, true>(p, hint, st, who, &sums)) return 1;
     }
+    SumJob jobs[SUM_JOBS];
+    int count = 0;
+    for (int i = 0; i < others_n; ++i) jobs[count++] = others[i];
     if (dbias) {
         if (sums.rows == 0) sums.rows = m;
         const int slots = (m + sums.rows - 1) / sums.rows * sums.per_tile;
-        const dim3 grid((unsigned)((n + 63) / 64), (unsigned)batches);
-        if (dtype == PLANMOE_F32) gemm_colsum_kernel<PLANMOE_F32><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, sums.rows, sums.per_tile, slots, dbias);
-        else gemm_colsum_kernel<PLANMOE_BF16><<<grid, 256, 0, st>>>(parts, live, live_planes, live_round, batches, m, n, sums.rows, sums.per_tile, slots, dbias);
-        PM_LAUNCH_CHECK(who);
+        jobs[count++] = SumJob{parts, dbias, batches, slots, n, live, live_planes, live_round, m, sums.rows, sums.per_tile};
     }
-    return 0;
+    return sum_slots(who, dtype, jobs, count, st);
+}
+
+extern "C" int planmoe_expert_gemm_relu_bwd(int dtype, const void *a, const void *b, const void *h, int batches, int m, int n,
+                                            int k, const int32_t *live, int live_planes, int live_round, int rows_hint, void *c,
+                                            void *dbias, void *workspace, size_t workspace_bytes, void *stream)
+{
+    return relu_bwd_with("planmoe_expert_gemm_relu_bwd", dtype, a, b, h, batches, m, n, k, live, live_planes, live_round, rows_hint, c, dbias, workspace,
+                         workspace_bytes, nullptr, 0, (hipStream_t)stream);
 }
 
 extern "C" int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int rows_out, void *out, void *stream)

@@ -1,5 +1,5 @@
 // The row passes of the layer whose experts' buffers never leave the GPU: combine and its backward
-// pass with the codec of the exchange in between, and the small reductions of the backward pass.
+// pass with the codec of the exchange in between.
 //
 // On one rank the all-to-all delivers what was sent, so what "int8" does to a row is
 // decompress(compress(row)) (int8.cpp:10-24, 46-60).  The kernels here apply that to a row while it is
@@ -8,106 +8,13 @@
 // codes, read E C M values, wrote and read their codes.  Only rows that hold a token are touched: empty
 // capacity slots are never written and never read.
 #include "rows.hpp"
-#include <type_traits>
 #include "int8_core.hpp"
+#include "layer_rows.hpp"
+#include "route_bwd.hpp"
+
+#include <type_traits>
 
 namespace pm {
-
-// a vector's codes as they are kept, one byte a value
-template <int DT> struct CodeWords { uint32_t w[Elem<DT>::VEC / 4]; };
-template <int DT>
-__device__ __forceinline__ void store_codes(uint8_t *to, const CodeWords<DT> &v)
-{
-    if constexpr (Elem<DT>::VEC == 8) stream_store(reinterpret_cast<uint2 *>(to), make_uint2(v.w[0], v.w[1]));
-    else stream_store(reinterpret_cast<uint32_t *>(to), v.w[0]);
-}
-
-// decompress(compress(row)) of a row held as CACHE vectors per lane (vectors past the end: copies of the last);
-// keep(c, codes) sees the codes of vector c.  Returns the row's minimum and scale.
-template <int DT, int CACHE, bool CANON, typename Keep>
-__device__ __forceinline__ float2 through_int8(uint4 (&row)[CACHE], Keep keep)
-{
-    using E = Elem<DT>;
-    RowStats<DT, CANON> stats;
-    stats.init();
-#pragma unroll
-    for (int c = 0; c < CACHE; ++c) stats.add(row[c]);
-    float mn, mx;
-    stats.finish(mn, mx);
-    const float scale = E::round(mx - mn);
-    const RowEncoder<DT> enc(mn, scale);
-    const RowDecoder<DT> dec(mn, scale);
-    auto body = [&](auto mode) {
-#pragma unroll
-        for (int c = 0; c < CACHE; ++c) {
-            CodeWords<DT> code;
-            float f[E::VEC];
-            enc.template encode<decltype(mode)::value>(row[c], code.w);
-            keep(c, code);
-#pragma unroll
-            for (int q = 0; q < E::VEC / 4; ++q) dec.word(code.w[q], f + 4 * q);
-            row[c] = E::pack(f);
-        }
-    };
-    if (enc.fast()) body(std::true_type{}); else body(std::false_type{});
-    return make_float2(mn, scale);
-}
-
-// The same with the decoder as a table: a row has 256 codes, so a wave works out gate * decoded(code) for four codes a
-// lane, into LDS, and a value is a lookup by its code.  (Decoding value by value, the 35 vector instructions of a pair
-// of bf16 values took as long as its bytes.  Combine at 16384 x 4096, top-2, 113 -> 81 us,
-// at 16384 x 1024 35 -> 27, its backward pass there 64 -> 48.)
-template <int DT>
-__device__ __forceinline__ void fill_table(float mn, float scale, float gate, float *table)
-{
-    float f[4];
-    RowDecoder<DT>(mn, scale).word(0x03020100u + 0x04040404u * (uint32_t)lane_id(), f);
-    *reinterpret_cast<float4 *>(table + 4 * lane_id()) = make_float4(gate * f[0], gate * f[1], gate * f[2], gate * f[3]);
-}
-template <int DT>
-struct RowTable {
-    RowEncoder<DT> enc;
-    const float *tab;                            // 256 values, the wave's own
-    float mn, scale;
-    template <int CACHE>
-    __device__ __forceinline__ RowTable(const uint4 (&row)[CACHE], float gate, float *table) : enc(0.f, 0.f), tab(table)
-    {
-        using E = Elem<DT>;
-        RowStats<DT, false> stats;
-        stats.init();
-#pragma unroll
-        for (int c = 0; c < CACHE; ++c) stats.add(row[c]);
-        float mx;
-        stats.finish(mn, mx);
-        scale = E::round(mx - mn);
-        enc = RowEncoder<DT>(mn, scale);
-        fill_table<DT>(mn, scale, gate, table);
-    }
-    template <bool FAST, typename Keep>
-    __device__ __forceinline__ void values(const uint4 &raw, float (&f)[Elem<DT>::VEC], Keep keep) const
-    {
-        uint32_t c[Elem<DT>::VEC];
-        enc.template codes<FAST>(raw, c);
-        CodeWords<DT> code;
-#pragma unroll
-        for (int q = 0; q < Elem<DT>::VEC / 4; ++q) code.w[q] = c[4 * q] | (c[4 * q + 1] << 8) | (c[4 * q + 2] << 16) | (c[4 * q + 3] << 24);
-        keep(code);
-#pragma unroll
-        for (int i = 0; i < Elem<DT>::VEC; ++i) f[i] = tab[c[i]];
-    }
-    template <bool FAST>
-    __device__ __forceinline__ void values(const uint4 &raw, float (&f)[Elem<DT>::VEC]) const
-    {
-        values<FAST>(raw, f, [](const CodeWords<DT> &) {});
-    }
-};
-// what a wave's lanes wrote to its LDS is there for all of them, and what they read has been read
-__device__ __forceinline__ void table_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // out[t] = sum_j gate_j * codec(rows[slot_j]), planes left to right, one rounding at the end.
 // One wave per token; the rows of two choices are requested before either is used and stay as they lie in
@@ -213,12 +120,15 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
 // passes around it, overlap.py:19-34).  The rows come as they are (SEEN_ROWS without a codec, SEEN_INT8 with), or as the codes,
 // minima and scales that the forward pass kept (SEEN_CODES): half or a quarter of the bytes, and no codes to work out.
 // 16384 x 1024 bf16, top-2: 48 us from the rows, 38 from the codes (33 MB of the gradient in, 34 of codes, 67 out).
+// grad_logits given: up to 64 choices, whose gates' gradients go on through the routing into the logits' while the wave has them, and
+// grad_gates is not written (a launch of its own reads and writes 100 bytes a token: 5 us, and as much of the host's time).
 enum { SEEN_ROWS, SEEN_INT8, SEEN_CODES };
 template <int DT, int CACHE, int SEEN>
 __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
     const void *__restrict__ grad, const void *__restrict__ rows, const void *__restrict__ bias, const void *__restrict__ scales,
     const float *__restrict__ gates, const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
-    int top_k, int samples, int model_dim, int capacity, void *__restrict__ grad_rows, float *__restrict__ grad_gates)
+    int top_k, int samples, int model_dim, int capacity, void *__restrict__ grad_rows, float *__restrict__ grad_gates,
+    const RouteBwd route, int scores_dtype, float *__restrict__ grad_logits)
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
@@ -235,11 +145,12 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) g_row[c] = src[min(c * WAVE + lane, units - 1)];
     }
+    float dgate = 0.f;                           // lane j: the gradient of gate j
     for (int j0 = 0; j0 < top_k; j0 += WAVE) {
         const int np = min(top_k - j0, WAVE);
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
-        if (lane < np && slot < 0) grad_gates[(int64_t)(j0 + lane) * stride + t] = 0.f;
+        if (grad_gates && lane < np && slot < 0) grad_gates[(int64_t)(j0 + lane) * stride + t] = 0.f;
         float mn = 0.f, scale = 0.f;
         if (SEEN == SEEN_CODES && lane < np && slot >= 0) { mn = E::load(bias, slot); scale = E::load(scales, slot); }
         // the next choice's row is on its way while this one's is worked on (a dropped choice reads slot 0, unused)
@@ -302,7 +213,8 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
                 }
             }
             acc = wave_sum(acc);
-            if (lane == 0) grad_gates[(int64_t)(j0 + j) * stride + t] = acc;
+            if (grad_gates && lane == 0) grad_gates[(int64_t)(j0 + j) * stride + t] = acc;
+            if (lane == j) dgate = acc;
             // the gradient row as the dispatcher stores it for this gate: round(0 + g * x)
             uint4 r[CACHE];
 #pragma unroll
@@ -333,128 +245,17 @@ __global__ __launch_bounds__(256) void layer_combine_bwd_kernel(
             }
         }
     }
-}
-
-// Column sums of the rows in use of every batch: out[e][n] = sum_{r < rows_e} a[e][r][n] (the bias gradient).
-// A work-group takes 64 vectors of columns and a share of the rows, four rows at a time side by side; the
-// shares' sums go to `parts` and the second kernel adds them in order.
-template <int DT>
-__global__ __launch_bounds__(256) void rows_colsum_kernel(const void *__restrict__ a, const int *__restrict__ live, int live_planes,
-                                                          int live_round, int batches, int rows, int cols, int shares, float *__restrict__ parts)
-{
-    using E = Elem<DT>;
-    constexpr int V = E::VEC;
-    __shared__ float s_sum[4][WAVE][V + 1];
-    const int e = blockIdx.z, share = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6;
-    const int units = cols / V, u = blockIdx.x * WAVE + lane, uc = min(u, units - 1);
-    int used = rows;
-    if (live) {
-        int n = 0;
-        for (int j = 0; j < live_planes; ++j) n += live[j * batches + e];
-        used = min(rows, (n + live_round - 1) / live_round * live_round);
-    }
-    const int per = (used + shares - 1) / shares, r0 = share * per, r1 = min(used, r0 + per);
-    const uint4 *src = reinterpret_cast<const uint4 *>((const char *)a + (int64_t)e * rows * cols * (int64_t)sizeof(typename E::store_t));
-    float acc[V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) acc[i] = 0.f;
-    constexpr int R = 4;
-    for (int r = r0 + wave * R; r < r1; r += 4 * R) {
-        uint4 v[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) v[q] = src[(int64_t)min(r + q, r1 - 1) * units + uc];
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            float f[V];
-            E::unpack(v[q], f);
-#pragma unroll
-            for (int i = 0; i < V; ++i) acc[i] += r + q < r1 ? f[i] : 0.f;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < V; ++i) s_sum[wave][lane][i] = acc[i];
-    __syncthreads();
-    for (int x = threadIdx.x; x < WAVE * V; x += 256) {
-        const int l = x / V, i = x % V, col = (blockIdx.x * WAVE + l) * V + i;
-        if (col < cols) parts[((int64_t)e * shares + share) * cols + col] = s_sum[0][l][i] + s_sum[1][l][i] + s_sum[2][l][i] + s_sum[3][l][i];
-    }
-}
-
-// out[e][c] = sum over the shares, in order within a wave's quarter: 64 columns per work-group, eight loads in flight
-// (a thread per column that walked the shares one by one took 35 us for 256 shares of 8 x 1024)
-template <int DT>
-__global__ __launch_bounds__(256) void parts_sum_kernel(const float *__restrict__ parts, int shares, int cols, void *__restrict__ out)
-{
-    __shared__ float s_sum[4][WAVE];
-    const int e = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6, c = blockIdx.x * WAVE + lane;
-    const float *from = parts + (int64_t)e * shares * cols + min(c, cols - 1);
-    const int per = (shares + 3) / 4, i1 = min(shares, (wave + 1) * per);
-    float s = 0.f;
-    for (int i = wave * per; i < i1; i += 8) {
-        float v[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = from[(int64_t)min(i + q, i1 - 1) * cols];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s += i + q < i1 ? v[q] : 0.f;
-    }
-    s_sum[wave][lane] = s;
-    __syncthreads();
-    if (wave == 0 && c < cols) Elem<DT>::store(out, (int64_t)e * cols + c, s_sum[0][lane] + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane]);
-}
-
-// Gate weight gradient: parts[share][e][m] = sum_{t in share} g[t][e] * x[t][m]; a work-group takes 64 vectors
-// of columns and a share of the tokens, its waves every fourth token; EP experts per pass.
-template <int DT, int EP>
-__global__ __launch_bounds__(256) void gate_dw_kernel(const void *__restrict__ x, const float *__restrict__ g, int samples, int model_dim,
-                                                      int experts, int e0, int shares, float *__restrict__ parts)
-{
-    using E = Elem<DT>;
-    constexpr int V = E::VEC;
-    __shared__ float s_sum[3][WAVE][EP * V + 1];
-    const int share = blockIdx.y, lane = lane_id(), wave = threadIdx.x >> 6;
-    const int units = model_dim / V, u = blockIdx.x * WAVE + lane, uc = min(u, units - 1);
-    const int per = (samples + shares - 1) / shares, t0 = share * per, t1 = min(samples, t0 + per);
-    const uint4 *src = reinterpret_cast<const uint4 *>(x);
-    float acc[EP][V];
-#pragma unroll
-    for (int e = 0; e < EP; ++e)
-#pragma unroll
-        for (int i = 0; i < V; ++i) acc[e][i] = 0.f;
-    constexpr int R = 4;
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    for (int t = t0 + wave_u * R; t < t1; t += 4 * R) {
-        uint4 v[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) v[q] = src[(int64_t)min(t + q, t1 - 1) * units + uc];
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            float f[V];
-            E::unpack(v[q], f);
-            const int tq = min(t + q, t1 - 1);
-#pragma unroll
-            for (int e = 0; e < EP; ++e) {
-                // (uniform: scalar loads; g rounded to x's dtype first, as the cast before a library GEMM would)
-                const float ge = e0 + e < experts && t + q < t1 ? E::round(g[(int64_t)tq * experts + e0 + e]) : 0.f;
-#pragma unroll
-                for (int i = 0; i < V; ++i) acc[e][i] = fmaf(ge, f[i], acc[e][i]);
-            }
-        }
-    }
-    if (wave > 0)
-#pragma unroll
-        for (int e = 0; e < EP; ++e)
-#pragma unroll
-            for (int i = 0; i < V; ++i) s_sum[wave - 1][lane][e * V + i] = acc[e][i];
-    __syncthreads();
-    if (wave == 0 && u < units) {
-#pragma unroll
-        for (int e = 0; e < EP; ++e) {
-            if (e0 + e >= experts) break;
-            float *to = parts + ((int64_t)share * experts + e0 + e) * model_dim + (int64_t)u * V;
-#pragma unroll
-            for (int i = 0; i < V; ++i)
-                to[i] = acc[e][i] + s_sum[0][lane][e * V + i] + s_sum[1][lane][e * V + i] + s_sum[2][lane][e * V + i];
-        }
+    if (grad_logits) {
+        const int at = lane < top_k ? indices[(int64_t)lane * stride + t] : -1;
+        auto logits = [&](auto dt) {
+            constexpr int ST = decltype(dt)::value;
+            route_bwd_token<ST>(route, t, lane % route.group, true, [&](int j) { return rl_i(at, j); },
+                                [&](int j) { return Elem<ST>::round(rl_f(dgate, j)); },
+                                [&](int e, float v) { if (lane < route.group) grad_logits[(int64_t)t * route.experts + e] = Elem<ST>::round(v); });
+        };
+        if (scores_dtype == PLANMOE_F32) logits(std::integral_constant<int, PLANMOE_F32>{});
+        else if (scores_dtype == PLANMOE_BF16) logits(std::integral_constant<int, PLANMOE_BF16>{});
+        else logits(std::integral_constant<int, PLANMOE_F16>{});
     }
 }
 
@@ -462,10 +263,10 @@ __global__ __launch_bounds__(256) void gate_dw_kernel(const void *__restrict__ x
 
 using namespace pm;
 
-namespace {
+namespace pm {
 
-int rows_check(const char *who, int dtype, const void *rows, const int32_t *indices, const int32_t *locations, int64_t stride,
-               int top_k, int samples, int model_dim, int experts, int capacity, int codec)
+int layer_rows_check(const char *who, int dtype, const void *rows, const int32_t *indices, const int32_t *locations, int64_t stride,
+                     int top_k, int samples, int model_dim, int experts, int capacity, int codec)
 {
     if (check_planes(who, indices, locations, stride, top_k, samples)) return 1;
     PM_REQUIRE(dtype_ok(dtype), "%s: bad dtype %d", who, dtype);
@@ -478,17 +279,7 @@ int rows_check(const char *who, int dtype, const void *rows, const int32_t *indi
     return 0;
 }
 
-}  // namespace
-
-// the rows a wave keeps in registers: 1, 2, 4, 8 or 16 vectors per lane
-#define PM_ROW_CACHE(CALL)                                    \
-    do {                                                      \
-        if (per_lane <= 1) CALL(1);                           \
-        else if (per_lane <= 2) CALL(2);                      \
-        else if (per_lane <= 4) CALL(4);                      \
-        else if (per_lane <= 8) CALL(8);                      \
-        else CALL(16);                                        \
-    } while (0)
+} // namespace pm
 
 // codes NULL: none are kept
 static int combine_int8_rows(const char *who, const void *rows, int dtype, const float *gates, const int32_t *indices, const int32_t *locations,
@@ -518,7 +309,7 @@ extern "C" int planmoe_layer_combine(const void *rows, int dtype, int codec, con
                                      int experts, int capacity, void *out, void *stream)
 {
     const char *who = "planmoe_layer_combine";
-    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
+    if (layer_rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
     if (codec == 0) return planmoe_combine_fwd(rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, stream);
     return combine_int8_rows(who, rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, nullptr, nullptr,
                              nullptr, stream);
@@ -529,7 +320,7 @@ extern "C" int planmoe_layer_combine_keep(const void *rows, int dtype, const flo
                                           void *out, uint8_t *codes, void *bias, void *scale, void *stream)
 {
     const char *who = "planmoe_layer_combine_keep";
-    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
+    if (layer_rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
     PM_REQUIRE(codes && bias && scale && aligned16(codes), "%s: NULL output, or codes not 16-byte aligned", who);
     return combine_int8_rows(who, rows, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out, codes, bias, scale,
                              stream);
@@ -538,14 +329,15 @@ extern "C" int planmoe_layer_combine_keep(const void *rows, int dtype, const flo
 // seen: SEEN_ROWS, SEEN_INT8 or SEEN_CODES (bias and scale are read with the last only)
 static int combine_bwd_rows(const char *who, int seen, const void *grad, const void *rows, const void *bias, const void *scale, int dtype,
                             const float *gates, const int32_t *indices, const int32_t *locations, int64_t plane_stride, int top_k,
-                            int samples, int model_dim, int capacity, void *grad_rows, float *grad_gates, void *stream)
+                            int samples, int model_dim, int capacity, void *grad_rows, float *grad_gates, void *stream,
+                            const RouteBwd &route = RouteBwd{}, int scores_dtype = 0, float *grad_logits = nullptr)
 {
     if (samples == 0) return 0;
-    PM_REQUIRE(grad && grad_rows && grad_gates && gates && aligned16(grad) && aligned16(grad_rows), "%s: NULL or unaligned argument", who);
+    PM_REQUIRE(grad && grad_rows && (grad_gates || grad_logits) && gates && aligned16(grad) && aligned16(grad_rows), "%s: NULL or unaligned argument", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
     hipStream_t st = (hipStream_t)stream;
 #define PM_LB_(CACHE, SEEN) (layer_combine_bwd_kernel<DT, CACHE, SEEN><<<(samples + 3) / 4, 256, 0, st>>>(grad, rows, bias, scale, gates, indices, \
-        locations, plane_stride, top_k, samples, model_dim, capacity, grad_rows, grad_gates))
+        locations, plane_stride, top_k, samples, model_dim, capacity, grad_rows, grad_gates, route, scores_dtype, grad_logits))
 #define PM_LB(CACHE)                                                                          \
     do {                                                                                      \
         if (seen == SEEN_CODES) PM_LB_(CACHE, SEEN_CODES);                                    \
@@ -565,7 +357,7 @@ extern "C" int planmoe_layer_combine_bwd(const void *grad, const void *rows, int
                                          float *grad_gates, void *stream)
 {
     const char *who = "planmoe_layer_combine_bwd";
-    if (rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
+    if (layer_rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
     return combine_bwd_rows(who, codec ? SEEN_INT8 : SEEN_ROWS, grad, rows, nullptr, nullptr, dtype, gates, indices, locations, plane_stride, top_k,
                             samples, model_dim, capacity, grad_rows, grad_gates, stream);
 }
@@ -576,66 +368,24 @@ extern "C" int planmoe_layer_combine_bwd_codes(const void *grad, const uint8_t *
                                                int capacity, void *grad_rows, float *grad_gates, void *stream)
 {
     const char *who = "planmoe_layer_combine_bwd_codes";
-    if (rows_check(who, dtype, codes, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
+    if (layer_rows_check(who, dtype, codes, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, 1)) return 1;
     PM_REQUIRE((bias && scale) || samples == 0, "%s: NULL argument", who);
     return combine_bwd_rows(who, SEEN_CODES, grad, codes, bias, scale, dtype, gates, indices, locations, plane_stride, top_k, samples, model_dim,
                             capacity, grad_rows, grad_gates, stream);
 }
 
-// how many shares a reduction over `rows` is cut into for `blocks` column blocks: enough work-groups for the GPU, at least 32 rows each
-static int reduction_shares(int64_t rows, int64_t blocks)
+extern "C" int planmoe_layer_combine_bwd_logits(const void *grad, const void *rows, const void *bias, const void *scale, int dtype, int codec,
+                                                const float *gates, const int32_t *indices, const int32_t *locations, int64_t plane_stride,
+                                                int top_k, int samples, int model_dim, int experts, int capacity, void *grad_rows,
+                                                const void *scores, int scores_dtype, int normalize_gate, const float *grad_l_aux,
+                                                const int32_t *first_choice_counts, float *grad_logits, void *stream)
 {
-    int64_t s = (1024 + blocks - 1) / blocks;
-    if (s > (rows + 31) / 32) s = (rows + 31) / 32;
-    return (int)(s < 1 ? 1 : s > 256 ? 256 : s);
-}
-
-extern "C" size_t planmoe_rows_colsum_workspace_bytes(int batches, int rows, int cols)
-{
-    if (batches < 1 || rows < 1 || cols < 1) return 16;
-    return (size_t)batches * reduction_shares(rows, (int64_t)batches * ((cols + 255) / 256)) * cols * 4;
-}
-
-extern "C" int planmoe_rows_colsum(const void *a, int dtype, int batches, int rows, int cols, const int32_t *live, int live_planes,
-                                   int live_round, void *out, void *workspace, size_t workspace_bytes, void *stream)
-{
-    const char *who = "planmoe_rows_colsum";
-    PM_REQUIRE(dtype_ok(dtype) && batches >= 1 && rows >= 1 && cols >= 1, "%s: bad shape", who);
-    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
-    PM_REQUIRE(cols % vec == 0 && a && out && aligned16(a), "%s: cols must be a multiple of %d, the rows 16-byte aligned", who, vec);
-    PM_REQUIRE(batches < 65536 && (!live || (live_planes >= 1 && live_round >= 1)), "%s: bad live rows", who);
-    PM_REQUIRE(workspace && workspace_bytes >= planmoe_rows_colsum_workspace_bytes(batches, rows, cols), "%s: workspace too small", who);
-    const int shares = reduction_shares(rows, (int64_t)batches * ((cols + 255) / 256));
-    const dim3 grid((unsigned)((cols / vec + WAVE - 1) / WAVE), (unsigned)shares, (unsigned)batches);
-    hipStream_t st = (hipStream_t)stream;
-    PM_DTYPE_SWITCH(dtype, DT,
-        (rows_colsum_kernel<DT><<<grid, 256, 0, st>>>(a, live, live_planes, live_round, batches, rows, cols, shares, (float *)workspace),
-         parts_sum_kernel<DT><<<dim3((unsigned)((cols + WAVE - 1) / WAVE), (unsigned)batches), 256, 0, st>>>((const float *)workspace, shares, cols, out)));
-    PM_LAUNCH_CHECK(who);
-    return 0;
-}
-
-extern "C" size_t planmoe_gate_dw_workspace_bytes(int samples, int model_dim, int experts)
-{
-    if (samples < 1 || model_dim < 1 || experts < 1) return 16;
-    return (size_t)reduction_shares(samples, (model_dim + 255) / 256) * experts * model_dim * 4;
-}
-
-extern "C" int planmoe_gate_dw(const void *x, int dtype, const float *grad_logits, int samples, int model_dim, int experts, void *out,
-                               void *workspace, size_t workspace_bytes, void *stream)
-{
-    const char *who = "planmoe_gate_dw";
-    PM_REQUIRE(dtype_ok(dtype) && samples >= 1 && model_dim >= 1 && experts >= 1, "%s: bad shape", who);
-    const int vec = dtype == PLANMOE_F32 ? 4 : 8;
-    PM_REQUIRE(model_dim % vec == 0 && x && grad_logits && out && aligned16(x), "%s: model_dim must be a multiple of %d, x 16-byte aligned", who, vec);
-    PM_REQUIRE(workspace && workspace_bytes >= planmoe_gate_dw_workspace_bytes(samples, model_dim, experts), "%s: workspace too small", who);
-    const int shares = reduction_shares(samples, (model_dim + 255) / 256);
-    const dim3 grid((unsigned)((model_dim / vec + WAVE - 1) / WAVE), (unsigned)shares);
-    hipStream_t st = (hipStream_t)stream;
-    for (int e0 = 0; e0 < experts; e0 += 8)
-        PM_DTYPE_SWITCH(dtype, DT, (gate_dw_kernel<DT, 8><<<grid, 256, 0, st>>>(x, grad_logits, samples, model_dim, experts, e0, shares, (float *)workspace)));
-    PM_DTYPE_SWITCH(dtype, DT, (parts_sum_kernel<DT><<<dim3((unsigned)(((int64_t)experts * model_dim + WAVE - 1) / WAVE), 1u), 256, 0, st>>>(
-        (const float *)workspace, shares, experts * model_dim, out)));
-    PM_LAUNCH_CHECK(who);
-    return 0;
+    const char *who = "planmoe_layer_combine_bwd_logits";
+    if (layer_rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
+    PM_REQUIRE(dtype_ok(scores_dtype) && top_k <= WAVE && top_k <= experts, "%s: bad scores dtype, or more than %d choices", who, WAVE);
+    PM_REQUIRE(codec == 0 || (bias && scale) || samples == 0, "%s: NULL argument", who);
+    PM_REQUIRE((scores && grad_logits && (!grad_l_aux || first_choice_counts)) || samples == 0, "%s: NULL argument", who);
+    const RouteBwd route{scores, grad_l_aux, grad_l_aux ? first_choice_counts : nullptr, samples, experts, top_k, normalize_gate, route_bwd_group(experts)};
+    return combine_bwd_rows(who, codec ? SEEN_CODES : SEEN_ROWS, grad, rows, bias, scale, dtype, gates, indices, locations, plane_stride, top_k, samples,
+                            model_dim, capacity, grad_rows, nullptr, stream, route, scores_dtype, grad_logits);
 }

@@ -19,6 +19,7 @@
 
 #include "common.hpp"
 #include "offsets.hpp"
+#include "route_bwd.hpp"
 #include "rows.hpp"
 
 namespace pm {
@@ -307,53 +308,18 @@ __global__ __launch_bounds__(TILE) void route_finish_kernel(
 
 // ------------------------------------------------------------------ routing backward
 // Gradient of the gates (and of the GShard loss) with respect to the scores, optionally carried
-// through the softmax to the logits.  A group of lanes per token, as many as there are experts (a power of
-// two, at most a wave), so that scores and gradients are read and written side by side and no lane walks
-// all experts (a thread per token: 9.5 us at 3001 x 10, three choices):
-//   g_j = s_j / D, D = max(sum_i s_i, eps)  =>  ds_j = (dg_j - [sum >= eps] * sum_i dg_i g_i) / D
-//   l_aux = sum_e me[e] ce[e] / T            =>  ds[t][e] += dl * ce[e] / T,  ce[e] = count0[e] * E / T
-//   softmax: dlogit_e = s_e * (ds_e - sum_i ds_i s_i)
+// through the softmax to the logits.  A group of lanes per token, so that scores and gradients are read and written side by
+// side and no lane walks all experts (a thread per token: 9.5 us at 3001 x 10, three choices).
 template <int DT>
-__global__ __launch_bounds__(256) void route_bwd_kernel(
-    const void *__restrict__ scores, const int32_t *__restrict__ indices, const void *__restrict__ dgates,
-    int64_t stride, int samples, int experts, int k, int normalize_gate, const float *__restrict__ dl_aux,
-    const int32_t *__restrict__ count0, int through_softmax, int group, void *__restrict__ dscores)
+__global__ __launch_bounds__(256) void route_bwd_kernel(const RouteBwd r, const int32_t *__restrict__ indices, const void *__restrict__ dgates,
+                                                        int64_t stride, int through_softmax, void *__restrict__ dscores)
 {
     using E = Elem<DT>;
-    const int per_block = 256 / group, t = blockIdx.x * per_block + threadIdx.x / group, e0 = threadIdx.x % group;
-    if (t >= samples) return;
-    const int64_t base = (int64_t)t * experts;
-    const float dl = dl_aux ? dl_aux[0] : 0.f;
-    const float lscale = dl * ((float)experts / (float)samples) / (float)samples;
-    float sum = 0.f, dot = 0.f;
-    for (int j = 0; j < k; ++j) {
-        const int e = indices[(int64_t)j * stride + t];
-        if (e < 0 || e >= experts) continue;             // (no expert: the choice is not there)
-        const float sj = E::load(scores, base + e);
-        sum = E::round(sum + sj);
-        dot += E::load(dgates, (int64_t)j * stride + t) * sj;
-    }
-    const float eps = DT == PLANMOE_F32 ? 1.1920928955078125e-07f : DT == PLANMOE_BF16 ? 0.0078125f : 0.0009765625f;
-    const bool norm = k > 1 && normalize_gate;
-    const float D = norm ? fmaxf(sum, eps) : 1.f;
-    const float corr = (norm && sum >= eps) ? dot / (D * D) : 0.f;      // sum_i dg_i g_i / D
-    auto ds_at = [&](int e) {
-        float v = count0 ? lscale * (float)count0[e] : 0.f;
-        for (int j = 0; j < k; ++j)
-            if (indices[(int64_t)j * stride + t] == e) v += E::load(dgates, (int64_t)j * stride + t) / D - corr;
-        return v;
-    };
-    if (!through_softmax) {
-        for (int e = e0; e < experts; e += group) E::store(dscores, base + e, ds_at(e));
-    } else {
-        float inner = 0.f;
-        for (int e = e0; e < experts; e += group) inner += ds_at(e) * E::load(scores, base + e);
-        for (int d = 1; d < group; d <<= 1) inner += __shfl_xor(inner, d);        // (a group's lanes are all here or all gone)
-        for (int e = e0; e < experts; e += group) {
-            const float s = E::load(scores, base + e);
-            E::store(dscores, base + e, s * (ds_at(e) - inner));
-        }
-    }
+    const int per_block = 256 / r.group, t = blockIdx.x * per_block + threadIdx.x / r.group;
+    if (t >= r.samples) return;                          // (a group's lanes are all here or all gone)
+    route_bwd_token<DT>(r, t, threadIdx.x % r.group, through_softmax, [&](int j) { return indices[(int64_t)j * stride + t]; },
+                        [&](int j) { return E::load(dgates, (int64_t)j * stride + t); },
+                        [&](int e, float v) { E::store(dscores, (int64_t)t * r.experts + e, v); });
 }
 
 // ------------------------------------------------------------------ stand-alone cumsum
@@ -462,14 +428,12 @@ extern "C" int planmoe_route_bwd(const void *scores, int dtype, const int32_t *i
     PM_REQUIRE(!grad_l_aux || first_choice_counts, "planmoe_route_bwd: grad_l_aux needs first_choice_counts");
     if (samples == 0) return 0;
     PM_REQUIRE(scores && indices && grad_gates && grad_scores, "planmoe_route_bwd: NULL argument");
-    const int k = top_k < experts ? top_k : experts;
-    int group = 1;
-    while (group < experts && group < WAVE) group <<= 1;
-    const int per_block = 256 / group;
+    const int group = route_bwd_group(experts), per_block = 256 / group;
+    const RouteBwd r{scores, grad_l_aux, grad_l_aux ? first_choice_counts : nullptr, samples, experts, top_k < experts ? top_k : experts,
+                     normalize_gate, group};
     PM_DTYPE_SWITCH(dtype, DT,
-        (route_bwd_kernel<DT><<<(samples + per_block - 1) / per_block, 256, 0, (hipStream_t)stream>>>(
-            scores, indices, grad_gates, plane_stride, samples, experts, k, normalize_gate, grad_l_aux,
-            grad_l_aux ? first_choice_counts : nullptr, through_softmax, group, grad_scores)));
+        (route_bwd_kernel<DT><<<(samples + per_block - 1) / per_block, 256, 0, (hipStream_t)stream>>>(r, indices, grad_gates, plane_stride,
+                                                                                                   through_softmax, grad_scores)));
     PM_LAUNCH_CHECK("planmoe_route_bwd");
     return 0;
 }

@@ -495,3 +495,37 @@ def test_inference_equals_the_pass_with_autograd(codec, dtype, fp32_gate, T, k):
     assert want.requires_grad
     for y in got:
         assert torch.equal(y, want) and torch.equal(y.l_aux, want.l_aux) and y.l_aux.dtype == want.l_aux.dtype
+
+
+# Everything asked for (the reductions share their launches, the gate's part is added in the combine) against one gradient at a time
+# (each by its own launches): the same sums in the same order.  Up to 8 experts and rows of at most 8 KB: dx in one pass; 9 and 16
+# experts: two groups of eight in the gate weight's gradient; M 4104 and, in fp32, 2056: rows above 8 KB; 4099 tokens: two a wave, one left.
+@pytest.mark.parametrize("T,M,H,E,k,cf", [(4, 8, 8, 1, 1, 1.0), (5, 264, 136, 8, 2, 1.25), (333, 1024, 264, 4, 1, 0.5), (700, 2056, 256, 3, 2, 1.0),
+                                          (40, 4104, 16, 4, 2, 1.0), (4099, 64, 72, 8, 2, 1.0), (130, 520, 72, 9, 3, 1.0), (2049, 256, 512, 16, 2, 1.2)])
+@pytest.mark.parametrize("codec,dtype,fp32_gate", [("no", torch.bfloat16, True), ("no", torch.bfloat16, False), ("int8", torch.bfloat16, True),
+                                                   ("no", torch.float32, True), ("int8", torch.float32, True), ("zfp", torch.float32, True)])
+@pytest.mark.parametrize("with_loss", [True, False])
+def test_all_gradients_equal_one_at_a_time(codec, dtype, fp32_gate, T, M, H, E, k, cf, with_loss):
+    import planmoe_amd
+    E = (E + 3) // 4 * 4 if codec == "zfp" else E          # (its extents are multiples of four)
+    M = min(M, 4096) if dtype == torch.float32 else M            # (as far as the node goes)
+    print("case", codec, dtype, fp32_gate, T, M, H, E, k, cf, with_loss, flush=True)
+    torch.manual_seed(T)
+    layer = planmoe_amd.moe_layer({"type": "top", "k": k, "capacity_factor": cf, "fp32_gate": fp32_gate}, M,
+                                  experts={"type": "ffn", "count_per_node": E, "hidden_size_per_expert": H}, compress_name=codec).to(DEV).to(dtype)
+    x = torch.randn(T, M, device=DEV).to(dtype).requires_grad_(True)
+    gy = torch.randn(T, M, device=DEV).to(dtype)
+    params = [x] + list(layer.parameters())
+
+    def grads(wanted):
+        for p in params: p.requires_grad_(any(p is w for w in wanted))
+        y = layer(x)
+        out = [y, y.l_aux] if with_loss else [y]
+        got = torch.autograd.grad(out, wanted, [gy, torch.full_like(y.l_aux, 0.5)] if with_loss else [gy], allow_unused=True)
+        torch.cuda.synchronize()
+        return got
+
+    whole = grads(params)
+    for p, got in zip(params, whole):
+        one = grads([p])[0]
+        assert got is not None and torch.equal(got, one), (tuple(p.shape), float((got.double() - one.double()).abs().max()))
