@@ -616,8 +616,9 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 // not full.  Between them 128, 160 and 192 rows by 256 columns, where the tiles of 256 rows leave compute units idle and 128 x 128
 // is bound by its operands: the height whose tiles fill the rounds best.  A launch takes its rounds; a round takes its k-tiles,
 // each faster with few compute units at work than with all of them (the clock sinks under the matrix cores), and what a tile
-// costs once; reading the weights is a floor (4.6 TB/s in tiles of 256 columns that are low, 3.3 otherwise).  Fitted to 42
-// timings of 14 shapes: what it picks takes 0.8 % longer than the best (1.10 times the best without the low tiles).
+// costs once.  Reading the weights is a floor: what memory gives, or, with few work-groups, what they have on their way (28 GB/s for each
+// in 128 x 128, 45 in 256 columns).  Fitted to 450 timings of 110 shapes with the weights in the last cache and out of it: what it picks takes
+// 1.1 % longer than the best.
 // us in one launch, rows +- sqrt(rows) in use, nn:
 //   experts x rows, in, out      128 x 128    256    128    160    192 x 256
 //   8 x 500, 2048, 2048             49         48     57     42     42     (54 in 256 and a launch of quarters)
@@ -626,6 +627,8 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 //   8 x 250, 2048, 2048             31         43     29     32     35
 //   8 x 2000, 4096, 1024           142        171    158    129    140
 //   8 x 4096, 4096, 4096          1125        846    987    968    930
+//   8 x 110, 2688, 2560             36         58     52     54     55     (weights cold)
+//   8 x 60, 1024, 4096              19         29     23     25     26     (weights cold)
 //
 // A last round of large tiles that is at most half full may be a launch of its own, in quarters (8 experts of 4096 +- 100
 // rows by 1024 columns: 512 tiles and a few, whose third round would take half as long again as the other two).
@@ -651,31 +654,53 @@ struct GemmCost {
     double quarters(double t) const              // tiles of 128 x 128, two work-groups per compute unit
     {
         const double full = std::floor(t / (2 * cu)), rest = t - full * 2 * cu;
-        return full * (kt + 2) + (rest <= 0.01 ? 0. : rest <= cu ? (0.41 + 0.19 * rest / cu) * kt + 2 : (0.6 + 0.4 * (rest - cu) / cu) * kt + 2);
+        return full * (kt + 2) + (rest <= 0.01 ? 0. : rest <= cu ? (0.41 + 0.19 * rest / cu) * kt + 2 : (0.85 + 0.25 * (rest - cu) / cu) * kt + 2);
     }
-    double floor(double rate) const { return (double)weight_bytes * 1e-6 / rate + 6; }
-    double small() const { return std::max(quarters(tiles(128, 128)) + 7, floor(3.3)); }
-    double big() const { return std::max(rounds(tiles(256, 256), 1.0, 1.4, 3) + 6, floor(3.3)); }
+    // reading the weights: what memory gives, or what the tiles' columns that are worked on ask for, each `each` TB/s
+    double floor(double t, int bn, double each, double once) const
+    {
+        const double columns = (double)((n + bn - 1) / bn * batches) * std::min(1., cu / t);
+        return (double)weight_bytes * 1e-6 / std::min(4.8, each * columns) + once;
+    }
+    double small() const
+    {
+        const double t = tiles(128, 128);
+        return std::max(quarters(t) + 4.5, t <= cu ? floor(t, 128, 0.028, 5.5) : (double)weight_bytes * 1e-6 / 3.5 + 6);
+    }
+    double big() const
+    {
+        const double t = tiles(256, 256);
+        return std::max(rounds(t, 1.0, 1.4, 3) + 6, floor(t, 256, 0.045, 8));
+    }
     // the last round as a launch of quarters; with many rounds it hardly counts
     double big_and_quarters() const
     {
         const double t = tiles(256, 256), full = std::floor(t / cu), last = t - full * cu;
-        return t < 6 * cu && full > 0 && last > 0.01 && 2 * last <= cu ? std::max(full * (1.4 * kt + 3) + 6 + quarters(4 * last) + 10, floor(3.3)) : 1e30;
+        return t < 6 * cu && full > 0 && last > 0.01 && 2 * last <= cu ? std::max(full * (1.4 * kt + 3) + 6 + quarters(4 * last) + 10, floor(t, 256, 0.045, 8)) : 1e30;
     }
     double low(int height) const                 // height: 128, 160, 192
     {
         const double t = tiles(height, 256), us = height == 128 ? rounds(t, 0.58, 0.9, 2) : height == 160 ? rounds(t, 0.7, 1.07, 2) : rounds(t, 0.79, 1.25, 2);
-        return std::max(us + 6, floor(4.6));
+        return std::max(us + 6, floor(t, 256, 0.045, 6));
     }
 };
 
 // The column sums of a masked product: a tile of so many rows has so many slots (0 rows: one slot for everything)
 struct GemmSlots { int rows, per_tile; };
 
-// few rows per batch against a whole weight
-bool gemm_is_skinny(int64_t m, int64_t n, int64_t k, int64_t batches)
+// Few rows per batch against a whole weight.  Up to 16 rows always; up to 32 where there is a compute unit for each
+// work-group, and up to 64 where there is in pieces of 64 columns: beyond that a tile's operands, read once for all its rows, win.
+// us, cold weights, few rows and tiles, nn, nt:
+//   8 x 40 rows, 2688 -> 2560     35, 33 and 33, 29      8 x 20, same       29, 28 and 32, 28
+//   16 x 40, 2688 -> 2560         66, 62 and 53, 47      16 x 20, same      56, 52 and 52, 46
+//   16 x 40, 1024 -> 4096         37, 36 and 31, 29      8 x 20, same       17, 16 and 19, 17
+//   8 x 40, 4096 -> 1024          35, 32 and 39, 36      8 x 8 2688 -> 2560 26, 25 and 32, 28
+bool gemm_is_skinny(bool nt, int m, int n, int64_t k, int batches)
 {
-    return m <= SKINNY_ROWS && batches <= 65535 && n * k * 2 < ((int64_t)1 << 31);
+    if (m > SKINNY_ROWS || batches > 65535 || n * k * 2 >= ((int64_t)1 << 31)) return false;
+    const int64_t cu = compute_units();
+    auto groups = [&](int width) { return (int64_t)((n + width - 1) / width) * batches; };
+    return m <= 16 || groups(m <= 32 ? gemm_skinny_width(nt, n, batches) : 64) <= cu;
 }
 
 template <bool TA, bool TB, bool GRAD>
@@ -684,7 +709,7 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
     if (sums) *sums = GemmSlots{128, 2};
     const bool contiguous = p.lda == p.K && p.ldb == (TB ? p.N : p.K) && p.ldc == p.N && p.sB == (int64_t)p.N * p.K && p.sA == (int64_t)p.M * p.K &&
                             p.sC == (int64_t)p.M * p.N;
-    if (!TA && contiguous && gemm_is_skinny(p.M, p.N, p.K, p.batches)) {
+    if (!TA && contiguous && gemm_is_skinny(!TB, p.M, p.N, p.K, p.batches)) {
         if (sums) *sums = GemmSlots{0, 1};
         SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
         return gemm_skinny_run(!TB, few, stream, who);

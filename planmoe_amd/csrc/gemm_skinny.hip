@@ -11,7 +11,7 @@
 //   nt: lane = (16 columns, 4 groups of 16 k): two loads of 8 k, operands as they are; the four groups of a
 //       row make 128 consecutive bytes.
 // 8 experts x 2 rows, 67 MB of weights: 1024 -> 4096 12.5 us, 4096 -> 1024 (64 columns for a work-group: 128
-// work-groups) 14.2 us (128 columns and one step in flight: 14.6 and 17.2 us; 128 x 128 tiles: 24 us).
+// work-groups) 14.2 us (128 x 128 tiles: 24 us).
 #include "gemm_skinny.hpp"
 
 namespace pm {
@@ -116,8 +116,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
     }
 
     // the waves' sums meet in LDS, 16 rows at a time; a lane has rows 4 g .. + 3 of column C l16 + c (nn) or 16 c + l16 (nt)
-    constexpr int PER = 16 * SK_COLS / (WAVES * 64);        // outputs of a thread: 1, 2 or 4 columns of a row
-    const int row_t = tid * PER / SK_COLS, col_t = tid * PER % SK_COLS;
+    constexpr int EACH = (16 * SK_COLS + WAVES * 64 - 1) / (WAVES * 64), PER = EACH == 3 ? 4 : EACH;        // outputs of a thread: 1, 2 or 4 columns of a row
+    const bool writes = tid * PER < 16 * SK_COLS;           // (96 columns: three threads in four)
+    const int row_t = writes ? tid * PER / SK_COLS : 0, col_t = tid * PER % SK_COLS;
     float *mine = part + wave * 16 * SK_PITCH;
     uint16_t *out = p.C + (int64_t)e * p.M * p.N;
     float colsum = 0.f;                                     // GRAD: of column n0 + tid
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
 #pragma unroll
             for (int x = 0; x < PER; ++x) v[x] += part[(w * 16 + row_t) * SK_PITCH + col_t + x];
         const int row = 16 * m + row_t, col = n0 + col_t;
-        const bool inside = row < rows && col < p.N;        // (N is a multiple of 8: a thread's columns are in or out together)
+        const bool inside = writes && row < rows && col < p.N;        // (N is a multiple of 8: a thread's columns are in or out together)
 #pragma unroll
         for (int x = 0; x < PER; ++x) {
             v[x] = bf16_to_f32(f32_to_bf16(v[x]));
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         if (GRAD && p.colsum) {
             __syncthreads();
 #pragma unroll
-            for (int x = 0; x < PER; ++x) part[row_t * SK_PITCH + col_t + x] = v[x];
+            for (int x = 0; x < PER; ++x) if (writes) part[row_t * SK_PITCH + col_t + x] = v[x];
             __syncthreads();
             if (tid < SK_COLS)
 #pragma unroll
@@ -190,8 +191,14 @@ static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *wh
     return 0;
 }
 
-// 64 columns for a work-group, and more steps in flight, where 128 would leave compute units idle (8 experts, 2048 x 2048:
-// nt 21.5 -> 16.8 us for 20 rows, 26.5 -> 19.1 for 40, nn 18.6 -> 17.7 for 40, but 16.4 against 17.1 for 20)
+// Columns of a work-group: 64, with more steps in flight, where there is a compute unit for each work-group; else the width that
+// takes a compute unit through the fewest columns, 128 where two widths do (nn in 96, whose pieces of a row are 12 bytes, is no faster than in 128).
+// us with cold weights, 64, 96 and 128 columns:
+//   8 experts x 8 rows, 2688 -> 2560    nn 36, 29, 26   nt 33, 25, 29        (320, 216 and 160 work-groups)
+//   8 x 8, 3072 -> 1536                 nn 20, 26, 25   nt 21, 25, 31
+//   16 x 8, 3072 -> 1536                nn 40, 35, 32   nt 40, 31, 35
+//   8 x 8, 1024 -> 4096                 nn 20, 20, 15   nt 17, 19, 14
+//   8 x 20, 4096 -> 1024                nn 28, 35, 36   nt 30, 35, 43
 int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
 {
     const bool grad = p.mask != nullptr;
@@ -199,11 +206,29 @@ int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
     (!nt ? skinny_launch<false, MF, C, U_NN, WAVES_NN, false>(p, stream, who)            \
      : grad ? skinny_launch<true, MF, C, U_NT, WAVES_NT, true>(p, stream, who)           \
             : skinny_launch<true, MF, C, U_NT, WAVES_NT, false>(p, stream, who))
-    const bool narrow = (int64_t)((p.N + 127) / 128) * p.batches < compute_units();
-    if (p.M <= 16) return narrow ? PM_SK(1, 4, 4, 16, 2, 16) : PM_SK(1, 8, 1, 16, 1, 16);
-    if (p.M <= 32) return narrow && nt ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);        // (nt holds 16 KB of weight per step: 8 waves' registers)
-    return narrow ? PM_SK(4, 4, 5, 8, 2, 8) : PM_SK(4, 8, 1, 8, 1, 8);
+    const int width = gemm_skinny_width(nt, p.N, p.batches);
+    // (what is not built is not asked for: nn in 96 columns; more than 32 rows in more than 64, gemm_is_skinny)
+    if (p.M <= 16) {
+        if (width == 96) return grad ? skinny_launch<true, 1, 6, 1, 16, true>(p, stream, who) : skinny_launch<true, 1, 6, 1, 16, false>(p, stream, who);
+        return width == 64 ? PM_SK(1, 4, 4, 16, 2, 16) : PM_SK(1, 8, 1, 16, 1, 16);
+    }
+    if (p.M <= 32) {                             // (nt holds 12 or 16 KB of weight per step: 8 waves' registers)
+        if (width == 96) return grad ? skinny_launch<true, 2, 6, 1, 8, true>(p, stream, who) : skinny_launch<true, 2, 6, 1, 8, false>(p, stream, who);
+        return width == 64 ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);
+    }
+    return PM_SK(4, 4, 5, 8, 2, 8);
 #undef PM_SK
+}
+
+int gemm_skinny_width(bool nt, int n, int batches)
+{
+    const int64_t cu = compute_units();
+    auto groups = [&](int width) { return (int64_t)((n + width - 1) / width) * batches; };
+    auto columns = [&](int width) { return (groups(width) + cu - 1) / cu * width; };
+    if (groups(64) <= cu) return 64;
+    if (!nt) return 128;
+    if (columns(128) <= columns(64) && columns(128) <= columns(96)) return 128;
+    return columns(96) <= columns(64) ? 96 : 64;
 }
 
 } // namespace pm

@@ -415,3 +415,41 @@ def test_expert_gemm_low_tiles(cap, n, k, hint, counts):
             assert bool((out[e, r:] == 7.0).all()), e
         stored = masked[e, :r].double()
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), e
+
+
+# Few rows where there are more pieces of 64 columns than compute units: up to 16 rows in 96 (nt) or 128 columns, up to 32 where those have a
+# compute unit each, in tiles otherwise; columns that no width divides, an expert without rows, and one with all.
+@pytest.mark.parametrize("B,n,k", [(8, 2568, 72), (16, 2488, 136), (7, 4104, 520), (64, 264, 1032)])
+@pytest.mark.parametrize("m", [3, 16, 17, 32, 33, 64, 65])
+def test_expert_gemm_few_rows_and_many_columns(B, n, k, m):
+    from planmoe_amd import ops
+    print("case", B, n, k, m, flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    dtype = torch.bfloat16
+    live = torch.randint(0, m + 1, (1, B), generator=g, dtype=torch.int32)
+    live[0, 0], live[0, 1] = 0, m
+    a, bias = torch.randn(B, m, k, generator=g).to(dtype).to(DEV), torch.randn(B, n, generator=g).to(dtype).to(DEV)
+    w, h = torch.randn(B, k, n, generator=g).to(dtype).to(DEV), torch.randn(B, m, n, generator=g).clamp(min=0).to(dtype).to(DEV)
+    for e in range(B):
+        a[e, int(live[0, e]):] = float("nan")
+    wt = w.transpose(1, 2).contiguous()
+    nn = torch.full((B, m, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    kw = dict(live=live.to(DEV), rows_hint=(m + 1) // 2)
+    ops.expert_gemm("nn", a, w, bias, relu=True, out=nn, **kw)
+    ops.expert_gemm("nt", a, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, out=masked, **kw)
+    torch.cuda.synchronize()
+    for e in range(B):
+        r = int(live[0, e])
+        x, y = a[e, :r].double(), w[e].double()
+        ref, mag = x @ y, x.abs() @ y.abs()
+        tol = _bound(ref, mag, k, dtype)
+        biased = ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all())
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all())
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all())
+        for out in (nn, nt, masked):
+            assert bool((out[e, r:] == 7.0).all())
+        stored = masked[e, :r].double()          # the sums are of what was stored
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, dtype)).all())
