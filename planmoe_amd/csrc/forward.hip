@@ -1,7 +1,7 @@
 // The forward chain in two launches (three when top_k > 4):
 //
 //   gate_route_kernel     x is read once: gate-logits GEMM on the matrix cores, then, for the
-//                         work-group's 64 (or 32) tokens = one routing group, softmax, k-fold
+//                         work-group's 64 (32 or 16) tokens = one routing group, softmax, k-fold
 //                         arg-max, gates, the rank of every token among the group's tokens with
 //                         the same choice, and the group's expert histogram.
 //   dispatch_int8_routed  slot = rank in group + entries of earlier groups and planes (all first
@@ -29,13 +29,17 @@
 namespace pm {
 
 // tokens per work-group of the gate kernel = tokens per routing group (one lane each in the
-// routing epilogue): 64, or 32 on the split-K path (up to 16 experts) when 64 would leave
-// compute units without a work-group
+// routing epilogue): 64, or fewer where 64 would leave compute units without a work-group
 inline int fwd_group_tokens(int experts, int samples)
 {
     // measured at 8 experts: 16384 tokens (256 groups of 64) 39 us with 64, 44 us with 32;
     // 8192 tokens 32 us with 64, 28 us with 32
-    return (experts <= 16 && samples < 64 * 256) ? 32 : 64;
+    if (experts <= 16) return samples < 64 * 256 ? 32 : 64;
+    // as many groups as compute units at most (16 tokens: where four waves find a share of the experts).  us of the send side, bf16, with 64, 32, 16:
+    //   64 experts x 1368   48 tokens 26, 22, 21;  4074 33, 29, 27;  8000 35, 32, 42;  16000 39, 47, 74
+    //   32 experts x 1368   48 tokens 24, 20;      4074 33, 24;      8000 35, 28;      16000 42, 42
+    if (experts > 32 && samples <= 16 * 256) return 16;
+    return samples <= 32 * 256 ? 32 : 64;
 }
 constexpr int FWD_LOSS_PARTS = 64;
 inline void *fwd_tables(void *workspace) { return (char *)workspace + FWD_TABLES_OFFSET; }
@@ -180,7 +184,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
 {
     using S = Elem<SDT>;
     const bool first = ONE == ONE_OFF || blockIdx.x == 0;        // (of work-groups that route the same tokens)
-    static_assert(GROUP == 64 || (SPLITK && GROUP == 32), "the LDS-shared variant is built for 64 tokens");
+    static_assert(GROUP == 64 || GROUP == 32 || (!SPLITK && GROUP == 16), "tokens of a group");
     constexpr int COLS = 16 * NT + 1;
     // split-K: part[4][GROUP][COLS] floats; else the weight buffers / logits[GROUP][COLS]
     __shared__ uint4 smem[SPLITK ? (4 * GROUP * COLS + 3) / 4 : gate_lds_vectors<NT>()];
@@ -224,7 +228,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
     } else if constexpr (SPLITK) {
         gate_tile_partials<DT, NT, GROUP / 16, 4, STATS>(x, wg, t0, samples, model_dim, experts, part, pstat);
     } else {
-        gate_tile_lds<DT, NT, STATS>(x, wg, t0, samples, model_dim, experts, smem, pstat[0]);
+        gate_tile_lds<DT, NT, STATS, GROUP>(x, wg, t0, samples, model_dim, experts, smem, pstat[0]);
     }
     __syncthreads();
 
@@ -765,7 +769,8 @@ static void launch_gate_route(int experts, int groups, int group_tokens, hipStre
 #define PM_GR_(NT, CAP, SPLITK, GROUP)                                                                   \
     gate_route_kernel<DT, SDT, NT, CAP, SPLITK, GROUP><<<groups, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
         k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws, nullptr, 0)
-#define PM_GR(NT, CAP, SPLITK) do { if (SPLITK && group_tokens == 32) PM_GR_(NT, CAP, SPLITK, (SPLITK ? 32 : 64)); \
+#define PM_GR(NT, CAP, SPLITK) do { if (group_tokens == 32) PM_GR_(NT, CAP, SPLITK, 32); \
+                                    else if (group_tokens == 16) PM_GR_(NT, CAP, SPLITK, (NT == 4 ? 16 : 32)); \
                                     else PM_GR_(NT, CAP, SPLITK, 64); } while (0)
     // split-K measured faster than the LDS-shared variant up to 16 experts (30.7 vs 44.4 us at
     // 16384 x 4096 bf16, 8 experts), and the other way round above (168 -> 48 us at 64 experts)
@@ -838,7 +843,7 @@ static void fwd_plan(FwdPlan &plan, void *workspace, int samples, int experts, i
     plan.experts_per_block = go_experts_per_block(experts, plan.k);
     plan.blocks = (experts + plan.experts_per_block - 1) / plan.experts_per_block;
     plan.merged = plan.k <= 4;
-    plan.one = plan.groups == 1 && plan.merged && plan.group_tokens == 32;
+    plan.one = plan.groups == 1 && plan.merged && experts <= 16 && plan.group_tokens == 32;
     plan.ws = fwd_ws(workspace, plan.groups, plan.k, experts, samples);
 }
 

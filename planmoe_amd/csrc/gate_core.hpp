@@ -191,25 +191,26 @@ __device__ __forceinline__ void gate_tile_partials(const void *__restrict__ x,
 // ---------------------------------------------------------------------------------------------
 // Variant for more than 16 experts: the gate weights are the larger operand per token tile, so
 // the work-group shares them through LDS instead of every wave streaming them from L2.
-//   * a work-group of 4 waves owns 64 tokens, wave w the tokens [16 w, 16 w + 16) over the
-//     whole K axis (no split-K: the accumulators of a token stay in one wave);
+//   * a work-group of 4 waves owns TOKENS tokens: 64, wave w the tokens [16 w, 16 w + 16) over the
+//     whole K axis (no split-K: the accumulators of a token and an expert stay in one wave), or 32 or 16, two or
+//     four waves to the same tokens and each with its share of the experts;
 //   * K is walked in chunks of 16 vectors (256 bytes of every row).  The chunk of all 16*NT
 //     gate-weight rows is copied global -> registers -> LDS by the 256 threads with fully
-//     coalesced 16-byte loads, double buffered, one barrier per chunk;
+//     coalesced 16-byte loads, two buffers, one barrier per chunk;
 //   * inside LDS a row's 16 vectors are stored at (vector ^ (row % 16)): the 16 lanes of an
 //     MFMA fragment read (different rows, same logical vector) hit 16 different vector slots,
 //     i.e. all 64 banks once;
-//   * token fragments go straight from global memory to registers, one chunk ahead.
+//   * token fragments go straight from global memory to registers; both are asked for DEPTH chunks ahead.
 // Result: logits[token][expert] (fp32) in LDS.  `smem` must hold gate_lds_vectors<NT>() uint4;
 // the logits alias the weight buffers (a barrier separates the two uses).
 // With STATS the wave leaves the words of RowStats<bf16>::reduced() of its rows in pstat[token].
 template <int NT> __host__ __device__ constexpr int gate_lds_vectors()
 {
-    // 2 buffers x (16 NT rows x 16 vectors)  vs  64 x (16 NT + 1) floats
+    // 2 buffers x (16 NT rows x 16 vectors)  vs  (up to) 64 x (16 NT + 1) floats
     return (2 * 16 * NT * 16) > ((64 * (16 * NT + 1) + 3) / 4) ? (2 * 16 * NT * 16) : ((64 * (16 * NT + 1) + 3) / 4);
 }
 
-template <int DT, int NT, bool STATS = false>
+template <int DT, int NT, bool STATS = false, int TOKENS = 64>
 __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const void *__restrict__ wg,
                                               int t0, int samples, int model_dim, int experts,
                                               uint4 *smem, int32_t (*pstat)[3] = nullptr)
@@ -217,16 +218,19 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
     static_assert(!STATS || DT == PLANMOE_BF16, "row statistics ride along for bf16 only");
     static_assert(NT == 1 || NT == 2 || NT == 4 || NT == 8, "16 NT rows are dealt to 256 threads, 16 per row");
     constexpr int V = Elem<DT>::VEC;
-    constexpr int ROWS = 16 * NT;
+    constexpr int ROWS = 16 * NT, SHARE = 64 / TOKENS, OWN = NT / SHARE;         // OWN: fragments of experts of a wave
+    static_assert(OWN >= 1 && OWN * SHARE == NT, "a wave's experts");
     constexpr int BV = ROWS / 16;                    // weight vectors per thread and chunk
+    constexpr int DEPTH = NT <= 2 ? 4 : NT == 4 ? 3 : 2;       // chunks on their way
     const int tid = threadIdx.x, w = tid >> 6, l = lane_id();
     const int m = l & 15, g = l >> 4;
+    const int tile = __builtin_amdgcn_readfirstlane(w / SHARE), own0 = __builtin_amdgcn_readfirstlane(w % SHARE) * OWN;
     const int nv = model_dim / V;                    // 16-byte vectors per row
 
     RowStats<PLANMOE_BF16, true> st;
     if constexpr (STATS) st.init();
 
-    const uint4 *ap = reinterpret_cast<const uint4 *>(x) + (int64_t)min(t0 + w * 16 + m, samples - 1) * nv;
+    const uint4 *ap = reinterpret_cast<const uint4 *>(x) + (int64_t)min(t0 + tile * 16 + m, samples - 1) * nv;
     const int bvec = tid & 15;                       // thread's vector inside the chunk
     const uint4 *bp[BV];
     int bdst[BV];
@@ -237,9 +241,9 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
         bdst[i] = row * 16 + (bvec ^ (row & 15));
     }
 
-    f32x4 acc[NT];
+    f32x4 acc[OWN];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < OWN; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int full = nv / 16, rem = nv % 16;
     // full chunks: straight-line loads (no predicate, no branch around a prefetch, so that the
@@ -258,14 +262,14 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
         for (int i = 0; i < BV; ++i) smem[buf * ROWS * 16 + bdst[i]] = b[i];
     };
     auto compute = [&](const uint4 (&a)[4], int buf) {
-        const uint4 *bb = smem + buf * ROWS * 16 + m * 16;
+        const uint4 *bb = smem + buf * ROWS * 16 + own0 * 256 + m * 16;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            uint4 bf[NT];
+            uint4 bf[OWN];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) bf[nt] = bb[nt * 256 + ((4 * s + g) ^ m)];
+            for (int nt = 0; nt < OWN; ++nt) bf[nt] = bb[nt * 256 + ((4 * s + g) ^ m)];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) Mma<DT>::run(a[s], bf[nt], acc[nt]);
+            for (int nt = 0; nt < OWN; ++nt) Mma<DT>::run(a[s], bf[nt], acc[nt]);
         }
     };
     auto scan = [&](const uint4 (&a)[4]) {
@@ -275,27 +279,34 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
         }
     };
 
-    uint4 a0[4], a1[4], bs[BV];
+    uint4 a[DEPTH][4], bs[DEPTH][BV];
+    auto chunk = [&](int c, int i) {
+        store_b(bs[i], c & 1);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");       // (not the loads)
+    };
     if (full > 0) {
-        load_a(a0, 0);
-        load_b(bs, 0);
-        store_b(bs, 0);
-        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) { load_b(bs[i], min(i, full - 1)); load_a(a[i], min(i, full - 1)); }
         int c = 0;
-        while (true) {
-            if (c + 1 >= full) { scan(a0); compute(a0, 0); __syncthreads(); break; }
-            load_a(a1, c + 1); load_b(bs, c + 1);
-            scan(a0); compute(a0, 0);
-            store_b(bs, 1);
-            __syncthreads();
-            ++c;
-            if (c + 1 >= full) { scan(a1); compute(a1, 1); __syncthreads(); break; }
-            load_a(a0, c + 1); load_b(bs, c + 1);
-            scan(a1); compute(a1, 1);
-            store_b(bs, 0);
-            __syncthreads();
-            ++c;
+        for (; c + DEPTH <= full; c += DEPTH) {
+#pragma unroll
+            for (int i = 0; i < DEPTH; ++i) {
+                const int then = min(c + i + DEPTH, full - 1);
+                chunk(c + i, i);
+                load_b(bs[i], then);
+                scan(a[i]);
+                compute(a[i], (c + i) & 1);
+                load_a(a[i], then);
+            }
         }
+#pragma unroll
+        for (int i = 0; i < DEPTH - 1; ++i)
+            if (c + i < full) {
+                chunk(c + i, i);
+                scan(a[i]);
+                compute(a[i], (c + i) & 1);
+            }
+        __syncthreads();
     }
     if (rem) {
         // last, partial chunk: vectors past the row end are read from a clamped index (valid
@@ -304,19 +315,19 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int v = 4 * s + g;
-            a0[s] = ap[o + min(v, rem - 1)];
+            a[0][s] = ap[o + min(v, rem - 1)];
         }
-        scan(a0);
+        scan(a[0]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) if (4 * s + g >= rem) a0[s] = make_uint4(0, 0, 0, 0);
+        for (int s = 0; s < 4; ++s) if (4 * s + g >= rem) a[0][s] = make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < BV; ++i) {
-            bs[i] = bp[i][o + min(bvec, rem - 1) - bvec];
-            if (bvec >= rem) bs[i] = make_uint4(0, 0, 0, 0);
+            bs[0][i] = bp[i][o + min(bvec, rem - 1) - bvec];
+            if (bvec >= rem) bs[0][i] = make_uint4(0, 0, 0, 0);
         }
-        store_b(bs, 0);                                  // every wave is past the barrier of the loop
+        store_b(bs[0], 0);                               // every wave is past the barrier behind the loop
         __syncthreads();
-        compute(a0, 0);
+        compute(a[0], 0);
         __syncthreads();
     }
 
@@ -329,15 +340,15 @@ __device__ __forceinline__ void gate_tile_lds(const void *__restrict__ x, const 
             b = max(b, __shfl_xor(b, off, WAVE));
             n = max(n, __shfl_xor(n, off, WAVE));
         }
-        if (g == 0) { pstat[w * 16 + m][0] = a; pstat[w * 16 + m][1] = b; pstat[w * 16 + m][2] = n; }
+        if (g == 0 && own0 == 0) { pstat[tile * 16 + m][0] = a; pstat[tile * 16 + m][1] = b; pstat[tile * 16 + m][2] = n; }
     }
 
     // every wave is past its last read of the weight buffers (barrier above): reuse them
     float (*logits)[ROWS + 1] = reinterpret_cast<float (*)[ROWS + 1]>(smem);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < OWN; ++nt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) logits[w * 16 + 4 * g + i][nt * 16 + m] = acc[nt][i];
+        for (int i = 0; i < 4; ++i) logits[tile * 16 + 4 * g + i][(own0 + nt) * 16 + m] = acc[nt][i];
 }
 
 } // namespace pm

@@ -223,6 +223,16 @@ def test_fused_forward_matches_unfused_and_oracle(T, M, E, k, cf, dtype, fp32_ga
         assert abs(float(r2["l_aux"]) - float(out["l_aux"])) <= 1e-6 * abs(float(out["l_aux"]))
 
 
+# more than 16 experts: groups of 16, 32 and 64 tokens, either side of where they change and of a group's end; rows of less than a
+# chunk, of as many chunks as are on their way, of one more and a piece; 17 to 64 experts
+@pytest.mark.parametrize("T,M,E,k,dtype", [
+    (1, 8, 64, 1, torch.bfloat16), (15, 128, 33, 2, torch.bfloat16), (16, 392, 64, 2, torch.bfloat16), (17, 256, 33, 4, torch.float32),
+    (33, 520, 17, 2, torch.bfloat16), (31, 640, 32, 1, torch.float32), (65, 512, 20, 3, torch.float16), (4096, 264, 48, 1, torch.bfloat16),
+    (4097, 384, 64, 2, torch.bfloat16), (8192, 64, 32, 2, torch.float32), (8193, 136, 17, 2, torch.bfloat16), (8193, 72, 64, 1, torch.bfloat16)])
+def test_fused_forward_many_experts_group_sizes(T, M, E, k, dtype):
+    test_fused_forward_matches_unfused_and_oracle(T, M, E, k, 1.25, dtype, True, T % 2 == 1)
+
+
 @pytest.mark.parametrize("T,M,E,k,cf,dtype,fp32_gate,use_bias", [
     (1000, 512, 8, 2, 1.25, torch.bfloat16, True, False), (33, 256, 4, 2, 1.0, torch.bfloat16, True, False),
     (4096, 1024, 64, 1, 1.0, torch.bfloat16, True, True), (500, 2048, 2, 2, 1.0, torch.float32, True, False),
