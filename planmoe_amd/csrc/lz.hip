@@ -15,14 +15,14 @@
 //           literals or one match per step with ballots and scalar bit scans.
 //   pack    token ranks and byte offsets come from one packed wave scan; flags and token bytes
 //           are put together in LDS and copied out with aligned word stores.
-// The launches: sizes of every block (match + parse, nothing written but two integers and a
-// class byte per block), an in-place exclusive scan of the sizes (chunks, then chunk totals),
-// placement (stored blocks are copied straight through, the others analysed again and packed at
-// their final offset), and a launch that zeroes what lies beyond the totals.  Up to 16 MB there is one
-// chunk: no totals to scan, and the placement's spare work-groups do the zeroing.  The reference
+// The launches: sizes of every block (match + parse; two integers and a class byte per block are written, and, of a block
+// with matches, its tokens: two bytes a position), an in-place exclusive scan of the sizes by chunks, and
+// placement (stored blocks are copied straight through, the tokens of the others packed at
+// their final offset; a wave adds up the totals of the chunks before its own, and spare work-groups zero what lies beyond all).  134 MB of N(0, 1):
+// 46 + 7 + 54 us; with matches everywhere (half of the values zero) 745 + 7 + 48, and 770 for the placement when it analysed those blocks again.  The reference
 // stages every block at a fixed stride in a buffer as large as the input, scans with a library
-// call and copies everything once more (gpulz.cu:148-211, 460-494, 220-258); here no
-// full-size temporary exists and no work-group ever waits for another.
+// call and copies everything once more (gpulz.cu:148-211, 460-494, 220-258); here stored blocks and
+// those of one value, all that most buffers are made of, are never staged and no work-group ever waits for another.
 #include "common.hpp"
 
 namespace pm {
@@ -90,6 +90,30 @@ struct LzBlock {
     uint32_t match_mask, start_mask;               // owned positions with a match / that start a token
     uint32_t tok_base, byte_base;                  // tokens and token bytes before this lane
     uint32_t flag_bytes, data_bytes;               // sizes of the block
+
+    // tokens and token bytes before this lane, totals of the block
+    __device__ __forceinline__ void count()
+    {
+        const uint32_t ntok = __popc(start_mask), nmatch = __popc(start_mask & match_mask);
+        uint32_t total;
+        const uint32_t before = wave_exclusive_sum(ntok | ((4u * ntok - 2u * nmatch) << 16), total);
+        tok_base = before & 0xffffu;
+        byte_base = before >> 16;
+        flag_bytes = ((total & 0xffffu) + 7u) >> 3;
+        data_bytes = total >> 16;
+    }
+    // the tokens that start at the lane's positions, 16 bits each: bit 15 a token, bit 14 a match, its offset - 1 and its length - 1
+    __device__ __forceinline__ uint4 tokens() const
+    {
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t l = (((i < 4 ? lens_lo : lens_hi) >> (8 * (i & 3))) - 1u) & 0x1fu, o = (((i < 4 ? offs_lo : offs_hi) >> (8 * (i & 3))) - 1u) & 0x1fu;
+            const uint32_t t = ((start_mask >> i) & 1u) ? ((match_mask >> i) & 1u ? 0xc000u | (o << 5) | l : 0x8000u) : 0u;
+            w[i >> 1] |= t << (16 * (i & 1));
+        }
+        return make_uint4(w[0], w[1], w[2], w[3]);
+    }
 };
 
 // 8 consecutive symbols per lane, zero beyond the end of the input
@@ -197,7 +221,7 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
         const int i = __builtin_ctz(todo);
         const uint32_t room = (uint32_t)(LZ_SYMS - 8 * lane - i);       // symbols left in the block
         const uint32_t mask = hmask[i * LZ_PITCH + lane];
-        uint32_t alive = mask, runs[6] = {0, 0, 0, 0, 0, 0};
+        uint32_t alive = mask, runs[6] = {0, 0, 0, 0, 0, 0}, room_mask = 0x7fffffffu;
 #pragma unroll 1
         for (int k0 = 0; k0 < LZ_WINDOW; k0 += 8) {
             if (__ballot(alive != 0) == 0) break;
@@ -207,14 +231,22 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
                 const int at = i + k0 + t + 1;
                 next[t] = hmask[(at & 7) * LZ_PITCH + lane + (at >> 3)];
             }
+            // k = k0 + t + 1: a run of k ends here, or (32 - j symbols from bit j on) with the window.  Seven of the eight k share
+            // their upper three bits; the eighth has the next ones and no lower bits.
+            uint32_t low = 0, last = 0;
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
-                const int k = k0 + t + 1;               // a run of k ends here, or (32 - j symbols from bit j on) with the window
-                const uint32_t on = alive & next[t] & (0x7fffffffu >> (k - 1)), dead = alive & ~on;
+                const uint32_t on = alive & next[t] & (room_mask >> t), dead = alive & ~on;
 #pragma unroll
-                for (int q = 0; q < 6; ++q) runs[q] |= dead & (0u - (((uint32_t)k >> q) & 1u));
+                for (int q = 0; q < 3; ++q) if (((t + 1) >> q) & 1) runs[q] |= dead;
+                if (t < 7) low |= dead; else last = dead;
                 alive = on;
             }
+            room_mask >>= 8;
+            const uint32_t here = (uint32_t)k0 >> 3, then = here + 1u;
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                runs[3 + q] |= (low & (0u - ((here >> q) & 1u))) | (last & (0u - ((then >> q) & 1u)));
         }
         uint32_t longest = 0, with = mask;              // of all runs, whether the walk gets to them or not
 #pragma unroll
@@ -265,22 +297,14 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
         cur = nxt + step;                              // step >= 1 whenever nxt < 512
     }
 
-    // ---- sizes: tokens and token bytes before this lane, totals of the block
-    const uint32_t ntok = __popc(b.start_mask);
-    const uint32_t nmatch = __popc(b.start_mask & b.match_mask);
-    uint32_t total;
-    const uint32_t before = wave_exclusive_sum(ntok | ((4u * ntok - 2u * nmatch) << 16), total);
-    b.tok_base = before & 0xffffu;
-    b.byte_base = before >> 16;
-    b.flag_bytes = ((total & 0xffffu) + 7u) >> 3;
-    b.data_bytes = total >> 16;
+    b.count();
     return LZ_GENERAL;
 }
 
 // ---- launch 1: sizes and class of every block
 __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
     const uint32_t *__restrict__ in, int64_t nsym, int64_t blocks, int32_t *__restrict__ flag_off,
-    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls)
+    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls, uint4 *__restrict__ tokens)
 {
     __shared__ __attribute__((aligned(16))) uint32_t keys[LZ_WAVES][LZ_WINDOW + LZ_SYMS];
     const int lane = lane_id();
@@ -291,6 +315,7 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
     lz_load(in, nsym, block, lane, raw);
     LzBlock b;
     const int c = lz_analyse(raw, keys[wave], lane, b);
+    if (c == LZ_GENERAL) tokens[block * WAVE + lane] = b.tokens();
     if (lane == 0) {
         flag_off[block] = (int32_t)b.flag_bytes;
         data_off[block] = (int32_t)b.data_bytes;
@@ -302,10 +327,9 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
 // ---- launch 2: both tables, in place: exclusive sums inside chunks of 8192 entries, chunk totals
 __global__ __launch_bounds__(256) void lz_scan_chunks_kernel(int32_t *__restrict__ flag_off,
                                                             int32_t *__restrict__ data_off, int64_t entries,
-                                                            uint32_t *__restrict__ totals, uint32_t *__restrict__ bases)
+                                                            uint32_t *__restrict__ totals)
 {
     __shared__ uint32_t wave_tot[4];
-    if (gridDim.x == 1 && threadIdx.x < 2) bases[threadIdx.x] = 0;       // (no chunks before it: launch 3 is left out)
     constexpr int PER = LZ_SCAN_CHUNK / 256;            // 32 entries per thread, contiguous
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
     const int64_t e0 = (int64_t)blockIdx.x * LZ_SCAN_CHUNK + (int64_t)threadIdx.x * PER;
@@ -348,29 +372,13 @@ __global__ __launch_bounds__(256) void lz_scan_chunks_kernel(int32_t *__restrict
     }
 }
 
-// ---- launch 3: chunk totals -> sums over all earlier chunks (one work-group)
-__global__ __launch_bounds__(LZ_MAX_CHUNKS) void lz_scan_totals_kernel(const uint32_t *__restrict__ totals,
-                                                                      int chunks, uint32_t *__restrict__ bases)
+// the sums of the first n chunks' totals: flags, data
+__device__ __forceinline__ uint2 lz_chunks_before(const uint32_t *__restrict__ totals, int n)
 {
-    __shared__ uint32_t wave_tot[2][LZ_MAX_CHUNKS / WAVE];
-    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    uint32_t before[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const uint32_t v = (int)threadIdx.x < chunks ? totals[2 * threadIdx.x + a] : 0u;
-        uint32_t total;
-        before[a] = wave_exclusive_sum(v, total);
-        if (lane == 0) wave_tot[a][wave] = total;
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < chunks) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            uint32_t run = before[a];
-            for (int w = 0; w < wave; ++w) run += wave_tot[a][w];
-            bases[2 * threadIdx.x + a] = run;
-        }
-    }
+    uint32_t f = 0, d = 0;
+    for (int c = lane_id(); c < n; c += WAVE) { f += totals[2 * c]; d += totals[2 * c + 1]; }
+    auto sum = [](uint32_t a, uint32_t b) { return a + b; };
+    return make_uint2((uint32_t)wave_allreduce((int)f, sum), (uint32_t)wave_allreduce((int)d, sum));
 }
 
 // zero flags[flag_total ..) and data[data_total ..): 16 bytes per lane and step, neighbouring lanes at
@@ -394,24 +402,23 @@ __device__ __forceinline__ void lz_clear_slack(int64_t tid, int64_t nthreads, in
 }
 
 struct __attribute__((aligned(16))) LzPlaceShared {
-    uint32_t keys[LZ_WAVES][LZ_WINDOW + LZ_SYMS];
     uint16_t stage[LZ_WAVES][LZ_BLOCK_BYTES / 2];   // token bytes of the block
     uint32_t flagw[LZ_WAVES][16];                   // flag bits of the block
 };
 
-// ---- launch 4: every block to its final place
+// ---- launch 3: every block to its final place, and zeros behind the last
 __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     const uint32_t *__restrict__ in, int64_t nsym, int64_t blocks, int32_t *__restrict__ flag_off,
-    int32_t *__restrict__ data_off, const uint8_t *__restrict__ cls, const uint32_t *__restrict__ bases,
+    int32_t *__restrict__ data_off, const uint8_t *__restrict__ cls, const uint32_t *__restrict__ totals, int chunks, const uint4 *__restrict__ tokens,
     uint8_t *__restrict__ flags, uint8_t *__restrict__ data)
 {
     __shared__ LzPlaceShared sh;
-    // With one chunk the totals are there already (their base is zero: the wave of the last block writes back what it
-    // read), and the work-groups behind the blocks' clear what lies beyond them: no launch 5.
+    // the work-groups behind the blocks' clear what lies beyond the totals
     const int64_t groups = (blocks + LZ_WAVES - 1) / LZ_WAVES;
     if (blockIdx.x >= groups) {
+        const uint2 all = lz_chunks_before(totals, chunks);
         lz_clear_slack(((int64_t)blockIdx.x - groups) * LZ_WAVES * WAVE + threadIdx.x, ((int64_t)gridDim.x - groups) * LZ_WAVES * WAVE,
-                       flag_off[blocks], data_off[blocks], blocks, flags, data);
+                       (int32_t)all.x, (int32_t)all.y, blocks, flags, data);
         return;
     }
     const int lane = lane_id();
@@ -422,20 +429,21 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     uint32_t raw[8];
     lz_load(in, nsym, block, lane, raw);
     const int64_t chunk = block / LZ_SCAN_CHUNK;
-    const uint32_t fbase = (uint32_t)flag_off[block] + bases[2 * chunk];
-    const uint32_t dbase = (uint32_t)data_off[block] + bases[2 * chunk + 1];
+    const uint2 before = lz_chunks_before(totals, (int)chunk);
+    const uint32_t fbase = (uint32_t)flag_off[block] + before.x;
+    const uint32_t dbase = (uint32_t)data_off[block] + before.y;
     int c = cls[block];
     c = __builtin_amdgcn_readfirstlane(c);
     // never let a wrong table move a write out of the buffers
     const uint32_t fb = min(fbase, (uint32_t)(block * (LZ_SYMS / 8)));
     const uint32_t db = min(dbase, (uint32_t)(block * LZ_BLOCK_BYTES)) & ~1u;
+    const uint2 all = block == blocks - 1 ? lz_chunks_before(totals, chunks) : make_uint2(0u, 0u);
     if (lane == 0) {
         flag_off[block] = (int32_t)fbase;
         data_off[block] = (int32_t)dbase;
         if (block == blocks - 1) {                     // the totals sit in the entry after the last block
-            const int64_t ce = blocks / LZ_SCAN_CHUNK;
-            flag_off[blocks] = (int32_t)((uint32_t)flag_off[blocks] + bases[2 * ce]);
-            data_off[blocks] = (int32_t)((uint32_t)data_off[blocks] + bases[2 * ce + 1]);
+            flag_off[blocks] = (int32_t)all.x;
+            data_off[blocks] = (int32_t)all.y;
         }
     }
     uint8_t *dst = data + db;
@@ -459,8 +467,17 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
         }
         if (lane == 0) flagw[0] = 0x001ffffeu;
     } else {
+        const uint4 packed = tokens[block * WAVE + lane];
+        const uint32_t words[4] = {packed.x, packed.y, packed.z, packed.w};
+        auto token = [&](int i) { return words[i >> 1] >> (16 * (i & 1)); };
         LzBlock b;
-        if (lz_analyse(raw, sh.keys[wave], lane, b) != LZ_GENERAL) return;   // the input changed between the launches
+        b.start_mask = b.match_mask = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            b.start_mask |= ((token(i) >> 15) & 1u) << i;
+            b.match_mask |= ((token(i) >> 14) & 1u) << i;
+        }
+        b.count();
         flag_bytes = b.flag_bytes;
         data_bytes = b.data_bytes;
         if (lane < 16) flagw[lane] = 0;
@@ -470,9 +487,7 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
         for (int i = 0; i < 8; ++i) {
             if ((b.start_mask >> i) & 1) {
                 if ((b.match_mask >> i) & 1) {
-                    const uint32_t l = ((i < 4 ? b.lens_lo : b.lens_hi) >> (8 * (i & 3))) & 0xffu;
-                    const uint32_t o = ((i < 4 ? b.offs_lo : b.offs_hi) >> (8 * (i & 3))) & 0xffu;
-                    stage[at] = (uint16_t)(l | (o << 8));
+                    stage[at] = (uint16_t)(((token(i) & 0x1fu) + 1u) | ((((token(i) >> 5) & 0x1fu) + 1u) << 8));
                     at += 1;
                     bits |= 1u << nb;
                 } else {
@@ -504,15 +519,6 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     }
     if (((data_bytes - head) & 2u) && lane == 0)
         *reinterpret_cast<uint16_t *>(dst + data_bytes - 2) = stage[data_bytes / 2 - 1];
-}
-
-// ---- launch 5: what lies beyond the totals
-__global__ __launch_bounds__(256) void lz_clear_slack_kernel(const int32_t *__restrict__ flag_off,
-                                                            const int32_t *__restrict__ data_off,
-                                                            int64_t blocks, uint8_t *__restrict__ flags,
-                                                            uint8_t *__restrict__ data)
-{
-    lz_clear_slack((int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256, flag_off[blocks], data_off[blocks], blocks, flags, data);
 }
 
 struct LzDecodeShared {
@@ -748,12 +754,14 @@ extern "C" int64_t planmoe_lz_blocks(int64_t nbytes)
     return nbytes <= 0 ? 0 : (nbytes + LZ_BLOCK_BYTES - 1) / LZ_BLOCK_BYTES;
 }
 
-// workspace: class byte per block | chunk totals | chunk bases
+// workspace: class byte per block | chunk totals | tokens of the blocks with matches, two bytes a position
 static size_t lz_class_bytes(int64_t blocks) { return round_up((size_t)blocks, 256); }
+static size_t lz_tokens_at(int64_t blocks) { return lz_class_bytes(blocks) + 2 * LZ_MAX_CHUNKS * sizeof(uint32_t); }
 
 extern "C" size_t planmoe_lz_workspace_bytes(int64_t nbytes)
 {
-    return lz_class_bytes(planmoe_lz_blocks(nbytes)) + 2 * (2 * LZ_MAX_CHUNKS * sizeof(uint32_t));
+    const int64_t blocks = planmoe_lz_blocks(nbytes);
+    return lz_tokens_at(blocks) + 16 + (size_t)blocks * LZ_SYMS * 2;       // (the tokens begin at the next 16 bytes)
 }
 
 extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets,
@@ -779,20 +787,17 @@ extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *f
                "planmoe_lz_compress: workspace too small or not 4-byte aligned");
     uint8_t *cls = (uint8_t *)workspace;
     uint32_t *totals = (uint32_t *)(cls + lz_class_bytes(blocks));
-    uint32_t *bases = totals + 2 * LZ_MAX_CHUNKS;
+    uint4 *tokens = (uint4 *)(((uintptr_t)workspace + lz_tokens_at(blocks) + 15) / 16 * 16);
     const int64_t groups = (blocks + LZ_WAVES - 1) / LZ_WAVES;
     const int64_t entries = blocks + 1;
     const int chunks = (int)((entries + LZ_SCAN_CHUNK - 1) / LZ_SCAN_CHUNK);      // <= 128 below 2^31 bytes
     lz_sizes_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
-                                                                flag_offsets, data_offsets, cls);
-    lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals, bases);
-    if (chunks > 1) lz_scan_totals_kernel<<<1, LZ_MAX_CHUNKS, 0, st>>>(totals, chunks, bases);
+                                                                flag_offsets, data_offsets, cls, tokens);
+    lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals);
     const int64_t slack_chunks = (blocks * LZ_BLOCK_BYTES / 16 + 255) / 256;          // enough for all of data
-    const int64_t clear_groups = chunks > 1 ? 0 : min((slack_chunks + 1) / 2, (int64_t)256);
+    const int64_t clear_groups = min((slack_chunks + 1) / 2, (int64_t)(chunks > 1 ? 2048 : 256));
     lz_place_kernel<<<(unsigned)(groups + clear_groups), LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks, flag_offsets,
-                                                                                 data_offsets, cls, bases, flags, data);
-    if (chunks > 1)
-        lz_clear_slack_kernel<<<(unsigned)min(slack_chunks, (int64_t)4096), 256, 0, st>>>(flag_offsets, data_offsets, blocks, flags, data);
+                                                                                 data_offsets, cls, totals, chunks, tokens, flags, data);
     PM_LAUNCH_CHECK("planmoe_lz_compress");
     return 0;
 }

@@ -208,3 +208,30 @@ def test_argument_errors():
         ops.lz_compress(torch.zeros((3,), dtype=torch.bfloat16, device=DEV))       # 6 bytes
     with pytest.raises(_lib.PlanMoEError):
         ops.lz_compress(torch.zeros((4,), dtype=torch.float32))                    # CPU tensor
+
+
+@pytest.mark.parametrize("nblocks", [1, 9, 8191, 8192, 16400])
+@pytest.mark.parametrize("at", [0, 4, 12])
+def test_tokens_of_every_length_and_offset(nblocks, at):
+    """Blocks whose tokens the placement takes from the workspace: runs of every length and distance up to the window's, zeros that begin
+    and end anywhere, stored blocks and blocks of one value between them; either side of a chunk of the scan (its last entry holds the
+    totals), a workspace at any word, exactly as large as asked for."""
+    rng = np.random.default_rng(nblocks + at)
+    x = rng.standard_normal((nblocks, 512)).astype(np.float32)
+    for b in range(0, nblocks, 3):                       # copies of what lies d back, 1 .. 32 symbols of it
+        p = 40
+        while p < 470:
+            n, d = int(rng.integers(1, 33)), int(rng.integers(1, 33))
+            for q in range(p, p + n): x[b, q] = x[b, q - d]
+            p += n + int(rng.integers(0, 40))
+        if b >= 300: x[b] = x[b % 300]
+    for b in range(1, nblocks, 3):
+        lo, hi = sorted(rng.integers(0, 513, 2))
+        x[b, lo:hi] = 0.0
+    x = x.reshape(-1)
+    words = (int(_lib.lib.planmoe_lz_workspace_bytes(x.nbytes)) + at + 16) // 4 * 4
+    whole = torch.full((words,), 0xA5, dtype=torch.uint8, device=DEV)
+    ws = whole[at:at + int(_lib.lib.planmoe_lz_workspace_bytes(x.nbytes))]
+    got = ops.lz_compress(torch.from_numpy(x).to(DEV), workspace=ws)
+    same_streams(got, oracle.lz_compress(x))
+    assert bool((whole[:at] == 0xA5).all()) and bool((whole[at + ws.numel():] == 0xA5).all())
