@@ -6,7 +6,10 @@
 // A 32 x 32 x 2 MFMA takes 64 clocks, so unlike bf16 nothing here is bound by operand traffic: a 128 x 128
 // tile reads 32 KB per k-tile of 32 for 4096 clocks of matrix core.  Four waves of 64 x 64 (32 x 32 in the small
 // tile), operands straight into LDS (buffer_load ... lds), the next k-tile in flight during the MFMAs of this one, two work-groups
-// per compute unit so that one's barrier and epilogue fall under the other's MFMAs.  A k-fast operand is
+// per compute unit so that one's barrier and epilogue fall under the other's MFMAs.  Where there are few tiles of 64 x 64 a wave is alone on its
+// matrix core, and what it issues ahead of a k-tile's products (a barrier, descriptors, loads, LDS reads: 440 of 1600 clocks) is time lost: the
+// form with four stages has one descriptor for a whole operand, places in LDS known when it is compiled, and puts every load and read
+// between two products.  A k-fast operand is
 // read four k at a time (16 bytes per lane), sixteen k are two reads, and the sums take them in the order
 // 0 4 8 12, 1 5 9 13, ..: the order of a product made of 16 x 16 x 4 instructions whose lanes read 16 bytes, so what such
 // a product (the fp32 library's) gives, this one gives bit for bit, and a relu behind it cuts the same elements.
@@ -17,11 +20,13 @@
 
 namespace pm {
 
-// F: 32 x 32 fragments of a wave on a side; the tile is 64 F x 64 F
-template <int F, bool TA, bool TB>
+// F: 32 x 32 fragments of a wave on a side; the tile is 64 F x 64 F.  STAGES: k-tiles in LDS, two or four.  With four a wave reads the first
+// fragments of the next k-tile beside the products of this one.  (us, cold weights, two and four stages: 4 experts x 256 rows, 1024 -> 512 25 and 19;
+// 3072 -> 1024 72 and 56; 8 x 24, 2048 -> 2048 b^T 55 and 38.)
+template <int F, bool TA, bool TB, int STAGES>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
 {
-    constexpr int G32_B = 64 * F, G32_OPERAND = G32_B * G32_BK * 4;         // tile side; one operand's k-tile in LDS (A0 A1 B0 B1)
+    constexpr int G32_B = 64 * F, G32_OPERAND = G32_B * G32_BK * 4;         // tile side; one operand's k-tile in LDS (A0 A1 .. B0 B1 ..)
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -54,7 +59,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     const int64_t ra = TA ? ((int64_t)(K - 1) * lda + (p.M - m0)) * 4 : ((int64_t)(M - m0 - 1) * lda + p.K) * 4;
     const int64_t rb = TB ? ((int64_t)(K - 1) * ldb + (p.N - n0)) * 4 : ((int64_t)(p.N - n0 - 1) * ldb + p.K) * 4;
     const int64_t step_a = TA ? (int64_t)G32_BK * lda * 4 : G32_BK * 4, step_b = TB ? (int64_t)G32_BK * ldb * 4 : G32_BK * 4;
-    const int KT = (K + G32_BK - 1) / G32_BK, k_tail = K % G32_BK ? K % G32_BK : G32_BK;
+    const int KT = __builtin_amdgcn_readfirstlane((K + G32_BK - 1) / G32_BK), k_tail = K % G32_BK ? K % G32_BK : G32_BK;
 
     // k fast: 64 F rows of 128 bytes, a load fills eight, chunk c of row r at unit c ^ (r >> 1) & 7.
     // k slow: 32 rows of 256 F bytes, a load fills 4 / F.
@@ -67,17 +72,29 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     // (chunks of a k-fast row past the end of K are asked for out of range)
     auto past = [&](int i) -> uint32_t { return (int)(((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 4) >= k_tail ? 0x80000000u : 0u; };
     const uint32_t past0 = past(0), past1 = past(1);
+    // (with four stages k-tiles past the end are asked for as well, out of range: the count of what is on its way stays the same)
+    // Four stages: the operands from their corner on are within reach of an offset (the caller sees to it), so a load is an offset away from
+    // one descriptor and fits under a product; past the end the last k-tile is asked for again, so that the count of what is on its way stays
+    // the same, and never used.
+    const g32_u32x4 whole_a = g32_desc(A, ra), whole_b = g32_desc(B, rb);
+    const int there = KT > 0 ? KT - 1 : 0;
+    auto load = [&](int kt, int stage, int n) {  // the n-th of a k-tile's 4 F
+        const bool last = kt == KT - 1 && k_tail != G32_BK, b = n >= 2 * F;
+        const int i = b ? n - 2 * F : n;
+        const bool T = b ? TB : TA;
+        const uint32_t ld = (uint32_t)(b ? ldb : lda), v = (b ? vb[i & 1] : va[i & 1]) | (!T && last ? ((i & 1) ? past1 : past0) : 0u);
+        const uint32_t rows = ld * 4u * (uint32_t)(T ? 4 / F * i : 8 * (i & ~1));
+        const uint32_t to = lds0 + stage * G32_OPERAND + wave * (2048 * F) + (b ? STAGES * G32_OPERAND : 0) + i * 1024;
+        if constexpr (STAGES == 4) {
+            g32_dma16(b ? whole_b : whole_a, v, __builtin_amdgcn_readfirstlane(rows + (uint32_t)(kt < KT ? kt : there) * (uint32_t)(b ? step_b : step_a)), to);
+        } else {
+            g32_dma16(b ? g32_desc(B + kt * step_b, rb - kt * step_b) : g32_desc(A + kt * step_a, ra - kt * step_a), v, rows, to);
+        }
+    };
     auto load_tile = [&](int kt) {
-        if (kt >= KT) return;
-        const g32_u32x4 da = g32_desc(A + kt * step_a, ra - kt * step_a), db = g32_desc(B + kt * step_b, rb - kt * step_b);
-        const uint32_t sa = lds0 + (kt & 1) * G32_OPERAND + wave * (2048 * F), sb = sa + 2 * G32_OPERAND;
-        const bool last = kt == KT - 1 && k_tail != G32_BK;
+        if (STAGES == 2 && kt >= KT) return;
 #pragma unroll
-        for (int i = 0; i < 2 * F; ++i)
-            g32_dma16(da, va[i & 1] | (!TA && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)lda * 4u * (uint32_t)(TA ? 4 / F * i : 8 * (i & ~1)), sa + i * 1024);
-#pragma unroll
-        for (int i = 0; i < 2 * F; ++i)
-            g32_dma16(db, vb[i & 1] | (!TB && last ? ((i & 1) ? past1 : past0) : 0u), (uint32_t)ldb * 4u * (uint32_t)(TB ? 4 / F * i : 8 * (i & ~1)), sb + i * 1024);
+        for (int n = 0; n < 4 * F; ++n) load(kt, kt & (STAGES - 1), n);
     };
 
     f32x16 acc[F][F];
@@ -104,32 +121,69 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
             }
     };
 
-    load_tile(0);
-    for (int kt = 0; kt < KT; ++kt) {
-        // this wave's share of k-tile kt is in; behind the barrier everybody's is, and everybody is done with kt - 1
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        load_tile(kt + 1);
-        const uint8_t *a = lds + (kt & 1) * G32_OPERAND, *b = a + 2 * G32_OPERAND;
-        f32x4 fa[2][F][2], fb[2][F][2];
-        read16(TA, a, wm, 0, fa[0]);
-        read16(TB, b, wn, 0, fb[0]);
+    f32x4 fa[2][F][2], fb[2][F][2];
+    auto read_a = [&](int stage, int s, int to) { read16(TA, lds + stage * G32_OPERAND, wm, s, fa[to]); };
+    auto read_b = [&](int stage, int s, int to) { read16(TB, lds + (STAGES + stage) * G32_OPERAND, wn, s, fb[to]); };
+    // (the second operand first: a lane then holds four consecutive columns of one row)
+    auto multiply = [&](int s, int x) {
+        const int q = x >> 1, h = x & 1;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            if (s == 0) { read16(TA, a, wm, 1, fa[1]); read16(TB, b, wn, 1, fb[1]); }
-            // (the second operand first: a lane then holds four consecutive columns of one row)
+        for (int i = 0; i < F; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int j = 0; j < F; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[s][j][h][q], fa[s][i][h][q], acc[i][j], 0, 0, 0);
+    };
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+    for (int kt = 0; kt < STAGES - 1; ++kt) load_tile(kt);
+    if constexpr (STAGES == 4) {
+        // behind the barrier of k-tile kt everybody's share of kt + 1 is in as well, and everybody is done with kt - 1; what else there is to do
+        // goes between the products, one thing at a time (ahead of them it left the matrix core idle for a third of a k-tile)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((STAGES - 2) * 4 * F) : "memory");
+        read_a(0, 0, 0);
+        read_b(0, 0, 0);
+        for (int k0 = 0; k0 < KT; k0 += STAGES) {
 #pragma unroll
-                    for (int i = 0; i < F; ++i)
+            for (int stage = 0; stage < STAGES; ++stage) {       // (where things lie in LDS is known)
+                const int kt = k0 + stage;
+                if (kt >= KT) break;
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((STAGES - 3) * 4 * F) : "memory");
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                        for (int j = 0; j < F; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[s][j][h][q], fa[s][i][h][q], acc[i][j], 0, 0, 0);
+                for (int x = 0; x < 8; ++x) {
+                    multiply(0, x);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (x == 0) read_a(stage, 1, 1);
+                    else if (x == 1) read_b(stage, 1, 1);
+                    else if (x - 2 < 4 * F) load(kt + STAGES - 1, (stage + STAGES - 1) % STAGES, x - 2);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int x = 0; x < 8; ++x) {
+                    multiply(1, x);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (x == 0) read_a((stage + 1) % STAGES, 0, 0);
+                    else if (x == 1) read_b((stage + 1) % STAGES, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    } else {
+        for (int kt = 0; kt < KT; ++kt) {
+            // this wave's share of k-tile kt is in; behind the barrier everybody's is, and everybody is done with kt - 1
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            load_tile(kt + 1);
+            read_a(kt & 1, 0, 0);
+            read_b(kt & 1, 0, 0);
+            read_a(kt & 1, 1, 1);
+            read_b(kt & 1, 1, 1);
+#pragma unroll
+            for (int x = 0; x < 16; ++x) multiply(x >> 3, x & 7);
         }
     }
 
     g32_store<F, F>(p, acc, e, m0, n0, M, wm, wn, m0 / G32_B * 2 + wm, tiles_m * 2);
+    // nothing may still be on its way into LDS that another work-group gets
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // Few rows: a wave on its own, 16 MF rows by 16 columns, operands from memory straight into registers
@@ -272,11 +326,11 @@ static int gemm_f32_wave_launch(const Gemm32Args &p, hipStream_t stream, const c
     return 0;
 }
 
-template <int F, bool TA, bool TB>
+template <int F, bool TA, bool TB, int STAGES = 2>
 static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
 {
-    constexpr int LDS = 4 * 64 * F * G32_BK * 4, SIDE = 64 * F;
-    const auto kernel = gemm_f32_kernel<F, TA, TB>;
+    constexpr int LDS = 2 * STAGES * 64 * F * G32_BK * 4, SIDE = 64 * F;
+    const auto kernel = gemm_f32_kernel<F, TA, TB, STAGES>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -292,21 +346,32 @@ static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *
     return 0;
 }
 
+// Four stages pay from eight k-tiles on (three are asked for before the first is multiplied), and need their operands within reach of an offset:
+// 128 k past the end of one whose k is the slow index.
+static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
+{
+    const int64_t reach = ((int64_t)1 << 31) / 4;
+    if ((form == 2 ? rows_hint : p.K) <= 7 * G32_BK) return false;
+    return (form == 1 || ((int64_t)p.K + 128) * p.N < reach) && (form != 2 || ((int64_t)p.K + 128) * p.M < reach);
+}
+
 // The tile's side: a compute unit's matrix cores take 1.7 us for a k-tile of 128 x 128 and a quarter of that, and
 // a tenth, for one of 64 x 64; what counts is the fullest compute unit (4 x 300 x 512 x 1024: 64 tiles of 128, 57 us).
-// 0, waves on their own, up to 32 rows, where they read the weight once (8 experts, 2 rows each: nn 1024 -> 4096 44 -> 27 us,
-// nt 41 -> 23, 4096 -> 1024 90 -> 39; 60 rows, nt 512 -> 2048: 23 -> 31).  The rows are those expected: with skewed routing an
+// Waves on their own, up to 16 rows (32 where a tile has less than eight k-tiles), where they read the weight once (8 experts, 2 rows each: nn
+// 1024 -> 4096 44 -> 27 us, nt 41 -> 23, 4096 -> 1024 90 -> 39; tiles of four stages take 1.2 - 1.6 of their time at 2 rows, 1.0 at 16, 0.95 at 20).
+// The rows are those expected: with skewed routing an
 // expert has more, and its weight is read once for every 32 of them, but all experts together have as many rows as before,
-// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves and in tiles, nn, nt:
+// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves and in tiles of two stages, nn, nt:
 //   8 experts, 256 rows, 4096 -> 1024    even 69, 86 and 90, 89;     128 of the rows on one 70, 88 and 91, 90
 //   8 experts, 128 rows, 1024 -> 4096    even 31, 32 and 43, 42;     64 on one 44, 52 and 42, 42
 //   16 experts, 256 rows, 4096 -> 1024   even 55, 60 and 93, 97;     128 on one 123, 140 and 152, 155
 //   64 experts, 2048 rows, 1024 -> 4096  even 388, 361 and 305, 303; by Zipf's law (1.2) 531, 525 and 918, 912
 //
 // On the bf16 matrix cores, in three parts a value (gemm_f32_split.hip), where there is more than one tile of 64 x 64 for a compute
-// unit; one tile on its own is bound by issuing the splits (8 experts, 128 rows, 1024 -> 1024: 25 us in fp32, 28 in parts) and stays here.
+// unit; one tile on its own is bound by issuing the splits (8 experts, 128 rows, 1024 -> 1024: 20 us in fp32, 28 in parts) and stays here.
 // A launch takes its rounds; us for a k-tile with few and with all compute units at work, and once for a tile, fitted to 60 shapes
-// (within 7 %): 64 x 64 0.6 alone, 0.44 each of several on a compute unit, + 6; 128 x 128 1.1 - 1.4, + 6; 256 x 128 1.9 - 2.5, + 7.
+// (within 7 %): in parts 64 x 64 0.6 alone, 0.44 each of several on a compute unit, + 6; 128 x 128 1.1 - 1.4, + 6; 256 x 128 1.9 - 2.5, + 7;
+// in fp32 64 x 64 with four stages 0.43, 0.44 and + 4.
 //   experts x rows, in, out       fp32 tiles    64     128    256 x 128
 //   16 x 512, 1024, 1024 nn          147        126     102     88
 //   16 x 512, 1024, 1024 tn          133        131     114     98
@@ -329,13 +394,17 @@ static Gemm32Kernel gemm_f32_pick_split(int form, const Gemm32Args &p, int rows_
     };
     const double small = std::ceil(tiles(64, 64) / cu), t64 = (small <= 1 ? 0.6 : 0.44 * small) * kt + 6;
     const double t128 = rounds(tiles(128, 128), 1.1, 1.4, 6), t256 = rounds(tiles(256, 128), 1.9, 2.5, 7);
-    if (t64 <= t128 && t64 <= t256) return small <= 1 ? G32_TILE_64 : G32_SPLIT_64;
+    const bool deep = gemm_f32_deep(form, p, rows_hint);
+    const double whole = deep ? (small <= 1 ? 0.43 : 0.44 * small) * kt + 3.5 + 0.5 * small : small <= 1 ? t64 : 1e30;
+    if (whole <= t64 && whole <= t128 && whole <= t256) return deep ? G32_DEEP_64 : G32_TILE_64;
+    if (t64 <= t128 && t64 <= t256) return G32_SPLIT_64;
     return t128 <= t256 ? G32_SPLIT_128 : G32_SPLIT_256;
 }
 
 Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
 {
-    if (form != 2 && rows_hint <= 32 && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
+    const bool deep = gemm_f32_deep(form, p, rows_hint);
+    if (form != 2 && rows_hint <= (deep ? 16 : 32) && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
         gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
         return G32_WAVES;
     if (p.relu != 1 && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
@@ -345,7 +414,7 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
         return (double)((tiles + cu - 1) / cu) * (us * kt + 2);
     };
-    return cost(64, 0.47) < cost(128, 1.7) ? G32_TILE_64 : G32_TILE_128;
+    return cost(64, deep ? 0.45 : 0.47) < cost(128, 1.7) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
 }
 
 int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who)
@@ -358,6 +427,10 @@ int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t
         if (form == 0) return gemm_f32_launch<1, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<1, false, false>(p, stream, who);
         return gemm_f32_launch<1, true, true>(p, stream, who);
+    case G32_DEEP_64:
+        if (form == 0) return gemm_f32_launch<1, false, true, 4>(p, stream, who);
+        if (form == 1) return gemm_f32_launch<1, false, false, 4>(p, stream, who);
+        return gemm_f32_launch<1, true, true, 4>(p, stream, who);
     case G32_TILE_128:
         if (form == 0) return gemm_f32_launch<2, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<2, false, false>(p, stream, who);

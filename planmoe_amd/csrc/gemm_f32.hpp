@@ -13,9 +13,9 @@ struct Gemm32Args {
     int relu;                              // 1; 2: and no backward pass asks which elements it cut
 };
 
-// Kernels: waves on their own; tiles of 64 x 64 and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128
+// Kernels: waves on their own; tiles of 64 x 64 (two and four k-tiles in LDS) and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128
 // on the bf16 matrix cores, the operands in three parts
-enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_TILE_128, G32_SPLIT_64, G32_SPLIT_128, G32_SPLIT_256 };
+enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_DEEP_64, G32_TILE_128, G32_SPLIT_64, G32_SPLIT_128, G32_SPLIT_256 };
 
 // form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  rows_hint: rows in use
 Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint);

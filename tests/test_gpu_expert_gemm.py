@@ -453,3 +453,51 @@ def test_expert_gemm_few_rows_and_many_columns(B, n, k, m):
             assert bool((out[e, r:] == 7.0).all())
         stored = masked[e, :r].double()          # the sums are of what was stored
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, dtype)).all())
+
+
+# Tiles of 64 x 64 with four k-tiles in LDS: one, two and three k-tiles more than a round of them, a piece of one; a k that is the slow index of one or
+# both operands, rows in use below the capacity and none, NaN behind them; against the same product with the rows expected that take other tiles
+# only by the rounding of its sums, and bit for bit against waves on their own where no split serves (n below 256).
+@pytest.mark.parametrize("B,cap,n,k", [(3, 70, 68, 228), (4, 130, 260, 256), (2, 100, 520, 292), (5, 40, 132, 324), (3, 200, 300, 1028), (2, 257, 64, 384)])
+def test_expert_gemm_fp32_four_stages(B, cap, n, k):
+    from planmoe_amd import ops
+    print("case", B, cap, n, k, flush=True)
+    g = torch.Generator().manual_seed(cap + n + k)
+    live = torch.tensor([[cap - 3, 0, 33, 1, 64][:B]], dtype=torch.int32)
+    a, w = torch.randn(B, cap, k, generator=g), torch.randn(B, k, n, generator=g)
+    h, bias = torch.randn(B, cap, n, generator=g).clamp(min=0), torch.randn(B, n, generator=g)
+    for e in range(B):
+        a[e, int(live[0, e]):] = float("nan")
+    wt = w.transpose(1, 2).contiguous()
+    a, w, wt, h, bias = (t.to(DEV) for t in (a, w, wt, h, bias))
+    kw = dict(live=live.to(DEV), rows_hint=33)
+    nn = torch.full((B, cap, n), 7.0, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    ops.expert_gemm("nn", a, w, bias, relu=True, out=nn, **kw)
+    ops.expert_gemm("nt", a, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, out=masked, **kw)
+    # a^T b over the rows in use, whose number has to reach eight k-tiles: the operands' other way round
+    rows = torch.tensor([[k - 5, 0, k, 226, 33][:B]], dtype=torch.int32)
+    x, d = torch.randn(B, k, 72, generator=g), torch.randn(B, k, n, generator=g)
+    for e in range(B):
+        x[e, int(rows[0, e]):] = d[e, int(rows[0, e]):] = float("nan")
+    tn = ops.expert_gemm("tn", x.to(DEV), d.to(DEV), live=rows.to(DEV), rows_hint=k)
+    if n < 256:
+        one = torch.empty_like(nn)
+        ops.expert_gemm("nn", a, w, bias, relu=True, out=one, live=live.to(DEV), rows_hint=1)
+    torch.cuda.synchronize()
+    for e in range(B):
+        r, q = int(live[0, e]), int(rows[0, e])
+        y, z = a[e, :r].double(), w[e].double()
+        ref, mag = y @ z, y.abs() @ z.abs()
+        tol = _bound(ref, mag, k, torch.float32)
+        assert bool(((nn[e, :r].double() - (ref + bias[e].double()).clamp(min=0)).abs() <= tol + _bound(ref, bias[e].double().abs()[None] + ref.abs(), 1, torch.float32)).all())
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all())
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all())
+        for out in (nn, nt, masked):
+            assert bool((out[e, r:] == 7.0).all())
+        stored = masked[e, :r].double()          # the sums are of what was stored
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, torch.float32)).all())
+        xs, ds = x[e, :q].double(), d[e, :q].double()
+        assert bool(((tn[e].double().cpu() - xs.t() @ ds).abs() <= _bound(xs.t() @ ds, xs.abs().t() @ ds.abs(), k, torch.float32)).all())
+        if n < 256: assert torch.equal(one[e, :r], nn[e, :r])
