@@ -355,8 +355,9 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
     return (form == 1 || ((int64_t)p.K + 128) * p.N < reach) && (form != 2 || ((int64_t)p.K + 128) * p.M < reach);
 }
 
-// The tile's side: a compute unit's matrix cores take 1.7 us for a k-tile of 128 x 128 and a quarter of that, and
-// a tenth, for one of 64 x 64; what counts is the fullest compute unit (4 x 300 x 512 x 1024: 64 tiles of 128, 57 us).
+// The tile's side under a relu whose backward pass asks what it cut: a compute unit takes 1.9 us for a k-tile of 128 x 128 and 4 for the tile, 0.52 and
+// 1.2 for 64 x 64, 0.47 with four stages; what counts is the fullest compute unit (us, 64 x 64, with four stages, 128 x 128: 4 x 1000 rows,
+// 2048 -> 512 77, 66, 137; 16 x 512, 1024 -> 1024 142, 131, 131; 512 -> 2048 152, 144, 138; 2 x 4096, 4096 -> 4096 2129, 1944, 1969).
 // Waves on their own, up to 16 rows (32 where a tile has less than eight k-tiles), where they read the weight once (8 experts, 2 rows each: nn
 // 1024 -> 4096 44 -> 27 us, nt 41 -> 23, 4096 -> 1024 90 -> 39; tiles of four stages take 1.2 - 1.6 of their time at 2 rows, 1.0 at 16, 0.95 at 20).
 // The rows are those expected: with skewed routing an
@@ -410,11 +411,11 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
     if (p.relu != 1 && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
-    auto cost = [&](int64_t side, double us) {
+    auto cost = [&](int64_t side, double us, double once) {
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
-        return (double)((tiles + cu - 1) / cu) * (us * kt + 2);
+        return (double)((tiles + cu - 1) / cu) * (us * kt + once);
     };
-    return cost(64, deep ? 0.45 : 0.47) < cost(128, 1.7) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
+    return cost(64, deep ? 0.47 : 0.52, 1.2) < cost(128, 1.9, 4) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
 }
 
 int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who)
