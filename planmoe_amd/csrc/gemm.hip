@@ -12,6 +12,7 @@
 //             dW = x^T @ dy        A = x  [rows, in],   B = dy [rows, out]    planmoe_gemm_tn_bf16
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
+#include "gemm_deep.hpp"
 #include "gemm_skinny.hpp"
 #include "sums.hpp"
 #include <algorithm>
@@ -688,20 +689,25 @@ struct GemmCost {
 // The column sums of a masked product: a tile of so many rows has so many slots (0 rows: one slot for everything)
 struct GemmSlots { int rows, per_tile; };
 
-// Few rows per batch against a whole weight.  Up to 16 rows always; up to 32 where there is a compute unit for each
-// work-group, and up to 64 where there is in pieces of 64 columns: beyond that a tile's operands, read once for all its rows, win.
+// Few rows per batch against a whole weight.  Up to 16 rows always, and up to 32 where there is a compute unit for each
+// work-group: beyond that a tile's operands, read once for all its rows, win.
 // us, cold weights, few rows and tiles, nn, nt:
-//   8 x 40 rows, 2688 -> 2560     35, 33 and 33, 29      8 x 20, same       29, 28 and 32, 28
+//   8 x 40 rows, 2688 -> 2560     35, 33 and 30, 27      8 x 20, same       29, 28 and 32, 28
 //   16 x 40, 2688 -> 2560         66, 62 and 53, 47      16 x 20, same      56, 52 and 52, 46
 //   16 x 40, 1024 -> 4096         37, 36 and 31, 29      8 x 20, same       17, 16 and 19, 17
-//   8 x 40, 4096 -> 1024          35, 32 and 39, 36      8 x 8 2688 -> 2560 26, 25 and 32, 28
+//   8 x 40, 4096 -> 1024          35, 32 and 36, 34      8 x 8 2688 -> 2560 26, 25 and 32, 28
 bool gemm_is_skinny(bool nt, int m, int n, int64_t k, int batches)
 {
     if (m > SKINNY_ROWS || batches > 65535 || n * k * 2 >= ((int64_t)1 << 31)) return false;
-    const int64_t cu = compute_units();
-    auto groups = [&](int width) { return (int64_t)((n + width - 1) / width) * batches; };
-    return m <= 16 || groups(m <= 32 ? gemm_skinny_width(nt, n, batches) : 64) <= cu;
+    const int width = gemm_skinny_width(nt, n, batches);
+    return m <= 16 || (int64_t)((n + width - 1) / width) * batches <= compute_units();
 }
+
+// 128 x 128 with a compute unit for each tile (gemm_deep.hip).  Not up to the last one: with rows up to the capacity a few experts have a
+// tile more than expected, and two of these work-groups do not fit on a compute unit.  us in gemm_bf16_kernel's 128 x 128 tiles and here, weights cold, in cache:
+//   8 experts x 80 rows, 4096 -> 1024    43, 33 and 41, 25      8 x 80, 1024 -> 512     13, 13 and 9, 9
+//   8 x 110, 2696 -> 2488                39, 32 and 37, 29      a^T b, 4 x 512 x 768 over 2000 rows    20 and 15
+bool gemm_is_deep(double tiles, int m) { return tiles <= 0.8 * compute_units() || (m <= 128 && tiles <= compute_units()); }
 
 template <bool TA, bool TB, bool GRAD>
 int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who, GemmSlots *sums = nullptr)
@@ -709,15 +715,16 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
     if (sums) *sums = GemmSlots{128, 2};
     const bool contiguous = p.lda == p.K && p.ldb == (TB ? p.N : p.K) && p.ldc == p.N && p.sB == (int64_t)p.N * p.K && p.sA == (int64_t)p.M * p.K &&
                             p.sC == (int64_t)p.M * p.N;
+    const SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
     if (!TA && contiguous && gemm_is_skinny(!TB, p.M, p.N, p.K, p.batches)) {
         if (sums) *sums = GemmSlots{0, 1};
-        SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
         return gemm_skinny_run(!TB, few, stream, who);
     }
     const int64_t cu = compute_units();
     const GemmCost cost{(double)(TA ? p.M : rows_hint), (double)(((TA ? rows_hint : p.K) + 63) / 64), (double)cu, p.M, p.N, p.batches,
                         TA ? 0 : (int64_t)p.N * p.K * p.batches * 2, !TA && p.live};
-    const double small = cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
+    const bool deep = contiguous && gemm_is_deep(cost.tiles(128, 128), p.M) && gemm_deep_reaches(TA ? 2 : TB ? 0 : 1, p.M, p.N, p.K);
+    const double small = (deep ? 0.88 : 1.) * cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
     if constexpr (!TA) {
         const double low[3] = {cost.low(128), cost.low(160), cost.low(192)};
         const int f = low[0] <= low[1] && low[0] <= low[2] ? 0 : low[1] <= low[2] ? 1 : 2;
@@ -728,7 +735,7 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
             return gemm_launch<GemmFlat<3, 3>, TA, TB, GRAD>(p, stream, who);
         }
     }
-    if (small < big) return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
+    if (small < big) return deep ? gemm_deep_run(TA ? 2 : TB ? 0 : 1, few, stream, who) : gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
     p.stay = (int)(cu / 8 * 8);
     p.split = big == split;
     if (gemm_launch<Gemm256, TA, TB, GRAD>(p, stream, who)) return 1;

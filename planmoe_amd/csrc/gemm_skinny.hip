@@ -1,10 +1,10 @@
-// The experts' product for few rows: up to 64 rows of an expert against its whole weight, bf16.
+// The experts' product for few rows: up to 32 rows of an expert against its whole weight, bf16.
 //
 //   C[e][r][n] = act( bf16( bf16( sum_k A[e][r][k] * B ) + bias[e][n] ) ),  B = B[e][k][n] (nn) or B[e][n][k] (nt)
 //
 // For experts that have only few rows (decode, small batches).  Bound by reading the weight once, so nothing
-// goes through LDS on the way in: a wave loads straight into registers, a work-group's waves (16, or 8 above
-// 32 rows) split the reduction between them, up to four steps each in flight, so that a compute unit has
+// goes through LDS on the way in: a wave loads straight into registers, a work-group's waves (16, or 8 where
+// registers ask for it) split the reduction between them, up to four steps each in flight, so that a compute unit has
 // 128 KB on its way; the waves' sums meet in LDS at the end.
 //   nn: lane = (16 chunks of C columns, 4 groups of 8 k): eight loads give an 8 x C patch whose columns are
 //       put together by byte permutes, each a matrix-core operand of its own (column C chunk + c).
@@ -207,16 +207,14 @@ int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
      : grad ? skinny_launch<true, MF, C, U_NT, WAVES_NT, true>(p, stream, who)           \
             : skinny_launch<true, MF, C, U_NT, WAVES_NT, false>(p, stream, who))
     const int width = gemm_skinny_width(nt, p.N, p.batches);
-    // (what is not built is not asked for: nn in 96 columns; more than 32 rows in more than 64, gemm_is_skinny)
+    // (nn in 96 columns is not built and not asked for)
     if (p.M <= 16) {
         if (width == 96) return grad ? skinny_launch<true, 1, 6, 1, 16, true>(p, stream, who) : skinny_launch<true, 1, 6, 1, 16, false>(p, stream, who);
         return width == 64 ? PM_SK(1, 4, 4, 16, 2, 16) : PM_SK(1, 8, 1, 16, 1, 16);
     }
-    if (p.M <= 32) {                             // (nt holds 12 or 16 KB of weight per step: 8 waves' registers)
-        if (width == 96) return grad ? skinny_launch<true, 2, 6, 1, 8, true>(p, stream, who) : skinny_launch<true, 2, 6, 1, 8, false>(p, stream, who);
-        return width == 64 ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);
-    }
-    return PM_SK(4, 4, 5, 8, 2, 8);
+    // (nt holds 12 or 16 KB of weight per step: 8 waves' registers)
+    if (width == 96) return grad ? skinny_launch<true, 2, 6, 1, 8, true>(p, stream, who) : skinny_launch<true, 2, 6, 1, 8, false>(p, stream, who);
+    return width == 64 ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);
 #undef PM_SK
 }
 

@@ -4,7 +4,7 @@
 
 namespace pm {
 
-constexpr int SKINNY_ROWS = 64;                             // the most rows of an expert it takes
+constexpr int SKINNY_ROWS = 32;                             // the most rows of an expert it takes
 
 struct SkinnyArgs {
     const uint16_t *A, *B, *bias;

@@ -501,3 +501,44 @@ def test_expert_gemm_fp32_four_stages(B, cap, n, k):
         xs, ds = x[e, :q].double(), d[e, :q].double()
         assert bool(((tn[e].double().cpu() - xs.t() @ ds).abs() <= _bound(xs.t() @ ds, xs.abs().t() @ ds.abs(), k, torch.float32)).all())
         if n < 256: assert torch.equal(one[e, :r], nn[e, :r])
+
+
+# Tiles of 128 x 128 with a compute unit each, four k-tiles of 64 in LDS: reductions of less than one, of one, of four, one more and pieces; rows in use of
+# none, one, either side of half a tile and of a tile; columns of a piece; every form, the masked one's column sums.
+@pytest.mark.parametrize("k", [8, 56, 64, 72, 256, 264, 520])
+@pytest.mark.parametrize("cap,n,counts", [(66, 136, [66, 0, 33, 1, 65]), (300, 264, [0, 127, 128, 129, 300]), (257, 8, [257, 256, 255, 64, 63])])
+def test_expert_gemm_tile_alone(cap, n, counts, k):
+    from planmoe_amd import ops
+    print("case", cap, n, counts, k, flush=True)
+    g = torch.Generator().manual_seed(cap + n + k)
+    B, dtype = 5, torch.bfloat16
+    live = torch.tensor([counts], dtype=torch.int32)
+    a, w = torch.randn(B, cap, k, generator=g).to(dtype), torch.randn(B, k, n, generator=g).to(dtype)
+    h, bias, d = torch.randn(B, cap, n, generator=g).clamp(min=0).to(dtype), torch.randn(B, n, generator=g).to(dtype), torch.randn(B, cap, n, generator=g).to(dtype)
+    for e in range(B):
+        a[e, counts[e]:] = d[e, counts[e]:] = float("nan")
+    a, w, h, bias, d = (t.to(DEV) for t in (a, w, h, bias, d))
+    wt = w.transpose(1, 2).contiguous()
+    nn = torch.full((B, cap, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    kw = dict(live=live.to(DEV), rows_hint=100)
+    ops.expert_gemm("nn", a, w, bias, relu=True, out=nn, **kw)
+    ops.expert_gemm("nt", a, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, out=masked, **kw)
+    tn = ops.expert_gemm("tn", a, d, **kw)
+    torch.cuda.synchronize()
+    for e in range(B):
+        r = counts[e]
+        x, y = a[e, :r].double(), w[e].double()
+        ref, mag = x @ y, x.abs() @ y.abs()
+        tol = _bound(ref, mag, k, dtype)
+        biased = ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all())
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all())
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all())
+        for out in (nn, nt, masked):
+            assert bool((out[e, r:] == 7.0).all())
+        stored = masked[e, :r].double()          # the sums are of what was stored
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, dtype)).all())
+        z = d[e, :r].double()
+        assert bool(((tn[e].double() - x.t() @ z).abs() <= _bound(x.t() @ z, x.abs().t() @ z.abs(), cap, dtype)).all())
