@@ -426,7 +426,8 @@ static int run_dispatch_int8(const char *who, const void *x, int dtype, const fl
                "%s: model_dim must be a multiple of %d and buffers 16-byte aligned; "
                "use the unfused entry points otherwise", who, vec);
     hipStream_t st = (hipStream_t)stream;
-    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity,
+                                    (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2), st);
     const int token_blocks = (samples + 3) / 4;
     const int per_lane = (model_dim / vec + WAVE - 1) / WAVE;
     PM_DTYPE_SWITCH(dtype, DT,

@@ -98,10 +98,10 @@ __device__ __forceinline__ void fetch_planes(const float *gates, const int32_t *
     }
 }
 
-// Which slots no live pair addresses.  Up to SLOT_FILL_PAIRS pairs the work-groups that write those slots' zero rows find out
-// themselves: there are 2^shift of them, one in 2^shift slots is a work-group's, and it walks the routing planes and keeps a bit
-// a slot in LDS.  They are the first of the grid, so that the walk is beside the rows of the tokens.  (Two small launches in front for flags
-// in memory cost 9 us of 193 in the routing API's pass at 8192 x 2048, and 10 us of host time in any.)  More pairs: flags.
+// Which slots no live pair addresses.  Up to SLOT_FILL_PAIRS pairs (of narrow rows fewer: slot_fill) the work-groups that write those slots' zero
+// rows find out themselves: there are 2^shift of them, one in 2^shift slots is a work-group's, and it walks the routing planes, 16 loads at once, and
+// keeps a bit a slot in LDS.  They are the first of the grid, so that the walk is beside the rows of the tokens.  (Two small launches in front for
+// flags in memory cost 9 us of 193 in the routing API's pass at 8192 x 2048, and 10 us of host time in any.)  More pairs: flags.
 constexpr int SLOT_FILL_PAIRS = 1 << 17, SLOT_FILL_BITS = 8192;
 struct SlotFill {
     const uint32_t *flags;                       // NULL: bits in LDS
@@ -126,21 +126,22 @@ __device__ __forceinline__ void fill_empty_slots(const SlotFill &fill, int numbe
         return;
     }
     __shared__ uint32_t s_used[SLOT_FILL_BITS / 32];
+    constexpr int AT_ONCE = 16;
     const int mine = (slots - number + (1 << fill.shift) - 1) >> fill.shift;          // slots number, number + 2^shift, ..
     for (int i = threadIdx.x; i < (mine + 31) / 32; i += 256) s_used[i] = 0u;
     __syncthreads();
     for (int j = 0; j < top_k; ++j) {
         const int32_t *idx = indices + (int64_t)j * stride, *loc = locations + (int64_t)j * stride;
-        for (int t0 = threadIdx.x; t0 < samples; t0 += 8 * 256) {
-            int e[8], l[8];
+        for (int t0 = threadIdx.x; t0 < samples; t0 += AT_ONCE * 256) {
+            int e[AT_ONCE], l[AT_ONCE];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < AT_ONCE; ++q) {
                 const int t = min(t0 + q * 256, samples - 1);      // (the last token again and again: its bit is its own)
                 e[q] = idx[t];
                 l[q] = loc[t];
             }
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < AT_ONCE; ++q) {
                 const int s = e[q] * capacity + l[q], at = s >> fill.shift;
                 if (e[q] >= 0 && e[q] < experts && l[q] >= 0 && l[q] < capacity && (s & ((1 << fill.shift) - 1)) == number) atomicOr(&s_used[at >> 5], 1u << (at & 31));
             }
@@ -152,7 +153,7 @@ __device__ __forceinline__ void fill_empty_slots(const SlotFill &fill, int numbe
 }
 // how the empty slots are found: the flags' launches, or nothing beforehand
 SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locations, int64_t stride, int top_k, int samples, int experts,
-                   int capacity, hipStream_t st);
+                   int capacity, int64_t row_bytes, hipStream_t st);
 int check_planes(const char *who, const int32_t *indices, const int32_t *locations,
                  int64_t stride, int top_k, int samples);
 // routing of up to 64 experts from [samples, experts] logits / scores with the forward chain's

@@ -337,14 +337,18 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
 }
 
 SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locations, int64_t stride, int top_k, int samples, int experts,
-                   int capacity, hipStream_t st)
+                   int capacity, int64_t row_bytes, hipStream_t st)
 {
     const int slots = experts * capacity;
     const int64_t pairs = (int64_t)samples * top_k;
     // as many work-groups as have 16 slots each, fewer where each has more to walk (8 bytes a pair, from the caches)
     int shift = 0;
     while (shift < (pairs <= 8192 ? 8 : pairs <= 32768 ? 7 : 6) && (slots >> (shift + 1)) >= 16) ++shift;
-    if (pairs <= SLOT_FILL_PAIRS && (slots >> shift) < SLOT_FILL_BITS) return SlotFill{nullptr, 1 << shift, shift};
+    // The walk is as long as the pairs are many, and the rows that hide it are as long as they are wide: up to 8192 pairs it is shorter than the
+    // launches for flags, beyond that from a byte of row for four pairs.  Forward pass of the routing API, flags and walk, us: 8000 pairs of 512
+    // bytes 46.8 and 45.1, 6000 of 2048 35.6 and 31.9; 13200 of 512 50.9 and 52.9, 32768 of 1024 41.6 and 47.9, 32768 of 2048 54.5 and 58.4, 20000 of
+    // 4096 66.8 and 68.8, 32768 of 4096 99.6 and 100.0; with the backward pass 13200 of 4096 130.3 and 125.1, 16384 of 8192 193.8 and 186.4.
+    if (pairs <= std::max<int64_t>(8192, std::min<int64_t>(4 * row_bytes, SLOT_FILL_PAIRS)) && (slots >> shift) < SLOT_FILL_BITS) return SlotFill{nullptr, 1 << shift, shift};
     uint32_t *flags = (uint32_t *)workspace;
     slot_flags_clear<<<(slots + 255) / 256, 256, 0, st>>>(flags, slots);
     if (samples > 0)
@@ -392,7 +396,8 @@ extern "C" int planmoe_dispatch_fwd(const void *x, int dtype, const float *gates
                "planmoe_dispatch_fwd: workspace too small (%zu < %zu)", workspace_bytes,
                planmoe_dispatch_workspace_bytes(experts, capacity));
     hipStream_t st = (hipStream_t)stream;
-    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity,
+                                    (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2), st);
     const int token_blocks = (samples + 3) / 4;
     const int mode = rows_mode(dtype, model_dim, x, dispatched);
     PM_DTYPE_SWITCH(dtype, DT, {
@@ -481,7 +486,8 @@ extern "C" int planmoe_combine_bwd(const void *grad, const void *dispatched, int
     PM_REQUIRE(grad && dispatched && grad_dispatched && grad_gates, "%s: NULL argument", who);
     PM_REQUIRE(workspace && workspace_bytes >= planmoe_dispatch_workspace_bytes(experts, capacity), "%s: workspace too small", who);
     hipStream_t st = (hipStream_t)stream;
-    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity, st);
+    const SlotFill fill = slot_fill(workspace, indices, locations, plane_stride, top_k, samples, experts, capacity,
+                                    (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2), st);
     const int token_blocks = (samples + 3) / 4;
     const int mode = std::min(rows_mode(dtype, model_dim, grad, dispatched), rows_mode(dtype, model_dim, grad_dispatched, grad_dispatched));
     PM_DTYPE_SWITCH(dtype, DT, {
