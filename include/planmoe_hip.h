@@ -642,8 +642,8 @@ int planmoe_bwd_gate_zfp(const void *stream_in, double rate, const float *grad_o
  * last partial block is coded as if padded with zero symbols (the reference reads past the end
  * of its input there, gpulz.cu:36-39), and decoding writes only the first nbytes.
  * Compression sizes every block, scans the sizes in place in the offset tables and then packs
- * every block at its final offset; there is no full-size staging buffer (gpulz.cu:148-211,
- * 220-258 have two).  All five pointers must be 16-byte aligned. */
+ * every block at its final offset; the workspace keeps the tokens of blocks with matches, half the input's size (gpulz.cu:148-211,
+ * 220-258 have two full-size staging buffers).  All five pointers must be 16-byte aligned. */
 int64_t planmoe_lz_blocks(int64_t nbytes);
 size_t planmoe_lz_workspace_bytes(int64_t nbytes);
 int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets, int32_t *data_offsets,

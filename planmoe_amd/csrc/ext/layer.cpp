@@ -1,7 +1,7 @@
 // The layer with its built-in experts as one node: gate, routing, encode, codec, FFN, codec, decode, and
 // the backward pass of all of them, driven from C++.
 //
-// A forward pass is five to nine launches of a few microseconds each at decode sizes; driven step by step
+// A forward pass is four to nine launches of a few microseconds each at decode sizes; driven step by step
 // from Python (an autograd node, a dozen tensor operations and a ctypes call with two dozen arguments for
 // each) the host took 160 us for 40 us of GPU work.  Here a pass is one call: outputs and workspaces from
 // torch's caching allocator, launches through the C ABI of libplanmoe_hip.
