@@ -262,11 +262,11 @@ def test_prescore_mode_gates_at_encode():
     assert np.array_equal(raw(out), want_out.view(np.int32))
 
 
-# empty slots found by the work-groups that fill them, and by flags in memory: pairs either side of 8192 (narrow rows), of a pair for a quarter of a
-# byte of row, and of 2^17; slots either side of the bits a work-group keeps, one slot, fewer slots than work-groups; pairs outside the experts and the
-# capacity, planes that are not adjacent
-@pytest.mark.parametrize("T,k,E,C,M", [(1, 1, 1, 1, 8), (5, 2, 3, 5, 8), (2049, 3, 7, 300, 8), (4096, 2, 58, 150, 8), (8193, 1, 58, 150, 8),
-                                       (8192, 2, 8, 2052, 1024), (8193, 2, 8, 2052, 1024), (65536, 2, 2, 2052, 8192), (65537, 2, 2, 2052, 8192),
+# empty slots found by the work-groups that fill them, and by flags in memory: pairs either side of 8192 and two more a byte
+# of row, with narrow and wide rows, and of 2^17; slots either side of the bits a work-group keeps, one slot, fewer slots than work-groups; pairs
+# outside the experts and the capacity, planes that are not adjacent
+@pytest.mark.parametrize("T,k,E,C,M", [(1, 1, 1, 1, 8), (5, 2, 3, 5, 8), (2049, 3, 7, 300, 8), (4128, 2, 58, 150, 8), (8257, 1, 58, 150, 8),
+                                       (8192, 2, 8, 2052, 1024), (8193, 2, 8, 2052, 1024), (65536, 2, 2, 2052, 16384), (65537, 2, 2, 2052, 16384),
                                        (8000, 1, 64, 32767, 8), (8000, 1, 64, 32768, 8), (300, 2, 64, 8180, 8)])
 def test_empty_slots_are_zero_rows(T, k, E, C, M):
     from planmoe_amd import ops
