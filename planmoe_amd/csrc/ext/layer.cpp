@@ -121,8 +121,7 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     }
     const Live live = live_rows(p, s, codec);
     p.h = at::empty({s.rows(), s.H}, x.options());
-    // (which elements a relu cut is asked by a backward pass only)
-    PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), keep ? 1 : 2, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
+    PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
                                 s.hint(), p.h.data_ptr(), st));
     p.ye = at::empty({s.rows(), s.M}, x.options());
     PM_CALL(planmoe_expert_gemm(0, s.dt, p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
@@ -149,7 +148,8 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
 }
 
 // A pass that nothing is kept of: what only its launches see lies in one buffer (eight allocations take the host 9 us, a third
-// of a decode step's time, three 3).  The lz codec has its own buffers.
+// of a decode step's time, three 3).  The lz codec has its own buffers.  The products are those of a pass that a backward pass follows: the
+// same bits with and without autograd (a checkpoint's first run is without, its second with).
 std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2,
                                           const Shape &s, bool fp32_gate, bool normalize, int codec)
 {
@@ -181,8 +181,7 @@ std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, con
         gates = (const float *)(base + wide_at);
     }
     const int round = codec == CODEC_ZFP ? 4 : 1;
-    // (which elements a relu cut is asked by a backward pass only)
-    PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 2, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
+    PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
     PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, round, s.hint(), ye, st));
     if (codec == CODEC_ZFP) PM_CALL(planmoe_layer_zfp_rows((float *)ye, s.M, s.E, s.cap, cnt, s.k, nullptr, 0, st));
     PM_CALL(planmoe_layer_combine(ye, s.dt, codec == CODEC_INT8, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));

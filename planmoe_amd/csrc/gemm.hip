@@ -829,7 +829,7 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
 {
     const char *who = "planmoe_expert_gemm";
     if (expert_gemm_check(who, form, dtype, a, b, batches, m, n, k, live, live_planes, live_round, c)) return 1;
-    PM_REQUIRE(activation >= 0 && activation <= 2, "%s: activation is 0 (none), 1 (relu) or 2 (relu without a backward pass)", who);
+    PM_REQUIRE(activation == 0 || activation == 1, "%s: activation is 0 (none) or 1 (relu)", who);
     PM_REQUIRE(!bias || form != 2, "%s: a weight gradient has no bias", who);
     hipStream_t st = (hipStream_t)stream;
     if (dtype == PLANMOE_F32) {

@@ -355,7 +355,7 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
     return (form == 1 || ((int64_t)p.K + 128) * p.N < reach) && (form != 2 || ((int64_t)p.K + 128) * p.M < reach);
 }
 
-// The tile's side under a relu whose backward pass asks what it cut: a compute unit takes 1.9 us for a k-tile of 128 x 128 and 4 for the tile, 0.52 and
+// The tile's side under a relu: a compute unit takes 1.9 us for a k-tile of 128 x 128 and 4 for the tile, 0.52 and
 // 1.2 for 64 x 64, 0.47 with four stages; what counts is the fullest compute unit (us, 64 x 64, with four stages, 128 x 128: 4 x 1000 rows,
 // 2048 -> 512 77, 66, 137; 16 x 512, 1024 -> 1024 142, 131, 131; 512 -> 2048 152, 144, 138; 2 x 4096, 4096 -> 4096 2129, 1944, 1969).
 // Waves on their own, up to 16 rows (32 where a tile has less than eight k-tiles), where they read the weight once (8 experts, 2 rows each: nn
@@ -379,8 +379,9 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 //   2 x 4096, 4096, 4096 nt         2005       1727    1434   1259
 //   4 x 1000, 512, 2048 tn            75         66      52     76
 //   8 x 300, 712, 712 nn              30         26      32     50
-// Not under a relu whose backward pass asks which elements it cut: one within rounding of zero that is cut here and kept there
-// changes a weight gradient by 1e-3 of itself at 2^20 elements, so that product keeps the library's order of sums.  Not up to
+// Not under a relu, whose backward pass asks which elements it cut: one within rounding of zero that is cut here and kept there
+// changes a weight gradient by 1e-3 of itself at 2^20 elements, so that product keeps the library's order of sums, and keeps it
+// where no backward pass follows (a pass without autograd has the bits of the one with it: a checkpoint runs both).  Not up to
 // 64 rows, where reading the weight takes as long as the fp32 matrix cores do (16 x 56, 1792 -> 1992 and back: 201 us in fp32, 205 in parts).  And not
 // with rows or columns of less than 256 values, where a product of few rows on waves has the same sums as one of many.
 static Gemm32Kernel gemm_f32_pick_split(int form, const Gemm32Args &p, int rows_hint)
@@ -408,7 +409,7 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
     if (form != 2 && rows_hint <= (deep ? 16 : 32) && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
         gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
         return G32_WAVES;
-    if (p.relu != 1 && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
+    if (!p.relu && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
     auto cost = [&](int64_t side, double us, double once) {

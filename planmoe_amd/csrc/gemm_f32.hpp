@@ -10,7 +10,7 @@ struct Gemm32Args {
     const int *live;                       // [live_planes][batches]: rows in use (k of a tn product), NULL: all
     int live_planes, live_round;
     int M, N, K, batches;                  // operands and result contiguous
-    int relu;                              // 1; 2: and no backward pass asks which elements it cut
+    int relu;
 };
 
 // Kernels: waves on their own; tiles of 64 x 64 (two and four k-tiles in LDS) and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128

@@ -78,6 +78,8 @@ def test_argument_errors_are_reported_without_a_gpu():
     assert rc != 0 and b"multiples of 8" in lib.planmoe_last_error()
     rc = lib.planmoe_gemm_nn_bf16(p16, p16, None, 2, 1, 64, 64, 64, 64, 64, 64, 0, 0, 0, p16, None)
     assert rc != 0 and b"activation" in lib.planmoe_last_error()
+    rc = lib.planmoe_expert_gemm(0, 0, p16, p16, p16, 2, 1, 64, 64, 64, None, 1, 1, 0, p16, None)
+    assert rc != 0 and b"activation" in lib.planmoe_last_error()
     assert lib.planmoe_gemm_tn_bf16(None, None, 0, 64, 64, 64, 64, 64, 64, 0, 0, 0, None, None) == 0
     # empty inputs are a successful no-op
     assert lib.planmoe_int8_compress(None, 0, 0, 8, None, None, None, None) == 0

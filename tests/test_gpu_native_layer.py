@@ -529,3 +529,34 @@ def test_all_gradients_equal_one_at_a_time(codec, dtype, fp32_gate, T, M, H, E, 
     for p, got in zip(params, whole):
         one = grads([p])[0]
         assert got is not None and torch.equal(got, one), (tuple(p.shape), float((got.double() - one.double()).abs().max()))
+
+
+# the same in fp32 where products go over in three bf16 parts a value (more than 64 rows an expert, rows of 256 values and more): the product
+# under the relu keeps one order of sums in both passes, so a frozen copy, an evaluation and a checkpoint's first run see the same bits
+@pytest.mark.parametrize("codec", ["no", "int8", "zfp", "lz"])
+@pytest.mark.parametrize("T", [500, 4096])
+def test_inference_equals_the_pass_with_autograd_in_larger_fp32_products(codec, T):
+    layer = _layer(torch.float32, codec, M=512, H=1024, E=8)
+    x = torch.randn(T, 512, device=DEV, generator=torch.Generator(device=DEV).manual_seed(T))
+    want = layer(x)
+    with torch.no_grad():
+        got = layer(x)
+    torch.cuda.synchronize()
+    assert want.requires_grad and torch.equal(got, want) and torch.equal(got.l_aux, want.l_aux)
+
+
+def test_reentrant_checkpoint_gives_the_gradients_of_the_plain_pass_in_fp32():
+    """Its first run is without autograd, its second with it."""
+    from torch.utils.checkpoint import checkpoint
+    layer = _layer(torch.float32, M=512, H=1024, E=8)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, gy = (torch.randn(4096, 512, device=DEV, generator=g) for _ in range(2))
+    want = _pass(layer, x, gy)
+    layer.zero_grad()
+    v = x.clone().requires_grad_(True)
+    y = checkpoint(layer, v, use_reentrant=True)
+    y.backward(gy)
+    got = {"y": y.detach(), "dx": v.grad, **{n: p.grad for n, p in layer.named_parameters()}}
+    torch.cuda.synchronize()
+    for name in want:
+        assert torch.equal(want[name], got[name]), name
