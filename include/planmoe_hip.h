@@ -442,8 +442,8 @@ int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int 
  * a [batches, m, k], b [batches, k, n]; form 1: c = a b^T, b [batches, n, k]; form 2: c = a^T b, a [batches,
  * k, m], b [batches, k, n].  Roundings as planmoe_gemm_*_bf16.  fp32: products and sums are no less precise than
  * an fp32 multiply and add a k; the order of the sums is that of the fp32 matrix cores' products of 16 x 16 x 4
- * with activation 1, and with row lengths under 256, where it does not depend on m; elsewhere it may differ from shape to shape.
- * activation: 0 none, 1 relu.
+ * with activation 1, and with row lengths under 256, where it does not depend on m; elsewhere it may differ from shape to shape
+ * (form, batches, m, n, k), but not with live or rows_hint.  activation: 0 none, 1 relu.
  * live, if not NULL: int32 [live_planes][batches], e.g. the expert_counts of the routing.  Batch e then has
  * min(sum of its entries rounded up to live_round, m) rows (form 2: that many k) in use; rows of c beyond
  * them are not written, rows of a and b beyond them are not read (up to 64 batches).  rows_hint: the number

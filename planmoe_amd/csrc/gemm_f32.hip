@@ -382,34 +382,55 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 // Not under a relu, whose backward pass asks which elements it cut: one within rounding of zero that is cut here and kept there
 // changes a weight gradient by 1e-3 of itself at 2^20 elements, so that product keeps the library's order of sums, and keeps it
 // where no backward pass follows (a pass without autograd has the bits of the one with it: a checkpoint runs both).  Not up to
-// 64 rows, where reading the weight takes as long as the fp32 matrix cores do (16 x 56, 1792 -> 1992 and back: 201 us in fp32, 205 in parts).  And not
+// 64 rows, where reading the weight takes as long as the fp32 matrix cores do (8 x 59, 3936 -> 3536: 136 us in fp32, 173 in parts).  And not
 // with rows or columns of less than 256 values, where a product of few rows on waves has the same sums as one of many.
-static Gemm32Kernel gemm_f32_pick_split(int form, const Gemm32Args &p, int rows_hint)
+// Which of the two it is depends on the buffers' shape alone, not on the rows in use or expected: in parts the sums run in another
+// order, and the layer as one node, which knows those rows, has to give the bits of its steps, which do not.  It is decided for all rows in use
+// and for 4 of 5 (a capacity factor of 1.25), and only the tile by the rows expected.  Of 30000 products of layers with capacity factors of 1 to
+// 1.5, 662 are computed in the slower way of the two for it, by 2.4 % on average by the figures above (for all rows alone 682, by 4.2 %).
+// The far ends (us, 8 experts, fp32 and parts): capacity 72, 59 in use, 3936 -> 3536 136 and 173, all 72 in use 237 and 184; 952,
+// 634 in use, 2240 -> 640 134 and 94.
+struct SplitCost {                               // us: 64 x 64 in fp32; 64 x 64, 128 x 128, 256 x 128 in parts
+    double whole, t64, t128, t256;
+    double in_parts() const { return std::min(t64, std::min(t128, t256)); }
+};
+
+static SplitCost gemm_f32_split_cost(int form, const Gemm32Args &p, int64_t m, int64_t k)
 {
-    const double cu = compute_units(), kt = (double)(((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK);
-    // (row counts from the device: an expectation, and a batch may have a standard deviation more)
-    const int64_t m = form == 2 ? p.M : p.live ? std::min<int64_t>(p.M, rows_hint + (int64_t)std::sqrt((double)rows_hint)) : rows_hint;
+    const double cu = compute_units(), kt = (double)((k + G32_BK - 1) / G32_BK);
     auto tiles = [&](int64_t bm, int64_t bn) { return (double)((m + bm - 1) / bm * ((p.N + bn - 1) / bn) * p.batches); };
     auto rounds = [&](double t, double low, double high, double once) {
         const double full = std::floor(t / cu), rest = t - full * cu;
         return full * (high * kt + once) + (rest > 0 ? (low + (high - low) * rest / cu) * kt + once : 0.);
     };
     const double small = std::ceil(tiles(64, 64) / cu), t64 = (small <= 1 ? 0.6 : 0.44 * small) * kt + 6;
-    const double t128 = rounds(tiles(128, 128), 1.1, 1.4, 6), t256 = rounds(tiles(256, 128), 1.9, 2.5, 7);
-    const bool deep = gemm_f32_deep(form, p, rows_hint);
-    const double whole = deep ? (small <= 1 ? 0.43 : 0.44 * small) * kt + 3.5 + 0.5 * small : small <= 1 ? t64 : 1e30;
-    if (whole <= t64 && whole <= t128 && whole <= t256) return deep ? G32_DEEP_64 : G32_TILE_64;
-    if (t64 <= t128 && t64 <= t256) return G32_SPLIT_64;
-    return t128 <= t256 ? G32_SPLIT_128 : G32_SPLIT_256;
+    // (with two stages 0.52 a k-tile)
+    const double whole = gemm_f32_deep(form, p, (int)k) ? (small <= 1 ? 0.43 : 0.44 * small) * kt + 3.5 + 0.5 * small : small <= 1 ? t64 : 1.18 * t64;
+    return SplitCost{whole, t64, rounds(tiles(128, 128), 1.1, 1.4, 6), rounds(tiles(256, 128), 1.9, 2.5, 7)};
+}
+
+static bool gemm_f32_in_parts(int form, const Gemm32Args &p)
+{
+    if (p.relu || p.N < 256 || (form == 2 ? p.M : p.K) < 256) return false;
+    const int64_t all = form == 2 ? p.K : p.M, most = (4 * all + 4) / 5;
+    if (form != 2 && most <= 64) return false;
+    auto cost = [&](int64_t rows) { return form == 2 ? gemm_f32_split_cost(form, p, p.M, rows) : gemm_f32_split_cost(form, p, rows, p.K); };
+    const SplitCost a = cost(all), b = cost(most);
+    return a.in_parts() * b.in_parts() < a.whole * b.whole;
 }
 
 Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
 {
+    if (gemm_f32_in_parts(form, p)) {
+        // (row counts from the device: an expectation, and a batch may have a standard deviation more)
+        const int64_t rows = p.live ? std::min<int64_t>(p.M, rows_hint + (int64_t)std::sqrt((double)rows_hint)) : rows_hint;
+        const SplitCost c = gemm_f32_split_cost(form, p, form == 2 ? p.M : rows, form == 2 ? rows_hint : p.K);
+        return c.t64 <= c.in_parts() ? G32_SPLIT_64 : c.t128 <= c.t256 ? G32_SPLIT_128 : G32_SPLIT_256;
+    }
     const bool deep = gemm_f32_deep(form, p, rows_hint);
     if (form != 2 && rows_hint <= (deep ? 16 : 32) && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
         gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
         return G32_WAVES;
-    if (!p.relu && p.N >= 256 && (form == 2 ? p.M : p.K) >= 256 && (form == 2 || rows_hint > 64)) return gemm_f32_pick_split(form, p, rows_hint);
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
     auto cost = [&](int64_t side, double us, double once) {

@@ -542,3 +542,34 @@ def test_expert_gemm_tile_alone(cap, n, counts, k):
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), r, dtype)).all())
         z = d[e, :r].double()
         assert bool(((tn[e].double() - x.t() @ z).abs() <= _bound(x.t() @ z, x.abs().t() @ z.abs(), cap, dtype)).all())
+
+
+# fp32: the order of the sums is the buffer's shape's, not that of the rows in use or expected: a product over the rows in use (the layer as one
+# node) has the bits of the one over the whole buffer (its steps).  Few rows expected of a capacity that is computed in parts and of one that is
+# not, capacities of 80 and one piece more, rows for which the other way would be the faster one; a tn product's reduction over few rows and all
+@pytest.mark.parametrize("B,cap,n,k,hint", [(16, 76, 1036, 1028, 60), (16, 100, 1036, 1028, 60), (16, 128, 2048, 512, 8), (8, 320, 1024, 1024, 100), (8, 200, 520, 512, 16),
+                                            (16, 80, 1024, 512, 64), (16, 84, 2048, 512, 64), (8, 952, 320, 1120, 634), (4, 600, 512, 1024, 256), (4, 300, 1024, 1028, 200)])
+def test_expert_gemm_fp32_does_not_depend_on_the_rows_in_use(B, cap, n, k, hint):
+    from planmoe_amd import ops
+    print("case", B, cap, n, k, hint, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(cap + n + k)
+    counts = [min(cap, max(0, hint + 7 * (e % 5 - 2))) for e in range(B)]
+    counts[0], counts[1] = 0, cap
+    live = torch.tensor([counts], dtype=torch.int32, device=DEV)
+    a, d = torch.randn(B, cap, k, device=DEV, generator=g), torch.randn(B, cap, n, device=DEV, generator=g)
+    w, bias, h = torch.randn(B, k, n, device=DEV, generator=g), torch.randn(B, n, device=DEV, generator=g), torch.randn(B, cap, n, device=DEV, generator=g).clamp(min=0)
+    for e, r in enumerate(counts):
+        a[e, r:] = d[e, r:] = 0.0
+    wt, kw = w.transpose(1, 2).contiguous(), dict(live=live, rows_hint=hint)
+    for relu in (False, True):
+        got, want = ops.expert_gemm("nn", a, w, bias, relu=relu, **kw), ops.expert_gemm("nn", a, w, bias, relu=relu)
+        for e, r in enumerate(counts):
+            assert torch.equal(got[e, :r], want[e, :r]), ("nn", relu, e)
+    got, want = ops.expert_gemm("nt", a, wt, **kw), ops.expert_gemm("nt", a, wt)
+    masked, _ = ops.expert_gemm_relu_bwd(a, wt, h, **kw)
+    for e, r in enumerate(counts):
+        assert torch.equal(got[e, :r], want[e, :r]), ("nt", e)
+        assert torch.equal(masked[e, :r], torch.where(h[e, :r] > 0, want[e, :r], torch.zeros((), device=DEV))), ("masked", e)
+    got, want = ops.expert_gemm("tn", a, d, **kw), ops.expert_gemm("tn", a, d)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

@@ -531,6 +531,18 @@ def test_all_gradients_equal_one_at_a_time(codec, dtype, fp32_gate, T, M, H, E, 
         assert got is not None and torch.equal(got, one), (tuple(p.shape), float((got.double() - one.double()).abs().max()))
 
 
+# fp32, products in three bf16 parts a value among them: the node's, over the rows in use, have the bits of the steps', over the whole buffer.  Capacities
+# on either side of the rows that are left to the fp32 matrix cores, some beyond the rows expected
+@pytest.mark.parametrize("codec,cf", [("no", 1.0), ("no", 1.25), ("no", 1.5), ("lz", 1.25)])
+@pytest.mark.parametrize("T", [240, 1000, 3000])
+def test_native_layer_has_the_bits_of_its_steps_in_fp32(codec, cf, T):
+    args = (codec, torch.float32, T, 512, 1024, 8, 2, cf)
+    for train in (False, True):
+        got, want = _run(True, *args, train), _run(False, *args, train)
+        for name in ["y", "l_aux"] + (["experts.batched_fc1_w", "experts.batched_fc2_w"] if train else []):      # (other sums have kernels of their own)
+            assert torch.equal(got[name], want[name]), (name, train)
+
+
 # the same in fp32 where products go over in three bf16 parts a value (more than 64 rows an expert, rows of 256 values and more): the product
 # under the relu keeps one order of sums in both passes, so a frozen copy, an evaluation and a checkpoint's first run see the same bits
 @pytest.mark.parametrize("codec", ["no", "int8", "zfp", "lz"])
