@@ -33,8 +33,9 @@ def _env_flag(name):
 
 
 def _first_parameter(module):
-    """next(module.parameters(), None), without the walk where the module holds parameters itself."""
-    if type(module).__dict__.get('parameters') is None and isinstance(module, torch.nn.Module) and 'parameters' not in module.__dict__:
+    """next(module.parameters(), None), without the walk where a plain module holds parameters itself."""
+    if (type(module) in _overlap.PLAIN_MODULES and type(module).parameters is torch.nn.Module.parameters and
+            'parameters' not in module.__dict__ and 'named_parameters' not in module.__dict__):
         for p in module._parameters.values():
             if p is not None:
                 return p
@@ -292,4 +293,5 @@ class MOELayer(torch.nn.Module):
                                     normalize_gate=self.normalize_gate, group=self.group, alignment=alignment)
 
 
+_overlap.PLAIN_MODULES.add(MOELayer)
 moe_layer = MOELayer

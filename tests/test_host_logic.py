@@ -208,3 +208,64 @@ def test_capacity_is_the_librarys():
                  (1 << 30, 1, 1, 4.0, 1)):
         with pytest.raises(PlanMoEError):
             ops.capacity(*args)
+
+
+def _small_layer(cls=planmoe_amd.moe_layer):
+    return cls({"type": "top", "k": 2}, 8, experts={"type": "ffn", "count_per_node": 4, "hidden_size_per_expert": 8})
+
+
+def test_submodules_and_parameters_of_a_subclass_are_what_it_says():
+    """Properties come before what a module registered, a search of the class's own after it; parameters() may come from a base class."""
+    from planmoe_amd.experts import FusedExpertsNetwork
+    from planmoe_amd.moe_layer import _first_parameter
+    from planmoe_amd.overlap import held
+    other = _small_layer()
+
+    class Elsewhere(planmoe_amd.moe_layer):
+        experts = property(lambda self: other.experts)
+        gates = property(lambda self: other.gates)
+
+    class Searching(planmoe_amd.moe_layer):
+        def __getattr__(self, name):
+            return getattr(other, name) if name in ("experts", "gates") and "built" in self.__dict__ else super().__getattr__(name)
+
+    found = torch.nn.Parameter(torch.zeros(1, dtype=torch.float64))
+
+    class Mixin:
+        def parameters(self, recurse=True):
+            yield found
+
+    class Base(Mixin, FusedExpertsNetwork):
+        pass
+
+    class Experts(Base):
+        pass
+
+    layer = _small_layer()
+    assert held(layer, "experts") is layer.experts and held(layer, "gates") is layer.gates
+    assert _first_parameter(layer.experts) is next(layer.experts.parameters())
+    for cls in (Elsewhere, Searching):
+        layer = _small_layer(cls)
+        layer.__dict__["built"] = True
+        assert layer.experts is other.experts and held(layer, "experts") is other.experts and held(layer, "gates") is other.gates, cls
+    experts = Experts(8)
+    experts.update(other)
+    assert next(experts.parameters()) is found and _first_parameter(experts) is found
+    plain = _small_layer().experts
+    plain.named_parameters = lambda *args, **kw: iter([("found", found)])
+    assert _first_parameter(plain) is next(plain.parameters()) is found
+
+
+def test_hooks_of_a_module_are_found_by_their_names():
+    """Not in its dictionary alone: a class may hold them."""
+    from planmoe_amd.overlap import _hooked
+
+    class Quiet(torch.nn.Linear):
+        _backward_pre_hooks = {}
+
+    module = Quiet(2, 2)
+    assert not _hooked(module)
+    del module.__dict__["_backward_pre_hooks"]
+    assert not _hooked(module)
+    module.register_forward_hook(lambda *args: None)
+    assert _hooked(module)
