@@ -68,9 +68,10 @@ def planes(tensors, dtype):
 
 # ------------------------------------------------------------------------------ routing
 def capacity(samples, experts, top_k, capacity_factor=1.0, alignment=1):
-    """planmoe_capacity, worked out here (a call of the library takes 1.5 us of every layer call); the library is asked
-    about what it may refuse."""
-    if samples >= 0 and experts >= 1 and top_k >= 1 and 0 < capacity_factor < 1 << 30 and alignment >= 1:
+    """planmoe_capacity, worked out here for plain numbers (a call of the library takes 1.5 us of every layer call); the
+    library is asked about what it may refuse, and about numbers of other types (tensors, numpy's, a fractional alignment)."""
+    if (type(samples) is type(experts) is type(top_k) is type(alignment) is int and type(capacity_factor) in (float, int) and
+            0 <= samples < 1 << 31 and experts >= 1 and top_k >= 1 and 0 < capacity_factor < 1 << 30 and alignment >= 1):
         out = min(top_k, experts) * int(float(capacity_factor) * -(-samples // experts))
         out += -out % alignment
         if out < 1 << 31:

@@ -210,6 +210,19 @@ def test_capacity_is_the_librarys():
             ops.capacity(*args)
 
 
+def test_capacity_of_other_numbers_than_plain_ones_is_the_librarys_too():
+    """A fractional alignment is cut, a factor may be a text, a fractional number of tokens is refused."""
+    import ctypes
+    import numpy as np
+    for args in ((64, 8, 2, 1.0, 2.5), (64, 8, 2, 1.0, 4.0), (64, 8, 2, 1.0, torch.tensor(4)), (64, 8, 2, "1.0", "4"),
+                 (torch.tensor(64), np.int64(8), 2, np.float32(1.0), np.int64(4))):
+        got = ops.capacity(*args)
+        assert type(got) is int and got == 16, args
+    for args in ((64.0, 8, 2), (64, 8, 2.0), (64, 8.0, 2)):
+        with pytest.raises(ctypes.ArgumentError):
+            ops.capacity(*args)
+
+
 def _small_layer(cls=planmoe_amd.moe_layer):
     return cls({"type": "top", "k": 2}, 8, experts={"type": "ffn", "count_per_node": 4, "hidden_size_per_expert": 8})
 
