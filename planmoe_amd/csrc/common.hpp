@@ -63,6 +63,14 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi)
     const f32x2_t p = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
 }
+// relu of two bf16 values.  As int16 what becomes zero is at most -128 (minus infinity), a NaN with its sign set above that: like
+// every other NaN it stays.
+__device__ __forceinline__ uint32_t relu_bf16x2(uint32_t v)
+{
+    typedef short s16x2 __attribute__((ext_vector_type(2)));
+    const s16x2 drop = __builtin_elementwise_add_sat(__builtin_bit_cast(s16x2, v), (s16x2)(short)127) >> 15;
+    return v & ~__builtin_bit_cast(uint32_t, drop);
+}
 
 __device__ __forceinline__ float f16_to_f32(uint32_t bits)
 {

@@ -465,12 +465,9 @@ __global__ __launch_bounds__(GEMM_WG, S::WAVES_PER_SIMD) void gemm_bf16_kernel(c
                             for (int x = 0; x < 4; ++x)
                                 v[x] = f32x2_to_bf16x2(__uint_as_float(v[x] << 16) + add[2 * x], __uint_as_float(v[x] & 0xffff0000u) + add[2 * x + 1]);
                         }
-                        if (!GRAD && p.relu) {    // (negative bf16 are negative int16; a NaN stays)
+                        if (!GRAD && p.relu) {
 #pragma unroll
-                            for (int x = 0; x < 4; ++x) {
-                                typedef short s16x2 __attribute__((ext_vector_type(2)));
-                                v[x] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, (uint32_t)v[x]), (s16x2)(short)0));
-                            }
+                            for (int x = 0; x < 4; ++x) v[x] = relu_bf16x2(v[x]);
                         }
                         if (GRAD) {               // relu's backward: kept where its output was positive
 #pragma unroll

@@ -183,10 +183,9 @@ __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
 #pragma unroll
                     for (int x = 0; x < 2; ++x) v[x] = f32x2_to_bf16x2(__uint_as_float(v[x] << 16) + add[2 * x], __uint_as_float(v[x] & 0xffff0000u) + add[2 * x + 1]);
                 }
-                if (!GRAD && p.relu) {           // (negative bf16 are negative int16; a NaN stays)
-                    typedef short s16x2 __attribute__((ext_vector_type(2)));
+                if (!GRAD && p.relu) {
 #pragma unroll
-                    for (int x = 0; x < 2; ++x) v[x] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, v[x]), (s16x2)(short)0));
+                    for (int x = 0; x < 2; ++x) v[x] = relu_bf16x2(v[x]);
                 }
                 if (GRAD) {                      // relu's backward: kept where its output was positive
                     const pm_u32x2 keep = __builtin_bit_cast(pm_u32x2, __builtin_amdgcn_raw_buffer_load_b64(mask, at, 0, 0));

@@ -573,3 +573,24 @@ def test_expert_gemm_fp32_does_not_depend_on_the_rows_in_use(B, cap, n, k, hint)
     got, want = ops.expert_gemm("tn", a, d, **kw), ops.expert_gemm("tn", a, d)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+# A NaN goes through the relu whatever its sign, from an operand and from the bias, in every kernel: few rows on waves, a tile alone, tiles of 128 and 256
+# rows by 256 columns and 128 x 128, and in fp32
+@pytest.mark.parametrize("dtype,B,m,n,k", [(torch.bfloat16, 2, 16, 72, 64), (torch.bfloat16, 2, 40, 72, 64), (torch.bfloat16, 8, 500, 2048, 200), (torch.bfloat16, 8, 4096, 1024, 64),
+                                           (torch.bfloat16, 8, 1030, 1032, 72), (torch.float32, 2, 16, 72, 64), (torch.float32, 2, 100, 72, 64)])
+def test_expert_gemm_relu_keeps_nan_of_either_sign(dtype, B, m, n, k):
+    from planmoe_amd import ops
+    print("case", dtype, B, m, n, k, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    a, w = torch.randn(B, m, k, device=DEV, generator=g).to(dtype), torch.randn(B, k, n, device=DEV, generator=g).to(dtype)
+    bias = torch.randn(B, n, device=DEV, generator=g).to(dtype)
+    bits, sign = (torch.int16, -64) if dtype == torch.bfloat16 else (torch.int32, -4194304)        # 0xffc0 (0000): a NaN with its sign set
+    bias.view(bits)[0, 3] = sign
+    bias[0, 6], bias[1, 5] = float("nan"), float("-inf")
+    if dtype == torch.bfloat16: bias.view(bits)[1, 8:10] = torch.tensor([-1, -127], dtype=bits, device=DEV)
+    a.view(bits)[B - 1, m - 1, 2] = sign
+    got = ops.expert_gemm("nn", a, w, bias, relu=True)
+    want = torch.relu(torch.bmm(a.float(), w.float()) + bias.float()[:, None])
+    torch.cuda.synchronize()
+    assert torch.equal(got.isnan(), want.isnan()) and bool((got[1, :m - 1, 5] == 0).all()) and bool((got[~got.isnan()] >= 0).all())
