@@ -454,6 +454,13 @@ int planmoe_expert_gemm(int form, int dtype, const void *a, const void *b, const
                         int batches, int m, int n, int k, const int32_t *live, int live_planes,
                         int live_round, int rows_hint, void *c, void *stream);
 
+/* Which kernel planmoe_expert_gemm takes such a product to on the current device (counted: with live), a name for logs and tests:
+ * "few rows", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"; fp32: "f32 waves",
+ * "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128".
+ * planmoe_expert_gemm_relu_bwd takes the one of form 1 without activation.  NULL where the product would be refused. */
+const char *planmoe_expert_gemm_kernel(int form, int dtype, int activation, int batches, int m, int n, int k,
+                                       int counted, int rows_hint);
+
 /* The gradient through the first product's relu: c = a b^T where h > 0, else 0 (a [batches, m, k] the
  * gradient of the second product's result, b [batches, n, k] its weight, h [batches, m, n] the activations),
  * and the first bias's gradient dbias [batches, n] = column sums of c over the rows in use (NULL: not

@@ -84,6 +84,7 @@ SIGNATURES = {
                                      c_int64, c_int64, c_void_p, c_void_p]),
     "planmoe_expert_gemm": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                     c_int, c_int, c_void_p, c_void_p]),
+    "planmoe_expert_gemm_kernel": (ctypes.c_char_p, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "planmoe_expert_gemm_relu_bwd_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "planmoe_expert_gemm_relu_bwd": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
                                              c_int, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

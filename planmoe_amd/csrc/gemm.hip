@@ -706,35 +706,60 @@ bool gemm_is_skinny(bool nt, int m, int n, int64_t k, int batches)
 //   8 x 110, 2696 -> 2488                39, 32 and 37, 29      a^T b, 4 x 512 x 768 over 2000 rows    20 and 15
 bool gemm_is_deep(double tiles, int m) { return tiles <= 0.8 * compute_units() || (m <= 128 && tiles <= compute_units()); }
 
+enum GemmKernel { GEMM_SKINNY, GEMM_DEEP, GEMM_128, GEMM_LOW_128, GEMM_LOW_160, GEMM_LOW_192, GEMM_256, GEMM_256_QUARTERS };
+
+// form: 0 nn, 1 nt, 2 tn; contiguous: the operands and the result are; rows: expected of a batch (tn: of its reduction)
+GemmKernel gemm_pick(int form, bool contiguous, int m, int n, int k, int batches, bool counted, int64_t rows)
+{
+    const bool tn = form == 2;
+    if (!tn && contiguous && gemm_is_skinny(form == 1, m, n, k, batches)) return GEMM_SKINNY;
+    const GemmCost cost{(double)(tn ? m : rows), (double)(((tn ? rows : k) + 63) / 64), (double)compute_units(), m, n, batches,
+                        tn ? 0 : (int64_t)n * k * batches * 2, !tn && counted};
+    const bool deep = contiguous && gemm_is_deep(cost.tiles(128, 128), m) && gemm_deep_reaches(form, m, n, k);
+    const double small = (deep ? 0.88 : 1.) * cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
+    if (!tn) {
+        const double low[3] = {cost.low(128), cost.low(160), cost.low(192)};
+        const int f = low[0] <= low[1] && low[0] <= low[2] ? 0 : low[1] <= low[2] ? 1 : 2;
+        if (low[f] < small && low[f] < big) return f == 0 ? GEMM_LOW_128 : f == 1 ? GEMM_LOW_160 : GEMM_LOW_192;
+    }
+    if (small < big) return deep ? GEMM_DEEP : GEMM_128;
+    return big == split ? GEMM_256_QUARTERS : GEMM_256;
+}
+
+bool gemm_contiguous(int form, int m, int n, int k, int lda, int ldb, int ldc, int64_t sa, int64_t sb, int64_t sc)
+{
+    return lda == k && ldb == (form == 1 ? k : n) && ldc == n && sb == (int64_t)n * k && sa == (int64_t)m * k && sc == (int64_t)m * n;
+}
+
+GemmSlots gemm_slots(GemmKernel kernel)
+{
+    switch (kernel) {
+    case GEMM_SKINNY: return GemmSlots{0, 1};
+    case GEMM_LOW_128: return GemmSlots{128, 1};
+    case GEMM_LOW_160: return GemmSlots{160, 1};
+    case GEMM_LOW_192: return GemmSlots{192, 1};
+    default: return GemmSlots{128, 2};
+    }
+}
+
 template <bool TA, bool TB, bool GRAD>
 int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who, GemmSlots *sums = nullptr)
 {
-    if (sums) *sums = GemmSlots{128, 2};
-    const bool contiguous = p.lda == p.K && p.ldb == (TB ? p.N : p.K) && p.ldc == p.N && p.sB == (int64_t)p.N * p.K && p.sA == (int64_t)p.M * p.K &&
-                            p.sC == (int64_t)p.M * p.N;
+    constexpr int form = TA ? 2 : TB ? 0 : 1;
+    const bool contiguous = gemm_contiguous(form, p.M, p.N, p.K, p.lda, p.ldb, p.ldc, p.sA, p.sB, p.sC);
     const SkinnyArgs few{p.A, p.B, p.bias, p.mask, p.C, p.colsum, p.live, p.live_planes, p.live_round, p.M, p.N, p.K, p.batches, p.relu};
-    if (!TA && contiguous && gemm_is_skinny(!TB, p.M, p.N, p.K, p.batches)) {
-        if (sums) *sums = GemmSlots{0, 1};
-        return gemm_skinny_run(!TB, few, stream, who);
-    }
-    const int64_t cu = compute_units();
-    const GemmCost cost{(double)(TA ? p.M : rows_hint), (double)(((TA ? rows_hint : p.K) + 63) / 64), (double)cu, p.M, p.N, p.batches,
-                        TA ? 0 : (int64_t)p.N * p.K * p.batches * 2, !TA && p.live};
-    const bool deep = contiguous && gemm_is_deep(cost.tiles(128, 128), p.M) && gemm_deep_reaches(TA ? 2 : TB ? 0 : 1, p.M, p.N, p.K);
-    const double small = (deep ? 0.88 : 1.) * cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
+    const GemmKernel kernel = gemm_pick(form, contiguous, p.M, p.N, p.K, p.batches, p.live, rows_hint);
+    if (sums) *sums = gemm_slots(kernel);
     if constexpr (!TA) {
-        const double low[3] = {cost.low(128), cost.low(160), cost.low(192)};
-        const int f = low[0] <= low[1] && low[0] <= low[2] ? 0 : low[1] <= low[2] ? 1 : 2;
-        if (low[f] < small && low[f] < big) {
-            if (sums) *sums = GemmSlots{128 + 32 * f, 1};
-            if (f == 0) return gemm_launch<GemmFlat<2, 2>, TA, TB, GRAD>(p, stream, who);
-            if (f == 1) return gemm_launch<GemmFlat<2, 3>, TA, TB, GRAD>(p, stream, who);
-            return gemm_launch<GemmFlat<3, 3>, TA, TB, GRAD>(p, stream, who);
-        }
+        if (kernel == GEMM_SKINNY) return gemm_skinny_run(!TB, few, stream, who);
+        if (kernel == GEMM_LOW_128) return gemm_launch<GemmFlat<2, 2>, TA, TB, GRAD>(p, stream, who);
+        if (kernel == GEMM_LOW_160) return gemm_launch<GemmFlat<2, 3>, TA, TB, GRAD>(p, stream, who);
+        if (kernel == GEMM_LOW_192) return gemm_launch<GemmFlat<3, 3>, TA, TB, GRAD>(p, stream, who);
     }
-    if (small < big) return deep ? gemm_deep_run(TA ? 2 : TB ? 0 : 1, few, stream, who) : gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
-    p.stay = (int)(cu / 8 * 8);
-    p.split = big == split;
+    if (kernel == GEMM_DEEP) return gemm_deep_run(form, few, stream, who);
+    if (kernel == GEMM_128) return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
+    p.stay = compute_units() / 8 * 8;
+    p.split = kernel == GEMM_256_QUARTERS;
     if (gemm_launch<Gemm256, TA, TB, GRAD>(p, stream, who)) return 1;
     if (!p.split) return 0;
     p.split = 2;
@@ -842,6 +867,27 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
     if (form == 0) return gemm_run<false, true, false>(p, hint, st, who);
     if (form == 1) return gemm_run<false, false, false>(p, hint, st, who);
     return gemm_run<true, true, false>(p, hint, st, who);
+}
+
+extern "C" const char *planmoe_expert_gemm_kernel(int form, int dtype, int activation, int batches, int m, int n, int k, int counted, int rows_hint)
+{
+    const char *who = "planmoe_expert_gemm_kernel";
+    static const int32_t __attribute__((aligned(16))) some[1] = {0};         // (stands for the operands, which are not read)
+    const int32_t *live = counted ? some : nullptr;
+    auto bad = [&]() -> int {
+        if (expert_gemm_check(who, form, dtype, some, some, batches, m, n, k, live, 1, 1, some)) return 1;
+        PM_REQUIRE(activation == 0 || activation == 1, "%s: activation is 0 (none) or 1 (relu)", who);
+        return 0;
+    };
+    if (bad()) return nullptr;
+    const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
+    if (dtype == PLANMOE_F32) {
+        static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
+        return names[gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint)];
+    }
+    static const char *const names[] = {"few rows", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"};
+    const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n;
+    return names[gemm_pick(form, gemm_contiguous(form, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n), m, n, k, batches, counted, hint)];
 }
 
 extern "C" size_t planmoe_expert_gemm_relu_bwd_workspace_bytes(int batches, int m, int n)

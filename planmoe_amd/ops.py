@@ -771,6 +771,13 @@ def expert_gemm(form, a, b, bias=None, relu=False, live=None, live_round=1, rows
     return out
 
 
+def expert_gemm_kernel(form, dtype, batches, m, n, k, relu=False, counted=False, rows_hint=0):
+    """The name of the kernel that expert_gemm takes a product of these sizes to (planmoe_expert_gemm_kernel; counted: with row counts)."""
+    name = lib.planmoe_expert_gemm_kernel(_FORMS[form], _DT[dtype], int(bool(relu)), batches, m, n, k, int(bool(counted)), int(rows_hint))
+    check(name is None)
+    return name.decode()
+
+
 def expert_gemm_relu_bwd(a, b, h, live=None, live_round=1, rows_hint=0, out=None):
     """(c, dbias): c = a @ b^T where h > 0, else 0; dbias its column sums (planmoe_expert_gemm_relu_bwd)."""
     _need_gpu(a, "expert_gemm_relu_bwd")

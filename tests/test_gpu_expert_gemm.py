@@ -594,3 +594,81 @@ def test_expert_gemm_relu_keeps_nan_of_either_sign(dtype, B, m, n, k):
     want = torch.relu(torch.bmm(a.float(), w.float()) + bias.float()[:, None])
     torch.cuda.synchronize()
     assert torch.equal(got.isnan(), want.isnan()) and bool((got[1, :m - 1, 5] == 0).all()) and bool((got[~got.isnan()] >= 0).all())
+
+
+# Every kernel of the experts' products by its name, and each form that it has: nn, nt and the masked nt with its column sums ("rows"), a^T b ("tn").  Rows in
+# use of none, one, either side of the tiles' sides, a capacity's and the rest as expected, NaN behind them and a sentinel in what must not be
+# written; an even and an odd number of k-tiles, each with a piece of one; columns that no tile divides.  What the shapes are for is asserted: the
+# rules between the kernels are fitted to times and move.
+IN_KERNEL = [
+    (torch.bfloat16, "rows", "few rows", 4, 8, 16, 200, 6), (torch.bfloat16, "rows", "128x128 alone", 4, 300, 264, 136, 200),
+    (torch.bfloat16, "rows", "128x128", 5, 2734, 160, 200, 2734), (torch.bfloat16, "rows", "128x128", 8, 1697, 144, 144, 1697),
+    (torch.bfloat16, "rows", "128x256", 8, 2618, 144, 720, 2356), (torch.bfloat16, "rows", "128x256", 8, 139, 3832, 440, 125),
+    (torch.bfloat16, "rows", "160x256", 8, 801, 1160, 200, 801), (torch.bfloat16, "rows", "160x256", 8, 2118, 392, 136, 2118),
+    (torch.bfloat16, "rows", "192x256", 5, 2722, 520, 200, 2722), (torch.bfloat16, "rows", "192x256", 8, 2765, 280, 144, 2765),
+    (torch.bfloat16, "rows", "256x256", 8, 429, 2608, 200, 429), (torch.bfloat16, "rows", "256x256", 8, 1551, 792, 136, 1551),
+    (torch.bfloat16, "rows", "256x256 and quarters", 8, 1755, 2528, 1264, 1755), (torch.bfloat16, "rows", "256x256 and quarters", 8, 2013, 2160, 1584, 2013),
+    (torch.bfloat16, "tn", "128x128", 4, 203, 16, 136, 182), (torch.bfloat16, "tn", "128x128", 4, 260, 264, 1144, 234),
+    (torch.bfloat16, "tn", "256x256", 8, 201, 2072, 392, 160), (torch.bfloat16, "tn", "256x256", 8, 270, 2712, 264, 216),
+    (torch.bfloat16, "tn", "256x256 and quarters", 4, 1098, 2784, 1512, 1098), (torch.bfloat16, "tn", "256x256 and quarters", 4, 1288, 2480, 1576, 1288),
+    (torch.float32, "rows", "f32 waves", 4, 9, 16, 168, 8), (torch.float32, "rows", "f32 64x64", 4, 37, 16, 164, 37),
+    (torch.float32, "rows", "f32 64x64 four stages", 4, 70, 68, 268, 60), (torch.float32, "rows", "f32 128x128", 8, 73, 3232, 176, 65),
+    (torch.float32, "rows", "f32 parts 64x64", 4, 2618, 260, 292, 2356), (torch.float32, "rows", "f32 parts 64x64", 8, 324, 1052, 260, 291),
+    (torch.float32, "rows", "f32 parts 128x128", 8, 389, 848, 300, 311), (torch.float32, "rows", "f32 parts 128x128", 4, 388, 1736, 268, 349),
+    (torch.float32, "rows", "f32 parts 256x128", 5, 2382, 388, 292, 2382), (torch.float32, "rows", "f32 parts 256x128", 16, 512, 1024, 1024, 512),
+    (torch.float32, "tn", "f32 64x64", 4, 240, 16, 136, 192), (torch.float32, "tn", "f32 64x64 four stages", 4, 266, 16, 144, 239),
+    (torch.float32, "tn", "f32 128x128", 5, 255, 2472, 196, 204), (torch.float32, "tn", "f32 parts 64x64", 8, 247, 392, 260, 247),
+    (torch.float32, "tn", "f32 parts 128x128", 4, 225, 264, 1732, 180), (torch.float32, "tn", "f32 parts 128x128", 8, 200, 652, 332, 160),
+    (torch.float32, "tn", "f32 parts 256x128", 8, 227, 1468, 388, 227), (torch.float32, "tn", "f32 parts 256x128", 4, 203, 3404, 332, 203)]
+
+
+@pytest.mark.parametrize("dtype,form,kernel,B,cap,n,k,hint", IN_KERNEL)
+def test_expert_gemm_in_every_kernel(dtype, form, kernel, B, cap, n, k, hint):
+    from planmoe_amd import ops
+    print("case", dtype, form, kernel, B, cap, n, k, hint, flush=True)
+    relu = dtype == torch.bfloat16 or "parts" not in kernel          # (a relu keeps the fp32 matrix cores' order of sums)
+    if form == "tn":
+        assert ops.expert_gemm_kernel("tn", dtype, B, k, n, cap, counted=True, rows_hint=hint) == kernel
+    else:
+        assert ops.expert_gemm_kernel("nn", dtype, B, cap, n, k, relu=relu, counted=True, rows_hint=hint) == kernel
+        assert ops.expert_gemm_kernel("nt", dtype, B, cap, n, k, counted=True, rows_hint=hint) == kernel
+    g = torch.Generator(device=DEV).manual_seed(cap + n + k)
+    edges = [cap, 0, 1, hint, 129, 256, 65, 127, 63, 257, 192, 160, 193, 161, 64, 128]
+    if form == "rows" and "quarters" in kernel:
+        edges = [hint] * 4 + [0, 1, 129, 257]       # (a round of 256 tiles, and a quarter of one)
+    rows = [min(cap, edges[e]) for e in range(B)]
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g).to(dtype)
+    live, a = torch.tensor([rows], dtype=torch.int32, device=DEV), rand(B, cap, k)
+    for e, r in enumerate(rows):
+        a[e, r:] = float("nan")
+    kw = dict(live=live, rows_hint=hint)
+    if form == "tn":
+        dy = rand(B, cap, n)
+        for e, r in enumerate(rows):
+            dy[e, r:] = float("nan")
+        got = ops.expert_gemm("tn", a, dy, **kw)
+        torch.cuda.synchronize()
+        for e, r in enumerate(rows):
+            x, d = a[e, :r].double().t().contiguous(), dy[e, :r].double()
+            ref = x @ d
+            assert bool(((got[e].double() - ref).abs() <= _bound(ref, x.abs() @ d.abs(), cap, dtype)).all()), (e, r)
+        return
+    w, bias, h = rand(B, k, n), rand(B, n), rand(B, cap, n).clamp(min=0)
+    wt = w.transpose(1, 2).contiguous()
+    nn = torch.full((B, cap, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    ops.expert_gemm("nn", a, w, bias, relu=relu, out=nn, **kw)
+    ops.expert_gemm("nt", a, wt, out=nt, **kw)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, out=masked, **kw)
+    torch.cuda.synchronize()
+    for e, r in enumerate(rows):
+        x, y = a[e, :r].double(), w[e].double()
+        ref, mag = x @ y, x.abs() @ y.abs()
+        tol, biased = _bound(ref, mag, k, dtype), ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - (biased.clamp(min=0) if relu else biased)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all()), (e, r)
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all()), (e, r)
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all()), (e, r)
+        for out in (nn, nt, masked):
+            assert bool((out[e, r:] == 7.0).all()), (e, r)
+        stored = masked[e, :r].double()          # the sums are of what was stored
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), (e, r)

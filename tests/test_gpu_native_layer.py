@@ -572,3 +572,12 @@ def test_reentrant_checkpoint_gives_the_gradients_of_the_plain_pass_in_fp32():
     torch.cuda.synchronize()
     for name in want:
         assert torch.equal(want[name], got[name]), name
+
+
+def test_native_layer_equals_its_steps_in_the_largest_parts():
+    """fp32 rows that are a tile of 256 x 128 in three parts a value, with the codec whose steps show a last bit."""
+    from planmoe_amd import ops
+    assert ops.expert_gemm_kernel("nt", torch.float32, 16, 512, 1024, 1024, counted=True, rows_hint=512) == "f32 parts 256x128"
+    args = ("zfp", torch.float32, 4096, 1024, 1024, 16, 2, 1.0)
+    for train in (False, True):
+        _compare(_run(True, *args, train), _run(False, *args, train), 1e-3)
