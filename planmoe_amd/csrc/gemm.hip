@@ -728,7 +728,7 @@ GemmKernel gemm_pick(int form, bool contiguous, int m, int n, int k, int batches
 
 bool gemm_contiguous(int form, int m, int n, int k, int lda, int ldb, int ldc, int64_t sa, int64_t sb, int64_t sc)
 {
-    return lda == k && ldb == (form == 1 ? k : n) && ldc == n && sb == (int64_t)n * k && sa == (int64_t)m * k && sc == (int64_t)m * n;
+    return lda == (form == 2 ? m : k) && ldb == (form == 1 ? k : n) && ldc == n && sb == (int64_t)n * k && sa == (int64_t)m * k && sc == (int64_t)m * n;
 }
 
 GemmSlots gemm_slots(GemmKernel kernel)

@@ -608,7 +608,8 @@ IN_KERNEL = [
     (torch.bfloat16, "rows", "192x256", 5, 2722, 520, 200, 2722), (torch.bfloat16, "rows", "192x256", 8, 2765, 280, 144, 2765),
     (torch.bfloat16, "rows", "256x256", 8, 429, 2608, 200, 429), (torch.bfloat16, "rows", "256x256", 8, 1551, 792, 136, 1551),
     (torch.bfloat16, "rows", "256x256 and quarters", 8, 1755, 2528, 1264, 1755), (torch.bfloat16, "rows", "256x256 and quarters", 8, 2013, 2160, 1584, 2013),
-    (torch.bfloat16, "tn", "128x128", 4, 203, 16, 136, 182), (torch.bfloat16, "tn", "128x128", 4, 260, 264, 1144, 234),
+    (torch.bfloat16, "tn", "128x128 alone", 4, 203, 16, 136, 182), (torch.bfloat16, "tn", "128x128 alone", 4, 260, 264, 1144, 234),
+    (torch.bfloat16, "tn", "128x128", 8, 202, 136, 1544, 202), (torch.bfloat16, "tn", "128x128", 8, 267, 144, 1552, 240),
     (torch.bfloat16, "tn", "256x256", 8, 201, 2072, 392, 160), (torch.bfloat16, "tn", "256x256", 8, 270, 2712, 264, 216),
     (torch.bfloat16, "tn", "256x256 and quarters", 4, 1098, 2784, 1512, 1098), (torch.bfloat16, "tn", "256x256 and quarters", 4, 1288, 2480, 1576, 1288),
     (torch.float32, "rows", "f32 waves", 4, 9, 16, 168, 8), (torch.float32, "rows", "f32 64x64", 4, 37, 16, 164, 37),
