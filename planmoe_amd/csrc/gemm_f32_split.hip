@@ -2,9 +2,13 @@
 //
 // An fp32 value is the sum of three bf16 values: h = bf16(x), m = bf16(x - h), l = x - h - m, each difference exact.  A product of
 // two such sums is nine products of bf16 values, each exact in fp32; six of them (hh, hm, mh, hl, mm, lh) hold everything down
-// to 2^-26 of the product, less than the rounding of an fp32 product, and are summed in fp32.  Six products at 16 times the
-// rate of v_mfma_f32_32x32x2_f32, and a rounding of the sum for every 16 / 6 k instead of every k: against 64 bits the relative error
-// (2-norm) of N(0, 1) operands is 3.4e-7 at k = 512 and 1.00e-6 at 4096 where the fp32 matrix cores give 4.1e-7 and 1.15e-6.
+// to 2^-26 of the product, less than the rounding of an fp32 product, and are summed in fp32, at 16 times the rate of v_mfma_f32_32x32x2_f32.
+// hh has a sum of its own and the five small products another, 2^-8 of it: a matrix core rounds a sum at every instruction, and downwards. All six
+// on one sum are six such roundings for 16 k: 0.85 of the fp32 matrix cores' error for N(0, 1) operands, but 1.15 behind a relu, whose zeros
+// those add without a rounding, and 1.7 in the column sums of a result, where what is rounded downwards adds up (1 - 3 % of the time for two).
+// Against 64 bits, relative 2-norm, fp32 matrix cores and here, k = 512, 1024, 4096: N(0, 1) 4.1e-7, 5.7e-7, 1.15e-6 and 1.3e-7, 1.9e-7, 4.0e-7;
+// one operand behind a relu 2.9e-7, 4.1e-7, 8.1e-7 and 1.0e-7, 1.4e-7, 3.2e-7; both positive 3.5e-7, 4.9e-7, 9.9e-7 and 1.3e-7, 1.8e-7, 3.5e-7;
+// column sums of 512 rows at k = 1024 5.8e-7 and 2.0e-7.
 //
 // Eight waves (four in the small tile).  Values come from memory into registers a k-tile of 32 ahead, are split there and go into
 // LDS as three planes, either operand with k running fastest whichever way it is stored; two stages, one barrier a k-tile.
@@ -12,8 +16,9 @@
 // k-tile (13 vector instructions a pair of values, 24 values a lane at 256 x 128: 1250 of 3070 clocks of matrix core), beside
 // those of the second it reads the first fragments of the next k-tile.
 //
-// What bounds it: the clock under the matrix cores at 256 x 128 (2 x 4096 x 4096 x 4096: 1260 us = 218 TFLOP/s, 1308 of bf16 products,
-// what gemm_bf16_kernel reaches; 2005 us on the fp32 matrix cores, 137), issuing the splits at 64 x 64.
+// What bounds it: the clock under the matrix cores at 256 x 128 (2 x 4096 x 4096 x 4096: 1317 us = 209 TFLOP/s, 1252 of bf16 products,
+// near what gemm_bf16_kernel reaches; 2000 us on the fp32 matrix cores, 137), issuing the splits at 64 x 64.  The two sums fill the registers there
+// (251 - 256 of 256, nothing spilt).
 #include "gemm_f32_core.hpp"
 
 namespace pm {
@@ -133,13 +138,13 @@ __global__ __launch_bounds__((SplitShape<WM, WN, FM, FN>::NT), 2) void gemm_f32_
         }
     };
 
-    f32x16 acc[FM][FN];
+    f32x16 acc[FM][FN], low[FM][FN];             // the sums of hh, and of all the others
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = low[i][j][q] = 0.f;
     // ---- fragments: lane = row l % 32, k-chunk l / 32 of the step's 16
     const int fr = lane & 31, fc = lane >> 5;
     uint32_t ro[2];
@@ -155,7 +160,8 @@ __global__ __launch_bounds__((SplitShape<WM, WN, FM, FN>::NT), 2) void gemm_f32_
     auto multiply = [&](int s, int x) {
         constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
         const int t = x / (FM * FN), i = x / FN % FM, j = x % FN;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[s][PB[t]][j], fa[s][PA[t]][i], acc[i][j], 0, 0, 0);
+        f32x16 &to = t == 5 ? acc[i][j] : low[i][j];
+        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[s][PB[t]][j], fa[s][PA[t]][i], to, 0, 0, 0);
     };
 
     constexpr int PAIRS = 4 * (UNITS_A + UNITS_B);
@@ -221,6 +227,7 @@ __global__ __launch_bounds__((SplitShape<WM, WN, FM, FN>::NT), 2) void gemm_f32_
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
+                acc[i][j][q] += low[i][j][q];
                 odd = __builtin_fmaf(acc[i][j][q], 0.f, odd);
                 acc[i][j][q] *= SP_UNSCALE;
             }

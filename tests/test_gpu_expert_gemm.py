@@ -673,3 +673,27 @@ def test_expert_gemm_in_every_kernel(dtype, form, kernel, B, cap, n, k, hint):
             assert bool((out[e, r:] == 7.0).all()), (e, r)
         stored = masked[e, :r].double()          # the sums are of what was stored
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), (e, r)
+
+
+# The parts are no less precise than the fp32 matrix cores (which serve the same product under a relu: where a result is positive, that is the product):
+# the results and their sums over the rows, in which what is rounded one way adds up, for operands of both signs, behind a relu, and positive
+@pytest.mark.parametrize("form,kernel,B,m,n,k", [("nn", "f32 parts 256x128", 16, 512, 1024, 1024), ("nt", "f32 parts 256x128", 16, 512, 1024, 1024),
+                                                 ("tn", "f32 parts 256x128", 16, 1024, 1024, 512), ("nn", "f32 parts 128x128", 8, 1024, 512, 512),
+                                                 ("tn", "f32 parts 128x128", 8, 332, 652, 200), ("nt", "f32 parts 64x64", 8, 750, 1536, 768),
+                                                 ("nn", "f32 parts 64x64", 8, 300, 2048, 2048), ("nn", "f32 parts 256x128", 2, 4096, 2048, 4096)])
+@pytest.mark.parametrize("operands", ["normal", "relu", "positive"])
+def test_expert_gemm_fp32_in_parts_is_no_less_precise(form, kernel, B, m, n, k, operands):
+    from planmoe_amd import ops
+    print("case", form, kernel, B, m, n, k, operands, flush=True)
+    assert ops.expert_gemm_kernel(form, torch.float32, B, m, n, k) == kernel
+    assert "parts" not in ops.expert_gemm_kernel(form, torch.float32, B, m, n, k, relu=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = torch.randn(*((B, k, m) if form == "tn" else (B, m, k)), device=DEV, generator=g)
+    b = torch.randn(*((B, n, k) if form == "nt" else (B, k, n)), device=DEV, generator=g)
+    a, b = (a.clamp(min=0), b) if operands == "relu" else (a.abs(), b.abs()) if operands == "positive" else (a, b)
+    got, fp32, ref = ops.expert_gemm(form, a, b).double(), ops.expert_gemm(form, a, b, relu=True).double(), _fp64(form, a, b)[0]
+    torch.cuda.synchronize()
+    there = (fp32 > 0) & (got > 0) & (ref > 0)
+    parts, whole = (got - ref) * there, (fp32 - ref) * there
+    assert float(parts.norm()) <= float(whole.norm())
+    assert float(parts.sum(1).norm()) <= float(whole.sum(1).norm())
