@@ -169,7 +169,9 @@ __global__ __launch_bounds__(256) void slots_sum_kernel(const SumJobs all)
 #pragma unroll
         for (int q = 0; q < 8; ++q) v[q] = from[(int64_t)min(i + q, used - 1) * p.cols];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) s += i + q < used ? v[q] : 0.f;
+        for (int q = 0; q < 8; ++q) v[q] = i + q < used ? v[q] : 0.f;
+        // (in pairs: up to eight slots are one wave's, and one after the other are seven roundings of the whole sum)
+        s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
     s_sum[wave][lane] = s;
     __syncthreads();

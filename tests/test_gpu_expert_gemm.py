@@ -697,3 +697,20 @@ def test_expert_gemm_fp32_in_parts_is_no_less_precise(form, kernel, B, m, n, k, 
     parts, whole = (got - ref) * there, (fp32 - ref) * there
     assert float(parts.norm()) <= float(whole.norm())
     assert float(parts.sum(1).norm()) <= float(whole.sum(1).norm())
+
+
+@pytest.mark.parametrize("shares", [2, 5, 8, 9, 16])
+def test_sums_of_shares_are_added_in_pairs(shares):
+    """Shares of 32 rows: the first one's sum is 1, those of the others half a unit of its last place, which one after the other are lost.  Eight in
+    pairs have three roundings, a wave's sums up to four more."""
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    a = torch.zeros(1, 32 * shares, 64, device=DEV)
+    a[0, ::32] = 2.0 ** -24
+    a[0, 0] = 1.0
+    out = torch.empty(1, 64, device=DEV)
+    ws = torch.empty(lib.planmoe_rows_colsum_workspace_bytes(1, 32 * shares, 64), dtype=torch.uint8, device=DEV)
+    check(lib.planmoe_rows_colsum(ops._ptr(a), ops._dt(a, "t"), 1, 32 * shares, 64, None, 1, 1, ops._ptr(out), ops._ptr(ws), ws.numel(), ops._stream(a)))
+    torch.cuda.synchronize()
+    want = 1.0 + (shares - 1) * 2.0 ** -24
+    assert bool(((out.double() - want).abs() <= 2.0 ** -23).all()), (out[0, 0].item() - 1.0) * 2 ** 24
