@@ -318,7 +318,7 @@ __global__ __launch_bounds__(GEMM_WG, S::WAVES_PER_SIMD) void gemm_bf16_kernel(c
 
     // one phase: quadrant (qa, qb); read half (ro, rh) of stage rs; ask for half (lo, lh) into stage lst
     // (the second operand first in the MFMA: a lane then holds four consecutive columns of one row)
-    // (r0, r1: which of the half's fragments, x0 of half (xo, xh) of the stage on top)
+    // (from fragment r0 of that half on; on top the first xn fragments of stage xs's half (0, 1))
 #define PM_PHASE(P, qa, qb, rs, ro, rh, r0, xs, xn, lst, lo, lh, cur)                                                \
     do {                                                                                                             \
         constexpr int share_ = S::I(qa), n_ = 4 * share_ * J, half_ = n_ / 2;                                         \

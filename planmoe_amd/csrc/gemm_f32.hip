@@ -72,7 +72,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     // (chunks of a k-fast row past the end of K are asked for out of range)
     auto past = [&](int i) -> uint32_t { return (int)(((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 4) >= k_tail ? 0x80000000u : 0u; };
     const uint32_t past0 = past(0), past1 = past(1);
-    // (with four stages k-tiles past the end are asked for as well, out of range: the count of what is on its way stays the same)
     // Four stages: the operands from their corner on are within reach of an offset (the caller sees to it), so a load is an offset away from
     // one descriptor and fits under a product; past the end the last k-tile is asked for again, so that the count of what is on its way stays
     // the same, and never used.

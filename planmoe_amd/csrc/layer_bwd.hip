@@ -181,8 +181,8 @@ __global__ __launch_bounds__(256) void slots_sum_kernel(const SumJobs all)
 // out[t] = round(sum_j codec(rows[slot_j])) + sum_e g[t][e] * wg[e]: the combine of the gradient rows and the gate's share of the
 // gradient of x in one pass (their own launches read and write out once more).  A wave per TOKENS tokens; up to EP experts, whose
 // weights come from the caches.  The roundings are those of planmoe_layer_combine and planmoe_gate_dx_accumulate.  Bound by the rows' bytes and, for
-// wide rows, by the weights out of L2.  bf16, top-2, 8 experts, both launches and this one: 16384 x 1024 39 and 23 us (int8 43 and 32), x 4096
-// 129 and 86 (int8 129 and 120), 1024 x 1024 17 and 5.
+// wide rows, by the weights out of L2.  bf16, top-2, 8 experts, both launches and this one: 16384 x 1024 44 and 24 us (int8 46 and 34), x 4096
+// 141 and 100 (int8 145 and 127), 1024 x 1024 17 and 7.5.
 template <int DT, int CACHE, bool INT8, int EP, int TOKENS>
 __global__ __launch_bounds__(256) void layer_dx_kernel(
     const void *__restrict__ rows, const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride, int top_k,

@@ -346,7 +346,9 @@ SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locat
     while (shift < (pairs <= 8192 ? 8 : pairs <= 32768 ? 7 : 6) && (slots >> (shift + 1)) >= 16) ++shift;
     // The walk is as long as the pairs are many, and the rows that hide it are as long as they are wide: the line is fitted between these.
     // Forward pass of the routing API, flags and walk, us: 8000 pairs of 512 bytes 46.8 and 45.1, 6000 of 2048 35.6 and 31.9; 13200 of 512 50.9 and 52.9, 32768 of 1024 41.6 and 47.9, 32768 of 2048 54.5 and 58.4, 20000 of
-    // 4096 66.8 and 68.8, 32768 of 4096 99.6 and 100.0; with the backward pass 13200 of 4096 130.3 and 125.1, 16384 of 8192 193.8 and 186.4.
+    // 4096 66.8 and 68.8, 32768 of 4096 99.6 and 100.0; the dispatch alone, rows of 2048 bytes, 12300 pairs 12.6 and 12.5, 16384 14.0 and 13.5, 20480 15.9 and
+    // 17.8, 32768 22.8 and 25.3.  A combine's backward pass, whose rows hide more, gains from the walk beyond the line (2048 bytes, 16384 pairs 21.1 and 17.6, 32768
+    // 40.8 and 35.6); the line serves both.  With the backward pass 13200 of 4096 130.3 and 125.1, 16384 of 8192 193.8 and 186.4.
     if (pairs <= std::min<int64_t>(8192 + 2 * row_bytes, SLOT_FILL_PAIRS) && (slots >> shift) < SLOT_FILL_BITS) return SlotFill{nullptr, 1 << shift, shift};
     uint32_t *flags = (uint32_t *)workspace;
     slot_flags_clear<<<(slots + 255) / 256, 256, 0, st>>>(flags, slots);

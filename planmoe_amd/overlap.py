@@ -216,12 +216,6 @@ def native_call(layer, gate, x, degree, reserve_dims, capacity):
     return (codec, *weights)
 
 
-def native_codec(layer, gate, x, degree, reserve_dims, capacity):
-    """The codec number of native_call, or None."""
-    call = native_call(layer, gate, x, degree, reserve_dims, capacity)
-    return None if call is None else call[0]
-
-
 class _GaveUp:
     """The give-up flag of a one-launch forward on its way to the host without stalling the stream:
     an asynchronous copy into pinned memory and an event behind it.  Asked at the end of the

@@ -74,7 +74,7 @@ def test_native_layer_leaves_hooks_and_frozen_parameters_to_autograd():
     seen = []
     handle = layer.experts.register_forward_hook(lambda *a: seen.append(1))
     y = layer(x)
-    assert seen and overlap.native_codec(layer, layer.gates[0], x, 1, 1, 4) is None
+    assert seen and overlap.native_call(layer, layer.gates[0], x, 1, 1, 4) is None
     handle.remove()
     z = layer(x)
     assert len(seen) == 1 and torch.allclose(y.float(), z.float(), rtol=2e-2, atol=1e-2)
