@@ -64,7 +64,9 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
 }
 // relu of two bf16 values.  As int16 what becomes zero is at most -128 (minus infinity), a NaN with its sign set above that: like
-// every other NaN it stays.
+// every other NaN it stays.  (Every NaN that comes out of the bf16 matrix cores has its sign set, so a signed maximum with zero, one instruction for these
+// three, makes zeros of all of them.  us of a product under a relu, with that maximum and here: 8 x 4096, 4096 -> 4096 889 and 898, 1024 -> 4096 272 and 279;
+// a maximum in fp32 that keeps NaN, two instructions a pair, 897 and 277, but 39.2 in place of 38.7 in 8 x 500, 2048 -> 2048.)
 __device__ __forceinline__ uint32_t relu_bf16x2(uint32_t v)
 {
     typedef short s16x2 __attribute__((ext_vector_type(2)));
