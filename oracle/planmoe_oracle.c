@@ -204,7 +204,7 @@ ORC_API void orc_route_topk(const void *scores, int is_bf16, int samples, int ex
             for (int e = 0; e < experts; ++e) {
                 if (taken[e]) continue;
                 float v = load_score(scores, is_bf16, (int64_t)t * experts + e);
-                if (best < 0 || v > bv) { best = e; bv = v; }
+                if (best < 0 || v > bv || (v != v && bv == bv)) { best = e; bv = v; }       /* NaN first, as torch.topk */
             }
             taken[best] = 1;
             indices[(int64_t)j * samples + t] = best;

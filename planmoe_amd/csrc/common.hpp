@@ -74,6 +74,11 @@ __device__ __forceinline__ uint32_t relu_bf16x2(uint32_t v)
     return v & ~__builtin_bit_cast(uint32_t, drop);
 }
 
+// The order of scores in an arg-max: NaN before every number, as torch.topk has it.  A total order: lanes that compare in different sequences agree,
+// and k of k or more experts are always found.  (With a plain > every lane of a token whose scores are all NaN keeps its own expert.)
+__device__ __forceinline__ bool score_above(float a, float b) { return a > b || (a != a && b == b); }
+__device__ __forceinline__ bool score_same(float a, float b) { return a == b || (a != a && b != b); }
+
 __device__ __forceinline__ float f16_to_f32(uint32_t bits)
 {
     union { uint16_t u; _Float16 h; } c; c.u = (uint16_t)bits; return (float)c.h;

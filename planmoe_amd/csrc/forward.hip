@@ -311,10 +311,10 @@ __global__ __launch_bounds__(256) void gate_route_kernel(
 #pragma unroll
             for (int q = 0; q < EPL; ++q) {
                 const bool free_ = !((taken >> q) & 1u) && q * LPT + el < experts;
-                if (free_ && (bi == 0x7fffffff || sc[q] > bv)) { bv = sc[q]; bi = q * LPT + el; }
+                if (free_ && (bi == 0x7fffffff || score_above(sc[q], bv))) { bv = sc[q]; bi = q * LPT + el; }
             }
             auto merge = [&](float ov, int oi) {
-                const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
+                const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || score_above(ov, bv) || (oi < bi && score_same(ov, bv)));
                 if (better) { bv = ov; bi = oi; }
             };
             if constexpr (LPT >= 2) merge(row_partner<1>(bv), row_partner<1>(bi));

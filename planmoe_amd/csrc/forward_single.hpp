@@ -280,7 +280,7 @@ __global__ __launch_bounds__(FS_THREADS) void forward_single_kernel(
                 float bv = -INFINITY; int bi = 0x7fffffff;
                 if (!taken && el < experts) { bv = sc; bi = el; }
                 auto merge = [&](float ov, int oi) {
-                    const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
+                    const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || score_above(ov, bv) || (oi < bi && score_same(ov, bv)));
                     if (better) { bv = ov; bi = oi; }
                 };
                 merge(row_partner<1>(bv), row_partner<1>(bi));

@@ -187,7 +187,7 @@ __global__ __launch_bounds__(TILE) void route_tile_kernel(
 #pragma unroll
                 for (int e = 0; e < CAP; ++e) {
                     const bool free_ = !((taken_lo >> e) & 1u) && e < experts;
-                    if (free_ && (best < 0 || s[e] > bv)) { best = e; bv = s[e]; }
+                    if (free_ && (best < 0 || score_above(s[e], bv))) { best = e; bv = s[e]; }
                 }
                 taken_lo |= (uint64_t)1 << best;
             } else {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(TILE) void route_tile_kernel(
                     bool free_ = true;
                     for (int p = 0; p < j; ++p) free_ = free_ && (indices[(int64_t)p * stride + t] != e);
                     const float v = row.score(e);
-                    if (free_ && (best < 0 || v > bv)) { best = e; bv = v; }
+                    if (free_ && (best < 0 || score_above(v, bv))) { best = e; bv = v; }
                 }
             }
             indices[(int64_t)j * stride + t] = best;

@@ -581,3 +581,37 @@ def test_native_layer_equals_its_steps_in_the_largest_parts():
     args = ("zfp", torch.float32, 4096, 1024, 1024, 16, 2, 1.0)
     for train in (False, True):
         _compare(_run(True, *args, train), _run(False, *args, train), 1e-3)
+
+
+# A token that is not finite is lost, the others are not: same outputs as beside a row of zeros, the same gradients of theirs.  Up to 32 tokens (the gate sends the
+# rows itself) and more; as one node and by its steps
+@pytest.mark.parametrize("codec,dtype", [("no", torch.bfloat16), ("int8", torch.bfloat16), ("no", torch.float32), ("int8", torch.float32), ("zfp", torch.float32),
+                                         ("lz", torch.float32)])
+@pytest.mark.parametrize("T,E,k", [(4, 8, 2), (32, 4, 3), (33, 8, 2), (300, 16, 2)])
+@pytest.mark.parametrize("native", [True, False])
+def test_layer_with_tokens_that_are_not_finite(native, T, E, k, codec, dtype):
+    from planmoe_amd import overlap
+    print("case", native, T, E, k, codec, dtype, flush=True)
+    overlap.NATIVE_LAYER = native
+    try:
+        layer = _layer(dtype, codec, M=128, H=256, E=E)
+        g = torch.Generator(device=DEV).manual_seed(T)
+        x, gy = (torch.randn(T, 128, device=DEV, generator=g).to(dtype) for _ in range(2))
+        lost = torch.arange(T, device=DEV) % 4 == 1
+        outs = []
+        for value in (0.0, float("nan"), float("inf")):
+            v = x.clone()
+            v[lost] = 0.0
+            v[lost, 3] = value
+            v.requires_grad_(True)
+            y = layer(v, top_k=k)
+            y.backward(gy)
+            torch.cuda.synchronize()
+            outs.append((y.detach(), v.grad))
+            layer.zero_grad(set_to_none=True)
+    finally:
+        overlap.NATIVE_LAYER = True
+    for y, dx in outs[1:]:
+        assert bool(y[lost].isnan().any())
+        if codec in ("no", "int8"):               # (a block of the other codecs holds rows of several tokens)
+            assert torch.equal(y[~lost], outs[0][0][~lost]) and bool(y[~lost].isfinite().all()) and torch.equal(dx[~lost], outs[0][1][~lost])

@@ -275,3 +275,66 @@ def test_batch_prioritized_routing(T, E, k):
         kept, dropped = top[m & (got[0] < cap)], top[m & (got[0] >= cap)]
         if len(kept) and len(dropped):
             assert kept.min() >= dropped.max()
+
+
+# Scores that are NaN, all of a token's or some: before every number, the lower expert first, and every choice another expert, whatever the lanes that
+# share the token compare first.  Lanes for 8, 16, 32 and 64 experts, and the kernels beyond those; one group of tokens and several
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,k", [(2, 2), (7, 3), (8, 2), (8, 8), (16, 4), (24, 5), (33, 2), (64, 4), (100, 3)])
+@pytest.mark.parametrize("T", [1, 33, 300])
+def test_nan_scores(T, E, k, dtype):
+    from planmoe_amd import ops
+    print("case", T, E, k, dtype, flush=True)
+    scores = tie_free_scores(T, E, k, seed=T + E).to(dtype)
+    g = torch.Generator().manual_seed(T * E)
+    for t in range(T):
+        if t % 4 == 0:
+            scores[t] = float("nan")
+        elif t % 4 < 3:
+            scores[t, torch.randperm(E, generator=g)[: 1 + t % 3]] = float("nan")
+    if T > 1:
+        scores[1, E - 1] = float("inf")
+    r = ops.route_topk(scores.to(DEV), k, want_counts=True)
+    torch.cuda.synchronize()
+    idx, loc, gates, counts = oracle.route_topk(to_np(scores), k, True)
+    assert np.array_equal(r["indices"].cpu().numpy(), idx)
+    assert np.array_equal(r["locations"].cpu().numpy(), loc)
+    assert np.array_equal(r["counts"].cpu().numpy(), counts)
+    finite = torch.isfinite(scores).all(1)
+    got, want = r["gates"].cpu()[:, finite], (torch.from_numpy(gates) if dtype == torch.float32 else torch.from_numpy(gates.view(np.int16)).view(torch.bfloat16))[:, finite]
+    assert torch.equal(got, want)
+
+
+# Tokens that are not finite: scores of NaN throughout, the choices and slots of a token whose scores are all the same (a row of zeros), the
+# other tokens' rows as they are beside such a row.  Every launch that routes: gate and routing, with dispatch, in one launch
+@pytest.mark.parametrize("dtype,fp32_gate", [(torch.float32, True), (torch.bfloat16, True), (torch.bfloat16, False), (torch.float16, True)])
+@pytest.mark.parametrize("E,k", [(2, 2), (8, 1), (8, 2), (9, 4), (16, 3), (33, 2), (64, 4), (8, 6)])
+@pytest.mark.parametrize("T", [1, 5, 32, 33, 300])
+def test_tokens_that_are_not_finite(T, E, k, dtype, fp32_gate):
+    from planmoe_amd import ops
+    print("case", T, E, k, dtype, fp32_gate, flush=True)
+    M, cap = 256, ops.capacity(T, E, k, 1.25, 4)
+    g = torch.Generator().manual_seed(T + E)
+    zero, wg = torch.randn(T, M, generator=g).to(dtype).to(DEV), (torch.randn(E, M, generator=g) * M ** -0.5).to(dtype).to(DEV)
+    lost = torch.arange(T) % 3 == 0
+    zero[lost] = 0
+    x = zero.clone()
+    for t in lost.nonzero()[:, 0].tolist():
+        x[t, 5] = (float("nan"), float("inf"), -float("inf"))[t // 3 % 3]
+    runs = [lambda v: ops.gate_route(v, wg, k, fp32_gate=fp32_gate, want_counts=True),
+            lambda v: ops.forward_plain(v, wg, k, cap, fp32_gate=fp32_gate, want_counts=True),
+            lambda v: ops.forward_int8(v, wg, k, cap, fp32_gate=fp32_gate, want_counts=True)]
+    if ops.forward_int8_single_serves(x, wg, k, fp32_gate):
+        runs.append(lambda v: ops.forward_int8_single(v, wg, k, cap, fp32_gate=fp32_gate, want_counts=True))
+    for number, run in enumerate(runs):
+        got, want = run(x), run(zero)
+        torch.cuda.synchronize()
+        for name in ("indices", "locations", "counts"):
+            assert torch.equal(got[name], want[name]), (number, name)
+        assert bool((got["indices"] >= 0).all()) and bool((got["indices"] < E).all())
+        assert bool(got["gates"][:, lost.to(DEV)].isnan().all()) and torch.equal(got["gates"][:, ~lost.to(DEV)], want["gates"][:, ~lost.to(DEV)])
+        slots = (got["indices"].long() * cap + got["locations"].long())[:, ~lost.to(DEV)]
+        slots = slots[got["locations"][:, ~lost.to(DEV)] < cap]
+        for name in ("dispatched", "codes", "bias", "scale"):
+            if name in got:
+                assert torch.equal(got[name][slots], want[name][slots]), (number, name)

@@ -161,3 +161,14 @@ def test_route_locations_ignores_out_of_range_indices():
     idx = np.array([[0, 5, -1, 1, 0, 7]], np.int32)
     loc, counts = oracle.route_locations(idx, 2)
     assert loc.tolist() == [[0, -1, -1, 0, 1, -1]] and counts.tolist() == [[2, 1]]
+
+
+def test_nan_comes_first_as_in_torch_topk():
+    scores = torch.rand(40, 9, generator=torch.Generator().manual_seed(2))
+    for t in range(40):
+        scores[t, t % 9] = float("nan")
+        scores[t, (t + 2) % 9] = float("inf")
+    idx = oracle.route_topk(scores.numpy(), 3, False)[0]
+    assert np.array_equal(idx, torch.topk(scores, 3, dim=1).indices.t().numpy())
+    scores[:] = float("nan")
+    assert np.array_equal(oracle.route_topk(scores.numpy(), 3, False)[0], np.repeat(np.arange(3, dtype=np.int32)[:, None], 40, 1))
