@@ -72,7 +72,8 @@ size_t planmoe_route_workspace_bytes(int samples, int experts, int top_k);
  *              first, in fp32, rounded to `dtype`).
  * logit_bias   optional fp32 [experts] added to the logits before the softmax (NULL = none;
  *              only with input_is_logits).
- * indices      out int32 k planes   expert id of the j-th largest score (ties: lower id)
+ * indices      out int32 k planes   expert id of the j-th largest score (ties: lower id; NaN
+ *              before every number, as torch.topk)
  * locations    out int32 k planes   slot inside that expert; all first choices of an expert
  *              come first in token order, then all second choices, ...
  * gates        out `dtype` k planes score of the chosen expert, divided by

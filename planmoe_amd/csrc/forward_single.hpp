@@ -272,7 +272,9 @@ __global__ __launch_bounds__(FS_THREADS) void forward_single_kernel(
                 for (int off = LPT; off < WAVE; off <<= 1) c += __shfl_xor(c, off, WAVE);
                 if (tk == 0) s_me[p * FS_WAVES + w][el] = c;
             }
-            // k-fold arg-max, the lower expert id wins among equal scores
+            // k-fold arg-max, the lower expert id wins among equal scores (which a token's are that are NaN: all are or none is)
+            const bool lost = sum != sum;
+            sc = lost ? 0.f : sc;
             bool taken = false;
             float denom = 0.f, my_gate = 0.f;
             int my_idx = 0;
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(FS_THREADS) void forward_single_kernel(
                 float bv = -INFINITY; int bi = 0x7fffffff;
                 if (!taken && el < experts) { bv = sc; bi = el; }
                 auto merge = [&](float ov, int oi) {
-                    const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || score_above(ov, bv) || (oi < bi && score_same(ov, bv)));
+                    const bool better = oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
                     if (better) { bv = ov; bi = oi; }
                 };
                 merge(row_partner<1>(bv), row_partner<1>(bi));
@@ -288,6 +290,7 @@ __global__ __launch_bounds__(FS_THREADS) void forward_single_kernel(
                 merge(row_partner<4>(bv), row_partner<4>(bi));
                 if constexpr (LPT >= 16) merge(row_partner<8>(bv), row_partner<8>(bi));
                 if (bi == el) taken = true;
+                if (lost) bv = NAN;
                 denom = (j == 0) ? bv : S::round(denom + bv);
                 if (el == 0 && valid) s_best[j][tok] = (uint8_t)bi;
                 if (el == j) { my_gate = bv; my_idx = bi; }
