@@ -14,8 +14,8 @@ def _bound(ref, mag, terms, dtype):
     return (terms + 2) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0) + 1e-30
 
 
-# tiles are 256 x 256 or 128 x 128, k-tiles 64 (bf16) or 32 (fp32) and taken in pairs: sizes one piece either side of
-# those, one k-tile, an odd number of them, more than eight tile columns, one row
+# sizes one piece either side of 256 and 128 and of k-tiles of 64 (bf16) and 32 (fp32), one k-tile, an odd number of them, more than eight tile columns, one row
+# (products as small as these go to the kernels for few rows and few tiles: test_expert_gemm_in_every_kernel has the others)
 SHAPES = [(1, 1, 8, 8), (2, 127, 136, 64), (3, 129, 264, 72), (2, 255, 520, 136), (2, 257, 128, 200), (1, 300, 2312, 64), (5, 40, 256, 320)]
 
 
@@ -135,11 +135,16 @@ def test_expert_gemm_with_few_rows(m, n, k):
 
 # 256 work-groups that stay take 256 x 256 tiles, four to a tile row here; what is left for a last round is a launch of
 # quarters up to 128 tiles.  Rows in use that leave 0, 4 (one row of the last tile), 128 and 132 tiles, and fewer than one round
+# (with k = 4096 and 8192 rows a batch expected; with k = 512 what is picked for the rows that are there)
 @pytest.mark.parametrize("rows", [16384, 16385, 24576, 24577, 300])
-def test_expert_gemm_last_round(rows):
+@pytest.mark.parametrize("k", [512, 4096])
+def test_expert_gemm_last_round(rows, k):
     from planmoe_amd import ops
-    print("case", rows, flush=True)
-    cap, n, k, dtype = 24832, 1024, 512, torch.bfloat16
+    print("case", rows, k, flush=True)
+    cap, n, dtype = 24832, 1024, torch.bfloat16
+    hint = 8192 if k == 4096 else rows // 2
+    kernels = [ops.expert_gemm_kernel(form, dtype, 2, cap // 2, n, k, counted=True, rows_hint=hint) for form in ("nn", "nt")]
+    assert kernels == ["256x256 and quarters" if k == 4096 else {150: "128x128 alone", 8192: "160x256", 12288: "256x256"}[rows // 2]] * 2
     g = torch.Generator(device=DEV).manual_seed(rows)
     a, w = torch.randn(2, cap // 2, k, device=DEV, generator=g).to(dtype), torch.randn(2, k, n, device=DEV, generator=g).to(dtype)
     first = 0 if rows < 512 else rows // 512 * 256          # (the odd row is the second batch's)
@@ -147,8 +152,8 @@ def test_expert_gemm_last_round(rows):
     h = torch.randn(2, cap // 2, n, device=DEV, generator=g).clamp(min=0).to(dtype)
     out = torch.full((2, cap // 2, n), 7.0, dtype=dtype, device=DEV)
     masked = out.clone()
-    ops.expert_gemm("nn", a, w, live=live, out=out, rows_hint=rows // 2)
-    _, db = ops.expert_gemm_relu_bwd(a, w.transpose(1, 2).contiguous(), h, live=live, out=masked, rows_hint=rows // 2)
+    ops.expert_gemm("nn", a, w, live=live, out=out, rows_hint=hint)
+    _, db = ops.expert_gemm_relu_bwd(a, w.transpose(1, 2).contiguous(), h, live=live, out=masked, rows_hint=hint)
     torch.cuda.synchronize()
     for e in range(2):
         r = int(live[0, e])
@@ -186,14 +191,18 @@ def test_gate_weight_gradient_and_row_sums(T, M, E, dtype):
     assert bool(((out[0].double().cpu() - rows.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * rows.abs().sum(0) + half * rows.sum(0).abs() + 1e-30).all())
 
 
-# Rows that end on a tile of 256 or 128 and just behind one, batches of less than a tile and of no rows: a quarter of the last
-# round that has no rows stores nothing; several tiles for a work-group; the last one has no row counts
-@pytest.mark.parametrize("n,k,hint,counts", [(1024, 512, 4096, [4096, 4097, 4160, 4161]), (1024, 512, 4096, [4224, 4225, 128, 1]),
-                                             (2048, 2048, 500, [512, 513, 576, 577, 500, 64, 1, 0]), (1024, 1024, 0, [4160] * 4)])
-def test_expert_gemm_rows_around_a_tile(n, k, hint, counts):
+# Rows that end on a tile of 256 or 128 and just behind one, batches of less than a tile and of no rows, in tiles of 160 rows and in those of 256 with
+# their last round in quarters: a quarter that has no rows stores nothing; several tiles for a work-group; some have no row counts
+@pytest.mark.parametrize("kernel,n,k,hint,counts", [
+    ("160x256", 1024, 512, 4096, [4096, 4097, 4160, 4161]), ("160x256", 1024, 512, 4096, [4224, 4225, 128, 1]),
+    ("160x256", 2048, 2048, 500, [512, 513, 576, 577, 500, 64, 1, 0]), ("160x256", 1024, 1024, 0, [4160] * 4),
+    ("256x256 and quarters", 1024, 4096, 4096, [4096, 4097, 4160, 4161, 4095, 4224, 4225, 4100]),
+    ("256x256 and quarters", 1024, 4096, 4096, [4352, 4353, 4225, 1, 4224, 128, 4097, 0]), ("256x256 and quarters", 1016, 4104, 0, [4160] * 8)])
+def test_expert_gemm_rows_around_a_tile(kernel, n, k, hint, counts):
     from planmoe_amd import ops
-    print("case", n, k, counts, flush=True)
+    print("case", kernel, n, k, counts, flush=True)
     B, cap, dtype = len(counts), max(counts) + (64 if hint else 0), torch.bfloat16
+    assert all(ops.expert_gemm_kernel(form, dtype, B, cap, n, k, counted=bool(hint), rows_hint=hint) == kernel for form in ("nn", "nt"))
     g = torch.Generator(device=DEV).manual_seed(sum(counts))
     a, w = torch.randn(B, cap, k, device=DEV, generator=g).to(dtype), torch.randn(B, k, n, device=DEV, generator=g).to(dtype)
     bias, h = torch.randn(B, n, device=DEV, generator=g).to(dtype), torch.randn(B, cap, n, device=DEV, generator=g).clamp(min=0).to(dtype)
@@ -317,8 +326,8 @@ def _fp64(form, a, b):
     return a @ b, a.abs() @ b.abs()
 
 
-# fp32 on the bf16 matrix cores in three parts a value: one shape for each tile (64, 128 and 256 rows; 256 compute units pick
-# them by the number of tiles), rows, columns and reductions that are no multiple of anything but 4, one past a tile and one
+# fp32 on the bf16 matrix cores in three parts a value (six of the shapes; four run in 64 x 64 tiles with four k-tiles in LDS, and the same holds of them; every tile and form
+# in parts is in test_expert_gemm_in_every_kernel): rows, columns and reductions that are no multiple of anything but 4, one past a tile and one
 # k-tile's edge.  A k-slow operand's rows need not be a multiple of 4.
 @pytest.mark.parametrize("form,B,m,n,k", [("nn", 8, 301, 712, 712), ("nt", 8, 299, 708, 700), ("tn", 8, 712, 716, 301), ("nn", 4, 999, 1004, 300),
                                           ("nt", 4, 1000, 1004, 292), ("tn", 4, 516, 2048, 1001), ("nn", 4, 2041, 1004, 260), ("nt", 16, 257, 1036, 1028),
@@ -381,7 +390,7 @@ def test_expert_gemm_fp32_in_parts_takes_the_rows_in_use_only(B, cap, n, k, hint
         assert bool(((dw[e].double() - x.t() @ d).abs() <= _bound(d, x.abs().t() @ d.abs(), cap, torch.float32)).all()), e
 
 
-# bf16 tiles of 128, 160 and 192 rows by 256 columns: rows that end on such a tile, one before and one behind, of one row and none;
+# bf16 tiles of 128, 160 and 192 rows by 256 columns (and, in the first and the seventh, of 128 x 128): rows that end on such a tile, one before and one behind, of one row and none;
 # columns around a multiple of 256, reductions of an odd and an even number of k-tiles with 8 k in the last one, of two k-tiles; no row counts
 @pytest.mark.parametrize("cap,n,k,hint,counts", [(400, 2040, 136, 290, [256, 257, 255, 0, 1, 128, 384, 400]), (160, 4000, 520, 120, [128, 129, 127, 160, 1, 0, 64, 33]),
                                                  (620, 2056, 200, 490, [480, 481, 479, 620, 0, 1, 160, 161]), (620, 2048, 520, 500, [320, 640, 159, 97, 96, 95, 64, 65]),
