@@ -15,109 +15,24 @@
 namespace pm {
 
 constexpr int TRIP_NW = 4;                       // words of a block
-constexpr int TRIP_WRITER = TRIP_NW * 256, TRIP_READER = BitReader<TRIP_NW>::STRIDE * 256;
+constexpr int TRIP_READER = BitReader<TRIP_NW>::STRIDE * 256;
 
-// f as the decoder gives it back, same bits.  writer, reader: LDS for blocks with an infinity.
-__device__ __forceinline__ void zfp_trip16(float (&f)[16], uint32_t *writer, uint32_t *reader)
+// f as the decoder gives it back, same bits; KEEP: the block's stream as well.  reader: LDS for blocks with an infinity, whose
+// exponent does not fit its bits and spills into the first plane's: such a block is coded and decoded.
+template <bool KEEP>
+__device__ __forceinline__ void zfp_trip16(float (&f)[16], uint32_t *s, const uint16_t *tab, uint32_t *reader)
 {
-    float m = 0.f;
+    if (code16<TRIP_NW, KEEP, true>(f, s, tab) != 255) return;
+    uint32_t w[TRIP_NW];
+    if constexpr (KEEP) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(f[i]));
-    if (!(m > 0.f)) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) f[i] = 0.f;
-        return;
+        for (int i = 0; i < TRIP_NW; ++i) w[i] = s[i];
+    } else {
+        code16<TRIP_NW, true, false>(f, w, group_codes.entry);
     }
-    const int field = (int)((__float_as_uint(m) >> 23) & 0xffu), emax = field - 126;
-    if (field == 255) {
-        // an exponent that does not fit its 8 bits spills into the first plane's: such a block is coded and decoded
-        BitWriter<TRIP_NW> bw;
-        encode_block<16, TRIP_NW>(f, bw, writer, group_codes.entry);
-        uint32_t w[TRIP_NW];
-        bw.words(writer, w);
-        BitReader<TRIP_NW> br;
-        br.init(reader, w);
-        decode_block<16, TRIP_NW>(br, f, gt16_table.step);
-        return;
-    }
-    const int se = 30 - emax;
-    const float s = se > 127 ? INFINITY : __uint_as_float((uint32_t)(se + 127) << 23);
-    int32_t q[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float v = f[i] * s;
-        q[i] = fabsf(v) < 2147483648.0f ? (int32_t)v : (int32_t)0x80000000;
-    }
-#pragma unroll
-    for (int y = 0; y < 4; ++y) fwd_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) fwd_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
-    uint32_t u[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) u[i] = to_negabinary(q[perm2(i)]);
-
-    // the plane that does not fit whole, what is left of the budget there (below zero from then on) and the values significant by then
-    int bits = 32 * TRIP_NW - 9, nsig = 0, cut = -1, cut_bits = 0, cut_nsig = 0;
-    uint32_t cut_plane = 0u;
-    auto plane = [&](uint32_t x, int k) __attribute__((always_inline)) {
-        // nsig bits as they are; then the group tests: a bit for every value up to the highest one, a test bit in front of the
-        // first and behind every one, where the last of them ends the plane (the block's last value: its one is implied, no test behind it)
-        const uint32_t r = x >> nsig;
-        const int next = nsig + 32 - __clz((int)r);
-        const int need = next + __builtin_popcount(r) + (next < 16 ? 1 : nsig < 16 ? -1 : 0);
-        const int left = bits - need;
-        const bool here = left < 0 && bits >= 0;
-        cut = here ? k : cut;
-        cut_plane = here ? x : cut_plane;
-        cut_bits = here ? bits : cut_bits;
-        cut_nsig = here ? nsig : cut_nsig;
-        bits = left < 0 ? -1 : left;
-        nsig = next;
-    };
-    uint32_t w[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w[j] = (u[2 * j] >> 16) | (u[2 * j + 1] & 0xffff0000u);
-    transpose16(w);
-#pragma unroll
-    for (int k = 15; k >= 0; --k)
-        if (__builtin_amdgcn_ballot_w64(bits >= 0) != 0) plane((k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu, k + 16);
-    if (__builtin_amdgcn_ballot_w64(bits >= 0) != 0) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = (u[2 * j] & 0xffffu) | (u[2 * j + 1] << 16);
-        transpose16(w);
-#pragma unroll
-        for (int k = 15; k >= 0; --k)
-            if (__builtin_amdgcn_ballot_w64(bits >= 0) != 0) plane((k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu, k);
-    }
-    if (cut >= 0) {
-        // what the decoder makes of the bits that are there: a run of zeros that the budget cuts short ends in a one
-        int n = cut_nsig, b = cut_bits;
-        const int mm = min(n, b);
-        uint32_t x = cut_plane & ((1u << mm) - 1u);
-        b -= mm;
-        while (n < 16 && b > 0) {
-            --b;
-            const uint32_t r = cut_plane >> n;
-            if (r == 0u) break;
-            const int z = __builtin_ctz(r), lim = min(15 - n, b);
-            b -= z < lim ? z + 1 : lim;
-            n += min(z, lim);
-            x |= 1u << n;
-            ++n;
-        }
-        const uint32_t whole = ~((2u << cut) - 1u);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) u[i] = (u[i] & whole) | (((x >> i) & 1u) << cut);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) q[perm2(i)] = from_negabinary(u[i]);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) inv_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
-#pragma unroll
-    for (int y = 0; y < 4; ++y) inv_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
-    const float back = ldexpf(1.0f, emax - 30);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) f[i] = (float)q[i] * back;
+    BitReader<TRIP_NW> br;
+    br.init(reader, w);
+    decode_block<16, TRIP_NW>(br, f, gt16_table.step);
 }
 
 // slot -> token that fills it, its gate (with `gates`) and its plane; a choice without a slot: its gate gradient is zero.
@@ -169,7 +84,7 @@ __global__ __launch_bounds__(256) void layer_zfp_dispatch_kernel(const float *__
                                                                  const int32_t *__restrict__ counts, int planes, int samples, int model_dim,
                                                                  int experts, int capacity, int64_t blocks, float *__restrict__ rows)
 {
-    __shared__ uint32_t lds[TRIP_WRITER + TRIP_READER];
+    __shared__ uint32_t lds[TRIP_READER];
     const TripBlock at(model_dim / 4, blocks, counts, planes, experts, capacity);
     if (at.live <= 0) return;
     const int4 tok = *reinterpret_cast<const int4 *>(src + 4 * at.by);
@@ -184,7 +99,7 @@ __global__ __launch_bounds__(256) void layer_zfp_dispatch_kernel(const float *__
         f[4 * j + 2] = live ? v.z : 0.f;
         f[4 * j + 3] = live ? v.w : 0.f;
     }
-    zfp_trip16(f, lds, lds + TRIP_WRITER);
+    zfp_trip16<false>(f, nullptr, nullptr, lds);
     float *p = rows + 4 * at.by * model_dim + 4 * at.bx;
 #pragma unroll
     for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);
@@ -195,8 +110,8 @@ template <bool KEEP>
 __global__ __launch_bounds__(256) void layer_zfp_rows_kernel(float *__restrict__ rows, const int32_t *__restrict__ counts, int planes,
                                                              int model_dim, int experts, int capacity, int64_t blocks, uint32_t *__restrict__ stream)
 {
-    __shared__ uint32_t lds[TRIP_WRITER + TRIP_READER];
-    __shared__ uint32_t tab[KEEP ? 512 : 1];
+    __shared__ uint32_t lds[TRIP_READER];
+    __shared__ __align__(4) uint16_t tab[KEEP ? 512 : 2];
     const TripBlock at(model_dim / 4, blocks, counts, planes, experts, capacity);
     if constexpr (KEEP) {
         if (!__syncthreads_or(at.live > 0)) return;
@@ -210,14 +125,9 @@ __global__ __launch_bounds__(256) void layer_zfp_rows_kernel(float *__restrict__
         const float4 v = *reinterpret_cast<const float4 *>(p + (int64_t)j * model_dim);
         f[4 * j] = v.x; f[4 * j + 1] = v.y; f[4 * j + 2] = v.z; f[4 * j + 3] = v.w;
     }
-    if constexpr (KEEP) {
-        BitWriter<TRIP_NW> bw;
-        encode_block<16, TRIP_NW>(f, bw, lds, tab);
-        uint32_t w[TRIP_NW];
-        bw.words(lds, w);
-        store_words<TRIP_NW>(stream + (at.by * (model_dim / 4) + at.bx) * TRIP_NW, w);
-    }
-    zfp_trip16(f, lds, lds + TRIP_WRITER);
+    uint32_t w[TRIP_NW];
+    zfp_trip16<KEEP>(f, w, tab, lds);
+    if constexpr (KEEP) store_words<TRIP_NW>(stream + (at.by * (model_dim / 4) + at.bx) * TRIP_NW, w);
 #pragma unroll
     for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);
 }
@@ -231,7 +141,7 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
                                                                     int planes, int64_t stride, int samples, int model_dim, int experts,
                                                                     int capacity, float *__restrict__ grad_rows, float *__restrict__ grad_gates)
 {
-    __shared__ uint32_t lds[TRIP_WRITER + TRIP_READER];
+    __shared__ uint32_t lds[TRIP_READER];
     __shared__ float s_part[4][4];
     __shared__ uint16_t tab[GT16_ENTRIES];
     const int64_t by = blockIdx.x;
@@ -251,7 +161,7 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
         uint32_t w[TRIP_NW];
         load_words<TRIP_NW>(stream + (by * nbx + bx) * TRIP_NW, w);
         BitReader<TRIP_NW> br;
-        br.init(lds + TRIP_WRITER, w);
+        br.init(lds, w);
         float f[16];
         decode_block<16, TRIP_NW>(br, f, tab);
 #pragma unroll
@@ -264,7 +174,7 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
             f[4 * j + 2] = j < live ? g[j] * v[j].z : 0.f;
             f[4 * j + 3] = j < live ? g[j] * v[j].w : 0.f;
         }
-        zfp_trip16(f, lds, lds + TRIP_WRITER);
+        zfp_trip16<false>(f, nullptr, nullptr, lds);
         float *p = grad_rows + 4 * by * model_dim + 4 * bx;
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);

@@ -109,38 +109,57 @@ __device__ __forceinline__ void fwd_lift(int32_t &x, int32_t &y, int32_t &z, int
     w += y >> 1; y -= w >> 1;
 }
 
+// (zfp's y += w; w = 2 w - y; and the like are a sum and a difference)
 __device__ __forceinline__ void inv_lift(int32_t &x, int32_t &y, int32_t &z, int32_t &w)
 {
     y += w >> 1; w -= y >> 1;
-    y += w; w = (int32_t)((uint32_t)w << 1); w -= y;
-    z += x; x = (int32_t)((uint32_t)x << 1); x -= z;
-    y += z; z = (int32_t)((uint32_t)z << 1); z -= y;
-    w += x; x = (int32_t)((uint32_t)x << 1); x -= w;
+    auto turn = [](int32_t &a, int32_t &b) { const int32_t t = a; a += b; b -= t; };
+    turn(y, w);
+    turn(z, x);
+    turn(y, z);
+    turn(w, x);
 }
 
 __device__ __forceinline__ uint32_t to_negabinary(int32_t v) { return ((uint32_t)v + 0xaaaaaaaau) ^ 0xaaaaaaaau; }
 __device__ __forceinline__ int32_t from_negabinary(uint32_t v) { return (int32_t)((v ^ 0xaaaaaaaau) - 0xaaaaaaaau); }
+// the largest of three, NaN if one of them is (one instruction, v_maximum3_f32)
+__device__ __forceinline__ float max3_nan(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 
-// 16 x 16 bit matrix transpose.  w[j] holds row 2j in its low and row 2j+1 in its high half;
-// afterwards bit i of row k is what bit k of row i was.  Used to turn the upper halves of the 16
-// coefficients of a 2-D block into their 16 upper bit planes (and back) in about 100
-// instructions instead of 32 per plane.
-__device__ __forceinline__ void transpose16(uint32_t (&w)[8])
+// 16 x 16 bit matrix transpose of 16-bit rows, two rows to a word: word j has rows j and j + 8, and afterwards
+// columns j and j + 8.  Four exchanges of blocks; the one of 8 x 8 blocks stays inside a word and is a byte permute, done
+// where the words are put together (planes_of16) or taken apart (values_of16).  The others are a shift and a bit select a word.
+__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) { return (m & a) | (~m & b); }
+__device__ __forceinline__ void transpose16_rest(uint32_t (&w)[8])
 {
     auto swap_blocks = [](uint32_t &a, uint32_t &b, int s, uint32_t m) {
-        const uint32_t t = ((a >> s) ^ b) & m;
-        b ^= t; a ^= t << s;
+        const uint32_t t = a >> s;
+        a = bit_select(m, a, b << s);
+        b = bit_select(m, t, b);
     };
 #pragma unroll
-    for (int j = 0; j < 4; ++j) swap_blocks(w[j], w[j + 4], 8, 0x00ff00ffu);
-    swap_blocks(w[0], w[2], 4, 0x0f0f0f0fu); swap_blocks(w[1], w[3], 4, 0x0f0f0f0fu);
-    swap_blocks(w[4], w[6], 4, 0x0f0f0f0fu); swap_blocks(w[5], w[7], 4, 0x0f0f0f0fu);
+    for (int j = 0; j < 4; ++j) swap_blocks(w[j], w[j + 4], 4, 0x0f0f0f0fu);
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) swap_blocks(w[j], w[j + 1], 2, 0x33333333u);
+    for (int j = 0; j < 8; ++j) if (!(j & 2)) swap_blocks(w[j], w[j + 2], 2, 0x33333333u);
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) swap_blocks(w[j], w[j + 1], 1, 0x55555555u);
+}
+// The bit planes of 16 negabinary values v + 0xaa.. ^ 0xaa.. (u holds v + 0xaa..): their upper 16 or their lower 16 bits, plane k
+// (of 16) in half k / 8 of word k % 8; bit i of a plane is value i's.
+template <bool HIGH>
+__device__ __forceinline__ void planes_of16(const uint32_t (&u)[16], uint32_t (&w)[8])
+{
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_perm(u[j + 8], u[j], HIGH ? 0x07030602u : 0x05010400u) ^ 0xaaaaaaaau;
+    transpose16_rest(w);
+}
+// and back: upper 16 bits of the values, zeros below
+__device__ __forceinline__ void values_of16(uint32_t (&w)[8], uint32_t (&u)[16])
+{
+    transpose16_rest(w);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const uint32_t t = ((w[j] >> 15) ^ w[j]) & 0x0000aaaau;
-        w[j] ^= t | (t << 15);
+        u[j] = __builtin_amdgcn_perm(0u, w[j], 0x02000c0cu);
+        u[j + 8] = __builtin_amdgcn_perm(0u, w[j], 0x03010c0cu);
     }
 }
 
@@ -155,11 +174,11 @@ __device__ constexpr int perm2(int i)
 // For the not yet significant part r of a plane (bit p = value nsig + p) zfp emits, segment by
 // segment, a test bit '1', the zeros below the next one bit and that one bit; i.e. the bits of r
 // up to its highest one with a '1' put in front of bit 0 and of every bit that follows a one.
-// The table holds that expansion for 8 bits of r at a time: entry [prev][byte] = code in the low
-// 16 bits, its length (8 + prev + ones among the low 7 bits) above.  What follows the highest
+// The table holds that expansion for 8 bits of r at a time: entry prev | byte << 1, up to 16 bits, of length
+// 8 + prev + ones among the low 7 bits.  What follows the highest
 // one (a single '0' test bit, or nothing at the block end) and the implicit last one are a
-// matter of the total length, see encode_block.
-__host__ __device__ constexpr uint32_t group_code_entry(int prev, int byte)
+// matter of the total length, see code16.
+__host__ __device__ constexpr uint16_t group_code_entry(int prev, int byte)
 {
     uint32_t code = 0; int len = 0;
     for (int p = 0; p < 8; ++p) {
@@ -168,118 +187,217 @@ __host__ __device__ constexpr uint32_t group_code_entry(int prev, int byte)
         code |= (uint32_t)bit << len; ++len;
         prev = bit;
     }
-    return code | ((uint32_t)len << 16);
+    return (uint16_t)code;
 }
-// all 256 threads of the work-group; tab has 512 entries
-__device__ __forceinline__ void group_code_table(uint32_t *tab)
-{
-    tab[threadIdx.x] = group_code_entry(0, threadIdx.x);
-    tab[256 + threadIdx.x] = group_code_entry(1, threadIdx.x);
-    __syncthreads();
-}
-// the same where no work-group fills one
 struct GroupCodeTable {
-    uint32_t entry[512];
+    uint16_t entry[512];
     constexpr GroupCodeTable() : entry()
     {
-        for (int i = 0; i < 512; ++i) entry[i] = group_code_entry(i >> 8, i & 255);
+        for (int i = 0; i < 512; ++i) entry[i] = group_code_entry(i & 1, i >> 1);
     }
 };
 __constant__ const GroupCodeTable group_codes = GroupCodeTable();
-__device__ __forceinline__ uint32_t low_bits(int n) { return (uint32_t)(((uint64_t)1 << n) - 1u); }   // n in 0..32
+// all 256 threads of the work-group; tab has 512 entries
+__device__ __forceinline__ void group_code_table(uint16_t *tab)
+{
+    reinterpret_cast<uint32_t *>(tab)[threadIdx.x] = reinterpret_cast<const uint32_t *>(group_codes.entry)[threadIdx.x];
+    __syncthreads();
+}
 
-// N = values per block (4 or 16).  f is consumed; the block's maxbits = 32*NW bits land in bw.
-template <int N, int NW>
-__device__ __forceinline__ void encode_block(const float *f, BitWriter<NW> &bw, uint32_t *lds,
-                                             const uint32_t *tab)
+// A block of 4 values; the block's maxbits = 32*NW bits land in bw.
+template <int NW>
+__device__ __forceinline__ void encode_block4(const float (&f)[4], BitWriter<NW> &bw, uint32_t *lds, const uint16_t *tab)
 {
     bw.init(lds);
-    float m = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(f[i]));
+    const float m = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
     if (!(m > 0.f)) return;                       // all-zero block: '0' flag and zero padding
     // frexp exponent clamped at 1 - 127, i.e. exponent field - 126 (a denormal maximum reads 0)
-    const int field = (int)((__float_as_uint(m) >> 23) & 0xffu);
-    const int emax = field - 126;
+    const int emax = (int)((__float_as_uint(m) >> 23) & 0xffu) - 126;
     bw.put(2u * (uint32_t)(emax + 127) + 1u, 9);
 
     // block-floating-point cast: q = (int32)(f * 2^(30 - emax)), x86 conversion on overflow
     const int se = 30 - emax;
     const float s = se > 127 ? INFINITY : __uint_as_float((uint32_t)(se + 127) << 23);
-    int32_t q[N];
+    int32_t q[4];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
+    for (int i = 0; i < 4; ++i) {
         const float v = f[i] * s;
         // -2^31 itself converts to INT_MIN either way
         q[i] = fabsf(v) < 2147483648.0f ? (int32_t)v : (int32_t)0x80000000;
     }
-    uint32_t u[N];
-    if constexpr (N == 4) {
-        fwd_lift(q[0], q[1], q[2], q[3]);
+    fwd_lift(q[0], q[1], q[2], q[3]);
+    uint32_t u[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[i] = to_negabinary(q[i]);
-    } else {
-#pragma unroll
-        for (int y = 0; y < 4; ++y) fwd_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) fwd_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) u[i] = to_negabinary(q[perm2(i)]);
-    }
+    for (int i = 0; i < 4; ++i) u[i] = to_negabinary(q[i]);
 
     // embedded coding: bit planes from the top, group-tested, until the budget is spent
     int bits = 32 * NW - 9;
     int nsig = 0;
-    auto code_plane = [&](uint32_t x) __attribute__((always_inline)) {
+    for (int k = 31; k >= 0 && bits > 0; --k) {
+        uint32_t x = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x |= ((u[i] >> k) & 1u) << i;
         const int mm = min(nsig, bits);
         bits -= mm;
         bw.put(x & ((1u << mm) - 1u), mm);
-        if (nsig < N && bits > 0) {
+        if (nsig < 4 && bits > 0) {
             const uint32_t r = x >> mm;                   // mm == nsig here
             // r == 0 runs through the same formulas: top = -1, no code bits, length 1 (the '0')
             const int top = 31 - __clz((int)r), ones = __builtin_popcount(r);
-            const uint32_t e0 = tab[256 + (r & 0xffu)];
-            uint32_t code = e0 & 0xffffu;
-            if constexpr (N > 8) {
-                const uint32_t e1 = tab[((r >> 7) & 1u) * 256 + (r >> 8)];
-                code |= (e1 & 0xffffu) << (e0 >> 16);
-            }
             // cut after the highest one bit (not emitted when it is the block's last value),
             // then one more '0' test bit unless the block ends there
-            const int last = nsig + top == N - 1;
-            const int lt = top + 1 + ones - last;
-            const int len = lt + (nsig + top + 1 < N ? 1 : 0);
-            const int emit = min(len, bits);
-            code &= low_bits(min(lt, emit));
-            bw.put(code, emit);
+            const int lt = top + 1 + ones - (nsig + top == 3);
+            const int emit = min(lt + (nsig + top < 3 ? 1 : 0), bits);
+            bw.put(tab[r * 2u + 1u] & ((1u << min(lt, emit)) - 1u), emit);
             bits -= emit;
             nsig += top + 1;
         }
-    };
-    if constexpr (N == 16) {
-        // planes 31..16 by one bit transpose of the coefficients' upper halves
-        uint32_t w[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = (u[2 * j] >> 16) | (u[2 * j + 1] & 0xffff0000u);
-        transpose16(w);
-#pragma unroll
-        for (int k = 15; k >= 0; --k)
-            if (bits > 0) code_plane((k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu);
-        for (int k = 15; k >= 0 && bits > 0; --k) {
-            uint32_t x = 0;
-#pragma unroll
-            for (int i = 0; i < N; ++i) x |= ((u[i] >> k) & 1u) << i;
-            code_plane(x);
-        }
-    } else {
-        for (int k = 31; k >= 0 && bits > 0; --k) {
-            uint32_t x = 0;
-#pragma unroll
-            for (int i = 0; i < N; ++i) x |= ((u[i] >> k) & 1u) << i;
-            code_plane(x);
-        }
     }
     bw.finish();
+}
+
+// A block of 4 x 4 values, in registers throughout.
+//   PACK  s: its maxbits = 32 * NW bits.  They come in from above: what a plane adds (31 bits at most: the verbatim bits of nsig
+//         values, then at most two for each of the others less one) shifts the whole down by its length, a funnel shift a
+//         word, and what the budget cuts off never comes in.  (Bits gathered in a register pair and stored to LDS word by word took two
+//         such appends a plane and a dozen instructions each.)
+//   TRIP  f: what the decoder makes of those bits, where the block's largest value is finite (else f is as it was; see zfp_trip16).
+//         It has the planes that fit whole, and the cut one as far as its bits are there.
+// Returns the exponent field of the largest magnitude.
+template <int NW, bool PACK, bool TRIP>
+__device__ __forceinline__ int code16(float (&f)[16], uint32_t *s, const uint16_t *tab)
+{
+    if constexpr (PACK) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) s[i] = 0u;
+    }
+    // the largest magnitude, NaN if there is one
+    float m = fabsf(f[0]);
+#pragma unroll
+    for (int i = 1; i < 15; i += 2) m = max3_nan(m, fabsf(f[i]), fabsf(f[i + 1]));
+    m = max3_nan(m, fabsf(f[15]), fabsf(f[15]));
+    int field = (int)(__float_as_uint(m) >> 23);
+    int32_t q[16];
+    // block-floating-point cast: q = (int32)(f * 2^(30 - emax)), x86 conversion on overflow: only where the factor itself is
+    // none (next to the denormals) or a value is not finite is there any
+    if (__builtin_amdgcn_ballot_w64((uint32_t)(field - 29) > 225u && m != 0.f) != 0) {
+        m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(f[i]));
+        field = (int)(__float_as_uint(m) >> 23);
+        const int se = 156 - field;
+        const float scale = se > 127 ? INFINITY : __uint_as_float((uint32_t)(se + 127) << 23);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float v = f[i] * scale;
+            // -2^31 itself converts to INT_MIN either way
+            q[i] = !(m > 0.f) ? 0 : fabsf(v) < 2147483648.0f ? (int32_t)v : (int32_t)0x80000000;
+        }
+    } else {
+        const float scale = __uint_as_float((uint32_t)(283 - max(field, 29)) << 23);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) q[i] = (int32_t)(f[i] * scale);
+    }
+    // all zero: a '0' and zeros behind it
+    const bool live = m > 0.f;
+    int bits = live ? 32 * NW - 9 : 0, nsig = 0;
+    // the flag and the exponent, frexp's clamped at 1 - 127, i.e. the field - 126 (a denormal maximum reads 0) and biased by 127.  That of an
+    // infinity has a bit too many, which gets into the first plane's.
+    const uint32_t head = live ? 2u * (uint32_t)(field + 1) + 1u : 0u;
+    if constexpr (PACK) s[NW - 1] = head << 23;
+
+#pragma unroll
+    for (int y = 0; y < 4; ++y) fwd_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) fwd_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
+    uint32_t u[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) u[i] = (uint32_t)q[perm2(i)] + 0xaaaaaaaau;
+
+    // Embedded coding: bit planes from the top, group-tested, until the budget is spent.  A plane is nsig bits as they are; then the
+    // group tests: a bit for every value up to the highest one, a test bit in front of the first and behind every one, where the last
+    // of them ends the plane (the block's last value: its one is implied, no test behind it).
+    bool whole = live;                            // (TRIP) every plane so far fits
+    int cut = -1;                                 // the plane that does not, from which on bits and nsig stay
+    uint32_t cut_plane = 0u;
+    auto plane = [&](uint32_t x, int k) __attribute__((always_inline)) {
+        const uint32_t r = x >> nsig, r1 = 2u * r + 1u;       // (a one in front: the table's index, and never zero)
+        const int top = 31 - __builtin_clz(r1), next = nsig + top, ones = __builtin_popcount(r);
+        const int coded = top + ones, need = max(coded + (next < 16 ? 1 : -1), 0);
+        const int total = nsig + need;
+        if constexpr (PACK) {
+            const uint32_t lo = tab[r1 & 0x1ffu], hi = tab[r1 >> 8];
+            const uint32_t code = lo | (hi << (9 + __builtin_popcount(r & 0x7fu)));
+            uint32_t v = __builtin_amdgcn_ubfe(x, 0u, nsig) | (__builtin_amdgcn_ubfe(code, 0u, min(coded, need)) << nsig);
+            if (k == 31) v |= head >> 9;
+            const int emit = TRIP && !whole ? 0 : min(total, bits);
+#pragma unroll
+            for (int i = 0; i < NW - 1; ++i) s[i] = __builtin_amdgcn_alignbit(s[i + 1], s[i], emit);
+            s[NW - 1] = __builtin_amdgcn_alignbit(v, s[NW - 1], emit);
+            if constexpr (!TRIP) { bits -= emit; nsig = next; }
+        }
+        if constexpr (TRIP) {
+            cut_plane = whole ? x : cut_plane;
+            cut = whole ? k : cut;
+            whole = whole && total <= bits;
+            bits = whole ? bits - total : bits;
+            nsig = whole ? next : nsig;
+        }
+    };
+    auto more = [&]() { return __builtin_amdgcn_ballot_w64(TRIP ? whole : bits > 0) != 0; };        // (a branch of the whole wave)
+    uint32_t w[8];
+    planes_of16<true>(u, w);
+#pragma unroll
+    for (int k = 15; k >= 0; --k) if (more()) plane(k < 8 ? w[k] & 0xffffu : w[k - 8] >> 16, k + 16);
+    if (more()) {
+        planes_of16<false>(u, w);
+#pragma unroll
+        for (int k = 15; k >= 0; --k) if (more()) plane(k < 8 ? w[k] & 0xffffu : w[k - 8] >> 16, k);
+    }
+    if constexpr (PACK) {
+        // (32 planes and bits to spare)
+        for (int left = TRIP && !whole ? 0 : bits; left > 0; left -= 31) {
+            const int n = min(left, 31);
+#pragma unroll
+            for (int i = 0; i < NW - 1; ++i) s[i] = __builtin_amdgcn_alignbit(s[i + 1], s[i], n);
+            s[NW - 1] >>= n;
+        }
+    }
+    if constexpr (TRIP) {
+        if (field == 255) return field;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) u[i] ^= 0xaaaaaaaau;
+        if (live && !whole) {
+            // what the decoder makes of the bits that are there: a run of zeros that the budget cuts short ends in a one
+            int n = nsig, b = bits;
+            const int mm = min(n, b);
+            uint32_t x = cut_plane & ((1u << mm) - 1u);
+            b -= mm;
+            while (n < 16 && b > 0) {
+                --b;
+                const uint32_t r = cut_plane >> n;
+                if (r == 0u) break;
+                const int z = __builtin_ctz(r), lim = min(15 - n, b);
+                b -= z < lim ? z + 1 : lim;
+                n += min(z, lim);
+                x |= 1u << n;
+                ++n;
+            }
+            const uint32_t above = ~((2u << cut) - 1u);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) u[i] = (u[i] & above) | (((x >> i) & 1u) << cut);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) q[perm2(i)] = from_negabinary(u[i]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) inv_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
+#pragma unroll
+        for (int y = 0; y < 4; ++y) inv_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
+        const float back = ldexpf(1.0f, field - 156);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) f[i] = (float)q[i] * back;
+    }
+    return field;
 }
 
 // ---- group tests of a 2-D block's bit plane, eight stream bits at a time
@@ -451,7 +569,7 @@ __device__ __forceinline__ void decode_block(BitReader<NW> &br, float *f, const 
                 uint32_t x;
                 const bool ok = fast_plane16(look, bits, nsig, x, tab);
                 br.skip(ok ? before - bits : 0);
-                w[k >> 1] |= ok ? x << (16 * (k & 1)) : 0u;
+                w[k & 7] |= ok ? x << (16 * (k >> 3)) : 0u;
                 last_k = ok ? last_k : k;
                 last_look = ok ? last_look : look;
                 last_bits = ok ? last_bits : before;
@@ -460,13 +578,11 @@ __device__ __forceinline__ void decode_block(BitReader<NW> &br, float *f, const 
             }
         }
         if (last_k >= 0) {
-            const uint32_t x = slow_plane16(last_look, last_bits, last_nsig) << (16 * (last_k & 1));
+            const uint32_t x = slow_plane16(last_look, last_bits, last_nsig) << (16 * (last_k >> 3));
 #pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] |= (last_k >> 1) == j ? x : 0u;
+            for (int j = 0; j < 8; ++j) w[j] |= (last_k & 7) == j ? x : 0u;
         }
-        transpose16(w);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { u[2 * j] = w[j] << 16; u[2 * j + 1] = w[j] & 0xffff0000u; }
+        values_of16(w, u);
         for (int k = 15; k >= 0 && bits > 0; --k) {
             const uint32_t x = read_plane();
 #pragma unroll

@@ -242,6 +242,36 @@ def test_zfp_2d_field_kinds_and_rates(rate):
         assert np.array_equal(dec.cpu().numpy().view(np.uint32), want.view(np.uint32)), name
 
 
+@pytest.mark.parametrize("nx", [4, 8, 12, 1016, 1020, 1024, 1028, 2052])
+@pytest.mark.parametrize("rate", [2, 8, 16])
+def test_zfp_2d_rows_of_blocks_and_values_that_are_not_finite(nx, rate):
+    """Rows of 1, 2, 3, 254 .. 257 and 513 blocks, so that a work-group's 256 blocks lie in many rows, in one and in two; blocks of zeros
+    alone, next to the denormals, with an infinity or a NaN, and with a few bits set (32 planes and budget to spare) in the same waves as
+    ordinary ones.  (What an infinity makes of its own block the oracle does not say: its exponent is none of zfp's.)"""
+    from planmoe_amd import ops
+    rng = np.random.default_rng(nx + rate)
+    ny = 4 * max(2, 2000 // nx + 3)
+    f = rng.standard_normal((ny, nx)).astype(np.float32)
+    b = f.reshape(ny // 4, 4, nx // 4, 4).transpose(0, 2, 1, 3).reshape(-1, 4, 4)
+    kinds = rng.integers(0, 10, len(b))
+    b[kinds == 0] = 0
+    b[kinds == 1] *= np.float32(1e-41)
+    b[kinds == 2] *= np.float32(2.0 ** -100)
+    b[kinds == 3, 1, 2] = np.inf
+    b[kinds == 4, 0, 3] = np.nan
+    b[kinds == 5] = np.nan
+    b[kinds == 6] = np.rint(b[kinds == 6] * 4)
+    b[kinds == 7, 2] = -np.inf
+    f = np.ascontiguousarray(b.reshape(ny // 4, nx // 4, 4, 4).transpose(0, 2, 1, 3).reshape(ny, nx))
+    st, n = oracle.zfp_compress(f, 2, float(rate)), len(b) * 2 * rate
+    got = ops.zfp_compress(torch.from_numpy(f).to(DEV), nx, ny, 2, float(rate))
+    ours = (kinds != 3) & (kinds != 7)
+    assert np.array_equal(got.cpu().numpy()[:n].reshape(len(b), -1)[ours], st[:n].reshape(len(b), -1)[ours])
+    dec = ops.zfp_decompress(got, nx, ny, 2, float(rate))
+    st = got.cpu().numpy()[:len(st)]
+    assert np.array_equal(raw(dec), oracle.zfp_decompress(st, ny, nx, 2, float(rate)).view(np.int32))
+
+
 @pytest.mark.parametrize("dims", [2, 1])
 def test_zfp_config5_full_size(dims):
     """[16, 8192, 1024] fp32 (65536 tokens x top-2 slots): whole stream against the oracle."""
