@@ -15,12 +15,11 @@
 namespace pm {
 
 constexpr int TRIP_NW = 4;                       // words of a block
-constexpr int TRIP_READER = BitReader<TRIP_NW>::STRIDE * 256;
 
-// f as the decoder gives it back, same bits; KEEP: the block's stream as well.  reader: LDS for blocks with an infinity, whose
-// exponent does not fit its bits and spills into the first plane's: such a block is coded and decoded.
+// f as the decoder gives it back, same bits; KEEP: the block's stream as well.  A block with an infinity, whose exponent does not fit its
+// bits and spills into the first plane's, is coded and decoded.
 template <bool KEEP>
-__device__ __forceinline__ void zfp_trip16(float (&f)[16], uint32_t *s, const uint16_t *tab, uint32_t *reader)
+__device__ __forceinline__ void zfp_trip16(float (&f)[16], uint32_t *s, const uint16_t *tab)
 {
     if (code16<TRIP_NW, KEEP, true>(f, s, tab) != 255) return;
     uint32_t w[TRIP_NW];
@@ -30,9 +29,7 @@ __device__ __forceinline__ void zfp_trip16(float (&f)[16], uint32_t *s, const ui
     } else {
         code16<TRIP_NW, true, false>(f, w, group_codes.entry);
     }
-    BitReader<TRIP_NW> br;
-    br.init(reader, w);
-    decode_block<16, TRIP_NW>(br, f, gt16_table.step);
+    decode16<TRIP_NW>(w, f, walk16_table.step);
 }
 
 // slot -> token that fills it, its gate (with `gates`) and its plane; a choice without a slot: its gate gradient is zero.
@@ -84,7 +81,6 @@ __global__ __launch_bounds__(256) void layer_zfp_dispatch_kernel(const float *__
                                                                  const int32_t *__restrict__ counts, int planes, int samples, int model_dim,
                                                                  int experts, int capacity, int64_t blocks, float *__restrict__ rows)
 {
-    __shared__ uint32_t lds[TRIP_READER];
     const TripBlock at(model_dim / 4, blocks, counts, planes, experts, capacity);
     if (at.live <= 0) return;
     const int4 tok = *reinterpret_cast<const int4 *>(src + 4 * at.by);
@@ -99,7 +95,7 @@ __global__ __launch_bounds__(256) void layer_zfp_dispatch_kernel(const float *__
         f[4 * j + 2] = live ? v.z : 0.f;
         f[4 * j + 3] = live ? v.w : 0.f;
     }
-    zfp_trip16<false>(f, nullptr, nullptr, lds);
+    zfp_trip16<false>(f, nullptr, nullptr);
     float *p = rows + 4 * at.by * model_dim + 4 * at.bx;
 #pragma unroll
     for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);
@@ -110,7 +106,6 @@ template <bool KEEP>
 __global__ __launch_bounds__(256) void layer_zfp_rows_kernel(float *__restrict__ rows, const int32_t *__restrict__ counts, int planes,
                                                              int model_dim, int experts, int capacity, int64_t blocks, uint32_t *__restrict__ stream)
 {
-    __shared__ uint32_t lds[TRIP_READER];
     __shared__ __align__(4) uint16_t tab[KEEP ? 512 : 2];
     const TripBlock at(model_dim / 4, blocks, counts, planes, experts, capacity);
     if constexpr (KEEP) {
@@ -126,7 +121,7 @@ __global__ __launch_bounds__(256) void layer_zfp_rows_kernel(float *__restrict__
         f[4 * j] = v.x; f[4 * j + 1] = v.y; f[4 * j + 2] = v.z; f[4 * j + 3] = v.w;
     }
     uint32_t w[TRIP_NW];
-    zfp_trip16<KEEP>(f, w, tab, lds);
+    zfp_trip16<KEEP>(f, w, tab);
     if constexpr (KEEP) store_words<TRIP_NW>(stream + (at.by * (model_dim / 4) + at.bx) * TRIP_NW, w);
 #pragma unroll
     for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);
@@ -141,13 +136,12 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
                                                                     int planes, int64_t stride, int samples, int model_dim, int experts,
                                                                     int capacity, float *__restrict__ grad_rows, float *__restrict__ grad_gates)
 {
-    __shared__ uint32_t lds[TRIP_READER];
     __shared__ float s_part[4][4];
-    __shared__ uint16_t tab[GT16_ENTRIES];
+    __shared__ __align__(16) uint16_t tab[WALK16_ENTRIES];
     const int64_t by = blockIdx.x;
     const int live = trip_rows_left(by, counts, planes, experts, capacity), nbx = model_dim / 4;
     if (live <= 0) return;                       // (the whole work-group)
-    gt16_load(tab);
+    walk16_load(tab);
     const int4 tok = *reinterpret_cast<const int4 *>(src + 4 * by);
     const float4 gv = *reinterpret_cast<const float4 *>(sgate + 4 * by);
     const uint32_t most = (uint32_t)samples - 1u;
@@ -160,10 +154,8 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
         for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float4 *>(grad + t[j] * model_dim + 4 * bx);
         uint32_t w[TRIP_NW];
         load_words<TRIP_NW>(stream + (by * nbx + bx) * TRIP_NW, w);
-        BitReader<TRIP_NW> br;
-        br.init(lds, w);
         float f[16];
-        decode_block<16, TRIP_NW>(br, f, tab);
+        decode16<TRIP_NW>(w, f, tab);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             acc[j] += ((f[4 * j] * v[j].x + f[4 * j + 1] * v[j].y) + f[4 * j + 2] * v[j].z) + f[4 * j + 3] * v[j].w;
@@ -174,7 +166,7 @@ __global__ __launch_bounds__(256) void layer_zfp_combine_bwd_kernel(const uint32
             f[4 * j + 2] = j < live ? g[j] * v[j].z : 0.f;
             f[4 * j + 3] = j < live ? g[j] * v[j].w : 0.f;
         }
-        zfp_trip16<false>(f, nullptr, nullptr, lds);
+        zfp_trip16<false>(f, nullptr, nullptr);
         float *p = grad_rows + 4 * by * model_dim + 4 * bx;
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<float4 *>(p + (int64_t)j * model_dim) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void zfp_decode1_kernel(const uint32_t *__rest
     BitReader<NW> br;
     br.init(lds, w);
     float f[4];
-    decode_block<4, NW>(br, f);
+    decode_block4<NW>(br, f);
     reinterpret_cast<float4 *>(field)[b] = make_float4(f[0], f[1], f[2], f[3]);
 }
 
@@ -307,27 +307,23 @@ __global__ __launch_bounds__(256) void zfp_encode2_kernel(const float *__restric
     store_words<NW>(out + b * NW, w);
 }
 
-// blocks per thread: the group-test table (9 KB) is copied into LDS once per work-group
+// blocks per thread: the group-test table (4 KB) is copied into LDS once per work-group
 constexpr int ZD2_PER_THREAD = 4;
 
 template <int NW>
 __global__ __launch_bounds__(256) void zfp_decode2_kernel(const uint32_t *__restrict__ in, const FieldBlocks g, int64_t blocks,
                                                           float *__restrict__ field)
 {
-    __shared__ uint32_t lds[NW <= 2 ? 1 : BitReader<NW>::STRIDE * 256];
-    __shared__ uint16_t tab[GT16_ENTRIES];
-    gt16_load(tab);
-    const int64_t b0 = (int64_t)blockIdx.x * (256 * ZD2_PER_THREAD) + threadIdx.x;
+    __shared__ __align__(16) uint16_t tab[WALK16_ENTRIES];
+    walk16_load(tab);
     for (int it = 0; it < ZD2_PER_THREAD; ++it) {
-        const int64_t b = b0 + 256 * it;
+        const int64_t first = (int64_t)blockIdx.x * (256 * ZD2_PER_THREAD) + 256 * it, b = first + threadIdx.x;
         if (b >= blocks) break;
         uint32_t w[NW];
         load_words<NW>(in + b * NW, w);
-        BitReader<NW> br;
-        br.init(lds, w);
         float f[16];
-        decode_block<16, NW>(br, f, tab);
-        char *p = const_cast<char *>(BlockPlace(g, b - threadIdx.x).corner(field, g));
+        decode16<NW>(w, f, tab);
+        char *p = const_cast<char *>(BlockPlace(g, first).corner(field, g));
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             *reinterpret_cast<float4 *>(p + 16 * j * g.nbx) = make_float4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3]);
@@ -416,8 +412,7 @@ __global__ __launch_bounds__(256) void combine_zfp2_kernel(const uint32_t *__res
 {
     // (one block per thread: with four, so that the table is copied once per 1024 blocks, the launch
     // takes 10 % longer: half the work-groups leave early and the rest run four times as long)
-    __shared__ uint32_t lds[NW <= 2 ? 1 : BitReader<NW>::STRIDE * 256];
-    __shared__ uint16_t tab[GT16_ENTRIES];
+    __shared__ __align__(16) uint16_t tab[WALK16_ENTRIES];
     const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool in_field = b < blocks;
     const int64_t by = (in_field ? b : blocks - 1) / nbx, bx = b - by * nbx;
@@ -428,7 +423,7 @@ __global__ __launch_bounds__(256) void combine_zfp2_kernel(const uint32_t *__res
                           in_field && tok.z >= 0 && pl.z == plane, in_field && tok.w >= 0 && pl.w == plane};
     const bool any_mine = mine[0] || mine[1] || mine[2] || mine[3];
     if (!__syncthreads_or(any_mine)) return;          // a work-group without a row of this plane leaves before the table
-    gt16_load(tab);
+    walk16_load(tab);
     if (!any_mine) return;
     float g[4] = {1.f, 1.f, 1.f, 1.f};
     if (sgate) {
@@ -444,10 +439,8 @@ __global__ __launch_bounds__(256) void combine_zfp2_kernel(const uint32_t *__res
     }
     uint32_t w[NW];
     load_words<NW>(in + b * NW, w);
-    BitReader<NW> br;
-    br.init(lds, w);
     float f[16];
-    decode_block<16, NW>(br, f, tab);
+    decode16<NW>(w, f, tab);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         if (!mine[j]) continue;
@@ -471,14 +464,13 @@ __global__ __launch_bounds__(256) void bwd_gate_zfp2_kernel(const uint32_t *__re
                                                            int64_t model_dim, int64_t nbx,
                                                            float *__restrict__ grad_gates)
 {
-    __shared__ uint32_t lds[NW <= 2 ? 1 : BitReader<NW>::STRIDE * 256];
     __shared__ float s_part[4][4];
-    __shared__ uint16_t tab[GT16_ENTRIES];
+    __shared__ __align__(16) uint16_t tab[WALK16_ENTRIES];
     const int64_t by = blockIdx.x;
     const int4 tok = *reinterpret_cast<const int4 *>(src + 4 * by);
     const int t[4] = {tok.x, tok.y, tok.z, tok.w};
     if (t[0] < 0 && t[1] < 0 && t[2] < 0 && t[3] < 0) return;        // four empty slots (the whole work-group leaves)
-    gt16_load(tab);
+    walk16_load(tab);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     for (int64_t bx0 = 0; bx0 < nbx; bx0 += 256) {
         const int64_t bx = bx0 + threadIdx.x;
@@ -490,10 +482,8 @@ __global__ __launch_bounds__(256) void bwd_gate_zfp2_kernel(const uint32_t *__re
             g[j] = *reinterpret_cast<const float4 *>(grad_out + (int64_t)max(t[j], 0) * model_dim + 4 * bxc);
         uint32_t w[NW];
         load_words<NW>(in + (by * nbx + bxc) * NW, w);
-        BitReader<NW> br;
-        br.init(lds, w);
         float f[16];
-        decode_block<16, NW>(br, f, tab);
+        decode16<NW>(w, f, tab);
         if (in_row) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)

@@ -35,12 +35,9 @@ struct BitWriter {
     }
 };
 
-// The decoder looks at the stream by bit position: the block's words sit in LDS (NW words per
+// The decoder of 1-D blocks looks at the stream by bit position: the block's words sit in LDS (NW words per
 // thread and three zero words behind them: an odd stride) and a look is neighbouring words
-// funnel-shifted, so there is no refill state to carry and no branch in the reader.  A bit plane
-// takes one look of 64 bits (a plane never uses more than 48) and is then parsed in registers: the
-// group tests of a 2-D block eight stream bits at a time by table (gt16_step), except the plane the
-// block's budget ends in, which is walked bit by bit.
+// funnel-shifted, so there is no refill state to carry and no branch in the reader.
 // Streams of one or two words stay in a register pair that is shifted as bits are consumed.
 template <int NW>
 struct BitReader {
@@ -74,17 +71,6 @@ struct BitReader {
         } else {
             const int i = pos >> 5;
             return __builtin_amdgcn_alignbit(words[i + 1], words[i], pos & 31);
-        }
-    }
-    // the next 64 bits
-    __device__ __forceinline__ uint64_t peek64() const
-    {
-        if constexpr (NW <= 2) {
-            return small;
-        } else {
-            const int i = pos >> 5, sh = pos & 31;
-            const uint32_t w0 = words[i], w1 = words[i + 1], w2 = words[i + 2];
-            return (uint64_t)__builtin_amdgcn_alignbit(w1, w0, sh) | ((uint64_t)__builtin_amdgcn_alignbit(w2, w1, sh) << 32);
         }
     }
     __device__ __forceinline__ void skip(int n)      // n <= 32 (NW <= 2), any n otherwise
@@ -400,79 +386,60 @@ __device__ __forceinline__ int code16(float (&f)[16], uint32_t *s, const uint16_
     return field;
 }
 
-// ---- group tests of a 2-D block's bit plane, eight stream bits at a time
+// ---- group tests of a 2-D block's bit plane, eleven stream bits at a time
 // The group-test bits of a plane are a walk with two states: a test bit is due (T), or the zeros of
-// a run up to the next one bit are being read (R).  What eight stream bits do to that walk depends
-// on the state and on how far away the block's last value is (its one is implied, and after it the
-// plane ends without another test bit).  gt16_step works that out once per (state, distance, byte):
-// bits 0..7 the one bits found (relative to the first value that was not significant), bits 8..11
-// the values passed, bits 12..15 a code c: c <= 8 = the plane ended after c bits; 9 / 10 = all eight
-// bits used and the walk goes on in state T / R.  The walk is zfp's own (decode_ints), minus the
-// budget: a step that would use up the budget is not taken, see fast_plane16.
-__host__ __device__ constexpr uint16_t gt16_step(int state, int r, uint32_t byte)
+// a run up to the next one bit are being read (R).  walk16_step is what eleven stream bits do to it from state T on, as if there were values
+// without end: in bits 0..9 the one bits found (relative to the first value that was not significant), in 10..13 the values passed, one
+// more in state R (the value being read), in 14 whether it ends in R, in 15 whether it goes on.  A walk that goes on in state R goes on in T
+// with a test bit in front.  Where the block's last value is reached its one is implied and the plane ends, and how many bits
+// a plane took follows from its values: its own for each, and a test bit for each one and the end.
+__host__ __device__ constexpr uint16_t walk16_step(uint32_t bits)
 {
-    const int last = r < 8 ? r : 99;            // the block's last value, if this step can reach it
-    int n = 0, used = 0, st = state;
-    uint32_t mask = 0;
-    bool done = false;
-    while (true) {
-        if (st == 0) {
-            if (n > last) { done = true; break; }
-            if (used == 8) break;
-            const uint32_t b = (byte >> used) & 1u; ++used;
-            if (!b) { done = true; break; }
-            st = 1;
-        }
-        bool out_of_bits = false;
-        while (n != last) {
-            if (used == 8) { out_of_bits = true; break; }
-            const uint32_t b = (byte >> used) & 1u; ++used;
-            if (b) break;
+    int n = 0, used = 0;
+    uint32_t ones = 0;
+    while (used < 11) {
+        if (!((bits >> used++) & 1u)) return (uint16_t)(ones | ((uint32_t)n << 10));
+        while (true) {
+            if (used == 11) return (uint16_t)(ones | ((uint32_t)(n + 1) << 10) | 0xc000u);
+            if ((bits >> used++) & 1u) break;
             ++n;
         }
-        if (out_of_bits) break;
-        mask |= 1u << n; ++n; st = 0;
-        if (n > last) { done = true; break; }
+        ones |= 1u << n++;
     }
-    const int c = done ? used : (st ? 10 : 9);
-    return (uint16_t)(mask | ((uint32_t)n << 8) | ((uint32_t)c << 12));
+    return (uint16_t)(ones | ((uint32_t)n << 10) | 0x8000u);
 }
-constexpr int GT16_ENTRIES = 9 * 2 * 256;      // [min(15 - nsig, 8)][state][byte]
-struct Gt16Table {
-    uint16_t step[GT16_ENTRIES];
-    constexpr Gt16Table() : step()
+constexpr int WALK16_ENTRIES = 2048;
+struct Walk16Table {
+    uint16_t step[WALK16_ENTRIES];
+    constexpr Walk16Table() : step()
     {
-        for (int i = 0; i < GT16_ENTRIES; ++i) step[i] = gt16_step((i >> 8) & 1, i >> 9, (uint32_t)i & 255u);
+        for (int i = 0; i < WALK16_ENTRIES; ++i) step[i] = walk16_step((uint32_t)i);
     }
 };
-__constant__ const Gt16Table gt16_table = Gt16Table();
+__constant__ const Walk16Table walk16_table __attribute__((aligned(16))) = Walk16Table();
 
-// all 256 threads of the work-group copy the table into LDS (9 KB); a barrier follows
-__device__ __forceinline__ void gt16_load(uint16_t *tab)
+// all 256 threads of the work-group copy the table into LDS (4 KB); a barrier follows
+__device__ __forceinline__ void walk16_load(uint16_t *tab)
 {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(gt16_table.step);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(tab);
-#pragma unroll
-    for (int i = 0; i < GT16_ENTRIES / 2 / 256; ++i) dst[threadIdx.x + 256 * i] = src[threadIdx.x + 256 * i];
+    reinterpret_cast<uint4 *>(tab)[threadIdx.x] = reinterpret_cast<const uint4 *>(walk16_table.step)[threadIdx.x];
     __syncthreads();
 }
 
-// One bit plane of a 2-D block, bit by bit as zfp walks it: look = the next 64 stream bits (a plane
-// never uses more than 48), bits = what is left of the block's budget, nsig = values significant so
+// One bit plane of a 2-D block, bit by bit as zfp walks it: look = the next 32 stream bits (a plane
+// never uses more than 31), bits = what is left of the block's budget, nsig = values significant so
 // far.  nsig verbatim bits, then segment by segment the test bit and the zeros up to the next one
 // bit (cut short by the budget or by the block's last value, whose one is implied).
-__device__ __forceinline__ uint32_t slow_plane16(uint64_t look, int &bits, int &nsig)
+__device__ __forceinline__ uint32_t slow_plane16(uint32_t look, int &bits, int &nsig)
 {
     constexpr int N = 16;
     const int mm = min(nsig, bits);
     bits -= mm;
-    uint32_t x = (uint32_t)look & ((1u << mm) - 1u);
+    uint32_t x = look & ((1u << mm) - 1u);
     look >>= mm;
     while (nsig < N && bits > 0) {
-        const uint32_t lo = (uint32_t)look;
-        if (!(lo & 1u)) { --bits; break; }
+        if (!(look & 1u)) { --bits; break; }
         const int lim = min(N - 1 - nsig, bits - 1);
-        const uint32_t win = (lo >> 1) & ((1u << lim) - 1u);
+        const uint32_t win = (look >> 1) & ((1u << lim) - 1u);
         const int z = win != 0u ? __builtin_ctz(win) : lim;       // zeros read
         const int used = 1 + (win != 0u ? z + 1 : lim);
         look >>= used; bits -= used; nsig += z;
@@ -482,135 +449,121 @@ __device__ __forceinline__ uint32_t slow_plane16(uint64_t look, int &bits, int &
     return x;
 }
 
-// The same plane by table, as long as the budget does not end inside it: false = it would (bits and
-// nsig are then whatever the walk left them at: the caller keeps its own copies and has
-// slow_plane16 do that plane, the block's last).  One exit and selects instead of branches: the
-// lanes of a wave are at different points of their walks.
-__device__ __forceinline__ bool fast_plane16(uint64_t look, int &bits, int &nsig, uint32_t &x, const uint16_t *tab)
-{
-    const int mm = min(nsig, bits);
-    bits -= mm;
-    x = (uint32_t)look & ((1u << mm) - 1u);
-    look >>= mm;
-    bool over = false, go = nsig < 16 && bits > 0;
-    uint32_t st = 0u;                          // state * 256
-    while (go) {
-        const uint32_t r = (uint32_t)min(15 - nsig, 8);
-        const uint32_t e = tab[(r << 9) | st | ((uint32_t)look & 255u)];
-        const uint32_t c = e >> 12;
-        const int used = (int)min(c, 8u);
-        over = used >= bits;
-        const int u = over ? 0 : used;
-        x |= (over ? 0u : (e & 255u)) << nsig;
-        nsig += over ? 0 : (int)((e >> 8) & 15u);
-        look >>= u; bits -= u;
-        st = (c & 1u) ? 0u : 256u;             // c = 9: state T, c = 10: state R (other values end the walk)
-        go = !over && c >= 9u;
-    }
-    return !over;
-}
-
-// tab: the group-test table in LDS (gt16_load), used by 2-D blocks only
-template <int N, int NW>
-__device__ __forceinline__ void decode_block(BitReader<NW> &br, float *f, const uint16_t *tab = nullptr)
+// A block of 4 values
+template <int NW>
+__device__ __forceinline__ void decode_block4(BitReader<NW> &br, float (&f)[4])
 {
     if (!br.get(1)) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) f[i] = 0.f;
+        for (int i = 0; i < 4; ++i) f[i] = 0.f;
         return;
     }
     const int emax = (int)br.get(8) - 127;
-    uint32_t u[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) u[i] = 0u;
+    uint32_t u[4] = {0u, 0u, 0u, 0u};
     int bits = 32 * NW - 9;
     int nsig = 0;
-    auto read_plane = [&]() __attribute__((always_inline)) {
-        if constexpr (N == 4) {
-            const int mm = min(nsig, bits);
-            bits -= mm;
-            uint32_t x = br.get(mm);
-            while (nsig < N && bits > 0) {
-                // tiny blocks: test bit and run are read separately (measured faster here)
-                --bits;
-                if (!br.get(1)) break;
-                const int lim = min(N - 1 - nsig, bits);
-                const uint32_t win = br.peek() & ((1u << lim) - 1u);
-                const int z = win != 0u ? __builtin_ctz(win) : lim;
-                const int used = win != 0u ? z + 1 : lim;
-                br.skip(used); bits -= used; nsig += z;
-                x |= 1u << nsig;
-                ++nsig;
-            }
-            return x;
-        } else {
-            // one look at the stream per plane
-            const int before = bits;
-            const uint32_t x = slow_plane16(br.peek64(), bits, nsig);
-            br.skip(before - bits);
-            return x;
+    for (int k = 31; k >= 0 && bits > 0; --k) {
+        const int mm = min(nsig, bits);
+        bits -= mm;
+        uint32_t x = br.get(mm);
+        while (nsig < 4 && bits > 0) {
+            // tiny blocks: test bit and run are read separately (measured faster here)
+            --bits;
+            if (!br.get(1)) break;
+            const int lim = min(3 - nsig, bits);
+            const uint32_t win = br.peek() & ((1u << lim) - 1u);
+            const int z = win != 0u ? __builtin_ctz(win) : lim;
+            const int used = win != 0u ? z + 1 : lim;
+            br.skip(used); bits -= used; nsig += z;
+            x |= 1u << nsig;
+            ++nsig;
         }
-    };
-    if constexpr (N == 16) {
-        // planes 31..16 are collected as rows and transposed into the coefficients' upper halves
-        uint32_t w[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = 0u;
-        // by table, up to the plane the budget ends in: that one is set aside (every lane has one, each
-        // at a plane of its own) and walked bit by bit afterwards, by all lanes at once
-        int last_k = -1, last_bits = 0, last_nsig = 0;
-        uint64_t last_look = 0;
-#pragma unroll
-        for (int k = 15; k >= 0; --k) {
-            // (a branch of the whole wave; a lane whose budget is spent walks a plane of no bits)
-            if (__builtin_amdgcn_ballot_w64(bits > 0) != 0) {
-                const uint64_t look = br.peek64();
-                const int before = bits, nsig0 = nsig;
-                uint32_t x;
-                const bool ok = fast_plane16(look, bits, nsig, x, tab);
-                br.skip(ok ? before - bits : 0);
-                w[k & 7] |= ok ? x << (16 * (k >> 3)) : 0u;
-                last_k = ok ? last_k : k;
-                last_look = ok ? last_look : look;
-                last_bits = ok ? last_bits : before;
-                last_nsig = ok ? last_nsig : nsig0;
-                bits = ok ? bits : 0;
-            }
-        }
-        if (last_k >= 0) {
-            const uint32_t x = slow_plane16(last_look, last_bits, last_nsig) << (16 * (last_k >> 3));
-#pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] |= (last_k & 7) == j ? x : 0u;
-        }
-        values_of16(w, u);
-        for (int k = 15; k >= 0 && bits > 0; --k) {
-            const uint32_t x = read_plane();
-#pragma unroll
-            for (int i = 0; i < N; ++i) u[i] |= ((x >> i) & 1u) << k;
-        }
-    } else {
-        for (int k = 31; k >= 0 && bits > 0; --k) {
-            const uint32_t x = read_plane();
-#pragma unroll
-            for (int i = 0; i < N; ++i) u[i] |= ((x >> i) & 1u) << k;
-        }
+        for (int i = 0; i < 4; ++i) u[i] |= ((x >> i) & 1u) << k;
     }
-    int32_t q[N];
-    if constexpr (N == 4) {
+    int32_t q[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) q[i] = from_negabinary(u[i]);
-        inv_lift(q[0], q[1], q[2], q[3]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) q[perm2(i)] = from_negabinary(u[i]);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) inv_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
-#pragma unroll
-        for (int y = 0; y < 4; ++y) inv_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
-    }
+    for (int i = 0; i < 4; ++i) q[i] = from_negabinary(u[i]);
+    inv_lift(q[0], q[1], q[2], q[3]);
     const float s = ldexpf(1.0f, emax - 30);
 #pragma unroll
-    for (int i = 0; i < N; ++i) f[i] = (float)q[i] * s;
+    for (int i = 0; i < 4; ++i) f[i] = (float)q[i] * s;
+}
+
+// A block of 4 x 4 values from its NW words s, which are shifted down as planes are read; tab: the table above.
+template <int NW>
+__device__ __forceinline__ void decode16(uint32_t (&s)[NW], float (&f)[16], const uint16_t *tab)
+{
+    auto skip = [&](int n) __attribute__((always_inline)) {          // n <= 31
+#pragma unroll
+        for (int i = 0; i < NW - 1; ++i) s[i] = __builtin_amdgcn_alignbit(s[i + 1], s[i], n);
+        s[NW - 1] >>= n;
+    };
+    const uint32_t head = s[0];
+    skip(9);
+    int bits = 32 * NW - 9, nsig = 0, cut = -1;
+    // A lane reads planes by table up to the one that the budget ends in (there is one in nearly every block): bits, nsig and the
+    // stream stay as they are there, and it is walked bit by bit afterwards, by all lanes at once.
+    bool whole = (head & 1u) != 0u;
+    // planes 31..16 are collected as rows and transposed into the coefficients' upper halves
+    uint32_t w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = 0u;
+#pragma unroll
+    for (int k = 15; k >= 0; --k) {
+        if (whole) {
+            uint32_t x = __builtin_amdgcn_ubfe(s[0], 0u, nsig), look = s[0] >> nsig;
+            int at = nsig, next;
+            while (true) {
+                const uint32_t e = tab[look & (WALK16_ENTRIES - 1)];
+                x |= (e & 0x3ffu) << at;
+                next = at + (int)__builtin_amdgcn_ubfe(e, 10u, 4u);
+                if (e < 0x8000u || next > 15) break;
+                const int reading = (int)__builtin_amdgcn_ubfe(e, 14u, 1u);
+                look = (look >> (11 - reading)) | (uint32_t)reading;
+                at = next - reading;
+            }
+            next = min(next, 16);
+            const int total = next + __builtin_popcount((x & 0x7fffu) >> nsig) + (next < 16);
+            x = (x & 0xffffu) | (next == 16 && nsig < 16 ? 0x8000u : 0u);
+            whole = total <= bits;
+            if (whole) {
+                w[k & 7] |= x << (16 * (k >> 3));
+                bits -= total;
+                nsig = next;
+                skip(total);
+            } else {
+                cut = k;
+            }
+        }
+    }
+    int cut_bits = bits, cut_nsig = nsig;
+    if (cut >= 0) {
+        const uint32_t x = slow_plane16(s[0], cut_bits, cut_nsig) << (16 * (cut >> 3));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] |= (cut & 7) == j ? x : 0u;
+    }
+    uint32_t u[16];
+    values_of16(w, u);
+    if (whole)
+        for (int k = 15; k >= 0 && bits > 0; --k) {
+            const int before = bits;
+            const uint32_t x = slow_plane16(s[0], bits, nsig);
+            skip(before - bits);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) u[i] |= ((x >> i) & 1u) << k;
+        }
+    int32_t q[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) q[perm2(i)] = from_negabinary(u[i]);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) inv_lift(q[x], q[x + 4], q[x + 8], q[x + 12]);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) inv_lift(q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]);
+    // (a block without a stream has values of zero: zeros whatever the factor, which is finite)
+    const float scale = ldexpf(1.0f, (int)((head >> 1) & 0xffu) - 157);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) f[i] = (float)q[i] * scale;
 }
 
 template <int NW>
