@@ -696,7 +696,7 @@ struct GemmSlots { int rows, per_tile; };
 bool gemm_is_skinny(bool nt, int m, int n, int64_t k, int batches)
 {
     if (m > SKINNY_ROWS || batches > 65535 || n * k * 2 >= ((int64_t)1 << 31)) return false;
-    const int width = gemm_skinny_width(nt, n, batches);
+    const int width = gemm_skinny_width(nt, n, k, batches);
     return m <= 16 || (int64_t)((n + width - 1) / width) * batches <= compute_units();
 }
 

@@ -4,14 +4,15 @@
 //
 // For experts that have only few rows (decode, small batches).  Bound by reading the weight once, so nothing
 // goes through LDS on the way in: a wave loads straight into registers, a work-group's waves (16, or 8 where
-// registers ask for it) split the reduction between them, up to four steps each in flight, so that a compute unit has
-// 128 KB on its way; the waves' sums meet in LDS at the end.
+// registers ask for it) split the reduction between them, one to eight steps each in flight, so that a compute unit has
+// 128 or 256 KB on its way; the waves' sums meet in LDS at the end.
 //   nn: lane = (16 chunks of C columns, 4 groups of 8 k): eight loads give an 8 x C patch whose columns are
 //       put together by byte permutes, each a matrix-core operand of its own (column C chunk + c).
 //   nt: lane = (16 columns, 4 groups of 16 k): two loads of 8 k, operands as they are; the four groups of a
 //       row make 128 consecutive bytes.
-// 8 experts x 2 rows, 67 MB of weights: 1024 -> 4096 12.5 us, 4096 -> 1024 (64 columns for a work-group: 128
-// work-groups) 14.2 us (128 x 128 tiles: 24 us).
+// 8 experts x 2 rows, 67 MB of weights that no cache holds (a plain read of them takes 11.5 - 14): 1024 -> 4096 14.8 -> 13.5 us with
+// nontemporal loads, 4096 -> 1024 22.9 -> 18.5 in 32 columns, b^T 20.3 -> 14.3 (128 x 128 tiles: 41 us).  Loads of the next steps go out
+// while a step is worked on: 4 x 20 rows, 4096 -> 4096 b^T 33.6 -> 28.1 (all of a wave's steps at once, then none until they are used).
 #include "gemm_skinny.hpp"
 
 namespace pm {
@@ -19,14 +20,23 @@ namespace pm {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 sk_bf16x8 __attribute__((ext_vector_type(8)));
 
-// MF: 16-row fragments; C: 16-column fragments of the weight, a work-group's columns / 16; U: steps of the reduction a wave has in flight
-template <bool NT, int MF, int C, int U, int WAVES, bool GRAD>
+// MF: 16-row fragments; C: 16-column fragments of the weight, a work-group's columns / 16; U: steps of the reduction a wave has in flight;
+// LARGE: the weight does not stay in the caches anyway (skinny_large)
+template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArgs p)
 {
     constexpr int SK_COLS = 16 * C, SK_PITCH = SK_COLS + 4;             // (floats between rows of a wave's sums in LDS)
     extern __shared__ __align__(16) float part[];           // [WAVES][16][SK_PITCH]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int e = blockIdx.y, n0 = blockIdx.x * SK_COLS;
+    int e = blockIdx.y, group = blockIdx.x;
+    if (LARGE && C == 2) {
+        // neighbours in columns (nn: they share lines of 128 bytes): of every 16 work-groups, i and i + 8, which go to one XCD
+        const int id = e * gridDim.x + group, in = id % 16, first = id - in;
+        const int at = first + 16 <= (int)(gridDim.x * gridDim.y) ? first + 2 * (in % 8) + in / 8 : id;
+        e = at / gridDim.x;
+        group = at % gridDim.x;
+    }
+    const int n0 = group * SK_COLS;
     int rows = p.M;
     if (p.live) {
         int n = 0;
@@ -40,6 +50,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A), 0, rows > 0 ? rows * p.K * 2 : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(B), 0, (int)((int64_t)p.N * p.K * 2), 0x00020000);
     constexpr uint32_t NOWHERE = 0x80000000u;
+    constexpr int ONCE = LARGE ? 2 : 0;                     // a weight is read once: nontemporal (nt: the two loads of 128 bytes meet in the cache)
     const int l16 = lane & 15, g = lane >> 4;
 
     f32x4 acc[MF][C];
@@ -51,68 +62,74 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
     constexpr int KS = NT ? 64 : 32;                        // k of a step
     const int steps = (p.K + KS - 1) / KS;
     const uint32_t place = n0 + C * l16 < p.N ? ((uint32_t)(8 * g) * (uint32_t)p.N + (uint32_t)(n0 + C * l16)) * 2u : NOWHERE;    // (nn)
-    for (int s0 = wave; s0 < steps; s0 += U * WAVES) {
-        // (steps past the end are asked for out of range: they read as zero)
-        if constexpr (!NT) {
-            typedef uint32_t weights __attribute__((ext_vector_type(C / 2)));
-            weights b[U][8];
-            pm_u32x4 a[U][MF];
+    // U steps of the wave are on their way: a step's loads go out as soon as the registers of the step U before it are free
+    auto walk = [&](auto load, auto use) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (wave + u * WAVES < steps) load(u, wave + u * WAVES);
+        for (int s0 = wave; s0 < steps; s0 += U * WAVES) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                // (a lane's place in a step stays, the step and the row are the scalar offset: K is a multiple of 8, so row
-                // s KS + q is inside and what lies behind it is the descriptor's business)
-                const int s = s0 + u * WAVES, k = s * KS + 8 * g;       // this lane's eight k
-                const uint32_t at = s < steps ? place : NOWHERE;
-                const uint32_t step = (uint32_t)min(s, steps - 1) * (uint32_t)(KS * 2) * (uint32_t)p.N;
+                if (s0 + u * WAVES < steps) use(u);
+                if (s0 + (U + u) * WAVES < steps) load(u, s0 + (U + u) * WAVES);
+            }
+        }
+    };
+    if constexpr (!NT) {
+        typedef uint32_t weights __attribute__((ext_vector_type(C / 2)));
+        weights b[U][8];
+        pm_u32x4 a[U][MF];
+        walk([&](int u, int s) {
+            // (a lane's place in a step stays, the step and the row are the scalar offset: K is a multiple of 8, so a lane's
+            // eight k are inside or the descriptor's business together)
+            const int k = s * KS + 8 * g;                   // this lane's eight k
+            const uint32_t at = place, step = (uint32_t)s * (uint32_t)(KS * 2) * (uint32_t)p.N;
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    if constexpr (C == 8) b[u][q] = __builtin_amdgcn_raw_buffer_load_b128(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, 0);
-                    else b[u][q] = __builtin_amdgcn_raw_buffer_load_b64(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, 0);
-                }
-#pragma unroll
-                for (int m = 0; m < MF; ++m)
-                    a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(da, k < p.K && 16 * m + l16 < rows ? ((uint32_t)(16 * m + l16) * (uint32_t)p.K + (uint32_t)k) * 2u : NOWHERE, 0, 0);
+            for (int q = 0; q < 8; ++q) {
+                if constexpr (C == 8) b[u][q] = __builtin_amdgcn_raw_buffer_load_b128(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
+                else if constexpr (C == 4) b[u][q] = __builtin_amdgcn_raw_buffer_load_b64(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
+                else b[u][q][0] = __builtin_amdgcn_raw_buffer_load_b32(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+            for (int m = 0; m < MF; ++m)
+                a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(da, k < p.K && 16 * m + l16 < rows ? ((uint32_t)(16 * m + l16) * (uint32_t)p.K + (uint32_t)k) * 2u : NOWHERE, 0, 0);
+        }, [&](int u) {
 #pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    pm_u32x4 f;
+            for (int c = 0; c < C; ++c) {
+                pm_u32x4 f;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)             // column c of rows 2 q and 2 q + 1
-                        f[q] = __builtin_amdgcn_perm(b[u][2 * q + 1][c >> 1], b[u][2 * q][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
+                for (int q = 0; q < 4; ++q)                 // column c of rows 2 q and 2 q + 1
+                    f[q] = __builtin_amdgcn_perm(b[u][2 * q + 1][c >> 1], b[u][2 * q][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
 #pragma unroll
-                    for (int m = 0; m < MF; ++m)
-                        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[u][m]), __builtin_bit_cast(sk_bf16x8, f), acc[m][c], 0, 0, 0);
+                for (int m = 0; m < MF; ++m)
+                    acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[u][m]), __builtin_bit_cast(sk_bf16x8, f), acc[m][c], 0, 0, 0);
+            }
+        });
+    } else {
+        pm_u32x4 b[U][C][2], a[U][MF][2];
+        walk([&](int u, int s) {
+            const int k = s * KS + 16 * g;
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int row = n0 + 16 * c + l16;
+                    b[u][c][j] = __builtin_amdgcn_raw_buffer_load_b128(db, row < p.N && k + 8 * j < p.K ? ((uint32_t)row * (uint32_t)p.K + (uint32_t)(k + 8 * j)) * 2u : NOWHERE, 0, 0);
                 }
-        } else {
-            pm_u32x4 b[U][C][2], a[U][MF][2];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = (s0 + u * WAVES) * KS + 16 * g;
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    a[u][m][j] = __builtin_amdgcn_raw_buffer_load_b128(da, k + 8 * j < p.K && 16 * m + l16 < rows ? ((uint32_t)(16 * m + l16) * (uint32_t)p.K + (uint32_t)(k + 8 * j)) * 2u : NOWHERE, 0, 0);
+        }, [&](int u) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int c = 0; c < C; ++c)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int row = n0 + 16 * c + l16;
-                        b[u][c][j] = __builtin_amdgcn_raw_buffer_load_b128(db, row < p.N && k + 8 * j < p.K ? ((uint32_t)row * (uint32_t)p.K + (uint32_t)(k + 8 * j)) * 2u : NOWHERE, 0, 0);
-                    }
-#pragma unroll
-                for (int m = 0; m < MF; ++m)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        a[u][m][j] = __builtin_amdgcn_raw_buffer_load_b128(da, k + 8 * j < p.K && 16 * m + l16 < rows ? ((uint32_t)(16 * m + l16) * (uint32_t)p.K + (uint32_t)(k + 8 * j)) * 2u : NOWHERE, 0, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int c = 0; c < C; ++c)
-#pragma unroll
-                        for (int m = 0; m < MF; ++m)
-                            acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[u][m][j]), __builtin_bit_cast(sk_bf16x8, b[u][c][j]), acc[m][c], 0, 0, 0);
-        }
+                    for (int m = 0; m < MF; ++m)
+                        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[u][m][j]), __builtin_bit_cast(sk_bf16x8, b[u][c][j]), acc[m][c], 0, 0, 0);
+        });
     }
 
     // the waves' sums meet in LDS, 16 rows at a time; a lane has rows 4 g .. + 3 of column C l16 + c (nn) or 16 c + l16 (nt)
@@ -130,8 +147,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
             float *to = mine + (4 * g + q) * SK_PITCH;
             if constexpr (!NT) {
 #pragma unroll
-                for (int c = 0; c < C; c += 4)
+                for (int c = 0; c + 4 <= C; c += 4)
                     *reinterpret_cast<float4 *>(to + C * l16 + c) = make_float4(acc[m][c][q], acc[m][c + 1][q], acc[m][c + 2][q], acc[m][c + 3][q]);
+                if constexpr (C == 2) *reinterpret_cast<float2 *>(to + 2 * l16) = make_float2(acc[m][0][q], acc[m][1][q]);
             } else {
 #pragma unroll
                 for (int c = 0; c < C; ++c) to[16 * c + l16] = acc[m][c][q];
@@ -173,11 +191,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
     if (GRAD && p.colsum && tid < SK_COLS && n0 + tid < p.N) p.colsum[(int64_t)e * p.N + n0 + tid] = colsum;
 }
 
-template <bool NT, int MF, int C, int U, int WAVES, bool GRAD>
+template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
 static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *who)
 {
     constexpr int COLS = 16 * C, LDS = WAVES * 16 * (COLS + 4) * 4;
-    const auto kernel = gemm_skinny_kernel<NT, MF, C, U, WAVES, GRAD>;
+    const auto kernel = gemm_skinny_kernel<NT, MF, C, U, WAVES, GRAD, LARGE>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -191,38 +209,54 @@ static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *wh
     return 0;
 }
 
-// Columns of a work-group: 64, with more steps in flight, where there is a compute unit for each work-group; else the width that
-// takes a compute unit through the fewest columns, 128 where two widths do (nn in 96, whose pieces of a row are 12 bytes, is no faster than in 128).
-// us with cold weights, 64, 96 and 128 columns:
-//   8 experts x 8 rows, 2688 -> 2560    nn 36, 29, 26   nt 33, 25, 29        (320, 216 and 160 work-groups)
-//   8 x 8, 3072 -> 1536                 nn 20, 26, 25   nt 21, 25, 31
-//   16 x 8, 3072 -> 1536                nn 40, 35, 32   nt 40, 31, 35
-//   8 x 8, 1024 -> 4096                 nn 20, 20, 15   nt 17, 19, 14
-//   8 x 20, 4096 -> 1024                nn 28, 35, 36   nt 30, 35, 43
+// From 16 MB on a weight is read past the caches; below, the next call may find it there (us, plain and nontemporal: 8 experts x 2,
+// 512 -> 512 4.0, 5.2; 4 x 2, 1024 -> 1024 4.7, 5.6; 8 x 2, 1024 -> 1024 6.8, 6.8; 16 x 2, 1024 -> 1024 8.8, 7.9).
+static bool skinny_large(int64_t n, int64_t k, int64_t batches) { return n * k * batches * 2 >= (int64_t)16 << 20; }
+
+// Columns of a work-group: 32 or 64 where that leaves a compute unit for each work-group (one compute unit gets at most 28 GB/s
+// from memory, however much it has on its way); else the width that takes a compute unit through the fewest columns, 128 where two
+// widths do (nn in 96, whose pieces of a row are 12 bytes, is no faster than in 128).
+// us with cold weights (every one of 1.6 GB in turn), rows in use of 8 and 24, in 32, 64, 96 and 128 columns:
+//   8 experts x 2, 1024 -> 4096         nn 23, 14.5, -, 13.5      nt 15, 14, -, 13.8
+//   8 x 2, 4096 -> 1024                 nn 18.5, 20.4, -, 27      nt 14.3, 20, -, 30
+//   8 x 2, 3072 -> 1536                 nn 28, 17.1, -, 24        nt 19, 16.5, -, 24          (384, 192, 96 work-groups)
+//   4 x 2, 4096 -> 512                  nn 16.4, 18.3, -, 24      nt 11, 19, -, 26
+//   8 x 20, 4096 -> 1024                nn 22.4, 25, -, 35        nt 17.4, 24, -, 43
+//   8 x 8, 2688 -> 2560                 nn 37, 30, 29, 23         nt 24, 33, 23, 29
+// (nn in 32 columns reads 64 bytes of a row, two work-groups a line: it takes the compute units that 64 leave idle, but no more)
 int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
 {
-    const bool grad = p.mask != nullptr;
-#define PM_SK(MF, C, U_NN, WAVES_NN, U_NT, WAVES_NT)                                     \
-    (!nt ? skinny_launch<false, MF, C, U_NN, WAVES_NN, false>(p, stream, who)            \
-     : grad ? skinny_launch<true, MF, C, U_NT, WAVES_NT, true>(p, stream, who)           \
-            : skinny_launch<true, MF, C, U_NT, WAVES_NT, false>(p, stream, who))
-    const int width = gemm_skinny_width(nt, p.N, p.batches);
-    // (nn in 96 columns is not built and not asked for)
-    if (p.M <= 16) {
-        if (width == 96) return grad ? skinny_launch<true, 1, 6, 1, 16, true>(p, stream, who) : skinny_launch<true, 1, 6, 1, 16, false>(p, stream, who);
-        return width == 64 ? PM_SK(1, 4, 4, 16, 2, 16) : PM_SK(1, 8, 1, 16, 1, 16);
+    const bool grad = p.mask != nullptr, large = skinny_large(p.N, p.K, p.batches);
+#define PM_SK_NN(MF, C, U, WAVES) (large ? skinny_launch<false, MF, C, U, WAVES, false, true>(p, stream, who)                    \
+                                         : skinny_launch<false, MF, C, U, WAVES, false, false>(p, stream, who))
+#define PM_SK_NT(MF, C, U, WAVES, LARGE) (grad ? skinny_launch<true, MF, C, U, WAVES, true, LARGE>(p, stream, who)               \
+                                               : skinny_launch<true, MF, C, U, WAVES, false, LARGE>(p, stream, who))
+    const int width = gemm_skinny_width(nt, p.N, p.K, p.batches);
+    const bool few = p.M <= 16;
+    if (!nt) {
+        if (width == 32) return few ? skinny_launch<false, 1, 2, 8, 16, false, true>(p, stream, who) : skinny_launch<false, 2, 2, 8, 8, false, true>(p, stream, who);
+        if (width == 64) return few ? PM_SK_NN(1, 4, 2, 16) : PM_SK_NN(2, 4, 2, 16);
+        return few ? PM_SK_NN(1, 8, 1, 16) : PM_SK_NN(2, 8, 1, 16);
     }
-    // (nt holds 12 or 16 KB of weight per step: 8 waves' registers)
-    if (width == 96) return grad ? skinny_launch<true, 2, 6, 1, 8, true>(p, stream, who) : skinny_launch<true, 2, 6, 1, 8, false>(p, stream, who);
-    return width == 64 ? PM_SK(2, 4, 1, 16, 1, 16) : PM_SK(2, 8, 1, 16, 1, 8);
-#undef PM_SK
+    // (12 or 16 KB of weight per step: with 17 rows and more 8 waves' registers)
+    switch (width) {
+    case 32:
+        if (large) return few ? PM_SK_NT(1, 2, 2, 16, true) : PM_SK_NT(2, 2, 4, 8, true);
+        return few ? PM_SK_NT(1, 2, 2, 16, false) : PM_SK_NT(2, 2, 4, 8, false);
+    case 64: return few ? PM_SK_NT(1, 4, 1, 16, false) : PM_SK_NT(2, 4, 1, 16, false);
+    case 96: return few ? PM_SK_NT(1, 6, 1, 16, false) : PM_SK_NT(2, 6, 1, 8, false);
+    default: return few ? PM_SK_NT(1, 8, 1, 16, false) : PM_SK_NT(2, 8, 1, 8, false);
+    }
+#undef PM_SK_NN
+#undef PM_SK_NT
 }
 
-int gemm_skinny_width(bool nt, int n, int batches)
+int gemm_skinny_width(bool nt, int n, int64_t k, int batches)
 {
     const int64_t cu = compute_units();
     auto groups = [&](int width) { return (int64_t)((n + width - 1) / width) * batches; };
     auto columns = [&](int width) { return (groups(width) + cu - 1) / cu * width; };
+    if (groups(32) <= cu && (nt || skinny_large(n, k, batches))) return 32;        // (nn, small: 4.0 us in 64 columns, 5.2 in 32)
     if (groups(64) <= cu) return 64;
     if (!nt) return 128;
     if (columns(128) <= columns(64) && columns(128) <= columns(96)) return 128;

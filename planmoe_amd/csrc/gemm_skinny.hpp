@@ -17,7 +17,7 @@ struct SkinnyArgs {
 };
 
 // the columns that a work-group takes
-int gemm_skinny_width(bool nt, int n, int batches);
+int gemm_skinny_width(bool nt, int n, int64_t k, int batches);
 // nt: b is [batches, N, K], else [batches, K, N]; the caller has checked shape and alignment
 int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who);
 

@@ -133,6 +133,41 @@ def test_expert_gemm_with_few_rows(m, n, k):
         assert bool(((db[e] - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all())
 
 
+# weights of 16 MB and more, read past the caches: 32 columns a work-group (99 and 195 of them: the last are no whole sixteen), 64 and 128;
+# rows either side of a fragment, a reduction whose last step is partial
+@pytest.mark.parametrize("m", [1, 16, 17, 32])
+@pytest.mark.parametrize("B,n,k", [(3, 1032, 4104), (3, 2072, 2056), (3, 4104, 1032), (5, 8200, 520)])
+def test_expert_gemm_with_few_rows_of_large_weights(m, B, n, k):
+    from planmoe_amd import ops
+    print("case", m, B, n, k, flush=True)
+    assert B * n * k * 2 >= 16 << 20
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    dtype = torch.bfloat16
+    randn = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
+    rows = [m, 0, max(m // 2, 1), m, 1][:B]
+    a, bias, w, h = randn(B, m, k), randn(B, n), randn(B, k, n), randn(B, m, n).clamp(min=0)
+    for e in range(B):
+        a[e, rows[e]:] = float("nan")
+    live = torch.tensor([rows], dtype=torch.int32, device=DEV)
+    wt = w.transpose(1, 2).contiguous()
+    nn = torch.full((B, m, n), 7.0, dtype=dtype, device=DEV)
+    nt, masked = nn.clone(), nn.clone()
+    ops.expert_gemm("nn", a, w, bias, relu=True, live=live, out=nn)
+    ops.expert_gemm("nt", a, wt, live=live, out=nt)
+    _, db = ops.expert_gemm_relu_bwd(a, wt, h, live=live, out=masked)
+    torch.cuda.synchronize()
+    for e, r in enumerate(rows):
+        x, y = a[e, :r].double(), w[e].double()
+        ref, mag = x @ y, x.abs() @ y.abs()
+        tol, biased = _bound(ref, mag, k, dtype), ref + bias[e].double()
+        assert bool(((nn[e, :r].double() - biased.clamp(min=0)).abs() <= tol + _bound(biased, bias[e].double().abs()[None], 1, dtype)).all())
+        assert bool(((nt[e, :r].double() - ref).abs() <= tol).all())
+        assert bool(((masked[e, :r].double() - ref * (h[e, :r] > 0)).abs() <= tol).all())
+        assert bool((nn[e, r:] == 7.0).all()) and bool((nt[e, r:] == 7.0).all()) and bool((masked[e, r:] == 7.0).all())
+        stored = masked[e, :r].double()
+        assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all())
+
+
 # 256 work-groups that stay take 256 x 256 tiles, four to a tile row here; what is left for a last round is a launch of
 # quarters up to 128 tiles.  Rows in use that leave 0, 4 (one row of the last tile), 128 and 132 tiles, and fewer than one round
 # (with k = 4096 and 8192 rows a batch expected; with k = 512 what is picked for the rows that are there)
