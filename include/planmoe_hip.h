@@ -483,6 +483,17 @@ int planmoe_layer_dispatch(const void *x, const void *wg, int dtype, int fp32_ga
                            int64_t plane_stride, void *scores_out, float *l_aux, int32_t *expert_counts,
                            void *rows, void *workspace, size_t workspace_bytes, void *stream);
 
+/* planmoe_layer_dispatch (no biases on the logits, no scores) and the experts' first product of its rows with w1 [experts, model_dim,
+ * hidden], b1 [experts, hidden] (NULL: none) and a relu, h [experts, capacity, hidden] (planmoe_expert_gemm): the same bits in one launch for
+ * few tokens, two otherwise.  `rows` [experts, capacity, model_dim] is scratch: whether it is written depends on the shape.  Nothing is kept for
+ * a backward pass.  expert_counts is not NULL. */
+int planmoe_layer_dispatch_product(const void *x, const void *wg, int dtype, int fp32_gate, int samples, int model_dim,
+                                   int experts, int top_k, int normalize_gate, int capacity, int codec,
+                                   int32_t *indices, int32_t *locations, void *gates, int64_t plane_stride,
+                                   float *l_aux, int32_t *expert_counts, const void *w1, const void *b1, int hidden,
+                                   int rows_hint, void *rows, void *h, void *workspace, size_t workspace_bytes,
+                                   void *stream);
+
 /* fast_decode (fast_dispatch.py:203-207) of the experts' rows, each taken through the int8 codec first when
  * codec = 1 (as the receive side's Compress / Decompress pair would, overlap.py:66-74).  Reads only rows that hold a
  * token.  gates NULL: all ones.  model_dim a multiple of 8 (fp32: 4), at most 8192 (fp32: 4096). */

@@ -173,15 +173,15 @@ std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, con
                                    nullptr, l_aux.data_ptr<float>(), cnt, ws, ws_bytes, st));
         PM_CALL(planmoe_layer_zfp_dispatch(floats(x), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt, (float *)xe, ws, ws_bytes, st));
     } else {
-        PM_CALL(planmoe_layer_dispatch(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, codec, idx, loc,
-                                       base + gates_at, s.T, nullptr, l_aux.data_ptr<float>(), cnt, xe, ws, ws_bytes, st));
+        PM_CALL(planmoe_layer_dispatch_product(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, s.T, s.M, s.E, s.k, normalize, s.cap, codec, idx, loc, base + gates_at,
+                                               s.T, l_aux.data_ptr<float>(), cnt, w1.data_ptr(), b1.data_ptr(), s.H, s.hint(), xe, h, ws, ws_bytes, st));
     }
     if (bf16_gate) {
         at::from_blob(base + wide_at, {s.k, s.T}, x.options().dtype(at::kFloat)).copy_(at::from_blob(base + gates_at, {s.k, s.T}, x.options()));
         gates = (const float *)(base + wide_at);
     }
     const int round = codec == CODEC_ZFP ? 4 : 1;
-    PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
+    if (codec == CODEC_ZFP) PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
     PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, round, s.hint(), ye, st));
     if (codec == CODEC_ZFP) PM_CALL(planmoe_layer_zfp_rows((float *)ye, s.M, s.E, s.cap, cnt, s.k, nullptr, 0, st));
     PM_CALL(planmoe_layer_combine(ye, s.dt, codec == CODEC_INT8, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));

@@ -13,30 +13,19 @@
 // 8 experts x 2 rows, 67 MB of weights that no cache holds (a plain read of them takes 11.5 - 14): 1024 -> 4096 14.8 -> 13.5 us with
 // nontemporal loads, 4096 -> 1024 22.9 -> 18.5 in 32 columns, b^T 20.3 -> 14.3 (128 x 128 tiles: 41 us).  Loads of the next steps go out
 // while a step is worked on: 4 x 20 rows, 4096 -> 4096 b^T 33.6 -> 28.1 (all of a wave's steps at once, then none until they are used).
-#include "gemm_skinny.hpp"
+#include "gemm_skinny_core.hpp"
 
 namespace pm {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 sk_bf16x8 __attribute__((ext_vector_type(8)));
-
 // MF: 16-row fragments; C: 16-column fragments of the weight, a work-group's columns / 16; U: steps of the reduction a wave has in flight;
-// LARGE: the weight does not stay in the caches anyway (skinny_large)
+// LARGE: the weight does not stay in the caches anyway (skinny_large): read nontemporally (nt: not, the two loads of 128 bytes meet in the cache)
 template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArgs p)
 {
-    constexpr int SK_COLS = 16 * C, SK_PITCH = SK_COLS + 4;             // (floats between rows of a wave's sums in LDS)
-    extern __shared__ __align__(16) float part[];           // [WAVES][16][SK_PITCH]
+    extern __shared__ __align__(16) float part[];           // [WAVES][16][16 C + 4]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int e = blockIdx.y, group = blockIdx.x;
-    if (LARGE && C == 2) {
-        // neighbours in columns (nn: they share lines of 128 bytes): of every 16 work-groups, i and i + 8, which go to one XCD
-        const int id = e * gridDim.x + group, in = id % 16, first = id - in;
-        const int at = first + 16 <= (int)(gridDim.x * gridDim.y) ? first + 2 * (in % 8) + in / 8 : id;
-        e = at / gridDim.x;
-        group = at % gridDim.x;
-    }
-    const int n0 = group * SK_COLS;
+    int e, n0;
+    skinny_tile<16 * C, LARGE && C == 2>(e, n0);
     int rows = p.M;
     if (p.live) {
         int n = 0;
@@ -49,8 +38,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
     const uint16_t *B = p.B + (int64_t)e * p.N * p.K;
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A), 0, rows > 0 ? rows * p.K * 2 : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(B), 0, (int)((int64_t)p.N * p.K * 2), 0x00020000);
-    constexpr uint32_t NOWHERE = 0x80000000u;
-    constexpr int ONCE = LARGE ? 2 : 0;                     // a weight is read once: nontemporal (nt: the two loads of 128 bytes meet in the cache)
+    constexpr uint32_t NOWHERE = SK_NOWHERE;
     const int l16 = lane & 15, g = lane >> 4;
 
     f32x4 acc[MF][C];
@@ -76,35 +64,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         }
     };
     if constexpr (!NT) {
-        typedef uint32_t weights __attribute__((ext_vector_type(C / 2)));
-        weights b[U][8];
+        SkinnyWeights<C, LARGE> b[U];
         pm_u32x4 a[U][MF];
         walk([&](int u, int s) {
-            // (a lane's place in a step stays, the step and the row are the scalar offset: K is a multiple of 8, so a lane's
-            // eight k are inside or the descriptor's business together)
             const int k = s * KS + 8 * g;                   // this lane's eight k
-            const uint32_t at = place, step = (uint32_t)s * (uint32_t)(KS * 2) * (uint32_t)p.N;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if constexpr (C == 8) b[u][q] = __builtin_amdgcn_raw_buffer_load_b128(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
-                else if constexpr (C == 4) b[u][q] = __builtin_amdgcn_raw_buffer_load_b64(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
-                else b[u][q][0] = __builtin_amdgcn_raw_buffer_load_b32(db, at, step + (uint32_t)(q * 2) * (uint32_t)p.N, ONCE);
-            }
+            b[u].load(db, place, s, p.N);
 #pragma unroll
             for (int m = 0; m < MF; ++m)
                 a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(da, k < p.K && 16 * m + l16 < rows ? ((uint32_t)(16 * m + l16) * (uint32_t)p.K + (uint32_t)k) * 2u : NOWHERE, 0, 0);
-        }, [&](int u) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                pm_u32x4 f;
-#pragma unroll
-                for (int q = 0; q < 4; ++q)                 // column c of rows 2 q and 2 q + 1
-                    f[q] = __builtin_amdgcn_perm(b[u][2 * q + 1][c >> 1], b[u][2 * q][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
-#pragma unroll
-                for (int m = 0; m < MF; ++m)
-                    acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[u][m]), __builtin_bit_cast(sk_bf16x8, f), acc[m][c], 0, 0, 0);
-            }
-        });
+        }, [&](int u) { b[u].multiply(a[u], acc); });
     } else {
         pm_u32x4 b[U][C][2], a[U][MF][2];
         walk([&](int u, int s) {
@@ -132,63 +100,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         });
     }
 
-    // the waves' sums meet in LDS, 16 rows at a time; a lane has rows 4 g .. + 3 of column C l16 + c (nn) or 16 c + l16 (nt)
-    constexpr int EACH = (16 * SK_COLS + WAVES * 64 - 1) / (WAVES * 64), PER = EACH == 3 ? 4 : EACH;        // outputs of a thread: 1, 2 or 4 columns of a row
-    const bool writes = tid * PER < 16 * SK_COLS;           // (96 columns: three threads in four)
-    const int row_t = writes ? tid * PER / SK_COLS : 0, col_t = tid * PER % SK_COLS;
-    float *mine = part + wave * 16 * SK_PITCH;
-    uint16_t *out = p.C + (int64_t)e * p.M * p.N;
-    float colsum = 0.f;                                     // GRAD: of column n0 + tid
-#pragma unroll
-    for (int m = 0; m < MF; ++m) {
-        if (m > 0) __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float *to = mine + (4 * g + q) * SK_PITCH;
-            if constexpr (!NT) {
-#pragma unroll
-                for (int c = 0; c + 4 <= C; c += 4)
-                    *reinterpret_cast<float4 *>(to + C * l16 + c) = make_float4(acc[m][c][q], acc[m][c + 1][q], acc[m][c + 2][q], acc[m][c + 3][q]);
-                if constexpr (C == 2) *reinterpret_cast<float2 *>(to + 2 * l16) = make_float2(acc[m][0][q], acc[m][1][q]);
-            } else {
-#pragma unroll
-                for (int c = 0; c < C; ++c) to[16 * c + l16] = acc[m][c][q];
-            }
-        }
-        __syncthreads();
-        float v[PER];
-#pragma unroll
-        for (int x = 0; x < PER; ++x) v[x] = 0.f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w)
-#pragma unroll
-            for (int x = 0; x < PER; ++x) v[x] += part[(w * 16 + row_t) * SK_PITCH + col_t + x];
-        const int row = 16 * m + row_t, col = n0 + col_t;
-        const bool inside = writes && row < rows && col < p.N;        // (N is a multiple of 8: a thread's columns are in or out together)
-#pragma unroll
-        for (int x = 0; x < PER; ++x) {
-            v[x] = bf16_to_f32(f32_to_bf16(v[x]));
-            if (!GRAD && p.bias && inside) v[x] = bf16_to_f32(f32_to_bf16(v[x] + bf16_to_f32(p.bias[(int64_t)e * p.N + col + x])));
-            if (!GRAD && p.relu) v[x] = v[x] < 0.f ? 0.f : v[x];
-            if (GRAD && !(inside && bf16_to_f32(p.mask[((int64_t)e * p.M + row) * p.N + col + x]) > 0.f)) v[x] = 0.f;
-        }
-        if (inside) {
-            uint16_t *to = out + (int64_t)row * p.N + col;
-            if constexpr (PER == 4) *reinterpret_cast<uint2 *>(to) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
-            else if constexpr (PER == 2) *reinterpret_cast<uint32_t *>(to) = f32x2_to_bf16x2(v[0], v[1]);
-            else *to = f32_to_bf16(v[0]);
-        }
-        if (GRAD && p.colsum) {
-            __syncthreads();
-#pragma unroll
-            for (int x = 0; x < PER; ++x) if (writes) part[row_t * SK_PITCH + col_t + x] = v[x];
-            __syncthreads();
-            if (tid < SK_COLS)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) colsum += part[r * SK_PITCH + tid];
-        }
-    }
-    if (GRAD && p.colsum && tid < SK_COLS && n0 + tid < p.N) p.colsum[(int64_t)e * p.N + n0 + tid] = colsum;
+    skinny_finish<NT, MF, C, WAVES, GRAD>(p, e, n0, rows, acc, part);
 }
 
 template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
@@ -211,7 +123,7 @@ static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *wh
 
 // From 16 MB on a weight is read past the caches; below, the next call may find it there (us, plain and nontemporal: 8 experts x 2,
 // 512 -> 512 4.0, 5.2; 4 x 2, 1024 -> 1024 4.7, 5.6; 8 x 2, 1024 -> 1024 6.8, 6.8; 16 x 2, 1024 -> 1024 8.8, 7.9).
-static bool skinny_large(int64_t n, int64_t k, int64_t batches) { return n * k * batches * 2 >= (int64_t)16 << 20; }
+bool skinny_large(int64_t n, int64_t k, int64_t batches) { return n * k * batches * 2 >= (int64_t)16 << 20; }
 
 // Columns of a work-group: 32 or 64 where that leaves a compute unit for each work-group (one compute unit gets at most 28 GB/s
 // from memory, however much it has on its way); else the width that takes a compute unit through the fewest columns, 128 where two

@@ -16,6 +16,8 @@ struct SkinnyArgs {
     int M, N, K, batches, relu;   // operands and result contiguous
 };
 
+// a weight that is read past the caches
+bool skinny_large(int64_t n, int64_t k, int64_t batches);
 // the columns that a work-group takes
 int gemm_skinny_width(bool nt, int n, int64_t k, int batches);
 // nt: b is [batches, N, K], else [batches, K, N]; the caller has checked shape and alignment

@@ -1,0 +1,180 @@
+// The layer's first product for few tokens (decode), which routes them itself.
+//
+// A decode step reads its weights once; before that the gate's launch takes 8 us of one work-group's latencies (8 tokens x 1024: launch,
+// loads, products, softmax, ranks, one after the other) while memory has nothing to do.  Here every work-group of the first product
+// (gemm_skinny.hip) routes all tokens for itself: four of its sixteen waves are the gate's work-group (gate_route.hpp; x and the gate's
+// weight come from L2), the other twelve have asked for their share of the expert's weight before they wait for them.  A work-group then knows
+// its expert's tokens and takes their rows straight from x, through the int8 codec where the exchange has one, so that
+// the dispatched rows are neither written nor read.  Same roundings and the same order of sums as the launches it stands for.
+//
+// Bound by reading the weights and the gate's latency under it.  A pass of 8 tokens x 1024, hidden 4096, 8 experts, weights cold: see
+// planmoe_layer_dispatch_product.
+#include "gate_route.hpp"
+#include "gemm_skinny_core.hpp"
+
+namespace pm {
+
+struct FirstArgs {
+    const void *x, *wg;
+    int samples, top_k, normalize_gate;
+    int32_t *indices, *locations;
+    void *gates;
+    int64_t stride;
+    float *l_aux;
+    int32_t *counts;
+};
+
+constexpr int FIRST_WAVES = 16, FIRST_TOKENS = 32, FIRST_ROWS = 16;          // a group's tokens, an expert's rows
+
+// CAP: bound of the number of experts.  DECODED: rows go through the int8 codec.  C, U, LARGE: as gemm_skinny_kernel
+template <int CAP, bool DECODED, int C, int U, bool LARGE>
+__global__ __launch_bounds__(FIRST_WAVES * 64) void layer_first_kernel(const SkinnyArgs p, const FirstArgs r)
+{
+    constexpr int ONE = DECODED ? OUT_DECODED : OUT_ROWS;
+    extern __shared__ __align__(16) float part[];           // [FIRST_WAVES][16][16 C + 4]
+    __shared__ GateShared<PLANMOE_BF16, 1, CAP, true, FIRST_TOKENS, 0, ONE> sh;
+    __shared__ int32_t s_token[FIRST_ROWS];                 // the expert's rows
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int e, n0;
+    skinny_tile<16 * C, LARGE && C == 2>(e, n0);
+    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(r.x), 0, r.samples * p.K * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.B + (int64_t)e * p.N * p.K), 0, (int)((int64_t)p.N * p.K * 2), 0x00020000);
+    const int l16 = lane & 15, g = lane >> 4, steps = (p.K + 31) / 32;
+    const uint32_t place = n0 + C * l16 < p.N ? ((uint32_t)(8 * g) * (uint32_t)p.N + (uint32_t)(n0 + C * l16)) * 2u : SK_NOWHERE;
+
+    SkinnyWeights<C, LARGE> b[U];
+    auto ask = [&] {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (wave + u * FIRST_WAVES < steps) b[u].load(db, place, wave + u * FIRST_WAVES, p.N);
+    };
+    if (wave < 4) {
+        const bool first = blockIdx.x == 0 && blockIdx.y == 0;
+        gate_route_group<PLANMOE_BF16, PLANMOE_F32, 1, CAP, true, FIRST_TOKENS, 0, ONE>(sh, first, 0, 1, r.x, r.wg, nullptr, r.samples, p.K, p.batches, r.top_k,
+            r.normalize_gate, r.indices, r.locations, r.gates, r.stride, nullptr, nullptr, first ? r.l_aux : nullptr, r.counts, nullptr, p.M);
+        if (wave == 0) {                                    // (the wave that wrote the slots)
+            __builtin_amdgcn_wave_barrier();
+            for (int j = 0; j < r.top_k; ++j) {
+                const int at = lane < FIRST_TOKENS ? sh.slot[j][lane] - e * p.M : -1;        // (-1 becomes negative: no slot)
+                if (at >= 0 && at < p.M) s_token[at] = lane;
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        ask();
+    } else {
+        ask();
+        // (as many barriers as the gate's waves meet at; what has been asked for stays on its way)
+        asm volatile("s_barrier\n\ts_barrier\n\ts_barrier" ::: "memory");
+    }
+    const int rows = min(p.M, __builtin_amdgcn_readfirstlane(sh.total[e]));
+    if (rows == 0) return;
+
+    // a lane's row of x, and what the codec makes of its values
+    const int token = l16 < rows ? s_token[l16] : -1;
+    const uint32_t at = token >= 0 ? ((uint32_t)token * (uint32_t)p.K + 8u * (uint32_t)g) * 2u : SK_NOWHERE;
+    float mn = 0.f, mx = 0.f;
+    if constexpr (DECODED) { mn = sh.range[max(token, 0)][0]; mx = sh.range[max(token, 0)][1]; }
+    const float scale = Elem<PLANMOE_BF16>::round(mx - mn);
+    const RowEncoder<PLANMOE_BF16> enc(mn, scale);
+    const RowDecoder<PLANMOE_BF16> dec(mn, scale);
+    const bool fast = __ballot(token >= 0 && !enc.rq.fast) == 0;        // (the wave's rows: what is right for all of them)
+    auto through_codec = [&](const pm_u32x4 &a, int step) {
+        if constexpr (!DECODED) return a;
+        const uint4 raw = make_uint4(a.x, a.y, a.z, a.w);
+        uint32_t w[2];
+        if (fast) enc.encode<true>(raw, w); else enc.encode<false>(raw, w);
+        float f[8];
+        dec.word(w[0], f);
+        dec.word(w[1], f + 4);
+        const uint4 v = Elem<PLANMOE_BF16>::pack(f);
+        // (what is no row, or behind a row's end, stays zero: a code of zero is the row's minimum)
+        return token >= 0 && step * 32 + 8 * g < p.K ? pm_u32x4{v.x, v.y, v.z, v.w} : pm_u32x4{0u, 0u, 0u, 0u};
+    };
+    pm_u32x4 a[U][1];
+    auto ask_rows = [&](int u, int s) { a[u][0] = __builtin_amdgcn_raw_buffer_load_b128(da, s * 32 + 8 * g < p.K ? at : SK_NOWHERE, (uint32_t)s * 64u, 0); };
+    f32x4 acc[1][C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[0][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (wave + u * FIRST_WAVES < steps) ask_rows(u, wave + u * FIRST_WAVES);
+    for (int s0 = wave; s0 < steps; s0 += U * FIRST_WAVES) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int s = s0 + u * FIRST_WAVES, next = s + U * FIRST_WAVES;
+            if (s < steps) {
+                const pm_u32x4 v[1] = {through_codec(a[u][0], s)};
+                b[u].multiply(v, acc);
+            }
+            if (next < steps) {
+                b[u].load(db, place, next, p.N);
+                ask_rows(u, next);
+            }
+        }
+    }
+    skinny_finish<false, 1, C, FIRST_WAVES, false>(p, e, n0, rows, acc, part);
+}
+
+template <int CAP, bool DECODED, int C, int U, bool LARGE>
+static int first_launch(const SkinnyArgs &p, const FirstArgs &r, hipStream_t stream, const char *who)
+{
+    constexpr int COLS = 16 * C, LDS = FIRST_WAVES * 16 * (COLS + 4) * 4;
+    const auto kernel = layer_first_kernel<CAP, DECODED, C, U, LARGE>;
+    static bool ready[64];                       // (per device; setting the attribute twice does no harm)
+    int dev = 0;
+    PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
+    if (dev >= 64 || !ready[dev]) {
+        PM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess,
+                   "%s: the kernel needs %d bytes of LDS", who, LDS);
+        if (dev < 64) ready[dev] = true;
+    }
+    kernel<<<dim3((unsigned)((p.N + COLS - 1) / COLS), (unsigned)p.batches), FIRST_WAVES * 64, LDS, stream>>>(p, r);
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+// Up to 32 tokens (one routing group), 16 experts, 4 choices and 16 rows an expert, and a compute unit for each work-group: a second
+// round of work-groups would route once more.
+static bool first_serves(int dtype, int fp32_gate, int samples, int model_dim, int experts, int top_k, int capacity, int hidden)
+{
+    if (dtype != PLANMOE_BF16 || !fp32_gate || samples > FIRST_TOKENS || experts > 16 || (top_k < experts ? top_k : experts) > 4) return false;
+    if (capacity < 1 || capacity > FIRST_ROWS || (int64_t)hidden * model_dim * 2 >= ((int64_t)1 << 31)) return false;
+    const int width = gemm_skinny_width(false, hidden, model_dim, experts);
+    return (int64_t)((hidden + width - 1) / width) * experts <= compute_units();
+}
+
+} // namespace pm
+
+using namespace pm;
+
+extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int dtype, int fp32_gate, int samples, int model_dim,
+                                              int experts, int top_k, int normalize_gate, int capacity, int codec,
+                                              int32_t *indices, int32_t *locations, void *gates, int64_t plane_stride,
+                                              float *l_aux, int32_t *expert_counts, const void *w1, const void *b1, int hidden,
+                                              int rows_hint, void *rows, void *h, void *workspace, size_t workspace_bytes,
+                                              void *stream)
+{
+    const char *who = "planmoe_layer_dispatch_product";
+    PM_REQUIRE(expert_counts, "%s: NULL routing output", who);
+    const bool shape = x && wg && w1 && h && indices && locations && gates && samples >= 1 && model_dim >= 8 && model_dim % 8 == 0 && experts >= 1 && top_k >= 1 &&
+                       hidden >= 8 && hidden % 8 == 0 && plane_stride >= samples && (codec == 0 || codec == 1) && aligned16(x) && aligned16(wg) && aligned16(w1) && aligned16(h);
+    // (a call that is not well formed goes on to the entry points that say what is wrong with it)
+    if (!shape || !first_serves(dtype, fp32_gate, samples, model_dim, experts, top_k, capacity, hidden)) {
+        if (planmoe_layer_dispatch(x, wg, dtype, fp32_gate, nullptr, samples, model_dim, experts, top_k, normalize_gate, capacity, codec, indices, locations,
+                                   gates, plane_stride, nullptr, l_aux, expert_counts, rows, workspace, workspace_bytes, stream)) return 1;
+        return planmoe_expert_gemm(0, dtype, rows, w1, b1, 1, experts, capacity, hidden, model_dim, expert_counts, top_k < experts ? top_k : experts, 1,
+                                   rows_hint, h, stream);
+    }
+    const SkinnyArgs p{nullptr, (const uint16_t *)w1, (const uint16_t *)b1, nullptr, (uint16_t *)h, nullptr, nullptr, 0, 1, capacity, hidden, model_dim, experts, 1};
+    const FirstArgs r{x, wg, samples, top_k < experts ? top_k : experts, normalize_gate, indices, locations, gates, plane_stride, l_aux, expert_counts};
+    hipStream_t st = (hipStream_t)stream;
+    const int width = gemm_skinny_width(false, hidden, model_dim, experts);
+    const bool large = skinny_large(hidden, model_dim, experts);
+#define PM_FIRST_(C, U, LARGE)                                                                                          \
+    (experts <= 8 ? (codec ? first_launch<8, true, C, U, LARGE>(p, r, st, who) : first_launch<8, false, C, U, LARGE>(p, r, st, who))      \
+                  : (codec ? first_launch<16, true, C, U, LARGE>(p, r, st, who) : first_launch<16, false, C, U, LARGE>(p, r, st, who)))
+#define PM_FIRST(C, U) (large ? PM_FIRST_(C, U, true) : PM_FIRST_(C, U, false))
+    return width == 32 ? PM_FIRST_(2, 8, true) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
+#undef PM_FIRST
+#undef PM_FIRST_
+}

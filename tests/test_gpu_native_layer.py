@@ -478,6 +478,57 @@ def test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec
     assert torch.equal(rows[used].view(bits), want["rows"].view(E * cap, M)[used].view(bits)) and bool((rows[~used] == 7.0).all())
 
 
+# The first product of up to 32 tokens routes them itself: the bits of the dispatch and the product behind it.  Columns of a work-group 32,
+# 64 and 128, read past the caches and not; rows that are no whole steps of the reduction; capacities that drop choices, 16 rows and (two
+# launches) 20; 16 experts, 17 and 33 tokens (two launches); experts without a row
+@pytest.mark.parametrize("T,M,E,k,cap,H", [(1, 8, 1, 1, 4, 8), (3, 64, 4, 2, 4, 200), (5, 1032, 9, 3, 4, 520), (31, 256, 16, 2, 4, 1024), (32, 2048, 8, 2, 12, 136),
+                                           (20, 2056, 4, 2, 16, 1032), (20, 4096, 4, 2, 16, 1032), (8, 1024, 8, 2, 4, 4096), (17, 520, 16, 4, 8, 2040), (32, 264, 8, 2, 16, 4088),
+                                           (30, 64, 2, 2, 20, 64), (33, 256, 16, 2, 8, 264), (8, 64, 17, 1, 4, 64), (4, 4096, 8, 4, 2, 3000)])
+@pytest.mark.parametrize("codec", [0, 1])
+@pytest.mark.parametrize("skewed", [False, True])
+def test_first_product_that_routes_equals_dispatch_and_product(T, M, E, k, cap, H, codec, skewed):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", T, M, E, k, cap, H, codec, skewed, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + M + E)
+    dtype = torch.bfloat16
+    randn = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, wg, w1, b1 = randn(T, M).to(dtype), (randn(E, M) * M ** -0.5).to(dtype), (randn(E, M, H) * M ** -0.5).to(dtype), randn(E, H).to(dtype)
+    if skewed:                                   # everything to the last experts, and values that are not finite
+        wg[:] = torch.arange(E, device=DEV)[:, None] / M
+        x = x.abs()
+        x[T // 2, 1] = float("nan")
+        x[T - 1, 0] = float("inf")
+    else:
+        x[T // 2] = 0.5                          # (a row of one value: no scale)
+        x[0, 0] = -0.0
+    hint = min(cap, (T * k + E - 1) // E)
+    ws = torch.empty(lib.planmoe_forward_workspace_bytes(T, E, k), dtype=torch.uint8, device=DEV)
+
+    def outputs():
+        ints = [torch.full(s, -7, dtype=torch.int32, device=DEV) for s in ((k, T), (k, T), (k, E))]
+        floats = [torch.full((k, T), 7.0, device=DEV), torch.full((), 7.0, device=DEV)]
+        return ints, floats, torch.full((E, cap, M), 7.0, dtype=dtype, device=DEV), torch.full((E, cap, H), 7.0, dtype=dtype, device=DEV)
+
+    ints, floats, rows, h = outputs()
+    check(lib.planmoe_layer_dispatch_product(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), 1, T, M, E, k, 1, cap, codec, ops._ptr(ints[0]), ops._ptr(ints[1]),
+                                             ops._ptr(floats[0]), T, ops._ptr(floats[1]), ops._ptr(ints[2]), ops._ptr(w1), ops._ptr(b1), H, hint, ops._ptr(rows),
+                                             ops._ptr(h), ops._ptr(ws), ws.numel(), ops._stream(x)))
+    want_ints, want_floats, want_rows, want_h = outputs()
+    check(lib.planmoe_layer_dispatch(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), 1, None, T, M, E, k, 1, cap, codec, ops._ptr(want_ints[0]), ops._ptr(want_ints[1]),
+                                     ops._ptr(want_floats[0]), T, None, ops._ptr(want_floats[1]), ops._ptr(want_ints[2]), ops._ptr(want_rows), ops._ptr(ws),
+                                     ws.numel(), ops._stream(x)))
+    ops.expert_gemm("nn", want_rows, w1, b1, relu=True, live=want_ints[2], rows_hint=hint, out=want_h)
+    torch.cuda.synchronize()
+    one = T <= 32 and E <= 16 and cap <= 16      # (then the rows stay where they are)
+    assert bool((rows == 7.0).all()) == one
+    bits = lambda t: t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+    for got, want in zip(ints, want_ints):
+        assert torch.equal(got, want)
+    for got, want in zip(floats + [h], want_floats + [want_h]):
+        assert torch.equal(bits(got), bits(want))
+
+
 # without autograd a pass lies in one buffer: the same bits as the pass that a backward pass may follow, gates in 16 bits among them
 @pytest.mark.parametrize("codec,dtype,fp32_gate", [("no", torch.bfloat16, True), ("no", torch.bfloat16, False), ("int8", torch.bfloat16, False),
                                                    ("int8", torch.float32, True), ("zfp", torch.float32, True), ("no", torch.float32, False)])
