@@ -668,6 +668,12 @@ size_t planmoe_lz_workspace_bytes(int64_t nbytes);
 int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets, int32_t *data_offsets,
                         uint8_t *flags, uint8_t *data, void *workspace, size_t workspace_bytes,
                         void *stream);
+/* The same, and `cleared` (nbytes, 16-byte aligned, no part of the others) set to zero in the first pass: the zeroed twin of the input that
+ * the receive side decodes into (lz.cpp:25). */
+int planmoe_lz_compress_clearing(const void *input, int64_t nbytes, int32_t *flag_offsets, int32_t *data_offsets,
+                                 uint8_t *flags, uint8_t *data, void *cleared, void *workspace,
+                                 size_t workspace_bytes, void *stream);
+
 /* Streams that this coder cannot have written (offsets out of order, a match that reaches
  * before its block) never make the kernel read or write out of bounds; the symbols they cover
  * decode as zero. */

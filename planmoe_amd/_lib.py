@@ -153,6 +153,7 @@ SIGNATURES = {
     "planmoe_lz_workspace_bytes": (c_size_t, [c_int64]),
     "planmoe_lz_compress": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                     c_size_t, c_void_p]),
+    "planmoe_lz_compress_clearing": (c_int, [c_void_p, c_int64] + [c_void_p] * 6 + [c_size_t, c_void_p]),
     "planmoe_lz_decompress": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
 }
 

@@ -139,10 +139,13 @@ torch::Tensor ZfpCompressor::compress(const torch::Tensor &input_)
     AT_ASSERTM(input.scalar_type() == at::kFloat, "zfp: the codec reads the buffer as fp32; pass a float32 tensor");
     const int64_t nx = sizes[2], ny = sizes[1] * sizes[0];
     const size_t bufsize = planmoe_zfp_max_bytes(2, nx, ny, compress_rate);
-    torch::Tensor output = torch::zeros({(int64_t)((bufsize + 1) / 2)}, input.options().dtype(at::kHalf));
+    length = planmoe_zfp_stream_bytes(2, nx, ny, compress_rate);
+    // the coder writes the whole stream: what is cleared is the last word and the slack up to the maximum size (134 MB: 20 us of a pass of 336)
+    torch::Tensor output = torch::empty({(int64_t)((bufsize + 1) / 2)}, input.options().dtype(at::kHalf));
+    const int64_t rest   = std::max<int64_t>((int64_t)length - 8, 0) / 2;
+    output.narrow(0, rest, output.numel() - rest).zero_();
     PM_CALL(planmoe_zfp_compress((const float *)input.data_ptr(), 2, nx, ny, compress_rate, output.data_ptr(),
                                  bufsize, current_stream()));
-    length = planmoe_zfp_stream_bytes(2, nx, ny, compress_rate);
     g_output = torch::empty_like(output);
     return output;
 }
@@ -175,15 +178,15 @@ torch::Tensor LzCompressor::compress(const torch::Tensor &input)
     flagArrGlobal              = at::empty({blocks * 64}, u8);          // the codec zeroes the slack itself
     compressedDataGlobal       = at::empty({blocks * 2048}, u8);
     workspace                  = at::empty({(int64_t)planmoe_lz_workspace_bytes(nbytes)}, u8);
-    PM_CALL(planmoe_lz_compress(x.data_ptr(), nbytes, flagArrOffsetGlobal.data_ptr<int>(),
-                                compressedDataOffsetGlobal.data_ptr<int>(), flagArrGlobal.data_ptr<uint8_t>(),
-                                compressedDataGlobal.data_ptr<uint8_t>(), workspace.data_ptr(),
-                                (size_t)workspace.nbytes(), current_stream()));
+    g_output = at::empty_like(x);
+    PM_CALL(planmoe_lz_compress_clearing(x.data_ptr(), nbytes, flagArrOffsetGlobal.data_ptr<int>(),
+                                         compressedDataOffsetGlobal.data_ptr<int>(), flagArrGlobal.data_ptr<uint8_t>(),
+                                         compressedDataGlobal.data_ptr<uint8_t>(), g_output.data_ptr(), workspace.data_ptr(),
+                                         (size_t)workspace.nbytes(), current_stream()));
     g_flagArrOffsetGlobal        = at::empty_like(flagArrOffsetGlobal);
     g_compressedDataOffsetGlobal = at::empty_like(compressedDataOffsetGlobal);
     g_flagArrGlobal              = at::empty_like(flagArrGlobal);
     g_compressedDataGlobal       = at::empty_like(compressedDataGlobal);
-    g_output                     = at::zeros_like(x);
     return input;
 }
 torch::Tensor LzCompressor::decompress(const torch::Tensor &input)

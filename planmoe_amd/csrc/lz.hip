@@ -304,7 +304,7 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
 // ---- launch 1: sizes and class of every block
 __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
     const uint32_t *__restrict__ in, int64_t nsym, int64_t blocks, int32_t *__restrict__ flag_off,
-    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls, uint4 *__restrict__ tokens)
+    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls, uint4 *__restrict__ tokens, uint32_t *__restrict__ cleared)
 {
     __shared__ __attribute__((aligned(16))) uint32_t keys[LZ_WAVES][LZ_WINDOW + LZ_SYMS];
     const int lane = lane_id();
@@ -313,6 +313,16 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
     if (block >= blocks) return;                       // no work-group barrier below
     uint32_t raw[8];
     lz_load(in, nsym, block, lane, raw);
+    // (a buffer to be cleared along with it: the vector ALUs bound this launch, memory has time; 134 MB of it: a codec pass 163.5 us with a fill
+    // of its own, 153.3)
+    if (cleared) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int64_t at = block * LZ_SYMS + (h * WAVE + lane) * 4;
+            if (at + 4 <= nsym) __builtin_nontemporal_store(pm_u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<pm_u32x4 *>(cleared + at));
+            else for (int64_t i = at; i < nsym; ++i) cleared[i] = 0u;
+        }
+    }
     LzBlock b;
     const int c = lz_analyse(raw, keys[wave], lane, b);
     if (c == LZ_GENERAL) tokens[block * WAVE + lane] = b.tokens();
@@ -764,27 +774,26 @@ extern "C" size_t planmoe_lz_workspace_bytes(int64_t nbytes)
     return lz_tokens_at(blocks) + 16 + (size_t)blocks * LZ_SYMS * 2;       // (the tokens begin at the next 16 bytes)
 }
 
-extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets,
-                                   int32_t *data_offsets, uint8_t *flags, uint8_t *data, void *workspace,
-                                   size_t workspace_bytes, void *stream)
+static int lz_compress_and_clear(const char *who, const void *input, int64_t nbytes, int32_t *flag_offsets, int32_t *data_offsets, uint8_t *flags,
+                                 uint8_t *data, void *workspace, size_t workspace_bytes, void *cleared, void *stream)
 {
-    if (lz_check("planmoe_lz_compress", nbytes)) return 1;
-    PM_REQUIRE(flag_offsets && data_offsets, "planmoe_lz_compress: offset tables must not be NULL");
+    if (lz_check(who, nbytes)) return 1;
+    PM_REQUIRE(flag_offsets && data_offsets, "%s: offset tables must not be NULL", who);
     hipStream_t st = (hipStream_t)stream;
     const int64_t blocks = planmoe_lz_blocks(nbytes);
     if (blocks == 0) {
         fill_u32((uint32_t *)flag_offsets, 1, 0u, st);
         fill_u32((uint32_t *)data_offsets, 1, 0u, st);
-        PM_LAUNCH_CHECK("planmoe_lz_compress");
+        PM_LAUNCH_CHECK(who);
         return 0;
     }
-    PM_REQUIRE(input && flags && data, "planmoe_lz_compress: NULL argument");
+    PM_REQUIRE(input && flags && data, "%s: NULL argument", who);
     PM_REQUIRE(aligned16(input) && aligned16(flags) && aligned16(data) && aligned16(flag_offsets) &&
                aligned16(data_offsets),
-               "planmoe_lz_compress: input, flags, data and the offset tables must be 16-byte aligned");
+               "%s: input, flags, data and the offset tables must be 16-byte aligned", who);
     PM_REQUIRE(workspace && workspace_bytes >= planmoe_lz_workspace_bytes(nbytes) &&
                (reinterpret_cast<uintptr_t>(workspace) & 3u) == 0,
-               "planmoe_lz_compress: workspace too small or not 4-byte aligned");
+               "%s: workspace too small or not 4-byte aligned", who);
     uint8_t *cls = (uint8_t *)workspace;
     uint32_t *totals = (uint32_t *)(cls + lz_class_bytes(blocks));
     uint4 *tokens = (uint4 *)(((uintptr_t)workspace + lz_tokens_at(blocks) + 15) / 16 * 16);
@@ -792,14 +801,30 @@ extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *f
     const int64_t entries = blocks + 1;
     const int chunks = (int)((entries + LZ_SCAN_CHUNK - 1) / LZ_SCAN_CHUNK);      // <= 128 below 2^31 bytes
     lz_sizes_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
-                                                                flag_offsets, data_offsets, cls, tokens);
+                                                                flag_offsets, data_offsets, cls, tokens, (uint32_t *)cleared);
     lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals);
     const int64_t slack_chunks = (blocks * LZ_BLOCK_BYTES / 16 + 255) / 256;          // enough for all of data
     const int64_t clear_groups = min((slack_chunks + 1) / 2, (int64_t)(chunks > 1 ? 2048 : 256));
     lz_place_kernel<<<(unsigned)(groups + clear_groups), LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks, flag_offsets,
                                                                                  data_offsets, cls, totals, chunks, tokens, flags, data);
-    PM_LAUNCH_CHECK("planmoe_lz_compress");
+    PM_LAUNCH_CHECK(who);
     return 0;
+}
+
+extern "C" int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets,
+                                   int32_t *data_offsets, uint8_t *flags, uint8_t *data, void *workspace,
+                                   size_t workspace_bytes, void *stream)
+{
+    return lz_compress_and_clear("planmoe_lz_compress", input, nbytes, flag_offsets, data_offsets, flags, data, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int planmoe_lz_compress_clearing(const void *input, int64_t nbytes, int32_t *flag_offsets,
+                                            int32_t *data_offsets, uint8_t *flags, uint8_t *data, void *cleared,
+                                            void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *who = "planmoe_lz_compress_clearing";
+    PM_REQUIRE((cleared && aligned16(cleared)) || nbytes == 0, "%s: the buffer to clear is NULL or not 16-byte aligned", who);
+    return lz_compress_and_clear(who, input, nbytes, flag_offsets, data_offsets, flags, data, workspace, workspace_bytes, cleared, stream);
 }
 
 extern "C" int planmoe_lz_decompress(void *output, int64_t nbytes, const int32_t *flag_offsets,

@@ -882,14 +882,16 @@ def bwd_gate_zfp(stream, grad_out, indices, locations, experts, capacity_, rate=
 LZ_BLOCK_BYTES = 2048
 
 
-def lz_compress(x, workspace=None):
+def lz_compress(x, workspace=None, cleared=None):
     """x: any contiguous GPU tensor whose byte size is a multiple of 4 (the reference takes fp32).
     Returns the reference's four tensors (gpulz.cu:502-507): flag_offsets, data_offsets int32
     [blocks + 1], flags uint8 [blocks * 64], data uint8 [blocks * 2048]; the byte tensors are zero
     beyond flag_offsets[-1] / data_offsets[-1].  `workspace` (uint8, lz_workspace_bytes) is
-    allocated when not given."""
+    allocated when not given.  `cleared`: a contiguous tensor of x's bytes that is set to zero in the same pass."""
     _need_gpu(x, "lz_compress")
     x = _contig(x, "lz_compress")
+    if cleared is not None and not (cleared.is_contiguous() and cleared.device == x.device and cleared.nbytes == x.nbytes):
+        raise PlanMoEError("lz_compress: what is cleared has to be contiguous, as large as x and on its device")
     nbytes = x.numel() * x.element_size()
     blocks = int(lib.planmoe_lz_blocks(nbytes))
     dev = x.device
@@ -899,6 +901,10 @@ def lz_compress(x, workspace=None):
     data = torch.empty((blocks * LZ_BLOCK_BYTES,), dtype=torch.uint8, device=dev)
     if workspace is None:
         workspace = _ws(lib.planmoe_lz_workspace_bytes(nbytes), dev)
+    if cleared is not None:
+        check(lib.planmoe_lz_compress_clearing(_ptr(x), nbytes, _ptr(flag_offsets), _ptr(data_offsets), _ptr(flags), _ptr(data),
+                                               _ptr(cleared), _ptr(workspace), workspace.numel(), _stream(x)))
+        return flag_offsets, data_offsets, flags, data
     check(lib.planmoe_lz_compress(_ptr(x), nbytes, _ptr(flag_offsets), _ptr(data_offsets), _ptr(flags),
                                   _ptr(data), _ptr(workspace), workspace.numel(), _stream(x)))
     return flag_offsets, data_offsets, flags, data

@@ -641,3 +641,18 @@ def test_combine_zfp_edge_cases():
     stream = ops.zfp_compress(torch.randn(32, 64, device=DEV), 64, 32, 2)
     assert ops.combine_zfp(stream, e, e, None, 0, 4, 8, 64).shape == (0, 64)
     del none
+
+
+# Compressor "zfp" clears only what the coder does not write: a buffer below the line that is cleared as a whole, and above, in memory that was in use
+@pytest.mark.parametrize("shape", [(4, 8, 64), (4, 1028, 1024)])
+def test_zfp_compressor_leaves_zeros_behind_the_stream(shape):
+    from planmoe_amd import compressor, ops
+    n = ops.zfp_max_bytes(2, shape[2], shape[0] * shape[1])
+    assert (n < compressor.ZFP_CLEARED_WHOLE) == (shape[1] == 8)
+    torch.full((n + (1 << 20),), 0x5a, dtype=torch.uint8, device=DEV)              # (given back at once: what the buffer is likely to be made of)
+    x = torch.randn(*shape, device=DEV)
+    codec = compressor.get_compressor("zfp", compressor.get_comm("naive"))
+    sent = codec.compress(x).view(torch.uint8)
+    want = ops.zfp_compress(x, shape[2], shape[0] * shape[1], 2)
+    torch.cuda.synchronize()
+    assert sent.numel() == (n + 1) // 2 * 2 and torch.equal(sent[:n], want) and not sent[codec.length:].any()

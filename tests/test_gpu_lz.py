@@ -235,3 +235,19 @@ def test_tokens_of_every_length_and_offset(nblocks, at):
     got = ops.lz_compress(torch.from_numpy(x).to(DEV), workspace=ws)
     same_streams(got, oracle.lz_compress(x))
     assert bool((whole[:at] == 0xA5).all()) and bool((whole[at + ws.numel():] == 0xA5).all())
+
+
+# the buffer that is cleared in the first pass: whole blocks, a last block of one symbol, of all but one and of no whole vector
+@pytest.mark.parametrize("nsym", [1, 3, 4, 511, 512, 513, 5 * 512 + 6, 300 * 512])
+def test_compress_clears_the_receive_buffer(nsym):
+    from planmoe_amd import ops
+    g = torch.Generator().manual_seed(nsym)
+    x = torch.randint(0, 3, (nsym,), generator=g).float().to(DEV)
+    whole = torch.full((nsym + 64,), 7.0, device=DEV)
+    got = ops.lz_compress(x, cleared=whole[:nsym])
+    want = ops.lz_compress(x)
+    torch.cuda.synchronize()
+    assert not whole[:nsym].any() and bool((whole[nsym:] == 7.0).all())
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with pytest.raises(Exception, match="cleared"):
+        ops.lz_compress(x, cleared=whole)
