@@ -494,6 +494,19 @@ int planmoe_layer_dispatch_product(const void *x, const void *wg, int dtype, int
                                    int rows_hint, void *rows, void *h, void *workspace, size_t workspace_bytes,
                                    void *stream);
 
+/* The experts' second product, rows = h w2 + b2 (planmoe_expert_gemm of h [experts, capacity, hidden], w2 [experts, hidden, model_dim], b2
+ * [experts, model_dim] or NULL, for the rows in use by expert_counts [top_k][experts], rounded up to count_round), and the combine of its rows
+ * (planmoe_layer_combine; codes not NULL: planmoe_layer_combine_keep).  expert_counts are the routing's own: no more than samples * top_k rows
+ * altogether.  `rows` [experts, capacity, model_dim]: with keep_rows it holds the rows that tokens have afterwards (codec 0), else it is scratch.
+ * Workspace: ..._workspace_bytes of the same sizes; 0, and not looked at, where the product is computed whole. */
+size_t planmoe_layer_product_combine_workspace_bytes(int dtype, int codec, int hidden, int top_k, int samples, int model_dim,
+                                                     int experts, int capacity, int rows_hint);
+int planmoe_layer_product_combine(const void *h, const void *w2, const void *b2, int dtype, int codec, int hidden, const float *gates,
+                                  const int32_t *indices, const int32_t *locations, int64_t plane_stride, int top_k, int samples,
+                                  int model_dim, int experts, int capacity, const int32_t *expert_counts, int count_round,
+                                  int rows_hint, void *rows, int keep_rows, uint8_t *codes, void *bias, void *scale, void *out,
+                                  void *workspace, size_t workspace_bytes, void *stream);
+
 /* fast_decode (fast_dispatch.py:203-207) of the experts' rows, each taken through the int8 codec first when
  * codec = 1 (as the receive side's Compress / Decompress pair would, overlap.py:66-74).  Reads only rows that hold a
  * token.  gates NULL: all ones.  model_dim a multiple of 8 (fp32: 4), at most 8192 (fp32: 4096). */

@@ -23,6 +23,11 @@ struct Shape {
     int64_t rows() const { return (int64_t)E * cap; }
     // rows an expert is expected to have in use: what the products pick their tiles by
     int hint() const { return (int)std::min<int64_t>(cap, ((int64_t)T * k + E - 1) / E); }
+    // what the second product leaves for the combine to add up
+    size_t shares(int codec) const
+    {
+        return codec > CODEC_INT8 ? 0 : planmoe_layer_product_combine_workspace_bytes(dt, codec == CODEC_INT8, H, k, T, M, E, cap, hint());
+    }
 };
 
 // which rows of an expert's buffer count: the tokens' own, a zfp block's four rows together, or (lz: the codec
@@ -124,25 +129,31 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     PM_CALL(planmoe_expert_gemm(0, s.dt, p.xe.data_ptr(), w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, live.counts, live.planes, live.round,
                                 s.hint(), p.h.data_ptr(), st));
     p.ye = at::empty({s.rows(), s.M}, x.options());
+    p.y = at::empty({s.T, s.M}, x.options());
+    const Tensor gates = float_gates(p.gates);
+    if (codec == CODEC_NONE || codec == CODEC_INT8) {
+        const size_t shares = s.shares(codec);
+        ws = shares ? bytes((int64_t)shares, x) : Tensor();
+        Kept kept;
+        if (codec == CODEC_INT8 && keep) {
+            // (the backward pass reads the codes: a byte a value is held until then, as between Compress and its backward)
+            p.codes = bytes(Kept::bytes(s, x.element_size()), x);
+            kept = Kept(p.codes, s, x.element_size());
+        }
+        PM_CALL(planmoe_layer_product_combine(p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, floats(gates), idx, loc, s.T, s.k, s.T,
+                                              s.M, s.E, s.cap, cnt, 1, s.hint(), p.ye.data_ptr(), keep, kept.codes, kept.bias, kept.scale, p.y.data_ptr(),
+                                              raw(ws), shares, st));
+        if (p.codes.defined()) p.ye = Tensor();
+        return p;
+    }
     PM_CALL(planmoe_expert_gemm(0, s.dt, p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
                                 s.hint(), p.ye.data_ptr(), st));
-    const Tensor gates = float_gates(p.gates);
     if (codec == CODEC_ZFP) {
         if (keep) p.stream = zfp_stream(s, x);
         zfp_rows(p.ye, p.stream, p, s, st);
     }
     if (codec == CODEC_LZ) p.ye = lz_round_trip(p.ye, st);
-    p.y = at::empty({s.T, s.M}, x.options());
-    if (codec == CODEC_INT8 && keep) {
-        // (the backward pass reads the codes: a byte a value is held until then, as between Compress and its backward)
-        p.codes = bytes(Kept::bytes(s, x.element_size()), x);
-        const Kept kept(p.codes, s, x.element_size());
-        PM_CALL(planmoe_layer_combine_keep(p.ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), kept.codes,
-                                           kept.bias, kept.scale, st));
-        p.ye = Tensor();
-        return p;
-    }
-    PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, codec == CODEC_INT8, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
+    PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, 0, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
     if (p.stream.defined()) p.ye = Tensor();         // (the backward pass reads the stream)
     return p;
 }
@@ -162,6 +173,8 @@ std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, con
     const int64_t idx_at = piece((int64_t)s.k * s.T * 4), loc_at = piece((int64_t)s.k * s.T * 4), cnt_at = piece((int64_t)s.k * s.E * 4),
                   gates_at = piece((int64_t)s.k * s.T * (bf16_gate ? size : 4)), wide_at = bf16_gate ? piece((int64_t)s.k * s.T * 4) : 0,
                   ws_at = piece((int64_t)ws_bytes), xe_at = piece(s.rows() * s.M * size), h_at = piece(s.rows() * s.H * size), ye_at = piece(s.rows() * s.M * size);
+    const size_t shares = s.shares(codec);
+    const int64_t shares_at = piece((int64_t)shares);
     const Tensor pool = bytes(end, x);
     uint8_t *const base = pool.data_ptr<uint8_t>();
     int32_t *const idx = (int32_t *)(base + idx_at), *const loc = (int32_t *)(base + loc_at), *const cnt = (int32_t *)(base + cnt_at);
@@ -180,11 +193,15 @@ std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, con
         at::from_blob(base + wide_at, {s.k, s.T}, x.options().dtype(at::kFloat)).copy_(at::from_blob(base + gates_at, {s.k, s.T}, x.options()));
         gates = (const float *)(base + wide_at);
     }
-    const int round = codec == CODEC_ZFP ? 4 : 1;
-    if (codec == CODEC_ZFP) PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, round, s.hint(), h, st));
-    PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, round, s.hint(), ye, st));
-    if (codec == CODEC_ZFP) PM_CALL(planmoe_layer_zfp_rows((float *)ye, s.M, s.E, s.cap, cnt, s.k, nullptr, 0, st));
-    PM_CALL(planmoe_layer_combine(ye, s.dt, codec == CODEC_INT8, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));
+    if (codec != CODEC_ZFP) {
+        PM_CALL(planmoe_layer_product_combine(h, w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt,
+                                              1, s.hint(), ye, 0, nullptr, nullptr, nullptr, y.data_ptr(), base + shares_at, shares, st));
+        return {y, l_aux};
+    }
+    PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, 4, s.hint(), h, st));
+    PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, 4, s.hint(), ye, st));
+    PM_CALL(planmoe_layer_zfp_rows((float *)ye, s.M, s.E, s.cap, cnt, s.k, nullptr, 0, st));
+    PM_CALL(planmoe_layer_combine(ye, s.dt, 0, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));
     return {y, l_aux};
 }
 

@@ -13,7 +13,7 @@
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
 #include "gemm_deep.hpp"
-#include "gemm_skinny.hpp"
+#include "gemm_shares.hpp"
 #include "sums.hpp"
 #include <algorithm>
 #include <cmath>
@@ -765,6 +765,44 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
     p.split = 2;
     return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
 }
+
+}  // namespace
+
+// In shares (layer_shares.hip): where the work-groups that the weight's columns make, for the experts that can have rows, leave half of the compute
+// units without one.  Up to 32 rows 64 columns (whole lines of 128 bytes) and shares of at least 512 k, 16 steps for 16 waves; beyond, tiles of
+// 128 x 128 and shares of at least 4 k-tiles.  Up to eight: the combine reads them all.
+// us whole and in shares (the combine apart), weights cold:
+//   8 experts x 2 rows, 4096 -> 1024     19.3 -> 13.8 (2 shares)      8 x 16, same      23.3 -> 16.4 (2)
+//   8 x 32, same                         37.5 -> 17.9 (4)             8 x 64, same      41.2 -> 19.4 (4)       8 x 128, same  43.9 -> 27.7 (2)
+//   8 x 32, 2048 -> 2048                 25.2 -> 17.5 (2)             4 x 32, 2048 -> 512   14.7 -> 6.0 (8)    4 x 512, same  17.3 -> 12.8 (3)
+//   2 of 8 experts with a row, 4096 -> 4096  26.5 -> 13.6 (2)         4096 -> 1024, same    16.8 -> 4.8 (8)
+GemmShares pm::gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs)
+{
+    const int64_t cu = compute_units();
+    const int active = (int)std::min<int64_t>(batches, pairs);
+    if (n * k * 2 >= ((int64_t)1 << 31) || batches > 64) return GemmShares{};
+    if (gemm_is_skinny(false, m, n, k, batches)) {
+        const int64_t groups = (int64_t)((n + 63) / 64) * active, splits = std::min<int64_t>({groups > 0 ? cu / groups : 0, k / 512, 8});
+        // (one share: where fewer experts than there are have rows, and the whole product would take them in wider columns)
+        if (splits >= 2 || (splits == 1 && active < batches && gemm_skinny_width(false, n, k, batches) > 64)) return GemmShares{(int)splits, active, true};
+        return GemmShares{};
+    }
+    if (!gemm_deep_reaches(0, m, n, k)) return GemmShares{};
+    const double tiles = GemmCost{(double)std::min<int64_t>(rows, m), 0., (double)cu, m, n, batches, 0, true}.tiles(128, 128);
+    const int64_t k_tiles = (k + DEEP_BK - 1) / DEEP_BK, splits = std::min<int64_t>({(int64_t)((double)cu / tiles), k_tiles / 4, 8});
+    if (splits < 2) return GemmShares{};
+    const int64_t each = (k_tiles + splits - 1) / splits;
+    return GemmShares{(int)((k_tiles + each - 1) / each), active, false};      // (none of them empty)
+}
+
+int pm::gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who)
+{
+    p.splits = how.splits;
+    p.active = how.active;
+    return how.few ? gemm_skinny_shares_run(p, stream, who) : gemm_deep_shares_run(p, stream, who);
+}
+
+namespace {
 
 // what the buffer descriptors cover: from a tile's corner, a tile of a k-fast operand and 64 rows of a k-slow one
 bool gemm_pitch_fits(int ld) { return (int64_t)ld * 2 * 256 < ((int64_t)1 << 31); }

@@ -16,7 +16,7 @@ typedef short dp_s16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dp_u32x4 __attribute__((ext_vector_type(4)));
 typedef const uint8_t __attribute__((address_space(3))) *dp_lds;
 
-constexpr int DP_BK = 64, DP_SIDE = 128, DP_STAGES = 4, DP_OPERAND = DP_SIDE * DP_BK * 2, DP_LDS = 2 * DP_STAGES * DP_OPERAND;
+constexpr int DP_BK = DEEP_BK, DP_SIDE = 128, DP_STAGES = 4, DP_OPERAND = DP_SIDE * DP_BK * 2, DP_LDS = 2 * DP_STAGES * DP_OPERAND;
 
 // (ds_read_b64_tr_b16 hands a lane four consecutive k of its column, see gemm.hip)
 __device__ __forceinline__ dp_bf16x8 dp_read_tr(dp_lds lo, dp_lds hi)
@@ -26,7 +26,8 @@ __device__ __forceinline__ dp_bf16x8 dp_read_tr(dp_lds lo, dp_lds hi)
     return __builtin_bit_cast(dp_bf16x8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <bool TA, bool TB, bool GRAD>
+// SHARES: of the work-groups of a tile each takes a share of the k-tiles and leaves its sums, in fp32, in a plane of its own
+template <bool TA, bool TB, bool GRAD, bool SHARES = false>
 __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
 {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -37,9 +38,14 @@ __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
 
     // XCD j (work-groups j, j + 8, ...) takes the j-th eighth of the tiles: batch, panel of 8 columns, row, column
     const int tiles_m = (p.M + DP_SIDE - 1) / DP_SIDE, tiles_n = (p.N + DP_SIDE - 1) / DP_SIDE;
-    const int total = tiles_m * tiles_n * p.batches, per_xcd = (total + 7) / 8;
-    const int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
+    const int total = tiles_m * tiles_n * p.batches * (SHARES ? p.splits : 1), per_xcd = (total + 7) / 8;
+    int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8, share = 0;
     if (blockIdx.x / 8 >= per_xcd || tile >= total) return;
+    if (SHARES) {                                // (the share before the tile: an XCD's work-groups are at the same k)
+        const int tiles = tiles_m * tiles_n * p.batches;
+        share = tile / tiles;
+        tile -= share * tiles;
+    }
     const int e = tile / (tiles_m * tiles_n);
     int in = tile - e * tiles_m * tiles_n;
     const int panel = in / (tiles_m * 8);
@@ -58,6 +64,12 @@ __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
     const int lda = TA ? p.M : p.K, ldb = TB ? p.N : p.K;
     const uint16_t *A = p.A + (int64_t)e * p.M * p.K + (TA ? (int64_t)m0 : (int64_t)m0 * lda);
     const uint16_t *B = p.B + (int64_t)e * p.N * p.K + (TB ? (int64_t)n0 : (int64_t)n0 * ldb);
+    if (SHARES) {
+        const int each = ((K + DP_BK - 1) / DP_BK + p.splits - 1) / p.splits * DP_BK, k0 = min(share * each, K);
+        A += TA ? (int64_t)k0 * lda : k0;
+        B += TB ? (int64_t)k0 * ldb : k0;
+        K = min(each, K - k0);
+    }
     auto desc = [](const void *base, int64_t bytes) {
         const uint64_t a = (uint64_t)base;
         return dp_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes <= 0 ? 0u : bytes > 0x7fffffff ? 0x7fffffffu : (uint32_t)bytes, 0x00020000u};
@@ -158,6 +170,24 @@ __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
     }
 
     // ---- a lane has row fr of fragment i, columns 8 q + 4 fc .. + 3 of fragment j in acc[i][j][4 q ..]
+    if constexpr (SHARES) {
+        float *plane = p.shares + ((int64_t)(share * p.batches + e) * p.M + m0) * p.N + n0;
+        const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(plane, 0, (int)min((int64_t)0x7fffffff, ((int64_t)(M - m0 - 1) * p.N + (p.N - n0)) * 4), 0x00020000);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = 64 * wn + 32 * j + 8 * q + 4 * fc;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int row = 64 * wm + 32 * i + fr;
+                    const pm_u32x4 v = {__float_as_uint(acc[i][j][4 * q]), __float_as_uint(acc[i][j][4 * q + 1]), __float_as_uint(acc[i][j][4 * q + 2]), __float_as_uint(acc[i][j][4 * q + 3])};
+                    __builtin_amdgcn_raw_buffer_store_b128(v, to, n0 + col < p.N ? ((uint32_t)row * (uint32_t)p.N + (uint32_t)col) * 4u : NOWHERE, 0, 0);
+                }
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
     const int64_t corner = (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0;
     const int bytes = (int)min((int64_t)0x7fffffff, ((int64_t)(M - m0 - 1) * p.N + (p.N - n0)) * 2);
     const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.C + corner, 0, bytes, 0x00020000);
@@ -211,10 +241,10 @@ __global__ __launch_bounds__(256, 1) void gemm_deep_kernel(const SkinnyArgs p)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <bool TA, bool TB, bool GRAD>
+template <bool TA, bool TB, bool GRAD, bool SHARES = false>
 static int deep_launch(const SkinnyArgs &p, hipStream_t stream, const char *who)
 {
-    const auto kernel = gemm_deep_kernel<TA, TB, GRAD>;
+    const auto kernel = gemm_deep_kernel<TA, TB, GRAD, SHARES>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -223,12 +253,14 @@ static int deep_launch(const SkinnyArgs &p, hipStream_t stream, const char *who)
                    "%s: the kernel needs %d bytes of LDS", who, DP_LDS);
         if (dev < 64) ready[dev] = true;
     }
-    const int64_t tiles = ((int64_t)p.M + DP_SIDE - 1) / DP_SIDE * (((int64_t)p.N + DP_SIDE - 1) / DP_SIDE) * p.batches;
+    const int64_t tiles = ((int64_t)p.M + DP_SIDE - 1) / DP_SIDE * (((int64_t)p.N + DP_SIDE - 1) / DP_SIDE) * p.batches * (SHARES ? p.splits : 1);
     PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
     kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, DP_LDS, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
+
+int gemm_deep_shares_run(const SkinnyArgs &p, hipStream_t stream, const char *who) { return deep_launch<false, true, false, true>(p, stream, who); }
 
 bool gemm_deep_reaches(int form, int m, int n, int64_t k)
 {

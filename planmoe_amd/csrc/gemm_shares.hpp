@@ -1,0 +1,18 @@
+// A product of the experts (bf16, nn) whose sums are left in shares of the reduction for the launch that reads them next.
+#pragma once
+#include "gemm_skinny.hpp"
+
+namespace pm {
+
+struct GemmShares {
+    int splits = 0;               // 0: the product is computed whole
+    int active = 0;               // the most batches that have rows
+    bool few = false;             // gemm_skinny.hip's kernel, else gemm_deep.hip's
+};
+
+// m, n, k: rows at most of a batch, columns, reduction; rows: expected of a batch; pairs: rows of all batches at most
+GemmShares gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs);
+// p.shares, p.live and at most 64 batches; the caller has checked shape and alignment (as planmoe_expert_gemm does)
+int gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who);
+
+} // namespace pm

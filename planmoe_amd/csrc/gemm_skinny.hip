@@ -19,15 +19,28 @@ namespace pm {
 
 // MF: 16-row fragments; C: 16-column fragments of the weight, a work-group's columns / 16; U: steps of the reduction a wave has in flight;
 // LARGE: the weight does not stay in the caches anyway (skinny_large): read nontemporally (nt: not, the two loads of 128 bytes meet in the cache)
-template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
+// SHARES: a grid of (column groups, batches that can have rows, shares of the reduction); the y-th batch is the y-th that has rows
+template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE, bool SHARES = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArgs p)
 {
     extern __shared__ __align__(16) float part[];           // [WAVES][16][16 C + 4]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int e, n0;
-    skinny_tile<16 * C, LARGE && C == 2>(e, n0);
-    int rows = p.M;
-    if (p.live) {
+    int e, n0, rows = p.M;
+    if constexpr (SHARES) {
+        int n = 0;
+        if (lane < p.batches)
+            for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + lane];
+        n = min(p.M, (n + p.live_round - 1) / p.live_round * p.live_round);
+        uint64_t used = __ballot(n > 0);
+        if ((int)blockIdx.y >= __popcll(used)) return;
+        for (int y = blockIdx.y; y > 0; --y) used &= used - 1;
+        e = __builtin_ctzll(used);
+        rows = __builtin_amdgcn_readlane(n, e);
+        n0 = blockIdx.x * 16 * C;
+    } else {
+        skinny_tile<16 * C, LARGE && C == 2>(e, n0);
+    }
+    if (!SHARES && p.live) {
         int n = 0;
         for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
         rows = min(p.M, (n + p.live_round - 1) / p.live_round * p.live_round);
@@ -48,14 +61,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         for (int c = 0; c < C; ++c) acc[m][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     constexpr int KS = NT ? 64 : 32;                        // k of a step
-    const int steps = (p.K + KS - 1) / KS;
+    int steps = (p.K + KS - 1) / KS, first = wave;          // of this wave: first, first + WAVES, .. below steps
+    if constexpr (SHARES) {
+        const int each = (steps + p.splits - 1) / p.splits;
+        first += blockIdx.z * each;
+        steps = min(steps, (int)(blockIdx.z + 1) * each);
+    }
     const uint32_t place = n0 + C * l16 < p.N ? ((uint32_t)(8 * g) * (uint32_t)p.N + (uint32_t)(n0 + C * l16)) * 2u : NOWHERE;    // (nn)
     // U steps of the wave are on their way: a step's loads go out as soon as the registers of the step U before it are free
     auto walk = [&](auto load, auto use) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (wave + u * WAVES < steps) load(u, wave + u * WAVES);
-        for (int s0 = wave; s0 < steps; s0 += U * WAVES) {
+            if (first + u * WAVES < steps) load(u, first + u * WAVES);
+        for (int s0 = first; s0 < steps; s0 += U * WAVES) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (s0 + u * WAVES < steps) use(u);
@@ -100,14 +118,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         });
     }
 
-    skinny_finish<NT, MF, C, WAVES, GRAD>(p, e, n0, rows, acc, part);
+    skinny_finish<NT, MF, C, WAVES, GRAD, SHARES>(p, e, n0, rows, acc, part);
 }
 
-template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE>
+template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE, bool SHARES = false>
 static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *who)
 {
     constexpr int COLS = 16 * C, LDS = WAVES * 16 * (COLS + 4) * 4;
-    const auto kernel = gemm_skinny_kernel<NT, MF, C, U, WAVES, GRAD, LARGE>;
+    const auto kernel = gemm_skinny_kernel<NT, MF, C, U, WAVES, GRAD, LARGE, SHARES>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -116,7 +134,7 @@ static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *wh
                    "%s: the kernel needs %d bytes of LDS", who, LDS);
         if (dev < 64) ready[dev] = true;
     }
-    kernel<<<dim3((unsigned)((p.N + COLS - 1) / COLS), (unsigned)p.batches), WAVES * 64, LDS, stream>>>(p);
+    kernel<<<dim3((unsigned)((p.N + COLS - 1) / COLS), (unsigned)(SHARES ? p.active : p.batches), (unsigned)(SHARES ? p.splits : 1)), WAVES * 64, LDS, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -161,6 +179,13 @@ int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
     }
 #undef PM_SK_NN
 #undef PM_SK_NT
+}
+
+int gemm_skinny_shares_run(const SkinnyArgs &p, hipStream_t stream, const char *who)
+{
+    const bool large = skinny_large(p.N, p.K, p.active);
+    if (p.M <= 16) return large ? skinny_launch<false, 1, 4, 2, 16, false, true, true>(p, stream, who) : skinny_launch<false, 1, 4, 2, 16, false, false, true>(p, stream, who);
+    return large ? skinny_launch<false, 2, 4, 2, 16, false, true, true>(p, stream, who) : skinny_launch<false, 2, 4, 2, 16, false, false, true>(p, stream, who);
 }
 
 int gemm_skinny_width(bool nt, int n, int64_t k, int batches)

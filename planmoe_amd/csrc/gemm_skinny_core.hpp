@@ -58,7 +58,8 @@ struct SkinnyWeights {
     }
 };
 
-template <bool NT, int MF, int C, int WAVES, bool GRAD>
+// SHARES: the sums as they are, into this work-group's share
+template <bool NT, int MF, int C, int WAVES, bool GRAD, bool SHARES = false>
 __device__ __forceinline__ void skinny_finish(const SkinnyArgs &p, int e, int n0, int rows, const f32x4 (&acc)[MF][C], float *part)
 {
     constexpr int SK_COLS = 16 * C, SK_PITCH = SK_COLS + 4;             // (floats between rows of a wave's sums in LDS)
@@ -96,6 +97,11 @@ __device__ __forceinline__ void skinny_finish(const SkinnyArgs &p, int e, int n0
             for (int x = 0; x < PER; ++x) v[x] += part[(w * 16 + row_t) * SK_PITCH + col_t + x];
         const int row = 16 * m + row_t, col = n0 + col_t;
         const bool inside = writes && row < rows && col < p.N;        // (N is a multiple of 8: a thread's columns are in or out together)
+        if constexpr (SHARES) {
+            static_assert(!SHARES || PER == 1, "64 columns, 16 waves");
+            if (inside) p.shares[((int64_t)(blockIdx.z * p.batches + e) * p.M + row) * p.N + col] = v[0];
+            continue;
+        }
 #pragma unroll
         for (int x = 0; x < PER; ++x) {
             v[x] = bf16_to_f32(f32_to_bf16(v[x]));

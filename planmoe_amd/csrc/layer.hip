@@ -10,6 +10,7 @@
 #include "rows.hpp"
 #include "int8_core.hpp"
 #include "layer_rows.hpp"
+#include "layer_shares.hpp"
 #include "route_bwd.hpp"
 
 #include <type_traits>
@@ -22,12 +23,12 @@ namespace pm {
 // registers and left two waves per SIMD).  16384 x 4096 bf16, top-2, 403 MB: 81 us = 5.0 TB/s.  More than two
 // choices keep their sum in fp32.  KEEP: the rows' codes, minima and scales are stored as well, by slot (what a backward
 // pass reads in place of the rows: a byte a value to hold between the passes; 16384 x 1024 bf16, top-2: 26.5 -> 32 us, and the
-// backward pass 48 -> 38).
-template <int DT, int CACHE, bool TWO, bool KEEP>
+// backward pass 48 -> 38).  SHARES: bf16 rows that the product left in shares; `rows` is not read.
+template <int DT, int CACHE, bool TWO, bool KEEP, bool SHARES = false>
 __global__ __launch_bounds__(256) void layer_combine_kernel(
     const void *__restrict__ rows, const float *__restrict__ gates, const int32_t *__restrict__ indices,
     const int32_t *__restrict__ locations, int64_t stride, int top_k, int samples, int model_dim, int capacity,
-    void *__restrict__ out, uint8_t *__restrict__ codes, void *__restrict__ bias, void *__restrict__ scales)
+    void *__restrict__ out, uint8_t *__restrict__ codes, void *__restrict__ bias, void *__restrict__ scales, const RowShares shares = RowShares{})
 {
     using E = Elem<DT>;
     constexpr int V = E::VEC;
@@ -38,6 +39,11 @@ __global__ __launch_bounds__(256) void layer_combine_kernel(
     const int64_t row_bytes = (int64_t)model_dim * (int64_t)sizeof(typename E::store_t);
     uint4 *dst = reinterpret_cast<uint4 *>((char *)out + (int64_t)t * row_bytes);
     auto request = [&](int s, uint4 (&r)[CACHE]) {
+        if constexpr (SHARES) {
+#pragma unroll
+            for (int c = 0; c < CACHE; ++c) r[c] = shares.vector(max(s, 0), min(c * WAVE + lane, units - 1));
+            return;
+        }
         const uint4 *src = reinterpret_cast<const uint4 *>((const char *)rows + (int64_t)max(s, 0) * row_bytes);
 #pragma unroll
         for (int c = 0; c < CACHE; ++c) r[c] = src[min(c * WAVE + lane, units - 1)];
@@ -300,6 +306,27 @@ static int combine_int8_rows(const char *who, const void *rows, int dtype, const
     PM_DTYPE_SWITCH(dtype, DT, PM_ROW_CACHE(PM_LC));
 #undef PM_LC
 #undef PM_LC_
+    PM_LAUNCH_CHECK(who);
+    return 0;
+}
+
+int pm::combine_int8_shares(const char *who, const RowShares &rows, const float *gates, const int32_t *indices, const int32_t *locations, int64_t plane_stride,
+                            int top_k, int samples, void *out, uint8_t *codes, void *bias, void *scale, hipStream_t st)
+{
+    const int per_lane = (rows.model_dim / 8 + WAVE - 1) / WAVE;
+#define PM_LS_(CACHE, TWO, KEEP) (layer_combine_kernel<PLANMOE_BF16, CACHE, TWO, KEEP, true><<<(samples + 3) / 4, 256, 0, st>>>(nullptr, gates, indices, locations, \
+        plane_stride, top_k, samples, rows.model_dim, rows.capacity, out, codes, bias, scale, rows))
+#define PM_LS(CACHE)                                                                          \
+    do {                                                                                      \
+        if (top_k <= 2) { if (codes) PM_LS_(CACHE, true, true); else PM_LS_(CACHE, true, false); }     \
+        else { if (codes) PM_LS_(CACHE, false, true); else PM_LS_(CACHE, false, false); }     \
+    } while (0)
+    if (per_lane <= 1) PM_LS(1);
+    else if (per_lane <= 2) PM_LS(2);
+    else if (per_lane <= 4) PM_LS(4);
+    else PM_LS(8);
+#undef PM_LS
+#undef PM_LS_
     PM_LAUNCH_CHECK(who);
     return 0;
 }

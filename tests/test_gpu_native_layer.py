@@ -666,3 +666,64 @@ def test_layer_with_tokens_that_are_not_finite(native, T, E, k, codec, dtype):
         assert bool(y[lost].isnan().any())
         if codec in ("no", "int8"):               # (a block of the other codecs holds rows of several tokens)
             assert torch.equal(y[~lost], outs[0][0][~lost]) and bool(y[~lost].isfinite().all()) and torch.equal(dx[~lost], outs[0][1][~lost])
+
+
+# The second product left in shares of its reduction, which the combine adds.  Rows against 64 bits: the sum and the biased sum are each rounded to
+# bf16 (2^-9 of them), the fp32 sums before it are off by at most H 2^-23 of the sum of magnitudes; everything behind the rows against the general
+# path on those rows, bit for bit.  Few rows (up to 16, up to 32) and tiles; fewer pairs than experts, one share; a last share that is shorter;
+# columns that are no whole tiles; one, two and three choices; capacities that drop; rows of 520 and 4096 values; an expert without a row.
+@pytest.mark.parametrize("T,M,H,E,k,cap,skewed", [
+    (1, 4096, 1024, 8, 2, 4, False), (2, 4096, 1024, 8, 2, 4, False), (1, 1032, 2056, 8, 1, 4, False), (8, 1024, 4096, 8, 2, 4, True), (7, 520, 1032, 4, 3, 16, False),
+    (30, 264, 2048, 4, 2, 24, True), (60, 520, 1032, 4, 2, 40, False), (200, 1024, 4096, 8, 2, 64, True), (333, 136, 520, 3, 3, 129, True),
+    (150, 4096, 576, 1, 1, 140, False), (90, 1000, 2000, 2, 1, 64, False)])
+@pytest.mark.parametrize("with_bias", [True, False])
+def test_product_in_shares_and_combine(T, M, H, E, k, cap, skewed, with_bias):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    print("case", T, M, H, E, k, cap, skewed, with_bias, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + M + E)
+    randn = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    scores = randn(T, E)
+    if skewed:
+        scores[:, E - 1] += 3.0
+        scores[:, 0] -= 9.0
+    routed = ops.route_topk(torch.softmax(scores, 1), k)
+    idx, loc, gates = routed["indices"].view(k, T), routed["locations"].view(k, T), routed["gates"].view(k, T).float()
+    counts = torch.stack([torch.bincount(idx[j].long(), minlength=E) for j in range(k)]).int()
+    h, w2 = randn(E, cap, H).bfloat16(), (randn(E, H, M) * H ** -0.5).bfloat16()
+    b2 = randn(E, M).bfloat16() if with_bias else None
+    hint = min(cap, (T * k + E - 1) // E)
+    p, dt, st = ops._ptr, ops._dt(h, "t"), ops._stream(h)
+
+    def run(codec, keep_rows, keep_codes):
+        rows, out = torch.full((E, cap, M), 7.0, dtype=torch.bfloat16, device=DEV), torch.full((T, M), 7.0, dtype=torch.bfloat16, device=DEV)
+        codes, mn, scale = (torch.zeros(E, cap, M, dtype=torch.uint8, device=DEV), torch.zeros(E, cap, dtype=torch.bfloat16, device=DEV),
+                            torch.zeros(E, cap, dtype=torch.bfloat16, device=DEV)) if keep_codes else (None, None, None)
+        size = lib.planmoe_layer_product_combine_workspace_bytes(dt, codec, H, k, T, M, E, cap, hint)
+        assert size > 0 and size % (E * cap * M * 4) == 0
+        ws = torch.full((size // 4,), float("nan"), device=DEV)
+        check(lib.planmoe_layer_product_combine(p(h), p(w2), p(b2), dt, codec, H, p(gates), p(idx), p(loc), T, k, T, M, E, cap, p(counts), 1, hint, p(rows),
+                                                int(keep_rows), p(codes), p(mn), p(scale), p(out), p(ws), size, st))
+        return rows, out, codes, mn, scale
+
+    rows, out = run(0, True, False)[:2]
+    alone, again = run(0, False, False)[:2]
+    torch.cuda.synchronize()
+    bits = lambda t: t.view(torch.int16)
+    assert torch.equal(bits(out), bits(again)) and bool((alone == 7.0).all())
+    used = (torch.arange(cap, device=DEV)[None] < counts.sum(0)[:, None])
+    assert bool((rows[~used] == 7.0).all())
+    exact = h.double() @ w2.double()
+    size = h.double().abs() @ w2.double().abs()
+    want = exact + (b2.double()[:, None] if with_bias else 0.0)
+    bound = exact.abs() * 2.0 ** -8 + want.abs() * 2.0 ** -8 + size * H * 2.0 ** -23 + 1e-30
+    assert bool(((rows.double() - want).abs() <= bound)[used].all())
+    check(lib.planmoe_layer_combine(p(rows), dt, 0, p(gates), p(idx), p(loc), T, k, T, M, E, cap, p(again), st))
+    assert torch.equal(bits(out), bits(again))
+    _, out8, codes, mn, scale = run(1, False, True)
+    plain8 = run(1, False, False)[1]
+    want_codes, want_mn, want_scale = torch.zeros_like(codes), torch.zeros_like(mn), torch.zeros_like(scale)
+    check(lib.planmoe_layer_combine_keep(p(rows), dt, p(gates), p(idx), p(loc), T, k, T, M, E, cap, p(again), p(want_codes), p(want_mn), p(want_scale), st))
+    torch.cuda.synchronize()
+    assert torch.equal(bits(out8), bits(again)) and torch.equal(bits(plain8), bits(again))
+    assert torch.equal(codes, want_codes) and torch.equal(mn, want_mn) and torch.equal(scale, want_scale)
