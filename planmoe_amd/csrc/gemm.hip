@@ -704,9 +704,16 @@ bool gemm_is_skinny(bool nt, int m, int n, int64_t k, int batches)
 // tile more than expected, and two of these work-groups do not fit on a compute unit.  us in gemm_bf16_kernel's 128 x 128 tiles and here, weights cold, in cache:
 //   8 experts x 80 rows, 4096 -> 1024    43, 33 and 41, 25      8 x 80, 1024 -> 512     13, 13 and 9, 9
 //   8 x 110, 2696 -> 2488                39, 32 and 37, 29      a^T b, 4 x 512 x 768 over 2000 rows    20 and 15
+// In 64 columns where that leaves a compute unit for each tile still: half of the weight for each, and five k-tiles on their way instead of four.
+// us in 128 and 64 columns, weights cold, nn and nt:
+//   8 x 32 rows, 4096 -> 1024            35.6, 26.8 and 34.3, 24.1      8 x 128, same            42.1, 34.9 and 39.5, 29.4
+//   8 x 32, 2048 -> 2048                 23.7, 17.6 and 21.5, 18.1      16 x 64, 1024 -> 1024    14.0, 11.6 and 13.1, 10.1
+//   4 x 64, 512 -> 2048                  8.8, 7.1 and 8.6, 6.6          4 x 256, 2048 -> 512     22.9, 18.0 and 21.2, 15.6
+//   4 x 64, 4096 -> 4096                 40.0, 32.6 and 41.6, 32.6      a^T b, 4 x 512 x 768 over 256 rows    6.7, 5.4
+// (four k-tiles: 8 x 32, 4096 -> 1024 30.9 and 29.7; six: the same as five there, 4 x 64, 4096 -> 4096 37.3)
 bool gemm_is_deep(double tiles, int m) { return tiles <= 0.8 * compute_units() || (m <= 128 && tiles <= compute_units()); }
 
-enum GemmKernel { GEMM_SKINNY, GEMM_DEEP, GEMM_128, GEMM_LOW_128, GEMM_LOW_160, GEMM_LOW_192, GEMM_256, GEMM_256_QUARTERS };
+enum GemmKernel { GEMM_SKINNY, GEMM_DEEP, GEMM_DEEP_64, GEMM_128, GEMM_LOW_128, GEMM_LOW_160, GEMM_LOW_192, GEMM_256, GEMM_256_QUARTERS };
 
 // form: 0 nn, 1 nt, 2 tn; contiguous: the operands and the result are; rows: expected of a batch (tn: of its reduction)
 GemmKernel gemm_pick(int form, bool contiguous, int m, int n, int k, int batches, bool counted, int64_t rows)
@@ -716,13 +723,14 @@ GemmKernel gemm_pick(int form, bool contiguous, int m, int n, int k, int batches
     const GemmCost cost{(double)(tn ? m : rows), (double)(((tn ? rows : k) + 63) / 64), (double)compute_units(), m, n, batches,
                         tn ? 0 : (int64_t)n * k * batches * 2, !tn && counted};
     const bool deep = contiguous && gemm_is_deep(cost.tiles(128, 128), m) && gemm_deep_reaches(form, m, n, k);
-    const double small = (deep ? 0.88 : 1.) * cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
+    const bool narrow = deep && gemm_is_deep(cost.tiles(128, 64), m);
+    const double small = (narrow ? 0.72 : deep ? 0.88 : 1.) * cost.small(), split = cost.big_and_quarters(), big = std::min(cost.big(), split);
     if (!tn) {
         const double low[3] = {cost.low(128), cost.low(160), cost.low(192)};
         const int f = low[0] <= low[1] && low[0] <= low[2] ? 0 : low[1] <= low[2] ? 1 : 2;
         if (low[f] < small && low[f] < big) return f == 0 ? GEMM_LOW_128 : f == 1 ? GEMM_LOW_160 : GEMM_LOW_192;
     }
-    if (small < big) return deep ? GEMM_DEEP : GEMM_128;
+    if (small < big) return narrow ? GEMM_DEEP_64 : deep ? GEMM_DEEP : GEMM_128;
     return big == split ? GEMM_256_QUARTERS : GEMM_256;
 }
 
@@ -756,7 +764,7 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
         if (kernel == GEMM_LOW_160) return gemm_launch<GemmFlat<2, 3>, TA, TB, GRAD>(p, stream, who);
         if (kernel == GEMM_LOW_192) return gemm_launch<GemmFlat<3, 3>, TA, TB, GRAD>(p, stream, who);
     }
-    if (kernel == GEMM_DEEP) return gemm_deep_run(form, few, stream, who);
+    if (kernel == GEMM_DEEP || kernel == GEMM_DEEP_64) return gemm_deep_run(form, kernel == GEMM_DEEP ? 128 : 64, few, stream, who);
     if (kernel == GEMM_128) return gemm_launch<Gemm128, TA, TB, GRAD>(p, stream, who);
     p.stay = compute_units() / 8 * 8;
     p.split = kernel == GEMM_256_QUARTERS;
@@ -923,7 +931,7 @@ extern "C" const char *planmoe_expert_gemm_kernel(int form, int dtype, int activ
         static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
         return names[gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint)];
     }
-    static const char *const names[] = {"few rows", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"};
+    static const char *const names[] = {"few rows", "128x128 alone", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"};
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n;
     return names[gemm_pick(form, gemm_contiguous(form, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n), m, n, k, batches, counted, hint)];
 }

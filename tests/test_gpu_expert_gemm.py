@@ -719,6 +719,14 @@ def test_expert_gemm_in_every_kernel(dtype, form, kernel, B, cap, n, k, hint):
         assert bool(((db[e].double() - stored.sum(0)).abs() <= _bound(stored.sum(0), stored.abs().sum(0), max(r, 1), dtype)).all()), (e, r)
 
 
+# The tile alone in 128 columns, where 64 would be more work-groups than there are compute units (the shapes above and test_expert_gemm_tile_alone's are
+# in 64): reductions of three k-tiles, of one more than LDS holds and of many
+@pytest.mark.parametrize("form,B,cap,n,k,hint", [("rows", 8, 128, 2056, 136, 110), ("rows", 8, 128, 2056, 328, 110), ("rows", 4, 128, 4104, 1032, 100), ("tn", 4, 260, 1208, 392, 234),
+                                                 ("tn", 4, 600, 1208, 392, 600)])
+def test_expert_gemm_tile_alone_in_128_columns(form, B, cap, n, k, hint):
+    test_expert_gemm_in_every_kernel(torch.bfloat16, form, "128x128 alone", B, cap, n, k, hint)
+
+
 # The parts are no less precise than the fp32 matrix cores (which serve the same product under a relu: where a result is positive, that is the product):
 # the results and their sums over the rows, in which what is rounded one way adds up, for operands of both signs, behind a relu, and positive
 @pytest.mark.parametrize("form,kernel,B,m,n,k", [("nn", "f32 parts 256x128", 16, 512, 1024, 1024), ("nt", "f32 parts 256x128", 16, 512, 1024, 1024),
