@@ -561,8 +561,8 @@ int planmoe_layer_relu_bwd(int dtype, const void *grad_rows, const void *w2, con
                            size_t workspace_bytes, const void *sums, size_t sums_bytes, int samples, void *db2,
                            void *dwg, void *stream);
 
-/* The gradient of x: planmoe_layer_combine without gates, then planmoe_gate_dx_accumulate (up to 8 experts), the
- * same roundings, in one pass where a row is at most 8 KB. */
+/* The gradient of x: planmoe_layer_combine without gates, then planmoe_gate_dx_accumulate, the same roundings, in one pass
+ * where a row is at most 8 KB (up to 8 experts; up to 16 for such rows). */
 int planmoe_layer_dx(const void *rows, int dtype, int codec, const int32_t *indices, const int32_t *locations,
                      int64_t plane_stride, int top_k, int samples, int model_dim, int experts, int capacity,
                      const float *grad_logits, const void *wg, void *out, void *stream);

@@ -86,6 +86,22 @@ struct Kept {
     void *bias = nullptr, *scale = nullptr;
 };
 
+// Whether the combine of the gradient rows adds the gate's share of the gradient of x (planmoe_layer_dx): up to 8 experts always.  Beyond, the other way is
+// the combine, a cast and the library's product with a reduction of as many as there are experts, and one pass reads 16 weights a value from L2.
+// us, 16 experts, one pass and the other way:
+//   bf16         64 x 1024 5.9, 11.2    4096 x 1024 11.2, 19.8    16384 x 1024 39.8, 41.3    1024 x 4096 14.0, 18.9    16384 x 4096 142, 143
+//   bf16, int8   64 x 1024 6.7, 12.1    4096 x 2048 26.5, 30.6    16384 x 1024 52.1, 44.7    1024 x 4096 18.0, 20.6    4096 x 4096 52.2, 45.4
+//   fp32         1024 x 256 4.9, 7.3    64 x 1024 8.4, 7.0        1024 x 1024 8.8, 9.9       4096 x 1024 13.4, 21.4    16384 x 2048 81, 125
+//   fp32, int8   1024 x 256 7.0, 8.0    1024 x 1024 14.6, 12.4    4096 x 1024 19.8, 25.5     16384 x 2048 124, 132
+bool dx_in_one(const Shape &s, int codec)
+{
+    if (s.E <= 8) return true;
+    const int64_t values = (int64_t)s.T * s.M;
+    if (s.E > 16 || (int64_t)s.M * (s.dt == PLANMOE_F32 ? 4 : 2) > 8192) return false;
+    if (s.dt == PLANMOE_F32) return s.M <= 512 || s.T >= 4096 || (s.T >= 1024 && codec != CODEC_INT8);
+    return codec != CODEC_INT8 || (s.T <= 8192 && values <= (1 << 23));
+}
+
 Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
 
 Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, const Shape &s,
@@ -268,6 +284,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         const bool need_x = ctx->needs_input_grad(0), need_gate = ctx->needs_input_grad(1), need_w1 = ctx->needs_input_grad(2),
                    need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
         Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates, gf;
+        bool gate_added = false;                     // (dx has the gate's share)
         Tensor gl = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
         const float *dl = gl.defined() ? floats(gl) : nullptr;
         const int32_t *count0 = gl.defined() ? ints(p.counts) : nullptr;
@@ -361,13 +378,20 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                     if (codec == CODEC_ZFP) zfp_rows(gxe, Tensor(), p, s, st);
                     if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
                     dx = at::empty_like(x);
-                    if (whole && s.E <= 8) {
+                    if (whole && dx_in_one(s, codec)) {
                         PM_CALL(planmoe_layer_dx(gxe.data_ptr(), s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
                                                  wg.data_ptr(), dx.data_ptr(), st));
                         return {dx, dwg, dw1, db1, dw2, db2, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
                     }
-                    PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
-                                                  dx.data_ptr(), st));
+                    if (s.E > 8 && dx_in_one(s, codec)) {
+                        if (!gf.defined()) gf = as_float(route_bwd());
+                        PM_CALL(planmoe_layer_dx(gxe.data_ptr(), s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
+                                                 wg.data_ptr(), dx.data_ptr(), st));
+                        gate_added = true;
+                    } else {
+                        PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                                                      dx.data_ptr(), st));
+                    }
                 }
             }
         }
@@ -379,7 +403,7 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
                 Tensor ws = bytes((int64_t)planmoe_gate_dw_workspace_bytes(s.T, s.M, s.E), x);
                 PM_CALL(planmoe_gate_dw(x.data_ptr(), s.dt, floats(gf), s.T, s.M, s.E, dwg.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), st));
             }
-            if (need_x) {
+            if (need_x && !gate_added) {
                 if (!dx.defined()) {
                     dx = at::mm(gf.to(x.scalar_type()), wg);
                 } else if (s.E <= 8) {

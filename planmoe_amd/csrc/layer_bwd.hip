@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void slots_sum_kernel(const SumJobs all)
 // gradient of x in one pass (their own launches read and write out once more).  A wave per TOKENS tokens; up to EP experts, whose
 // weights come from the caches.  The roundings are those of planmoe_layer_combine and planmoe_gate_dx_accumulate.  Bound by the rows' bytes and, for
 // wide rows, by the weights out of L2.  bf16, top-2, 8 experts, both launches and this one: 16384 x 1024 44 and 24 us (int8 46 and 34), x 4096
-// 141 and 100 (int8 145 and 127), 1024 x 1024 17 and 7.5.
+// 141 and 100 (int8 145 and 127), 1024 x 1024 17 and 7.5.  (Up to 16 experts: where it pays, by dx_in_one of ext/layer.cpp.)
 template <int DT, int CACHE, bool INT8, int EP, int TOKENS>
 __global__ __launch_bounds__(256) void layer_dx_kernel(
     const void *__restrict__ rows, const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride, int top_k,
@@ -420,10 +420,11 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
 {
     const char *who = "planmoe_layer_dx";
     if (layer_rows_check(who, dtype, rows, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, codec)) return 1;
-    PM_REQUIRE(experts <= 8, "%s: built for up to 8 experts (got %d); a GEMM is faster above that", who, experts);
+    PM_REQUIRE(experts <= 16, "%s: built for up to 16 experts (got %d)", who, experts);
     if (samples == 0) return 0;
     PM_REQUIRE(grad_logits && wg && out && aligned16(wg) && aligned16(out), "%s: NULL or unaligned argument", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
+    PM_REQUIRE(experts <= 8 || per_lane <= 8, "%s: more than 8 experts: rows of up to 8 KB", who);
     if (per_lane > 8) {
         if (planmoe_layer_combine(rows, dtype, codec, nullptr, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, out, stream)) return 1;
         return planmoe_gate_dx_accumulate(out, dtype, grad_logits, wg, samples, model_dim, experts, stream);
@@ -431,8 +432,8 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
     hipStream_t st = (hipStream_t)stream;
     // Two tokens a wave read the weights once where they are as wide as the cache they come from and there are waves enough
     // (fp32, 8 experts x 1024 x 16384 tokens, no codec: 69 us with one, 34 with two; x 1024 tokens: 7.3 and 6.0, int8 10.1 and 11.4; bf16, whose rows
-    // take twice the registers unpacked: 43 and 39, int8 59 and 61).
-    const bool pairs = dtype == PLANMOE_F32 && samples >= 4096;
+    // take twice the registers unpacked: 43 and 39, int8 59 and 61).  16 experts' weights at any number of tokens (fp32, 64 x 1024: 12.6 and 8.4).
+    const bool pairs = dtype == PLANMOE_F32 && (samples >= 4096 || experts > 8);
 #define PM_DX__(CACHE, INT8, EP, TOKENS) (layer_dx_kernel<DT, CACHE, INT8, EP, TOKENS><<<(samples + 4 * TOKENS - 1) / (4 * TOKENS), 256, 0, st>>>( \
         rows, indices, locations, plane_stride, top_k, samples, model_dim, capacity, grad_logits, wg, experts, out))
 #define PM_DX_(CACHE, INT8, EP)                                                                                 \
@@ -442,8 +443,8 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
     } while (0)
 #define PM_DX(CACHE)                                                                                            \
     do {                                                                                                        \
-        if (codec) { if (experts <= 4) PM_DX_(CACHE, true, 4); else PM_DX_(CACHE, true, 8); }                   \
-        else { if (experts <= 4) PM_DX_(CACHE, false, 4); else PM_DX_(CACHE, false, 8); }                       \
+        if (codec) { if (experts <= 4) PM_DX_(CACHE, true, 4); else if (experts <= 8) PM_DX_(CACHE, true, 8); else PM_DX_(CACHE, true, 16); }      \
+        else { if (experts <= 4) PM_DX_(CACHE, false, 4); else if (experts <= 8) PM_DX_(CACHE, false, 8); else PM_DX_(CACHE, false, 16); }         \
     } while (0)
     PM_DTYPE_SWITCH(dtype, DT, { if (per_lane <= 1) PM_DX(1); else if (per_lane <= 2) PM_DX(2); else if (per_lane <= 4) PM_DX(4); else PM_DX(8); });
 #undef PM_DX

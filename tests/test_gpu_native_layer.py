@@ -727,3 +727,31 @@ def test_product_in_shares_and_combine(T, M, H, E, k, cap, skewed, with_bias):
     torch.cuda.synchronize()
     assert torch.equal(bits(out8), bits(again)) and torch.equal(bits(plain8), bits(again))
     assert torch.equal(codes, want_codes) and torch.equal(mn, want_mn) and torch.equal(scale, want_scale)
+
+
+# The combine that adds the gate's share of the gradient of x, for 9 to 16 experts: against the combine as it is and the product in 64 bits.  One token,
+# an odd number (two a wave in fp32), rows of one piece, of one more than a wave's 64 and of 8 KB; choices without a slot
+@pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 9, 1, 1), (5, 520, 16, 2, 1), (301, 1032, 11, 3, 40), (64, 2048, 16, 2, 8), (33, 4096, 16, 2, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("codec", [0, 1])
+def test_layer_dx_of_up_to_16_experts(T, M, E, k, cap, dtype, codec):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    if dtype == torch.float32 and M > 2048:
+        pytest.skip("rows of up to 8 KB")
+    print("case", T, M, E, k, cap, dtype, codec, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + M + E)
+    routed = ops.route_topk(torch.softmax(torch.randn(T, E, generator=g, device=DEV), 1), k)
+    idx, loc = routed["indices"].view(k, T), routed["locations"].view(k, T)
+    rows, wg = torch.randn(E * cap, M, generator=g, device=DEV).to(dtype), torch.randn(E, M, generator=g, device=DEV).to(dtype)
+    gl = torch.randn(T, E, generator=g, device=DEV)
+    out, plain = torch.empty(T, M, dtype=dtype, device=DEV), torch.empty(T, M, dtype=dtype, device=DEV)
+    p, dt, st = ops._ptr, ops._dt(rows, "t"), ops._stream(rows)
+    check(lib.planmoe_layer_dx(p(rows), dt, codec, p(idx), p(loc), T, k, T, M, E, cap, p(gl), p(wg), p(out), st))
+    check(lib.planmoe_layer_combine(p(rows), dt, codec, None, p(idx), p(loc), T, k, T, M, E, cap, p(plain), st))
+    torch.cuda.synchronize()
+    share, size = gl.to(dtype).double() @ wg.double(), gl.to(dtype).double().abs() @ wg.double().abs() + plain.double().abs()
+    want = plain.double() + share
+    # E + 1 terms in fp32, then one rounding
+    bound = want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) + size * (E + 1) * 2.0 ** -24 + 1e-30
+    assert bool(((out.double() - want).abs() <= bound).all())
