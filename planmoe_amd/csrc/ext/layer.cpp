@@ -37,8 +37,47 @@ struct Live {
     int planes, round;
 };
 
+// What the routing says, in one buffer that a backward pass keeps (a view or an allocation takes the host 1.5 - 2 us, and a training step of few
+// tokens is the host's): indices [k, T], locations [k, T], counts [k, E], gates [k, T], scores [T, E]
+struct Routing {
+    Routing() = default;
+    Routing(const Shape &s, at::ScalarType score_type) : type(score_type)
+    {
+        const int64_t each = score_type == at::kFloat ? 4 : 2, plane = (int64_t)s.k * s.T;
+        auto piece = [&](int64_t n) { const int64_t at = words; words += (n + 255) / 256 * 64; return at; };
+        idx_at = piece(plane * 4);
+        loc_at = piece(plane * 4);
+        cnt_at = piece((int64_t)s.k * s.E * 4);
+        gates_at = piece(plane * each);
+        scores_at = piece((int64_t)s.T * s.E * each);
+    }
+    void lie_in(const Tensor &buffer)
+    {
+        held = buffer;
+        int32_t *base = buffer.data_ptr<int32_t>();
+        idx = base + idx_at;
+        loc = base + loc_at;
+        cnt = base + cnt_at;
+        gates = base + gates_at;
+        scores = base + scores_at;
+    }
+    // the gates in fp32; `wide` holds what was converted
+    const float *float_gates(const Shape &s, Tensor &wide) const
+    {
+        if (type == at::kFloat) return (const float *)gates;
+        wide = at::from_blob(gates, {s.k, s.T}, held.options().dtype(type)).to(at::kFloat);
+        return floats(wide);
+    }
+    at::ScalarType type = at::kFloat;
+    int64_t words = 0, idx_at = 0, loc_at = 0, cnt_at = 0, gates_at = 0, scores_at = 0;
+    Tensor held;
+    int32_t *idx = nullptr, *loc = nullptr, *cnt = nullptr;
+    void *gates = nullptr, *scores = nullptr;
+};
+
 struct Pass {
-    Tensor y, l_aux, gates, indices, locations, counts, scores, xe, h, ye, stream, codes;
+    Tensor y, l_aux, xe, h, ye, stream, codes;
+    Routing r;
 };
 
 Tensor lz_round_trip(const Tensor &buf, void *st)
@@ -55,9 +94,9 @@ Tensor lz_round_trip(const Tensor &buf, void *st)
 
 Tensor zfp_stream(const Shape &s, const Tensor &like) { return bytes((int64_t)planmoe_zfp_stream_bytes(2, s.M, s.rows(), ZFP_RATE), like); }
 
-void zfp_rows(const Tensor &rows, const Tensor &stream, const Pass &p, const Shape &s, void *st)
+void zfp_rows(void *rows, const Tensor &stream, const Pass &p, const Shape &s, void *st)
 {
-    PM_CALL(planmoe_layer_zfp_rows(rows.data_ptr<float>(), s.M, s.E, s.cap, ints(p.counts), s.k, raw(stream), stream.defined() ? (size_t)stream.numel() : 0, st));
+    PM_CALL(planmoe_layer_zfp_rows((float *)rows, s.M, s.E, s.cap, p.r.cnt, s.k, raw(stream), stream.defined() ? (size_t)stream.numel() : 0, st));
 }
 
 Tensor zfp_workspace(const Shape &s, const Tensor &like) { return bytes((int64_t)planmoe_layer_zfp_workspace_bytes(s.E, s.cap), like); }
@@ -65,7 +104,7 @@ Tensor zfp_workspace(const Shape &s, const Tensor &like) { return bytes((int64_t
 Live live_rows(const Pass &p, const Shape &s, int codec)
 {
     if (codec == CODEC_LZ) return Live{nullptr, 1, 1};
-    return Live{ints(p.counts), s.k, codec == CODEC_ZFP ? 4 : 1};
+    return Live{p.r.cnt, s.k, codec == CODEC_ZFP ? 4 : 1};
 }
 
 // a gradient as the kernels read rows: contiguous and 16-byte aligned (what comes back through torch.cat is contiguous,
@@ -102,28 +141,23 @@ bool dx_in_one(const Shape &s, int codec)
     return codec != CODEC_INT8 || (s.T <= 8192 && values <= (1 << 23));
 }
 
-Tensor float_gates(const Tensor &gates) { return gates.scalar_type() == at::kFloat ? gates : gates.to(at::kFloat); }
-
 Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, const Shape &s,
                   bool fp32_gate, bool normalize, int codec, bool keep)
 {
     void *st = current_stream();
     Pass p;
     const auto score_type = fp32_gate ? at::kFloat : x.scalar_type();
-    const auto i32 = x.options().dtype(at::kInt);
-    // [k, T] of indices and of locations, [k, E] of counts
-    Tensor planes = at::empty({2 * (int64_t)s.k * s.T + (int64_t)s.k * s.E}, i32);
-    p.indices = planes.narrow(0, 0, (int64_t)s.k * s.T);
-    p.locations = planes.narrow(0, (int64_t)s.k * s.T, (int64_t)s.k * s.T);
-    p.counts = planes.narrow(0, 2 * (int64_t)s.k * s.T, (int64_t)s.k * s.E);
-    p.gates = at::empty({s.k, s.T}, x.options().dtype(score_type));
+    p.r = Routing(s, score_type);
+    p.r.lie_in(at::empty({p.r.words}, x.options().dtype(at::kInt)));
     p.l_aux = at::empty({}, x.options().dtype(at::kFloat));
-    if (keep) p.scores = at::empty({s.T, s.E}, x.options().dtype(score_type));
-    Tensor ws = bytes((int64_t)planmoe_forward_workspace_bytes(s.T, s.E, s.k), x);
-    int32_t *idx = p.indices.data_ptr<int32_t>(), *loc = p.locations.data_ptr<int32_t>(), *cnt = p.counts.data_ptr<int32_t>();
+    const int64_t ws_bytes = ((int64_t)planmoe_forward_workspace_bytes(s.T, s.E, s.k) + 255) / 256 * 256;
+    const size_t shares = s.shares(codec);
+    Tensor ws = bytes(ws_bytes + (int64_t)shares, x);
+    int32_t *idx = p.r.idx, *loc = p.r.loc, *cnt = p.r.cnt;
+    void *const scores = keep ? p.r.scores : nullptr;
     if (codec == CODEC_ZFP) {
-        PM_CALL(planmoe_gate_route(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, idx, loc, raw(p.gates),
-                                   s.T, nullptr, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, ws.data_ptr(), (size_t)ws.numel(), st));
+        PM_CALL(planmoe_gate_route(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, idx, loc, p.r.gates,
+                                   s.T, nullptr, scores, p.l_aux.data_ptr<float>(), cnt, ws.data_ptr(), (size_t)ws.numel(), st));
         p.xe = at::empty({s.rows(), s.M}, x.options());
         ws = zfp_workspace(s, x);
         PM_CALL(planmoe_layer_zfp_dispatch(floats(x), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt, p.xe.data_ptr<float>(), ws.data_ptr(),
@@ -131,13 +165,13 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
     } else if (codec == CODEC_LZ) {
         p.xe = at::empty({s.rows(), s.M}, x.options());
         PM_CALL(planmoe_forward_plain(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, idx, loc,
-                                      raw(p.gates), s.T, nullptr, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
+                                      p.r.gates, s.T, nullptr, scores, p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
                                       (size_t)ws.numel(), st));
         p.xe = lz_round_trip(p.xe, st);
     } else {
         p.xe = at::empty({s.rows(), s.M}, x.options());
         PM_CALL(planmoe_layer_dispatch(x.data_ptr(), wg.data_ptr(), s.dt, fp32_gate, nullptr, s.T, s.M, s.E, s.k, normalize, s.cap, codec, idx, loc,
-                                       raw(p.gates), s.T, raw(p.scores), p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
+                                       p.r.gates, s.T, scores, p.l_aux.data_ptr<float>(), cnt, p.xe.data_ptr(), ws.data_ptr(),
                                        (size_t)ws.numel(), st));
     }
     const Live live = live_rows(p, s, codec);
@@ -146,19 +180,18 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
                                 s.hint(), p.h.data_ptr(), st));
     p.ye = at::empty({s.rows(), s.M}, x.options());
     p.y = at::empty({s.T, s.M}, x.options());
-    const Tensor gates = float_gates(p.gates);
+    Tensor wide;
+    const float *const gates = p.r.float_gates(s, wide);
     if (codec == CODEC_NONE || codec == CODEC_INT8) {
-        const size_t shares = s.shares(codec);
-        ws = shares ? bytes((int64_t)shares, x) : Tensor();
         Kept kept;
         if (codec == CODEC_INT8 && keep) {
             // (the backward pass reads the codes: a byte a value is held until then, as between Compress and its backward)
             p.codes = bytes(Kept::bytes(s, x.element_size()), x);
             kept = Kept(p.codes, s, x.element_size());
         }
-        PM_CALL(planmoe_layer_product_combine(p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, floats(gates), idx, loc, s.T, s.k, s.T,
+        PM_CALL(planmoe_layer_product_combine(p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, gates, idx, loc, s.T, s.k, s.T,
                                               s.M, s.E, s.cap, cnt, 1, s.hint(), p.ye.data_ptr(), keep, kept.codes, kept.bias, kept.scale, p.y.data_ptr(),
-                                              raw(ws), shares, st));
+                                              ws.data_ptr<uint8_t>() + ws_bytes, shares, st));
         if (p.codes.defined()) p.ye = Tensor();
         return p;
     }
@@ -166,10 +199,10 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
                                 s.hint(), p.ye.data_ptr(), st));
     if (codec == CODEC_ZFP) {
         if (keep) p.stream = zfp_stream(s, x);
-        zfp_rows(p.ye, p.stream, p, s, st);
+        zfp_rows(p.ye.data_ptr(), p.stream, p, s, st);
     }
     if (codec == CODEC_LZ) p.ye = lz_round_trip(p.ye, st);
-    PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, 0, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
+    PM_CALL(planmoe_layer_combine(p.ye.data_ptr(), s.dt, 0, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.y.data_ptr(), st));
     if (p.stream.defined()) p.ye = Tensor();         // (the backward pass reads the stream)
     return p;
 }
@@ -253,12 +286,8 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
     {
         const Shape s = shape_of(x, wg, w1, k, cap);
         Pass p = forward_pass(x, wg, w1, b1, w2, b2, s, fp32_gate, normalize, (int)codec, true);
-        ctx->save_for_backward({x, wg, w1, w2, p.scores, p.gates, p.indices, p.locations, p.counts, p.xe, p.h,
-                                codec == CODEC_ZFP ? p.stream : codec == CODEC_INT8 ? p.codes : p.ye});
-        ctx->saved_data["k"] = k;
-        ctx->saved_data["cap"] = cap;
-        ctx->saved_data["normalize"] = normalize;
-        ctx->saved_data["codec"] = codec;
+        ctx->save_for_backward({x, wg, w1, w2, p.r.held, p.xe, p.h, codec == CODEC_ZFP ? p.stream : codec == CODEC_INT8 ? p.codes : p.ye});
+        ctx->saved_data["form"] = std::vector<int64_t>{k, cap, normalize, codec, fp32_gate};
         ctx->set_materialize_grads(false);
         return {p.y, p.l_aux};
     }
@@ -266,33 +295,33 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &wg = saved[1], &w1 = saved[2], &w2 = saved[3], &scores = saved[4];
+        const Tensor &x = saved[0], &wg = saved[1], &w1 = saved[2], &w2 = saved[3];
         const c10::DeviceGuard guard(x.device());
-        const int codec = (int)ctx->saved_data["codec"].toInt();
-        const bool normalize = ctx->saved_data["normalize"].toBool();
-        const Shape s = shape_of(x, wg, w1, ctx->saved_data["k"].toInt(), ctx->saved_data["cap"].toInt());
+        const std::vector<int64_t> form = ctx->saved_data["form"].toIntVector();
+        const int codec = (int)form[3];
+        const bool normalize = form[2] != 0;
+        const Shape s = shape_of(x, wg, w1, form[0], form[1]);
         void *st = current_stream();
         Pass p;
-        p.gates = saved[5];
-        p.indices = saved[6];
-        p.locations = saved[7];
-        p.counts = saved[8];
-        p.xe = saved[9];
-        p.h = saved[10];
-        const Tensor &ye = saved[11];                // (the rows; zfp: their stream; int8: their codes)
-        const int32_t *idx = ints(p.indices), *loc = ints(p.locations);
+        p.r = Routing(s, form[4] ? at::kFloat : x.scalar_type());
+        p.r.lie_in(saved[4]);
+        p.xe = saved[5];
+        p.h = saved[6];
+        const Tensor &ye = saved[7];                 // (the rows; zfp: their stream; int8: their codes)
+        const int32_t *idx = p.r.idx, *loc = p.r.loc;
+        const auto score_options = x.options().dtype(p.r.type);
         const bool need_x = ctx->needs_input_grad(0), need_gate = ctx->needs_input_grad(1), need_w1 = ctx->needs_input_grad(2),
                    need_b1 = ctx->needs_input_grad(3), need_w2 = ctx->needs_input_grad(4), need_b2 = ctx->needs_input_grad(5);
         Tensor dx, dwg, dw1, db1, dw2, db2, grad_gates, gf;
         bool gate_added = false;                     // (dx has the gate's share)
         Tensor gl = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
         const float *dl = gl.defined() ? floats(gl) : nullptr;
-        const int32_t *count0 = gl.defined() ? ints(p.counts) : nullptr;
+        const int32_t *count0 = gl.defined() ? p.r.cnt : nullptr;
         // the logits' gradient, in the scores' precision
         auto route_bwd = [&]() {
-            Tensor gg = grad_gates.defined() ? grad_gates.to(scores.scalar_type()) : at::zeros({s.k, s.T}, scores.options());
-            Tensor g = at::empty_like(scores);
-            PM_CALL(planmoe_route_bwd(scores.data_ptr(), pm_dtype(scores.scalar_type()), idx, gg.data_ptr(), s.T, s.T, s.E, s.k, normalize, dl, count0, 1,
+            Tensor gg = grad_gates.defined() ? grad_gates.to(p.r.type) : at::zeros({s.k, s.T}, score_options);
+            Tensor g = at::empty({s.T, s.E}, score_options);
+            PM_CALL(planmoe_route_bwd(p.r.scores, pm_dtype(p.r.type), idx, gg.data_ptr(), s.T, s.T, s.E, s.k, normalize, dl, count0, 1,
                                       g.data_ptr(), st));
             return g;
         };
@@ -301,95 +330,110 @@ struct FfnLayer : public torch::autograd::Function<FfnLayer> {
         const bool whole = grads[0].defined() && need_x && need_gate && need_w1 && need_b1 && need_w2 && need_b2;
         if (grads[0].defined()) {
             const Tensor grad = as_rows(grads[0]);
-            const Tensor gates = float_gates(p.gates);
+            Tensor wide;
+            const float *const gates = p.r.float_gates(s, wide);
             const Live live = live_rows(p, s, codec);
             const bool logits = whole && s.k <= 64 && (codec == CODEC_NONE || codec == CODEC_INT8);
+            // what only this pass sees; with everything asked for in one buffer
+            const int64_t size = x.element_size(), wide_rows = s.rows() * s.M * size, hidden_rows = s.rows() * s.H * size;
+            const int64_t sums_bytes = whole ? (int64_t)planmoe_layer_sums_workspace_bytes(s.E, s.cap, s.T, s.M) : 0;
+            const int64_t db1_bytes = need_b1 ? (int64_t)planmoe_expert_gemm_relu_bwd_workspace_bytes(s.E, s.cap, s.H) : 0;
+            auto room = [](int64_t n) { return (n + 255) / 256 * 256; };
+            Tensor pool, alone[5];
+            int64_t used = 0;
+            int count = 0;
+            if (whole && codec != CODEC_LZ) pool = bytes(2 * room(wide_rows) + room(hidden_rows) + room(sums_bytes) + room(db1_bytes), x);
+            auto scratch = [&](int64_t n) -> void * {
+                if (!pool.defined()) return (alone[count++] = bytes(n, x)).data_ptr();
+                used += room(n);
+                return pool.data_ptr<uint8_t>() + used - room(n);
+            };
             (logits ? gf : grad_gates) = at::empty({logits ? s.T : s.k, logits ? s.E : s.T}, x.options().dtype(at::kFloat));
-            Tensor gye, sums;
+            Tensor coded_rows;                       // (lz)
+            void *gye, *sums = nullptr;
             if (codec == CODEC_ZFP) {
-                gye = at::empty({s.rows(), s.M}, x.options());
+                gye = scratch(wide_rows);
                 Tensor ws = zfp_workspace(s, x);
-                PM_CALL(planmoe_layer_zfp_combine_bwd(ye.data_ptr(), floats(grad), floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, ints(p.counts),
-                                                      gye.data_ptr<float>(), grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
+                PM_CALL(planmoe_layer_zfp_combine_bwd(ye.data_ptr(), floats(grad), gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, p.r.cnt,
+                                                      (float *)gye, grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
             } else if (codec == CODEC_LZ) {
                 Tensor buf = at::empty({s.rows(), s.M}, x.options()), ws = bytes((int64_t)planmoe_dispatch_workspace_bytes(s.E, s.cap), x);
-                PM_CALL(planmoe_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, buf.data_ptr(),
+                PM_CALL(planmoe_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, buf.data_ptr(),
                                             grad_gates.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), st));
-                gye = lz_round_trip(buf, st);
+                coded_rows = lz_round_trip(buf, st);
+                gye = coded_rows.data_ptr();
             } else {
-                gye = at::empty({s.rows(), s.M}, x.options());
+                gye = scratch(wide_rows);
                 if (logits) {
                     const bool coded = codec == CODEC_INT8;
                     const Kept kept = coded ? Kept(ye, s, x.element_size()) : Kept{};
                     PM_CALL(planmoe_layer_combine_bwd_logits(grad.data_ptr(), coded ? kept.codes : ye.data_ptr(), kept.bias, kept.scale, s.dt, coded,
-                                                             floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, gye.data_ptr(), scores.data_ptr(),
-                                                             pm_dtype(scores.scalar_type()), normalize, dl, count0, gf.data_ptr<float>(), st));
+                                                             gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, gye, p.r.scores,
+                                                             pm_dtype(p.r.type), normalize, dl, count0, gf.data_ptr<float>(), st));
                 } else if (codec == CODEC_INT8) {
                     const Kept kept(ye, s, x.element_size());
-                    PM_CALL(planmoe_layer_combine_bwd_codes(grad.data_ptr(), kept.codes, kept.bias, kept.scale, s.dt, floats(gates), idx, loc, s.T, s.k,
-                                                            s.T, s.M, s.E, s.cap, gye.data_ptr(), grad_gates.data_ptr<float>(), st));
+                    PM_CALL(planmoe_layer_combine_bwd_codes(grad.data_ptr(), kept.codes, kept.bias, kept.scale, s.dt, gates, idx, loc, s.T, s.k,
+                                                            s.T, s.M, s.E, s.cap, gye, grad_gates.data_ptr<float>(), st));
                 } else {
-                    PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, 0, floats(gates), idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
-                                                      gye.data_ptr(), grad_gates.data_ptr<float>(), st));
+                    PM_CALL(planmoe_layer_combine_bwd(grad.data_ptr(), ye.data_ptr(), s.dt, 0, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                                                      gye, grad_gates.data_ptr<float>(), st));
                 }
             }
             if (whole) {
                 if (!gf.defined()) gf = as_float(route_bwd());
-                sums = bytes((int64_t)planmoe_layer_sums_workspace_bytes(s.E, s.cap, s.T, s.M), x);
-                PM_CALL(planmoe_layer_sums(gye.data_ptr(), s.dt, s.E, s.cap, live.counts, live.planes, live.round, x.data_ptr(), floats(gf), s.T, s.M,
-                                           sums.data_ptr(), (size_t)sums.numel(), st));
+                sums = scratch(sums_bytes);
+                PM_CALL(planmoe_layer_sums(gye, s.dt, s.E, s.cap, live.counts, live.planes, live.round, x.data_ptr(), floats(gf), s.T, s.M,
+                                           sums, (size_t)sums_bytes, st));
                 db2 = at::empty({s.E, s.M}, x.options());
                 dwg = at::empty_like(wg);
             }
-            auto colsum = [&](const Tensor &a, int cols) {
+            auto colsum = [&](const void *a, int cols) {
                 Tensor out = at::empty({s.E, cols}, x.options()), ws = bytes((int64_t)planmoe_rows_colsum_workspace_bytes(s.E, s.cap, cols), x);
-                PM_CALL(planmoe_rows_colsum(a.data_ptr(), s.dt, s.E, s.cap, cols, live.counts, live.planes, live.round, out.data_ptr(), ws.data_ptr(),
+                PM_CALL(planmoe_rows_colsum(a, s.dt, s.E, s.cap, cols, live.counts, live.planes, live.round, out.data_ptr(), ws.data_ptr(),
                                             (size_t)ws.numel(), st));
                 return out;
             };
             if (need_w2) {
                 dw2 = at::empty_like(w2);
-                PM_CALL(planmoe_expert_gemm(2, s.dt, p.h.data_ptr(), gye.data_ptr(), nullptr, 0, s.E, s.H, s.M, s.cap, live.counts, live.planes, live.round,
+                PM_CALL(planmoe_expert_gemm(2, s.dt, p.h.data_ptr(), gye, nullptr, 0, s.E, s.H, s.M, s.cap, live.counts, live.planes, live.round,
                                             s.hint(), dw2.data_ptr(), st));
             }
             if (need_b2 && !whole) db2 = colsum(gye, s.M);
             if (need_x || need_w1 || need_b1) {
-                Tensor gh = at::empty({s.rows(), s.H}, x.options()), ws;
-                if (need_b1) {
-                    db1 = at::empty({s.E, s.H}, x.options());
-                    ws = bytes((int64_t)planmoe_expert_gemm_relu_bwd_workspace_bytes(s.E, s.cap, s.H), x);
-                }
+                void *const gh = scratch(hidden_rows), *const ws = need_b1 ? scratch(db1_bytes) : nullptr;
+                if (need_b1) db1 = at::empty({s.E, s.H}, x.options());
                 if (whole)
-                    PM_CALL(planmoe_layer_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
-                                                   live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), (size_t)ws.numel(), sums.data_ptr(),
-                                                   (size_t)sums.numel(), s.T, raw(db2), raw(dwg), st));
+                    PM_CALL(planmoe_layer_relu_bwd(s.dt, gye, w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
+                                                   live.round, s.hint(), gh, raw(db1), ws, (size_t)db1_bytes, sums,
+                                                   (size_t)sums_bytes, s.T, raw(db2), raw(dwg), st));
                 else
-                    PM_CALL(planmoe_expert_gemm_relu_bwd(s.dt, gye.data_ptr(), w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
-                                                         live.round, s.hint(), gh.data_ptr(), raw(db1), raw(ws), ws.defined() ? (size_t)ws.numel() : 0, st));
+                    PM_CALL(planmoe_expert_gemm_relu_bwd(s.dt, gye, w2.data_ptr(), p.h.data_ptr(), s.E, s.cap, s.H, s.M, live.counts, live.planes,
+                                                         live.round, s.hint(), gh, raw(db1), ws, (size_t)db1_bytes, st));
                 if (need_w1) {
                     dw1 = at::empty_like(w1);
-                    PM_CALL(planmoe_expert_gemm(2, s.dt, p.xe.data_ptr(), gh.data_ptr(), nullptr, 0, s.E, s.M, s.H, s.cap, live.counts, live.planes,
+                    PM_CALL(planmoe_expert_gemm(2, s.dt, p.xe.data_ptr(), gh, nullptr, 0, s.E, s.M, s.H, s.cap, live.counts, live.planes,
                                                 live.round, s.hint(), dw1.data_ptr(), st));
                 }
                 if (need_x) {
-                    Tensor gxe = at::empty({s.rows(), s.M}, x.options());
-                    PM_CALL(planmoe_expert_gemm(1, s.dt, gh.data_ptr(), w1.data_ptr(), nullptr, 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
-                                                s.hint(), gxe.data_ptr(), st));
+                    Tensor lz_rows = codec == CODEC_LZ ? at::empty({s.rows(), s.M}, x.options()) : Tensor();
+                    void *gxe = codec == CODEC_LZ ? lz_rows.data_ptr() : scratch(wide_rows);
+                    PM_CALL(planmoe_expert_gemm(1, s.dt, gh, w1.data_ptr(), nullptr, 0, s.E, s.cap, s.M, s.H, live.counts, live.planes, live.round,
+                                                s.hint(), gxe, st));
                     if (codec == CODEC_ZFP) zfp_rows(gxe, Tensor(), p, s, st);
-                    if (codec == CODEC_LZ) gxe = lz_round_trip(gxe, st);
+                    if (codec == CODEC_LZ) gxe = (lz_rows = lz_round_trip(lz_rows, st)).data_ptr();
                     dx = at::empty_like(x);
                     if (whole && dx_in_one(s, codec)) {
-                        PM_CALL(planmoe_layer_dx(gxe.data_ptr(), s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
+                        PM_CALL(planmoe_layer_dx(gxe, s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
                                                  wg.data_ptr(), dx.data_ptr(), st));
                         return {dx, dwg, dw1, db1, dw2, db2, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
                     }
                     if (s.E > 8 && dx_in_one(s, codec)) {
                         if (!gf.defined()) gf = as_float(route_bwd());
-                        PM_CALL(planmoe_layer_dx(gxe.data_ptr(), s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
+                        PM_CALL(planmoe_layer_dx(gxe, s.dt, codec == CODEC_INT8, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, floats(gf),
                                                  wg.data_ptr(), dx.data_ptr(), st));
                         gate_added = true;
                     } else {
-                        PM_CALL(planmoe_layer_combine(gxe.data_ptr(), s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
+                        PM_CALL(planmoe_layer_combine(gxe, s.dt, codec == CODEC_INT8, nullptr, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap,
                                                       dx.data_ptr(), st));
                     }
                 }
