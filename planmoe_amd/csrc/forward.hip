@@ -459,7 +459,7 @@ static void launch_gate_route(int experts, int groups, int group_tokens, hipStre
     gate_route_kernel<DT, SDT, NT, CAP, SPLITK, GROUP><<<groups, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
         k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws, nullptr, 0)
 #define PM_GR(NT, CAP, SPLITK) do { if (group_tokens == 32) PM_GR_(NT, CAP, SPLITK, 32); \
-                                    else if (group_tokens == 16) PM_GR_(NT, CAP, SPLITK, (NT == 4 ? 16 : 32)); \
+                                    else if (group_tokens == 16) PM_GR_(NT, CAP, SPLITK, (NT == 2 ? 32 : 16)); \
                                     else PM_GR_(NT, CAP, SPLITK, 64); } while (0)
     // split-K measured faster than the LDS-shared variant up to 16 experts (30.7 vs 44.4 us at
     // 16384 x 4096 bf16, 8 experts), and the other way round above (168 -> 48 us at 64 experts)

@@ -50,13 +50,13 @@ struct GateFrag {
 // Partial logits of tokens [t0, t0 + 16*TPW) against experts [0, 16*NT): wave w of the NW waves
 // of the work-group accumulates the K steps w, w+NW, ... (a step is 16 vectors = 256 bytes of
 // every row) and leaves its tiles in part[w][token][expert].  Rows past the end of x / wg are clamped to the last valid
-// row: their products land in tile entries nobody reads.  Loads of the next step are issued
-// before the MFMAs of the current one.
+// row: their products land in tile entries nobody reads.  DEPTH steps are on their way from memory: where a work-group is alone on its
+// compute unit and a wave has few steps, it is their latencies that bound it.  The order of the sums does not depend on DEPTH.
 // With STATS (bf16 only) the wave also keeps the running min / max / NaN scan of every token row
 // it streams (the VALU is idle while the loads are in flight) and leaves, per wave, the three
 // 32-bit words of RowStats<bf16>::reduced() in pstat[w][token][0..2].
 // Requires model_dim % VEC == 0 and 16-byte aligned x / wg.  Call with all 64*NW threads.
-template <int DT, int NT, int TPW, int NW = 4, bool STATS = false>
+template <int DT, int NT, int TPW, int NW = 4, bool STATS = false, int DEPTH = 2>
 __device__ __forceinline__ void gate_tile_partials(const void *__restrict__ x,
                                                    const void *__restrict__ wg, int t0, int samples,
                                                    int model_dim, int experts,
@@ -116,21 +116,53 @@ __device__ __forceinline__ void gate_tile_partials(const void *__restrict__ x,
             }
     };
 
-    GateFrag<NT, TPW> f0, f1;
-    if (w < full) {
-        const int nsteps = (full - w + NW - 1) / NW;     // steps of this wave: w, w + NW, ...
-        const int last = w + (nsteps - 1) * NW;
-        int step = w;
-        if (nsteps & 1) { load(f0, step); mma(f0); step += NW; }
-        if (step <= last) {
-            // pairs of steps, one straight-line body: each buffer is re-filled while the MFMAs of
-            // the other run.  The last prefetch re-reads the wave's last step (a cache hit).
-            load(f0, step);
-            for (; step <= last; step += 2 * NW) {
-                load(f1, step + NW);
-                mma(f0);
-                load(f0, min(step + 2 * NW, last));
-                mma(f1);
+    static_assert(DEPTH == 2 || DEPTH == 4, "steps on their way");
+    if constexpr (DEPTH == 4) {
+        const int nsteps = w < full ? (full - w + NW - 1) / NW : 0;
+        int step = w, left = nsteps;
+        GateFrag<NT, TPW> f[4];
+        // first what four does not divide, then fours: no step is asked for twice
+        if (left & 3) {
+            const int end = w + ((left & 3) - 1) * NW;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) load(f[d], min(step + d * NW, end));
+            mma(f[0]);
+            if (left & 2) mma(f[1]);
+            if ((left & 3) == 3) mma(f[2]);
+            step += (left & 3) * NW;
+            left &= ~3;
+        }
+        if (left) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) load(f[d], step + d * NW);
+            for (; left > 4; left -= 4) {
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    mma(f[d]);
+                    load(f[d], step + (d + 4) * NW);
+                }
+                step += 4 * NW;
+            }
+#pragma unroll
+            for (int d = 0; d < 4; ++d) mma(f[d]);
+        }
+    } else {
+        GateFrag<NT, TPW> f0, f1;
+        if (w < full) {
+            const int nsteps = (full - w + NW - 1) / NW;     // steps of this wave: w, w + NW, ...
+            const int last = w + (nsteps - 1) * NW;
+            int step = w;
+            if (nsteps & 1) { load(f0, step); mma(f0); step += NW; }
+            if (step <= last) {
+                // pairs of steps, one straight-line body: each buffer is re-filled while the MFMAs of
+                // the other run.  The last prefetch re-reads the wave's last step (a cache hit).
+                load(f0, step);
+                for (; step <= last; step += 2 * NW) {
+                    load(f1, step + NW);
+                    mma(f0);
+                    load(f0, min(step + 2 * NW, last));
+                    mma(f1);
+                }
             }
         }
     }

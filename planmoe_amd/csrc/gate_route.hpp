@@ -10,8 +10,15 @@ namespace pm {
 inline int fwd_group_tokens(int experts, int samples)
 {
     // measured at 8 experts: 16384 tokens (256 groups of 64) 39 us with 64, 44 us with 32;
-    // 8192 tokens 32 us with 64, 28 us with 32
-    if (experts <= 16) return samples < 64 * 256 ? 32 : 64;
+    // 8192 tokens 32 us with 64, 28 us with 32.  One compute unit gets some 30 GB/s, so fewer tokens in a group are fewer bytes in that chain, up to one
+    // group a compute unit; beyond, two groups on some units take longer than one of 32.  us of the send side with 32 and with 16 tokens:
+    //   bf16, 8 x 512     40 tokens 10.2, 10.5   1999 12.2, 12.4   4096 13.8, 13.9   5000 14.3, 16.9
+    //   bf16, 8 x 2048    40 tokens 13.2, 11.5   1999 15.9, 14.0   4096 19.0, 17.1   5000 20.1, 22.0
+    //   bf16, 16 x 4096   40 tokens 22.1, 17.3   1999 25.1, 20.4   4096 34.1, 28.2   5000 36.4, 38.0
+    //   fp32, 16 x 1024   40 tokens 16.0, 13.0   1999 18.6, 15.9   4096 22.6, 18.1   5000 23.4, 24.6
+    //   fp32, 8 x 4096    40 tokens 32.5, 25.9   1999 38.8, 31.7   4096 50.9, 48.4   5000 56.2, 64.1
+    // (up to 32 tokens are one group, and one launch: plan.one)
+    if (experts <= 16) return samples > 32 && samples <= 16 * 256 ? 16 : samples < 64 * 256 ? 32 : 64;
     // as many groups as compute units at most (16 tokens: where four waves find a share of the experts).  us of the send side, bf16, with 64, 32, 16:
     //   64 experts x 1368   48 tokens 26, 22, 21;  4074 33, 29, 27;  8000 35, 32, 42;  16000 39, 47, 74
     //   32 experts x 1368   48 tokens 24, 20;      4074 33, 24;      8000 35, 28;      16000 42, 42
@@ -93,7 +100,7 @@ __device__ __forceinline__ void gate_route_group(
     float *__restrict__ l_aux, int32_t *__restrict__ counts_out, void *__restrict__ workspace, int capacity)
 {
     using S = Elem<SDT>;
-    static_assert(GROUP == 64 || GROUP == 32 || (!SPLITK && GROUP == 16), "tokens of a group");
+    static_assert(GROUP == 64 || GROUP == 32 || GROUP == 16, "tokens of a group");
     constexpr int COLS = 16 * NT + 1;
     auto &smem = sh.smem;
     auto &s_hist = sh.hist;
@@ -133,8 +140,9 @@ __device__ __forceinline__ void gate_route_group(
             }
         }
     } else if constexpr (SPLITK) {
-        if constexpr (STATS) gate_tile_partials<DT, NT, GROUP / 16, 4, true>(x, wg, t0, samples, model_dim, experts, part, pstat);
-        else gate_tile_partials<DT, NT, GROUP / 16, 4>(x, wg, t0, samples, model_dim, experts, part);
+        constexpr int DEPTH = GROUP == 16 ? 4 : 2;            // (groups of 32, two on some compute units: 8 x 4096 fp32, 6500 tokens 68 us with two, 70 with four)
+        if constexpr (STATS) gate_tile_partials<DT, NT, GROUP / 16, 4, true, DEPTH>(x, wg, t0, samples, model_dim, experts, part, pstat);
+        else gate_tile_partials<DT, NT, GROUP / 16, 4, false, DEPTH>(x, wg, t0, samples, model_dim, experts, part);
     } else {
         if constexpr (STATS) gate_tile_lds<DT, NT, true, GROUP>(x, wg, t0, samples, model_dim, experts, smem, pstat[0]);
         else gate_tile_lds<DT, NT, false, GROUP>(x, wg, t0, samples, model_dim, experts, smem);

@@ -233,6 +233,17 @@ def test_fused_forward_many_experts_group_sizes(T, M, E, k, dtype):
     test_fused_forward_matches_unfused_and_oracle(T, M, E, k, 1.25, dtype, True, T % 2 == 1)
 
 
+# up to 16 experts: groups of 16 and 32 tokens, either side of where they change and of a group's end; rows of less than a step, and of as
+# many steps that a wave has one to nine of them, with and without a piece at the end
+@pytest.mark.parametrize("T,M,E,k,dtype", [
+    (32, 128, 8, 2, torch.bfloat16), (33, 8, 8, 2, torch.bfloat16), (47, 520, 16, 3, torch.bfloat16), (48, 1032, 9, 2, torch.float32),
+    (49, 256, 1, 1, torch.float32), (64, 1536, 16, 1, torch.float16), (65, 2056, 7, 5, torch.bfloat16), (100, 2560, 5, 2, torch.bfloat16),
+    (130, 3080, 8, 2, torch.bfloat16), (34, 3592, 10, 2, torch.bfloat16), (50, 4096, 8, 2, torch.bfloat16), (35, 2304, 16, 2, torch.float32),
+    (4096, 264, 8, 2, torch.bfloat16), (4097, 136, 16, 2, torch.bfloat16), (4095, 72, 3, 2, torch.float32)])
+def test_fused_forward_few_experts_group_sizes(T, M, E, k, dtype):
+    test_fused_forward_matches_unfused_and_oracle(T, M, E, k, 1.25, dtype, True, T % 2 == 1)
+
+
 @pytest.mark.parametrize("T,M,E,k,cf,dtype,fp32_gate,use_bias", [
     (1000, 512, 8, 2, 1.25, torch.bfloat16, True, False), (33, 256, 4, 2, 1.0, torch.bfloat16, True, False),
     (4096, 1024, 64, 1, 1.0, torch.bfloat16, True, True), (500, 2048, 2, 2, 1.0, torch.float32, True, False),
