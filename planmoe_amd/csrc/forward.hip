@@ -559,23 +559,38 @@ static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t 
                                                                         l_aux);
 }
 
-// stand-alone routing from logits / scores in memory: the epilogue of gate_route_kernel on 64-token
-// groups, then the prefix over the groups and the final slots
-template <int SDT, int ONE>
+// stand-alone routing from logits / scores in memory: the epilogue of gate_route_kernel on groups of 64, 32 or 16
+// tokens, then the prefix over the groups and the final slots
+template <int SDT, int GROUP, int ONE>
 static void launch_route_groups(int experts, int groups, int mode, hipStream_t st, const void *input, const float *bias,
                                 int samples, int k, int normalize, int32_t *indices, int32_t *locations, void *gates,
                                 int64_t stride, void *scores_out, float *l_aux, int32_t *counts, void *ws)
 {
 #define PM_RG_(NT, CAP, MODE)                                                                              \
-    gate_route_kernel<SDT, SDT, NT, CAP, false, 64, MODE, ONE><<<groups, 256, 0, st>>>(input, nullptr, bias, samples, 0, \
+    gate_route_kernel<SDT, SDT, NT, CAP, false, GROUP, MODE, ONE><<<groups, 256, 0, st>>>(input, nullptr, bias, samples, 0, \
         experts, k, normalize, indices, locations, gates, stride, nullptr, scores_out, l_aux, counts, ws, nullptr, 0)
 #define PM_RG(NT, CAP) do { if (mode == 1) PM_RG_(NT, CAP, 1); else PM_RG_(NT, CAP, 2); } while (0)
-    if (experts <= 8) PM_RG(1, 8);
-    else if (experts <= 16) PM_RG(1, 16);
+    if constexpr (GROUP > 16) {
+        if (experts <= 8) { PM_RG(1, 8); return; }
+    }
+    if (experts <= 16) PM_RG(1, 16);
     else if (experts <= 32) PM_RG(2, 32);
     else PM_RG(4, 64);
 #undef PM_RG
 #undef PM_RG_
+}
+
+// Tokens of a group: a wave walks its quarter of them four at a time (eight where eight lanes share a token), k searches each, one latency
+// after the other, so groups are small as long as each finds a compute unit; more than that and the groups take turns.  Up to 64 tokens are one
+// group, which needs no second launch.  us, both launches, with groups of 64, 32 and 16 tokens (experts, choices):
+//   8, 2    1000 tokens 11.2, 10.1, 10.3   4096 11.6, 10.7, 11.0   8192 12.3, 11.0, 13.6   16384 14.3, 14.7, 17.9
+//   10, 3   1000 18.5, 15.3, 12.9          4096 19.3, 15.2, 13.3   8192 20.3, 16.6, 16.6   12000 22.1, 20.4, 20.5   32768 35.8, 32.5, 46.6
+//   24, 2   1000 20.6, 17.8, 14.7          4096 21.8, 17.7, 15.4   8192 22.3, 18.7, 20.3   16384 22.7, 23.0, 28.1
+//   64, 8   1000 68.9, 43.8, 30.6          4096 69.0, 45.5, 34.7   8192 70.6, 48.4, 44.6   16384 73.8, 59.2, 64.2
+static int route_group_tokens(int experts, int samples)
+{
+    if (experts > 8 && (samples <= 16 || (samples > 64 && samples <= 16 * 256))) return 16;
+    return samples <= 32 || (samples > 64 && samples <= 32 * 256) ? 32 : 64;
 }
 
 int route_groups(const void *input, int dtype, int is_logits, const float *logit_bias, int samples, int experts,
@@ -584,21 +599,23 @@ int route_groups(const void *input, int dtype, int is_logits, const float *logit
 {
     FwdPlan plan;
     plan.k = top_k < experts ? top_k : experts;
-    plan.group_tokens = 64;
-    plan.groups = (samples + 63) / 64;
+    plan.group_tokens = route_group_tokens(experts, samples);
+    plan.groups = (samples + plan.group_tokens - 1) / plan.group_tokens;
     plan.experts_per_block = go_experts_per_block(experts, plan.k);
     plan.blocks = (experts + plan.experts_per_block - 1) / plan.experts_per_block;
     plan.merged = false;
     workspace = fwd_tables(workspace);
     plan.ws = fwd_ws(workspace, plan.groups, plan.k, experts, samples);
     const int mode = is_logits ? 1 : 2;
-#define PM_ROUTE(ONE) PM_DTYPE_SWITCH(dtype, SDT, (launch_route_groups<SDT, ONE>(experts, plan.groups, mode, st, input, is_logits ? logit_bias : nullptr, \
+#define PM_ROUTE(GROUP, ONE) PM_DTYPE_SWITCH(dtype, SDT, (launch_route_groups<SDT, GROUP, ONE>(experts, plan.groups, mode, st, input, is_logits ? logit_bias : nullptr, \
                           samples, plan.k, normalize_gate, indices, locations, gates, stride, is_logits ? scores_out : nullptr, l_aux, counts, workspace)))
+#define PM_ROUTE_G(ONE) do { if (plan.group_tokens == 16) { PM_ROUTE(16, ONE) } else if (plan.group_tokens == 32) { PM_ROUTE(32, ONE) } else { PM_ROUTE(64, ONE) } } while (0)
     if (plan.groups == 1) {                      // (its slots are the final ones)
-        PM_ROUTE(ONE_ROUTING);
+        PM_ROUTE_G(ONE_ROUTING);
         return 0;
     }
-    PM_ROUTE(ONE_OFF);
+    PM_ROUTE_G(ONE_OFF);
+#undef PM_ROUTE_G
 #undef PM_ROUTE
     finish_routing(plan, indices, locations, stride, samples, experts, l_aux, counts, st);
     return 0;

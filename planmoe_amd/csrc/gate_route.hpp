@@ -66,7 +66,7 @@ enum { OUT_CODES = 0, OUT_ROWS = 1, OUT_DECODED = 2 };
 // NT > 1: weights shared through LDS, a wave per 16 tokens.
 // MODE 0: logits = x . wg^T computed here.  MODE 1 / 2: no GEMM; x holds the [samples, experts]
 // logits / scores in the routing dtype (the stand-alone routing entry point) and only the
-// epilogue runs, on 64-token groups.
+// epilogue runs.
 // ONE (not ONE_OFF): all tokens are one group, so what the group knows is all there is, and slots, loss and counts are
 // final.  OUT_ROWS / OUT_DECODED: the rows go to their slots as well; every work-group routes all tokens for itself, sends the
 // rows of four, and the first one writes the routing.  (A pass of the layer at 8 tokens x 1024, hidden 4096, 8 experts: 51.0 us
@@ -119,7 +119,7 @@ __device__ __forceinline__ void gate_route_group(
         lbias[q] = (MODE != 2 && logit_bias && e < experts) ? logit_bias[e] : 0.f;
     }
     constexpr bool STATS = DT == PLANMOE_BF16 && MODE == 0;
-    static_assert(MODE == 0 || (!SPLITK && GROUP == 64), "routing from memory runs on 64-token groups");
+    static_assert(MODE == 0 || !SPLITK, "routing from memory has one part");
     auto &pstat = sh.pstat;
     if constexpr (MODE != 0) {
         // the group's rows land where the GEMM would have left its logits: 8 loads in flight per

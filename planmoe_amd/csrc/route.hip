@@ -493,8 +493,8 @@ extern "C" int planmoe_route_topk(const void *input, int dtype, int input_is_log
                "planmoe_route_topk: workspace too small (%zu < %zu)", workspace_bytes,
                planmoe_route_workspace_bytes(samples, experts, top_k));
     if (experts <= 64) {
-        // lanes share a token and the experts of a row (softmax and arg-max as butterflies), 64-token
-        // groups: several times the parallelism of the thread-per-token tiles below
+        // lanes share a token and the experts of a row (softmax and arg-max as butterflies), groups of up to 64
+        // tokens: several times the parallelism of the thread-per-token tiles below
         if (route_groups(input, dtype, input_is_logits, logit_bias, samples, experts, top_k, normalize_gate, indices,
                          locations, gates, plane_stride, scores_out, l_aux, expert_counts, workspace, st)) return 1;
         PM_LAUNCH_CHECK("planmoe_route_topk");

@@ -46,6 +46,15 @@ def test_against_oracle(T, E, k):
     _check(tie_free_scores(T, E, k, seed=T + E), k)
 
 
+# groups of 16, 32 and 64 tokens: either side of where they change and of a group's end, with one group and with several
+@pytest.mark.parametrize("T,E,k", [(15, 9, 2), (16, 64, 8), (17, 16, 3), (16, 8, 8), (32, 8, 2), (33, 10, 3), (64, 33, 4), (65, 9, 1), (65, 8, 2), (80, 64, 64),
+                                   (81, 17, 5), (97, 5, 2), (4095, 10, 3), (4096, 64, 1), (4097, 24, 2), (8191, 48, 6), (8192, 2, 2), (8193, 16, 2),
+                                   (8193, 7, 1)])
+def test_group_sizes(T, E, k):
+    _check(tie_free_scores(T, E, k, seed=T + E), k)
+    _check(random_scores(T, E, seed=T, dtype=torch.bfloat16), k)
+
+
 @pytest.mark.parametrize("T,E,k", [(600000, 8, 2), (400000, 128, 2), (300001, 64, 1)])
 def test_many_tokens(T, E, k):
     """Token counts an order of magnitude above the configs (thousands of routing tiles / groups)."""
