@@ -537,14 +537,17 @@ static void fwd_plan(FwdPlan &plan, void *workspace, int samples, int experts, i
 }
 
 // ranks in groups -> final slots (and the loss and the expert counts): one launch in which every
-// wave sums the histogram columns it needs (top_k <= 4 and a small histogram), else the prefix
+// wave sums the histogram columns it needs (few choices, experts and groups), else the prefix
 // over the groups and a launch that adds it
 static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t *locations, int64_t stride,
                            int samples, int experts, float *l_aux, int32_t *counts, hipStream_t st)
 {
-    // measured: 38.4 vs 39.7 us (256 groups x 8 experts), 58.6 vs 45.2 us (512 groups x 64 experts, where
-    // nothing hides the one block that sums every column for the loss)
-    if (plan.k <= 4 && (int64_t)plan.groups * experts <= 8192) {
+    // One launch more takes 2 - 4 us.  Without it the first work-group sums every expert's column for the loss by itself, and every token's wave
+    // k (k + 1) / 2 columns.  us of the routing, in one launch and in two (experts, choices, tokens):
+    //   4, 1   20000 12.6, 16.2   32768 15.2, 17.4     8, 2   4096 10.7, 13.6   20000 16.6, 18.0   32768 21.0, 19.6     10, 3  4096 13.5, 16.7   12000 22.1, 22.7
+    //   16384 23.8, 23.1   32768 35.9, 28.3            16, 4  4096 15.7, 18.7   8192 20.5, 21.3    12000 27.7, 26.3     32, 4  8192 26.0, 27.2   16384 38.4, 35.6
+    //   48, 2  100 16.2, 15.7     1000 19.5, 16.2      64, 4  1000 27.1, 21.3   (more than 8192 entries a plane: 512 groups x 64 experts 58.6, 45.2)
+    if (plan.k <= 4 && experts <= 32 && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= 90000) {
         route_locations_merged_kernel<<<1 + (samples + 3) / 4, 256, 0, st>>>(
             indices, locations, stride, plan.k, samples, experts, plan.ws.rank, plan.group_tokens, plan.ws.hist_t,
             plan.ws.me_t, plan.groups, plan.ws.gstride, counts, l_aux);
