@@ -873,8 +873,8 @@ extern "C" int planmoe_gemm_tn_bf16(const void *a, const void *b, int batches, i
 }
 
 // ---------------------------------------------------------------- the experts' products on contiguous buffers
-static int expert_gemm_check(const char *who, int form, int dtype, const void *a, const void *b, int batches, int m, int n, int k,
-                             const int32_t *live, int live_planes, int live_round, const void *c)
+int pm::expert_gemm_check(const char *who, int form, int dtype, const void *a, const void *b, int batches, int m, int n, int k,
+                          const int32_t *live, int live_planes, int live_round, const void *c)
 {
     PM_REQUIRE(form >= 0 && form <= 2, "%s: form is 0 (a b), 1 (a b^T) or 2 (a^T b)", who);
     PM_REQUIRE(dtype == PLANMOE_BF16 || dtype == PLANMOE_F32, "%s: bf16 or fp32", who);

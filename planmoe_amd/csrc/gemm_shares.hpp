@@ -14,5 +14,8 @@ struct GemmShares {
 GemmShares gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs);
 // p.shares, p.live and at most 64 batches; the caller has checked shape and alignment (as planmoe_expert_gemm does)
 int gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who);
+// what planmoe_expert_gemm refuses of its operands and their sizes
+int expert_gemm_check(const char *who, int form, int dtype, const void *a, const void *b, int batches, int m, int n, int k,
+                      const int32_t *live, int live_planes, int live_round, const void *c);
 
 } // namespace pm

@@ -10,6 +10,7 @@
 // Bound by reading the weights and the gate's latency under it.  A pass of 8 tokens x 1024, hidden 4096, 8 experts, weights cold: see
 // planmoe_layer_dispatch_product.
 #include "gate_route.hpp"
+#include "gemm_shares.hpp"
 #include "gemm_skinny_core.hpp"
 
 namespace pm {
@@ -134,7 +135,7 @@ static int first_launch(const SkinnyArgs &p, const FirstArgs &r, hipStream_t str
 }
 
 // Up to 32 tokens (one routing group), 16 experts, 4 choices and 16 rows an expert, and a compute unit for each work-group: a second
-// round of work-groups would route once more.
+// round of work-groups would route once more.  (Rows are below 4 MB, as the products ask for, so that one descriptor covers x.)
 static bool first_serves(int dtype, int fp32_gate, int samples, int model_dim, int experts, int top_k, int capacity, int hidden)
 {
     if (dtype != PLANMOE_BF16 || !fp32_gate || samples > FIRST_TOKENS || experts > 16 || (top_k < experts ? top_k : experts) > 4) return false;
@@ -156,9 +157,11 @@ extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int
 {
     const char *who = "planmoe_layer_dispatch_product";
     PM_REQUIRE(expert_counts, "%s: NULL routing output", who);
-    const bool shape = x && wg && w1 && h && indices && locations && gates && samples >= 1 && model_dim >= 8 && model_dim % 8 == 0 && experts >= 1 && top_k >= 1 &&
-                       hidden >= 8 && hidden % 8 == 0 && plane_stride >= samples && (codec == 0 || codec == 1) && aligned16(x) && aligned16(wg) && aligned16(w1) && aligned16(h);
-    // (a call that is not well formed goes on to the entry points that say what is wrong with it)
+    PM_REQUIRE(top_k >= 1, "%s: bad shape", who);
+    // what the product would refuse, before anything is enqueued: its operands' ranges (the rows come from x where there is one launch), too
+    if (expert_gemm_check(who, 0, dtype, x, w1, experts, capacity, hidden, model_dim, expert_counts, top_k < experts ? top_k : experts, 1, h)) return 1;
+    const bool shape = wg && indices && locations && gates && samples >= 1 && plane_stride >= samples && (codec == 0 || codec == 1) && aligned16(wg);
+    // (a call that is not well formed goes on to the entry point that says what is wrong with it)
     if (!shape || !first_serves(dtype, fp32_gate, samples, model_dim, experts, top_k, capacity, hidden)) {
         if (planmoe_layer_dispatch(x, wg, dtype, fp32_gate, nullptr, samples, model_dim, experts, top_k, normalize_gate, capacity, codec, indices, locations,
                                    gates, plane_stride, nullptr, l_aux, expert_counts, rows, workspace, workspace_bytes, stream)) return 1;

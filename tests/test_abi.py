@@ -88,6 +88,19 @@ def test_argument_errors_are_reported_without_a_gpu():
     assert lib.planmoe_combine_fwd(None, 0, None, ctypes.c_void_p(16), ctypes.c_void_p(16), 0, 1, 0, 8, 4, None, None) == 0
 
 
+# One launch or two: what the product refuses is refused, before the dispatch is enqueued.  (The one launch covers x, and a row's place in
+# it, by 32-bit offsets: rows of 2^25 values and 32 tokens were out of their range, and taken.)
+@pytest.mark.parametrize("tokens,dim,hidden,dtype,capacity,says", [
+    (2, 1 << 22, 8, 1, 4, b"2 GiB"), (32, 1 << 25, 8, 1, 4, b"2 GiB"), (2, 8, 1 << 22, 1, 4, b"2 GiB"), (2, 1 << 21, 8, 0, 4, b"2 GiB"),
+    (2, 64, 12, 1, 4, b"multiple of 8"), (40, 64, 12, 1, 4, b"multiple of 8"), (2, 64, 64, 2, 4, b"bf16 or fp32"), (2, 64, 64, 1, 0, b"shape")])
+def test_first_product_refuses_what_the_product_refuses(tokens, dim, hidden, dtype, capacity, says):
+    from planmoe_amd._lib import lib
+    p16 = ctypes.c_void_p(16)
+    rc = lib.planmoe_layer_dispatch_product(p16, p16, dtype, 1, tokens, dim, 1, 1, 1, capacity, 0, p16, p16, p16, tokens, p16, p16, p16, p16, hidden, 1,
+                                            p16, p16, p16, 1 << 40, None)
+    assert rc != 0 and b"planmoe_layer_dispatch_product" in lib.planmoe_last_error() and says in lib.planmoe_last_error(), lib.planmoe_last_error()
+
+
 def test_size_queries():
     from planmoe_amd import ops
     assert ops.zfp_stream_bytes(2, 1024, 131072) == 1024 * 131072          # 8 bits per value
