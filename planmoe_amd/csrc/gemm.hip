@@ -784,20 +784,20 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
 //   8 x 32, same                         37.5 -> 17.9 (4)             8 x 64, same      41.2 -> 19.4 (4)       8 x 128, same  43.9 -> 27.7 (2)
 //   8 x 32, 2048 -> 2048                 25.2 -> 17.5 (2)             4 x 32, 2048 -> 512   14.7 -> 6.0 (8)    4 x 512, same  17.3 -> 12.8 (3)
 //   2 of 8 experts with a row, 4096 -> 4096  26.5 -> 13.6 (2)         4096 -> 1024, same    16.8 -> 4.8 (8)
-GemmShares pm::gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs)
+GemmShares pm::gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, int64_t most)
 {
     const int64_t cu = compute_units();
     const int active = (int)std::min<int64_t>(batches, pairs);
     if (n * k * 2 >= ((int64_t)1 << 31) || batches > 64) return GemmShares{};
     if (gemm_is_skinny(false, m, n, k, batches)) {
-        const int64_t groups = (int64_t)((n + 63) / 64) * active, splits = std::min<int64_t>({groups > 0 ? cu / groups : 0, k / 512, 8});
+        const int64_t groups = (int64_t)((n + 63) / 64) * active, splits = std::min<int64_t>({groups > 0 ? cu / groups : 0, k / 512, 8, most});
         // (one share: where fewer experts than there are have rows, and the whole product would take them in wider columns)
         if (splits >= 2 || (splits == 1 && active < batches && gemm_skinny_width(false, n, k, batches) > 64)) return GemmShares{(int)splits, active, true};
         return GemmShares{};
     }
     if (!gemm_deep_reaches(0, m, n, k)) return GemmShares{};
     const double tiles = GemmCost{(double)std::min<int64_t>(rows, m), 0., (double)cu, m, n, batches, 0, true}.tiles(128, 128);
-    const int64_t k_tiles = (k + DEEP_BK - 1) / DEEP_BK, splits = std::min<int64_t>({(int64_t)((double)cu / tiles), k_tiles / 4, 8});
+    const int64_t k_tiles = (k + DEEP_BK - 1) / DEEP_BK, splits = std::min<int64_t>({(int64_t)((double)cu / tiles), k_tiles / 4, 8, most});
     if (splits < 2) return GemmShares{};
     const int64_t each = (k_tiles + splits - 1) / splits;
     return GemmShares{(int)((k_tiles + each - 1) / each), active, false};      // (none of them empty)

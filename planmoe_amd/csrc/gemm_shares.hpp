@@ -10,8 +10,8 @@ struct GemmShares {
     bool few = false;             // gemm_skinny.hip's kernel, else gemm_deep.hip's
 };
 
-// m, n, k: rows at most of a batch, columns, reduction; rows: expected of a batch; pairs: rows of all batches at most
-GemmShares gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs);
+// m, n, k: rows at most of a batch, columns, reduction; rows: expected of a batch; pairs: rows of all batches at most; most: shares at most
+GemmShares gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, int64_t most);
 // p.shares, p.live and at most 64 batches; the caller has checked shape and alignment (as planmoe_expert_gemm does)
 int gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who);
 // what planmoe_expert_gemm refuses of its operands and their sizes

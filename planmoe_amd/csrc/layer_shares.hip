@@ -44,6 +44,11 @@ __global__ __launch_bounds__(256) void combine_shares_kernel(const RowShares row
     if (u < units) stream_store(reinterpret_cast<uint4 *>(out + (int64_t)t * rows.model_dim) + u, E::pack(acc));
 }
 
+// The planes have a row for every slot, used or not, so a capacity far beyond the rows that are expected (no token dropped: as many slots an expert
+// as there are tokens) would have them take many times what is read: 64 experts of 8192 slots x 128 values, 4 shares, 1 GB beside rows of 134 MB.
+// The rows in use of a chip full of tiles are 17 MB altogether; four times that is where shares become fewer, or the product whole.
+constexpr int64_t SHARES_BYTES = (int64_t)64 << 20;
+
 static GemmShares shares_of(int dtype, int codec, int hidden, int top_k, int samples, int model_dim, int experts, int capacity, int rows_hint)
 {
     // (vectors of 8 values, up to 64 choices a lane each, rows of the codec's kernel in registers; elsewhere the general path)
@@ -51,7 +56,8 @@ static GemmShares shares_of(int dtype, int codec, int hidden, int top_k, int sam
     if (experts < 1 || experts > 64 || top_k < 1 || top_k > experts || samples < 1 || capacity < 1) return GemmShares{};
     if ((int64_t)(hidden > model_dim ? hidden : model_dim) * 512 >= ((int64_t)1 << 31) || (int64_t)experts * capacity >= ((int64_t)1 << 31)) return GemmShares{};
     const int hint = rows_hint >= 1 && rows_hint < capacity ? rows_hint : capacity;
-    return gemm_shares_pick(capacity, model_dim, hidden, experts, hint, (int64_t)samples * top_k);
+    const int64_t most = SHARES_BYTES / ((int64_t)experts * capacity * model_dim * 4);
+    return gemm_shares_pick(capacity, model_dim, hidden, experts, hint, (int64_t)samples * top_k, most);
 }
 
 } // namespace pm

@@ -101,6 +101,18 @@ def test_first_product_refuses_what_the_product_refuses(tokens, dim, hidden, dty
     assert rc != 0 and b"planmoe_layer_dispatch_product" in lib.planmoe_last_error() and says in lib.planmoe_last_error(), lib.planmoe_last_error()
 
 
+# The shares of a second product have a row for every slot: whatever the capacity, they stay small beside what a pass holds anyway
+@pytest.mark.parametrize("tokens,dim,hidden,experts,top_k", [(8192, 128, 4096, 64, 1), (4096, 256, 4096, 16, 2), (64, 1024, 4096, 8, 2), (1, 4096, 4096, 64, 2), (2000, 512, 2048, 4, 1)])
+def test_shares_do_not_grow_with_the_capacity(tokens, dim, hidden, experts, top_k):
+    from planmoe_amd._lib import lib
+    hint = max(1, tokens * top_k // experts)
+    for capacity in sorted({max(4, hint), 32, 4 * hint, tokens, 65536}):
+        plane = experts * capacity * dim * 4
+        for codec in (0, 1):
+            size = lib.planmoe_layer_product_combine_workspace_bytes(1, codec, hidden, top_k, tokens, dim, experts, capacity, hint)
+            assert size % plane == 0 and size <= 64 << 20, (capacity, codec, size)
+
+
 def test_size_queries():
     from planmoe_amd import ops
     assert ops.zfp_stream_bytes(2, 1024, 131072) == 1024 * 131072          # 8 bits per value

@@ -729,6 +729,16 @@ def test_product_in_shares_and_combine(T, M, H, E, k, cap, skewed, with_bias):
     assert torch.equal(codes, want_codes) and torch.equal(mn, want_mn) and torch.equal(scale, want_scale)
 
 
+# a capacity that leaves room for fewer shares than the eight that there would be
+@pytest.mark.parametrize("T,M,H,E,k,cap,splits", [(64, 512, 2048, 4, 2, 2048, 4), (64, 512, 2048, 4, 2, 4096, 2)])
+def test_product_in_fewer_shares(T, M, H, E, k, cap, splits):
+    from planmoe_amd._lib import lib
+    hint = min(cap, (T * k + E - 1) // E)
+    assert lib.planmoe_layer_product_combine_workspace_bytes(1, 0, H, k, T, M, E, cap, hint) == splits * E * cap * M * 4
+    assert lib.planmoe_layer_product_combine_workspace_bytes(1, 0, H, k, T, M, E, cap // 2, hint) == 2 * splits * E * (cap // 2) * M * 4
+    test_product_in_shares_and_combine(T, M, H, E, k, cap, False, True)
+
+
 # The combine that adds the gate's share of the gradient of x, for 9 to 16 experts: against the combine as it is and the product in 64 bits.  One token,
 # an odd number (two a wave in fp32), rows of one piece, of one more than a wave's 64 and of 8 KB; choices without a slot
 @pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 9, 1, 1), (5, 520, 16, 2, 1), (301, 1032, 11, 3, 40), (64, 2048, 16, 2, 8), (33, 4096, 16, 2, 4)])
