@@ -173,11 +173,16 @@ extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int
     hipStream_t st = (hipStream_t)stream;
     const int width = gemm_skinny_width(false, hidden, model_dim, experts);
     const bool large = skinny_large(hidden, model_dim, experts);
-#define PM_FIRST_(C, U, LARGE)                                                                                          \
-    (experts <= 8 ? (codec ? first_launch<8, true, C, U, LARGE>(p, r, st, who) : first_launch<8, false, C, U, LARGE>(p, r, st, who))      \
-                  : (codec ? first_launch<16, true, C, U, LARGE>(p, r, st, who) : first_launch<16, false, C, U, LARGE>(p, r, st, who)))
-#define PM_FIRST(C, U) (large ? PM_FIRST_(C, U, true) : PM_FIRST_(C, U, false))
-    return width == 32 ? PM_FIRST_(2, 8, true) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
+// (U8: steps on their way through the codec)
+#define PM_FIRST_(C, U, U8, LARGE)                                                                                      \
+    (experts <= 8 ? (codec ? first_launch<8, true, C, U8, LARGE>(p, r, st, who) : first_launch<8, false, C, U, LARGE>(p, r, st, who))     \
+                  : (codec ? first_launch<16, true, C, U8, LARGE>(p, r, st, who) : first_launch<16, false, C, U, LARGE>(p, r, st, who)))
+#define PM_FIRST(C, U) (large ? PM_FIRST_(C, U, U, true) : PM_FIRST_(C, U, U, false))
+    // (32 columns through the codec, whose values take registers: of eight steps seven registers were spilled, and a load that is spilled is waited
+    // for.  us, 1 token, weights in the last cache and cold, two launches, eight steps, four:
+    //   8 experts, 1024 -> 1024   11.7, 10.8, 9.1    13.0, 13.3, 10.6      4 experts, 4096 -> 2048   22.6, 31.7, 22.9    29.8, 33.8, 25.3
+    //   8 experts, 2048 -> 1024   14.8, 17.7, 13.8   18.6, 20.1, 17.0      8 experts, 4096 -> 1024   21.4, 31.2, 22.7    29.3, 33.2, 25.4)
+    return width == 32 ? PM_FIRST_(2, 8, 4, true) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
 #undef PM_FIRST
 #undef PM_FIRST_
 }
