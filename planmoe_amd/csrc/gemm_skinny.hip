@@ -18,7 +18,8 @@
 namespace pm {
 
 // MF: 16-row fragments; C: 16-column fragments of the weight, a work-group's columns / 16; U: steps of the reduction a wave has in flight;
-// LARGE: the weight does not stay in the caches anyway (skinny_large): read nontemporally (nt: not, the two loads of 128 bytes meet in the cache)
+// LARGE: the weight does not stay in the caches anyway (skinny_large): read nontemporally (nt: not, the two loads of 128 bytes meet in the cache; nn in
+// 32 columns: not, two work-groups' halves of a line do)
 // SHARES: a grid of (column groups, batches that can have rows, shares of the reduction); the y-th batch is the y-th that has rows
 template <bool NT, int MF, int C, int U, int WAVES, bool GRAD, bool LARGE, bool SHARES = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArgs p)
@@ -38,7 +39,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const SkinnyArg
         rows = __builtin_amdgcn_readlane(n, e);
         n0 = blockIdx.x * 16 * C;
     } else {
-        skinny_tile<16 * C, LARGE && C == 2>(e, n0);
+        skinny_tile<16 * C, C == 2 && (LARGE || !NT)>(e, n0);
     }
     if (!SHARES && p.live) {
         int n = 0;
@@ -140,7 +141,9 @@ static int skinny_launch(const SkinnyArgs &p, hipStream_t stream, const char *wh
 }
 
 // From 16 MB on a weight is read past the caches; below, the next call may find it there (us, plain and nontemporal: 8 experts x 2,
-// 512 -> 512 4.0, 5.2; 4 x 2, 1024 -> 1024 4.7, 5.6; 8 x 2, 1024 -> 1024 6.8, 6.8; 16 x 2, 1024 -> 1024 8.8, 7.9).
+// 512 -> 512 4.0, 5.2; 4 x 2, 1024 -> 1024 4.7, 5.6; 8 x 2, 1024 -> 1024 6.8, 6.8; 16 x 2, 1024 -> 1024 8.8, 7.9).  What a model's other layers
+// have pushed out of the last cache (256 MB) gains by it; a weight that the same call read before loses: 8 x 8, 2048 -> 2048 in 64
+// columns 16.6, 14.6 cold and 11.9, 12.7 in the cache; 16 x 8, 1024 -> 4096 27.8, 25.5 and 21.9, 24.2.
 bool skinny_large(int64_t n, int64_t k, int64_t batches) { return n * k * batches * 2 >= (int64_t)16 << 20; }
 
 // Columns of a work-group: 32 or 64 where that leaves a compute unit for each work-group (one compute unit gets at most 28 GB/s
@@ -153,7 +156,11 @@ bool skinny_large(int64_t n, int64_t k, int64_t batches) { return n * k * batche
 //   4 x 2, 4096 -> 512                  nn 16.4, 18.3, -, 24      nt 11, 19, -, 26
 //   8 x 20, 4096 -> 1024                nn 22.4, 25, -, 35        nt 17.4, 24, -, 43
 //   8 x 8, 2688 -> 2560                 nn 37, 30, 29, 23         nt 24, 33, 23, 29
-// (nn in 32 columns reads 64 bytes of a row, two work-groups a line: it takes the compute units that 64 leave idle, but no more)
+// (nn in 32 columns reads 64 bytes of a row, two work-groups a line: it takes the compute units that 64 leave idle, but no more.  Not nontemporally, or
+// the second of them finds its half gone.  us in 64 columns, in 32 nontemporal and in 32, weights in the last cache and cold:
+//   8 x 8, 4096 -> 1024    13.9, 18.2, 14.5    23.9, 20.0, 20.8      4 x 8, 4096 -> 1024    12.4, 13.5, 10.9    21.1, 18.6, 19.1
+//   8 x 24, same           17.6, 22.9, 16.6    27.8, 23.9, 24.2      8 x 8, 3072 -> 768     12.0, 11.6, 9.0     17.4, 13.8, 14.0
+//   8 x 8, 8192 -> 512     23.2, 32.8, 21.3    39.4, 35.2, 34.9      16 x 8, 8192 -> 256    22.5, 29.1, 18.8    34.6, 30.8, 31.0)
 int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
 {
     const bool grad = p.mask != nullptr, large = skinny_large(p.N, p.K, p.batches);
@@ -164,7 +171,7 @@ int gemm_skinny_run(bool nt, SkinnyArgs p, hipStream_t stream, const char *who)
     const int width = gemm_skinny_width(nt, p.N, p.K, p.batches);
     const bool few = p.M <= 16;
     if (!nt) {
-        if (width == 32) return few ? skinny_launch<false, 1, 2, 8, 16, false, true>(p, stream, who) : skinny_launch<false, 2, 2, 8, 8, false, true>(p, stream, who);
+        if (width == 32) return few ? skinny_launch<false, 1, 2, 8, 16, false, false>(p, stream, who) : skinny_launch<false, 2, 2, 8, 8, false, false>(p, stream, who);
         if (width == 64) return few ? PM_SK_NN(1, 4, 2, 16) : PM_SK_NN(2, 4, 2, 16);
         return few ? PM_SK_NN(1, 8, 1, 16) : PM_SK_NN(2, 8, 1, 16);
     }

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(FIRST_WAVES * 64) void layer_first_kernel(const Ski
     __shared__ int32_t s_token[FIRST_ROWS];                 // the expert's rows
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int e, n0;
-    skinny_tile<16 * C, LARGE && C == 2>(e, n0);
+    skinny_tile<16 * C, C == 2>(e, n0);
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(r.x), 0, r.samples * p.K * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.B + (int64_t)e * p.N * p.K), 0, (int)((int64_t)p.N * p.K * 2), 0x00020000);
     const int l16 = lane & 15, g = lane >> 4, steps = (p.K + 31) / 32;
@@ -182,7 +182,9 @@ extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int
     // for.  us, 1 token, weights in the last cache and cold, two launches, eight steps, four:
     //   8 experts, 1024 -> 1024   11.7, 10.8, 9.1    13.0, 13.3, 10.6      4 experts, 4096 -> 2048   22.6, 31.7, 22.9    29.8, 33.8, 25.3
     //   8 experts, 2048 -> 1024   14.8, 17.7, 13.8   18.6, 20.1, 17.0      8 experts, 4096 -> 1024   21.4, 31.2, 22.7    29.3, 33.2, 25.4)
-    return width == 32 ? PM_FIRST_(2, 8, 4, true) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
+    // (and not nontemporally, see gemm_skinny.hip: without the codec, 1 token, nontemporal and not, 8 experts, 4096 -> 1024 22.2, 18.3 and 24.8, 25.5;
+    // 4 experts, 4096 -> 2048 22.5, 17.9 and 24.3, 25.4; 8 experts, 8192 -> 1024 38.5, 28.7 and 40.7, 40.2)
+    return width == 32 ? PM_FIRST_(2, 8, 4, false) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
 #undef PM_FIRST
 #undef PM_FIRST_
 }
