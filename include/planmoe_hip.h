@@ -499,7 +499,11 @@ int planmoe_layer_dispatch_product(const void *x, const void *wg, int dtype, int
  * [experts, model_dim] or NULL, for the rows in use by expert_counts [top_k][experts], rounded up to count_round), and the combine of its rows
  * (planmoe_layer_combine; codes not NULL: planmoe_layer_combine_keep).  expert_counts are the routing's own: no more than samples * top_k rows
  * altogether.  `rows` [experts, capacity, model_dim]: with keep_rows it holds the rows that tokens have afterwards (codec 0), else it is scratch.
- * Workspace: ..._workspace_bytes of the same sizes; 0, and not looked at, where the product is computed whole. */
+ * Workspace: ..._workspace_bytes of the same sizes; 0, and not looked at, where the product is computed whole.
+ * ..._pays: whether that is faster than planmoe_expert_gemm and planmoe_layer_combine by themselves (0: it is not, or the product is computed
+ * whole here, too). */
+int planmoe_layer_product_combine_pays(int dtype, int codec, int hidden, int top_k, int samples, int model_dim,
+                                       int experts, int capacity, int rows_hint);
 size_t planmoe_layer_product_combine_workspace_bytes(int dtype, int codec, int hidden, int top_k, int samples, int model_dim,
                                                      int experts, int capacity, int rows_hint);
 int planmoe_layer_product_combine(const void *h, const void *w2, const void *b2, int dtype, int codec, int hidden, const float *gates,

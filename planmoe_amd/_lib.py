@@ -94,6 +94,7 @@ SIGNATURES = {
     "planmoe_layer_dispatch_product": (c_int, [c_void_p, c_void_p] + [c_int] * 9 + [c_void_p] * 3 + [c_int64] + [c_void_p] * 4 + [c_int] * 2
                                        + [c_void_p] * 3 + [c_size_t, c_void_p]),
     "planmoe_layer_product_combine_workspace_bytes": (c_size_t, [c_int] * 9),
+    "planmoe_layer_product_combine_pays": (c_int, [c_int] * 9),
     "planmoe_layer_product_combine": (c_int, [c_void_p] * 3 + [c_int] * 3 + [c_void_p] * 3 + [c_int64] + [c_int] * 5 + [c_void_p] + [c_int] * 2
                                       + [c_void_p, c_int] + [c_void_p] * 5 + [c_size_t, c_void_p]),
     "planmoe_layer_combine": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,

@@ -23,10 +23,11 @@ struct Shape {
     int64_t rows() const { return (int64_t)E * cap; }
     // rows an expert is expected to have in use: what the products pick their tiles by
     int hint() const { return (int)std::min<int64_t>(cap, ((int64_t)T * k + E - 1) / E); }
-    // what the second product leaves for the combine to add up
+    // what the second product leaves for the combine to add up, where that is the faster way
     size_t shares(int codec) const
     {
-        return codec > CODEC_INT8 ? 0 : planmoe_layer_product_combine_workspace_bytes(dt, codec == CODEC_INT8, H, k, T, M, E, cap, hint());
+        if (codec > CODEC_INT8 || !planmoe_layer_product_combine_pays(dt, codec == CODEC_INT8, H, k, T, M, E, cap, hint())) return 0;
+        return planmoe_layer_product_combine_workspace_bytes(dt, codec == CODEC_INT8, H, k, T, M, E, cap, hint());
     }
 };
 
@@ -141,6 +142,21 @@ bool dx_in_one(const Shape &s, int codec)
     return codec != CODEC_INT8 || (s.T <= 8192 && values <= (1 << 23));
 }
 
+// The second product and the combine, without a codec or through the int8 codec; kept: its codes, keep: the rows without it, for a backward pass
+void product_combine(const Shape &s, int codec, const void *h, const Tensor &w2, const Tensor &b2, const float *gates, const int32_t *idx, const int32_t *loc,
+                     const int32_t *cnt, void *ye, bool keep, const Kept &kept, const Tensor &y, void *shares_at, size_t shares, void *st)
+{
+    const int coded = codec == CODEC_INT8;
+    if (shares > 0) {
+        PM_CALL(planmoe_layer_product_combine(h, w2.data_ptr(), b2.data_ptr(), s.dt, coded, s.H, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt, 1, s.hint(), ye,
+                                              keep, kept.codes, kept.bias, kept.scale, y.data_ptr(), shares_at, shares, st));
+        return;
+    }
+    PM_CALL(planmoe_expert_gemm(0, s.dt, h, w2.data_ptr(), b2.data_ptr(), 0, s.E, s.cap, s.M, s.H, cnt, s.k, 1, s.hint(), ye, st));
+    if (kept.codes) PM_CALL(planmoe_layer_combine_keep(ye, s.dt, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), kept.codes, kept.bias, kept.scale, st));
+    else PM_CALL(planmoe_layer_combine(ye, s.dt, coded, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, y.data_ptr(), st));
+}
+
 Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Tensor &b1, const Tensor &w2, const Tensor &b2, const Shape &s,
                   bool fp32_gate, bool normalize, int codec, bool keep)
 {
@@ -189,9 +205,7 @@ Pass forward_pass(const Tensor &x, const Tensor &wg, const Tensor &w1, const Ten
             p.codes = bytes(Kept::bytes(s, x.element_size()), x);
             kept = Kept(p.codes, s, x.element_size());
         }
-        PM_CALL(planmoe_layer_product_combine(p.h.data_ptr(), w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, gates, idx, loc, s.T, s.k, s.T,
-                                              s.M, s.E, s.cap, cnt, 1, s.hint(), p.ye.data_ptr(), keep, kept.codes, kept.bias, kept.scale, p.y.data_ptr(),
-                                              ws.data_ptr<uint8_t>() + ws_bytes, shares, st));
+        product_combine(s, codec, p.h.data_ptr(), w2, b2, gates, idx, loc, cnt, p.ye.data_ptr(), keep, kept, p.y, ws.data_ptr<uint8_t>() + ws_bytes, shares, st);
         if (p.codes.defined()) p.ye = Tensor();
         return p;
     }
@@ -243,8 +257,7 @@ std::tuple<Tensor, Tensor> inference_pass(const Tensor &x, const Tensor &wg, con
         gates = (const float *)(base + wide_at);
     }
     if (codec != CODEC_ZFP) {
-        PM_CALL(planmoe_layer_product_combine(h, w2.data_ptr(), b2.data_ptr(), s.dt, codec == CODEC_INT8, s.H, gates, idx, loc, s.T, s.k, s.T, s.M, s.E, s.cap, cnt,
-                                              1, s.hint(), ye, 0, nullptr, nullptr, nullptr, y.data_ptr(), base + shares_at, shares, st));
+        product_combine(s, codec, h, w2, b2, gates, idx, loc, cnt, ye, false, Kept{}, y, base + shares_at, shares, st);
         return {y, l_aux};
     }
     PM_CALL(planmoe_expert_gemm(0, s.dt, xe, w1.data_ptr(), b1.data_ptr(), 1, s.E, s.cap, s.H, s.M, cnt, s.k, 4, s.hint(), h, st));

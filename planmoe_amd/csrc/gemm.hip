@@ -779,11 +779,6 @@ int gemm_run(GemmArgs p, int64_t rows_hint, hipStream_t stream, const char *who,
 // In shares (layer_shares.hip): where the work-groups that the weight's columns make, for the experts that can have rows, leave half of the compute
 // units without one.  Up to 32 rows 64 columns (whole lines of 128 bytes) and shares of at least 512 k, 16 steps for 16 waves; beyond, tiles of
 // 128 x 128 and shares of at least 4 k-tiles.  Up to eight: the combine reads them all.
-// us whole and in shares (the combine apart), weights cold:
-//   8 experts x 2 rows, 4096 -> 1024     19.3 -> 13.8 (2 shares)      8 x 16, same      23.3 -> 16.4 (2)
-//   8 x 32, same                         37.5 -> 17.9 (4)             8 x 64, same      41.2 -> 19.4 (4)       8 x 128, same  43.9 -> 27.7 (2)
-//   8 x 32, 2048 -> 2048                 25.2 -> 17.5 (2)             4 x 32, 2048 -> 512   14.7 -> 6.0 (8)    4 x 512, same  17.3 -> 12.8 (3)
-//   2 of 8 experts with a row, 4096 -> 4096  26.5 -> 13.6 (2)         4096 -> 1024, same    16.8 -> 4.8 (8)
 GemmShares pm::gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, int64_t most)
 {
     const int64_t cu = compute_units();
@@ -801,6 +796,36 @@ GemmShares pm::gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t ro
     if (splits < 2) return GemmShares{};
     const int64_t each = (k_tiles + splits - 1) / splits;
     return GemmShares{(int)((k_tiles + each - 1) / each), active, false};      // (none of them empty)
+}
+
+// Product and combine together, against the whole product (in 32 or 64 columns, where that leaves compute units without a tile) and the
+// combine of its rows.  Up to 32 rows: from 1536 k on; from 1024 on where fewer experts than there are have rows.  Tiles: the k-tiles that a
+// work-group has fewer, 0.2 us each, against 2 us and 0.3 for every MB of shares; with no more work-groups than the whole product has of tiles of 64
+// columns only where an expert's rows are a whole tile's and more (its weight is read by half as many).  Through the codec a wave adds up a row's
+// shares, 512 values at a time: 1.5 us each, twice that with more than four; for few rows, whose whole product takes less, only rows of up to
+// 512, or 1024 with a reduction of 4096.  Top-2, us whole and in shares, weights in the last cache and cold, without the codec, then through it:
+//   8 experts, 4096 -> 1024     4 tokens 14.4, 14.7 and 22.3, 16.2     128: 21.2, 18.9 and 31.3, 22.5     512: 26.6, 23.7 and 40.5, 32.2
+//                                        15.4, 17.8     23.1, 19.3          22.0, 22.1     32.1, 25.8          27.6, 26.8     41.0, 35.2
+//   4 experts, 2048 -> 512      4        9.7, 7.7       10.1, 8.1      128: 13.1, 12.7     14.4, 12.9     512: 13.9, 17.5     16.5, 17.7 *
+//                                        9.9, 8.6       10.4, 9.0           13.4, 13.6     14.7, 13.8 *        14.2, 18.3     16.7, 18.5 *
+//   8 experts, 2048 -> 2048     1        9.7, 7.8       13.9, 9.9      128: 17.6, 18.5     22.3, 23.0 *   400: 21.0, 21.7     25.9, 25.6
+//                                        11.2, 13.5     15.5, 15.8 *        19.2, 26.8     23.8, 31.4 *        22.7, 29.3     27.4, 33.3 *
+//   4 experts, 1024 -> 1024     1        7.1, 7.1       7.2, 7.4       128: 10.7, 11.6     11.4, 11.8 *   512: 11.9, 19.1     12.8, 18.9 *
+//   16 experts, 4096 -> 1024    256      27.8, 28.5     34.8, 37.2 *   (* computed whole)
+// 254 shapes (256 to 4096 columns, 512 to 4096 k, 1 to 2048 tokens), against the whole product each: 0.91 in the last cache, 0.81 cold; with the shares wherever
+// they fit 0.95 and 0.82, through the codec 1.14 and 0.97, now 0.96 and 0.89.
+bool pm::gemm_shares_pay(const GemmShares &how, int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, bool coded)
+{
+    if (how.splits == 0) return false;
+    if (how.few) {
+        if (coded && !(n <= 512 || (n <= 1024 && k >= 4096))) return false;
+        return k >= 1536 || (k >= 1024 && how.active < batches);
+    }
+    const GemmCost cost{(double)std::min<int64_t>(rows, m), 0., (double)compute_units(), m, n, batches, 0, true};
+    const int64_t k_tiles = (k + DEEP_BK - 1) / DEEP_BK, each = (k_tiles + how.splits - 1) / how.splits;
+    if (how.splits * cost.tiles(128, 128) < 1.25 * cost.tiles(128, 64)) return rows > 96 && (coded ? k_tiles >= 64 && n <= 1024 : k_tiles >= 32);
+    const double mb = 4e-6 * how.splits * n * (double)std::min<int64_t>(pairs, (int64_t)batches * m);
+    return 0.2 * (double)(k_tiles - each) > 2. + 0.3 * mb + (coded ? 1.5 * ((n + 511) / 512) * (how.splits > 4 ? 2 : 1) : 0.);
 }
 
 int pm::gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who)

@@ -12,6 +12,8 @@ struct GemmShares {
 
 // m, n, k: rows at most of a batch, columns, reduction; rows: expected of a batch; pairs: rows of all batches at most; most: shares at most
 GemmShares gemm_shares_pick(int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, int64_t most);
+// Whether they are the faster way, the combine's share of the work with them; coded: the combine takes the rows through the int8 codec
+bool gemm_shares_pay(const GemmShares &how, int m, int n, int64_t k, int batches, int64_t rows, int64_t pairs, bool coded);
 // p.shares, p.live and at most 64 batches; the caller has checked shape and alignment (as planmoe_expert_gemm does)
 int gemm_shares_run(const GemmShares &how, SkinnyArgs p, hipStream_t stream, const char *who);
 // what planmoe_expert_gemm refuses of its operands and their sizes

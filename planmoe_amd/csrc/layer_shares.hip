@@ -1,12 +1,11 @@
 // The layer's second product and the combine behind it.
 //
 // Where the product has few columns the weight is read by few compute units, and one compute unit gets at most 28 GB/s from memory
-// (8 experts of 40 rows, 4096 -> 1024: 64 tiles of 128 x 128, 37 us for 67 MB).  There its reduction is divided between work-groups that
+// (8 experts of 32 rows, 4096 -> 1024: 128 tiles of 128 x 64, 31 us with the combine for 67 MB).  There its reduction is divided between work-groups that
 // each leave fp32 sums in a plane of their own, and the combine, which reads the rows anyway, adds the planes of a row, rounds, adds the
-// bias and rounds again, as the product's own epilogue would: no work-group waits for another and no launch is added.
-// The shares are read once: 2.6 MB each at 320 rows of 1024 values beside 67 MB of weights; the combine takes 4.2 - 5.0 us in place of 4.0 - 4.7
-// with up to four shares, 5.8 with eight, 8.0 in place of 5 through the int8 codec.  Pass of 8 tokens, 1024 -> 4096 -> 1024: 38.7 -> 35.3 us,
-// 128 tokens 73 -> 55, 512 tokens 87 -> 73.
+// bias and rounds again, as the product's own epilogue would: no work-group waits for another and no launch is added (22.5 us).
+// The shares are written and read once, beside 67 MB of weights: 256 rows of 1024 values 1 MB each.  Where that takes longer than it saves is
+// gemm_shares_pay's rule.
 #include "rows.hpp"
 #include "int8_core.hpp"
 #include "layer_rows.hpp"
@@ -49,20 +48,27 @@ __global__ __launch_bounds__(256) void combine_shares_kernel(const RowShares row
 // The rows in use of a chip full of tiles are 17 MB altogether; four times that is where shares become fewer, or the product whole.
 constexpr int64_t SHARES_BYTES = (int64_t)64 << 20;
 
+static int rows_expected(int rows_hint, int capacity) { return rows_hint >= 1 && rows_hint < capacity ? rows_hint : capacity; }
+
 static GemmShares shares_of(int dtype, int codec, int hidden, int top_k, int samples, int model_dim, int experts, int capacity, int rows_hint)
 {
     // (vectors of 8 values, up to 64 choices a lane each, rows of the codec's kernel in registers; elsewhere the general path)
     if (dtype != PLANMOE_BF16 || (codec != 0 && codec != 1) || hidden < 8 || hidden % 8 != 0 || model_dim < 8 || model_dim % 8 != 0 || model_dim > 4096) return GemmShares{};
     if (experts < 1 || experts > 64 || top_k < 1 || top_k > experts || samples < 1 || capacity < 1) return GemmShares{};
     if ((int64_t)(hidden > model_dim ? hidden : model_dim) * 512 >= ((int64_t)1 << 31) || (int64_t)experts * capacity >= ((int64_t)1 << 31)) return GemmShares{};
-    const int hint = rows_hint >= 1 && rows_hint < capacity ? rows_hint : capacity;
     const int64_t most = SHARES_BYTES / ((int64_t)experts * capacity * model_dim * 4);
-    return gemm_shares_pick(capacity, model_dim, hidden, experts, hint, (int64_t)samples * top_k, most);
+    return gemm_shares_pick(capacity, model_dim, hidden, experts, rows_expected(rows_hint, capacity), (int64_t)samples * top_k, most);
 }
 
 } // namespace pm
 
 using namespace pm;
+
+extern "C" int planmoe_layer_product_combine_pays(int dtype, int codec, int hidden, int top_k, int samples, int model_dim, int experts, int capacity, int rows_hint)
+{
+    const GemmShares how = shares_of(dtype, codec, hidden, top_k, samples, model_dim, experts, capacity, rows_hint);
+    return how.splits > 0 && gemm_shares_pay(how, capacity, model_dim, hidden, experts, rows_expected(rows_hint, capacity), (int64_t)samples * top_k, codec == 1);
+}
 
 extern "C" size_t planmoe_layer_product_combine_workspace_bytes(int dtype, int codec, int hidden, int top_k, int samples, int model_dim,
                                                                 int experts, int capacity, int rows_hint)

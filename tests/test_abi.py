@@ -113,6 +113,24 @@ def test_shares_do_not_grow_with_the_capacity(tokens, dim, hidden, experts, top_
             assert size % plane == 0 and size <= 64 << 20, (capacity, codec, size)
 
 
+# Where the shares of a second product pay (bf16; tokens, model_dim, hidden, experts, choices, codec): few rows and tiles, shares that are no more
+# work-groups than whole tiles of 64 columns are, shares that take longer to read than they save, rows through the codec; and what has none
+@pytest.mark.parametrize("tokens,dim,hidden,experts,top_k,codec,pays", [
+    (8, 1024, 4096, 8, 2, 0, 1), (8, 1024, 4096, 8, 2, 1, 1), (1, 4096, 1024, 8, 2, 0, 1), (1, 4096, 1024, 8, 2, 1, 0), (32, 1024, 1024, 8, 2, 0, 0), (32, 512, 2048, 8, 2, 1, 1),
+    (16, 1536, 1536, 4, 2, 0, 1), (16, 1536, 1536, 4, 2, 1, 0), (128, 1024, 4096, 8, 2, 0, 1), (128, 1024, 4096, 8, 2, 1, 1), (512, 1024, 4096, 8, 2, 0, 1),
+    (128, 2048, 2048, 8, 2, 0, 0), (400, 2048, 2048, 8, 2, 0, 1), (128, 2048, 2048, 8, 2, 1, 0), (128, 512, 2048, 4, 2, 0, 1), (512, 512, 2048, 4, 2, 0, 0), (400, 1024, 1024, 8, 2, 0, 0),
+    (256, 1024, 4096, 16, 2, 0, 0), (1024, 1024, 4096, 8, 2, 0, 0), (1999, 2048, 2048, 8, 2, 1, 0), (16384, 4096, 4096, 8, 2, 0, 0)])
+def test_where_shares_pay(tokens, dim, hidden, experts, top_k, codec, pays):
+    from planmoe_amd._lib import lib
+    from planmoe_amd import ops
+    capacity = ops.capacity(tokens, experts, top_k, 1.25, 4)
+    hint = min(capacity, (tokens * top_k + experts - 1) // experts)
+    size = (codec, hidden, top_k, tokens, dim, experts, capacity, hint)
+    assert lib.planmoe_layer_product_combine_pays(1, *size) == pays
+    assert not pays or lib.planmoe_layer_product_combine_workspace_bytes(1, *size) > 0
+    assert lib.planmoe_layer_product_combine_pays(0, *size) == 0 and lib.planmoe_layer_product_combine_pays(1, 2, *size[1:]) == 0
+
+
 def test_size_queries():
     from planmoe_amd import ops
     assert ops.zfp_stream_bytes(2, 1024, 131072) == 1024 * 131072          # 8 bits per value
