@@ -524,10 +524,10 @@ struct FwdPlan {
     bool one;             // one group: the gate kernel's slots can be the final ones
     FwdWs ws;
 };
-static void fwd_plan(FwdPlan &plan, void *workspace, int samples, int experts, int top_k)
+static void fwd_plan(FwdPlan &plan, void *workspace, int dtype, int samples, int model_dim, int experts, int top_k)
 {
     plan.k = top_k < experts ? top_k : experts;
-    plan.group_tokens = fwd_group_tokens(experts, samples);
+    plan.group_tokens = fwd_group_tokens(experts, samples, (int64_t)model_dim * dtype_bytes(dtype));
     plan.groups = (samples + plan.group_tokens - 1) / plan.group_tokens;
     plan.experts_per_block = go_experts_per_block(experts, plan.k);
     plan.blocks = (experts + plan.experts_per_block - 1) / plan.experts_per_block;
@@ -632,7 +632,7 @@ static int run_gate_route(const void *x, const void *wg, int dtype, int fp32_gat
                           int32_t *counts, void *workspace, hipStream_t st, FwdPlan &plan,
                           bool offsets_follow, int one = ONE_OFF, void *rows = nullptr, int capacity = 0)
 {
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     const int k = plan.k, groups = plan.groups;
     if (fp32_gate || dtype == PLANMOE_F32) {
         PM_DTYPE_SWITCH(dtype, DT, (launch_gate_route<DT, PLANMOE_F32>(
@@ -815,7 +815,7 @@ extern "C" int planmoe_gate_route(const void *x, const void *wg, int dtype, int 
     workspace = fwd_tables(workspace);
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     const bool one = plan.one && dtype != PLANMOE_F16;
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k,
                        normalize_gate, indices, locations, gates, plane_stride, logits_out, scores_out,
@@ -843,7 +843,7 @@ extern "C" int planmoe_forward_int8(const void *x, const void *wg, int dtype, in
     workspace = fwd_tables(workspace);
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k,
                        normalize_gate, indices, locations, gates, plane_stride, logits_out, scores_out,
                        l_aux, expert_counts, workspace, st, plan, !plan.merged)) return 1;
@@ -871,7 +871,7 @@ extern "C" int planmoe_forward_plain(const void *x, const void *wg, int dtype, i
     workspace = fwd_tables(workspace);
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k,
                        normalize_gate, indices, locations, gates, plane_stride, logits_out, scores_out,
                        l_aux, expert_counts, workspace, st, plan, !plan.merged)) return 1;
@@ -900,7 +900,7 @@ extern "C" int planmoe_layer_dispatch(const void *x, const void *wg, int dtype, 
     workspace = fwd_tables(workspace);
     hipStream_t st = (hipStream_t)stream;
     FwdPlan plan;
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     const int out = codec ? OUT_DECODED : OUT_ROWS;
     const bool one = plan.one && dtype != PLANMOE_F16;
     if (run_gate_route(x, wg, dtype, fp32_gate, logit_bias, samples, model_dim, experts, top_k, normalize_gate, indices,
@@ -1079,7 +1079,7 @@ extern "C" int planmoe_forward_int8_redispatch(const void *x, int dtype, int sam
                "planmoe_forward_int8_redispatch: bad alignment");
     workspace = fwd_tables(workspace);
     FwdPlan plan;
-    fwd_plan(plan, workspace, samples, experts, top_k);
+    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     if (run_dispatch_routed(x, dtype, samples, model_dim, experts, capacity, indices, locations,
                             plane_stride, nullptr, nullptr, codes, bias, scale, plan, (hipStream_t)stream)) return 1;
     PM_LAUNCH_CHECK("planmoe_forward_int8_redispatch");

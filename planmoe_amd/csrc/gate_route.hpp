@@ -6,19 +6,24 @@
 namespace pm {
 
 // tokens per work-group of the gate kernel = tokens per routing group (one lane each in the
-// routing epilogue): 64, or fewer where 64 would leave compute units without a work-group
-inline int fwd_group_tokens(int experts, int samples)
+// routing epilogue): 64, or fewer where 64 would leave compute units without a work-group; row_bytes: of a token
+inline int fwd_group_tokens(int experts, int samples, int64_t row_bytes)
 {
     // measured at 8 experts: 16384 tokens (256 groups of 64) 39 us with 64, 44 us with 32;
     // 8192 tokens 32 us with 64, 28 us with 32.  One compute unit gets some 30 GB/s, so fewer tokens in a group are fewer bytes in that chain, up to one
     // group a compute unit; beyond, two groups on some units take longer than one of 32.  us of the send side with 32 and with 16 tokens:
-    //   bf16, 8 x 512     40 tokens 10.2, 10.5   1999 12.2, 12.4   4096 13.8, 13.9   5000 14.3, 16.9
-    //   bf16, 8 x 2048    40 tokens 13.2, 11.5   1999 15.9, 14.0   4096 19.0, 17.1   5000 20.1, 22.0
+    //   bf16, 8 x 2048    40 tokens 13.3, 11.5   1999 16.9, 14.9   4096 20.5, 19.0   5000 20.1, 22.0
+    //   bf16, 16 x 512    40 tokens 11.9, 10.9   1999 14.2, 13.1   4096 17.0, 14.5
     //   bf16, 16 x 4096   40 tokens 22.1, 17.3   1999 25.1, 20.4   4096 34.1, 28.2   5000 36.4, 38.0
-    //   fp32, 16 x 1024   40 tokens 16.0, 13.0   1999 18.6, 15.9   4096 22.6, 18.1   5000 23.4, 24.6
+    //   fp32, 16 x 1024   40 tokens 15.9, 13.1   1999 19.7, 16.7   4096 24.1, 19.6   5000 23.4, 24.6
     //   fp32, 8 x 4096    40 tokens 32.5, 25.9   1999 38.8, 31.7   4096 50.9, 48.4   5000 56.2, 64.1
+    // With up to 8 experts from rows of 2 KB on: below, the bytes are few, and more groups are more columns to sum behind them.
+    //   bf16, 8 x 256     40 tokens 9.4, 9.5     200  9.6, 9.8     4096 12.8, 13.0
+    //   bf16, 8 x 512     40 tokens 9.5, 9.8     200 10.0, 10.5    4096 14.0, 14.1      8 x 1024   10.9, 10.7   11.4, 11.2   16.4, 16.1
+    //   fp32, 8 x 256     40 tokens 9.1, 9.4     200  9.9, 10.5    4096 14.0, 14.2      8 x 512    10.8, 10.8   11.0, 11.1   16.4, 16.6
+    //   fp32, 4 x 512     40 tokens 9.0, 9.0     200  9.5, 9.3     4096 13.4, 13.4      8 x 768    11.8, 10.9   12.4, 11.5   18.9, 18.1
     // (up to 32 tokens are one group, and one launch: plan.one)
-    if (experts <= 16) return samples > 32 && samples <= 16 * 256 ? 16 : samples < 64 * 256 ? 32 : 64;
+    if (experts <= 16) return samples > 32 && samples <= 16 * 256 && (experts > 8 || row_bytes >= 2048) ? 16 : samples < 64 * 256 ? 32 : 64;
     // as many groups as compute units at most (16 tokens: where four waves find a share of the experts).  us of the send side, bf16, with 64, 32, 16:
     //   64 experts x 1368   48 tokens 26, 22, 21;  4074 33, 29, 27;  8000 35, 32, 42;  16000 39, 47, 74
     //   32 experts x 1368   48 tokens 24, 20;      4074 33, 24;      8000 35, 28;      16000 42, 42

@@ -244,6 +244,13 @@ def test_fused_forward_few_experts_group_sizes(T, M, E, k, dtype):
     test_fused_forward_matches_unfused_and_oracle(T, M, E, k, 1.25, dtype, True, T % 2 == 1)
 
 
+# up to 8 experts: groups of 32 tokens where rows are shorter than 2 KB, of 16 from there on; 9 experts: of 16 for short rows, too
+@pytest.mark.parametrize("T,E", [(33, 8), (49, 3), (4096, 8), (65, 9)])
+@pytest.mark.parametrize("M,dtype", [(1016, torch.bfloat16), (1024, torch.bfloat16), (1016, torch.float16), (508, torch.float32), (512, torch.float32)])
+def test_fused_forward_group_sizes_by_the_rows_bytes(T, E, M, dtype):
+    test_fused_forward_matches_unfused_and_oracle(T, M, E, 2, 1.25, dtype, True, T % 2 == 1)
+
+
 @pytest.mark.parametrize("T,M,E,k,cf,dtype,fp32_gate,use_bias", [
     (1000, 512, 8, 2, 1.25, torch.bfloat16, True, False), (33, 256, 4, 2, 1.0, torch.bfloat16, True, False),
     (4096, 1024, 64, 1, 1.0, torch.bfloat16, True, True), (500, 2048, 2, 2, 1.0, torch.float32, True, False),
