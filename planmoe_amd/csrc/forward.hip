@@ -547,7 +547,7 @@ static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t 
     //   4, 1   20000 12.6, 16.2   32768 15.2, 17.4     8, 2   4096 10.7, 13.6   20000 16.6, 18.0   32768 21.0, 19.6     10, 3  4096 13.5, 16.7   12000 22.1, 22.7
     //   16384 23.8, 23.1   32768 35.9, 28.3            16, 4  4096 15.7, 18.7   8192 20.5, 21.3    12000 27.7, 26.3     32, 4  8192 26.0, 27.2   16384 38.4, 35.6
     //   48, 2  100 16.2, 15.7     1000 19.5, 16.2      64, 4  1000 27.1, 21.3   (more than 8192 entries a plane: 512 groups x 64 experts 58.6, 45.2)
-    if (plan.k <= 4 && experts <= 32 && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= 90000) {
+    if (plan.k <= 4 && experts <= 32 && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= (int64_t)90000 * compute_units() / 256) {
         route_locations_merged_kernel<<<1 + (samples + 3) / 4, 256, 0, st>>>(
             indices, locations, stride, plan.k, samples, experts, plan.ws.rank, plan.group_tokens, plan.ws.hist_t,
             plan.ws.me_t, plan.groups, plan.ws.gstride, counts, l_aux);
@@ -592,8 +592,9 @@ static void launch_route_groups(int experts, int groups, int mode, hipStream_t s
 //   64, 8   1000 68.9, 43.8, 30.6          4096 69.0, 45.5, 34.7   8192 70.6, 48.4, 44.6   16384 73.8, 59.2, 64.2
 static int route_group_tokens(int experts, int samples)
 {
-    if (experts > 8 && (samples <= 16 || (samples > 64 && samples <= 16 * 256))) return 16;
-    return samples <= 32 || (samples > 64 && samples <= 32 * 256) ? 32 : 64;
+    const int cu = compute_units();
+    if (experts > 8 && (samples <= 16 || (samples > 64 && samples <= 16 * cu))) return 16;
+    return samples <= 32 || (samples > 64 && samples <= 32 * cu) ? 32 : 64;
 }
 
 int route_groups(const void *input, int dtype, int is_logits, const float *logit_bias, int samples, int experts,

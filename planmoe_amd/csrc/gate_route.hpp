@@ -9,6 +9,7 @@ namespace pm {
 // routing epilogue): 64, or fewer where 64 would leave compute units without a work-group; row_bytes: of a token
 inline int fwd_group_tokens(int experts, int samples, int64_t row_bytes)
 {
+    const int cu = compute_units();
     // measured at 8 experts: 16384 tokens (256 groups of 64) 39 us with 64, 44 us with 32;
     // 8192 tokens 32 us with 64, 28 us with 32.  One compute unit gets some 30 GB/s, so fewer tokens in a group are fewer bytes in that chain, up to one
     // group a compute unit; beyond, two groups on some units take longer than one of 32.  us of the send side with 32 and with 16 tokens:
@@ -23,12 +24,12 @@ inline int fwd_group_tokens(int experts, int samples, int64_t row_bytes)
     //   fp32, 8 x 256     40 tokens 9.1, 9.4     200  9.9, 10.5    4096 14.0, 14.2      8 x 512    10.8, 10.8   11.0, 11.1   16.4, 16.6
     //   fp32, 4 x 512     40 tokens 9.0, 9.0     200  9.5, 9.3     4096 13.4, 13.4      8 x 768    11.8, 10.9   12.4, 11.5   18.9, 18.1
     // (up to 32 tokens are one group, and one launch: plan.one)
-    if (experts <= 16) return samples > 32 && samples <= 16 * 256 && (experts > 8 || row_bytes >= 2048) ? 16 : samples < 64 * 256 ? 32 : 64;
+    if (experts <= 16) return samples > 32 && samples <= 16 * cu && (experts > 8 || row_bytes >= 2048) ? 16 : samples < 64 * cu ? 32 : 64;
     // as many groups as compute units at most (16 tokens: where four waves find a share of the experts).  us of the send side, bf16, with 64, 32, 16:
     //   64 experts x 1368   48 tokens 26, 22, 21;  4074 33, 29, 27;  8000 35, 32, 42;  16000 39, 47, 74
     //   32 experts x 1368   48 tokens 24, 20;      4074 33, 24;      8000 35, 28;      16000 42, 42
-    if (experts > 32 && samples <= 16 * 256) return 16;
-    return samples <= 32 * 256 ? 32 : 64;
+    if (experts > 32 && samples <= 16 * cu) return 16;
+    return samples <= 32 * cu ? 32 : 64;
 }
 constexpr int FWD_LOSS_PARTS = 64;
 inline void *fwd_tables(void *workspace) { return (char *)workspace + FWD_TABLES_OFFSET; }

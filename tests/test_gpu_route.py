@@ -55,6 +55,14 @@ def test_group_sizes(T, E, k):
     _check(random_scores(T, E, seed=T, dtype=torch.bfloat16), k)
 
 
+# the slots in the routing's launch or in one of their own: either side of 32 experts, of as many sums as a round of the chip takes (k (k + 1) / 2 a token, 90000), of
+# 8192 entries a plane (32 experts, groups of 64) and of four choices
+@pytest.mark.parametrize("T,E,k", [(100, 32, 2), (100, 33, 2), (30000, 8, 2), (30001, 8, 2), (9000, 16, 4), (9001, 16, 4), (16384, 32, 2), (16385, 32, 2), (200, 10, 4), (200, 10, 5)])
+def test_slots_in_one_launch_or_two(T, E, k):
+    _check(tie_free_scores(T, E, k, seed=T + E), k)
+    _check(random_scores(T, E, seed=T, dtype=torch.bfloat16), k)
+
+
 @pytest.mark.parametrize("T,E,k", [(600000, 8, 2), (400000, 128, 2), (300001, 64, 1)])
 def test_many_tokens(T, E, k):
     """Token counts an order of magnitude above the configs (thousands of routing tiles / groups)."""
