@@ -724,6 +724,9 @@ def test_expert_gemm_in_every_kernel(dtype, form, kernel, B, cap, n, k, hint):
 @pytest.mark.parametrize("form,B,cap,n,k,hint", [("rows", 8, 128, 2056, 136, 110), ("rows", 8, 128, 2056, 328, 110), ("rows", 4, 128, 4104, 1032, 100), ("tn", 4, 260, 1208, 392, 234),
                                                  ("tn", 4, 600, 1208, 392, 600)])
 def test_expert_gemm_tile_alone_in_128_columns(form, B, cap, n, k, hint):
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    narrow = B * ((n + 63) // 64) * (1 if form == "rows" else (k + 127) // 128)          # (both widths have one name)
+    assert narrow > (units if form == "rows" else 0.8 * units)
     test_expert_gemm_in_every_kernel(torch.bfloat16, form, "128x128 alone", B, cap, n, k, hint)
 
 

@@ -487,13 +487,18 @@ def test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec
 @pytest.mark.parametrize("codec", [0, 1])
 @pytest.mark.parametrize("skewed", [False, True])
 def test_first_product_that_routes_equals_dispatch_and_product(T, M, E, k, cap, H, codec, skewed):
+    _first_product(T, M, E, k, cap, H, codec, skewed)
+
+
+def _first_product(T, M, E, k, cap, H, codec, skewed, with_bias=True, normalize=1, gap=0, dtype=torch.bfloat16, fp32_gate=True):
+    """gap: entries of a plane behind its tokens."""
     from planmoe_amd import ops
     from planmoe_amd._lib import check, lib
-    print("case", T, M, E, k, cap, H, codec, skewed, flush=True)
+    print("case", T, M, E, k, cap, H, codec, skewed, with_bias, normalize, gap, dtype, fp32_gate, flush=True)
     g = torch.Generator(device=DEV).manual_seed(T + M + E)
-    dtype = torch.bfloat16
     randn = lambda *s: torch.randn(*s, generator=g, device=DEV)
-    x, wg, w1, b1 = randn(T, M).to(dtype), (randn(E, M) * M ** -0.5).to(dtype), (randn(E, M, H) * M ** -0.5).to(dtype), randn(E, H).to(dtype)
+    x, wg, w1 = randn(T, M).to(dtype), (randn(E, M) * M ** -0.5).to(dtype), (randn(E, M, H) * M ** -0.5).to(dtype)
+    b1 = randn(E, H).to(dtype) if with_bias else None
     if skewed:                                   # everything to the last experts, and values that are not finite
         wg[:] = torch.arange(E, device=DEV)[:, None] / M
         x = x.abs()
@@ -502,31 +507,44 @@ def test_first_product_that_routes_equals_dispatch_and_product(T, M, E, k, cap, 
     else:
         x[T // 2] = 0.5                          # (a row of one value: no scale)
         x[0, 0] = -0.0
-    hint = min(cap, (T * k + E - 1) // E)
+    hint, stride = min(cap, (T * k + E - 1) // E), T + gap
     ws = torch.empty(lib.planmoe_forward_workspace_bytes(T, E, k), dtype=torch.uint8, device=DEV)
 
     def outputs():
-        ints = [torch.full(s, -7, dtype=torch.int32, device=DEV) for s in ((k, T), (k, T), (k, E))]
-        floats = [torch.full((k, T), 7.0, device=DEV), torch.full((), 7.0, device=DEV)]
+        ints = [torch.full(s, -7, dtype=torch.int32, device=DEV) for s in ((k, stride), (k, stride), (k, E))]
+        floats = [torch.full((k, stride), 7.0, dtype=torch.float32 if fp32_gate else dtype, device=DEV), torch.full((), 7.0, device=DEV)]
         return ints, floats, torch.full((E, cap, M), 7.0, dtype=dtype, device=DEV), torch.full((E, cap, H), 7.0, dtype=dtype, device=DEV)
 
     ints, floats, rows, h = outputs()
-    check(lib.planmoe_layer_dispatch_product(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), 1, T, M, E, k, 1, cap, codec, ops._ptr(ints[0]), ops._ptr(ints[1]),
-                                             ops._ptr(floats[0]), T, ops._ptr(floats[1]), ops._ptr(ints[2]), ops._ptr(w1), ops._ptr(b1), H, hint, ops._ptr(rows),
-                                             ops._ptr(h), ops._ptr(ws), ws.numel(), ops._stream(x)))
+    check(lib.planmoe_layer_dispatch_product(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), int(fp32_gate), T, M, E, k, normalize, cap, codec, ops._ptr(ints[0]),
+                                             ops._ptr(ints[1]), ops._ptr(floats[0]), stride, ops._ptr(floats[1]), ops._ptr(ints[2]), ops._ptr(w1), ops._ptr(b1), H,
+                                             hint, ops._ptr(rows), ops._ptr(h), ops._ptr(ws), ws.numel(), ops._stream(x)))
     want_ints, want_floats, want_rows, want_h = outputs()
-    check(lib.planmoe_layer_dispatch(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), 1, None, T, M, E, k, 1, cap, codec, ops._ptr(want_ints[0]), ops._ptr(want_ints[1]),
-                                     ops._ptr(want_floats[0]), T, None, ops._ptr(want_floats[1]), ops._ptr(want_ints[2]), ops._ptr(want_rows), ops._ptr(ws),
-                                     ws.numel(), ops._stream(x)))
+    check(lib.planmoe_layer_dispatch(ops._ptr(x), ops._ptr(wg), ops._dt(x, "t"), int(fp32_gate), None, T, M, E, k, normalize, cap, codec, ops._ptr(want_ints[0]),
+                                     ops._ptr(want_ints[1]), ops._ptr(want_floats[0]), stride, None, ops._ptr(want_floats[1]), ops._ptr(want_ints[2]),
+                                     ops._ptr(want_rows), ops._ptr(ws), ws.numel(), ops._stream(x)))
     ops.expert_gemm("nn", want_rows, w1, b1, relu=True, live=want_ints[2], rows_hint=hint, out=want_h)
     torch.cuda.synchronize()
-    one = T <= 32 and E <= 16 and cap <= 16      # (then the rows stay where they are)
+    # (then the rows stay where they are; a product in 32 or 64 columns has them where that is no more work-groups than there are compute units)
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    one = T <= 32 and E <= 16 and cap <= 16 and k <= 4 and dtype == torch.bfloat16 and fp32_gate and (H + 127) // 128 * E <= units
     assert bool((rows == 7.0).all()) == one
     bits = lambda t: t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
     for got, want in zip(ints, want_ints):
         assert torch.equal(got, want)
     for got, want in zip(floats + [h], want_floats + [want_h]):
         assert torch.equal(bits(got), bits(want))
+
+
+# the same: gates as they are, no bias, planes wider than the tokens; and what has two launches: more work-groups than there are compute units (and as
+# many), five choices, a gate in bf16, rows in fp32
+@pytest.mark.parametrize("T,M,E,k,cap,H,kw", [
+    (9, 520, 8, 2, 8, 264, dict(with_bias=False)), (32, 1024, 16, 3, 8, 72, dict(normalize=0)), (7, 264, 4, 2, 8, 2056, dict(gap=25)),
+    (20, 2048, 8, 4, 16, 520, dict(with_bias=False, normalize=0, gap=1)), (8, 64, 16, 2, 4, 2048, {}), (8, 64, 16, 2, 4, 2056, {}), (8, 64, 8, 5, 8, 136, {}),
+    (8, 264, 8, 2, 8, 136, dict(fp32_gate=False)), (8, 264, 8, 2, 8, 136, dict(dtype=torch.float32, gap=3)), (16, 128, 4, 4, 16, 4096, dict(gap=7, normalize=0))])
+@pytest.mark.parametrize("codec", [0, 1])
+def test_first_product_that_routes_with_other_options(T, M, E, k, cap, H, kw, codec):
+    _first_product(T, M, E, k, cap, H, codec, False, **kw)
 
 
 # without autograd a pass lies in one buffer: the same bits as the pass that a backward pass may follow, gates in 16 bits among them
