@@ -140,7 +140,8 @@ torch::Tensor ZfpCompressor::compress(const torch::Tensor &input_)
     const int64_t nx = sizes[2], ny = sizes[1] * sizes[0];
     const size_t bufsize = planmoe_zfp_max_bytes(2, nx, ny, compress_rate);
     length = planmoe_zfp_stream_bytes(2, nx, ny, compress_rate);
-    // the coder writes the whole stream: what is cleared is the last word and the slack up to the maximum size (134 MB: 20 us of a pass of 336)
+    // the coder writes the whole stream: what is cleared is the last word and the slack up to the maximum size (134 MB: 20 us of a pass of 336; short
+    // streams take 17.5 us either way, a view and its fill being as quick here as the whole one's is)
     torch::Tensor output = torch::empty({(int64_t)((bufsize + 1) / 2)}, input.options().dtype(at::kHalf));
     const int64_t rest   = std::max<int64_t>((int64_t)length - 8, 0) / 2;
     output.narrow(0, rest, output.numel() - rest).zero_();

@@ -112,6 +112,23 @@ def test_zfp_shape_assertion_like_the_reference():
     ck.clear_ptr_lst()
 
 
+# what the coder does not write is zero, in memory that was in use: a short stream and one of 4 MB
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [8, 1024])
+def test_cpp_zfp_stream_and_its_slack(rows):
+    from planmoe_amd import ext
+    ck = ext.load()
+    x = torch.randn(4, rows, 1036, generator=torch.Generator().manual_seed(rows)).to(DEV)
+    want = oracle.zfp_compress(x.cpu().numpy().reshape(-1, 1036), 2)
+    size = (oracle.zfp_max_bytes(2, 1036, x.shape[0] * x.shape[1]) + 1) // 2
+    used = torch.full((size,), float("nan"), dtype=torch.float16, device=DEV)
+    del used
+    ck.clear_ptr_lst()
+    got = ck.compress_operation(x, "zfp", "naive").view(torch.uint8).cpu().numpy()
+    ck.clear_ptr_lst()
+    assert got.size == 2 * size and np.array_equal(got[:len(want)], want) and not got[len(want):].any()
+
+
 @pytest.mark.gpu
 def test_pipeline_through_the_cpp_registry():
     from planmoe_amd import ext
