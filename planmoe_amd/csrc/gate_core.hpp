@@ -121,7 +121,7 @@ __device__ __forceinline__ void gate_tile_partials(const void *__restrict__ x,
         const int nsteps = w < full ? (full - w + NW - 1) / NW : 0;
         int step = w, left = nsteps;
         GateFrag<NT, TPW> f[4];
-        // first what four does not divide, then fours: no step is asked for twice
+        // first what four does not divide (of one or two such steps the last is asked for three times: a cache hit), then fours
         if (left & 3) {
             const int end = w + ((left & 3) - 1) * NW;
 #pragma unroll

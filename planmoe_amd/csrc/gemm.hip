@@ -615,8 +615,9 @@ int gemm_launch(const GemmArgs &p, hipStream_t stream, const char *who)
 // is bound by its operands: the height whose tiles fill the rounds best.  A launch takes its rounds; a round takes its k-tiles,
 // each faster with few compute units at work than with all of them (the clock sinks under the matrix cores), and what a tile
 // costs once.  Reading the weights is a floor: what memory gives, or, with few work-groups, what they have on their way (28 GB/s for each
-// in 128 x 128, 45 in 256 columns).  Fitted to 450 timings of 110 shapes with the weights in the last cache and out of it: what it picks takes
-// 1.1 % longer than the best.
+// in 128 x 128, 45 in 256 columns).  Fitted to 450 timings of 110 shapes with the weights in the last cache and out of it: what it picked took
+// 1.1 % longer than the best, before there was a tile of 128 x 64 (gemm_pick takes 0.72 of small() for it, the weight's floor in it included, which
+// is what half the columns on twice the compute units give in gemm_is_deep's table).
 // us in one launch, rows +- sqrt(rows) in use, nn:
 //   experts x rows, in, out      128 x 128    256    128    160    192 x 256
 //   8 x 500, 2048, 2048             49         48     57     42     42     (54 in 256 and a launch of quarters)

@@ -7,8 +7,14 @@
 // its expert's tokens and takes their rows straight from x, through the int8 codec where the exchange has one, so that
 // the dispatched rows are neither written nor read.  Same roundings and the same order of sums as the launches it stands for.
 //
-// Bound by reading the weights and the gate's latency under it.  A pass of 8 tokens x 1024, hidden 4096, 8 experts, weights cold: see
-// planmoe_layer_dispatch_product.
+// Bound by reading the weights and the gate's latency under it.  us in two launches and in one, without a codec and through it, weights in the last cache
+// (where they fit) and cold, 4 experts top-1, 8 and 16 top-2:
+//   1 token     4, 4096 -> 512   18.3, 11.9 and 20.0, 18.0   21.8, 21.1 and 22.4, 20.0      8, 1024 -> 4096  14.6, 13.1 and 15.2, 13.7   15.2, 15.0 and 16.0, 15.6
+//               8, 2048 -> 4096  23.1, 21.1 and 23.9, 22.8   23.6, 23.2 and 24.3, 24.5
+//   8 tokens    8, 256 -> 512    8.4, 6.3 and 8.8, 6.9       8.8, 6.6 and 9.2, 7.2          8, 1024 -> 4096  18.8, 15.6 and 18.9, 16.2   20.1, 17.0 and 20.9, 17.5
+//   32 tokens   8, 4096 -> 512   29.9, 23.1 and 31.7, 27.1   37.7, 30.8 and 39.3, 32.0      8, 4096 -> 4096  60.7, 54.5 and 62.1, 55.4   60.0, 54.9 and 61.8, 55.9
+//               16, 4096 -> 2048 63.2, 56.4 and 63.8, 57.2   62.7, 57.0 and 64.4, 57.7      4, 4096 -> 2048  30.1, 23.1 and 31.8, 26.4   37.3, 30.1 and 39.0, 31.5
+// (190 shapes of 1, 8 and 32 tokens, 256 to 4096 -> 512 to 4096: 0.84 of two launches, at worst 1.03)
 #include "gate_route.hpp"
 #include "gemm_shares.hpp"
 #include "gemm_skinny_core.hpp"

@@ -6,10 +6,10 @@
 // lengths alone, so no bits are packed and none are walked, except those of the one plane that the budget ends in.  Blocks of empty
 // capacity slots are neither read nor written.
 //
-// Under the profiler, 4096 x 1024 tokens, top-2, 16 experts x 512 slots: dispatch 20 us (dispatch with the coder, then the decoder: 40), rows in place 18,
-// with their stream kept 32 (coder, then a decoding combine of a launch a choice: 16 + 47; the combine of decoded rows is 9),
-// combine's backward pass 37 (42 + 19), and one slot map a pass instead of five (47 -> 10).  Bound by the vector ALUs: 16 bytes a
-// lane and about 600 instructions a block in the dispatch and the rows, the decoder's walk where a stream is read.
+// Under the profiler, 4096 x 1024 tokens, top-2, 16 experts x 512 slots: dispatch 16 us, rows in place 17, with their stream kept 21.5, combine's backward
+// pass 31, one slot map a pass 9.  (The codec's own entry points, when these kernels took 20, 18, 32, 37 and 10: dispatch with the coder, then
+// the decoder 40; coder, then a decoding combine of a launch a choice 16 + 47, where the combine of decoded rows is 9; backward pass 42 + 19; five slot maps 47.)
+// Bound by the vector ALUs: 16 bytes a lane and about 600 instructions a block in the dispatch and the rows, the decoder's walk where a stream is read.
 #include "zfp_core.hpp"
 
 namespace pm {

@@ -283,10 +283,10 @@ struct BlockPlace {
     __device__ __forceinline__ int64_t bx(const FieldBlocks &g) const { return col + threadIdx.x - (down ? down * g.nbx : 0); }
 };
 
-// Bound by memory where it was bound by issuing vector instructions: 16 x 8192 x 1024 values (512 MB in, 128 MB out) 212 -> 165 us under the
-// profiler, 981 vector instructions a wave before: appends by funnel shifts in place of a word stored at a time (two dozen a plane -> five),
-// the group-test table copied and not worked out by each work-group, casts without the overflow that only blocks next to
-// the denormals and not finite ones have, a transpose by byte permutes and bit selects, no 64-bit division a lane.
+// Bound by issuing vector instructions (655 a wave are 140 us at 2.4 GHz) and, nearly as much, by memory (137 us at a copy's rate): 16 x 8192 x 1024
+// values (512 MB in, 128 MB out) 212 -> 155 - 165 us under the profiler.  981 vector instructions a wave before: appends by funnel shifts in place
+// of a word stored at a time (two dozen a plane -> five), the group-test table copied and not worked out by each work-group, casts without the
+// overflow that only blocks next to the denormals and not finite ones have, a transpose by byte permutes and bit selects, no 64-bit division a lane.
 template <int NW>
 __global__ __launch_bounds__(256) void zfp_encode2_kernel(const float *__restrict__ field, const FieldBlocks g, int64_t blocks,
                                                           uint32_t *__restrict__ out)
