@@ -30,26 +30,34 @@ namespace pm {
 
 // This lane's share of the sum of col[0 .. limit): col is 16-byte aligned and readable up to the
 // next multiple of 4 entries, limit is the same in every lane.  The wave reduction is left to the
-// caller so that several columns can be loaded back to back and reduced together (one memory
-// round trip and interleaved shuffle chains instead of one after the other).
-__device__ __forceinline__ int column_partial(const int32_t *__restrict__ col, int limit)
-{
-    int s = 0;
-    for (int i = lane_id() * 4; i < limit; i += 4 * WAVE) {
-        const int4 v = *reinterpret_cast<const int4 *>(col + i);
-        s += v.x + (i + 1 < limit ? v.y : 0) + (i + 2 < limit ? v.z : 0) + (i + 3 < limit ? v.w : 0);
+// caller.  AHEAD: the first load, too, so that those of several columns are on their way together; a loop of its own makes each column wait
+// for memory by itself.  (34 experts, 2 choices, 165 tokens: 17.1 us of routing, 14.5 with the loads together;
+// 16, 4, 1000 tokens 15.7, 13.4.)  Four registers a
+// column: not where rows are held (dispatch_int8_routed_kernel 35 -> 76 registers), which hides the chain anyway.
+template <typename T, bool AHEAD>
+struct ColumnPartial {
+    static_assert(sizeof(T) == 4, "words");
+    uint4 v;
+    __device__ __forceinline__ void load(const T *__restrict__ col, int limit)
+    {
+        if constexpr (AHEAD) v = *reinterpret_cast<const uint4 *>(col + min(lane_id() * 4, max(limit - 1, 0) & ~3));      // (clamped, not predicated)
     }
-    return s;
-}
-__device__ __forceinline__ float column_partial(const float *__restrict__ col, int limit)
-{
-    float s = 0.f;
-    for (int i = lane_id() * 4; i < limit; i += 4 * WAVE) {
-        const float4 v = *reinterpret_cast<const float4 *>(col + i);
-        s += (v.x + (i + 1 < limit ? v.y : 0.f)) + ((i + 2 < limit ? v.z : 0.f) + (i + 3 < limit ? v.w : 0.f));
+    __device__ __forceinline__ T sum(const T *__restrict__ col, int limit) const
+    {
+        auto part = [&](const uint4 &w, int i) {
+            auto at = [&](uint32_t x, int n) { return i + n < limit ? __builtin_bit_cast(T, x) : T(0); };
+            return (at(w.x, 0) + at(w.y, 1)) + (at(w.z, 2) + at(w.w, 3));
+        };
+        T s = T(0);
+        int i = lane_id() * 4;
+        if constexpr (AHEAD) {
+            s = part(v, i);
+            i += 4 * WAVE;
+        }
+        for (; i < limit; i += 4 * WAVE) s += part(*reinterpret_cast<const uint4 *>(col + i), i);
+        return s;
     }
-    return s;
-}
+};
 // wave sums of N values at once
 template <typename T, int N>
 __device__ __forceinline__ void wave_sum_n(T (&v)[N])
@@ -178,6 +186,7 @@ __global__ __launch_bounds__(256) void route_offsets_kernel(const int32_t *__res
 
 // Lane j (< top_k) returns the slot of choice j of token t inside its expert: rank in the group +
 // entries of the earlier planes + entries of the earlier groups of plane j.  e_l: its expert.
+template <bool AHEAD>
 __device__ __forceinline__ int merged_location(const int32_t *__restrict__ indices, const int32_t *__restrict__ rank,
                                                const int32_t *__restrict__ hist_t, int64_t stride, int top_k,
                                                int samples, int experts, int t, int group_tokens, int groups,
@@ -198,8 +207,12 @@ __device__ __forceinline__ int merged_location(const int32_t *__restrict__ indic
     for (int j = 0; j < 4; ++j) {
         if (j < top_k) {
             const int e = rl_i(e_l, j);
-            before[j] = column_partial(hist_t + ((int64_t)j * experts + e) * gstride, g);
-            for (int jp = 0; jp < j; ++jp) before[j] += column_partial(hist_t + ((int64_t)jp * experts + e) * gstride, groups);
+            auto column = [&](int plane) { return hist_t + ((int64_t)plane * experts + e) * gstride; };
+            ColumnPartial<int32_t, AHEAD> c[4];
+#pragma unroll
+            for (int jp = 0; jp <= j; ++jp) c[jp].load(column(jp), jp < j ? groups : g);
+#pragma unroll
+            for (int jp = 0; jp <= j; ++jp) before[j] += c[jp].sum(column(jp), jp < j ? groups : g);
         }
     }
     wave_sum_n(before);
@@ -210,6 +223,7 @@ __device__ __forceinline__ int merged_location(const int32_t *__restrict__ indic
 
 // One work-group (4 waves) finishes the GShard loss and the per-plane expert counts.
 // s_loss: 64 floats of LDS.
+template <bool AHEAD>
 __device__ __forceinline__ void merged_stats(const int32_t *__restrict__ hist_t, const float *__restrict__ me_t,
                                              int groups, int gstride, int experts, int top_k, int samples,
                                              int32_t *__restrict__ counts_out, float *__restrict__ l_aux,
@@ -218,36 +232,42 @@ __device__ __forceinline__ void merged_stats(const int32_t *__restrict__ hist_t,
     const int wave = threadIdx.x >> 6, lane = lane_id();
     // the one block that finishes the loss: l_aux = sum_e me[e] * ce[e] / T with
     // me[e] = column sum of the scores, ce[e] = first-choice count * E / T
-    // four experts per pass and wave: the loads of a pass are in flight together
+    // four experts per pass and wave: a plane's loads are in flight together, and the scores' with the first plane's (past the last expert
+    // its own again, unused)
     for (int e0 = wave * 4; e0 < experts; e0 += 16) {
-        int c0[4] = {0, 0, 0, 0};
-        float m[4] = {0.f, 0.f, 0.f, 0.f};
+        auto at = [&](int q) { return (int64_t)min(e0 + q, experts - 1) * gstride; };
+        ColumnPartial<float, AHEAD> me[4];
+        ColumnPartial<int32_t, AHEAD> c[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (e0 + q < experts) {
-                c0[q] = column_partial(hist_t + (int64_t)(e0 + q) * gstride, groups);
-                if (l_aux) m[q] = column_partial(me_t + (int64_t)(e0 + q) * gstride, groups);
-            }
+        for (int q = 0; q < 4; ++q) c[q].load(hist_t + at(q), groups);
+        if (l_aux) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) me[q].load(me_t + at(q), groups);
         }
-        wave_sum_n(c0);
-        wave_sum_n(m);
+        int n[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (lane == 0 && e0 + q < experts) {
-                if (counts_out) counts_out[e0 + q] = c0[q];
-                s_loss[e0 + q] = m[q] * ((float)c0[q] * ((float)experts / (float)samples));
-            }
+        for (int q = 0; q < 4; ++q) n[q] = c[q].sum(hist_t + at(q), groups);
+        wave_sum_n(n);
+        if (l_aux) {
+            float m[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m[q] = me[q].sum(me_t + at(q), groups);
+            wave_sum_n(m);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) s_loss[e0 + q] = m[q] * ((float)n[q] * ((float)experts / (float)samples));
         }
-        if (counts_out) {
-            for (int j = 1; j < top_k; ++j) {
-                int c[4] = {0, 0, 0, 0};
+        if (!counts_out) continue;
+        for (int j = 0; j < top_k; ++j) {
+            if (j > 0) {
+                const int32_t *plane = hist_t + (int64_t)j * experts * gstride;
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (e0 + q < experts) c[q] = column_partial(hist_t + ((int64_t)j * experts + e0 + q) * gstride, groups);
-                wave_sum_n(c);
+                for (int q = 0; q < 4; ++q) c[q].load(plane + at(q), groups);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) counts_out[j * experts + e0 + q] = c[q];
+                for (int q = 0; q < 4; ++q) n[q] = c[q].sum(plane + at(q), groups);
+                wave_sum_n(n);
             }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) counts_out[j * experts + e0 + q] = n[q];
         }
     }
     __syncthreads();
@@ -269,13 +289,13 @@ __global__ __launch_bounds__(256) void route_locations_merged_kernel(
     __shared__ float s_loss[64];
     if (blockIdx.x == 0) {
         if (l_aux || counts_out)
-            merged_stats(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
+            merged_stats<true>(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
         return;
     }
     const int t = ((int)blockIdx.x - 1) * 4 + (int)(threadIdx.x >> 6);
     if (t >= samples) return;
     int e_l;
-    const int l = merged_location(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
+    const int l = merged_location<true>(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
                                   gstride, e_l);
     if (lane_id() < top_k) locations[(int64_t)lane_id() * stride + t] = l;
 }
@@ -319,7 +339,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
     if (fill_first && bid >= 0) bid = bid < fill_blocks ? token_blocks + bid : bid - fill_blocks;
     if constexpr (MERGED) {
         if ((int)blockIdx.x < stat_blocks) {
-            merged_stats(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
+            merged_stats<false>(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
             return;
         }
     }
@@ -335,7 +355,8 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (e0 + q < experts)
-                        for (int j = 0; j < top_k; ++j) c[q] += column_partial(hist_t + ((int64_t)j * experts + e0 + q) * gstride, groups);
+                        for (int j = 0; j < top_k; ++j)
+                            c[q] += ColumnPartial<int32_t, false>().sum(hist_t + ((int64_t)j * experts + e0 + q) * gstride, groups);
                 wave_sum_n(c);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) s_tot[e0 + q] = c[q];
@@ -383,7 +404,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
         int slot = -1;
         if constexpr (MERGED) {
             int e_l;
-            const int l = merged_location(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
+            const int l = merged_location<false>(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
                                           gstride, e_l);
             if (lane < top_k) {
                 locations[(int64_t)lane * stride + t] = l;
@@ -542,12 +563,16 @@ static void fwd_plan(FwdPlan &plan, void *workspace, int dtype, int samples, int
 static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t *locations, int64_t stride,
                            int samples, int experts, float *l_aux, int32_t *counts, hipStream_t st)
 {
-    // One launch more takes 2 - 4 us.  Without it the first work-group sums every expert's column for the loss by itself, and every token's wave
-    // k (k + 1) / 2 columns.  us of the routing, in one launch and in two (experts, choices, tokens):
-    //   4, 1   20000 12.6, 16.2   32768 15.2, 17.4     8, 2   4096 10.7, 13.6   20000 16.6, 18.0   32768 21.0, 19.6     10, 3  4096 13.5, 16.7   12000 22.1, 22.7
-    //   16384 23.8, 23.1   32768 35.9, 28.3            16, 4  4096 15.7, 18.7   8192 20.5, 21.3    12000 27.7, 26.3     32, 4  8192 26.0, 27.2   16384 38.4, 35.6
-    //   48, 2  100 16.2, 15.7     1000 19.5, 16.2      64, 4  1000 27.1, 21.3   (more than 8192 entries a plane: 512 groups x 64 experts 58.6, 45.2)
-    if (plan.k <= 4 && experts <= 32 && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= (int64_t)90000 * compute_units() / 256) {
+    // One launch more takes the GPU 2 - 4 us and the host 3.4, which a training step of few tokens waits for.  Without it the first work-group sums
+    // every expert's columns for the loss and the counts by itself, sixteen experts at a time, and every token's wave k (k + 1) / 2 columns.  us of the
+    // routing on the GPU, in one launch and in two (experts, choices, tokens):
+    //   4, 1   20000 11.4, 13.9   32768 14.7, 15.4     8, 2   4096 8.7, 11.5    20000 16.0, 15.6   32768 21.5, 17.4     8, 4   9000 16.0, 16.0   20000 27.7, 19.5
+    //   16, 4  1000 13.4, 15.2    9000 23.8, 23.8      24, 4  1000 18.4, 17.1   32, 2  4096 13.0, 14.6    20000 27.1, 25.5   32, 4  1000 19.0, 17.4
+    //   34, 2  165 14.5, 13.7     4096 15.4, 15.5      48, 2  165 15.1, 13.6    4096 16.0, 15.0           64, 1  165 12.8, 11.6   4096 13.3, 12.8
+    //   34, 4  165 21.4, 17.8     64, 2  165 17.9, 14.2   64, 4  1000 26.8, 18.9   (more than 8192 entries a plane: 64, 1, 20000 28.0, 22.0)
+    // So two launches from where they gain more on the GPU than half of what they cost the host.
+    const bool few = experts <= 32 || experts * plan.k <= 96;
+    if (plan.k <= 4 && few && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= (int64_t)90000 * compute_units() / 256) {
         route_locations_merged_kernel<<<1 + (samples + 3) / 4, 256, 0, st>>>(
             indices, locations, stride, plan.k, samples, experts, plan.ws.rank, plan.group_tokens, plan.ws.hist_t,
             plan.ws.me_t, plan.groups, plan.ws.gstride, counts, l_aux);
