@@ -30,17 +30,36 @@ namespace pm {
 
 // This lane's share of the sum of col[0 .. limit): col is 16-byte aligned and readable up to the
 // next multiple of 4 entries, limit is the same in every lane.  The wave reduction is left to the
-// caller.  AHEAD: the first load, too, so that those of several columns are on their way together; a loop of its own makes each column wait
-// for memory by itself.  (34 experts, 2 choices, 165 tokens: 17.1 us of routing, 14.5 with the loads together;
-// 16, 4, 1000 tokens 15.7, 13.4.)  Four registers a
-// column: not where rows are held (dispatch_int8_routed_kernel 35 -> 76 registers), which hides the chain anyway.
-template <typename T, bool AHEAD>
+// caller so that several columns can be loaded back to back and reduced together (one memory
+// round trip and interleaved shuffle chains instead of one after the other).
+__device__ __forceinline__ int column_partial(const int32_t *__restrict__ col, int limit)
+{
+    int s = 0;
+    for (int i = lane_id() * 4; i < limit; i += 4 * WAVE) {
+        const int4 v = *reinterpret_cast<const int4 *>(col + i);
+        s += v.x + (i + 1 < limit ? v.y : 0) + (i + 2 < limit ? v.z : 0) + (i + 3 < limit ? v.w : 0);
+    }
+    return s;
+}
+__device__ __forceinline__ float column_partial(const float *__restrict__ col, int limit)
+{
+    float s = 0.f;
+    for (int i = lane_id() * 4; i < limit; i += 4 * WAVE) {
+        const float4 v = *reinterpret_cast<const float4 *>(col + i);
+        s += (v.x + (i + 1 < limit ? v.y : 0.f)) + ((i + 2 < limit ? v.z : 0.f) + (i + 3 < limit ? v.w : 0.f));
+    }
+    return s;
+}
+// The same with the first load left to the caller, so that those of several columns are on their way together; in the loop above each column waits
+// for memory by itself.  (Routing by itself: 34 experts, 2 choices, 165 tokens 17.1 us, 14.5 with the loads together; 16, 4, 1000 tokens 15.7, 13.4.)
+// Four registers a column: not where rows are held (dispatch_int8_routed_kernel 35 -> 76 registers), which hides the chain anyway.
+template <typename T>
 struct ColumnPartial {
     static_assert(sizeof(T) == 4, "words");
     uint4 v;
     __device__ __forceinline__ void load(const T *__restrict__ col, int limit)
     {
-        if constexpr (AHEAD) v = *reinterpret_cast<const uint4 *>(col + min(lane_id() * 4, max(limit - 1, 0) & ~3));      // (clamped, not predicated)
+        v = *reinterpret_cast<const uint4 *>(col + min(lane_id() * 4, max(limit - 1, 0) & ~3));      // (clamped, not predicated)
     }
     __device__ __forceinline__ T sum(const T *__restrict__ col, int limit) const
     {
@@ -48,13 +67,8 @@ struct ColumnPartial {
             auto at = [&](uint32_t x, int n) { return i + n < limit ? __builtin_bit_cast(T, x) : T(0); };
             return (at(w.x, 0) + at(w.y, 1)) + (at(w.z, 2) + at(w.w, 3));
         };
-        T s = T(0);
-        int i = lane_id() * 4;
-        if constexpr (AHEAD) {
-            s = part(v, i);
-            i += 4 * WAVE;
-        }
-        for (; i < limit; i += 4 * WAVE) s += part(*reinterpret_cast<const uint4 *>(col + i), i);
+        T s = part(v, lane_id() * 4);
+        for (int i = lane_id() * 4 + 4 * WAVE; i < limit; i += 4 * WAVE) s += part(*reinterpret_cast<const uint4 *>(col + i), i);
         return s;
     }
 };
@@ -208,11 +222,16 @@ __device__ __forceinline__ int merged_location(const int32_t *__restrict__ indic
         if (j < top_k) {
             const int e = rl_i(e_l, j);
             auto column = [&](int plane) { return hist_t + ((int64_t)plane * experts + e) * gstride; };
-            ColumnPartial<int32_t, AHEAD> c[4];
+            if constexpr (AHEAD) {
+                ColumnPartial<int32_t> c[4];
 #pragma unroll
-            for (int jp = 0; jp <= j; ++jp) c[jp].load(column(jp), jp < j ? groups : g);
+                for (int jp = 0; jp <= j; ++jp) c[jp].load(column(jp), jp < j ? groups : g);
 #pragma unroll
-            for (int jp = 0; jp <= j; ++jp) before[j] += c[jp].sum(column(jp), jp < j ? groups : g);
+                for (int jp = 0; jp <= j; ++jp) before[j] += c[jp].sum(column(jp), jp < j ? groups : g);
+            } else {
+                before[j] = column_partial(column(j), g);
+                for (int jp = 0; jp < j; ++jp) before[j] += column_partial(column(jp), groups);
+            }
         }
     }
     wave_sum_n(before);
@@ -232,42 +251,64 @@ __device__ __forceinline__ void merged_stats(const int32_t *__restrict__ hist_t,
     const int wave = threadIdx.x >> 6, lane = lane_id();
     // the one block that finishes the loss: l_aux = sum_e me[e] * ce[e] / T with
     // me[e] = column sum of the scores, ce[e] = first-choice count * E / T
-    // four experts per pass and wave: a plane's loads are in flight together, and the scores' with the first plane's (past the last expert
+    // four experts per pass and wave; AHEAD: the loads of a plane are in flight together, those of the scores with the first plane's (past the last expert
     // its own again, unused)
     for (int e0 = wave * 4; e0 < experts; e0 += 16) {
         auto at = [&](int q) { return (int64_t)min(e0 + q, experts - 1) * gstride; };
-        ColumnPartial<float, AHEAD> me[4];
-        ColumnPartial<int32_t, AHEAD> c[4];
+        int c0[4] = {0, 0, 0, 0};
+        float m[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (AHEAD) {
+            ColumnPartial<int32_t> c[4];
+            ColumnPartial<float> me[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) c[q].load(hist_t + at(q), groups);
-        if (l_aux) {
+            for (int q = 0; q < 4; ++q) c[q].load(hist_t + at(q), groups);
+            if (l_aux) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) me[q].load(me_t + at(q), groups);
-        }
-        int n[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) n[q] = c[q].sum(hist_t + at(q), groups);
-        wave_sum_n(n);
-        if (l_aux) {
-            float m[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) m[q] = me[q].sum(me_t + at(q), groups);
-            wave_sum_n(m);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) s_loss[e0 + q] = m[q] * ((float)n[q] * ((float)experts / (float)samples));
-        }
-        if (!counts_out) continue;
-        for (int j = 0; j < top_k; ++j) {
-            if (j > 0) {
-                const int32_t *plane = hist_t + (int64_t)j * experts * gstride;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) c[q].load(plane + at(q), groups);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) n[q] = c[q].sum(plane + at(q), groups);
-                wave_sum_n(n);
+                for (int q = 0; q < 4; ++q) me[q].load(me_t + at(q), groups);
             }
 #pragma unroll
-            for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) counts_out[j * experts + e0 + q] = n[q];
+            for (int q = 0; q < 4; ++q) c0[q] = c[q].sum(hist_t + at(q), groups);
+            if (l_aux) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) m[q] = me[q].sum(me_t + at(q), groups);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (e0 + q < experts) {
+                    c0[q] = column_partial(hist_t + (int64_t)(e0 + q) * gstride, groups);
+                    if (l_aux) m[q] = column_partial(me_t + (int64_t)(e0 + q) * gstride, groups);
+                }
+            }
+        }
+        wave_sum_n(c0);
+        wave_sum_n(m);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (lane == 0 && e0 + q < experts) {
+                if (counts_out) counts_out[e0 + q] = c0[q];
+                s_loss[e0 + q] = m[q] * ((float)c0[q] * ((float)experts / (float)samples));
+            }
+        }
+        if (counts_out) {
+            for (int j = 1; j < top_k; ++j) {
+                const int32_t *plane = hist_t + (int64_t)j * experts * gstride;
+                int c[4] = {0, 0, 0, 0};
+                if constexpr (AHEAD) {
+                    ColumnPartial<int32_t> v[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q].load(plane + at(q), groups);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) c[q] = v[q].sum(plane + at(q), groups);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (e0 + q < experts) c[q] = column_partial(plane + (int64_t)(e0 + q) * gstride, groups);
+                }
+                wave_sum_n(c);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) counts_out[j * experts + e0 + q] = c[q];
+            }
         }
     }
     __syncthreads();
@@ -355,8 +396,7 @@ __global__ __launch_bounds__(256) void dispatch_int8_routed_kernel(
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (e0 + q < experts)
-                        for (int j = 0; j < top_k; ++j)
-                            c[q] += ColumnPartial<int32_t, false>().sum(hist_t + ((int64_t)j * experts + e0 + q) * gstride, groups);
+                        for (int j = 0; j < top_k; ++j) c[q] += column_partial(hist_t + ((int64_t)j * experts + e0 + q) * gstride, groups);
                 wave_sum_n(c);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) if (lane == 0 && e0 + q < experts) s_tot[e0 + q] = c[q];
@@ -611,10 +651,10 @@ static void launch_route_groups(int experts, int groups, int mode, hipStream_t s
 // Tokens of a group: a wave walks its quarter of them four at a time (eight where eight lanes share a token), k searches each, one latency
 // after the other, so groups are small as long as each finds a compute unit; more than that and the groups take turns.  Up to 64 tokens are one
 // group, which needs no second launch.  us, both launches, with groups of 64, 32 and 16 tokens (experts, choices):
-//   8, 2    1000 tokens 11.2, 10.1, 10.3   4096 11.6, 10.7, 11.0   8192 12.3, 11.0, 13.6   16384 14.3, 14.7, 17.9
-//   10, 3   1000 18.5, 15.3, 12.9          4096 19.3, 15.2, 13.3   8192 20.3, 16.6, 16.6   12000 22.1, 20.4, 20.5   32768 35.8, 32.5, 46.6
-//   24, 2   1000 20.6, 17.8, 14.7          4096 21.8, 17.7, 15.4   8192 22.3, 18.7, 20.3   16384 22.7, 23.0, 28.1
-//   64, 8   1000 68.9, 43.8, 30.6          4096 69.0, 45.5, 34.7   8192 70.6, 48.4, 44.6   16384 73.8, 59.2, 64.2
+//   8, 2    1000 tokens 9.5, 8.1, 8.9      4096 9.5, 8.3, 9.1      8192 10.6, 9.3, 11.9    16384 12.9, 13.4, 17.7
+//   10, 3   1000 17.4, 13.3, 11.4          4096 17.4, 13.5, 11.5   8192 18.5, 14.6, 15.1   12000 20.1, 19.0, 19.9   32768 26.4, 30.8, 45.1
+//   24, 2   1000 19.0, 14.9, 12.3          4096 19.2, 15.0, 12.7   8192 19.5, 15.4, 18.1   16384 20.6, 20.9, 26.2
+//   64, 8   1000 66.1, 41.7, 29.0          4096 67.3, 43.7, 33.0   8192 68.9, 47.5, 43.0   16384 72.9, 58.2, 62.9
 static int route_group_tokens(int experts, int samples)
 {
     const int cu = compute_units();
