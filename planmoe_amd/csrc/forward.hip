@@ -321,6 +321,7 @@ __device__ __forceinline__ void merged_stats(const int32_t *__restrict__ hist_t,
 
 // locations of a stand-alone routing call (top_k <= 4): block 0 finishes the loss and the counts,
 // the others take a token per wave
+template <bool AHEAD>
 __global__ __launch_bounds__(256) void route_locations_merged_kernel(
     const int32_t *__restrict__ indices, int32_t *__restrict__ locations, int64_t stride, int top_k, int samples,
     int experts, const int32_t *__restrict__ rank, int group_tokens, const int32_t *__restrict__ hist_t,
@@ -330,13 +331,13 @@ __global__ __launch_bounds__(256) void route_locations_merged_kernel(
     __shared__ float s_loss[64];
     if (blockIdx.x == 0) {
         if (l_aux || counts_out)
-            merged_stats<true>(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
+            merged_stats<AHEAD>(hist_t, me_t, groups, gstride, experts, top_k, samples, counts_out, l_aux, s_loss);
         return;
     }
     const int t = ((int)blockIdx.x - 1) * 4 + (int)(threadIdx.x >> 6);
     if (t >= samples) return;
     int e_l;
-    const int l = merged_location<true>(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
+    const int l = merged_location<AHEAD>(indices, rank, hist_t, stride, top_k, samples, experts, t, group_tokens, groups,
                                   gstride, e_l);
     if (lane_id() < top_k) locations[(int64_t)lane_id() * stride + t] = l;
 }
@@ -608,14 +609,18 @@ static void finish_routing(const FwdPlan &plan, const int32_t *indices, int32_t 
     // routing on the GPU, in one launch and in two (experts, choices, tokens):
     //   4, 1   20000 11.4, 13.9   32768 14.7, 15.4     8, 2   4096 8.7, 11.5    20000 16.0, 15.6   32768 21.5, 17.4     8, 4   9000 16.0, 16.0   20000 27.7, 19.5
     //   16, 4  1000 13.4, 15.2    9000 23.8, 23.8      24, 4  1000 18.4, 17.1   32, 2  4096 13.0, 14.6    20000 27.1, 25.5   32, 4  1000 19.0, 17.4
-    //   34, 2  165 14.5, 13.7     4096 15.4, 15.5      48, 2  165 15.1, 13.6    4096 16.0, 15.0           64, 1  165 12.8, 11.6   4096 13.3, 12.8
+    //   40, 1  300 10.9, 11.1     3000 11.3, 12.3      48, 1  300 10.8, 11.4    34, 2  165 14.5, 13.7     48, 2  165 15.1, 13.6   64, 1  165 12.8, 11.6
     //   34, 4  165 21.4, 17.8     64, 2  165 17.9, 14.2   64, 4  1000 26.8, 18.9   (more than 8192 entries a plane: 64, 1, 20000 28.0, 22.0)
-    // So two launches from where they gain more on the GPU than half of what they cost the host.
-    const bool few = experts <= 32 || experts * plan.k <= 96;
+    // So two launches with more than 32 experts where they gain the GPU something; for up to 512 tokens, where a pass of the routing API is the host's (22 us without a
+    // backward pass), where they gain it more than half of what they cost the host.
+    const bool few = experts <= 32 || experts * plan.k <= 48 || (experts * plan.k <= 96 && samples <= 512);
     if (plan.k <= 4 && few && (int64_t)plan.groups * experts <= 8192 && (int64_t)samples * plan.k * (plan.k + 1) / 2 <= (int64_t)90000 * compute_units() / 256) {
-        route_locations_merged_kernel<<<1 + (samples + 3) / 4, 256, 0, st>>>(
-            indices, locations, stride, plan.k, samples, experts, plan.ws.rank, plan.group_tokens, plan.ws.hist_t,
-            plan.ws.me_t, plan.groups, plan.ws.gstride, counts, l_aux);
+        // (columns together: 76 registers, and every lane asks.  With few experts and many tokens that is the longer way: 8, 1 and 32768 tokens 13.5 us one
+        // after the other, 14.6 together; 16384 9.6, 10.2; 8192 8.2, 7.6; 24, 1 and 16384 15.8, 14.2)
+        const bool ahead = experts > 16 || samples < 32 * compute_units();
+        const auto kernel = ahead ? route_locations_merged_kernel<true> : route_locations_merged_kernel<false>;
+        kernel<<<1 + (samples + 3) / 4, 256, 0, st>>>(indices, locations, stride, plan.k, samples, experts, plan.ws.rank, plan.group_tokens, plan.ws.hist_t,
+                                                      plan.ws.me_t, plan.groups, plan.ws.gstride, counts, l_aux);
         return;
     }
     group_offsets_kernel<<<plan.blocks, 256, 0, st>>>(plan.ws.hist, plan.ws.offs, plan.ws.me, plan.groups, plan.k, experts,

@@ -55,9 +55,9 @@ def test_group_sizes(T, E, k):
     _check(random_scores(T, E, seed=T, dtype=torch.bfloat16), k)
 
 
-# the slots in the routing's launch or in one of their own: either side of 32 experts and of 96 experts times choices, of as many sums as a round of the
+# the slots in the routing's launch or in one of their own: either side of 32 experts, of 48 and 96 experts times choices and of 512 tokens, of as many sums as a round of the
 # chip takes (k (k + 1) / 2 a token, 90000), of 8192 entries a plane (32 experts, groups of 64) and of four choices; more groups than the 256 that a wave reads at once
-@pytest.mark.parametrize("T,E,k", [(100, 32, 2), (100, 33, 2), (100, 32, 4), (100, 33, 3), (165, 48, 2), (165, 49, 2), (4095, 64, 1), (70, 64, 2), (32769, 4, 1), (17000, 7, 3), (30000, 8, 2), (30001, 8, 2), (9000, 16, 4), (9001, 16, 4), (16384, 32, 2), (16385, 32, 2), (200, 10, 4), (200, 10, 5)])
+@pytest.mark.parametrize("T,E,k", [(100, 32, 2), (100, 33, 2), (100, 32, 4), (100, 33, 3), (165, 48, 2), (165, 49, 2), (4095, 48, 1), (512, 64, 1), (513, 64, 1), (9000, 24, 2), (8191, 16, 1), (70, 64, 2), (32769, 4, 1), (17000, 7, 3), (30000, 8, 2), (30001, 8, 2), (9000, 16, 4), (9001, 16, 4), (16384, 32, 2), (16385, 32, 2), (200, 10, 4), (200, 10, 5)])
 def test_slots_in_one_launch_or_two(T, E, k):
     _check(tie_free_scores(T, E, k, seed=T + E), k)
     _check(random_scores(T, E, seed=T, dtype=torch.bfloat16), k)
