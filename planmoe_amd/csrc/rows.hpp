@@ -1,6 +1,7 @@
 // Row access helpers shared by the kernels that move token rows to and from capacity slots.
 #pragma once
 #include "common.hpp"
+#include <type_traits>
 
 namespace pm {
 
@@ -12,7 +13,7 @@ enum { ROWS_1 = 0, ROWS_4 = 1, ROWS_16 = 2 };
 
 typedef uint32_t pm_u32x4_dwords __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int DT, int MODE>
+template <int DT, int MODE, bool STREAM = true>
 struct RowIO {
     using E = Elem<DT>;
     static constexpr int U = MODE ? E::VEC : 1;        // elements per lane access
@@ -32,6 +33,25 @@ struct RowIO {
             f[0] = E::load(p, 0);
         }
     }
+    // what a lane has asked for, kept as it lies in memory until it is used
+    typedef std::conditional_t<MODE == ROWS_1, float, uint4> raw_t;
+    __device__ static __forceinline__ raw_t load_raw(const void *row, int off)
+    {
+        const char *p = (const char *)row + off;
+        if constexpr (MODE == ROWS_16) {
+            return *reinterpret_cast<const uint4 *>(p);
+        } else if constexpr (MODE == ROWS_4) {
+            const pm_u32x4_dwords v = *reinterpret_cast<const pm_u32x4_dwords *>(p);
+            return make_uint4(v.x, v.y, v.z, v.w);
+        } else {
+            return E::load(p, 0);
+        }
+    }
+    __device__ static __forceinline__ void unpack(const raw_t &v, float *f)
+    {
+        if constexpr (MODE == ROWS_1) f[0] = v;
+        else E::unpack(v, f);
+    }
     // for launches that store nothing in bulk (measured: streaming loads next to streaming
     // stores slow the dispatch / combine kernels down, alone they help)
     __device__ static __forceinline__ void load_stream(const void *row, int off, float *f)
@@ -49,7 +69,8 @@ struct RowIO {
     __device__ static __forceinline__ void store_bits(void *row, int off, const uint4 &v)
     {
         char *p = (char *)row + off;
-        if constexpr (MODE == ROWS_16) stream_store(reinterpret_cast<uint4 *>(p), v);
+        if constexpr (MODE == ROWS_16 && STREAM) stream_store(reinterpret_cast<uint4 *>(p), v);
+        else if constexpr (MODE == ROWS_16) *reinterpret_cast<uint4 *>(p) = v;
         else *reinterpret_cast<pm_u32x4_dwords *>(p) = pm_u32x4_dwords{v.x, v.y, v.z, v.w};
     }
     __device__ static __forceinline__ void store(void *row, int off, const float *f)

@@ -33,15 +33,16 @@ __global__ __launch_bounds__(256) void slot_flags_mark(uint32_t *flags, const in
 
 // ------------------------------------------------------------------ dispatch (scatter rows)
 // token_blocks work-groups move token rows: dispatched[slot] = 0 + gate * x[t]; the others write zero rows into the slots
-// no live pair addresses.
-template <int DT, int MODE>
+// no live pair addresses.  Bound by memory: 8192 x 2048 fp32, two choices, 201 MB in 31 us, 14020 x 3528 bf16 317 MB in 69 (a unit at a
+// time 32 and 77).
+template <int DT, int MODE, bool STREAM>
 __global__ __launch_bounds__(256) void dispatch_kernel(
     const void *__restrict__ x, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
     void *__restrict__ dispatched, const SlotFill fill, int token_blocks)
 {
-    using IO = RowIO<DT, MODE>;
+    using IO = RowIO<DT, MODE, STREAM>;
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int units = IO::units(model_dim);
     const int64_t row_bytes = (int64_t)model_dim * sizeof(typename Elem<DT>::store_t);
@@ -64,25 +65,37 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, j0, np, experts, capacity, slot, gate);
         if (__ballot(slot >= 0) == 0) continue;          // every choice of this pass dropped: the row is not read
-        for (int u = lane; u < units; u += WAVE) {
-            float v[IO::U];
-            IO::load(src, IO::at(u, (int)row_bytes), v);
+        // four units of a row per lane are asked for before the first is stored: a wait for a load waits for the stores
+        // ahead of it too, and there is one a unit where they alternate
+        constexpr int B = 4;
+        for (int u0 = lane; u0 < units; u0 += B * WAVE) {
+            typename IO::raw_t row[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) row[b] = IO::load_raw(src, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes));
             for (int j = 0; j < np; ++j) {
                 const int s = rl_i(slot, j);
                 if (s < 0) continue;
                 const float g = rl_f(gate, j);
-                float o[IO::U];
+                char *to = (char *)dispatched + (int64_t)s * row_bytes;
 #pragma unroll
-                for (int i = 0; i < IO::U; ++i) o[i] = 0.f + g * v[i];
-                IO::store((char *)dispatched + (int64_t)s * row_bytes, IO::at(u, (int)row_bytes), o);
+                for (int b = 0; b < B; ++b) {
+                    float v[IO::U], o[IO::U];
+                    IO::unpack(row[b], v);
+#pragma unroll
+                    for (int i = 0; i < IO::U; ++i) o[i] = 0.f + g * v[i];
+                    if (u0 + b * WAVE < units) IO::store(to, IO::at(u0 + b * WAVE, (int)row_bytes), o);
+                }
             }
         }
     }
 }
 
 // ------------------------------------------------------------------ combine (gather rows)
-// out[t] = sum_j (live_j ? gate_j * dispatched[slot_j] : 0), planes added left to right.
-template <int DT, int MODE>
+// out[t] = sum_j (live_j ? gate_j * dispatched[slot_j] : 0), planes added left to right.  Bound by memory.  A wave asks for B units a lane
+// of two choices' rows before it adds any (a dropped choice reads slot 0 and contributes zeros): one wait a pass over 4 KB rows, and
+// over 8 KB rows with B = 8 (8192 x 2048 fp32, two choices, 201 MB: 36.7 us, 38.5 with four units of one choice at a time, 38.8 of two; 14020 x 3528 bf16
+// 54.8, 57.7, 57.5; rows of 2 KB lose with eight: 16384 x 1024 bf16 17.5 and 23.6).
+template <int DT, int MODE, int B>
 __global__ __launch_bounds__(256) void combine_kernel(
     const void *__restrict__ dispatched, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
@@ -99,25 +112,32 @@ __global__ __launch_bounds__(256) void combine_kernel(
     if (top_k <= WAVE) {
         int slot; float gate;
         fetch_planes(gates, indices, locations, stride, t, 0, top_k, 0x7fffffff, capacity, slot, gate);
-        // four units of a row per lane and pass, fetched with straight-line loads at clamped
-        // addresses (a dropped choice reads slot 0 and contributes zeros): four loads in flight
-        // per choice instead of one load, one wait
-        constexpr int B = 4;
         for (int u0 = lane; u0 < units; u0 += B * WAVE) {
             float acc[B][IO::U];
-            for (int j = 0; j < top_k; ++j) {
-                const int s = rl_i(slot, j);
-                const float g = rl_f(gate, j);
-                const char *row = (const char *)dispatched + (int64_t)max(s, 0) * row_bytes;
-                float term[B][IO::U];
+            constexpr int G = 2;
+            for (int j0 = 0; j0 < top_k; j0 += G) {
+                typename IO::raw_t row[G][B];
 #pragma unroll
-                for (int b = 0; b < B; ++b) IO::load(row, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes), term[b]);
+                for (int j = 0; j < G; ++j) {
+                    if (j0 + j >= top_k) break;
+                    const char *from = (const char *)dispatched + (int64_t)max(rl_i(slot, j0 + j), 0) * row_bytes;
 #pragma unroll
-                for (int b = 0; b < B; ++b) {
+                    for (int b = 0; b < B; ++b) row[j][b] = IO::load_raw(from, IO::at(min(u0 + b * WAVE, units - 1), (int)row_bytes));
+                }
 #pragma unroll
-                    for (int i = 0; i < IO::U; ++i) {
-                        const float v = s >= 0 ? g * term[b][i] : 0.f;
-                        acc[b][i] = (j == 0) ? v : acc[b][i] + v;
+                for (int j = 0; j < G; ++j) {
+                    if (j0 + j >= top_k) break;
+                    const int s = rl_i(slot, j0 + j);
+                    const float g = rl_f(gate, j0 + j);
+#pragma unroll
+                    for (int b = 0; b < B; ++b) {
+                        float term[IO::U];
+                        IO::unpack(row[j][b], term);
+#pragma unroll
+                        for (int i = 0; i < IO::U; ++i) {
+                            const float v = s >= 0 ? g * term[i] : 0.f;
+                            acc[b][i] = (j0 + j == 0) ? v : acc[b][i] + v;
+                        }
                     }
                 }
             }
@@ -226,14 +246,14 @@ __global__ __launch_bounds__(256) void bwd_gate_kernel(
 // dispatch_kernel's scatter of the gated gradient and bwd_gate_kernel's products in one pass over the gradient:
 // grad_rows[slot_j] = 0 + gate_j * grad[t], grad_gates[j][t] = <rows[slot_j], grad[t]>.  Bound by memory (8192 x
 // 2048 fp32, two choices: 335 MB where the two launches move 402).
-template <int DT, int MODE>
+template <int DT, int MODE, bool STREAM>
 __global__ __launch_bounds__(256) void combine_bwd_kernel(
     const void *__restrict__ grad, const void *__restrict__ rows, const float *__restrict__ gates,
     const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride,
     int top_k, int samples, int model_dim, int experts, int capacity,
     void *__restrict__ grad_rows, float *__restrict__ grad_gates, const SlotFill fill, int token_blocks)
 {
-    using IO = RowIO<DT, MODE>;
+    using IO = RowIO<DT, MODE, STREAM>;
     constexpr int G = 4, B = 2;
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int units = IO::units(model_dim);
@@ -336,6 +356,18 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
     }
 }
 
+// Rows that the call after this one reads are stored past the caches where they would not all be there by then, and plainly where the 256 MB of
+// the memory-side cache hold them: what follows a dispatch reads its rows, a combine's backward pass reads rows and writes as many.  us, dispatch, combine, its
+// backward pass, combine, by what is stored plainly: none, the dispatch's rows, the backward pass's too
+//   rows of 134 MB in all 174, 162, 159     218 MB 281, 267, 284     246 MB 270, 262, 274     335 MB 374, 399, 420     84 MB 104.6, 101.9, 99.2
+// (What a combine stores is stored past them: 8192 x 2048 fp32 171 in place of 159.)
+static bool stays(int64_t bytes) { return bytes <= (int64_t)256 << 20; }
+#define PM_STREAM_SWITCH(streams, MODE, STREAM, ...)                                                 \
+    do {                                                                                             \
+        if (MODE == ROWS_16 && (streams)) { constexpr bool STREAM = MODE == ROWS_16; __VA_ARGS__; }  \
+        else { constexpr bool STREAM = false; __VA_ARGS__; }                                         \
+    } while (0)
+
 SlotFill slot_fill(void *workspace, const int32_t *indices, const int32_t *locations, int64_t stride, int top_k, int samples, int experts,
                    int capacity, int64_t row_bytes, hipStream_t st)
 {
@@ -401,10 +433,11 @@ extern "C" int planmoe_dispatch_fwd(const void *x, int dtype, const float *gates
                                     (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2), st);
     const int token_blocks = (samples + 3) / 4;
     const int mode = rows_mode(dtype, model_dim, x, dispatched);
+    const int64_t buffer_bytes = (int64_t)slots * model_dim * (dtype == PLANMOE_F32 ? 4 : 2);
     PM_DTYPE_SWITCH(dtype, DT, {
-        PM_ROWS_SWITCH(mode, MODE, (dispatch_kernel<DT, MODE><<<token_blocks + fill.blocks, 256, 0, st>>>(
+        PM_ROWS_SWITCH(mode, MODE, PM_STREAM_SWITCH(!stays(buffer_bytes), MODE, STREAM, (dispatch_kernel<DT, MODE, STREAM><<<token_blocks + fill.blocks, 256, 0, st>>>(
             x, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, dispatched, fill,
-            token_blocks)));
+            token_blocks))));
     });
     PM_LAUNCH_CHECK("planmoe_dispatch_fwd");
     return 0;
@@ -424,6 +457,7 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     hipStream_t st = (hipStream_t)stream;
     const int mode = rows_mode(dtype, model_dim, out, dispatched);
     const int blocks = (samples + 3) / 4;
+    const bool wide = (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2) > 4096;
     if (capacity == 0) {
         // no slot exists, every choice is dropped: zero rows.  (combine_kernel fetches rows with
         // unconditional loads at clamped slots and must not run without a row to read.)
@@ -434,8 +468,10 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
         return 0;
     }
     PM_DTYPE_SWITCH(dtype, DT, {
-        PM_ROWS_SWITCH(mode, MODE, (combine_kernel<DT, MODE><<<blocks, 256, 0, st>>>(
-            dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out)));
+        PM_ROWS_SWITCH(mode, MODE, ({
+            if (wide) combine_kernel<DT, MODE, 8><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
+            else combine_kernel<DT, MODE, 4><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
+        }));
     });
     PM_LAUNCH_CHECK("planmoe_combine_fwd");
     return 0;
@@ -491,10 +527,11 @@ extern "C" int planmoe_combine_bwd(const void *grad, const void *dispatched, int
                                     (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2), st);
     const int token_blocks = (samples + 3) / 4;
     const int mode = std::min(rows_mode(dtype, model_dim, grad, dispatched), rows_mode(dtype, model_dim, grad_dispatched, grad_dispatched));
+    const int64_t buffer_bytes = (int64_t)experts * capacity * model_dim * (dtype == PLANMOE_F32 ? 4 : 2);
     PM_DTYPE_SWITCH(dtype, DT, {
-        PM_ROWS_SWITCH(mode, MODE, (combine_bwd_kernel<DT, MODE><<<token_blocks + fill.blocks, 256, 0, st>>>(
+        PM_ROWS_SWITCH(mode, MODE, PM_STREAM_SWITCH(!stays(2 * buffer_bytes), MODE, STREAM, (combine_bwd_kernel<DT, MODE, STREAM><<<token_blocks + fill.blocks, 256, 0, st>>>(
             grad, dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity,
-            grad_dispatched, grad_gates, fill, token_blocks)));
+            grad_dispatched, grad_gates, fill, token_blocks))));
     });
     PM_LAUNCH_CHECK(who);
     return 0;

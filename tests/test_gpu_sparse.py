@@ -64,6 +64,54 @@ def test_dispatch_and_combine_bit_exact(T, M, E, k, cf, dtype):
         assert np.array_equal(raw(gotc), raw(wantc))
 
 
+@pytest.mark.parametrize("M,dtype", [(1020, torch.float32), (1028, torch.float32), (2048, torch.float32), (2052, torch.float32), (2056, torch.bfloat16),
+                                     (4104, torch.bfloat16), (2050, torch.float16), (257, torch.float16), (2051, torch.bfloat16)])
+@pytest.mark.parametrize("k", [1, 3, 5])
+def test_rows_around_a_pass_bit_exact(M, dtype, k):
+    """Rows that end around the vectors a wave asks for at once (four or eight a lane), odd numbers of choices."""
+    from planmoe_amd import ops
+    T, E = 41, 6
+    idx, loc, gates, C = _routing(T, E, k, 0.75, seed=M + k)
+    g = torch.Generator().manual_seed(3)
+    x, eo = torch.randn(T, M, generator=g).to(dtype), torch.randn(E * C, M, generator=g).to(dtype)
+    i, l, gt = _dev(idx), _dev(loc), _dev(gates)
+    want = torch.from_numpy(oracle.encode(x.float().numpy(), list(idx), list(loc), list(gates), E, C)).to(dtype)
+    assert np.array_equal(raw(ops.dispatch_fwd(x.to(DEV), i, l, gt, E, C)), raw(want))
+    want = torch.from_numpy(oracle.decode(eo.float().numpy(), list(idx), list(loc), list(gates), T, C)).to(dtype)
+    assert np.array_equal(raw(ops.combine_fwd(eo.to(DEV), i, l, gt, T, C)), raw(want))
+
+
+def test_rows_stored_past_the_caches_are_those_stored_plainly():
+    """A dispatch and a combine's backward pass over more than 256 MB of rows, against their halves below that."""
+    from planmoe_amd import ops
+    T, M, E, C = 17000, 2048, 4, 10000
+    g = torch.Generator(device=DEV).manual_seed(4)
+    x, rows = torch.randn(T, M, generator=g, device=DEV), torch.randn(E * C, M, generator=g, device=DEV)
+    idx = [torch.randint(0, E, (T,), generator=g, device=DEV, dtype=torch.int32) for _ in range(2)]
+    # every pair a slot of its own
+    order = torch.cat(idx)
+    loc = torch.empty_like(order)
+    for e in range(E):
+        at = (order == e).nonzero().flatten()
+        loc[at] = torch.arange(len(at), device=DEV, dtype=torch.int32)
+    loc = [loc[:T].contiguous(), loc[T:].contiguous()]
+    gates = [torch.rand(T, generator=g, device=DEV) for _ in range(2)]
+    got = ops.dispatch_fwd(x, idx, loc, gates, E, C).view(E * C, M)
+    assert got.numel() * 4 > 256 << 20
+    want = torch.zeros(E * C, M, device=DEV)
+    for i, l, w in zip(idx, loc, gates):
+        keep = l < C
+        want[(i * C + l)[keep].long()] = (w[:, None] * x)[keep]
+    assert torch.equal(got, want)
+    i, l, w = torch.stack(idx), torch.stack(loc), torch.stack(gates)
+    grad_rows, grad_gates = torch.empty_like(rows), torch.empty(2, T, device=DEV)
+    ws = torch.empty(ops.lib.planmoe_dispatch_workspace_bytes(E, C), dtype=torch.uint8, device=DEV)
+    ops.check(ops.lib.planmoe_combine_bwd(ops._ptr(x), ops._ptr(rows), 0, ops._ptr(w), ops._ptr(i), ops._ptr(l), T, 2, T, M, E, C, ops._ptr(grad_rows),
+                                          ops._ptr(grad_gates), ops._ptr(ws), ws.numel(), ops._stream(x)))
+    assert torch.equal(grad_rows, want)
+    assert torch.equal(grad_gates, ops.bwd_gate(x, rows, idx, loc, C))
+
+
 @pytest.mark.parametrize("T,M,E,k,dtype,rtol", [(300, 512, 8, 2, torch.float32, 1e-5), (300, 4096, 8, 2, torch.bfloat16, 1e-2),
                                                 (50, 77, 4, 3, torch.float32, 1e-5), (40, 64, 16, 6, torch.float32, 1e-5)])
 def test_bwd_gate(T, M, E, k, dtype, rtol):
