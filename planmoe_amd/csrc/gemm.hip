@@ -930,7 +930,7 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
         Gemm32Args p{(const float *)a, (const float *)b, (const float *)bias, nullptr, (float *)c, nullptr, live, live_planes, live_round,
                      m, n, k, batches, activation};
         const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
-        return gemm_f32_run(form, p, gemm_f32_pick(form, p, hint), st, who);
+        return gemm_f32_run(form, p, gemm_f32_pick(form, p, hint), hint, st, who);
     }
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n, most = form == 2 ? k : m;
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, live, live_planes,
@@ -983,7 +983,7 @@ int pm::relu_bwd_with(const char *who, int dtype, const void *a, const void *b, 
         Gemm32Args p{(const float *)a, (const float *)b, nullptr, (const float *)h, (float *)c, parts, live, live_planes, live_round, m, n, k, batches, 0};
         const Gemm32Kernel kernel = gemm_f32_pick(1, p, hint);
         sums = GemmSlots{gemm_f32_slot_rows(kernel), 2};
-        if (gemm_f32_run(1, p, kernel, st, who)) return 1;
+        if (gemm_f32_run(1, p, kernel, hint, st, who)) return 1;
     } else {
         GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, nullptr, (const uint16_t *)h, (uint16_t *)c, parts, live, live_planes, live_round,
                    m, n, k, k, k, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, 0, 0, 0, false};

@@ -185,13 +185,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// Few rows: a wave on its own, 16 MF rows by 16 columns, operands from memory straight into registers
+// Few rows: a wave on its own, 16 MF rows by 16 C columns, operands from memory straight into registers
 // (no LDS, no barrier), 2 U steps of 16 k in flight.  v_mfma_f32_16x16x4_f32 with lane group g at k = 4 g + q: the sums
 // take the k in the same order as the tiles do, so which kernel serves a shape does not show in the result.
-// Bound by reading the weight (tiles of 64 x 64 wait a trip to memory for every 32 k and there are few of them: 8 experts
-// of 2 rows, 4096 -> 1024, 134 MB: 90 us, here 39).  U: nn reads a k at a time, 64 bytes of a row, and takes twice
-// the steps in flight that nt does (nn with 8: 90 us; nt with 16: 40 us, and 26 in place of 23 at 1024 -> 4096).
-template <int MF, int U, bool TB>
+// Bound by reading the weight, or, where a wave of 16 columns is all that a SIMD has, by what one wave has on its way (63 loads at most): nn reads
+// a row of k at a time, 64 bytes with C = 1, a whole line with 2, 256 bytes with 4.  NT: past the caches.
+template <int MF, int C, int U, bool TB, bool NT>
 __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args p)
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
@@ -202,7 +201,7 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
     // Column sums have two slots for every 64 rows in use: the second of them may have no rows.
     auto blocks_of = [&](int rows) { return ((p.colsum ? (rows + 63) / 64 * 64 : rows) + 16 * MF - 1) / (16 * MF); };
     auto round_up = [&](int n) { return min(p.M, (n + p.live_round - 1) / p.live_round * p.live_round); };
-    const int number = blockIdx.x, cols = (p.N + 63) / 64, most = blocks_of(p.M);
+    const int waves = blockDim.x >> 6, wide = 16 * C * waves, number = blockIdx.x, cols = (p.N + wide - 1) / wide, most = blocks_of(p.M);
     int e = number / (most * cols), M = p.M, blocks = most, piece = number - e * most * cols;
     if (p.live && most == 1) {                   // (a batch is a row block at most)
         int n = 0;
@@ -224,19 +223,21 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
         blocks = blocks_of(M);
         piece = number - (e > 0 ? __builtin_amdgcn_readlane(ends, e - 1) : 0);
     }
-    const int m0 = piece % blocks * 16 * MF, n0 = (piece / blocks * 4 + wave) * 16;
+    const int m0 = piece % blocks * 16 * MF, n0 = (piece / blocks * waves + wave) * 16 * C;
     if (M == 0 || n0 >= p.N) return;
     const float *A = p.A + (int64_t)e * p.M * p.K, *B = p.B + (int64_t)e * p.N * p.K;
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, M * p.K * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, p.N * p.K * 4, 0x00020000);
     constexpr uint32_t NOWHERE = 0x80000000u;
-    const int steps = (p.K + 15) / 16, col = n0 + l16;
+    const int steps = (p.K + 15) / 16, col = n0 + C * l16;        // a lane's columns: C in a row, one in each fragment
 
-    f32x4 acc[MF], fa[2][U][MF], fb[2][U];
+    f32x4 acc[MF][C], fa[2][U][MF], fb[2][U][C];
 #pragma unroll
-    for (int m = 0; m < MF; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[m][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     // rows and columns past the end, and k past the end, read as zero
-    auto load = [&](f32x4 (&a)[U][MF], f32x4 (&b)[U], int s0) {
+    auto load = [&](f32x4 (&a)[U][MF], f32x4 (&b)[U][C], int s0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = 16 * (s0 + u) + 4 * g;
@@ -249,20 +250,37 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
             if (TB) {
                 const uint32_t at = in_k && col < p.N ? ((uint32_t)k * (uint32_t)p.N + (uint32_t)col) * 4u : NOWHERE;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) b[u][q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(db, at, (uint32_t)(q * 4) * (uint32_t)p.N, 0));
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t row = (uint32_t)(q * 4) * (uint32_t)p.N;
+                    if constexpr (C == 4) {
+                        const pm_u32x4 v = __builtin_bit_cast(pm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(db, at, row, NT ? 2 : 0));
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) b[u][c][q] = __uint_as_float(v[c]);
+                    } else if constexpr (C == 2) {
+                        const pm_u32x2 v = __builtin_bit_cast(pm_u32x2, __builtin_amdgcn_raw_buffer_load_b64(db, at, row, NT ? 2 : 0));
+                        b[u][0][q] = __uint_as_float(v[0]);
+                        b[u][1][q] = __uint_as_float(v[1]);
+                    } else {
+                        b[u][0][q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(db, at, row, NT ? 2 : 0));
+                    }
+                }
             } else {
-                b[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(db, in_k && col < p.N ? ((uint32_t)col * (uint32_t)p.K + (uint32_t)k) * 4u : NOWHERE, 0, 0));
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    b[u][c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(db, in_k && col < p.N ? ((uint32_t)(col + c) * (uint32_t)p.K + (uint32_t)k) * 4u : NOWHERE, 0, NT ? 2 : 0));
             }
         }
     };
     // (the second operand first: a lane then holds four consecutive columns of one row)
-    auto multiply = [&](const f32x4 (&a)[U][MF], const f32x4 (&b)[U]) {
+    auto multiply = [&](const f32x4 (&a)[U][MF], const f32x4 (&b)[U][C]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int m = 0; m < MF; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][q], a[u][m][q], acc[m], 0, 0, 0);
+                for (int m = 0; m < MF; ++m)
+#pragma unroll
+                    for (int c = 0; c < C; ++c) acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][c][q], a[u][m][q], acc[m][c], 0, 0, 0);
     };
     load(fa[0], fb[0], 0);
     for (int s = 0; s < steps; s += 2 * U) {
@@ -277,52 +295,90 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    const int c = n0 + 4 * g;                    // (N is a multiple of 4: a lane's columns are in or out together)
-    const bool in_n = c < p.N;
-    f32x4 add = {0.f, 0.f, 0.f, 0.f}, sums = add;
-    if (p.bias && in_n)
+    const int n = n0 + 4 * C * g;                // a lane's results: columns n .. n + 4 C - 1 of row l16, four in or out together
+    float add[4 * C], sums[4 * C];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) add[x] = p.bias[(int64_t)e * p.N + c + x];
+    for (int x = 0; x < 4 * C; ++x) {
+        sums[x] = 0.f;
+        add[x] = p.bias && n + x < p.N ? p.bias[(int64_t)e * p.N + n + x] : 0.f;
+    }
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
         const int row = m0 + 16 * m + l16;
-        const int64_t at = ((int64_t)e * p.M + row) * p.N + c;
-        const bool inside = in_n && row < M;
-        f32x4 v = acc[m];
-        if (p.bias) v += add;
-        if (p.relu)
 #pragma unroll
-            for (int x = 0; x < 4; ++x) v[x] = v[x] < 0.f ? 0.f : v[x];
-        if (p.mask) {
-            f32x4 k = {0.f, 0.f, 0.f, 0.f};
-            if (inside) k = *reinterpret_cast<const f32x4 *>(p.mask + at);
+        for (int h = 0; h < C; ++h) {
+            const int64_t at = ((int64_t)e * p.M + row) * p.N + n + 4 * h;
+            const bool inside = n + 4 * h < p.N && row < M;
+            f32x4 v, k = {0.f, 0.f, 0.f, 0.f};
+            if (p.mask && inside) k = *reinterpret_cast<const f32x4 *>(p.mask + at);
 #pragma unroll
-            for (int x = 0; x < 4; ++x) { v[x] = k[x] > 0.f ? v[x] : 0.f; sums[x] += v[x]; }
+            for (int x = 0; x < 4; ++x) {
+                const int y = 4 * h + x;         // (column y: result y / C of fragment y % C)
+                v[x] = acc[m][y % C][y / C];
+                if (p.bias) v[x] += add[y];
+                if (p.relu) v[x] = v[x] < 0.f ? 0.f : v[x];
+                if (p.mask) { v[x] = k[x] > 0.f ? v[x] : 0.f; sums[y] += v[x]; }
+            }
+            if (inside) *reinterpret_cast<f32x4 *>(p.C + at) = v;
         }
-        if (inside) *reinterpret_cast<f32x4 *>(p.C + at) = v;
     }
     if (p.colsum) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
+        for (int x = 0; x < 4 * C; ++x)
 #pragma unroll
             for (int d = 1; d < 16; d <<= 1) sums[x] += __shfl_xor(sums[x], d);
-        if (l16 == 0 && in_n) *reinterpret_cast<f32x4 *>(p.colsum + ((int64_t)e * ((p.M + 63) / 64 * 2) + m0 / 32) * p.N + c) = sums;
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            if (l16 == 0 && n + 4 * h < p.N)
+                *reinterpret_cast<f32x4 *>(p.colsum + ((int64_t)e * ((p.M + 63) / 64 * 2) + m0 / 32) * p.N + n + 4 * h) = f32x4{sums[4 * h], sums[4 * h + 1], sums[4 * h + 2], sums[4 * h + 3]};
     }
 }
 
-// how many pieces of `rows` by 64 columns the products have at most
-static int64_t gemm_f32_wave_pieces(const Gemm32Args &p, int rows)
+// how many pieces of `rows` by `columns` the products have at most
+static int64_t gemm_f32_wave_pieces(const Gemm32Args &p, int rows, int columns)
 {
     const int64_t m = p.colsum ? ((int64_t)p.M + 63) / 64 * 64 : p.M;
-    return (m + rows - 1) / rows * (((int64_t)p.N + 63) / 64) * p.batches;
+    return (m + rows - 1) / rows * (((int64_t)p.N + columns - 1) / columns) * p.batches;
 }
 
-template <int MF, int U, bool TB>
-static int gemm_f32_wave_launch(const Gemm32Args &p, hipStream_t stream, const char *who)
+template <int MF, int C, int U, bool TB, bool NT = false>
+static int gemm_f32_wave_launch(const Gemm32Args &p, int waves, hipStream_t stream, const char *who)
 {
-    gemm_f32_wave_kernel<MF, U, TB><<<dim3((unsigned)gemm_f32_wave_pieces(p, 16 * MF)), 256, 0, stream>>>(p);
+    gemm_f32_wave_kernel<MF, C, U, TB, NT><<<dim3((unsigned)gemm_f32_wave_pieces(p, 16 * MF, 16 * C * waves)), 64 * waves, 0, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
+}
+
+// waves of 32 rows (16 where no batch has more) by 16 columns that the rows expected make
+static int64_t gemm_f32_strips(const Gemm32Args &p, int rows_hint)
+{
+    const int rows = p.M <= 16 && !p.colsum ? 16 : 32;
+    return (int64_t)((rows_hint + rows - 1) / rows) * ((p.N + 15) / 16) * p.batches;
+}
+
+// Columns and waves of a work-group.  Where there are waves enough of 32 columns for the SIMDs a wave reads whole lines; fewer than that and 16 columns put
+// more waves to work, each on a compute unit of its own (four to a work-group where there are several a compute unit anyway: they share lines); weights that the
+// last cache (256 MB) does not hold go past the caches, with few rows 64 columns of them.  b^T: a wave reads 64 bytes of every row whatever its columns.
+// us before (16 columns, four waves, twice the steps in nn) and now, weights cold, in the last cache:
+//   nn, up to 16 rows   8 x 1024 -> 4096    33, 28 and 27, 22       8 x 2600 -> 3440    80, 72 and 58, 52      16 x 3328 -> 3072  149 and 95 (cold)
+//                       4 x 1024 -> 1024    14, 14 and 12, 12       16 x 1896 -> 688    26, 24 and 24, 21      8 x 4096 -> 1024   51, 39 and 49, 37
+//                       16 x 512 -> 2048    20, 19 and 15, 14       (16 columns in single waves: 8 x 4096 -> 1024 47, 44)
+//   nn, up to 32        16 x 1472 -> 2176   82, 66 and 68, 60       8 x 2816 -> 1728    49, 46 and 43, 41
+//                       8 x 1024 -> 4096    44, 38 (tiles) and 34, 28
+//   nt                  4 x 1024 -> 1024    16, 16 and 9, 9         8 x 4096 -> 1024    41, 40 and 30, 29      16 x 3072 -> 3328  147 and 132
+static int gemm_f32_waves(int form, const Gemm32Args &p, int rows_hint, hipStream_t stream, const char *who)
+{
+    const int64_t strips = gemm_f32_strips(p, rows_hint), cu = compute_units();
+    const bool past = (int64_t)p.batches * p.N * p.K * 4 > (int64_t)256 << 20;
+    if (p.M <= 16 && !p.colsum) {
+        if (form == 1) return strips <= 2 * cu ? gemm_f32_wave_launch<1, 1, 8, false>(p, 1, stream, who) : gemm_f32_wave_launch<1, 1, 4, false>(p, 1, stream, who);
+        if (strips < 4 * cu) return gemm_f32_wave_launch<1, 1, 8, true>(p, strips < 2 * cu ? 1 : 4, stream, who);
+        if (past && strips >= 8 * cu) return gemm_f32_wave_launch<1, 4, 2, true, true>(p, 1, stream, who);
+        return gemm_f32_wave_launch<1, 2, 4, true>(p, strips < 5 * cu ? 1 : 4, stream, who);
+    }
+    if (form == 1) return strips < 4 * cu ? gemm_f32_wave_launch<2, 1, 4, false>(p, 1, stream, who) : gemm_f32_wave_launch<2, 2, 2, false>(p, 1, stream, who);
+    if (strips < 4 * cu) return gemm_f32_wave_launch<2, 1, 4, true>(p, strips <= 2 * cu ? 1 : 4, stream, who);
+    return past ? gemm_f32_wave_launch<2, 2, 4, true, true>(p, 1, stream, who) : gemm_f32_wave_launch<2, 2, 4, true>(p, 1, stream, who);
 }
 
 template <int F, bool TA, bool TB, int STAGES = 2>
@@ -357,11 +413,12 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 // The tile's side under a relu: a compute unit takes 1.9 us for a k-tile of 128 x 128 and 4 for the tile, 0.52 and
 // 1.2 for 64 x 64, 0.47 with four stages; what counts is the fullest compute unit (us, 64 x 64, with four stages, 128 x 128: 4 x 1000 rows,
 // 2048 -> 512 77, 66, 137; 16 x 512, 1024 -> 1024 142, 131, 131; 512 -> 2048 152, 144, 138; 2 x 4096, 4096 -> 4096 2129, 1944, 1969).
-// Waves on their own, up to 16 rows (32 where a tile has less than eight k-tiles), where they read the weight once (8 experts, 2 rows each: nn
-// 1024 -> 4096 44 -> 27 us, nt 41 -> 23, 4096 -> 1024 90 -> 39; tiles of four stages take 1.2 - 1.6 of their time at 2 rows, 1.0 at 16, 0.95 at 20).
+// Waves on their own, up to 32 rows, where they read the weight once (us in tiles of four stages and in waves, cold, nn, 8 experts x 20 rows, 1024 -> 4096
+// 48 and 34, 32 rows 1024 -> 1024 21 and 20, 21 rows 1896 -> 568 34 and 28, b^T 35 and 22), and beyond where all the strips of 32 rows by 16 columns
+// are few (4 x 64, 2048 -> 512 36 and 29).
 // The rows are those expected: with skewed routing an
 // expert has more, and its weight is read once for every 32 of them, but all experts together have as many rows as before,
-// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves and in tiles of two stages, nn, nt:
+// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves of 16 columns and in tiles of two stages, nn, nt:
 //   8 experts, 256 rows, 4096 -> 1024    even 69, 86 and 90, 89;     128 of the rows on one 70, 88 and 91, 90
 //   8 experts, 128 rows, 1024 -> 4096    even 31, 32 and 43, 42;     64 on one 44, 52 and 42, 42
 //   16 experts, 256 rows, 4096 -> 1024   even 55, 60 and 93, 97;     128 on one 123, 140 and 152, 155
@@ -427,8 +484,10 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
         return c.t64 <= c.in_parts() ? G32_SPLIT_64 : c.t128 <= c.t256 ? G32_SPLIT_128 : G32_SPLIT_256;
     }
     const bool deep = gemm_f32_deep(form, p, rows_hint);
-    if (form != 2 && rows_hint <= (deep ? 16 : 32) && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
-        gemm_f32_wave_pieces(p, 16) < ((int64_t)1 << 30))
+    // (few strips: a SIMD has one wave whichever it is, and one that reads for itself takes 12.6 ns for a k (b^T 9.5), a tile 15.2)
+    const bool few = rows_hint <= 32 || (p.K >= 512 && gemm_f32_strips(p, rows_hint) <= (form == 0 ? 5 : 8) * (int64_t)compute_units() / 4);
+    if (form != 2 && few && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
+        gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30))
         return G32_WAVES;
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
@@ -439,12 +498,11 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
     return cost(64, deep ? 0.47 : 0.52, 1.2) < cost(128, 1.9, 4) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
 }
 
-int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who)
+int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, int rows_hint, hipStream_t stream, const char *who)
 {
     switch (kernel) {
     case G32_WAVES:
-        if (p.M <= 16 && !p.colsum) return form == 0 ? gemm_f32_wave_launch<1, 16, true>(p, stream, who) : gemm_f32_wave_launch<1, 8, false>(p, stream, who);
-        return form == 0 ? gemm_f32_wave_launch<2, 8, true>(p, stream, who) : gemm_f32_wave_launch<2, 4, false>(p, stream, who);
+        return gemm_f32_waves(form, p, rows_hint, stream, who);
     case G32_TILE_64:
         if (form == 0) return gemm_f32_launch<1, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<1, false, false>(p, stream, who);

@@ -19,7 +19,7 @@ enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_DEEP_64, G32_TILE_128, G32_SPLIT
 
 // form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  rows_hint: rows in use
 Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint);
-int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who);
+int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, int rows_hint, hipStream_t stream, const char *who);
 int gemm_f32_split_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who);
 // column sums have two slots for so many rows
 inline int gemm_f32_slot_rows(Gemm32Kernel kernel) { return kernel == G32_TILE_128 || kernel == G32_SPLIT_128 || kernel == G32_SPLIT_256 ? 128 : 64; }

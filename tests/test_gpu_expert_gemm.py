@@ -769,3 +769,40 @@ def test_sums_of_shares_are_added_in_pairs(shares):
     torch.cuda.synchronize()
     want = 1.0 + (shares - 1) * 2.0 ** -24
     assert bool(((out.double() - want).abs() <= 2.0 ** -23).all()), (out[0, 0].item() - 1.0) * 2 ** 24
+
+
+# fp32, few rows: 16 and 32 rows of a wave, 16, 32 and 64 columns, work-groups of one and four waves, past the caches; columns and reductions that
+# nothing divides.  The same rows in a larger buffer go through the tiles, and the sums have the same order.
+@pytest.mark.parametrize("form,B,cap,n,k", [
+    ("nn", 4, 12, 52, 300), ("nn", 16, 16, 520, 36), ("nn", 16, 8, 1036, 148), ("nn", 16, 9, 1300, 20), ("nn", 16, 4, 2100, 2080),
+    ("nn", 4, 40, 52, 300), ("nn", 16, 33, 516, 44), ("nn", 16, 20, 1036, 212), ("nn", 16, 24, 1100, 3900), ("nn", 2, 70, 148, 724),
+    ("nt", 4, 12, 52, 200), ("nt", 16, 16, 1036, 148), ("nt", 4, 40, 68, 200), ("nt", 16, 33, 1060, 44)])
+def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
+    from planmoe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    hint, more = min(cap, 30), 100 if cap <= 64 else 600
+    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=True, rows_hint=cap if cap > 64 else hint) == "f32 waves"
+    edges = [cap, 0, 1, hint, 16, 17, 31, 33, 15, 32, 2, 5]
+    rows = [min(cap, edges[e % 12]) for e in range(B)]
+    live = torch.tensor([rows], dtype=torch.int32, device=DEV)
+    wide = rand(B, more, k)
+    few, w, bias = wide[:, :cap].contiguous(), rand(B, k, n) if form == "nn" else rand(B, n, k), rand(B, n)
+    for e, r in enumerate(rows):
+        few[e, r:] = float("nan")
+    sentinel = lambda rows: torch.full((B, rows, n), 7.0, device=DEV)
+    kw = dict(live=live, relu=form == "nn")
+    got = ops.expert_gemm(form, few, w, bias, out=sentinel(cap), rows_hint=cap if cap > 64 else hint, **kw)
+    want = ops.expert_gemm(form, wide, w, bias, out=sentinel(more), rows_hint=more, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want[:, :cap])
+    if form == "nt":
+        h = rand(B, more, n)
+        got, db = ops.expert_gemm_relu_bwd(few, w, h[:, :cap].contiguous(), live=live, out=sentinel(cap), rows_hint=hint)
+        want, _ = ops.expert_gemm_relu_bwd(wide, w, h, live=live, out=sentinel(more), rows_hint=more)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want[:, :cap])
+        for e, r in enumerate(rows):
+            ref = got[e, :r].double().sum(0)
+            # (at most cap additions, each rounded to 2^-24 of the sum so far)
+            assert bool(((db[e].double() - ref).abs() <= cap * 2.0 ** -24 * got[e, :r].double().abs().sum(0)).all())
