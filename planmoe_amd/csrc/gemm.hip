@@ -13,6 +13,7 @@
 // all with the operands as they lie in memory.
 #include "gemm_f32.hpp"
 #include "gemm_deep.hpp"
+#include "gemm_outer.hpp"
 #include "gemm_shares.hpp"
 #include "sums.hpp"
 #include <algorithm>
@@ -926,16 +927,20 @@ extern "C" int planmoe_expert_gemm(int form, int dtype, const void *a, const voi
     PM_REQUIRE(activation == 0 || activation == 1, "%s: activation is 0 (none) or 1 (relu)", who);
     PM_REQUIRE(!bias || form != 2, "%s: a weight gradient has no bias", who);
     hipStream_t st = (hipStream_t)stream;
+    const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
+    const OuterArgs outer{a, b, c, live, live_planes, live_round, m, n, k, batches};
     if (dtype == PLANMOE_F32) {
         Gemm32Args p{(const float *)a, (const float *)b, (const float *)bias, nullptr, (float *)c, nullptr, live, live_planes, live_round,
                      m, n, k, batches, activation};
-        const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
-        return gemm_f32_run(form, p, gemm_f32_pick(form, p, hint), hint, st, who);
+        const Gemm32Kernel kernel = gemm_f32_pick(form, p, hint);
+        // (products in parts only: the fp32 tiles have other sums)
+        if (form == 2 && kernel >= G32_SPLIT_64 && gemm_outer_serves(dtype, m, n, k, batches, hint)) return gemm_outer_run(dtype, outer, st, who);
+        return gemm_f32_run(form, p, kernel, hint, st, who);
     }
-    const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n, most = form == 2 ? k : m;
+    if (form == 2 && !activation && gemm_outer_serves(dtype, m, n, k, batches, hint)) return gemm_outer_run(dtype, outer, st, who);
+    const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n;
     GemmArgs p{(const uint16_t *)a, (const uint16_t *)b, (const uint16_t *)bias, nullptr, (uint16_t *)c, nullptr, live, live_planes,
                live_round, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n, batches, activation, 0, 0, !aligned16(bias)};
-    const int64_t hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
     if (form == 0) return gemm_run<false, true, false>(p, hint, st, who);
     if (form == 1) return gemm_run<false, false, false>(p, hint, st, who);
     return gemm_run<true, true, false>(p, hint, st, who);
@@ -955,8 +960,10 @@ extern "C" const char *planmoe_expert_gemm_kernel(int form, int dtype, int activ
     const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
     if (dtype == PLANMOE_F32) {
         static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
-        return names[gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint)];
+        const Gemm32Kernel kernel = gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint);
+        return form == 2 && kernel >= G32_SPLIT_64 && gemm_outer_serves(dtype, m, n, k, batches, hint) ? "f32 parts few rows" : names[kernel];
     }
+    if (form == 2 && !activation && gemm_outer_serves(dtype, m, n, k, batches, hint)) return "few rows";
     static const char *const names[] = {"few rows", "128x128 alone", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"};
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n;
     return names[gemm_pick(form, gemm_contiguous(form, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n), m, n, k, batches, counted, hint)];

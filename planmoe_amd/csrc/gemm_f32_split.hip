@@ -20,26 +20,12 @@
 // near what gemm_bf16_kernel reaches; 2000 us on the fp32 matrix cores, 137), issuing the splits at 64 x 64.  The two sums fill the registers there
 // (251 - 256 of 256, nothing spilt).
 #include "gemm_f32_core.hpp"
+#include "sp_split.hpp"
 
 namespace pm {
 
 typedef __bf16 sp_bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint8_t __attribute__((address_space(3))) *sp_lds;
-
-// The matrix cores read subnormal bf16 values as zero.  Times 2^24 every part of every fp32 value is a normal one (the last bit of a
-// subnormal fp32 value is 2^-149); what then overflows is found at the end.
-constexpr float SP_SCALE = 0x1p24f, SP_UNSCALE = 0x1p-48f;
-// two values into their parts, lo in bits 0 .. 15
-__device__ __forceinline__ void sp_split(float x0, float x1, uint32_t &h, uint32_t &m, uint32_t &l)
-{
-    x0 *= SP_SCALE;
-    x1 *= SP_SCALE;
-    h = f32x2_to_bf16x2(x0, x1);
-    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
-    m = f32x2_to_bf16x2(r0, r1);
-    const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
-    l = __builtin_amdgcn_perm(__float_as_uint(s1), __float_as_uint(s0), 0x07060302u);
-}
 
 // WM x WN waves of FM x FN fragments of 32 x 32
 template <int WM, int WN, int FM, int FN>

@@ -806,3 +806,43 @@ def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
             ref = got[e, :r].double().sum(0)
             # (at most cap additions, each rounded to 2^-24 of the sum so far)
             assert bool(((db[e].double() - ref).abs() <= cap * 2.0 ** -24 * got[e, :r].double().abs().sum(0)).all())
+
+
+# Weight gradients over few rows, stored past the caches and plainly, 64, 128 and 256 columns of a wave; sizes that nothing divides.  The same rows in a
+# larger buffer go through the tiles, and the sums have the same order.
+@pytest.mark.parametrize("dtype,B,cap,m,n", [
+    (torch.float32, 8, 1, 1028, 1024), (torch.float32, 8, 17, 1036, 1060), (torch.float32, 4, 100, 1024, 2084), (torch.float32, 8, 24, 2052, 4100),
+    (torch.float32, 8, 150, 712, 1024), (torch.bfloat16, 4, 1, 8, 16), (torch.bfloat16, 4, 16, 40, 64), (torch.bfloat16, 8, 33, 264, 1032),
+    (torch.bfloat16, 4, 90, 1032, 192), (torch.bfloat16, 3, 12, 72, 2056)])
+def test_expert_gemm_weight_gradients_of_few_rows_have_the_tiles_bits(dtype, B, cap, m, n):
+    from planmoe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    hint, more = min(cap, 100 if dtype == torch.float32 else 60), 300
+    assert ops.expert_gemm_kernel("tn", dtype, B, m, n, cap, counted=True, rows_hint=hint) == ("f32 parts few rows" if dtype == torch.float32 else "few rows")
+    tiles = ops.expert_gemm_kernel("tn", dtype, B, m, n, more, counted=True, rows_hint=more)
+    assert "few rows" not in tiles and (dtype != torch.float32 or "parts" in tiles)
+    edges = [cap, 0, 1, hint, 16, 17, 31, 33]
+    rows = [min(cap, edges[e % 8]) for e in range(B)]
+    live = torch.tensor([rows], dtype=torch.int32, device=DEV)
+    a, dy = (torch.randn(B, more, w, device=DEV, generator=g).to(dtype) for w in (m, n))
+    a[B - 1, 0, 3], dy[0, 0, 5] = float("inf"), float("nan")
+    few, few_dy = a[:, :cap].contiguous(), dy[:, :cap].contiguous()
+    for e, r in enumerate(rows):
+        few[e, r:], few_dy[e, r:] = float("nan"), float("nan")
+    behind = torch.full((B * m * n + 64,), 7.0, dtype=dtype, device=DEV)
+    out = behind[:B * m * n].view(B, m, n)
+    got = ops.expert_gemm("tn", few, few_dy, live=live, rows_hint=hint, out=out)
+    want = ops.expert_gemm("tn", a, dy, live=live, rows_hint=more)
+    torch.cuda.synchronize()
+    assert bool((behind[B * m * n:] == 7.0).all())
+    assert torch.equal(got.isnan(), want.isnan())
+    # (in parts a wave that meets what is not finite sums again in another order, and waves are not the same everywhere)
+    whole = [e for e in range(B) if bool(want[e].isfinite().all())]
+    assert len(whole) >= B - 2 and all(torch.equal(got[e], want[e]) for e in whole)
+    for e in set(range(B)) - set(whole):
+        keep = want[e].isfinite()
+        assert torch.equal(got[e].isfinite(), keep)
+        size = few[e, :rows[e]].double().abs().t().contiguous() @ few_dy[e, :rows[e]].double().abs()
+        # (up to cap products rounded to 2^-24 and as many sums, twice; a bf16 result is rounded to 2^-8 on top)
+        bound = (4 * cap * 2.0 ** -24 + (0 if dtype == torch.float32 else 2.0 ** -8)) * size
+        assert bool(((got[e].double() - want[e].double()).abs() <= bound)[keep].all())
