@@ -13,9 +13,12 @@
 //           slot) has a closed form and is not analysed at all.
 //   parse   the greedy token walk (gpulz.cu:98-127, one thread there) advances a whole run of
 //           literals or one match per step with ballots and scalar bit scans.
+//           Runs of one value with nothing else that repeats, as empty slots make between rows, have a closed form too: matches of 1, 2, 4, 8,
+//           16 and 32 symbols from their second on.  (Walked, such a block took a wave 20 us: 112 x 2600 with 40 % empty slots 29.8 us to compress,
+//           now 12.5 with the launch for the scan that small inputs go without.)
 //   pack    token ranks and byte offsets come from one packed wave scan; flags and token bytes
 //           are put together in LDS and copied out with aligned word stores.
-// The launches: sizes of every block (match + parse; two integers and a class byte per block are written, and, of a block
+// The launches (up to 16 MB without the second: a work-group of the placement adds up the sizes before its own itself): sizes of every block (match + parse; two integers and a class byte per block are written, and, of a block
 // with matches, its tokens: two bytes a position), an in-place exclusive scan of the sizes by chunks, and
 // placement (stored blocks are copied straight through, the tokens of the others packed at
 // their final offset; a wave adds up the totals of the chunks before its own, and spare work-groups zero what lies beyond all).  134 MB of N(0, 1):
@@ -34,6 +37,7 @@ constexpr int LZ_BLOCK_BYTES = 2048;
 constexpr int LZ_PITCH = WAVE + 4;        // words between a position's masks and the next one's of a lane
 constexpr int LZ_WAVES = 8;              // blocks per work-group
 constexpr int LZ_SCAN_CHUNK = 8192;      // table entries scanned by one work-group
+constexpr int LZ_SUMMED = 8192;          // up to so many blocks the placement adds up the sizes before its own by itself
 constexpr int LZ_MAX_CHUNKS = 256;       // (2^31 / 2048 + 1) / 8192 rounded up to the scan's width
 constexpr uint32_t NAN_WINDOW = 0x7f800002u;   // key of a NaN seen as a window symbol ...
 constexpr uint32_t NAN_AHEAD = 0x7f800001u;    // ... and as a look-ahead symbol: never equal
@@ -165,20 +169,27 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
         const uint4 v = *reinterpret_cast<const uint4 *>(keys + 8 * lane + 4 * q);
         win[4 * q] = v.x; win[4 * q + 1] = v.y; win[4 * q + 2] = v.z; win[4 * q + 3] = v.w;
     }
-    uint64_t hit[8], some = 0;                          // lane masks, kept in scalar registers
+    // (a lane whose first two symbols are equal, as in every run of ten and more: the masks below are wanted in any case; 2.3 us of a wave on its own)
+    uint64_t hit[8];                                    // lane masks, kept in scalar registers
+    if (__ballot(ahead_key(own[1]) == own[0]) == 0) {
+        uint64_t some = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t k = ahead_key(own[i]);
-        hit[i] = 0;
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t k = ahead_key(own[i]);
+            hit[i] = 0;
 #pragma unroll
-        for (int j = 0; j < LZ_WINDOW; ++j) hit[i] |= __ballot(k == win[i + j]);
-        some |= hit[i];
-    }
-    if (some == 0) {                                    // 512 literals, 64 zero flag bytes
-        wave_sync();                                    // the keys may be overwritten by the next block
-        b.flag_bytes = LZ_SYMS / 8;
-        b.data_bytes = LZ_BLOCK_BYTES;
-        return LZ_STORED;
+            for (int j = 0; j < LZ_WINDOW; ++j) hit[i] |= __ballot(k == win[i + j]);
+            some |= hit[i];
+        }
+        if (some == 0) {                                // 512 literals, 64 zero flag bytes
+            wave_sync();                                // the keys may be overwritten by the next block
+            b.flag_bytes = LZ_SYMS / 8;
+            b.data_bytes = LZ_BLOCK_BYTES;
+            return LZ_STORED;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) hit[i] = 1;
     }
     uint32_t live = 0;                                  // positions that some lane has a hit at
 #pragma unroll
@@ -194,6 +205,19 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
     wave_sync();
     // position 8 q + i lies at i * LZ_PITCH + q: the lanes' reads at one distance are neighbours.  Zero behind the block.
     if (lane < 32) hmask[(lane >> 2) * LZ_PITCH + WAVE + (lane & 3)] = 0;
+    uint32_t breaks = 0;                                // bit i: symbol 8l+i is not the one before it
+#pragma unroll
+    for (int i = 0; i < 8; ++i) breaks |= (ahead_key(own[i]) != win[LZ_WINDOW - 1 + i] ? 1u : 0u) << i;
+    // A run of one value: q symbols of it lie right before a position.  If a position's hits are those and no others, everywhere, the tokens have a
+    // closed form.
+    const uint64_t breaking = __ballot(breaks != 0);    // (lane 0: its first symbol)
+    const uint64_t lower = breaking & ((1ull << lane) - 1ull), upper = lane < WAVE - 1 ? breaking & ~((2ull << lane) - 1ull) : 0ull;
+    const int from = lower ? 63 - __builtin_clzll(lower) : 0, next = upper ? __builtin_ctzll(upper) : 0;
+    const uint32_t from_breaks = __shfl(breaks, from), next_breaks = __shfl(breaks, next);
+    const int begin = 8 * from + 31 - __builtin_clz(from_breaks | 1u);              // where the run that reaches the lane begins
+    const int end = upper ? 8 * next + __builtin_ctz(next_breaks | 256u) : LZ_SYMS;     // and where the one that leaves it ends
+    uint32_t others = 0;
+    int q = 8 * lane - begin - 1;
 #pragma unroll 1
     for (int i = 0; i < 8; ++i) {
         uint32_t m = 0;
@@ -202,11 +226,34 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
 #pragma unroll
             for (int j = LZ_WINDOW - 1; j >= 0; --j) m = shift_in_equal(m, k, win[j]);
         }
+        q = (breaks >> i) & 1u ? 0 : q + 1;
+        others |= m ^ (q == 0 ? 0u : q >= 32 ? 0xffffffffu : 0xffffffffu << (32 - q));
         hmask[i * LZ_PITCH + lane] = m;
 #pragma unroll
         for (int j = 0; j < 39; ++j) win[j] = win[j + 1];          // the next position's window and symbol
     }
     wave_sync();
+    if (__ballot(others != 0) == 0) {
+        // a literal, then matches of 1, 2, 4, 8, 16 and 32 symbols, each as far back as it is long, the last one as long as the run is
+        uint64_t lens = 0, offs = 0;
+        b.start_mask = b.match_mask = 0;
+        q = 8 * lane - begin - 1;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            q = (breaks >> i) & 1u ? 0 : q + 1;
+            const uint32_t above = breaks >> (i + 1);
+            const int left = above ? 1 + __builtin_ctz(above) : end - 8 * lane - i, reach = min(q, LZ_WINDOW);
+            b.start_mask |= (uint32_t)((q < LZ_WINDOW ? q & (q - 1) : q & (LZ_WINDOW - 1)) == 0) << i;
+            b.match_mask |= (uint32_t)(q != 0) << i;
+            lens |= (uint64_t)min(reach, left) << (8 * i);
+            offs |= (uint64_t)reach << (8 * i);
+        }
+        b.lens_lo = (uint32_t)lens; b.lens_hi = (uint32_t)(lens >> 32);
+        b.offs_lo = (uint32_t)offs; b.offs_hi = (uint32_t)(offs >> 32);
+        wave_sync();                                    // hmask is the key area of the next block
+        b.count();
+        return LZ_GENERAL;
+    }
 
     // ---- the reference's matcher (gpulz.cu:46-85) on the masks: a run starts at the next hit,
     // grows while the following positions hit at the same distance, and the window symbol after
@@ -301,15 +348,18 @@ __device__ __forceinline__ int lz_analyse(const uint32_t (&raw)[8], uint32_t *ke
     return LZ_GENERAL;
 }
 
-// ---- launch 1: sizes and class of every block
-__global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
+// ---- launch 1: sizes and class of every block.  WAVES: blocks of a work-group, which stays until the last of them is through.  Two where there are
+// work-groups enough, eight otherwise (us to compress, 8 and 2: 32768 x 1024, 30 % empty 98.9, 93.4; 65536 x 1000 247, 223; 16384 x 512 34.6, 36.6;
+// 8192 x 1024, none empty, 35.9, 37.1)
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * WAVE) void lz_sizes_kernel(
     const uint32_t *__restrict__ in, int64_t nsym, int64_t blocks, int32_t *__restrict__ flag_off,
-    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls, uint4 *__restrict__ tokens, uint32_t *__restrict__ cleared)
+    int32_t *__restrict__ data_off, uint8_t *__restrict__ cls, uint32_t *__restrict__ sizes, uint4 *__restrict__ tokens, uint32_t *__restrict__ cleared)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t keys[LZ_WAVES][LZ_WINDOW + LZ_SYMS];
+    __shared__ __attribute__((aligned(16))) uint32_t keys[WAVES][LZ_WINDOW + LZ_SYMS];
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
-    const int64_t block = (int64_t)blockIdx.x * LZ_WAVES + wave;
+    const int64_t block = (int64_t)blockIdx.x * WAVES + wave;
     if (block >= blocks) return;                       // no work-group barrier below
     uint32_t raw[8];
     lz_load(in, nsym, block, lane, raw);
@@ -327,10 +377,14 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_sizes_kernel(
     const int c = lz_analyse(raw, keys[wave], lane, b);
     if (c == LZ_GENERAL) tokens[block * WAVE + lane] = b.tokens();
     if (lane == 0) {
-        flag_off[block] = (int32_t)b.flag_bytes;
-        data_off[block] = (int32_t)b.data_bytes;
         cls[block] = (uint8_t)c;
-        if (block == blocks - 1) { flag_off[blocks] = 0; data_off[blocks] = 0; }
+        if (sizes) {
+            sizes[block] = b.flag_bytes | b.data_bytes << 16;
+        } else {
+            flag_off[block] = (int32_t)b.flag_bytes;
+            data_off[block] = (int32_t)b.data_bytes;
+            if (block == blocks - 1) { flag_off[blocks] = 0; data_off[blocks] = 0; }
+        }
     }
 }
 
@@ -411,22 +465,52 @@ __device__ __forceinline__ void lz_clear_slack(int64_t tid, int64_t nthreads, in
     }
 }
 
+// the sums of the first n blocks' sizes and, in wave w, of w more: flags, data.  All waves of the work-group call it; n <= LZ_SUMMED
+__device__ __forceinline__ uint2 lz_sizes_before(const uint32_t *__restrict__ sizes, int n, int more, int64_t blocks, uint32_t (*partial)[2])
+{
+    const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
+    const uint32_t own = sizes[min((int64_t)n + lane, blocks - 1)];
+    uint32_t f = 0, d = 0;
+    for (int i0 = threadIdx.x; i0 - (int)threadIdx.x < n; i0 += 4 * LZ_WAVES * WAVE) {
+        uint32_t v[4];                                  // (straight-line loads at addresses that are there)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = sizes[min(i0 + q * LZ_WAVES * WAVE, n - 1)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t x = i0 + q * LZ_WAVES * WAVE < n ? v[q] : 0u;
+            f += x & 0xffffu;
+            d += x >> 16;
+        }
+    }
+    auto sum = [](uint32_t a, uint32_t b) { return a + b; };
+    f = (uint32_t)wave_allreduce((int)f, sum);
+    d = (uint32_t)wave_allreduce((int)d, sum);
+    if (lane == 0) { partial[wave][0] = f; partial[wave][1] = d; }
+    __syncthreads();
+    f = d = 0;
+    if (lane < LZ_WAVES) { f = partial[lane][0]; d = partial[lane][1]; }
+    if (lane < more) { f += own & 0xffffu; d += own >> 16; }
+    return make_uint2((uint32_t)wave_allreduce((int)f, sum), (uint32_t)wave_allreduce((int)d, sum));
+}
+
 struct __attribute__((aligned(16))) LzPlaceShared {
     uint16_t stage[LZ_WAVES][LZ_BLOCK_BYTES / 2];   // token bytes of the block
     uint32_t flagw[LZ_WAVES][16];                   // flag bits of the block
 };
 
-// ---- launch 3: every block to its final place, and zeros behind the last
+// ---- the last launch: every block to its final place, and zeros behind the last.  SUMMED: by the blocks' sizes, without a scan before
+template <bool SUMMED>
 __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     const uint32_t *__restrict__ in, int64_t nsym, int64_t blocks, int32_t *__restrict__ flag_off,
-    int32_t *__restrict__ data_off, const uint8_t *__restrict__ cls, const uint32_t *__restrict__ totals, int chunks, const uint4 *__restrict__ tokens,
-    uint8_t *__restrict__ flags, uint8_t *__restrict__ data)
+    int32_t *__restrict__ data_off, const uint8_t *__restrict__ cls, const uint32_t *__restrict__ totals, int chunks, const uint32_t *__restrict__ sizes,
+    const uint4 *__restrict__ tokens, uint8_t *__restrict__ flags, uint8_t *__restrict__ data)
 {
     __shared__ LzPlaceShared sh;
+    __shared__ uint32_t partial[LZ_WAVES][2];
     // the work-groups behind the blocks' clear what lies beyond the totals
     const int64_t groups = (blocks + LZ_WAVES - 1) / LZ_WAVES;
     if (blockIdx.x >= groups) {
-        const uint2 all = lz_chunks_before(totals, chunks);
+        const uint2 all = SUMMED ? lz_sizes_before(sizes, (int)blocks, 0, blocks, partial) : lz_chunks_before(totals, chunks);
         lz_clear_slack(((int64_t)blockIdx.x - groups) * LZ_WAVES * WAVE + threadIdx.x, ((int64_t)gridDim.x - groups) * LZ_WAVES * WAVE,
                        (int32_t)all.x, (int32_t)all.y, blocks, flags, data);
         return;
@@ -434,20 +518,29 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
     const int64_t block = (int64_t)blockIdx.x * LZ_WAVES + wave;
-    if (block >= blocks) return;                       // no work-group barrier below
+    if (!SUMMED && block >= blocks) return;            // no work-group barrier below
 
     uint32_t raw[8];
     lz_load(in, nsym, block, lane, raw);
-    const int64_t chunk = block / LZ_SCAN_CHUNK;
-    const uint2 before = lz_chunks_before(totals, (int)chunk);
-    const uint32_t fbase = (uint32_t)flag_off[block] + before.x;
-    const uint32_t dbase = (uint32_t)data_off[block] + before.y;
+    uint2 before;
+    if (SUMMED) {
+        before = lz_sizes_before(sizes, (int)blockIdx.x * LZ_WAVES, wave, blocks, partial);
+        if (block >= blocks) return;                   // no work-group barrier below
+    } else {
+        before = lz_chunks_before(totals, (int)(block / LZ_SCAN_CHUNK));
+    }
+    const uint32_t fbase = (SUMMED ? 0u : (uint32_t)flag_off[block]) + before.x;
+    const uint32_t dbase = (SUMMED ? 0u : (uint32_t)data_off[block]) + before.y;
     int c = cls[block];
     c = __builtin_amdgcn_readfirstlane(c);
     // never let a wrong table move a write out of the buffers
     const uint32_t fb = min(fbase, (uint32_t)(block * (LZ_SYMS / 8)));
     const uint32_t db = min(dbase, (uint32_t)(block * LZ_BLOCK_BYTES)) & ~1u;
-    const uint2 all = block == blocks - 1 ? lz_chunks_before(totals, chunks) : make_uint2(0u, 0u);
+    uint2 all = make_uint2(0u, 0u);
+    if (block == blocks - 1) {
+        if (SUMMED) { const uint32_t own = sizes[block]; all = make_uint2(fbase + (own & 0xffffu), dbase + (own >> 16)); }
+        else all = lz_chunks_before(totals, chunks);
+    }
     if (lane == 0) {
         flag_off[block] = (int32_t)fbase;
         data_off[block] = (int32_t)dbase;
@@ -531,9 +624,11 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_place_kernel(
         *reinterpret_cast<uint16_t *>(dst + data_bytes - 2) = stage[data_bytes / 2 - 1];
 }
 
+constexpr int LZ_DEC_WAVES = 2;          // a work-group's waves wait for its slowest: 65536 x 1000, 30 % empty, 1, 2, 4, 8 waves 74, 77, 84, 109 us
+
 struct LzDecodeShared {
-    uint32_t bytes[LZ_WAVES][LZ_BLOCK_BYTES / 4 + 1];  // token bytes of the block (one spare word)
-    uint32_t out[LZ_WAVES][LZ_SYMS];
+    uint32_t bytes[LZ_DEC_WAVES][LZ_BLOCK_BYTES / 4 + 1];  // token bytes of the block (one spare word)
+    uint32_t out[LZ_DEC_WAVES][LZ_SYMS];
 };
 
 __device__ __forceinline__ uint32_t lds_u16(const uint32_t *words, uint32_t byte_at)   // byte_at even
@@ -648,9 +743,9 @@ __device__ __forceinline__ void lz_decode_block(uint32_t *__restrict__ out, int6
     }
 }
 
-constexpr int LZ_DEC_PER = 4;            // blocks per wavefront: their loads are in flight together
-
-__global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_decompress_kernel(
+// A wave a block.  (Two and four blocks a wave with their loads in flight together wait for each other where blocks have matches: us of 1, 2 and 4,
+// 134 MB with 30 % empty slots 37.5, 38.5, 39.8; 10 MB, rows of 640, 9.1, 13.4, 18.7; 400 rows of 300, half of them empty, 7.8, 13.0, 23.2.)
+__global__ __launch_bounds__(LZ_DEC_WAVES * WAVE) void lz_decompress_kernel(
     uint32_t *__restrict__ out, int64_t nsym, int64_t blocks, const int32_t *__restrict__ flag_off,
     const int32_t *__restrict__ data_off, const uint8_t *__restrict__ flags,
     const uint8_t *__restrict__ data)
@@ -658,91 +753,42 @@ __global__ __launch_bounds__(LZ_WAVES * WAVE) void lz_decompress_kernel(
     __shared__ LzDecodeShared sh;
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
-    const int64_t first = ((int64_t)blockIdx.x * LZ_WAVES + wave) * LZ_DEC_PER;
-    if (first >= blocks) return;                       // no work-group barrier below
+    const int64_t block = (int64_t)blockIdx.x * LZ_DEC_WAVES + wave;
+    if (block >= blocks) return;                       // no work-group barrier below
 
-    // All loads below are unconditional, at clamped addresses: a load under a branch would make
-    // every later wait drain the whole queue, and the blocks would be fetched one after the other.
-    const int64_t fcap = blocks * (LZ_SYMS / 8), dcap = blocks * LZ_BLOCK_BYTES;
-    int32_t fo[LZ_DEC_PER + 1], dofs[LZ_DEC_PER + 1];
-#pragma unroll
-    for (int u = 0; u <= LZ_DEC_PER; ++u) {
-        const int64_t e = min(first + u, blocks);
-        fo[u] = flag_off[e];
-        dofs[u] = data_off[e];
-    }
+    // All loads up to the first branch are unconditional, at clamped addresses: a load under a branch would make
+    // every later wait drain the whole queue.
     // offsets of a stream of this coder ascend and stay inside the buffers; clamp all the same
-    int64_t f0[LZ_DEC_PER], d0[LZ_DEC_PER];
-    uint32_t nflag[LZ_DEC_PER], nbytes[LZ_DEC_PER], fb[LZ_DEC_PER];
-    bool direct[LZ_DEC_PER];
-    pm_u32x4 va[LZ_DEC_PER], vb[LZ_DEC_PER];
-#pragma unroll
-    for (int u = 0; u < LZ_DEC_PER; ++u) {
-        const int64_t block = min(first + u, blocks - 1);
-        f0[u] = min(max((int64_t)fo[u], (int64_t)0), fcap);
-        const int64_t f1 = min(max((int64_t)fo[u + 1], f0[u]), min(f0[u] + LZ_SYMS / 8, fcap));
-        d0[u] = min(max((int64_t)dofs[u], (int64_t)0), dcap) & ~(int64_t)1;
-        const int64_t d1 = min(max((int64_t)dofs[u + 1], d0[u]), min(d0[u] + LZ_BLOCK_BYTES, dcap));
-        nflag[u] = (uint32_t)(f1 - f0[u]);
-        nbytes[u] = (uint32_t)(d1 - d0[u]);
-        // a stored block (512 literals) is its own bytes: fetch them before the flags are known
-        direct[u] = nflag[u] == LZ_SYMS / 8 && nbytes[u] == LZ_BLOCK_BYTES && block * LZ_SYMS + LZ_SYMS <= nsym;
-    }
-#pragma unroll
-    for (int u = 0; u < LZ_DEC_PER; ++u) {
-        fb[u] = flags[min(f0[u] + lane, fcap - 1)];                        // lane l: tokens 8l .. 8l+7
-        const lz_u32x4_a2 *src = reinterpret_cast<const lz_u32x4_a2 *>(data + (direct[u] ? d0[u] : 0));
-        va[u] = src[lane];                             // 1 KB per instruction
-        vb[u] = src[lane + WAVE];
-    }
-    uint32_t rest = 0;
-#pragma unroll
-    for (int u = 0; u < LZ_DEC_PER; ++u) {
-        const int64_t block = first + u;
-        if (block >= blocks) break;
-        if (direct[u] && __ballot((uint32_t)lane < nflag[u] && fb[u] != 0) == 0) {
-            pm_u32x4 *dst = reinterpret_cast<pm_u32x4 *>(out + block * LZ_SYMS);
-            __builtin_nontemporal_store(va[u], dst + lane);
-            __builtin_nontemporal_store(vb[u], dst + lane + WAVE);
-        } else {
-            rest |= 1u << u;
-        }
+    const int64_t fcap = blocks * (LZ_SYMS / 8), dcap = blocks * LZ_BLOCK_BYTES;
+    const int64_t f0 = min(max((int64_t)flag_off[block], (int64_t)0), fcap), d0 = min(max((int64_t)data_off[block], (int64_t)0), dcap) & ~(int64_t)1;
+    const int64_t f1 = min(max((int64_t)flag_off[block + 1], f0), min(f0 + LZ_SYMS / 8, fcap));
+    const int64_t d1 = min(max((int64_t)data_off[block + 1], d0), min(d0 + LZ_BLOCK_BYTES, dcap));
+    const uint32_t nflag = (uint32_t)(f1 - f0), nbytes = (uint32_t)(d1 - d0);
+    // a stored block (512 literals) is its own bytes: fetch them before the flags are known
+    const bool whole = block * LZ_SYMS + LZ_SYMS <= nsym, direct = nflag == LZ_SYMS / 8 && nbytes == LZ_BLOCK_BYTES && whole;
+    const uint32_t fb = flags[min(f0 + lane, fcap - 1)];                   // lane l: tokens 8l .. 8l+7
+    const lz_u32x4_a2 *src = reinterpret_cast<const lz_u32x4_a2 *>(data + (direct ? d0 : 0));
+    const pm_u32x4 va = src[lane], vb = src[lane + WAVE];                  // 1 KB per instruction
+    pm_u32x4 *dst = reinterpret_cast<pm_u32x4 *>(out + block * LZ_SYMS);
+    if (direct && __ballot((uint32_t)lane < nflag && fb != 0) == 0) {
+        __builtin_nontemporal_store(va, dst + lane);
+        __builtin_nontemporal_store(vb, dst + lane + WAVE);
+        return;
     }
     // Blocks of one repeated value (empty capacity slots): this coder's 44 bytes for it -- the value, (1,1) (2,2) (4,4) (8,8)
-    // (16,16) and (32,32) to the end -- are recognised as a whole and not walked match by match.  All four blocks' bytes are
-    // asked for together.  (134 MB with 30 % of its slots empty: decompress 70 us when they were walked, 50 now.)
-    uint32_t token[LZ_DEC_PER];
-#pragma unroll
-    for (int u = 0; u < LZ_DEC_PER; ++u) token[u] = 0;
-    if (rest != 0) {
-#pragma unroll
-        for (int u = 0; u < LZ_DEC_PER; ++u)
-            token[u] = *reinterpret_cast<const uint16_t *>(data + min(d0[u] + 2 * min(lane, 21), dcap - 2));
+    // (16,16) and (32,32) to the end -- are recognised as a whole and not walked match by match.  (134 MB with 30 % of its slots
+    // empty: 70 us when they were walked.)
+    if (nflag == 3 && nbytes == 44 && whole) {
+        const uint32_t token = *reinterpret_cast<const uint16_t *>(data + min(d0 + 2 * min(lane, 21), dcap - 2));
         const uint32_t n = lane < 7 ? 1u << max(lane - 2, 0) : 32u, flag = lane == 0 ? 0xfeu : lane == 1 ? 0xffu : 0x1fu;
-#pragma unroll
-        for (int u = 0; u < LZ_DEC_PER; ++u) {
-            const int64_t block = first + u;
-            const bool odd = (lane >= 2 && lane < 22 && token[u] != (n | (n << 8))) || (lane < 3 && fb[u] != flag);
-            if (!((rest >> u) & 1u) || nflag[u] != 3 || nbytes[u] != 44 || block * LZ_SYMS + LZ_SYMS > nsym || __ballot(odd) != 0) continue;
-            const uint32_t v = __builtin_amdgcn_readlane(token[u], 0) | (__builtin_amdgcn_readlane(token[u], 1) << 16);
-            pm_u32x4 *dst = reinterpret_cast<pm_u32x4 *>(out + block * LZ_SYMS);
+        if (__ballot((lane >= 2 && lane < 22 && token != (n | (n << 8))) || (lane < 3 && fb != flag)) == 0) {
+            const uint32_t v = __builtin_amdgcn_readlane(token, 0) | (__builtin_amdgcn_readlane(token, 1) << 16);
             __builtin_nontemporal_store(pm_u32x4{v, v, v, v}, dst + lane);
             __builtin_nontemporal_store(pm_u32x4{v, v, v, v}, dst + lane + WAVE);
-            rest &= ~(1u << u);
+            return;
         }
     }
-    // (one copy of the decoder's code: four, each walked once, were 24 KB of instructions to wait for)
-#pragma unroll 1
-    for (; rest != 0; rest &= rest - 1) {
-        const int u = __builtin_ctz(rest);
-        int64_t d = d0[0];
-        uint32_t nf = nflag[0], nb = nbytes[0], bits = fb[0];
-#pragma unroll
-        for (int w = 1; w < LZ_DEC_PER; ++w)
-            if (u == w) { d = d0[w]; nf = nflag[w]; nb = nbytes[w]; bits = fb[w]; }
-        lz_decode_block(out, nsym, first + u, lane, (uint32_t)lane < nf ? bits : 0u, nf, d, nb, data, sh.bytes[wave], sh.out[wave]);
-        wave_sync();                                   // the LDS of the wavefront serves the next block
-    }
+    lz_decode_block(out, nsym, block, lane, (uint32_t)lane < nflag ? fb : 0u, nflag, d0, nbytes, data, sh.bytes[wave], sh.out[wave]);
 }
 
 int lz_check(const char *who, int64_t nbytes)
@@ -764,9 +810,10 @@ extern "C" int64_t planmoe_lz_blocks(int64_t nbytes)
     return nbytes <= 0 ? 0 : (nbytes + LZ_BLOCK_BYTES - 1) / LZ_BLOCK_BYTES;
 }
 
-// workspace: class byte per block | chunk totals | tokens of the blocks with matches, two bytes a position
+// workspace: class byte per block | chunk totals | sizes, up to LZ_SUMMED blocks | tokens of the blocks with matches, two bytes a position
 static size_t lz_class_bytes(int64_t blocks) { return round_up((size_t)blocks, 256); }
-static size_t lz_tokens_at(int64_t blocks) { return lz_class_bytes(blocks) + 2 * LZ_MAX_CHUNKS * sizeof(uint32_t); }
+static size_t lz_sizes_at(int64_t blocks) { return lz_class_bytes(blocks) + 2 * LZ_MAX_CHUNKS * sizeof(uint32_t); }
+static size_t lz_tokens_at(int64_t blocks) { return lz_sizes_at(blocks) + (blocks <= LZ_SUMMED ? round_up((size_t)blocks * 4, 256) : 0); }
 
 extern "C" size_t planmoe_lz_workspace_bytes(int64_t nbytes)
 {
@@ -796,17 +843,22 @@ static int lz_compress_and_clear(const char *who, const void *input, int64_t nby
                "%s: workspace too small or not 4-byte aligned", who);
     uint8_t *cls = (uint8_t *)workspace;
     uint32_t *totals = (uint32_t *)(cls + lz_class_bytes(blocks));
+    const bool summed = blocks <= LZ_SUMMED;
+    uint32_t *sizes = summed ? (uint32_t *)(cls + lz_sizes_at(blocks)) : nullptr;
     uint4 *tokens = (uint4 *)(((uintptr_t)workspace + lz_tokens_at(blocks) + 15) / 16 * 16);
     const int64_t groups = (blocks + LZ_WAVES - 1) / LZ_WAVES;
     const int64_t entries = blocks + 1;
     const int chunks = (int)((entries + LZ_SCAN_CHUNK - 1) / LZ_SCAN_CHUNK);      // <= 128 below 2^31 bytes
-    lz_sizes_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
-                                                                flag_offsets, data_offsets, cls, tokens, (uint32_t *)cleared);
-    lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals);
+    const int64_t waves = blocks > 2 * LZ_SUMMED ? 2 : LZ_WAVES;
+    const auto classify = waves == 2 ? lz_sizes_kernel<2> : lz_sizes_kernel<LZ_WAVES>;
+    classify<<<(unsigned)((blocks + waves - 1) / waves), waves * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks,
+                                                                flag_offsets, data_offsets, cls, sizes, tokens, (uint32_t *)cleared);
+    if (!summed) lz_scan_chunks_kernel<<<chunks, 256, 0, st>>>(flag_offsets, data_offsets, entries, totals);
     const int64_t slack_chunks = (blocks * LZ_BLOCK_BYTES / 16 + 255) / 256;          // enough for all of data
     const int64_t clear_groups = min((slack_chunks + 1) / 2, (int64_t)(chunks > 1 ? 2048 : 256));
-    lz_place_kernel<<<(unsigned)(groups + clear_groups), LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks, flag_offsets,
-                                                                                 data_offsets, cls, totals, chunks, tokens, flags, data);
+    const auto place = summed ? lz_place_kernel<true> : lz_place_kernel<false>;
+    place<<<(unsigned)(groups + clear_groups), LZ_WAVES * WAVE, 0, st>>>((const uint32_t *)input, nbytes / 4, blocks, flag_offsets, data_offsets, cls, totals, chunks,
+                                                                       sizes, tokens, flags, data);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -837,8 +889,8 @@ extern "C" int planmoe_lz_decompress(void *output, int64_t nbytes, const int32_t
     PM_REQUIRE(output && flag_offsets && data_offsets && flags && data, "planmoe_lz_decompress: NULL argument");
     PM_REQUIRE(aligned16(output) && (reinterpret_cast<uintptr_t>(data) & 3u) == 0,
                "planmoe_lz_decompress: output must be 16-byte and data 4-byte aligned");
-    const int64_t groups = (blocks + LZ_WAVES * LZ_DEC_PER - 1) / (LZ_WAVES * LZ_DEC_PER);
-    lz_decompress_kernel<<<(unsigned)groups, LZ_WAVES * WAVE, 0, (hipStream_t)stream>>>(
+    const int64_t groups = (blocks + LZ_DEC_WAVES - 1) / LZ_DEC_WAVES;
+    lz_decompress_kernel<<<(unsigned)groups, LZ_DEC_WAVES * WAVE, 0, (hipStream_t)stream>>>(
         (uint32_t *)output, nbytes / 4, blocks, flag_offsets, data_offsets, flags, data);
     PM_LAUNCH_CHECK("planmoe_lz_decompress");
     return 0;

@@ -83,6 +83,36 @@ def test_dispatched_buffer_with_empty_slots():
     assert int(do[-1]) < x.nbytes                        # the empty slots shrink
 
 
+@pytest.mark.parametrize("seed", range(4))
+def test_runs_of_one_value(seed):
+    """Runs of every length, zero and not, NaN, across and at the ends of blocks; blocks with nothing else and blocks where something else repeats."""
+    rng = np.random.default_rng(100 + seed)
+    parts, at = [], 0
+    while at < 600 * 512:
+        n = int(rng.choice([1, 2, 3, 4, 5, 8, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 100, 255, 511, 512, 513, 700])) + int(rng.integers(0, 3))
+        parts.append(np.full(n, rng.choice([0.0, -0.0, np.nan, 1.5, float(rng.standard_normal())]), np.float32))
+        between = rng.standard_normal(int(rng.choice([0, 1, 2, 30, 33, 40, 480, 512]))).astype(np.float32)
+        if seed % 2 and between.size > 20:
+            between[rng.integers(0, between.size)] = parts[-1][0]          # (and once more, near or far)
+        parts.append(between)
+        at += n + between.size
+    x = np.concatenate(parts)[:600 * 512]
+    check(x)
+    for first in range(0, 40):                           # one break in a block, at every place of a lane
+        b = np.zeros(512, np.float32)
+        b[first * 13 % 512:] = np.arange(512 - first * 13 % 512) + 1 if first % 2 else 3.0
+        check(b)
+
+
+@pytest.mark.parametrize("nblocks", [1, 7, 8, 9, 511, 513, 2048, 4095, 8191, 8192, 8193])
+def test_offsets_with_and_without_a_scan(nblocks):
+    rng = np.random.default_rng(nblocks)
+    x = rng.standard_normal(nblocks * 512).astype(np.float32).reshape(nblocks, 512)
+    x[rng.random(nblocks) < 0.3] = 0.0
+    x[rng.random(nblocks) < 0.2, 100:300] = 2.0
+    check(x)
+
+
 def test_many_blocks_and_scan_chunks():
     # 40 000 blocks: the offset tables span several chunks of the scan
     rng = np.random.default_rng(6)
