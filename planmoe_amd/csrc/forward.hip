@@ -504,9 +504,10 @@ static void launch_gate_route(int experts, int groups, int group_tokens, hipStre
                               int32_t *indices, int32_t *locations, void *gates, int64_t stride,
                               void *logits_out, void *scores_out, float *l_aux, int32_t *counts, void *ws, int one, void *rows, int capacity)
 {
-#define PM_GR_1(CAP, ONE, WGS)                                                                           \
-    gate_route_kernel<DT, SDT, 1, CAP, true, 32, 0, ONE><<<WGS, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
+#define PM_GR_2(CAP, ONE, WGS, GROUP)                                                                    \
+    gate_route_kernel<DT, SDT, 1, CAP, true, GROUP, 0, ONE><<<WGS, 256, 0, st>>>(x, wg, bias, samples, model_dim, experts, \
         k, normalize, indices, locations, gates, stride, logits_out, scores_out, l_aux, counts, ws, (uint8_t *)rows, capacity)
+#define PM_GR_1(CAP, ONE, WGS) do { if (group_tokens == 16) PM_GR_2(CAP, ONE, WGS, 16); else PM_GR_2(CAP, ONE, WGS, 32); } while (0)
 #define PM_GR_ONE(CAP) do { if (one == OUT_ROWS) PM_GR_1(CAP, OUT_ROWS, (samples + 3) / 4);              \
                             else if (one == OUT_DECODED) PM_GR_1(CAP, OUT_DECODED, (samples + 3) / 4); else PM_GR_1(CAP, ONE_ROUTING, 1); } while (0)
     if constexpr (DT != PLANMOE_F16) {
@@ -515,6 +516,7 @@ static void launch_gate_route(int experts, int groups, int group_tokens, hipStre
             return;
         }
     }
+#undef PM_GR_2
 #undef PM_GR_1
 #undef PM_GR_ONE
 #define PM_GR_(NT, CAP, SPLITK, GROUP)                                                                   \
@@ -594,7 +596,7 @@ static void fwd_plan(FwdPlan &plan, void *workspace, int dtype, int samples, int
     plan.experts_per_block = go_experts_per_block(experts, plan.k);
     plan.blocks = (experts + plan.experts_per_block - 1) / plan.experts_per_block;
     plan.merged = plan.k <= 4;
-    plan.one = plan.groups == 1 && plan.merged && experts <= 16 && plan.group_tokens == 32;
+    plan.one = plan.groups == 1 && plan.merged && experts <= 16 && plan.group_tokens <= 32;
     plan.ws = fwd_ws(workspace, plan.groups, plan.k, experts, samples);
 }
 
@@ -700,10 +702,9 @@ static int run_gate_route(const void *x, const void *wg, int dtype, int fp32_gat
                           const float *logit_bias, int samples, int model_dim, int experts, int top_k,
                           int normalize_gate, int32_t *indices, int32_t *locations, void *gates,
                           int64_t stride, void *logits_out, void *scores_out, float *l_aux,
-                          int32_t *counts, void *workspace, hipStream_t st, FwdPlan &plan,
+                          int32_t *counts, void *workspace, hipStream_t st, const FwdPlan &plan,
                           bool offsets_follow, int one = ONE_OFF, void *rows = nullptr, int capacity = 0)
 {
-    fwd_plan(plan, workspace, dtype, samples, model_dim, experts, top_k);
     const int k = plan.k, groups = plan.groups;
     if (fp32_gate || dtype == PLANMOE_F32) {
         PM_DTYPE_SWITCH(dtype, DT, (launch_gate_route<DT, PLANMOE_F32>(

@@ -23,8 +23,12 @@ inline int fwd_group_tokens(int experts, int samples, int64_t row_bytes)
     //   bf16, 8 x 512     40 tokens 9.5, 9.8     200 10.0, 10.5    4096 14.0, 14.1      8 x 1024   10.9, 10.7   11.4, 11.2   16.4, 16.1
     //   fp32, 8 x 256     40 tokens 9.1, 9.4     200  9.9, 10.5    4096 14.0, 14.2      8 x 512    10.8, 10.8   11.0, 11.1   16.4, 16.6
     //   fp32, 4 x 512     40 tokens 9.0, 9.0     200  9.5, 9.3     4096 13.4, 13.4      8 x 768    11.8, 10.9   12.4, 11.5   18.9, 18.1
-    // (up to 32 tokens are one group, and one launch: plan.one)
-    if (experts <= 16) return samples > 32 && samples <= 16 * cu && (experts > 8 || row_bytes >= 2048) ? 16 : samples < 64 * cu ? 32 : 64;
+    // Up to 32 tokens are one group, and one launch (plan.one); up to 16 of them have the products of 16, half the loads and in fp32 half the matrix cores' time.  us of a layer's pass on the GPU with 32 and with 16,
+    // 8 tokens: bf16, 8 x 1024 -> 4096 37.5, 36.0; 16 x 3840 -> 256 35.3, 32.8
+    if (experts <= 16) {
+        if (samples <= 16) return 16;
+        return samples > 32 && samples <= 16 * cu && (experts > 8 || row_bytes >= 2048) ? 16 : samples < 64 * cu ? 32 : 64;
+    }
     // as many groups as compute units at most (16 tokens: where four waves find a share of the experts).  us of the send side, bf16, with 64, 32, 16:
     //   64 experts x 1368   48 tokens 26, 22, 21;  4074 33, 29, 27;  8000 35, 32, 42;  16000 39, 47, 74
     //   32 experts x 1368   48 tokens 24, 20;      4074 33, 24;      8000 35, 28;      16000 42, 42
@@ -96,7 +100,8 @@ struct GateShared {
 
 // Group `block` of `groups`; with ONE, where several work-groups route the same tokens, the `first` writes the routing.
 // Two barriers; what is left in `sh` is there behind another.
-template <int DT, int SDT, int NT, int CAP, bool SPLITK, int GROUP, int MODE, int ONE>
+// DEPTH: steps of the products on their way, up to 16 experts
+template <int DT, int SDT, int NT, int CAP, bool SPLITK, int GROUP, int MODE, int ONE, int DEPTH = GROUP == 16 ? 4 : 2>
 __device__ __forceinline__ void gate_route_group(
     GateShared<DT, NT, CAP, SPLITK, GROUP, MODE, ONE> &sh, bool first, int block, int groups,
     const void *__restrict__ x, const void *__restrict__ wg, const float *__restrict__ logit_bias,
@@ -146,7 +151,7 @@ __device__ __forceinline__ void gate_route_group(
             }
         }
     } else if constexpr (SPLITK) {
-        constexpr int DEPTH = GROUP == 16 ? 4 : 2;            // (groups of 32, two on some compute units: 8 x 4096 fp32, 6500 tokens 68 us with two, 70 with four)
+        // (DEPTH: groups of 32, two on some compute units: 8 x 4096 fp32, 6500 tokens 68 us with two, 70 with four)
         if constexpr (STATS) gate_tile_partials<DT, NT, GROUP / 16, 4, true, DEPTH>(x, wg, t0, samples, model_dim, experts, part, pstat);
         else gate_tile_partials<DT, NT, GROUP / 16, 4, false, DEPTH>(x, wg, t0, samples, model_dim, experts, part);
     } else {

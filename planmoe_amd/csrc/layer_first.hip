@@ -33,13 +33,13 @@ struct FirstArgs {
 
 constexpr int FIRST_WAVES = 16, FIRST_TOKENS = 32, FIRST_ROWS = 16;          // a group's tokens, an expert's rows
 
-// CAP: bound of the number of experts.  DECODED: rows go through the int8 codec.  C, U, LARGE: as gemm_skinny_kernel
-template <int CAP, bool DECODED, int C, int U, bool LARGE>
+// TOKENS: a group's, 16 or 32.  CAP: bound of the number of experts.  DECODED: rows go through the int8 codec.  C, U, LARGE: as gemm_skinny_kernel
+template <int TOKENS, int CAP, bool DECODED, int C, int U, bool LARGE>
 __global__ __launch_bounds__(FIRST_WAVES * 64) void layer_first_kernel(const SkinnyArgs p, const FirstArgs r)
 {
     constexpr int ONE = DECODED ? OUT_DECODED : OUT_ROWS;
     extern __shared__ __align__(16) float part[];           // [FIRST_WAVES][16][16 C + 4]
-    __shared__ GateShared<PLANMOE_BF16, 1, CAP, true, FIRST_TOKENS, 0, ONE> sh;
+    __shared__ GateShared<PLANMOE_BF16, 1, CAP, true, TOKENS, 0, ONE> sh;
     __shared__ int32_t s_token[FIRST_ROWS];                 // the expert's rows
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int e, n0;
@@ -57,12 +57,14 @@ __global__ __launch_bounds__(FIRST_WAVES * 64) void layer_first_kernel(const Ski
     };
     if (wave < 4) {
         const bool first = blockIdx.x == 0 && blockIdx.y == 0;
-        gate_route_group<PLANMOE_BF16, PLANMOE_F32, 1, CAP, true, FIRST_TOKENS, 0, ONE>(sh, first, 0, 1, r.x, r.wg, nullptr, r.samples, p.K, p.batches, r.top_k,
+        // (16 tokens with four steps on their way, as the gate's launch has them, are more registers than these waves have: 16 x 3840 -> 256, 8 tokens, a pass
+        // of the layer 36.8 us, with two 32.8)
+        gate_route_group<PLANMOE_BF16, PLANMOE_F32, 1, CAP, true, TOKENS, 0, ONE, 2>(sh, first, 0, 1, r.x, r.wg, nullptr, r.samples, p.K, p.batches, r.top_k,
             r.normalize_gate, r.indices, r.locations, r.gates, r.stride, nullptr, nullptr, first ? r.l_aux : nullptr, r.counts, nullptr, p.M);
         if (wave == 0) {                                    // (the wave that wrote the slots)
             __builtin_amdgcn_wave_barrier();
             for (int j = 0; j < r.top_k; ++j) {
-                const int at = lane < FIRST_TOKENS ? sh.slot[j][lane] - e * p.M : -1;        // (-1 becomes negative: no slot)
+                const int at = lane < TOKENS ? sh.slot[j][lane] - e * p.M : -1;        // (-1 becomes negative: no slot)
                 if (at >= 0 && at < p.M) s_token[at] = lane;
             }
         }
@@ -122,11 +124,11 @@ __global__ __launch_bounds__(FIRST_WAVES * 64) void layer_first_kernel(const Ski
     skinny_finish<false, 1, C, FIRST_WAVES, false>(p, e, n0, rows, acc, part);
 }
 
-template <int CAP, bool DECODED, int C, int U, bool LARGE>
+template <int TOKENS, int CAP, bool DECODED, int C, int U, bool LARGE>
 static int first_launch(const SkinnyArgs &p, const FirstArgs &r, hipStream_t stream, const char *who)
 {
     constexpr int COLS = 16 * C, LDS = FIRST_WAVES * 16 * (COLS + 4) * 4;
-    const auto kernel = layer_first_kernel<CAP, DECODED, C, U, LARGE>;
+    const auto kernel = layer_first_kernel<TOKENS, CAP, DECODED, C, U, LARGE>;
     static bool ready[64];                       // (per device; setting the attribute twice does no harm)
     int dev = 0;
     PM_REQUIRE(hipGetDevice(&dev) == hipSuccess, "%s: no device", who);
@@ -180,9 +182,10 @@ extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int
     const int width = gemm_skinny_width(false, hidden, model_dim, experts);
     const bool large = skinny_large(hidden, model_dim, experts);
 // (U8: steps on their way through the codec)
-#define PM_FIRST_(C, U, U8, LARGE)                                                                                      \
-    (experts <= 8 ? (codec ? first_launch<8, true, C, U8, LARGE>(p, r, st, who) : first_launch<8, false, C, U, LARGE>(p, r, st, who))     \
-                  : (codec ? first_launch<16, true, C, U8, LARGE>(p, r, st, who) : first_launch<16, false, C, U, LARGE>(p, r, st, who)))
+#define PM_FIRST__(TOKENS, C, U, U8, LARGE)                                                                              \
+    (experts <= 8 ? (codec ? first_launch<TOKENS, 8, true, C, U8, LARGE>(p, r, st, who) : first_launch<TOKENS, 8, false, C, U, LARGE>(p, r, st, who))     \
+                  : (codec ? first_launch<TOKENS, 16, true, C, U8, LARGE>(p, r, st, who) : first_launch<TOKENS, 16, false, C, U, LARGE>(p, r, st, who)))
+#define PM_FIRST_(C, U, U8, LARGE) (samples <= 16 ? PM_FIRST__(16, C, U, U8, LARGE) : PM_FIRST__(FIRST_TOKENS, C, U, U8, LARGE))
 #define PM_FIRST(C, U) (large ? PM_FIRST_(C, U, U, true) : PM_FIRST_(C, U, U, false))
     // (32 columns through the codec, whose values take registers: of eight steps seven registers were spilled, and a load that is spilled is waited
     // for.  us, 1 token, weights in the last cache and cold, two launches, eight steps, four:
@@ -193,4 +196,5 @@ extern "C" int planmoe_layer_dispatch_product(const void *x, const void *wg, int
     return width == 32 ? PM_FIRST_(2, 8, 4, false) : width == 64 ? PM_FIRST(4, 2) : PM_FIRST(8, 1);
 #undef PM_FIRST
 #undef PM_FIRST_
+#undef PM_FIRST__
 }

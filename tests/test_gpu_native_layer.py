@@ -478,6 +478,14 @@ def test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec
     assert torch.equal(rows[used].view(bits), want["rows"].view(E * cap, M)[used].view(bits)) and bool((rows[~used] == 7.0).all())
 
 
+# (a routing group of 16 tokens, full and one short of it)
+@pytest.mark.parametrize("T,M,E,k,cap", [(15, 264, 16, 2, 4), (16, 2056, 8, 2, 4), (16, 64, 3, 3, 16)])
+@pytest.mark.parametrize("codec", [0, 1])
+@pytest.mark.parametrize("dtype,fp32_gate", [(torch.bfloat16, True), (torch.float32, True)])
+def test_layer_dispatch_of_sixteen_tokens_equals_two_launches(T, M, E, k, cap, codec, dtype, fp32_gate):
+    test_layer_dispatch_of_few_tokens_equals_two_launches(T, M, E, k, cap, codec, dtype, fp32_gate)
+
+
 # The first product of up to 32 tokens routes them itself: the bits of the dispatch and the product behind it.  Columns of a work-group 32,
 # 64 and 128, read past the caches and not; rows that are no whole steps of the reduction; capacities that drop choices, 16 rows and (two
 # launches) 20; 16 experts, 17 and 33 tokens (two launches); experts without a row
