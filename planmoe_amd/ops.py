@@ -26,8 +26,13 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    # (without the stream object of torch.cuda.current_stream: 2.1 us of every call, 0.2 so)
+    return ctypes.c_void_p(_raw_stream(t.device.index))
 
 
 def _need_gpu(t, who):
@@ -50,18 +55,26 @@ def planes(tensors, dtype):
 
     Returns (base tensor, plane stride in elements).  When the tensors already are equally
     spaced views of one allocation (as route_topk returns them) no copy is made."""
-    k = len(tensors)
-    n = tensors[0].numel()
-    ok = all(t.dtype == dtype and t.dim() == 1 and t.numel() == n and t.is_contiguous() for t in tensors)
-    if ok:
-        if k == 1:
-            return tensors[0], max(n, 1)
-        es = tensors[0].element_size()
-        d = tensors[1].data_ptr() - tensors[0].data_ptr()
-        if d >= n * es and d % es == 0 and all(
-                tensors[j].data_ptr() - tensors[0].data_ptr() == j * d for j in range(k)) and \
-                tensors[0].untyped_storage().data_ptr() == tensors[-1].untyped_storage().data_ptr():
-            return tensors[0], d // es
+    # (written out, without generators: three of these are a third of the host's time for a call)
+    first = tensors[0]
+    n = first.numel()
+    for t in tensors:
+        if t.dtype is not dtype or t.dim() != 1 or t.numel() != n or not t.is_contiguous():
+            break
+    else:
+        if len(tensors) == 1:
+            return first, max(n, 1)
+        base, es = first.data_ptr(), first.element_size()
+        d = tensors[1].data_ptr() - base
+        if d >= n * es and d % es == 0:
+            at = base + d
+            for t in tensors[2:]:
+                at += d
+                if t.data_ptr() != at:
+                    break
+            else:
+                if first.untyped_storage().data_ptr() == tensors[-1].untyped_storage().data_ptr():
+                    return first, d // es
     stacked = torch.stack([t.reshape(-1).to(dtype) for t in tensors]).contiguous()
     return stacked, max(n, 1)
 
