@@ -959,7 +959,7 @@ extern "C" const char *planmoe_expert_gemm_kernel(int form, int dtype, int activ
     if (bad()) return nullptr;
     const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
     if (dtype == PLANMOE_F32) {
-        static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
+        static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 64x64 four stages", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
         const Gemm32Kernel kernel = gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint);
         return form == 2 && kernel >= G32_SPLIT_64 && gemm_outer_serves(dtype, m, n, k, batches, hint) ? "f32 parts few rows" : names[kernel];
     }

@@ -17,6 +17,7 @@
 #include "gemm_f32_core.hpp"
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace pm {
 
@@ -33,25 +34,32 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     const int wm = wave >> 1, wn = wave & 1;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
 
-    // XCD j (work-groups j, j + 8, ...) takes the j-th eighth of the tiles: batch, panel of 8 columns, row, column
     const int tiles_m = (p.M + G32_B - 1) / G32_B, tiles_n = (p.N + G32_B - 1) / G32_B;
-    const int total = tiles_m * tiles_n * p.batches, per_xcd = (total + 7) / 8;
-    const int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per_xcd || tile >= total) return;
-    const int e = tile / (tiles_m * tiles_n);
-    int in = tile - e * tiles_m * tiles_n;
-    const int panel = in / (tiles_m * 8);
-    in -= panel * tiles_m * 8;
-    const int width = min(8, tiles_n - panel * 8);
-    const int m0 = in / width * G32_B, n0 = (panel * 8 + in % width) * G32_B;
-    int M = p.M, K = p.K;
-    if (p.live) {
-        int n = 0;
-        for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
-        n = (n + p.live_round - 1) / p.live_round * p.live_round;
-        if (TA) K = min(K, n); else M = min(M, n);
+    int e, m0, n0, M = p.M, K = p.K;
+    if constexpr (TA) {                          // (the rows in use are the reduction's)
+        const int total = tiles_m * tiles_n * p.batches, per_xcd = (total + 7) / 8;
+        const int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
+        if (blockIdx.x / 8 >= per_xcd || tile >= total) return;
+        e = tile / (tiles_m * tiles_n);
+        int in = tile - e * tiles_m * tiles_n;
+        const int panel = in / (tiles_m * 8);
+        in -= panel * tiles_m * 8;
+        const int width = min(8, tiles_n - panel * 8);
+        m0 = in / width * G32_B;
+        n0 = (panel * 8 + in % width) * G32_B;
+        if (p.live) {
+            int n = 0;
+            for (int j = 0; j < p.live_planes; ++j) n += p.live[j * p.batches + e];
+            K = min(K, (n + p.live_round - 1) / p.live_round * p.live_round);
+        }
+    } else {
+        const G32Tile tile = g32_tile(p, G32_B, STAGES == 4 && F == 1 ? 32 : 0, tiles_n, 1);
+        if (tile.e < 0) return;
+        e = tile.e;
+        m0 = tile.m * G32_B;
+        n0 = tile.n * G32_B;
+        M = tile.rows;
     }
-    if (m0 >= M) return;
 
     const int lda = TA ? p.M : p.K, ldb = TB ? p.N : p.K;
     const uint8_t *A = reinterpret_cast<const uint8_t *>(p.A + (int64_t)e * p.M * p.K + (TA ? (int64_t)m0 : (int64_t)m0 * lda));
@@ -134,6 +142,101 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const Gemm32Args p)
     };
 #pragma unroll
     for (int kt = 0; kt < STAGES - 1; ++kt) load_tile(kt);
+    // A tile of up to 32 rows, the last one of an expert as a rule: its waves take 16 columns each of all its rows, half (up to 16 rows a quarter) of the
+    // time on the matrix cores that a wave with 32 rows of zeros beside the others takes.  A compute unit that has such a tile beside a whole one is what the
+    // launch waits for.  16 x 16 x 4 with lane group g at k = 4 g + q: the sums have the same order.
+    // us, 4 experts of 260, 250, 270 and 244 rows, 512 -> 1024, a pass of the product 21.9, so 17.3; b^T 21.3 and 16.2
+    if constexpr (STAGES == 4 && F == 1 && !TA) {
+        if (M - m0 <= 32) {
+            const int l16 = lane & 15, g = lane >> 4, col = 16 * wave + l16;
+            auto rows = [&](auto halves) {
+                constexpr int H = decltype(halves)::value;        // 16 rows each
+                f32x4 sum[H], a[2][H], b[2];
+#pragma unroll
+                for (int h = 0; h < H; ++h) sum[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                auto read = [&](int stage, int s, int to) {
+                    const uint8_t *at = lds + stage * G32_OPERAND, *bt = lds + (STAGES + stage) * G32_OPERAND;
+#pragma unroll
+                    for (int h = 0; h < H; ++h)
+                        a[to][h] = *reinterpret_cast<const f32x4 *>(at + (16 * h + l16) * 128 + (((4 * s + g) ^ ((l16 >> 1) & 7)) * 16));
+                    if (TB) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) b[to][q] = *reinterpret_cast<const float *>(bt + (16 * s + 4 * g + q) * 256 + col * 4);
+                    } else {
+                        b[to] = *reinterpret_cast<const f32x4 *>(bt + col * 128 + (((4 * s + g) ^ ((l16 >> 1) & 7)) * 16));
+                    }
+                };
+                auto products = [&](int from) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int h = 0; h < H; ++h) sum[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[from][q], a[from][h][q], sum[h], 0, 0, 0);
+                };
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((STAGES - 2) * 4 * F) : "memory");
+                read(0, 0, 0);
+                for (int k0 = 0; k0 < KT; k0 += STAGES) {
+#pragma unroll
+                    for (int stage = 0; stage < STAGES; ++stage) {
+                        const int kt = k0 + stage;
+                        if (kt >= KT) break;
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((STAGES - 3) * 4 * F) : "memory");
+                        __builtin_amdgcn_sched_barrier(0);
+                        read(stage, 1, 1);
+#pragma unroll
+                        for (int n = 0; n < 4 * F; ++n) load(kt + STAGES - 1, (stage + STAGES - 1) % STAGES, n);
+                        __builtin_amdgcn_sched_barrier(0);
+                        products(0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        read((stage + 1) % STAGES, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        products(1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                // a lane has columns 4 g .. + 3 of the wave's 16 of row l16
+                const int n = n0 + 16 * wave + 4 * g;
+                const bool in_n = n < p.N;                   // (N is a multiple of 4: a lane's columns are in or out together)
+                float add[4], sums[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int x = 0; x < 4; ++x) add[x] = p.bias && in_n ? p.bias[(int64_t)e * p.N + n + x] : 0.f;
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const int row = m0 + 16 * h + l16;
+                    const int64_t to = ((int64_t)e * p.M + row) * p.N + n;
+                    const bool inside = in_n && row < M;
+                    f32x4 v = sum[h], keep = {0.f, 0.f, 0.f, 0.f};
+                    float part[4];
+                    if (p.mask && inside) keep = *reinterpret_cast<const f32x4 *>(p.mask + to);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        if (p.bias) v[x] += add[x];
+                        if (p.relu) v[x] = v[x] < 0.f ? 0.f : v[x];
+                        if (p.mask) v[x] = keep[x] > 0.f ? v[x] : 0.f;
+                        part[x] = inside ? v[x] : 0.f;
+                    }
+                    if (inside) *reinterpret_cast<f32x4 *>(p.C + to) = v;
+                    if (p.colsum) {                          // (16 rows and 16 rows, as g32_store adds up the 32 of a wave)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+#pragma unroll
+                            for (int d = 1; d < 16; d <<= 1) part[x] += __shfl_xor(part[x], d);
+                            sums[x] += part[x];
+                        }
+                    }
+                }
+                if (p.colsum && l16 == 0 && in_n) {          // (two slots a tile; the second 32 rows are none)
+                    float *to = p.colsum + ((int64_t)e * tiles_m * 2 + m0 / G32_B * 2) * p.N + n;
+                    *reinterpret_cast<f32x4 *>(to) = f32x4{sums[0], sums[1], sums[2], sums[3]};
+                    *reinterpret_cast<f32x4 *>(to + p.N) = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            };
+            if (M - m0 <= 16) rows(std::integral_constant<int, 1>{});
+            else rows(std::integral_constant<int, 2>{});
+            // nothing may still be on its way into LDS that another work-group gets
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            return;
+        }
+    }
     if constexpr (STAGES == 4) {
         // behind the barrier of k-tile kt everybody's share of kt + 1 is in as well, and everybody is done with kt - 1; what else there is to do
         // goes between the products, one thing at a time (ahead of them it left the matrix core idle for a third of a k-tile)
@@ -334,6 +437,15 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
     }
 }
 
+// weights that the last cache does not hold
+static bool gemm_f32_past_caches(const Gemm32Args &p) { return (int64_t)p.batches * p.N * p.K * 4 > (int64_t)256 << 20; }
+// pieces of 32 rows (16 where waves of 16 serve all of a batch's) by `columns` that the rows expected make
+static int64_t gemm_f32_pieces(const Gemm32Args &p, int rows_hint, int columns)
+{
+    const int rows = p.M <= 16 && !p.colsum ? 16 : 32;
+    return (int64_t)((rows_hint + rows - 1) / rows) * ((p.N + columns - 1) / columns) * p.batches;
+}
+
 // how many pieces of `rows` by `columns` the products have at most
 static int64_t gemm_f32_wave_pieces(const Gemm32Args &p, int rows, int columns)
 {
@@ -349,36 +461,20 @@ static int gemm_f32_wave_launch(const Gemm32Args &p, int waves, hipStream_t stre
     return 0;
 }
 
-// waves of 32 rows (16 where no batch has more) by 16 columns that the rows expected make
-static int64_t gemm_f32_strips(const Gemm32Args &p, int rows_hint)
-{
-    const int rows = p.M <= 16 && !p.colsum ? 16 : 32;
-    return (int64_t)((rows_hint + rows - 1) / rows) * ((p.N + 15) / 16) * p.batches;
-}
-
-// Columns and waves of a work-group.  Where there are waves enough of 32 columns for the SIMDs a wave reads whole lines; fewer than that and 16 columns put
-// more waves to work, each on a compute unit of its own (four to a work-group where there are several a compute unit anyway: they share lines); weights that the
-// last cache (256 MB) does not hold go past the caches, with few rows 64 columns of them.  b^T: a wave reads 64 bytes of every row whatever its columns.
-// us before (16 columns, four waves, twice the steps in nn) and now, weights cold, in the last cache:
-//   nn, up to 16 rows   8 x 1024 -> 4096    33, 28 and 27, 22       8 x 2600 -> 3440    80, 72 and 58, 52      16 x 3328 -> 3072  149 and 95 (cold)
-//                       4 x 1024 -> 1024    14, 14 and 12, 12       16 x 1896 -> 688    26, 24 and 24, 21      8 x 4096 -> 1024   51, 39 and 49, 37
-//                       16 x 512 -> 2048    20, 19 and 15, 14       (16 columns in single waves: 8 x 4096 -> 1024 47, 44)
-//   nn, up to 32        16 x 1472 -> 2176   82, 66 and 68, 60       8 x 2816 -> 1728    49, 46 and 43, 41
-//                       8 x 1024 -> 4096    44, 38 (tiles) and 34, 28
-//   nt                  4 x 1024 -> 1024    16, 16 and 9, 9         8 x 4096 -> 1024    41, 40 and 30, 29      16 x 3072 -> 3328  147 and 132
+// Columns and waves of a work-group.  A wave reads whole lines with 32 columns, where there are such waves enough; 16 columns of short reductions;
+// weights that the last cache (256 MB) does not hold go past the caches, 64 columns a wave.  b^T: a wave reads 64 bytes of every row whatever its columns.
+// us with 16 columns and four waves a work-group everywhere, and now, weights cold, in the last cache:
+//   8 x 1 row, 1024 -> 4096   33, 28 and 27, 22       8 x 7, 2600 -> 3440    80, 72 and 58, 52       16 x 512 -> 2048   20, 19 and 15, 14
+//   8 x 20, 1024 -> 4096      44, 38 and 34, 28       16 x 1, 3328 -> 3072  149 and 95 (cold)
 static int gemm_f32_waves(int form, const Gemm32Args &p, int rows_hint, hipStream_t stream, const char *who)
 {
-    const int64_t strips = gemm_f32_strips(p, rows_hint), cu = compute_units();
-    const bool past = (int64_t)p.batches * p.N * p.K * 4 > (int64_t)256 << 20;
-    if (p.M <= 16 && !p.colsum) {
-        if (form == 1) return strips <= 2 * cu ? gemm_f32_wave_launch<1, 1, 8, false>(p, 1, stream, who) : gemm_f32_wave_launch<1, 1, 4, false>(p, 1, stream, who);
-        if (strips < 4 * cu) return gemm_f32_wave_launch<1, 1, 8, true>(p, strips < 2 * cu ? 1 : 4, stream, who);
-        if (past && strips >= 8 * cu) return gemm_f32_wave_launch<1, 4, 2, true, true>(p, 1, stream, who);
-        return gemm_f32_wave_launch<1, 2, 4, true>(p, strips < 5 * cu ? 1 : 4, stream, who);
-    }
-    if (form == 1) return strips < 4 * cu ? gemm_f32_wave_launch<2, 1, 4, false>(p, 1, stream, who) : gemm_f32_wave_launch<2, 2, 2, false>(p, 1, stream, who);
-    if (strips < 4 * cu) return gemm_f32_wave_launch<2, 1, 4, true>(p, strips <= 2 * cu ? 1 : 4, stream, who);
-    return past ? gemm_f32_wave_launch<2, 2, 4, true, true>(p, 1, stream, who) : gemm_f32_wave_launch<2, 2, 4, true>(p, 1, stream, who);
+    const int64_t strips = gemm_f32_pieces(p, rows_hint, 16), cu = compute_units();
+    const bool one = p.M <= 16 && !p.colsum;
+    if (form == 1) return one ? gemm_f32_wave_launch<1, 1, 4, false>(p, 1, stream, who) : gemm_f32_wave_launch<2, 1, 4, false>(p, 1, stream, who);
+    if (strips < 4 * cu) return one ? gemm_f32_wave_launch<1, 1, 8, true>(p, 1, stream, who) : gemm_f32_wave_launch<2, 1, 4, true>(p, 1, stream, who);
+    if (!one) return gemm_f32_wave_launch<2, 2, 4, true>(p, 1, stream, who);
+    if (gemm_f32_past_caches(p) && strips >= 8 * cu) return gemm_f32_wave_launch<1, 4, 2, true, true>(p, 1, stream, who);
+    return gemm_f32_wave_launch<1, 2, 4, true>(p, strips < 5 * cu ? 1 : 4, stream, who);
 }
 
 template <int F, bool TA, bool TB, int STAGES = 2>
@@ -396,7 +492,7 @@ static int gemm_f32_launch(const Gemm32Args &p, hipStream_t stream, const char *
     }
     const int64_t tiles = ((int64_t)p.M + SIDE - 1) / SIDE * (((int64_t)p.N + SIDE - 1) / SIDE) * p.batches;
     PM_REQUIRE(tiles < ((int64_t)1 << 30), "%s: too many tiles", who);
-    kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, LDS, stream>>>(p);
+    kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8 + (TA ? 0 : 8))), 256, LDS, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
@@ -413,17 +509,20 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 // The tile's side under a relu: a compute unit takes 1.9 us for a k-tile of 128 x 128 and 4 for the tile, 0.52 and
 // 1.2 for 64 x 64, 0.47 with four stages; what counts is the fullest compute unit (us, 64 x 64, with four stages, 128 x 128: 4 x 1000 rows,
 // 2048 -> 512 77, 66, 137; 16 x 512, 1024 -> 1024 142, 131, 131; 512 -> 2048 152, 144, 138; 2 x 4096, 4096 -> 4096 2129, 1944, 1969).
-// Waves on their own, up to 32 rows, where they read the weight once (us in tiles of four stages and in waves, cold, nn, 8 experts x 20 rows, 1024 -> 4096
-// 48 and 34, 32 rows 1024 -> 1024 21 and 20, 21 rows 1896 -> 568 34 and 28, b^T 35 and 22), and beyond where all the strips of 32 rows by 16 columns
-// are few (4 x 64, 2048 -> 512 36 and 29).
-// The rows are those expected: with skewed routing an
-// expert has more, and its weight is read once for every 32 of them, but all experts together have as many rows as before,
-// so never more than one weight an expert on top, and the tiles get slower with skew as well.  us in waves of 16 columns and in tiles of two stages, nn, nt:
-//   8 experts, 256 rows, 4096 -> 1024    even 69, 86 and 90, 89;     128 of the rows on one 70, 88 and 91, 90
-//   8 experts, 128 rows, 1024 -> 4096    even 31, 32 and 43, 42;     64 on one 44, 52 and 42, 42
-//   16 experts, 256 rows, 4096 -> 1024   even 55, 60 and 93, 97;     128 on one 123, 140 and 152, 155
-//   64 experts, 2048 rows, 1024 -> 4096  even 388, 361 and 305, 303; by Zipf's law (1.2) 531, 525 and 918, 912
-//
+// Up to 32 rows tiles of 32 x 32 (gemm_f32_slim.hip; five k-tiles in LDS, eight where that leaves work-groups room), or waves on their own: with fewer than
+// eight k-tiles, where there is a wave of 32 columns for each SIMD and hardly a tile more than four for a compute unit to take in turn, and for weights past the
+// caches.  us, weights cold, in the last cache, waves and tiles of 32 x 32:
+//   nn  8 x 21 rows, 1896 -> 568  28, 28 and 16, 14      4 x 21, 2808 -> 1040  39, 39 and 19, 18      8 x 2, 4096 -> 1024    49, 37 and 27, 24
+//       8 x 1, 1024 -> 4096       27, 23 and 34, 29      8 x 7, 3440 -> 2600   76, 66 and 65, 55      16 x 7, 1536 -> 2304   59, 51 and 51, 45
+//       16 x 16, 1472 -> 2176     68, 60 and 49, 39      8 x 20, 1024 -> 4096  34, 27 and 38, 30      16 x 1, 2048 -> 2560   55, 55 and 70, 66
+//   nt  8 x 21, 1896 -> 568       22, 22 and 14, 14      8 x 9, 2048 -> 2048   31, 27 and 31, 22      8 x 1, 1024 -> 4096    28, 23 and 32, 24
+//       16 x 1, 3072 -> 3328      131 and 121            8 x 20, 1024 -> 4096  36, 29 and 33, 23
+//   skewed, 8 experts, 128 of 256 rows on one, 4096 -> 1024 nn 67, 58 and 49, 40 (64 x 64 123)
+// Beyond, a compute unit takes 0.26 us for a k-tile of up to two tiles of 32 x 32, whose chains of products hide behind each other, 0.145 for each of more, and
+// 0.475 for one of 64 x 64, a third more where it has a small one beside it.
+//   nn  4 x 260 rows, 512 -> 1024  17, 17 and 19, 19      1024 -> 512          22, 21 and 19, 18      8 x 163, 2048 -> 256  36, 36 and 23, 23
+//       8 x 66, 1024 -> 1024       22, 22 and 21, 19      4 x 48, 3648 -> 1088 60, 59 and 34, 34      8 x 100, 1024 -> 1024 23, 22 and 25, 22
+//       16 x 45, 1024 -> 256       20, 20 and 9, 9        4 x 48, 1088 -> 3648 23, 23 and 26, 23      16 x 97, 1536 -> 512  31, 30 and 34, 30
 // On the bf16 matrix cores, in three parts a value (gemm_f32_split.hip), where there is more than one tile of 64 x 64 for a compute
 // unit; one tile on its own is bound by issuing the splits (8 experts, 128 rows, 1024 -> 1024: 20 us in fp32, 28 in parts) and stays here.
 // A launch takes its rounds; us for a k-tile with few and with all compute units at work, and once for a tile, fitted to 60 shapes
@@ -484,17 +583,38 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
         return c.t64 <= c.in_parts() ? G32_SPLIT_64 : c.t128 <= c.t256 ? G32_SPLIT_128 : G32_SPLIT_256;
     }
     const bool deep = gemm_f32_deep(form, p, rows_hint);
-    // (few strips: a SIMD has one wave whichever it is, and one that reads for itself takes 12.6 ns for a k (b^T 9.5), a tile 15.2)
-    const bool few = rows_hint <= 32 || (p.K >= 512 && gemm_f32_strips(p, rows_hint) <= (form == 0 ? 5 : 8) * (int64_t)compute_units() / 4);
-    if (form != 2 && few && (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) &&
-        gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30))
-        return G32_WAVES;
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
     const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
+    if (form != 2 && rows_hint <= 32) {
+        const int64_t pieces = gemm_f32_pieces(p, rows_hint, 32);
+        const bool one = p.M <= 16 && !p.colsum, past = gemm_f32_past_caches(p);
+        const bool lines = pieces > 3 * cu && pieces <= 4 * cu && (one || (form == 0 && !past));
+        const bool fits = (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30);
+        if (fits && (!deep || lines || (form == 0 && one && past && pieces >= 4 * cu))) return G32_WAVES;
+        if (deep) return 2 * pieces <= 3 * cu ? G32_SLIM_ALONE : G32_SLIM;
+    }
     auto cost = [&](int64_t side, double us, double once) {
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
         return (double)((tiles + cu - 1) / cu) * (us * kt + once);
     };
+    if (deep && form != 2) {
+        // (row counts from the device: an expectation, and of many batches with a standard deviation of its root)
+        double whole = 0, small = 0, slim = 0;
+        for (const double q : {-1.5, -0.5, 0.5, 1.5}) {
+            const int64_t r = p.live ? std::min<int64_t>(p.M, std::max<int64_t>(1, (int64_t)(m + q * std::sqrt((double)m)))) : m, rest = r % 64;
+            whole += 0.25 * (double)(r / 64 + (rest > 32));
+            small += 0.25 * (rest > 0 && rest <= 32);
+            slim += 0.25 * (double)((r + 31) / 32);
+        }
+        const double columns = (double)((p.N + 63) / 64 * p.batches);
+        whole *= columns;
+        small *= columns;
+        slim *= (double)((p.N + 31) / 32 * p.batches) / cu;
+        const double units = whole <= cu ? whole + small > cu ? 1.35 : 1. : std::ceil(whole / cu);
+        const double weight = slim > 2 ? 1e-7 * (double)p.batches * p.N * p.K * 4 : 0.;          // (0.1 us for every MB: its lines are asked for by more of them)
+        const double us = std::max(0.262, 0.145 * std::ceil(slim)) * kt + 2.5 + weight;
+        if (1.03 * us < 0.475 * kt * units + 6 && us < cost(128, 1.9, 4)) return slim <= 1.5 ? G32_SLIM_ALONE : G32_SLIM;
+    }
     return cost(64, deep ? 0.47 : 0.52, 1.2) < cost(128, 1.9, 4) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
 }
 
@@ -511,6 +631,8 @@ int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, int rows_hi
         if (form == 0) return gemm_f32_launch<1, false, true, 4>(p, stream, who);
         if (form == 1) return gemm_f32_launch<1, false, false, 4>(p, stream, who);
         return gemm_f32_launch<1, true, true, 4>(p, stream, who);
+    case G32_SLIM: return gemm_f32_slim_run(form, false, p, stream, who);
+    case G32_SLIM_ALONE: return gemm_f32_slim_run(form, true, p, stream, who);
     case G32_TILE_128:
         if (form == 0) return gemm_f32_launch<2, false, true>(p, stream, who);
         if (form == 1) return gemm_f32_launch<2, false, false>(p, stream, who);

@@ -13,13 +13,14 @@ struct Gemm32Args {
     int relu;
 };
 
-// Kernels: waves on their own; tiles of 64 x 64 (two and four k-tiles in LDS) and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128
+// Kernels: waves on their own; tiles of 64 x 64 (two and four k-tiles in LDS), 32 x 32 (five, and eight), and 128 x 128 on the fp32 matrix cores; tiles of 64 x 64, 128 x 128 and 256 x 128
 // on the bf16 matrix cores, the operands in three parts
-enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_DEEP_64, G32_TILE_128, G32_SPLIT_64, G32_SPLIT_128, G32_SPLIT_256 };
+enum Gemm32Kernel { G32_WAVES, G32_TILE_64, G32_DEEP_64, G32_SLIM, G32_SLIM_ALONE, G32_TILE_128, G32_SPLIT_64, G32_SPLIT_128, G32_SPLIT_256 };
 
 // form: 0 nn, 1 nt, 2 tn; the caller has checked shape and alignment.  rows_hint: rows in use
 Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint);
 int gemm_f32_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, int rows_hint, hipStream_t stream, const char *who);
+int gemm_f32_slim_run(int form, bool alone, const Gemm32Args &p, hipStream_t stream, const char *who);        // nn, nt
 int gemm_f32_split_run(int form, const Gemm32Args &p, Gemm32Kernel kernel, hipStream_t stream, const char *who);
 // column sums have two slots for so many rows
 inline int gemm_f32_slot_rows(Gemm32Kernel kernel) { return kernel == G32_TILE_128 || kernel == G32_SPLIT_128 || kernel == G32_SPLIT_256 ? 128 : 64; }

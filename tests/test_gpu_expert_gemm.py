@@ -771,18 +771,18 @@ def test_sums_of_shares_are_added_in_pairs(shares):
     assert bool(((out.double() - want).abs() <= 2.0 ** -23).all()), (out[0, 0].item() - 1.0) * 2 ** 24
 
 
-# fp32, few rows: 16 and 32 rows of a wave, 16, 32 and 64 columns, work-groups of one and four waves, past the caches; columns and reductions that
+# fp32, waves on their own: 16 and 32 rows, 16, 32 and 64 columns, work-groups of one and four waves, past the caches; columns and reductions that
 # nothing divides.  The same rows in a larger buffer go through the tiles, and the sums have the same order.
 @pytest.mark.parametrize("form,B,cap,n,k", [
-    ("nn", 4, 12, 52, 300), ("nn", 16, 16, 520, 36), ("nn", 16, 8, 1036, 148), ("nn", 16, 9, 1300, 20), ("nn", 16, 4, 2100, 2080),
-    ("nn", 4, 40, 52, 300), ("nn", 16, 33, 516, 44), ("nn", 16, 20, 1036, 212), ("nn", 16, 24, 1100, 3900), ("nn", 2, 70, 148, 724),
+    ("nn", 4, 12, 52, 200), ("nn", 16, 16, 520, 36), ("nn", 16, 8, 1036, 148), ("nn", 16, 9, 1300, 20), ("nn", 16, 4, 2100, 2080),
+    ("nn", 4, 40, 52, 200), ("nn", 16, 33, 1060, 44), ("nn", 16, 20, 1700, 300),
     ("nt", 4, 12, 52, 200), ("nt", 16, 16, 1036, 148), ("nt", 4, 40, 68, 200), ("nt", 16, 33, 1060, 44)])
 def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
     from planmoe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(n + k)
     rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
-    hint, more = min(cap, 30), 100 if cap <= 64 else 600
-    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=True, rows_hint=cap if cap > 64 else hint) == "f32 waves"
+    hint, more = min(cap, 30), 100
+    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=True, rows_hint=hint) == "f32 waves"
     edges = [cap, 0, 1, hint, 16, 17, 31, 33, 15, 32, 2, 5]
     rows = [min(cap, edges[e % 12]) for e in range(B)]
     live = torch.tensor([rows], dtype=torch.int32, device=DEV)
@@ -792,7 +792,7 @@ def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
         few[e, r:] = float("nan")
     sentinel = lambda rows: torch.full((B, rows, n), 7.0, device=DEV)
     kw = dict(live=live, relu=form == "nn")
-    got = ops.expert_gemm(form, few, w, bias, out=sentinel(cap), rows_hint=cap if cap > 64 else hint, **kw)
+    got = ops.expert_gemm(form, few, w, bias, out=sentinel(cap), rows_hint=hint, **kw)
     want = ops.expert_gemm(form, wide, w, bias, out=sentinel(more), rows_hint=more, **kw)
     torch.cuda.synchronize()
     assert torch.equal(got, want[:, :cap])
@@ -802,10 +802,53 @@ def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
         want, _ = ops.expert_gemm_relu_bwd(wide, w, h, live=live, out=sentinel(more), rows_hint=more)
         torch.cuda.synchronize()
         assert torch.equal(got, want[:, :cap])
-        for e, r in enumerate(rows):
-            ref = got[e, :r].double().sum(0)
-            # (at most cap additions, each rounded to 2^-24 of the sum so far)
-            assert bool(((db[e].double() - ref).abs() <= cap * 2.0 ** -24 * got[e, :r].double().abs().sum(0)).all())
+        _column_sums_hold(db, got, rows, cap)
+
+
+def _column_sums_hold(db, got, rows, cap):
+    for e, r in enumerate(rows):
+        ref = got[e, :r].double().sum(0)
+        # (at most cap additions, each rounded to 2^-24 of the sum so far)
+        assert bool(((db[e].double() - ref).abs() <= cap * 2.0 ** -24 * got[e, :r].double().abs().sum(0)).all())
+
+
+# fp32 tiles of 32 x 32, five and eight k-tiles in LDS, and of 64 x 64 with small ones of 16 and 32 rows behind them (the last shape); columns, reductions
+# and row counts around their sides, with and without counts.  Each 32 rows go through the waves as well, among more columns, and the bits are theirs.
+@pytest.mark.parametrize("counted", [True, False])
+@pytest.mark.parametrize("form,B,cap,n,k,hint", [
+    ("nn", 4, 12, 52, 300, 9), ("nn", 16, 20, 1036, 292, 20), ("nn", 2, 70, 148, 724, 70), ("nn", 8, 163, 260, 2044, 163), ("nn", 1, 33, 4, 228, 33),
+    ("nt", 4, 40, 68, 236, 30), ("nt", 16, 33, 1060, 236, 30), ("nt", 3, 97, 100, 240, 97), ("nn", 16, 108, 512, 1536, 97), ("nt", 16, 108, 1028, 252, 97)])
+def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(form, B, cap, n, k, hint, counted):
+    from planmoe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=counted, rows_hint=hint) == "f32 64x64 four stages"
+    edges = [cap, 0, 1, 65, 80, 81, 96, 97, 15, 16, 17, 31, 32, 33, 63, 64]
+    rows = [min(cap, edges[e % 16]) if counted else cap for e in range(B)]
+    live = torch.tensor([rows], dtype=torch.int32, device=DEV) if counted else None
+    a, w, bias, h = rand(B, cap, k), rand(B, k, n), rand(B, n), rand(B, cap, n)
+    if not counted and form == "nt":
+        a[0, 0, k - 1], w[0, k - 1, 1] = float("inf"), float("nan")
+    columns = -(-25600 // B // 4) * 4
+    many = w.repeat(1, 1, -(-columns // n))[:, :, :columns].contiguous()
+    assert columns >= n and ops.expert_gemm_kernel("nn", torch.float32, B, 32, columns, k) == "f32 waves"
+    want = torch.cat([ops.expert_gemm("nn", a[:, i:i + 32].contiguous(), many)[:, :, :n] for i in range(0, cap, 32)], 1)
+    for e, r in enumerate(rows):
+        a[e, r:] = float("nan")
+    b = w if form == "nn" else w.transpose(1, 2).contiguous()
+    sentinel = torch.full((B, cap, n), 7.0, device=DEV)
+    got = ops.expert_gemm(form, a, b, bias, relu=form == "nn", live=live, rows_hint=hint, out=sentinel.clone())
+    ref = want + bias[:, None]
+    if form == "nn":
+        ref = torch.where(ref < 0, torch.zeros_like(ref), ref)
+    there = (torch.arange(cap, device=DEV)[None, :] < torch.tensor(rows, device=DEV)[:, None])[:, :, None]
+    same = lambda x, y: torch.equal(torch.where(there, y, sentinel).nan_to_num(123.0), x.nan_to_num(123.0))
+    assert same(got, ref)
+    if form == "nt":
+        got, db = ops.expert_gemm_relu_bwd(a, b, h, live=live, rows_hint=hint, out=sentinel.clone())
+        assert same(got, torch.where(h > 0, want, torch.zeros_like(want)))
+        if counted:
+            _column_sums_hold(db, got, rows, cap)
 
 
 # Weight gradients over few rows, stored past the caches and plainly, 64, 128 and 256 columns of a wave; sizes that nothing divides.  The same rows in a
