@@ -328,6 +328,11 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_wave_kernel(const Gemm32Args 
     }
     const int m0 = piece % blocks * 16 * MF, n0 = (piece / blocks * waves + wave) * 16 * C;
     if (M == 0 || n0 >= p.N) return;
+    if (m0 >= M) {                               // (a second slot without rows)
+        if (lane < 4 * C && n0 + 4 * lane < p.N)
+            *reinterpret_cast<f32x4 *>(p.colsum + ((int64_t)e * ((p.M + 63) / 64 * 2) + m0 / 32) * p.N + n0 + 4 * lane) = f32x4{0.f, 0.f, 0.f, 0.f};
+        return;
+    }
     const float *A = p.A + (int64_t)e * p.M * p.K, *B = p.B + (int64_t)e * p.N * p.K;
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, M * p.K * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, p.N * p.K * 4, 0x00020000);
