@@ -278,6 +278,106 @@ __global__ __launch_bounds__(256) void layer_dx_kernel(
     }
 }
 
+// The same for few tokens, bound by trips to memory one after the other: the waves of a work-group share a token's row, PER vectors a lane each, and what
+// does not depend on the slots, the weights above all, is asked for before them (layer_dx_kernel asks for EP vectors, then the next EP, behind the
+// rows).  With the codec every wave reads the whole row, whose minimum and scale it needs.  The same operations in the same order.  us, layer_dx_kernel
+// and this one, two choices of 8 experts, 5, 300, 1500 and 3000 tokens:
+//   fp32        x 920  9.0, 3.2   11.7, 4.2   14.6, 7.1    16.7, 10.3      x 2048  16.2, 3.6   21.4, 5.2   27.0, 11.3   29.1, 17.3
+//   fp32, int8  x 768  10.4, 5.0  12.6, 6.1   15.0, 12.1   16.8, 19.1      bf16, int8  x 4096  12.4, 6.2  13.5, 9.1  19.5, 21.9  31.0, 39.8
+template <int DT, int CACHE, bool INT8, int EP>
+__global__ __launch_bounds__(256) void layer_dx_few_kernel(
+    const void *__restrict__ rows, const int32_t *__restrict__ indices, const int32_t *__restrict__ locations, int64_t stride, int top_k,
+    int samples, int model_dim, int capacity, const float *__restrict__ g, const void *__restrict__ wg, int experts, void *__restrict__ out)
+{
+    using E = Elem<DT>;
+    constexpr int V = E::VEC, PER = CACHE > 4 ? CACHE / 4 : 1, ACROSS = CACHE / PER;       // vectors of a wave, waves of a token
+    __shared__ __align__(16) float s_table[INT8 ? 4 : 1][256];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), units = model_dim / V;
+    const int t = blockIdx.x * (4 / ACROSS) + wave / ACROSS, c0 = wave % ACROSS * PER;
+    if (t >= samples) return;                    // (no work-group barrier below)
+    float *const table = s_table[INT8 ? wave : 0];
+    auto unit = [&](int c) { return min((c0 + c) * WAVE + lane, units - 1); };
+    uint4 weight[EP][PER];
+    float ge[EP];
+#pragma unroll
+    for (int e = 0; e < EP; ++e) {
+        ge[e] = g[(int64_t)t * experts + min(e, experts - 1)];
+#pragma unroll
+        for (int c = 0; c < PER; ++c) weight[e][c] = reinterpret_cast<const uint4 *>(wg)[(int64_t)min(e, experts - 1) * units + unit(c)];
+    }
+    float acc[PER][V];
+    for (int j0 = 0; j0 < top_k; j0 += WAVE) {
+        const int np = min(top_k - j0, WAVE);
+        int slot; float gate;
+        fetch_planes(nullptr, indices, locations, stride, t, j0, np, 0x7fffffff, capacity, slot, gate);
+        // the next choice's row is on its way while this one's is worked on (a dropped choice reads slot 0, unused)
+        uint4 next[PER], all[INT8 ? CACHE : 1];       // (a wave that has the whole row has it once)
+        auto request = [&](int j) {
+            const uint4 *src = reinterpret_cast<const uint4 *>(rows) + (int64_t)max(rl_i(slot, j), 0) * units;
+            if constexpr (!INT8 || ACROSS > 1)
+#pragma unroll
+                for (int c = 0; c < PER; ++c) next[c] = src[unit(c)];
+            if constexpr (INT8)
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) all[c] = src[min(c * WAVE + lane, units - 1)];
+        };
+        request(0);
+        for (int j = 0; j < np; ++j) {
+            const int s = rl_i(slot, j);
+            uint4 row[PER], whole[INT8 ? CACHE : 1];
+#pragma unroll
+            for (int c = 0; c < PER; ++c) row[c] = INT8 && ACROSS == 1 ? all[c] : next[c];
+            if constexpr (INT8)
+#pragma unroll
+                for (int c = 0; c < CACHE; ++c) whole[c] = all[c];
+            if (j + 1 < np) request(j + 1);
+            auto add = [&](int c, const float (&f)[V]) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const float v = s >= 0 ? f[i] : 0.f;
+                    acc[c][i] = j0 + j == 0 ? v : acc[c][i] + v;
+                }
+            };
+            if constexpr (INT8) {
+                const RowTable<DT> tab(whole, 1.f, table);
+                table_sync();
+                auto body = [&](auto mode) {
+#pragma unroll
+                    for (int c = 0; c < PER; ++c) {
+                        float f[V];
+                        tab.template values<decltype(mode)::value>(row[c], f);
+                        add(c, f);
+                    }
+                };
+                if (tab.enc.fast()) body(std::true_type{}); else body(std::false_type{});
+                table_sync();                    // (the next choice's table takes this one's place)
+            } else {
+#pragma unroll
+                for (int c = 0; c < PER; ++c) {
+                    float f[V];
+                    E::unpack(row[c], f);
+                    add(c, f);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[c][i] = E::round(acc[c][i]);
+#pragma unroll
+        for (int e = 0; e < EP; ++e) {
+            const float scale = E::round(ge[e]);
+            float w[V];
+            E::unpack(weight[e][c], w);
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[c][i] = e < experts ? fmaf(scale, w[i], acc[c][i]) : acc[c][i];
+        }
+        const int u = (c0 + c) * WAVE + lane;
+        if (u < units) stream_store(reinterpret_cast<uint4 *>(out) + (int64_t)t * units + u, E::pack(acc[c]));
+    }
+}
+
 // how many shares a reduction over `rows` is cut into for `blocks` column blocks: enough work-groups for the GPU, at least 32 rows each
 int reduction_shares(int64_t rows, int64_t blocks)
 {
@@ -425,19 +525,31 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
     PM_REQUIRE(grad_logits && wg && out && aligned16(wg) && aligned16(out), "%s: NULL or unaligned argument", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
     PM_REQUIRE(experts <= 8 || per_lane <= 8, "%s: more than 8 experts: rows of up to 8 KB", who);
-    if (per_lane > 8) {
+    // Few tokens (layer_dx_few_kernel) up to where the trips are hidden by other waves: 4200 tokens without the codec 13.1 and 12.7 us (fp32 x 920, 8 experts),
+    // 14.5 and 13.3 (bf16 x 1024, 16), 8000 tokens 19.1 and 21.6, 20.6 and 20.4; with it 700 tokens 8.7 and 7.9 (bf16 x 1888), 12.9 and 7.2 (fp32 x 768),
+    // 1500 tokens 11.4 and 12.2, 15.0 and 12.1.  16 experts' weights in fp32 are read once for two tokens beyond (x 1024, 1500 tokens 10.9 and 9.4, 4000 15.2 and 18.4); rows
+    // of more than 8 KB, four times through the codec, one compute unit each (fp32 x 4096, the two launches and this one, 100 tokens 21.6 and 12.0, 700 25.7 and 34.2).
+    const bool few = samples <= (codec ? per_lane > 8 ? 1 : 3 : dtype == PLANMOE_F32 && experts > 8 ? 8 : 16) * compute_units();
+    if (per_lane > 8 && !few) {
         if (planmoe_layer_combine(rows, dtype, codec, nullptr, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, out, stream)) return 1;
         return planmoe_gate_dx_accumulate(out, dtype, grad_logits, wg, samples, model_dim, experts, stream);
     }
     hipStream_t st = (hipStream_t)stream;
     // Two tokens a wave read the weights once where they are as wide as the cache they come from and there are waves enough
     // (fp32, 8 experts x 1024 x 16384 tokens, no codec: 69 us with one, 34 with two; x 1024 tokens: 7.3 and 6.0, int8 10.1 and 11.4; bf16, whose rows
-    // take twice the registers unpacked: 43 and 39, int8 59 and 61).  16 experts' weights at any number of tokens (fp32, 64 x 1024: 12.6 and 8.4).
+    // take twice the registers unpacked: 43 and 39, int8 59 and 61).  16 experts' weights at any number of tokens that is not few.
     const bool pairs = dtype == PLANMOE_F32 && (samples >= 4096 || experts > 8);
 #define PM_DX__(CACHE, INT8, EP, TOKENS) (layer_dx_kernel<DT, CACHE, INT8, EP, TOKENS><<<(samples + 4 * TOKENS - 1) / (4 * TOKENS), 256, 0, st>>>( \
         rows, indices, locations, plane_stride, top_k, samples, model_dim, capacity, grad_logits, wg, experts, out))
+#define PM_DX_FEW(CACHE, INT8, EP)                                                                              \
+    do {                                                                                                        \
+        constexpr int TOKENS = CACHE >= 4 ? 1 : 4 / CACHE;                                                      \
+        layer_dx_few_kernel<DT, CACHE, INT8, EP><<<(samples + TOKENS - 1) / TOKENS, 256, 0, st>>>(              \
+            rows, indices, locations, plane_stride, top_k, samples, model_dim, capacity, grad_logits, wg, experts, out);            \
+    } while (0)
 #define PM_DX_(CACHE, INT8, EP)                                                                                 \
     do {                                                                                                        \
+        if (few) { PM_DX_FEW(CACHE, INT8, EP); break; }                                                         \
         if constexpr (DT == PLANMOE_F32) { if (pairs) { PM_DX__(CACHE, INT8, EP, 2); break; } }                 \
         PM_DX__(CACHE, INT8, EP, 1);                                                                            \
     } while (0)
@@ -446,7 +558,10 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
         if (codec) { if (experts <= 4) PM_DX_(CACHE, true, 4); else if (experts <= 8) PM_DX_(CACHE, true, 8); else PM_DX_(CACHE, true, 16); }      \
         else { if (experts <= 4) PM_DX_(CACHE, false, 4); else if (experts <= 8) PM_DX_(CACHE, false, 8); else PM_DX_(CACHE, false, 16); }         \
     } while (0)
-    PM_DTYPE_SWITCH(dtype, DT, { if (per_lane <= 1) PM_DX(1); else if (per_lane <= 2) PM_DX(2); else if (per_lane <= 4) PM_DX(4); else PM_DX(8); });
+#define PM_DX_WIDE() do { if (codec) PM_DX_FEW(16, true, 8); else PM_DX_FEW(16, false, 8); } while (0)
+    PM_DTYPE_SWITCH(dtype, DT, { if (per_lane <= 1) PM_DX(1); else if (per_lane <= 2) PM_DX(2); else if (per_lane <= 4) PM_DX(4); else if (per_lane <= 8) PM_DX(8); else PM_DX_WIDE(); });
+#undef PM_DX_WIDE
+#undef PM_DX_FEW
 #undef PM_DX
 #undef PM_DX_
 #undef PM_DX__

@@ -791,3 +791,32 @@ def test_layer_dx_of_up_to_16_experts(T, M, E, k, cap, dtype, codec):
     # E + 1 terms in fp32, then one rounding
     bound = want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) + size * (E + 1) * 2.0 ** -24 + 1e-30
     assert bool(((out.double() - want).abs() <= bound).all())
+
+
+# Few tokens, up to 8 experts: the same bits as the combine and the gate's share in launches of their own.  One token, an odd number; rows of less than a
+# wave's 64 pieces, of one more, of two, five and nine times 64 and of sixteen, the widest; the last number of tokens that is few and the first that is not
+@pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 1, 1, 1), (5, 264, 8, 2, 1), (255, 520, 3, 2, 100), (37, 1288, 8, 2, 8), (131, 2568, 5, 3, 64), (9, 4096, 8, 2, 4), (7, 8192, 4, 2, 4),
+                                         (256, 3080, 2, 1, 100), (257, 3080, 2, 1, 100), (768, 776, 8, 2, 200), (769, 776, 8, 2, 200), (4096, 264, 4, 1, 1000), (4097, 264, 4, 1, 1000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("codec", [0, 1])
+def test_layer_dx_of_few_tokens(T, M, E, k, cap, dtype, codec):
+    from planmoe_amd import ops
+    from planmoe_amd._lib import check, lib
+    if dtype == torch.float32 and M > 4096:
+        pytest.skip("rows of up to 16 KB")
+    print("case", T, M, E, k, cap, dtype, codec, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + M + E)
+    routed = ops.route_topk(torch.softmax(torch.randn(T, E, generator=g, device=DEV), 1), k)
+    idx, loc = routed["indices"].view(k, T), routed["locations"].view(k, T)
+    rows, wg = torch.randn(E * cap, M, generator=g, device=DEV).to(dtype), torch.randn(E, M, generator=g, device=DEV).to(dtype)
+    rows[0] = float("inf")                   # (what a choice without a slot reads and does not use)
+    gl = torch.randn(T, E, generator=g, device=DEV)
+    out, want = torch.empty(T, M, dtype=dtype, device=DEV), torch.empty(T, M, dtype=dtype, device=DEV)
+    p, dt, st = ops._ptr, ops._dt(rows, "t"), ops._stream(rows)
+    check(lib.planmoe_layer_dx(p(rows), dt, codec, p(idx), p(loc), T, k, T, M, E, cap, p(gl), p(wg), p(out), st))
+    check(lib.planmoe_layer_combine(p(rows), dt, codec, None, p(idx), p(loc), T, k, T, M, E, cap, p(want), st))
+    check(lib.planmoe_gate_dx_accumulate(p(want), dt, p(gl), p(wg), T, M, E, st))
+    torch.cuda.synchronize()
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    same = (out.view(bits) == want.view(bits)) | (out.isnan() & want.isnan())
+    assert bool(same.all())
