@@ -8,7 +8,9 @@
 //
 // Stored past the caches: an optimizer reads a weight gradient once and late.  Rows that are not whole lines share a line with the next row's wave, which
 // the caches put together: such rows are stored plainly, in bf16 256 columns a wave so that there are fewer of those lines, in fp32 only where the last
-// cache (256 MB) does not hold the result.  us: the tiles, then 32 x 128 (bf16 256) plain and past the caches, 32 x 64 (bf16 128) plain and past them
+// cache (256 MB) does not hold the result.  In bf16 the waves that share lines are brought together as well (8 experts x 8 rows, 2600 x 3440, 37 and 31 us; x 29,
+// 1888 x 1256, 15.8 and 14.7; x 64, 1896 x 1032, 19.3 and 17.6; in fp32 16 x 1, 3328 x 3072 103 and 117).  Neither a step of k asked for ahead of the
+// products nor 128 rows of 64 columns a work-group gained anything in the others.  us, before that: the tiles, then 32 x 128 (bf16 256) plain and past the caches, 32 x 64 (bf16 128) plain and past them
 //   fp32  16 x 1, 3328 x 3072  220: 119, 116, 134, 112     8 x 8, 2600 x 3440   100: 56, 58, 56, 63     16 x 2, 1896 x 688   33: 23, 22, 20, 19
 //         8 x 2, 4096 x 4096   178: 94, 84, 108, 89        8 x 64, 2048 x 2048   65: 52, 50, 50, 50     8 x 128, 2048 x 2048 95: 81, 80, 85, 83
 //         4 x 128, 512 x 1024  10.5: 14.8, 13.5, 10.9, 10.3
@@ -30,10 +32,16 @@ __global__ __launch_bounds__(256, (F32 ? J == 4 : J == 8) ? 2 : 4) void gemm_out
     typedef uint32_t words __attribute__((ext_vector_type(W)));
     constexpr uint32_t NOWHERE = 0x80000000u;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 31, fc = lane >> 5;
-    const int groups_n = (p.N + 4 * COLS - 1) / (4 * COLS), tiles_m = (p.M + 31) / 32;
-    const int e = blockIdx.x / (groups_n * tiles_m), in = blockIdx.x - e * groups_n * tiles_m;
-    const int m0 = in / groups_n * 32, n0 = (in % groups_n * 4 + wave) * COLS;
-    if (n0 >= p.N) return;
+    // The waves of a work-group lie next to each other; DOWN: one below the other, and XCD j (work-groups j, j + 8, ...) takes the j-th eighth, so that what shares a
+    // line of C shares an L2
+    constexpr bool DOWN = !F32 && J == 8;
+    constexpr int BELOW = DOWN ? 4 : 1, BESIDE = 4 / BELOW;
+    const int groups_n = (p.N + BESIDE * COLS - 1) / (BESIDE * COLS), groups_m = (p.M + 32 * BELOW - 1) / (32 * BELOW), total = groups_n * groups_m * p.batches;
+    const int number = DOWN ? blockIdx.x % 8 * ((total + 7) / 8) + blockIdx.x / 8 : blockIdx.x;
+    if (number >= total || (DOWN && (int)blockIdx.x / 8 >= (total + 7) / 8)) return;
+    const int e = number / (groups_n * groups_m), in = number - e * groups_n * groups_m;
+    const int m0 = (in / groups_n * BELOW + (DOWN ? wave : 0)) * 32, n0 = (in % groups_n * BESIDE + (DOWN ? 0 : wave)) * COLS;
+    if (n0 >= p.N || m0 >= p.M) return;
     int K = p.K;
     if (p.live) {
         int n = 0;
@@ -150,16 +158,24 @@ __global__ __launch_bounds__(256, (F32 ? J == 4 : J == 8) ? 2 : 4) void gemm_out
 template <bool F32, int J, bool NT>
 static int outer_launch(const OuterArgs &p, hipStream_t stream, const char *who)
 {
-    const int64_t blocks = ((int64_t)p.M + 31) / 32 * (((int64_t)p.N + 128 * J - 1) / (128 * J)) * p.batches;
-    gemm_outer_kernel<F32, J, NT><<<dim3((unsigned)blocks), 256, 0, stream>>>(p);
+    const int64_t down = !F32 && J == 8 ? 128 : 32, across = !F32 && J == 8 ? 32 * J : 128 * J;          // a work-group's
+    const int64_t blocks = ((int64_t)p.M + down - 1) / down * (((int64_t)p.N + across - 1) / across) * p.batches;
+    gemm_outer_kernel<F32, J, NT><<<dim3((unsigned)((blocks + 7) / 8 * 8)), 256, 0, stream>>>(p);
     PM_LAUNCH_CHECK(who);
     return 0;
 }
 
-// Up to 100 rows in fp32 (where the result is small nothing is gained beyond) and 64 in bf16, whose tiles take less for a row; an expert may have half as many again.
+// Up to 100 rows in fp32 and 64 in bf16, whose tiles take less for a row; an expert may have half as many again.  Fewer where the result has few waves, whose steps of 16
+// rows are a trip to memory each, and in bf16 where rows are not whole lines.  us, the tiles and this
+//   bf16  5 x 264 x 520, 33 rows 4.4, 5.0;  4 x 256 x 256, 24 rows 4.4, 3.8;  4, 40 and 64 rows
+//         8 x 512 x 512 5.9, 3.8   5.9, 5.3   6.1, 6.8   8 x 1024 x 1024 10.0, 6.0   10.1, 6.8   10.1, 8.0   16 x 1024 x 1032 16.7, 10.5   17.0, 14.8   17.5, 18.8
+//   fp32  4, 40 and 100 rows  8 x 264 x 520 5.5, 5.1   6.6, 6.9   8.6, 10.8  8 x 512 x 512     6.1, 5.0    7.3, 6.7    9.4, 10.7  8 x 1024 x 1024  15.1, 8.9    18.1, 12.7   22.3, 20.4
 bool gemm_outer_serves(int dtype, int m, int n, int64_t k, int batches, int64_t rows)
 {
-    const int64_t size = dtype == PLANMOE_F32 ? 4 : 2, most = dtype == PLANMOE_F32 ? 100 : 64;
+    const int64_t size = dtype == PLANMOE_F32 ? 4 : 2, values = (int64_t)m * n * batches;
+    const bool large = values > (int64_t)4 << 20;
+    const int64_t most = dtype == PLANMOE_F32 ? large ? 100 : values > (int64_t)3 << 19 ? 48 : 8
+                                                        : large && (int64_t)n * size % 128 == 0 ? 64 : values > (int64_t)3 << 19 ? 40 : 24;
     return rows <= most && 2 * k <= 3 * most && k * m * size < ((int64_t)1 << 31) && k * n * size < ((int64_t)1 << 31) &&
            ((int64_t)m + 31) / 32 * (((int64_t)n + 255) / 256) * batches < ((int64_t)1 << 30);
 }

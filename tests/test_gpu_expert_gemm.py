@@ -856,7 +856,7 @@ def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(form, B, cap, n, k, hi
 @pytest.mark.parametrize("dtype,B,cap,m,n", [
     (torch.float32, 8, 1, 1028, 1024), (torch.float32, 8, 17, 1036, 1060), (torch.float32, 4, 100, 1024, 2084), (torch.float32, 8, 24, 2052, 4100),
     (torch.float32, 8, 150, 712, 1024), (torch.bfloat16, 4, 1, 8, 16), (torch.bfloat16, 4, 16, 40, 64), (torch.bfloat16, 8, 33, 264, 1032),
-    (torch.bfloat16, 4, 90, 1032, 192), (torch.bfloat16, 3, 12, 72, 2056)])
+    (torch.bfloat16, 4, 90, 1032, 1024), (torch.bfloat16, 3, 12, 72, 2056), (torch.bfloat16, 3, 24, 200, 520)])
 def test_expert_gemm_weight_gradients_of_few_rows_have_the_tiles_bits(dtype, B, cap, m, n):
     from planmoe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(m + n)
