@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
 // out[t] = sum_j (live_j ? gate_j * dispatched[slot_j] : 0), planes added left to right.  Bound by memory.  A wave asks for B units a lane
 // of two choices' rows before it adds any (a dropped choice reads slot 0 and contributes zeros): one wait a pass over 4 KB rows, and
 // over 8 KB rows with B = 8 (8192 x 2048 fp32, two choices, 201 MB: 36.7 us, 38.5 with four units of one choice at a time, 38.8 of two; 14020 x 3528 bf16
-// 54.8, 57.7, 57.5; rows of 2 KB lose with eight: 16384 x 1024 bf16 17.5 and 23.6).
+// 54.8, 57.7, 57.5; rows of 2 KB lose with eight: 16384 x 1024 bf16 17.5 and 23.6; which rows take eight: planmoe_combine_fwd).
 template <int DT, int MODE, int B>
 __global__ __launch_bounds__(256) void combine_kernel(
     const void *__restrict__ dispatched, const float *__restrict__ gates,
@@ -457,7 +457,13 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     hipStream_t st = (hipStream_t)stream;
     const int mode = rows_mode(dtype, model_dim, out, dispatched);
     const int blocks = (samples + 3) / 4;
-    const bool wide = (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2) > 4096;
+    // Eight units a lane: rows above 4 KB, in 16 bits, whose units take twice the registers unpacked, only where the caches do not hold what is moved (14020 x
+    // 3528 beside the kernel), or where eight lanes at most have a unit of a row's last pass of four a lane.  us, two choices, bf16 rows that the caches hold, with
+    // four and with eight:  1400 tokens x 3876 6.8, 7.5   4000 x 4096 15.9, 17.8   4000 x 2176 10.9, 11.8   8000 x 2304 19.2, 20.9   1400 x 2112 7.0, 5.8
+    // fp32:  1400 x 1056 5.5, 4.6   1400 x 2048 5.9, 5.5   4000 x 2560 19.3, 19.5   6800 x 4096 66, 62
+    const int64_t row_bytes = (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2);
+    const bool few_lanes = ((row_bytes + 15) / 16 + 255) % 256 < 8;
+    const bool wide = row_bytes > 4096 && (dtype == PLANMOE_F32 || mode == ROWS_1 || few_lanes || !stays(row_bytes * samples * (top_k + 1)));
     if (capacity == 0) {
         // no slot exists, every choice is dropped: zero rows.  (combine_kernel fetches rows with
         // unconditional loads at clamped slots and must not run without a row to read.)

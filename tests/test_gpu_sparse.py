@@ -65,7 +65,7 @@ def test_dispatch_and_combine_bit_exact(T, M, E, k, cf, dtype):
 
 
 @pytest.mark.parametrize("M,dtype", [(1020, torch.float32), (1028, torch.float32), (2048, torch.float32), (2052, torch.float32), (2056, torch.bfloat16),
-                                     (4104, torch.bfloat16), (2050, torch.float16), (257, torch.float16), (2051, torch.bfloat16)])
+                                     (4104, torch.bfloat16), (2050, torch.float16), (257, torch.float16), (2051, torch.bfloat16), (2112, torch.bfloat16), (2120, torch.bfloat16), (3876, torch.bfloat16)])
 @pytest.mark.parametrize("k", [1, 3, 5])
 def test_rows_around_a_pass_bit_exact(M, dtype, k):
     """Rows that end around the vectors a wave asks for at once (four or eight a lane), odd numbers of choices."""
