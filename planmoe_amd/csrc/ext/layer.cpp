@@ -133,13 +133,14 @@ struct Kept {
 //   bf16, int8   64 x 1024 6.7, 12.1    4096 x 2048 26.5, 30.6    16384 x 1024 52.1, 44.7    1024 x 4096 18.0, 20.6    4096 x 4096 52.2, 45.4
 //   fp32         1024 x 256 4.9, 7.3    4096 x 1024 13.4, 21.4    16384 x 2048 81, 125
 //   fp32, int8   1024 x 256 7.0, 8.0    1024 x 1024 14.6, 12.4    4096 x 1024 19.8, 25.5     16384 x 2048 124, 132
-// (fp32 up to 4096 tokens, with int8 768, is planmoe_layer_dx's kernel for few: x 1024, 64 tokens 4.2 where the other way takes 7.0, with int8 5.9 and 700 tokens 9.1.)
+// (fp32, fewer tokens and rows above 2 KB: one pass would be the faster one here too, 64 x 1024 4.2 and 7.0, but it rounds the sum once an expert where the other way adds the gate's
+// whole product: error against 64 bits 1.0e-7 of the norm, and 3.8e-8.)
 bool dx_in_one(const Shape &s, int codec)
 {
     if (s.E <= 8) return true;
     const int64_t values = (int64_t)s.T * s.M;
     if (s.E > 16 || (int64_t)s.M * (s.dt == PLANMOE_F32 ? 4 : 2) > 8192) return false;
-    if (s.dt == PLANMOE_F32) return s.M <= 512 || s.T >= 4096 || s.T <= 768 || codec != CODEC_INT8;
+    if (s.dt == PLANMOE_F32) return s.M <= 512 || s.T >= 4096 || (s.T >= 1024 && codec != CODEC_INT8);
     return codec != CODEC_INT8 || (s.T <= 8192 && values <= (1 << 23));
 }
 
