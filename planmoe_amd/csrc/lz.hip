@@ -810,10 +810,11 @@ extern "C" int64_t planmoe_lz_blocks(int64_t nbytes)
     return nbytes <= 0 ? 0 : (nbytes + LZ_BLOCK_BYTES - 1) / LZ_BLOCK_BYTES;
 }
 
-// workspace: class byte per block | chunk totals | sizes, up to LZ_SUMMED blocks | tokens of the blocks with matches, two bytes a position
+// workspace: class byte per block | chunk totals | sizes of LZ_SUMMED blocks at most (unused by more, but counted: what serves an input serves every shorter
+// one) | tokens of the blocks with matches, two bytes a position
 static size_t lz_class_bytes(int64_t blocks) { return round_up((size_t)blocks, 256); }
 static size_t lz_sizes_at(int64_t blocks) { return lz_class_bytes(blocks) + 2 * LZ_MAX_CHUNKS * sizeof(uint32_t); }
-static size_t lz_tokens_at(int64_t blocks) { return lz_sizes_at(blocks) + (blocks <= LZ_SUMMED ? round_up((size_t)blocks * 4, 256) : 0); }
+static size_t lz_tokens_at(int64_t blocks) { return lz_sizes_at(blocks) + round_up((size_t)min(blocks, (int64_t)LZ_SUMMED) * 4, 256); }
 
 extern "C" size_t planmoe_lz_workspace_bytes(int64_t nbytes)
 {

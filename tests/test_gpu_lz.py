@@ -132,6 +132,17 @@ def test_one_workspace_call_after_call():
         same_streams(got, oracle.lz_compress(x))
 
 
+def test_one_workspace_around_the_last_input_without_a_scan():
+    """A workspace for 8193 blocks, whose offsets are scanned, serves 8192, whose sizes are added up, and the other way round after it."""
+    rng = np.random.default_rng(10)
+    big = rng.integers(0, 3, size=8193 * 512).astype(np.float32)
+    ws = torch.empty((int(_lib.lib.planmoe_lz_workspace_bytes(big.nbytes)),), dtype=torch.uint8, device=DEV)
+    for x in (big, big[512:], big):
+        x = np.ascontiguousarray(x)
+        got = ops.lz_compress(torch.from_numpy(x).to(DEV), workspace=ws)
+        same_streams(got, oracle.lz_compress(x))
+
+
 def test_config5_full_size():
     """The [16, 8192, 1024] fp32 buffer of config 5 (512 MiB, 262 144 blocks): a quarter of the
     capacity slots empty, some rows thinned out like an activation after a ReLU, the rest dense.

@@ -282,3 +282,10 @@ def test_hooks_of_a_module_are_found_by_their_names():
     assert not _hooked(module)
     module.register_forward_hook(lambda *args: None)
     assert _hooked(module)
+
+
+def test_lz_workspace_for_an_input_serves_every_shorter_one():
+    from planmoe_amd._lib import lib
+    sizes = [int(lib.planmoe_lz_workspace_bytes(4 * symbols)) for blocks in [*range(1, 40), *range(8100, 8400), *range(16300, 16500), 262144]
+             for symbols in (512 * blocks - 511, 512 * blocks)]
+    assert sizes == sorted(sizes)
