@@ -456,10 +456,10 @@ int planmoe_expert_gemm(int form, int dtype, const void *a, const void *b, const
                         int live_round, int rows_hint, void *c, void *stream);
 
 /* Which kernel planmoe_expert_gemm takes such a product to on the current device (counted: with live), a name for logs and tests:
- * "few rows", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"; fp32: "f32 waves",
- * "f32 64x64", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128".  ("128x128 alone": 128 rows
- * by 128 or 64 columns.)
- * planmoe_expert_gemm_relu_bwd takes the one of form 1 without activation.  NULL where the product would be refused. */
+ * "few rows", "few rows of a^T b", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"; fp32:
+ * "f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 32x32", "f32 32x32 eight stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128",
+ * "f32 parts 256x128", "f32 parts few rows of a^T b".  ("128x128 alone": 128 rows by 128 or 64 columns.)
+ * planmoe_expert_gemm_relu_bwd takes the one of form 1 without activation (fp32 with dbias and m up to 16: the one of m = 17).  NULL where the product would be refused. */
 const char *planmoe_expert_gemm_kernel(int form, int dtype, int activation, int batches, int m, int n, int k,
                                        int counted, int rows_hint);
 

@@ -959,11 +959,11 @@ extern "C" const char *planmoe_expert_gemm_kernel(int form, int dtype, int activ
     if (bad()) return nullptr;
     const int most = form == 2 ? k : m, hint = rows_hint >= 1 && rows_hint < most ? rows_hint : most;
     if (dtype == PLANMOE_F32) {
-        static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 64x64 four stages", "f32 64x64 four stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
+        static const char *const names[] = {"f32 waves", "f32 64x64", "f32 64x64 four stages", "f32 32x32", "f32 32x32 eight stages", "f32 128x128", "f32 parts 64x64", "f32 parts 128x128", "f32 parts 256x128"};
         const Gemm32Kernel kernel = gemm_f32_pick(form, Gemm32Args{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, live, 1, 1, m, n, k, batches, activation}, hint);
-        return form == 2 && kernel >= G32_SPLIT_64 && gemm_outer_serves(dtype, m, n, k, batches, hint) ? "f32 parts few rows" : names[kernel];
+        return form == 2 && kernel >= G32_SPLIT_64 && gemm_outer_serves(dtype, m, n, k, batches, hint) ? "f32 parts few rows of a^T b" : names[kernel];
     }
-    if (form == 2 && !activation && gemm_outer_serves(dtype, m, n, k, batches, hint)) return "few rows";
+    if (form == 2 && !activation && gemm_outer_serves(dtype, m, n, k, batches, hint)) return "few rows of a^T b";
     static const char *const names[] = {"few rows", "128x128 alone", "128x128 alone", "128x128", "128x256", "160x256", "192x256", "256x256", "256x256 and quarters"};
     const int lda = form == 2 ? m : k, ldb = form == 1 ? k : n;
     return names[gemm_pick(form, gemm_contiguous(form, m, n, k, lda, ldb, n, (int64_t)m * k, (int64_t)n * k, (int64_t)m * n), m, n, k, batches, counted, hint)];

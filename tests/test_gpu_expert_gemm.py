@@ -657,7 +657,10 @@ IN_KERNEL = [
     (torch.bfloat16, "tn", "256x256", 8, 201, 2072, 392, 160), (torch.bfloat16, "tn", "256x256", 8, 270, 2712, 264, 216),
     (torch.bfloat16, "tn", "256x256 and quarters", 4, 1098, 2784, 1512, 1098), (torch.bfloat16, "tn", "256x256 and quarters", 4, 1288, 2480, 1576, 1288),
     (torch.float32, "rows", "f32 waves", 4, 9, 16, 168, 8), (torch.float32, "rows", "f32 64x64", 4, 37, 16, 164, 37),
-    (torch.float32, "rows", "f32 64x64 four stages", 4, 70, 68, 268, 60), (torch.float32, "rows", "f32 128x128", 8, 73, 3232, 176, 65),
+    (torch.float32, "rows", "f32 64x64 four stages", 16, 81, 880, 264, 79), (torch.float32, "rows", "f32 64x64 four stages", 16, 81, 844, 240, 79),
+    (torch.float32, "rows", "f32 32x32", 8, 70, 548, 260, 70), (torch.float32, "rows", "f32 32x32", 8, 44, 780, 240, 43),
+    (torch.float32, "rows", "f32 32x32 eight stages", 4, 70, 68, 268, 60), (torch.float32, "rows", "f32 32x32 eight stages", 4, 78, 36, 236, 70),
+    (torch.float32, "rows", "f32 128x128", 8, 73, 3232, 176, 65),
     (torch.float32, "rows", "f32 parts 64x64", 4, 2618, 260, 292, 2356), (torch.float32, "rows", "f32 parts 64x64", 8, 324, 1052, 260, 291),
     (torch.float32, "rows", "f32 parts 128x128", 8, 389, 848, 300, 311), (torch.float32, "rows", "f32 parts 128x128", 4, 388, 1736, 268, 349),
     (torch.float32, "rows", "f32 parts 256x128", 5, 2382, 388, 292, 2382), (torch.float32, "rows", "f32 parts 256x128", 16, 512, 1024, 1024, 512),
@@ -812,17 +815,19 @@ def _column_sums_hold(db, got, rows, cap):
         assert bool(((db[e].double() - ref).abs() <= cap * 2.0 ** -24 * got[e, :r].double().abs().sum(0)).all())
 
 
-# fp32 tiles of 32 x 32, five and eight k-tiles in LDS, and of 64 x 64 with small ones of 16 and 32 rows behind them (the last shape); columns, reductions
+# fp32 tiles of 32 x 32, five and eight k-tiles in LDS, and of 64 x 64 with small ones of 16 and 32 rows behind them; columns, reductions
 # and row counts around their sides, with and without counts.  Each 32 rows go through the waves as well, among more columns, and the bits are theirs.
 @pytest.mark.parametrize("counted", [True, False])
-@pytest.mark.parametrize("form,B,cap,n,k,hint", [
-    ("nn", 4, 12, 52, 300, 9), ("nn", 16, 20, 1036, 292, 20), ("nn", 2, 70, 148, 724, 70), ("nn", 8, 163, 260, 2044, 163), ("nn", 1, 33, 4, 228, 33),
-    ("nt", 4, 40, 68, 236, 30), ("nt", 16, 33, 1060, 236, 30), ("nt", 3, 97, 100, 240, 97), ("nn", 16, 108, 512, 1536, 97), ("nt", 16, 108, 1028, 252, 97)])
-def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(form, B, cap, n, k, hint, counted):
+@pytest.mark.parametrize("kernel,form,B,cap,n,k,hint", [
+    ("f32 32x32 eight stages", "nn", 4, 12, 52, 300, 9), ("f32 32x32", "nn", 16, 20, 1036, 292, 20), ("f32 32x32 eight stages", "nn", 2, 70, 148, 724, 70),
+    ("f32 32x32", "nn", 8, 163, 260, 2044, 163), ("f32 32x32 eight stages", "nn", 1, 33, 4, 228, 33), ("f32 32x32 eight stages", "nt", 4, 40, 68, 236, 30),
+    ("f32 32x32", "nt", 16, 33, 1060, 236, 30), ("f32 32x32 eight stages", "nt", 3, 97, 100, 240, 97), ("f32 64x64 four stages", "nn", 16, 108, 512, 1536, 97),
+    ("f32 64x64 four stages", "nn", 16, 81, 880, 264, 79), ("f32 64x64 four stages", "nt", 16, 81, 844, 252, 79), ("f32 64x64 four stages", "nt", 16, 81, 880, 264, 79)])
+def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(kernel, form, B, cap, n, k, hint, counted):
     from planmoe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(n + k)
     rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
-    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=counted, rows_hint=hint) == "f32 64x64 four stages"
+    assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=counted, rows_hint=hint) == kernel
     edges = [cap, 0, 1, 65, 80, 81, 96, 97, 15, 16, 17, 31, 32, 33, 63, 64]
     rows = [min(cap, edges[e % 16]) if counted else cap for e in range(B)]
     live = torch.tensor([rows], dtype=torch.int32, device=DEV) if counted else None
@@ -861,7 +866,7 @@ def test_expert_gemm_weight_gradients_of_few_rows_have_the_tiles_bits(dtype, B, 
     from planmoe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(m + n)
     hint, more = min(cap, 100 if dtype == torch.float32 else 60), 300
-    assert ops.expert_gemm_kernel("tn", dtype, B, m, n, cap, counted=True, rows_hint=hint) == ("f32 parts few rows" if dtype == torch.float32 else "few rows")
+    assert ops.expert_gemm_kernel("tn", dtype, B, m, n, cap, counted=True, rows_hint=hint) == ("f32 parts few rows of a^T b" if dtype == torch.float32 else "few rows of a^T b")
     tiles = ops.expert_gemm_kernel("tn", dtype, B, m, n, more, counted=True, rows_hint=more)
     assert "few rows" not in tiles and (dtype != torch.float32 or "parts" in tiles)
     edges = [cap, 0, 1, hint, 16, 17, 31, 33]
