@@ -523,11 +523,15 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 //   nt  8 x 21, 1896 -> 568       22, 22 and 14, 14      8 x 9, 2048 -> 2048   31, 27 and 31, 22      8 x 1, 1024 -> 4096    28, 23 and 32, 24
 //       16 x 1, 3072 -> 3328      131 and 121            8 x 20, 1024 -> 4096  36, 29 and 33, 23
 //   skewed, 8 experts, 128 of 256 rows on one, 4096 -> 1024 nn 67, 58 and 49, 40 (64 x 64 123)
-// Beyond, a compute unit takes 0.26 us for a k-tile of up to two tiles of 32 x 32, whose chains of products hide behind each other, 0.145 for each of more, and
-// 0.475 for one of 64 x 64, a third more where it has a small one beside it.
-//   nn  4 x 260 rows, 512 -> 1024  17, 17 and 19, 19      1024 -> 512          22, 21 and 19, 18      8 x 163, 2048 -> 256  36, 36 and 23, 23
-//       8 x 66, 1024 -> 1024       22, 22 and 21, 19      4 x 48, 3648 -> 1088 60, 59 and 34, 34      8 x 100, 1024 -> 1024 23, 22 and 25, 22
-//       16 x 45, 1024 -> 256       20, 20 and 9, 9        4 x 48, 1088 -> 3648 23, 23 and 26, 23      16 x 97, 1536 -> 512  31, 30 and 34, 30
+// Beyond, tiles of 32 x 32 up to two a compute unit (eight k-tiles in LDS up to one), whose chains of products hide behind each other: a k-tile takes 0.275 us
+// for both.  With more of them one takes 0.158 us each, a compute unit takes them in whole numbers, and 0.55 us each once; a k-tile of 64 x 64 takes 0.5 us, 1.5 of that
+// beside a small one (several: 0.75 for each small one).  The weight costs 32 x 32 more, whose lines are asked for by more of them, and with its rows of k more
+// still.  (Fitted to 2025 products of 33 to 400 rows, half of them within 5 %; what is picked is within 5 % of the faster one in 93 % of them.)  us, weights cold, tiles of 64 x 64
+// and of 32 x 32:
+//   nn  4 x 260 rows, 512 -> 1024  17, 19      1024 -> 512         22, 19      8 x 163, 2048 -> 256    36, 23      4 x 276, 1664 -> 2304   90, 91
+//       8 x 66, 1024 -> 1024       22, 21      4 x 48, 3648 -> 1088 60, 34     8 x 100, 1024 -> 1024   23, 25      16 x 124, 3316 -> 768  115, 137
+//       16 x 45, 1024 -> 256       20,  9      4 x 48, 1088 -> 3648 23, 26     16 x 97, 1536 -> 512    31, 34      8 x 288, 3200 -> 512   110, 91
+//   nt  4 x 306, 972 -> 704        23, 24      8 x 178, 512 -> 512  14, 12     4 x 151, 2400 -> 2048   85, 70      4 x 330, 384 -> 1408    19, 21
 // On the bf16 matrix cores, in three parts a value (gemm_f32_split.hip), where there is more than one tile of 64 x 64 for a compute
 // unit; one tile on its own is bound by issuing the splits (8 experts, 128 rows, 1024 -> 1024: 20 us in fp32, 28 in parts) and stays here.
 // A launch takes its rounds; us for a k-tile with few and with all compute units at work, and once for a tile, fitted to 60 shapes
@@ -589,14 +593,14 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
     }
     const bool deep = gemm_f32_deep(form, p, rows_hint);
     const int64_t m = form == 2 ? p.M : rows_hint, cu = compute_units();
-    const double kt = (double)((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK;
+    const double kt = (double)(((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK);
     if (form != 2 && rows_hint <= 32) {
         const int64_t pieces = gemm_f32_pieces(p, rows_hint, 32);
         const bool one = p.M <= 16 && !p.colsum, past = gemm_f32_past_caches(p);
         const bool lines = pieces > 3 * cu && pieces <= 4 * cu && (one || (form == 0 && !past));
         const bool fits = (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30);
         if (fits && (!deep || lines || (form == 0 && one && past && pieces >= 4 * cu))) return G32_WAVES;
-        if (deep) return 2 * pieces <= 3 * cu ? G32_SLIM_ALONE : G32_SLIM;
+        if (deep) return pieces <= cu ? G32_SLIM_ALONE : G32_SLIM;
     }
     auto cost = [&](int64_t side, double us, double once) {
         const int64_t tiles = (m + side - 1) / side * ((p.N + side - 1) / side) * p.batches;
@@ -611,14 +615,13 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
             small += 0.25 * (rest > 0 && rest <= 32);
             slim += 0.25 * (double)((r + 31) / 32);
         }
-        const double columns = (double)((p.N + 63) / 64 * p.batches);
+        const double columns = (double)((p.N + 63) / 64 * p.batches) / cu, mb = 4e-6 * (double)p.batches * p.N * p.K;
         whole *= columns;
         small *= columns;
         slim *= (double)((p.N + 31) / 32 * p.batches) / cu;
-        const double units = whole <= cu ? whole + small > cu ? 1.35 : 1. : std::ceil(whole / cu);
-        const double weight = slim > 2 ? 1e-7 * (double)p.batches * p.N * p.K * 4 : 0.;          // (0.1 us for every MB: its lines are asked for by more of them)
-        const double us = std::max(0.262, 0.145 * std::ceil(slim)) * kt + 2.5 + weight;
-        if (1.03 * us < 0.475 * kt * units + 6 && us < cost(128, 1.9, 4)) return slim <= 1.5 ? G32_SLIM_ALONE : G32_SLIM;
+        const double us = kt * std::max(0.275, 0.158 * std::ceil(slim)) + 3.2 + 0.55 * slim + (form == 0 ? 0.065 : 0.027) * mb;
+        const double deep_us = kt * 0.5 * (whole > 1 ? std::ceil(whole) + 0.75 * small : whole + small > 1 ? 1.46 : 1.) + 4.8 + 0.03 * mb;
+        if ((slim <= 2 || us < deep_us) && us < cost(128, 1.9, 4)) return slim <= 1 ? G32_SLIM_ALONE : G32_SLIM;
     }
     return cost(64, deep ? 0.47 : 0.52, 1.2) < cost(128, 1.9, 4) ? deep ? G32_DEEP_64 : G32_TILE_64 : G32_TILE_128;
 }
