@@ -515,8 +515,9 @@ static bool gemm_f32_deep(int form, const Gemm32Args &p, int rows_hint)
 // 1.2 for 64 x 64, 0.47 with four stages; what counts is the fullest compute unit (us, 64 x 64, with four stages, 128 x 128: 4 x 1000 rows,
 // 2048 -> 512 77, 66, 137; 16 x 512, 1024 -> 1024 142, 131, 131; 512 -> 2048 152, 144, 138; 2 x 4096, 4096 -> 4096 2129, 1944, 1969).
 // Up to 32 rows tiles of 32 x 32 (gemm_f32_slim.hip; five k-tiles in LDS, eight where that leaves work-groups room), or waves on their own: with fewer than
-// eight k-tiles, where there is a wave of 32 columns for each SIMD and hardly a tile more than four for a compute unit to take in turn, and for weights past the
-// caches.  us, weights cold, in the last cache, waves and tiles of 32 x 32:
+// eight k-tiles, where there is a wave of 32 columns for each SIMD and hardly a tile more than four for a compute unit to take in turn, for weights past the
+// caches, and b^T with up to 16 rows where a compute unit has more than one tile and up to one and a half (up to two with up to 4 rows: a wave reads all rows for its 16
+// columns): waves 0.86 - 0.94 of the tiles' time at any k, cold (8 x 3, 384 -> 1408 6.3 and 7.3, 4 x 14, 1180 -> 2176 14.8 and 15.8, 4 x 3, 3264 -> 2440 32 and 36).  us, weights cold, in the last cache, waves and tiles of 32 x 32:
 //   nn  8 x 21 rows, 1896 -> 568  28, 28 and 16, 14      4 x 21, 2808 -> 1040  39, 39 and 19, 18      8 x 2, 4096 -> 1024    49, 37 and 27, 24
 //       8 x 1, 1024 -> 4096       27, 23 and 34, 29      8 x 7, 3440 -> 2600   76, 66 and 65, 55      16 x 7, 1536 -> 2304   59, 51 and 51, 45
 //       16 x 16, 1472 -> 2176     68, 60 and 49, 39      8 x 20, 1024 -> 4096  34, 27 and 38, 30      16 x 1, 2048 -> 2560   55, 55 and 70, 66
@@ -599,7 +600,8 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
         const bool one = p.M <= 16 && !p.colsum, past = gemm_f32_past_caches(p);
         const bool lines = pieces > 3 * cu && pieces <= 4 * cu && (one || (form == 0 && !past));
         const bool fits = (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30);
-        if (fits && (!deep || lines || (form == 0 && one && past && pieces >= 4 * cu))) return G32_WAVES;
+        const bool turns = form == 1 && one && pieces > cu && 2 * pieces <= (rows_hint <= 4 ? 4 : 3) * cu;
+        if (fits && (!deep || lines || turns || (form == 0 && one && past && pieces >= 4 * cu))) return G32_WAVES;
         if (deep) return pieces <= cu ? G32_SLIM_ALONE : G32_SLIM;
     }
     auto cost = [&](int64_t side, double us, double once) {

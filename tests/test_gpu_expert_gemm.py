@@ -779,7 +779,7 @@ def test_sums_of_shares_are_added_in_pairs(shares):
 @pytest.mark.parametrize("form,B,cap,n,k", [
     ("nn", 4, 12, 52, 200), ("nn", 16, 16, 520, 36), ("nn", 16, 8, 1036, 148), ("nn", 16, 9, 1300, 20), ("nn", 16, 4, 2100, 2080),
     ("nn", 4, 40, 52, 200), ("nn", 16, 33, 1060, 44), ("nn", 16, 20, 1700, 300),
-    ("nt", 4, 12, 52, 200), ("nt", 16, 16, 1036, 148), ("nt", 4, 40, 68, 200), ("nt", 16, 33, 1060, 44)])
+    ("nt", 4, 12, 52, 200), ("nt", 16, 16, 1036, 148), ("nt", 4, 40, 68, 200), ("nt", 16, 33, 1060, 44), ("nt", 16, 14, 572, 1172), ("nt", 16, 4, 1020, 260)])
 def test_expert_gemm_few_fp32_rows_have_the_tiles_bits(form, B, cap, n, k):
     from planmoe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(n + k)
@@ -860,7 +860,8 @@ def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(kernel, form, B, cap, 
 @pytest.mark.parametrize("kernel,form,B,cap,n,k,hint", [
     ("f32 64x64 four stages", "nn", 4, 320, 1024, 512, 256), ("f32 64x64 four stages", "nt", 4, 320, 1024, 512, 256), ("f32 32x32", "nn", 4, 320, 512, 1024, 256),
     ("f32 64x64 four stages", "nn", 8, 35, 1976, 384, 35), ("f32 64x64 four stages", "nn", 4, 114, 1792, 388, 114), ("f32 32x32", "nt", 4, 95, 2104, 2848, 95),
-    ("f32 32x32", "nt", 8, 197, 1024, 3520, 157)])
+    ("f32 32x32", "nt", 8, 197, 1024, 3520, 157), ("f32 waves", "nt", 8, 5, 1408, 384, 3), ("f32 waves", "nt", 4, 4, 3784, 228, 4),
+    ("f32 32x32", "nt", 4, 15, 3636, 1920, 15), ("f32 32x32 eight stages", "nt", 16, 7, 448, 524, 5)])
 def test_expert_gemm_fp32_tiles_by_what_they_measured(kernel, form, B, cap, n, k, hint):
     from planmoe_amd import ops
     assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=True, rows_hint=hint) == kernel
