@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
 // out[t] = sum_j (live_j ? gate_j * dispatched[slot_j] : 0), planes added left to right.  Bound by memory.  A wave asks for B units a lane
 // of two choices' rows before it adds any (a dropped choice reads slot 0 and contributes zeros): one wait a pass over 4 KB rows, and
 // over 8 KB rows with B = 8 (8192 x 2048 fp32, two choices, 201 MB: 36.7 us, 38.5 with four units of one choice at a time, 38.8 of two; 14020 x 3528 bf16
-// 54.8, 57.7, 57.5; rows of 2 KB lose with eight: 16384 x 1024 bf16 17.5 and 23.6; which rows take eight: planmoe_combine_fwd).
+// 54.8, 57.7, 57.5; rows of 2 KB lose with eight: 16384 x 1024 bf16 17.5 and 23.6; which rows take one and which eight: planmoe_combine_fwd).
 template <int DT, int MODE, int B>
 __global__ __launch_bounds__(256) void combine_kernel(
     const void *__restrict__ dispatched, const float *__restrict__ gates,
@@ -464,6 +464,9 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     const int64_t row_bytes = (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2);
     const bool few_lanes = ((row_bytes + 15) / 16 + 255) % 256 < 8;
     const bool wide = row_bytes > 4096 && (dtype == PLANMOE_F32 || mode == ROWS_1 || few_lanes || !stays(row_bytes * samples * (top_k + 1)));
+    // One unit a lane where a wave covers a row with them: more are loads that are thrown away.  us, two choices, four units of one choice at a time, four of two, one of two:
+    // 2156 x 64 bf16 4.9, 5.4, 2.8   1514 x 32 fp16 4.7, 6.1, 2.7   12971 x 100 fp32 7.2, 6.5, 4.4   16000 x 512 bf16 11.8, 12.0, 8.4
+    const bool narrow = model_dim <= WAVE * (mode == ROWS_1 ? 1 : dtype == PLANMOE_F32 ? 4 : 8);
     if (capacity == 0) {
         // no slot exists, every choice is dropped: zero rows.  (combine_kernel fetches rows with
         // unconditional loads at clamped slots and must not run without a row to read.)
@@ -475,7 +478,8 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     }
     PM_DTYPE_SWITCH(dtype, DT, {
         PM_ROWS_SWITCH(mode, MODE, ({
-            if (wide) combine_kernel<DT, MODE, 8><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
+            if (narrow) combine_kernel<DT, MODE, 1><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
+            else if (wide) combine_kernel<DT, MODE, 8><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
             else combine_kernel<DT, MODE, 4><<<blocks, 256, 0, st>>>(dispatched, gates, indices, locations, plane_stride, top_k, samples, model_dim, capacity, out);
         }));
     });

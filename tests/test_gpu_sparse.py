@@ -65,10 +65,12 @@ def test_dispatch_and_combine_bit_exact(T, M, E, k, cf, dtype):
 
 
 @pytest.mark.parametrize("M,dtype", [(1020, torch.float32), (1028, torch.float32), (2048, torch.float32), (2052, torch.float32), (2056, torch.bfloat16),
-                                     (4104, torch.bfloat16), (2050, torch.float16), (257, torch.float16), (2051, torch.bfloat16), (2112, torch.bfloat16), (2120, torch.bfloat16), (3876, torch.bfloat16)])
-@pytest.mark.parametrize("k", [1, 3, 5])
+                                     (4104, torch.bfloat16), (2050, torch.float16), (257, torch.float16), (2051, torch.bfloat16), (2112, torch.bfloat16), (2120, torch.bfloat16), (3876, torch.bfloat16),
+                                     (4, torch.float32), (256, torch.float32), (260, torch.float32), (512, torch.bfloat16), (520, torch.float16), (100, torch.bfloat16),
+                                     (1, torch.float16), (64, torch.float16), (63, torch.bfloat16), (65, torch.float32)])
+@pytest.mark.parametrize("k", [1, 2, 3, 5])
 def test_rows_around_a_pass_bit_exact(M, dtype, k):
-    """Rows that end around the vectors a wave asks for at once (four or eight a lane), odd numbers of choices."""
+    """Rows that end around the vectors a wave asks for at once (one, four or eight a lane), odd numbers of choices."""
     from planmoe_amd import ops
     T, E = 41, 6
     idx, loc, gates, C = _routing(T, E, k, 0.75, seed=M + k)
