@@ -514,6 +514,29 @@ extern "C" int planmoe_layer_relu_bwd(int dtype, const void *grad_rows, const vo
                          workspace_bytes, others, 2, (hipStream_t)stream);
 }
 
+// Up to how many tokens layer_dx_few_kernel takes less than layer_dx_kernel (for rows above 8 KB than the two launches), whose trips other waves hide beyond.
+// Time of the first by that of the second, means over row lengths, one choice and two, 7 experts and 12 and 16, at so many tokens:
+//   vectors a lane, fp32 (7)                  16 bits (7)                               fp32 (12, 16)              16 bits (12, 16)
+//   1                1000 0.84   4000 0.85    1000 0.97   1400 1.02                     2000 0.89   2800 1.00      60 1.05   1000 1.02
+//   2 to 4           1000 0.69   4000 0.72    1000 0.93   1400 0.95   2000 1.04         1400 0.85   2000 0.96      1000 0.94   1400 0.98   2000 1.12
+//   5 to 8           1000 0.50   4000 0.68    1000 0.88   1400 0.90   2000 1.05         1400 0.94   2000 1.17      767 0.91   1000 1.06
+//   9 to 16          1000 0.56   4000 0.85    1000 0.54   2800 0.82   4000 0.93 (12 KB, 3 and 4 experts 1.07)
+// and through the codec, where every wave reads the whole row
+//   1                500 0.87   767 0.87      500 0.98   767 0.97                       500 0.71   767 0.71        60 1.04   767 1.01
+//   2 to 4           500 0.67   767 0.76      500 0.82   767 0.99                       500 0.56   767 0.65        500 0.79   767 0.97
+//   5 to 8           500 0.51   767 0.74      500 0.75   767 0.99                       500 0.50   767 0.72        500 0.92   767 1.29
+//   9 to 16 (beyond 256 fp32 x 4096 25.7 us at 700 tokens, 34.2 so)   60 0.48           16 bits 60 0.39
+static int64_t dx_few_tokens(int dtype, int codec, int per_lane, int experts)
+{
+    const bool f32 = dtype == PLANMOE_F32, many = experts > 8;
+    int64_t a_unit;                              // tokens a compute unit
+    if (!f32 && many && per_lane == 1) a_unit = 0;
+    else if (codec) a_unit = per_lane > 8 ? 1 : f32 ? 3 : 2;
+    else if (f32) a_unit = !many ? 16 : per_lane > 2 ? 6 : 8;
+    else a_unit = per_lane > 8 ? 12 : per_lane > 4 ? many ? 3 : 6 : per_lane > 1 ? 5 : 4;
+    return a_unit * compute_units();
+}
+
 extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const int32_t *indices, const int32_t *locations, int64_t plane_stride,
                                 int top_k, int samples, int model_dim, int experts, int capacity, const float *grad_logits, const void *wg,
                                 void *out, void *stream)
@@ -525,11 +548,7 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
     PM_REQUIRE(grad_logits && wg && out && aligned16(wg) && aligned16(out), "%s: NULL or unaligned argument", who);
     const int per_lane = (model_dim / (dtype == PLANMOE_F32 ? 4 : 8) + WAVE - 1) / WAVE;
     PM_REQUIRE(experts <= 8 || per_lane <= 8, "%s: more than 8 experts: rows of up to 8 KB", who);
-    // Few tokens (layer_dx_few_kernel) up to where the trips are hidden by other waves: 4200 tokens without the codec 13.1 and 12.7 us (fp32 x 920, 8 experts),
-    // 14.5 and 13.3 (bf16 x 1024, 16), 8000 tokens 19.1 and 21.6, 20.6 and 20.4; with it 700 tokens 8.7 and 7.9 (bf16 x 1888), 12.9 and 7.2 (fp32 x 768),
-    // 1500 tokens 11.4 and 12.2, 15.0 and 12.1.  16 experts' weights in fp32 are read once for two tokens beyond (x 1024, 1500 tokens 10.9 and 9.4, 4000 15.2 and 18.4); rows
-    // of more than 8 KB, four times through the codec, one compute unit each (fp32 x 4096, the two launches and this one, 100 tokens 21.6 and 12.0, 700 25.7 and 34.2).
-    const bool few = samples <= (codec ? per_lane > 8 ? 1 : 3 : dtype == PLANMOE_F32 && experts > 8 ? 8 : 16) * compute_units();
+    const bool few = samples <= dx_few_tokens(dtype, codec, per_lane, experts);
     if (per_lane > 8 && !few) {
         if (planmoe_layer_combine(rows, dtype, codec, nullptr, indices, locations, plane_stride, top_k, samples, model_dim, experts, capacity, out, stream)) return 1;
         return planmoe_gate_dx_accumulate(out, dtype, grad_logits, wg, samples, model_dim, experts, stream);
@@ -549,7 +568,7 @@ extern "C" int planmoe_layer_dx(const void *rows, int dtype, int codec, const in
     } while (0)
 #define PM_DX_(CACHE, INT8, EP)                                                                                 \
     do {                                                                                                        \
-        if (few) { PM_DX_FEW(CACHE, INT8, EP); break; }                                                         \
+        if constexpr (DT == PLANMOE_F32 || EP <= 8 || CACHE > 1) { if (few) { PM_DX_FEW(CACHE, INT8, EP); break; } }                \
         if constexpr (DT == PLANMOE_F32) { if (pairs) { PM_DX__(CACHE, INT8, EP, 2); break; } }                 \
         PM_DX__(CACHE, INT8, EP, 1);                                                                            \
     } while (0)

@@ -767,7 +767,8 @@ def test_product_in_fewer_shares(T, M, H, E, k, cap, splits):
 
 # The combine that adds the gate's share of the gradient of x, for 9 to 16 experts: against the combine as it is and the product in 64 bits.  One token,
 # an odd number (two a wave in fp32), rows of one piece, of one more than a wave's 64 and of 8 KB; choices without a slot
-@pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 9, 1, 1), (5, 520, 16, 2, 1), (301, 1032, 11, 3, 40), (64, 2048, 16, 2, 8), (33, 4096, 16, 2, 4)])
+@pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 9, 1, 1), (5, 520, 16, 2, 1), (301, 1032, 11, 3, 40), (64, 2048, 16, 2, 8), (33, 4096, 16, 2, 4),
+                                         (1281, 1032, 12, 2, 200), (2049, 264, 16, 1, 100)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("codec", [0, 1])
 def test_layer_dx_of_up_to_16_experts(T, M, E, k, cap, dtype, codec):
@@ -796,7 +797,9 @@ def test_layer_dx_of_up_to_16_experts(T, M, E, k, cap, dtype, codec):
 # Few tokens, up to 8 experts: the same bits as the combine and the gate's share in launches of their own.  One token, an odd number; rows of less than a
 # wave's 64 pieces, of one more, of two, five and nine times 64 and of sixteen, the widest; the last number of tokens that is few and the first that is not
 @pytest.mark.parametrize("T,M,E,k,cap", [(1, 8, 1, 1, 1), (5, 264, 8, 2, 1), (255, 520, 3, 2, 100), (37, 1288, 8, 2, 8), (131, 2568, 5, 3, 64), (9, 4096, 8, 2, 4), (7, 8192, 4, 2, 4),
-                                         (256, 3080, 2, 1, 100), (257, 3080, 2, 1, 100), (768, 776, 8, 2, 200), (769, 776, 8, 2, 200), (4096, 264, 4, 1, 1000), (4097, 264, 4, 1, 1000)])
+                                         (256, 3080, 2, 1, 100), (257, 3080, 2, 1, 100), (768, 776, 8, 2, 200), (769, 776, 8, 2, 200), (4096, 264, 4, 1, 1000), (4097, 264, 4, 1, 1000),
+                                         (512, 776, 8, 2, 100), (513, 776, 8, 2, 100), (1024, 264, 8, 2, 300), (1025, 264, 8, 2, 300), (1280, 1032, 8, 2, 300), (1281, 1032, 8, 2, 300),
+                                         (1536, 2568, 4, 1, 500), (1537, 2568, 4, 1, 500), (3072, 4104, 2, 1, 2000), (3073, 4104, 2, 1, 2000)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("codec", [0, 1])
 def test_layer_dx_of_few_tokens(T, M, E, k, cap, dtype, codec):
