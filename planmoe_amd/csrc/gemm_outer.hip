@@ -4,19 +4,25 @@
 // barrier: it has nothing to wait for but its few loads, and what it stores is 256 bytes of a row at a time (a lane's columns are next to each
 // other: fragment j of the second operand is every J-th column from the j-th on).  The tiles of the other kernels load a whole k-tile of 32
 // or 64, pass it through LDS and, in fp32, store 32 bytes of a row at a time, two or three of them on a compute unit.
-// fp32 as in gemm_f32_split.hip, in three bf16 parts, the sums in the same order: the same bits.
+// fp32 as in gemm_f32_split.hip, in three bf16 parts, the sums in the same order: the same bits where operands and sums are finite.  A wave with one that is not
+// sums its 32 x 64 again in another order, the tiles theirs, so that what is finite beside it may differ in its last bits.
+//
+// us, the tiles and this:
+//   fp32  16 x 1 row, 3328 x 3072 204, 98    8 x 8, 2600 x 3440 94, 56    16 x 2, 1896 x 688 31, 18    8 x 2, 4096 x 4096 162, 81    8 x 64, 2048 x 2048 59, 45
+//   bf16  16 x 1 row, 3328 x 3072  85, 53    8 x 8, 2600 x 3440 54, 31    8 x 29, 1888 x 1256 17, 12   8 x 2, 4096 x 4096  67, 42    8 x 64, 2048 x 2048 22, 18
 //
 // Stored past the caches: an optimizer reads a weight gradient once and late.  Rows that are not whole lines share a line with the next row's wave, which
 // the caches put together: such rows are stored plainly, in bf16 256 columns a wave so that there are fewer of those lines, in fp32 only where the last
-// cache (256 MB) does not hold the result.  In bf16 the waves that share lines are brought together as well (8 experts x 8 rows, 2600 x 3440, 37 and 31 us; x 29,
-// 1888 x 1256, 15.8 and 14.7; x 64, 1896 x 1032, 19.3 and 17.6; in fp32 16 x 1, 3328 x 3072 103 and 117).  Neither a step of k asked for ahead of the
-// products nor 128 rows of 64 columns a work-group gained anything in the others.  us, before that: the tiles, then 32 x 128 (bf16 256) plain and past the caches, 32 x 64 (bf16 128) plain and past them
-//   fp32  16 x 1, 3328 x 3072  220: 119, 116, 134, 112     8 x 8, 2600 x 3440   100: 56, 58, 56, 63     16 x 2, 1896 x 688   33: 23, 22, 20, 19
-//         8 x 2, 4096 x 4096   178: 94, 84, 108, 89        8 x 64, 2048 x 2048   65: 52, 50, 50, 50     8 x 128, 2048 x 2048 95: 81, 80, 85, 83
-//         4 x 128, 512 x 1024  10.5: 14.8, 13.5, 10.9, 10.3
-//   bf16  16 x 1, 3328 x 3072   91: 63, 65, 61, 59         8 x 8, 2600 x 3440    56: 38, 41, 42, 48     16 x 2, 1896 x 688   20: 12, 12, 16, 16
-//         8 x 2, 4096 x 4096    73: 57, 55, 45, 43         8 x 64, 2048 x 2048   24: 27, 25, 22, 18     8 x 80, 2048 x 2048  24: 29, 27, 24, 22
-//         8 x 64, 1896 x 1032   18: 17, 17, 17, 16         8 x 100, 2048 x 2048  24: 32, 31, 29, 27
+// cache (256 MB) does not hold the result.  In bf16 the waves that share lines are brought together as well (8 experts x 8 rows, 2600 x 3440, 37 and 31 us; in fp32 16 x 1,
+// 3328 x 3072 103 and 117).  Neither a step of k asked for ahead of the products nor 128 rows of 64 columns a work-group gained anything in the others.  What that choice
+// is from, us, before the waves were brought together: 32 x 128 (bf16 256) plain and past the caches, 32 x 64 (bf16 128) plain and past them; of these fp32 has the last two, bf16 the
+// first and the last, the others were not kept
+//   fp32  16 x 1, 3328 x 3072  119, 116, 134, 112     8 x 8, 2600 x 3440    56, 58, 56, 63     16 x 2, 1896 x 688   23, 22, 20, 19
+//         8 x 2, 4096 x 4096   94, 84, 108, 89        8 x 64, 2048 x 2048   52, 50, 50, 50     8 x 128, 2048 x 2048 81, 80, 85, 83
+//         4 x 128, 512 x 1024  14.8, 13.5, 10.9, 10.3
+//   bf16  16 x 1, 3328 x 3072  63, 65, 61, 59         8 x 8, 2600 x 3440    38, 41, 42, 48     16 x 2, 1896 x 688   12, 12, 16, 16
+//         8 x 2, 4096 x 4096   57, 55, 45, 43         8 x 64, 2048 x 2048   27, 25, 22, 18     8 x 80, 2048 x 2048  29, 27, 24, 22
+//         8 x 64, 1896 x 1032  17, 17, 17, 16         8 x 100, 2048 x 2048  32, 31, 29, 27
 #include "gemm_outer.hpp"
 #include "sp_split.hpp"
 
@@ -26,7 +32,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 op_bf16x8 __attribute__((ext_vector_type(8)));
 
 template <bool F32, int J, bool NT>
-__global__ __launch_bounds__(256, (F32 ? J == 4 : J == 8) ? 2 : 4) void gemm_outer_kernel(const OuterArgs p)
+__global__ __launch_bounds__(256, !F32 && J == 8 ? 2 : 4) void gemm_outer_kernel(const OuterArgs p)
 {
     constexpr int COLS = 32 * J, SIZE = F32 ? 4 : 2, W = J * SIZE / 4;        // W: words of a lane's columns
     typedef uint32_t words __attribute__((ext_vector_type(W)));
