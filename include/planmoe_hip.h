@@ -444,7 +444,8 @@ int planmoe_transpose_bf16(const void *in, int batches, int rows, int cols, int 
  * k, m], b [batches, k, n].  Roundings as planmoe_gemm_*_bf16.  fp32: products and sums are no less precise than
  * an fp32 multiply and add a k; the order of the sums is that of the fp32 matrix cores' products of 16 x 16 x 4
  * with activation 1, and with row lengths under 256, where it does not depend on m; elsewhere it may differ from shape to shape
- * (form, batches, m, n, k), but not with live or rows_hint.  activation: 0 none, 1 relu.
+ * (form, batches, m, n, k), but not with live or rows_hint (there, what is finite beside an infinity, a NaN or a sum above 2^80 may differ in its last
+ * bits with them).  activation: 0 none, 1 relu.
  * live, if not NULL: int32 [live_planes][batches], e.g. the expert_counts of the routing.  Batch e then has
  * min(sum of its entries rounded up to live_round, m) rows (form 2: that many k) in use; rows of c beyond
  * them are not written, rows of a and b beyond them are not read (up to 64 batches).  rows_hint: the number
@@ -566,7 +567,7 @@ int planmoe_layer_relu_bwd(int dtype, const void *grad_rows, const void *w2, con
                            void *dwg, void *stream);
 
 /* The gradient of x: planmoe_layer_combine without gates, then planmoe_gate_dx_accumulate, the same roundings, in one pass
- * where a row is at most 8 KB (up to 8 experts; up to 16 for such rows). */
+ * where a row is at most 8 KB (up to 8 experts; up to 16 for such rows) and for few tokens whatever a row is (up to 16 KB, 8 experts), in two otherwise. */
 int planmoe_layer_dx(const void *rows, int dtype, int codec, const int32_t *indices, const int32_t *locations,
                      int64_t plane_stride, int top_k, int samples, int model_dim, int experts, int capacity,
                      const float *grad_logits, const void *wg, void *out, void *stream);
@@ -678,9 +679,10 @@ int planmoe_bwd_gate_zfp(const void *stream_in, double rate, const float *grad_o
  * with blocks = planmoe_lz_blocks(nbytes).  nbytes must be a multiple of 4 and below 2^31; a
  * last partial block is coded as if padded with zero symbols (the reference reads past the end
  * of its input there, gpulz.cu:36-39), and decoding writes only the first nbytes.
- * Compression sizes every block, scans the sizes in place in the offset tables and then packs
- * every block at its final offset; the workspace keeps the tokens of blocks with matches, half the input's size (gpulz.cu:148-211,
- * 220-258 have two full-size staging buffers).  All five pointers must be 16-byte aligned. */
+ * Compression sizes every block and packs every block at its final offset, which up to 8192 blocks (16 MB) a work-group adds up from
+ * the sizes itself; of more the sizes are scanned in place in the offset tables in between.  The workspace keeps a class byte a block, the sizes of up to 8192 blocks and
+ * the tokens of blocks with matches, half the input's size (gpulz.cu:148-211, 220-258 have two full-size staging buffers); one for an input serves every
+ * shorter one.  input, flags, data and the offset tables must be 16-byte aligned, the workspace 4. */
 int64_t planmoe_lz_blocks(int64_t nbytes);
 size_t planmoe_lz_workspace_bytes(int64_t nbytes);
 int planmoe_lz_compress(const void *input, int64_t nbytes, int32_t *flag_offsets, int32_t *data_offsets,

@@ -360,7 +360,8 @@ __global__ __launch_bounds__(256) void combine_bwd_kernel(
 // the memory-side cache hold them: what follows a dispatch reads its rows, a combine's backward pass reads rows and writes as many.  us, dispatch, combine, its
 // backward pass, combine, by what is stored plainly: none, the dispatch's rows, the backward pass's too
 //   rows of 134 MB in all 174, 162, 159     218 MB 281, 267, 284     246 MB 270, 262, 274     335 MB 374, 399, 420     84 MB 104.6, 101.9, 99.2
-// (What a combine stores is stored past them: 8192 x 2048 fp32 171 in place of 159.)
+// (What a combine stores is stored past them: 8192 x 2048 fp32 171 in place of 159.)  A call alone, one after the other into the same rows that nothing reads, is up to 16 % slower for
+// it (5779 x 2176 fp16 dispatch 13.5 and 15.7), with the combine behind it 500 sizes take 0.93 - 0.94 of the time.
 static bool stays(int64_t bytes) { return bytes <= (int64_t)256 << 20; }
 #define PM_STREAM_SWITCH(streams, MODE, STREAM, ...)                                                 \
     do {                                                                                             \
@@ -461,6 +462,7 @@ extern "C" int planmoe_combine_fwd(const void *dispatched, int dtype, const floa
     // 3528 beside the kernel), or where eight lanes at most have a unit of a row's last pass of four a lane.  us, two choices, bf16 rows that the caches hold, with
     // four and with eight:  1400 tokens x 3876 6.8, 7.5   4000 x 4096 15.9, 17.8   4000 x 2176 10.9, 11.8   8000 x 2304 19.2, 20.9   1400 x 2112 7.0, 5.8
     // fp32:  1400 x 1056 5.5, 4.6   1400 x 2048 5.9, 5.5   4000 x 2560 19.3, 19.5   6800 x 4096 66, 62
+    // An element at a time (rows that start anywhere), in bf16:  300 x 3877 10.0, 7.9   2000 x 2051 8.9, 7.9   2000 x 3877 14.7, 11.8   8000 x 2051 19.2, 19.7   14000 x 3877 69, 65
     const int64_t row_bytes = (int64_t)model_dim * (dtype == PLANMOE_F32 ? 4 : 2);
     const bool few_lanes = ((row_bytes + 15) / 16 + 255) % 256 < 8;
     const bool wide = row_bytes > 4096 && (dtype == PLANMOE_F32 || mode == ROWS_1 || few_lanes || !stays(row_bytes * samples * (top_k + 1)));
