@@ -471,6 +471,7 @@ static int gemm_f32_wave_launch(const Gemm32Args &p, int waves, hipStream_t stre
 // us with 16 columns and four waves a work-group everywhere, and now, weights cold, in the last cache:
 //   8 x 1 row, 1024 -> 4096   33, 28 and 27, 22       8 x 7, 2600 -> 3440    80, 72 and 58, 52       16 x 512 -> 2048   20, 19 and 15, 14
 //   8 x 20, 1024 -> 4096      44, 38 and 34, 28       16 x 1, 3328 -> 3072  149 and 95 (cold)
+// (A row an expert by counts from the device, some of them without: single waves find a compute unit each, 16 x 224 -> 3136, 4 in use 11.0 and 8.5 us, all 14.1 and 13.0.)
 static int gemm_f32_waves(int form, const Gemm32Args &p, int rows_hint, hipStream_t stream, const char *who)
 {
     const int64_t strips = gemm_f32_pieces(p, rows_hint, 16), cu = compute_units();
@@ -479,7 +480,7 @@ static int gemm_f32_waves(int form, const Gemm32Args &p, int rows_hint, hipStrea
     if (strips < 4 * cu) return one ? gemm_f32_wave_launch<1, 1, 8, true>(p, 1, stream, who) : gemm_f32_wave_launch<2, 1, 4, true>(p, 1, stream, who);
     if (!one) return gemm_f32_wave_launch<2, 2, 4, true>(p, 1, stream, who);
     if (gemm_f32_past_caches(p) && strips >= 8 * cu) return gemm_f32_wave_launch<1, 4, 2, true, true>(p, 1, stream, who);
-    return gemm_f32_wave_launch<1, 2, 4, true>(p, strips < 5 * cu ? 1 : 4, stream, who);
+    return gemm_f32_wave_launch<1, 2, 4, true>(p, strips < 5 * cu || (p.live && rows_hint == 1) ? 1 : 4, stream, who);
 }
 
 template <int F, bool TA, bool TB, int STAGES = 2>
@@ -597,9 +598,14 @@ Gemm32Kernel gemm_f32_pick(int form, const Gemm32Args &p, int rows_hint)
     const double kt = (double)(((form == 2 ? rows_hint : p.K) + G32_BK - 1) / G32_BK);
     if (form != 2 && rows_hint <= 32) {
         const int64_t pieces = gemm_f32_pieces(p, rows_hint, 32);
+        // Rows for as many batches at most, by counts from the device: how many of those have one is not known, and waves of 32 and 64 columns that would fill the chip for all
+        // are too few for a weight or three.  64 x 64, whose waves take 16 columns of up to 16 rows, is near the better one for any number.  us, waves and these, 16 experts, 2328 -> 3712:
+        // 1 in use 50, 20   3 51, 22   8 58, 43   12 66, 83   16 82, 91;  8 experts, 2688 -> 4096: 1 55, 24   4 58, 36   8 59, 61;  512 -> 4096: 1 10.4, 7.9   4 13.4, 11.4   8 16.2, 18.7
+        const bool some = p.live && rows_hint == 1 && deep;
         const bool one = p.M <= 16 && !p.colsum, past = gemm_f32_past_caches(p);
         const bool lines = pieces > 3 * cu && pieces <= 4 * cu && (one || (form == 0 && !past));
         const bool fits = (int64_t)p.M * p.K * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31) && gemm_f32_wave_pieces(p, 16, 16) < ((int64_t)1 << 30);
+        if (some && form == 0 && (lines || (one && past && pieces >= 4 * cu))) return G32_DEEP_64;
         const bool turns = form == 1 && one && pieces > cu && 2 * pieces <= (rows_hint <= 4 ? 4 : 3) * cu;
         if (fits && (!deep || lines || turns || (form == 0 && one && past && pieces >= 4 * cu))) return G32_WAVES;
         if (deep) return pieces <= cu ? G32_SLIM_ALONE : G32_SLIM;

@@ -856,12 +856,29 @@ def test_expert_gemm_small_fp32_tiles_have_the_waves_bits(kernel, form, B, cap, 
             _column_sums_hold(db, got, rows, cap)
 
 
+# A row an expert, of which any number may be without one: tiles of 64 x 64, none of them whole, where waves would do for all; the bits are the waves'
+@pytest.mark.parametrize("B,cap,n,k", [(16, 4, 1700, 300), (8, 12, 3300, 260)])
+@pytest.mark.parametrize("rows", [[0, 0, 1], [1], [0], [4, 0, 2, 0, 0, 1, 12]])
+def test_expert_gemm_of_a_row_an_expert(B, cap, n, k, rows):
+    from planmoe_amd import ops
+    assert [ops.expert_gemm_kernel("nn", torch.float32, B, cap, n, k, counted=True, relu=True, rows_hint=h) for h in (1, 2)] == ["f32 64x64 four stages", "f32 waves"]
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rows = [min(cap, rows[e % len(rows)]) for e in range(B)]
+    live = torch.tensor([rows], dtype=torch.int32, device=DEV)
+    a, w, bias = (torch.randn(*shape, device=DEV, generator=g) for shape in ((B, cap, k), (B, k, n), (B, n)))
+    for e, r in enumerate(rows):
+        a[e, r:] = float("nan")
+    got, want = (ops.expert_gemm("nn", a, w, bias, relu=True, live=live, rows_hint=h, out=torch.full((B, cap, n), 7.0, device=DEV)) for h in (1, 2))
+    assert torch.equal(got, want) and all(bool((got[e, r:] == 7.0).all() and got[e, :r].isfinite().all()) for e, r in enumerate(rows))
+
+
 # fp32 tiles of 64 x 64 where those of 32 x 32 are several a compute unit in turn and measured slower (16.7 and 18.9 us the first), and the other way round
 @pytest.mark.parametrize("kernel,form,B,cap,n,k,hint", [
     ("f32 64x64 four stages", "nn", 4, 320, 1024, 512, 256), ("f32 64x64 four stages", "nt", 4, 320, 1024, 512, 256), ("f32 32x32", "nn", 4, 320, 512, 1024, 256),
     ("f32 64x64 four stages", "nn", 8, 35, 1976, 384, 35), ("f32 64x64 four stages", "nn", 4, 114, 1792, 388, 114), ("f32 32x32", "nt", 4, 95, 2104, 2848, 95),
     ("f32 32x32", "nt", 8, 197, 1024, 3520, 157), ("f32 waves", "nt", 8, 5, 1408, 384, 3), ("f32 waves", "nt", 4, 4, 3784, 228, 4),
-    ("f32 32x32", "nt", 4, 15, 3636, 1920, 15), ("f32 32x32 eight stages", "nt", 16, 7, 448, 524, 5)])
+    ("f32 64x64 four stages", "nn", 16, 4, 3712, 2328, 1), ("f32 64x64 four stages", "nn", 8, 4, 4096, 512, 1), ("f32 waves", "nn", 8, 4, 4096, 512, 2),
+    ("f32 waves", "nn", 8, 4, 4096, 200, 1), ("f32 32x32", "nt", 4, 15, 3636, 1920, 15), ("f32 32x32 eight stages", "nt", 16, 7, 448, 524, 5)])
 def test_expert_gemm_fp32_tiles_by_what_they_measured(kernel, form, B, cap, n, k, hint):
     from planmoe_amd import ops
     assert ops.expert_gemm_kernel(form, torch.float32, B, cap, n, k, relu=form == "nn", counted=True, rows_hint=hint) == kernel
